@@ -1,13 +1,197 @@
 // C = A B^T for a few rows of A (a batch's decode step): bound by streaming B, (N, K), once.
 //
-// A block takes 16 rows of B -- the 16x16x32 MFMA's first operand -- and its eight waves deal K in pieces
-// of 64 columns (a whole 128-byte line of each row), all of A's rows (up to 16 * MT) the second operand.
-// The waves' sums meet in LDS.  With GATED a second matrix is streamed beside the first and the output is
-// act(A B^T) * (A B2^T), rounded where the separate steps round.
+// Two kernels.  `gemm_strips_kernel` takes B eight rows at a time through LDS; `gemm_few_kernel` takes sixteen straight into the
+// MFMA's registers and stands where the first's operands do not fit.  With GATED a second matrix is streamed beside the first and
+// the output is act(A B^T) * (A B2^T), rounded where the separate steps round.
 #include "../../include/iron_hip.h"
 #include "common.h"
 
+#include <type_traits>
+
 namespace iron {
+
+// A block's eight waves deal K in strips of 256 columns: a strip of a tile's eight rows of B is 4 KB, sent from memory into the wave's own
+// part of LDS as 512-byte runs (16-byte pieces XORed by the row, so that the MFMA's fragments read back without bank conflicts), STAGES - 1
+// strips ahead; no wave waits for another until a tile's sums meet.  With SINGLE (K up to eight strips) a wave keeps its strip of A in
+// registers over all of a block's tiles; else a strip of A is fetched with each of B.
+//
+// What bounds it is the way to the memory, so the shape follows that: eight rows a tile and not the MFMA's sixteen (half of each product is
+// dropped; the matrix cores idle anyway), because 2048 rows of B then occupy all 256 CUs; up to sixteen rows of A as contiguous runs, because
+// rows a power of two apart, read a fragment at a time by every block, meet on one L2 channel.  Eight rows of A over cold weights, us with
+// gemm_few_kernel and with this: 2048 x 2048 5.1 / 4.1, 2048 x 8192 14.1 / 9.3, 4160 x 2048 8.0 / 6.0, 8192 x 2048 10.2 / 8.8,
+// 10240 x 2048 15.0 / 10.3, 128256 x 2048 106 / 86 (6.1 TB/s); thirty-two rows: 4160 x 2048 14.3 / 9.6, 128256 x 2048 163 / 92.
+constexpr int STRIP = 256, STRIP_BYTES = 512, STRIP_WAVES = 8, STRIP_ROWS = 8;
+constexpr int STRIP_OUT = 64;   // columns of C staged for a store of whole lines: 128256 x 2048 98 -> 86 us with the loads past the caches
+
+__device__ __forceinline__ void lds_write_b128(unsigned addr, const f32x4& v) { asm volatile("ds_write_b128 %0, %1" ::"v"(addr), "v"(v) : "memory"); }
+// A barrier behind the wave's own LDS accesses that leaves its loads from memory in flight.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// MT: tiles of sixteen rows of A; one of them has MA rows at the most and comes by LDS, more come straight into registers.
+template <int MT, int MA, bool SINGLE, int STAGES>
+struct Strips {
+  static constexpr bool A_BY_LDS = MT == 1;
+  static constexpr int A_BYTES = A_BY_LDS ? MA * STRIP_BYTES : 0, B_BYTES = STRIP_ROWS * STRIP_BYTES;
+  static constexpr int ITEM = (SINGLE ? 0 : A_BYTES) + B_BYTES, WAVE = ITEM * STAGES + (SINGLE ? A_BYTES : 0);
+  static constexpr int PART = STRIP_WAVES * MT * 1024, OUT = MT * 16 * STRIP_OUT * 2;
+  static constexpr int LDS = STRIP_WAVES * WAVE + 2 * PART + 2 * OUT;
+  static constexpr int A_INST = A_BYTES / 1024, B_INST = B_BYTES / 1024, INST = ITEM / 1024;
+};
+
+template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM>
+__global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
+                                                                       bf16_t* __restrict__ C, int M, int N, int K) {
+  typedef Strips<MT, MA, SINGLE, STAGES> S;
+  constexpr int W = STRIP_WAVES, R = STRIP_ROWS, GROUP = STRIP_OUT / R;   // GROUP: tiles whose columns are stored together
+  constexpr int NOWHERE = 0x7ffffff0;   // an offset past the end of every run of rows (the entry point bounds M * K)
+  extern __shared__ __align__(1024) char lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l16 = lane & 15, quad = lane >> 4;
+  const int strips = (K + STRIP - 1) / STRIP, mine = SINGLE ? 1 : (strips - wave + W - 1) / W, most = SINGLE ? 1 : (strips + W - 1) / W;
+  // A block's tiles are neighbours, so that its columns of C leave as whole lines.
+  const unsigned tiles = (N + R - 1) / R;   // (up to 2^19, the blocks 256)
+  const int tile0 = blockIdx.x * tiles / gridDim.x, my_tiles = (blockIdx.x + 1) * tiles / gridDim.x - tile0, items = my_tiles * mine;
+  char* const own = lds + wave * S::WAVE;
+  char* const held = own + (SINGLE ? S::A_BYTES : 0);
+  const unsigned lds0 = (unsigned)(uintptr_t)IRON_LDS_PTR(lds), part0 = lds0 + W * S::WAVE, out0 = part0 + 2 * S::PART;
+
+  // `count` loads of two rows each, `past` the caches or not: a lane's place in LDS is fixed, so the row's pieces are chosen by it.  Past the
+  // rows or K: zeros.
+  auto fetch_rows = [&](const bf16_t* base, int rows, int strip, char* to, auto count, auto past) {
+    const __amdgpu_buffer_rsrc_t run = bounded_bytes(base, rows * K * 2);
+#pragma unroll
+    for (int i = 0; i < decltype(count)::value; ++i) {
+      const int r = 2 * i + (lane >> 5), col = strip * STRIP + (((lane & 31) ^ (r & 15)) << 3);
+      const int offset = col < K && r < rows ? (r * K + col) * 2 : NOWHERE;
+      if (decltype(past)::value) __builtin_amdgcn_raw_ptr_buffer_load_lds(run, IRON_LDS_PTR(to + i * 1024), 16, offset, 0, 0, 2);   // non-temporal
+      else __builtin_amdgcn_raw_ptr_buffer_load_lds(run, IRON_LDS_PTR(to + i * 1024), 16, offset, 0, 0, 0);
+    }
+  };
+  auto fetch = [&](int item) {
+    char* to = held + item % STAGES * S::ITEM;
+    const int t = SINGLE ? item : item / max(mine, 1), strip = wave + W * (SINGLE ? 0 : item - t * mine), row0 = (tile0 + t) * R;
+    const int rows = item < items ? min(R, N - row0) : 0;   // past the last item: as many loads, of nothing
+    if (!SINGLE && S::A_BY_LDS) {
+      fetch_rows(A, rows > 0 ? M : 0, strip, to, std::integral_constant<int, S::A_INST>(), std::false_type());
+      to += S::A_BYTES;
+    }
+    fetch_rows(B + (rows > 0 ? (size_t)row0 * K : 0), rows, strip, to, std::integral_constant<int, S::B_INST>(), std::integral_constant<bool, STREAM>());
+  };
+  // Fragments: lane (quad, l16) has columns 32 k + 8 quad .. + 7 of row l16 (of B's eight rows l16 % 8; of a row of A past the last whatever
+  // is there, for columns of the product that are not stored).
+  const int ar = l16 & (MA - 1), br = l16 & (R - 1);
+  const unsigned a_at = ar * STRIP_BYTES + ((quad ^ ar) << 4), b_at = br * STRIP_BYTES + ((quad ^ br) << 4);
+  bf16x8 af[MT][8];
+  auto a_from_memory = [&](int strip) {
+    const __amdgpu_buffer_rsrc_t run = bounded_bytes(A, M * K * 2);
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const int col = strip * STRIP + k * 32 + quad * 8, r = m * 16 + l16;
+        af[m][k] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(run, r < M && col < K ? (r * K + col) * 2 : NOWHERE, 0, 0));
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto a_from_lds = [&](unsigned at) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) af[0][k] = lds_read_b128_at<0>((at + a_at) ^ (k << 6));
+  };
+  if (SINGLE) {
+    if (S::A_BY_LDS) fetch_rows(A, M, wave, own, std::integral_constant<int, S::A_INST>(), std::false_type());
+    else a_from_memory(wave);
+  }
+#pragma unroll
+  for (int i = 0; i < STAGES - 1; ++i) fetch(i);
+  if (SINGLE && S::A_BY_LDS) {
+    __builtin_amdgcn_sched_barrier(0);
+    wait_vmcnt<(STAGES - 1) * S::INST>();
+    a_from_lds(lds0 + (unsigned)(own - lds));
+#pragma unroll
+    for (int k = 0; k < 8; ++k) lds_wait_for<0>(af[0][k]);
+  }
+  const bool whole = N % 8 == 0;   // C's rows take 16-byte pieces
+  // The columns of `count` tiles from `first` on, from half `half` of the out stage, by one wave.
+  auto flush = [&](int first, int count, int half) {
+    for (int e = lane; e < M * count; e += 64) {
+      const int r = e / count, p = e - r * count, n = (tile0 + first + p) * R;
+      bf16x8 v = lds_read_b128_at<0>(out0 + half * S::OUT + (r * STRIP_OUT + p * R) * 2);
+      lds_wait_for<0>(v);
+      if (n < N) *reinterpret_cast<bf16x8*>(C + (size_t)r * N + n) = v;
+    }
+  };
+  int item = 0;
+  for (int t = 0; t < my_tiles; ++t) {
+    f32x4 acc[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < most; ++s) {
+      if (s >= mine) continue;   // (the other waves' last strips)
+      if (!SINGLE && !S::A_BY_LDS) a_from_memory(wave + W * s);
+      fetch(item + STAGES - 1);
+      __builtin_amdgcn_sched_barrier(0);
+      wait_vmcnt<(STAGES - 1) * S::INST>();
+      __builtin_amdgcn_sched_barrier(0);
+      const unsigned at = lds0 + (unsigned)(held - lds) + item % STAGES * S::ITEM;
+      if (!SINGLE && S::A_BY_LDS) a_from_lds(at);
+      bf16x8 bf[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) bf[k] = lds_read_b128_at<0>((at + (SINGLE ? 0 : S::A_BYTES) + b_at) ^ (k << 6));
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        if (!SINGLE && S::A_BY_LDS) lds_wait_for<0>(af[0][k]);
+        lds_wait_for<0>(bf[k]);
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[k], af[m][k], acc[m], 0, 0, 0);
+      ++item;
+    }
+    // The waves' sums meet, through assembly: the compiler would wait for every strip in flight before each access to LDS.
+    const unsigned pa = part0 + (t & 1) * S::PART;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      f32x4 v = acc[m];
+      asm volatile("s_nop 15\n\ts_nop 3" : "+v"(v));   // (the matrix cores' results, which assembly is not waited for with)
+      lds_write_b128(pa + ((wave * MT + m) * 64 + lane) * 16, v);
+    }
+    lds_barrier();
+    if (whole && t > 0 && t % GROUP == 0 && wave == (t + W / 2) % W) flush(t - GROUP, GROUP, (t / GROUP - 1) & 1);
+    // Tile t's sums by wave t % 8: lane (quad, l16) of the first two quads has columns 4 quad .. + 3 of row l16.
+    if (wave == t % W && lane < 32) {
+      const int n = (tile0 + t) * R + quad * 4;
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        bf16x8 p[W];
+#pragma unroll
+        for (int q = 0; q < W; ++q) p[q] = lds_read_b128_at<0>(pa + ((q * MT + m) * 64 + lane) * 16);
+#pragma unroll
+        for (int q = 0; q < W; ++q) lds_wait_for<0>(p[q]);
+        float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < W; ++q)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] += __builtin_bit_cast(f32x4, p[q])[j];
+        const int r = m * 16 + l16;
+        if (whole) {
+          const unsigned to = out0 + (t / GROUP & 1) * S::OUT + (r * STRIP_OUT + t % GROUP * R + quad * 4) * 2;
+          const uint64_t four = (uint64_t)pack_bf16(v[2], v[3]) << 32 | pack_bf16(v[0], v[1]);
+          asm volatile("ds_write_b64 %0, %1" ::"v"(to), "v"(four) : "memory");
+        } else if (r < M) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (n + j < N) C[(size_t)r * N + n + j] = f32_to_bf16(v[j]);
+        }
+      }
+    }
+  }
+  if (whole && my_tiles > 0) {
+    lds_barrier();
+    const int first = (my_tiles - 1) / GROUP * GROUP;
+    if (wave == 0) flush(first, my_tiles - first, first / GROUP & 1);
+  }
+  wait_vmcnt<0>();   // (loads of nothing may still be on their way into LDS)
+}
 
 constexpr int FEW_WAVES = 8, FEW_STEP = 64;   // K columns a wave takes at a time
 
@@ -124,6 +308,44 @@ static int launch_gemm_few(const bf16_t* A, const bf16_t* B, const bf16_t* B2, b
   IRON_LAUNCH_CHECK();
 }
 
+template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM>
+static int launch_gemm_strips(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s) {
+  typedef Strips<MT, MA, SINGLE, STAGES> S;
+  static_assert(S::LDS <= 163840, "a CU's LDS");
+  static LdsOptIn opt;
+  auto kernel = &gemm_strips_kernel<MT, MA, SINGLE, STAGES, STREAM>;
+  const hipError_t e = opt.ensure(reinterpret_cast<const void*>(kernel), S::LDS);
+  if (e != hipSuccess) {
+    set_error("gemm_few: %s", hipGetErrorString(e));
+    return (int)e;
+  }
+  const int tiles = (N + STRIP_ROWS - 1) / STRIP_ROWS;
+  hipLaunchKernelGGL(kernel, dim3(tiles < 256 ? tiles : 256), dim3(STRIP_WAVES * 64), S::LDS, s, A, B, C, M, N, K);
+  IRON_LAUNCH_CHECK();
+}
+
+// Which products go by strips.  Below 4 MB of B a launch is mostly its start, which gemm_few_kernel's is shorter (777 x 1000, 8 rows: 3.3 us
+// against 3.5).  K up to eight strips: up to 32 rows of A (33: 8192 x 2048 15.1 us against 12.6).  A longer K: the strips of A that come with
+// every tile cost as much as B's own, so up to eight rows of A, more only where a block has one tile (16 rows: 2048 x 8192 11.2 us against
+// 16.6, 4096 x 4096 11.0 against 9.9; 48 rows: 30.4 against 33.9, 23.3 against 15.2 at 3072 x 3072).  The loads go past the caches except
+// where a block has one tile over a long K (2048 x 8192, 8 rows: 9.3 us, past them 10.5; 4096 x 4096 10.1 and 9.4).
+// Returns -1 where it is not for them.
+static int strips_for(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s) {
+  if ((long long)N * K < (1 << 21)) return -1;
+  const bool one_tile = N <= 256 * STRIP_ROWS;
+  if (K <= STRIP * STRIP_WAVES) {
+    if (M <= 8) return launch_gemm_strips<1, 8, true, 2, true>(A, B, C, M, N, K, s);
+    if (M <= 16) return launch_gemm_strips<1, 16, true, 2, true>(A, B, C, M, N, K, s);
+    return M <= 32 ? launch_gemm_strips<2, 16, true, 2, true>(A, B, C, M, N, K, s) : -1;
+  }
+  if ((long long)64 * K * 2 >= 0x7ffffff0ll) return -1;   // (offsets within 64 rows are 32 bits wide)
+  if (M <= 8)
+    return one_tile ? launch_gemm_strips<1, 8, false, 2, false>(A, B, C, M, N, K, s) : launch_gemm_strips<1, 8, false, 2, true>(A, B, C, M, N, K, s);
+  if (!one_tile) return -1;
+  if (M <= 16) return launch_gemm_strips<1, 16, false, 1, false>(A, B, C, M, N, K, s);
+  return M <= 32 ? launch_gemm_strips<2, 16, false, 2, false>(A, B, C, M, N, K, s) : launch_gemm_strips<4, 16, false, 2, false>(A, B, C, M, N, K, s);
+}
+
 }  // namespace iron
 
 using namespace iron;
@@ -137,6 +359,10 @@ extern "C" int iron_gemm_few_bf16(const uint16_t* A, const uint16_t* B, const ui
   IRON_REQUIRE(B2 == nullptr || (activation >= 1 && activation <= 3), "gemm_few: activation (%d) is 1 (SiLU), 2 (GELU, tanh form) or 3 (ReLU)",
                activation);
   hipStream_t s = (hipStream_t)stream;
+  if (B2 == nullptr) {
+    const int done = strips_for(A, B, C, M, N, K, s);
+    if (done >= 0) return done;
+  }
   if (B2 != nullptr) return launch_gemm_few<FEW_GATED>(A, B, B2, C, M, N, K, activation, s);
   if (N >= 8192) return launch_gemm_few<FEW_TWO>(A, B, nullptr, C, M, N, K, 0, s);
   return launch_gemm_few<FEW_ONE>(A, B, nullptr, C, M, N, K, 0, s);

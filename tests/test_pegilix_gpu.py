@@ -91,6 +91,23 @@ def test_a_product_over_few_rows(cuda, M, N, K_):
         assert np.abs(from_torch(C) - gated).max() <= 1.5e-2 * np.abs(gated).max(), act
 
 
+# Products that go by strips of K: a tile of B's rows and less, a block's first second tile, groups of eight tiles stored together and the
+# ninth, N no multiple of 8; K just over a strip, to eight strips and past them with waves that have none; the rows of A at every edge.
+@pytest.mark.parametrize("M,N,K_", [(1, 1024, 2048), (8, 2049, 1032), (9, 2056, 1960), (16, 16384 + 72, 264), (17, 18500, 136), (32, 4104, 2048),
+                                    (2, 1027, 2056), (8, 2048, 8192), (7, 2064, 4104), (16, 520, 5000), (29, 2040, 2304), (33, 600, 4096), (63, 999, 2816)])
+def test_a_product_over_few_rows_by_strips(cuda, M, N, K_):
+    rng = np.random.default_rng(N)
+    a, b = bf(rng, M, K_), bf(rng, N, K_, scale=0.1)
+    A, B, C = (device(x, BF16) for x in (a, b, np.full((M + 1, N), 7.0, F32)))
+    K.gemm(A, B, C[:M], M=M, N=N, K=K_, b_col_maj=True)
+    got, want = from_torch(C), a.astype(np.float64) @ b.T
+    # one rounding to bf16 (seven bits behind the point: half of the last place is 2^-8 of the value at the most) and at most K float32
+    # sums of exact products (K 2^-24 of their magnitudes)
+    bound = 2.0**-8 * np.abs(want) + K_ * 2.0**-24 * (np.abs(a).astype(np.float64) @ np.abs(b).T)
+    assert (np.abs(got[:M] - want) <= 1.01 * bound).all()
+    assert (got[M] == 7).all()
+
+
 # ---------------------------------------------------------------- recurrences
 
 
