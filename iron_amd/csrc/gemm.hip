@@ -6,7 +6,7 @@
 // 72 elements so the 16-byte fragment reads of 32 consecutive rows fall in distinct banks),
 // double-buffered; a wave owns a (BM/WM) x (BN/WN) sub-tile as 32x32x16 MFMA tiles; B as (K,N) is
 // transposed on its way into LDS (a thread loads a 4(k) x 8(n) patch and writes eight 8-byte
-// k-runs).  The fast ones (K a multiple of 64, row-major C) feed LDS straight from global memory
+// k-runs).  The fast ones (K at least 64, no bound on K) feed LDS straight from global memory
 // and come in four tile sizes: 64 x 64, 128 x 128, 128 x 192 / 128 x 64 for the fused projections,
 // and 256 x 256; each is described where it stands.
 //
@@ -372,6 +372,14 @@ __device__ __forceinline__ bool live_tile(int bid, int tiles_m, int tiles_n, int
   return true;
 }
 
+// A K that is no whole number of stages: the FIRST stage is the short one.  Stage kt covers k from kt BK
+// - pad, so the loop and its wait counts are the same for every K, and only the loads of stage 0, before
+// the loop, ask where a lane's piece lies: those below k = 0 go to an offset past every buffer's
+// end, for which the load brings zeros into LDS, for A and B alike (0 x 0 adds nothing, whatever lies
+// before the row).  K a multiple of 8, at least BK.
+__host__ __device__ __forceinline__ int k_pad(int K) { return (BK - K % BK) % BK; }
+constexpr int NOWHERE = (int)0x80000000u;   // past stage_rows' 2^31 - 1 bytes, whatever scalar offset is added
+
 // 64 x 64 tiles, B as (N,K), for problems -- or row bounds -- whose 128 x 128 tiles would leave CUs
 // idle (k/v projections, short chunks): the direct-to-LDS pipeline of the 128 x 128 kernel below
 // (buffer loads, XOR-swizzled chunks) with a wave owning one 32x32x16 MFMA tile.  A stage is four
@@ -408,28 +416,30 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const int lrow = lane >> 3, pch = lane & 7;
-  int a_voff[INST], b_voff[INST];
+  int a_voff[INST], b_voff[INST], head_ch[INST];
 #pragma unroll
   for (int i = 0; i < INST; ++i) {
     const int r = (wave * INST + i) * 8 + lrow;
     const int lch = pch ^ ((r >> 1) & 7);
+    head_ch[i] = lch * 8;
     // Rows past the end re-read the last row; what they produce is never stored.
     a_voff[i] = (int)(((size_t)(min(m0 + r, M - 1) - m0) * K + lch * 8) * 2);
     b_voff[i] = (int)(((size_t)(min(n0 + r, N - 1) - n0) * K + lch * 8) * 2);
   }
-  const bf16_t* a_tile = A + (size_t)m0 * K;
-  const bf16_t* b_tile = B + (size_t)n0 * K;
+  const int pad = k_pad(K);
+  const bf16_t* a_tile = A + (size_t)m0 * K - pad;
+  const bf16_t* b_tile = B + (size_t)n0 * K - pad;
   // One load of the 2*INST a wave issues per stage (A's first, then B's).
-  auto issue_one = [&](char* st, int kt, int idx) {
+  auto issue_one = [&](char* st, int kt, int idx, bool head) {
     const int k0 = kt * BK;
     if (idx < INST) {
       const __amdgpu_buffer_rsrc_t rows = stage_rows(a_tile + k0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, IRON_LDS_PTR(st + (wave * INST + idx) * 1024), 16,
-                                               (int)a_voff[idx], 0, 0, 0);
+                                               head && head_ch[idx] < pad ? NOWHERE : a_voff[idx], 0, 0, 0);
     } else {
       const __amdgpu_buffer_rsrc_t rows = stage_rows(b_tile + k0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, IRON_LDS_PTR(st + NT_A_BYTES + (wave * INST + idx - INST) * 1024),
-                                               16, (int)b_voff[idx - INST], 0, 0, 0);
+                                               16, head && head_ch[idx - INST] < pad ? NOWHERE : b_voff[idx - INST], 0, 0, 0);
     }
   };
 
@@ -452,13 +462,13 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
       res[q] = *reinterpret_cast<const uint2*>(qkv.residual + (size_t)min(m, M - 1) * N + min(nb + 8 * q, N - 4));
   }
 
-  const int nk = K / BK;
+  const int nk = (K + pad) / BK;
   // Always STAGES-1 stages in flight before the loop (short K repeats its last stage), so the
   // loop's wait counts hold from the first iteration.
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s)
 #pragma unroll
-    for (int idx = 0; idx < LOADS; ++idx) issue_one(smem_nt + s * NT_STAGE_BYTES, min(s, nk - 1), idx);
+    for (int idx = 0; idx < LOADS; ++idx) issue_one(smem_nt + s * NT_STAGE_BYTES, min(s, nk - 1), idx, s == 0);
 
   const int ra = wm * 32 + fr, rb = wn * 32 + fr;
   const int a_off = ra * 128, a_swz = (ra >> 1) & 7, b_off = NT_A_BYTES + rb * 128, b_swz = (rb >> 1) & 7;
@@ -489,7 +499,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
       __builtin_amdgcn_sched_barrier(0);
       af[P ^ 1][ks] = a_frag(st1, ks);
       bfr[P ^ 1][ks] = b_frag(st1, ks);
-      issue_one(nst, kn, ks);
+      issue_one(nst, kn, ks, false);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -554,7 +564,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
 // through LDS so that it leaves as whole 128-byte row segments (16 bytes a lane).  QKV: the fused
 // projections' per-tile choice of weight and output, RoPE on the accumulators.  Otherwise `qkv`
 // carries the optional residual epilogue.
-template <bool QKV, bool B_KN = false>
+template <bool QKV, bool B_KN = false, bool C_NM = false>
 __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B_,
                                                bf16_t* __restrict__ C_, int M, int N_, int K,
                                                const int* __restrict__ valid, int tiles_m, int tiles_n,
@@ -565,6 +575,7 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
   constexpr int LOADS = 2 * INST;
   static_assert(BK == 64 && INST == 4, "two 32-wide k-steps a stage, eight loads a wave");
   static_assert(!(B_KN && QKV), "the fused projections read weights as stored, (N,K)");
+  static_assert(B_KN || !C_NM, "with B (N,K) the (N,M) output is the product of B and A");
   extern __shared__ __align__(16) char smem_nt[];
   const int Mv = bound_or(valid, M);
 
@@ -591,19 +602,22 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
       N = qkv.kv_n;
     }
   }
-  const int n0 = tn * NT_BN;
+  // (K,N): B's columns are read in whole tiles, so the last tile is moved back to end at N (what two
+  // tiles both cover comes out the same from both).
+  const int n0 = B_KN ? min(tn * NT_BN, N - NT_BN) : tn * NT_BN;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const int lrow = lane >> 3, pch = lane & 7;
   auto kn_swizzle = [](int k) { return ((k & 3) << 1) | (((k >> 3) & 1) << 3); };
-  int a_voff[INST], b_voff[INST];
+  int a_voff[INST], b_voff[INST], a_head[INST], b_head[INST];   // *_head: the k of a stage the lane's piece begins at
 #pragma unroll
   for (int i = 0; i < INST; ++i) {
     const int r = (wave * INST + i) * 8 + lrow;
     const int lch = pch ^ ((r >> 1) & 7);
     // Rows past the end re-read the last row; what they produce is never stored.
     a_voff[i] = (int)(((size_t)(min(m0 + r, M - 1) - m0) * K + lch * 8) * 2);
+    a_head[i] = b_head[i] = lch * 8;
     if constexpr (!B_KN) {
       b_voff[i] = (int)(((size_t)(min(n0 + r, N - 1) - n0) * K + lch * 8) * 2);
     } else {
@@ -611,21 +625,23 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
       // instruction), a row's 16 chunks XORed with kn_swizzle(row) for the transposing reads below.
       const int kr = (wave * INST + i) * 4 + (lane >> 4);
       b_voff[i] = (int)(((size_t)kr * N + ((lane & 15) ^ kn_swizzle(kr)) * 8) * 2);
+      b_head[i] = kr;
     }
   }
   const int k_first = QKV || B_KN ? 0 : qkv.k_begin;
-  const bf16_t* a_tile = A + (size_t)m0 * K + k_first;
-  const bf16_t* b_tile = B_KN ? B + n0 : B + (size_t)n0 * K + k_first;
-  auto issue_one = [&](char* st, int kt, int idx) {
+  const int pad = QKV ? 0 : k_pad(K);
+  const bf16_t* a_tile = A + (size_t)m0 * K + k_first - pad;
+  const bf16_t* b_tile = B_KN ? B + n0 - (size_t)pad * N : B + (size_t)n0 * K + k_first - pad;
+  auto issue_one = [&](char* st, int kt, int idx, bool head) {
     const int k0 = kt * BK;
     if (idx < INST) {
       const __amdgpu_buffer_rsrc_t rows = stage_rows(a_tile + k0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, IRON_LDS_PTR(st + (wave * INST + idx) * 1024), 16,
-                                               (int)a_voff[idx], 0, 0, 0);
+                                               head && a_head[idx] < pad ? NOWHERE : a_voff[idx], 0, 0, 0);
     } else {
       const __amdgpu_buffer_rsrc_t rows = stage_rows(b_tile + (B_KN ? (size_t)k0 * N : (size_t)k0));
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, IRON_LDS_PTR(st + NT_A_BYTES + (wave * INST + idx - INST) * 1024),
-                                               16, (int)b_voff[idx - INST], 0, 0, 0);
+                                               16, head && b_head[idx - INST] < pad ? NOWHERE : b_voff[idx - INST], 0, 0, 0);
     }
   };
 
@@ -654,11 +670,11 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
     }
   }
 
-  const int nk = (!QKV && !B_KN && qkv.k_len > 0 ? qkv.k_len : K) / BK;
+  const int nk = (!QKV && !B_KN && qkv.k_len > 0 ? qkv.k_len : K + pad) / BK;
 #pragma unroll
   for (int s = 0; s < NT_STAGES - 1; ++s)
 #pragma unroll
-    for (int idx = 0; idx < LOADS; ++idx) issue_one(smem_nt + s * NT_STAGE_BYTES, min(s, nk - 1), idx);
+    for (int idx = 0; idx < LOADS; ++idx) issue_one(smem_nt + s * NT_STAGE_BYTES, min(s, nk - 1), idx, s == 0);
 
   // Fragments: lane -> row fr of a 16-row tile, 16-byte chunk kq of the k-step's four.
   const int fr = lane & 15, kq = lane >> 4;
@@ -790,7 +806,9 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          mfma_16x16x32_in_place(acc[i][j], bfr[ks][j], af[ks][i]);
+          // (the operands' order decides whether a lane owns four columns of a row or four rows of a column)
+          if constexpr (C_NM) mfma_16x16x32_in_place(acc[i][j], af[ks][i], bfr[ks][j]);
+          else mfma_16x16x32_in_place(acc[i][j], bfr[ks][j], af[ks][i]);
           __builtin_amdgcn_sched_barrier(0);
           const int slot = i * 4 + j;
           if (slot < 4) {
@@ -807,7 +825,7 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
             } else {
               af[nks][slot - 4] = a_frag(from, nks, slot - 4);
             }
-          } else if (slot & 1) issue_one(nst, kn, ks * 4 + (slot - 9) / 2);
+          } else if (slot & 1) issue_one(nst, kn, ks * 4 + (slot - 9) / 2, false);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -872,13 +890,33 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      *reinterpret_cast<uint2*>(ot + (i * 16 + fr) * OROWB + (j * 16 + 4 * kq) * 2) =
+      *reinterpret_cast<uint2*>(ot + ((C_NM ? j : i) * 16 + fr) * OROWB + ((C_NM ? i : j) * 16 + 4 * kq) * 2) =
           make_uint2(pack_bf16(acc[i][j][0], acc[i][j][1]), pack_bf16(acc[i][j][2], acc[i][j][3]));
   // The tile is private to the wave, whose LDS operations execute in order: no block barrier,
   // only a fence to keep the compiler from moving the reads above other lanes' writes.
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if constexpr (C_NM) {   // the tile's rows are C's columns n, 8 consecutive m of each a lane
+    const int out_m = m0 + wm * 64 + out_col;
+    const bool whole_m = (M & 7) == 0 && out_m + 8 <= M;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int row = r * 8 + out_row;
+      const uint4 v = *reinterpret_cast<const uint4*>(ot + row * OROWB + out_col * 2);
+      if (out_m >= M) continue;
+      bf16_t* p = C + (size_t)(n0 + wn * 64 + row) * M + out_m;
+      if (whole_m) {
+        *reinterpret_cast<uint4*>(p) = v;
+      } else {
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (out_m + e < M) p[e] = (bf16_t)((e & 1) ? (w[e >> 1] >> 16) : (w[e >> 1] & 0xffffu));
+      }
+    }
+    return;
+  }
   const bool whole = (N & 7) == 0 && out_n + 8 <= N;
 #pragma unroll
   for (int r = 0; r < 8; ++r) {
@@ -915,7 +953,7 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
 }
 
 
-template <bool B_KN, bool QKV, int T, int STAGES64 = 4>
+template <bool B_KN, bool QKV, int T, int STAGES64 = 4, bool C_NM = false>
 __global__ __launch_bounds__(256) void gemm_nt_kernel(const bf16_t* __restrict__ A,
                                                       const bf16_t* __restrict__ B,
                                                       bf16_t* __restrict__ C, int M, int N, int K,
@@ -924,12 +962,12 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(const bf16_t* __restrict__
   if constexpr (QKV) to_cache_rows(qkv, valid, M);
   static_assert(T == 2 || (T == 1 && !B_KN && !QKV), "64x64 tiles: B (N,K), plain or residual output");
   if constexpr (T == 2)
-    gemm_nt16_body<QKV, B_KN>(A, B, C, M, N, K, valid, tiles_m, tiles_n, patched, qkv);
+    gemm_nt16_body<QKV, B_KN, C_NM>(A, B, C, M, N, K, valid, tiles_m, tiles_n, patched, qkv);
   else
     gemm_nt64_body<STAGES64>(A, B, C, M, N, K, valid, tiles_m, tiles_n, patched, qkv);
 }
 
-template <bool B_KN, bool QKV = false, int T = 2, int STAGES64 = 4>
+template <bool B_KN, bool QKV = false, int T = 2, int STAGES64 = 4, bool C_NM = false>
 static int launch_gemm_nt(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K,
                           const int* valid, hipStream_t s, QkvTail qkv = QkvTail{}) {
   constexpr int BM = 64 * T, BN = 64 * T;
@@ -942,12 +980,12 @@ static int launch_gemm_nt(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, in
   }
   const size_t lds = (size_t)(T == 1 ? STAGES64 : NT_STAGES) * (BM + BN) * BK * 2;
   static LdsOptIn opt_in;
-  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_nt_kernel<B_KN, QKV, T, STAGES64>), lds); e != hipSuccess) {
+  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_nt_kernel<B_KN, QKV, T, STAGES64, C_NM>), lds); e != hipSuccess) {
     set_error("gemm: %s", hipGetErrorString(e));
     return (int)e;
   }
   const int patched = (tiles_m % 8 == 0 && tiles_n % 4 == 0 && ((tiles_m / 8) * (tiles_n / 4)) % 8 == 0) ? 1 : 0;
-  hipLaunchKernelGGL((gemm_nt_kernel<B_KN, QKV, T, STAGES64>), dim3(tiles_m * tiles_n), dim3(256), lds, s, A, B, C, M, N, K,
+  hipLaunchKernelGGL((gemm_nt_kernel<B_KN, QKV, T, STAGES64, C_NM>), dim3(tiles_m * tiles_n), dim3(256), lds, s, A, B, C, M, N, K,
                      valid, tiles_m, tiles_n, patched, qkv);
   IRON_LAUNCH_CHECK();
 }
@@ -1342,8 +1380,10 @@ __device__ __forceinline__ void gemm_nt256_body(const bf16_t* __restrict__ A, co
 
   int tm, tn;
   if (!live_tile(blockIdx.x, tiles_m, tiles_n, patched, (Mv + BIG_BM - 1) / BIG_BM, tm, tn)) return;
-  const int m0 = tm * BIG_BM, n0 = tn * BIG_BN;
-  if (m0 >= Mv) return;
+  if (tm * BIG_BM >= Mv) return;
+  // The last tile of each direction is moved back to end at the matrix's edge, so that every tile is
+  // whole; what two tiles both cover comes out the same from both.
+  const int m0 = min(tm * BIG_BM, M - BIG_BM), n0 = min(tn * BIG_BN, N - BIG_BN);
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // uniform: LDS and global bases stay in scalar registers
   const int wm = wave / (WAVES / 2), wn = wave % (WAVES / 2);
@@ -1351,21 +1391,24 @@ __device__ __forceinline__ void gemm_nt256_body(const bf16_t* __restrict__ A, co
   // chunk); the logical chunk it fetches is the physical one swizzled by the row.
   const int lrow = lane / CPR, pch = lane % CPR;
   unsigned ld_off[2];   // byte offset of this lane's 16 bytes within an even / odd instruction's rows
+  int ld_head[2];       // ... and the k of a stage at which they begin
 #pragma unroll
   for (int par = 0; par < 2; ++par) {
     const int r = par * RPI + lrow;
+    ld_head[par] = (pch ^ ((r >> 1) & (CPR - 1))) * 8;
     ld_off[par] = (unsigned)(((size_t)lrow * K + (pch ^ ((r >> 1) & (CPR - 1))) * 8) * 2);
   }
   // Loads go out as buffer loads straight into LDS: the rows a wave fetches are one buffer, the
   // lane's place within an instruction's rows is the (constant) vector offset and the instruction's
   // rows and the stage's k are the scalar offset, so a load costs two scalar adds and no vector ALU
   // work between two MFMAs.
-  const __amdgpu_buffer_rsrc_t a_rows = stage_rows(A + (size_t)(m0 + wave * INST * RPI) * K);
+  const int pad = k_pad(K);
+  const __amdgpu_buffer_rsrc_t a_rows = stage_rows(A + (size_t)(m0 + wave * INST * RPI) * K - pad);
   // B as (K,N) lands as stored: the stage's 64 k-rows of 256 columns (512 bytes a row, two rows an
   // instruction), a row's 32 chunks XORed with kn_swizzle(row) so that the transposing reads below
   // find the four rows of a 16-lane group, and the groups of a pass, in different banks.
   const __amdgpu_buffer_rsrc_t b_rows =
-      stage_rows(B_KN ? B + n0 + (size_t)(wave * INST * 2) * N : B + (size_t)(n0 + wave * INST * RPI) * K);
+      stage_rows(B_KN ? B + n0 + ((ptrdiff_t)(wave * INST * 2) - pad) * N : B + (size_t)(n0 + wave * INST * RPI) * K - pad);
   auto kn_swizzle = [](int k) { return ((k & 3) << 1) | (((k >> 3) & 3) << 3); };
   int kn_off[INST];   // (K,N): this lane's 16 bytes within instruction idx's two rows
 #pragma unroll
@@ -1374,17 +1417,20 @@ __device__ __forceinline__ void gemm_nt256_body(const bf16_t* __restrict__ A, co
     kn_off[idx] = (int)(((size_t)(lane >> 5) * N + ((lane & 31) ^ kn_swizzle(kr)) * 8) * 2);
   }
   const int inst_stride = RPI * K * 2;
-  auto issue_one = [&](char* st, int kt, int idx) {
+  auto issue_one = [&](char* st, int kt, int idx, bool head) {
     const int k_off = kt * KB * 2;
     if (idx < INST)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rows, IRON_LDS_PTR(st + (wave * INST + idx) * 1024), 16,
-                                               (int)ld_off[idx & 1], idx * inst_stride + k_off, 0, 0);
+                                               head && ld_head[idx & 1] < pad ? NOWHERE : (int)ld_off[idx & 1],
+                                               idx * inst_stride + k_off, 0, 0);
     else if constexpr (!B_KN)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rows, IRON_LDS_PTR(st + A_BYTES + (wave * INST + idx - INST) * 1024),
-                                               16, (int)ld_off[idx & 1], (idx - INST) * inst_stride + k_off, 0, 0);
+                                               16, head && ld_head[idx & 1] < pad ? NOWHERE : (int)ld_off[idx & 1],
+                                               (idx - INST) * inst_stride + k_off, 0, 0);
     else
       __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rows, IRON_LDS_PTR(st + A_BYTES + (wave * INST + idx - INST) * 1024),
-                                               16, (int)kn_off[idx - INST], ((idx - INST) * 2 + kt * KB) * N * 2, 0, 0);
+                                               16, head && (wave * INST + idx - INST) * 2 + (lane >> 5) < pad ? NOWHERE : kn_off[idx - INST],
+                                               ((idx - INST) * 2 + kt * KB) * N * 2, 0, 0);
   };
 
   // The product runs on 16x16x32 MFMAs (a k-step is 32 wide, two a stage): on random operands the
@@ -1399,14 +1445,14 @@ __device__ __forceinline__ void gemm_nt256_body(const bf16_t* __restrict__ A, co
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.f;
 
-  const int nk = K / KB;
+  const int nk = (K + pad) / KB;
   static_assert(KB == 64 && (WAVES == 4 || WAVES == 8), "the loop below is written for two 64-wide stages and four or eight waves");
   // A stage's 2 INST loads go out in two halves of INST: the first under the last quarter of the
   // stage two before it (right after that stage's barrier freed the buffer), the second under the
   // first quarter of the stage before it; two quarters later, at that stage's barrier, all have landed.
-  auto issue_half = [&](char* st, int kt, int half, int slot) { issue_one(st, kt, half * INST + slot); };
+  auto issue_half = [&](char* st, int kt, int half, int slot) { issue_one(st, kt, half * INST + slot, false); };
 #pragma unroll
-  for (int idx = 0; idx < 2 * INST; ++idx) issue_one(smem_big, 0, idx);
+  for (int idx = 0; idx < 2 * INST; ++idx) issue_one(smem_big, 0, idx, true);
 #pragma unroll
   for (int slot = 0; slot < INST; ++slot) issue_half(smem_big + STAGE_BYTES, min(1, nk - 1), 0, slot);
 
@@ -2120,7 +2166,7 @@ int launch_grouped(const bf16_t* A, const bf16_t* B, bf16_t* C, int N, int K, co
 template <bool B_KN, bool STREAM_OUT>
 static int launch_gemm_nt256_as(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K,
                                 const int* valid, hipStream_t s) {
-  const int tiles_m = M / BIG_BM, tiles_n = N / BIG_BN;
+  const int tiles_m = (M + BIG_BM - 1) / BIG_BM, tiles_n = (N + BIG_BN - 1) / BIG_BN;
   constexpr size_t out_bytes = (size_t)BIG_WAVES * 128 * BIG_OUT_ROW_BYTES(8 / BIG_WAVES * 2);
   const size_t lds = out_bytes > (size_t)2 * BIG_STAGE_BYTES ? out_bytes : (size_t)2 * BIG_STAGE_BYTES;
   static LdsOptIn opt_in;
@@ -2160,13 +2206,37 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
   IRON_REQUIRE(b_col_maj || N % 8 == 0,
                "gemm: N (%d) must be a multiple of 8 when B is (K,N) (16-byte loads along N)", N);
   hipStream_t s = (hipStream_t)stream;
+  // The (N,M) output of A and B (N,K) is the (M,N) output of B and A: both are rows of K (2048^3 41.5 ->
+  // 19.4 us against the general kernel's strided stores).
+  if (b_col_maj && c_col_maj && valid == nullptr && valid_k == nullptr && M <= (1 << 22)) {
+    const uint16_t* rows = A;
+    A = B, B = rows;
+    const int m = M;
+    M = N, N = m;
+    c_col_maj = 0;
+  }
   // Fewer rows than the smallest tile: bound by streaming B.
   if (M < 64 && b_col_maj && !c_col_maj && valid == nullptr && valid_k == nullptr)
     return iron_gemm_few_bf16(A, B, nullptr, C, M, N, K, 0, stream);
-  if (!c_col_maj && valid_k == nullptr && K % BK == 0 && M >= 64 && N >= 64) {
-    // Enough whole 256x256 tiles to fill the chip: the large-tile kernel (offsets are 32-bit).
-    if (b_col_maj && M % BIG_BM == 0 && N % BIG_BN == 0 && (long)(M / BIG_BM) * (N / BIG_BN) >= 192 &&
-        K <= (1 << 24)) {
+  // The direct-to-LDS kernels take any K from one stage on (k_pad), any M, and any N of B (N,K); against
+  // the general kernel below, which loads through registers: 2048 x 2048 x 2056 42.5 -> 26.0 us, 86 x 1728 x
+  // 5560 59 -> 26.5, (K,N) 2048 x 2048 x 2040 65 -> 22.0, 300 x 1000 x 1000 33.6 -> 9.8.  (A K that is no
+  // multiple of 64 stays dearer than its neighbour that is, 26.0 us against 19.4: its rows' 128-byte
+  // pieces straddle two cache lines.)  (K,N) wants a whole tile of columns.
+  if (valid_k == nullptr && K >= BK && (b_col_maj ? !c_col_maj : M >= 64 && N >= 128 && (!c_col_maj || valid == nullptr))) {
+    if (c_col_maj) return launch_gemm_nt<true, false, 2, 4, true>(A, B, C, M, N, K, valid, s);
+    const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
+    // Enough 256x256 tiles to fill the chip: the large-tile kernel (offsets are 32-bit).  A round of
+    // them takes as long as about 3.2 rounds of 128x128 ones (4000 x 4096 x 4096: 256 tiles 129 us, 1024 smaller
+    // ones 158; 777 x 10240 x 2560: 160 tiles 69 us, 560 smaller ones 61), so 192 it is, and edges
+    // that waste more than a fifth of the large tiles stay with the smaller; where rows straddle cache
+    // lines the large tile, which reads half as much, gains more (1500 x 6000 x 3000: 144 tiles 93 us
+    // against 110).
+    const long tiles256 = (long)((M + BIG_BM - 1) / BIG_BM) * ((N + BIG_BN - 1) / BIG_BN);
+    const bool whole = M % BIG_BM == 0 && N % BIG_BN == 0;
+    const bool big = M >= BIG_BM && N >= BIG_BN && N % 8 == 0 && tiles256 >= (K % BK == 0 ? 192 : 144) &&
+                     5 * tiles128 >= 16 * tiles256;
+    if (b_col_maj && big && (valid == nullptr || whole)) {
       // Under a row bound read on the device the large tiles may cover too few rows to fill the
       // chip (512 valid rows of 2048 leave 64 of 256 tiles): the blocks of one launch then choose
       // the tile size where the bound is known, on the device.
@@ -2180,20 +2250,18 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
       // 128x128 tiles that would occupy under half the CUs give way to 64x64 ones: always, where
       // the shape says so; under a row bound, the blocks of one launch choose where the bound is
       // known (the few-row 64x64 tiles run the eight-stage pipeline, a block a CU, so nothing is
-      // lost to the launch's 128 KB of LDS and the second, empty launch is saved).
+      // lost to the launch's 128 KB of LDS and the second, empty launch is saved).  So do tiles that
+      // up to 64 rows would half fill at most (64 x 16384 x 8184: 93 -> 68 us).
       const int tiles_n128 = (N + 127) / 128;
-      const long tiles128 = (long)((M + 127) / 128) * tiles_n128;
-      if (tiles128 < 128) return launch_gemm_nt<false, false, 1>(A, B, C, M, N, K, valid, s);
+      if (tiles128 < 128 || M <= 64) return launch_gemm_nt<false, false, 1>(A, B, C, M, N, K, valid, s);
       const int few = tiles_n128 >= 128 ? 0 : 128 * (127 / tiles_n128);   // rows up to which 64x64 tiles win
       if (valid == nullptr || few == 0 || few >= M) return launch_gemm_nt<false>(A, B, C, M, N, K, valid, s);
       return launch_gemm_either<false>(A, B, C, M, N, K, valid, s, 0, few);
     }
-    // (K,N) B is read in whole tiles straight into LDS: N must be whole tiles.  Enough whole
-    // 256x256 tiles to fill the chip, and a matrix a 32-bit byte offset spans: the large-tile kernel.
-    if (valid == nullptr && M % BIG_BM == 0 && N % BIG_BN == 0 && (long)(M / BIG_BM) * (N / BIG_BN) >= 192 &&
-        (long)K * N * 2 < (1L << 31))
+    // (K,N): the same line, for a matrix a 32-bit byte offset spans.
+    if (valid == nullptr && big && (long)(K + BK) * N * 2 < (1L << 31))
       return launch_gemm_nt256<true>(A, B, C, M, N, K, valid, s);
-    if (N % 128 == 0) return launch_gemm_nt<true>(A, B, C, M, N, K, valid, s);
+    return launch_gemm_nt<true>(A, B, C, M, N, K, valid, s);
   }
   // 128x128 tiles fill the 256 CUs once at 2048x2048; narrower problems take 64-wide tiles.
   const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);

@@ -100,6 +100,33 @@ def test_gemm_layouts(cuda, b_col_maj, c_col_maj):
     assert np.all(np.abs(from_torch(C) - want) <= bound)
 
 
+@pytest.mark.parametrize("b_col_maj", [False, True])
+@pytest.mark.parametrize("c_col_maj", [False, True])
+@pytest.mark.parametrize("M,Kdim,N", [
+    (64, 64, 128), (65, 72, 136), (40, 120, 200), (129, 136, 248), (191, 1000, 264), (333, 72, 1000),   # 64 and 128 tiles
+    (2049, 200, 1160), (3500, 72, 3400), (3584, 248, 3584), (3329, 128, 3592), (16384, 72, 40),          # ... and 256 ones
+])
+def test_gemm_at_the_edges_of_tiles_and_stages(cuda, M, Kdim, N, b_col_maj, c_col_maj):
+    """A K that ends inside a stage (one piece over it, one piece short, alone in its second stage), edges
+    that move the last tile back, one row or column group more than a tile, in every layout.  The
+    operands lie between NaNs: a piece read from outside them would show in the sums."""
+    rng = np.random.default_rng(M + N + Kdim)
+    A, B = bf(rng, M, Kdim), bf(rng, (N if b_col_maj else Kdim), (Kdim if b_col_maj else N), scale=0.05)
+
+    def between_nans(x):
+        room = 64 * max(x.shape)
+        buf = torch.full((x.size + 2 * room,), float("nan"), dtype=torch.bfloat16, device=cuda)
+        inside = buf[room:room + x.size].view(*x.shape)
+        inside.copy_(dev(x, cuda))
+        return inside
+
+    C = out_like((N, M) if c_col_maj else (M, N), cuda, fill=float("nan"))
+    K.gemm(between_nans(A), between_nans(B), C, M=M, N=N, K=Kdim, b_col_maj=b_col_maj, c_col_maj=c_col_maj)
+    want = ops.gemm(A, B, b_col_maj=b_col_maj, c_col_maj=c_col_maj)
+    # The bound the layouts are held to above: 2 units of 2^-8 |A|@|B|.
+    assert np.all(np.abs(from_torch(C) - want) <= ops.gemm_bound(A, B, b_col_maj=b_col_maj, c_col_maj=c_col_maj))
+
+
 @pytest.mark.parametrize("b_col_maj", [True, False])
 @pytest.mark.parametrize("n", [4096, 8192])
 def test_gemm_large_squares_on_sampled_rows(cuda, n, b_col_maj):
