@@ -372,6 +372,27 @@ __device__ __forceinline__ bool live_tile(int bid, int tiles_m, int tiles_n, int
   return true;
 }
 
+// The epilogue over a piece of a row: x, the product as it would be stored, and r, the second operand's piece, become
+// scale * x + r, or bf16(act(r)) * x.  The kind is asked once a piece: asked an element, every branch was
+// a wait (gated product 2048 x 2048 x 2048 27.9 -> 22.7 us, residual sum 23.0 -> 21.8).
+template <int COUNT>
+__device__ __forceinline__ void tail_of(const QkvTail& qkv, float (&x)[COUNT], const float (&r)[COUNT]) {
+  auto gate = [&](auto kind) {
+#pragma unroll
+    for (int e = 0; e < COUNT; ++e) x[e] = round_bf16(gate_of(decltype(kind)::value, r[e])) * x[e];
+  };
+  if (qkv.gated == 0) {
+#pragma unroll
+    for (int e = 0; e < COUNT; ++e) x[e] = fmaf(qkv.residual_scale, x[e], r[e]);
+  } else if (qkv.gated == 1) {
+    gate(std::integral_constant<int, 1>{});
+  } else if (qkv.gated == 2) {
+    gate(std::integral_constant<int, 2>{});
+  } else {
+    gate(std::integral_constant<int, 3>{});
+  }
+}
+
 // A K that is no whole number of stages: the FIRST stage is the short one.  Stage kt covers k from kt BK
 // - pad, so the loop and its wait counts are the same for every K, and only the loads of stage 0, before
 // the loop, ask where a lane's piece lies: those below k = 0 go to an offset past every buffer's
@@ -533,11 +554,12 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
         for (int e = 0; e < 4; ++e)
           if (n + e < N) rf[e] = bf16_to_f32(r[e]);
       }
+      float prod[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float prod = round_bf16(acc[0][4 * q + e]);
-        acc[0][4 * q + e] = qkv.gated ? round_bf16(gate_of(qkv.gated, rf[e])) * prod : fmaf(qkv.residual_scale, prod, rf[e]);
-      }
+      for (int e = 0; e < 4; ++e) prod[e] = round_bf16(acc[0][4 * q + e]);
+      tail_of(qkv, prod, rf);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[0][4 * q + e] = prod[e];
     }
     if (vec && n + 4 <= N) {
       *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16(acc[0][4 * q], acc[0][4 * q + 1]),
@@ -935,9 +957,7 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
           for (int e = 0; e < 8; ++e)   // (constant indices: a runtime trip count puts the array in scratch memory)
             if (out_n + e < N) rf[e] = bf16_to_f32(qkv.residual[(size_t)m * N + out_n + e]);
         }
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          x[e] = qkv.gated ? round_bf16(gate_of(qkv.gated, rf[e])) * x[e] : fmaf(qkv.residual_scale, x[e], rf[e]);
+        tail_of(qkv, x, rf);
         v = pack8(x);
       }
     }
@@ -1362,11 +1382,18 @@ constexpr int BIG_KB = IRON_BIG_KB;   // k per stage: 64 (2 stages); 32 (4 stage
 #define BIG_OUT_ROW_BYTES(TN) ((TN) * 64 + 16)
 constexpr int BIG_STAGE_BYTES = (BIG_BM + BIG_BN) * BK * 2;
 
-template <int WAVES, int KB, bool B_KN = false, bool STREAM_OUT = false>
+// The operands of a gated feed-forward's two first projections beyond the gate's own.
+struct GatedPair {
+  const bf16_t* up;      // the up projection's weights, (N,K) as the gate's
+  bf16_t* gate_out;      // where the gate's product goes
+  int activation;
+};
+
+template <int WAVES, int KB, bool B_KN = false, bool STREAM_OUT = false, bool PAIR = false>
 __device__ __forceinline__ void gemm_nt256_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
                                                 bf16_t* __restrict__ C, int M, int N, int K,
                                                 const int* __restrict__ valid, int tiles_m, int tiles_n,
-                                                int patched) {
+                                                int patched, const GatedPair& pair = GatedPair{}) {
   static_assert(KB == 64, "k per stage: 64 (32 with four stages of half-line rows measured 13 % slower)");
   constexpr int ROWB = KB * 2;               // bytes of a tile row in LDS
   constexpr int CPR = KB / 8;                // its 16-byte chunks
@@ -1383,7 +1410,7 @@ __device__ __forceinline__ void gemm_nt256_body(const bf16_t* __restrict__ A, co
   if (tm * BIG_BM >= Mv) return;
   // The last tile of each direction is moved back to end at the matrix's edge, so that every tile is
   // whole; what two tiles both cover comes out the same from both.
-  const int m0 = min(tm * BIG_BM, M - BIG_BM), n0 = min(tn * BIG_BN, N - BIG_BN);
+  const int m0 = min(tm * BIG_BM, M - BIG_BM), n0 = PAIR ? tn * (BIG_BN / 2) : min(tn * BIG_BN, N - BIG_BN);
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // uniform: LDS and global bases stay in scalar registers
   const int wm = wave / (WAVES / 2), wn = wave % (WAVES / 2);
@@ -1408,6 +1435,7 @@ __device__ __forceinline__ void gemm_nt256_body(const bf16_t* __restrict__ A, co
   // instruction), a row's 32 chunks XORed with kn_swizzle(row) so that the transposing reads below
   // find the four rows of a 16-lane group, and the groups of a pass, in different banks.
   const __amdgpu_buffer_rsrc_t b_rows =
+      PAIR ? stage_rows(((wave & 1) ? pair.up : B) + (size_t)(n0 + (wave >> 1) * INST * RPI) * K - pad) :
       stage_rows(B_KN ? B + n0 + ((ptrdiff_t)(wave * INST * 2) - pad) * N : B + (size_t)(n0 + wave * INST * RPI) * K - pad);
   auto kn_swizzle = [](int k) { return ((k & 3) << 1) | (((k >> 3) & 3) << 3); };
   int kn_off[INST];   // (K,N): this lane's 16 bytes within instruction idx's two rows
@@ -1611,6 +1639,60 @@ __device__ __forceinline__ void gemm_nt256_body(const bf16_t* __restrict__ A, co
   wait_vmcnt<0>();   // the last iteration's idle fetch must land before LDS is reused
   block_barrier();   // every wave is done reading the stages
 
+  if constexpr (PAIR) {
+    // Columns 0 .. NT / 2 - 1 of the wave's tiles are the gate's product, the rest the up projection's, of
+    // the same 8 NT columns of the output: the gate's product leaves as it is stored, then, made in the
+    // accumulators' own layout, bf16(bf16(act(bf16 g)) * bf16 u).
+    constexpr int HT = NT / 2, OROWB = HT * 32 + 16, LPRW = HT * 2, ORPI = 64 / LPRW;
+    char* ot = smem_big + wave * (128 * OROWB);
+    const int lr = lane / LPRW, lc = lane % LPRW;
+    const size_t first = (size_t)(m0 + wm * 128) * N + n0 + wn * HT * 16 + lc * 8;
+    auto leave = [&](bf16_t* to) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll 4
+      for (int r0 = 0; r0 < 128; r0 += ORPI) {
+        const int r = r0 + lr;
+        const uint4 v = *reinterpret_cast<const uint4*>(ot + r * OROWB + lc * 16);
+        if (m0 + wm * 128 + r < Mv) *reinterpret_cast<uint4*>(to + first + (size_t)r * N) = v;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();   // the rows are read before the next product overwrites them
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    // (The kind of gate is chosen once: asked an element, its branches made the lone wave of a SIMD wait 128 times over, and a
+    // 2048 x 8192 x 2048 pair take 143 us instead of 130.)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < HT; ++j)
+        *reinterpret_cast<uint2*>(ot + (i * 16 + fr) * OROWB + (j * 16 + 4 * kq) * 2) =
+            make_uint2(pack_bf16(acc[i][j][0], acc[i][j][1]), pack_bf16(acc[i][j][2], acc[i][j][3]));
+    leave(pair.gate_out);
+    auto gated = [&](auto kind) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      // A tile row at a time leaves the accumulation registers: all at once they would not fit.
+#pragma unroll
+      for (int j = 0; j < NT; ++j) asm volatile("" : "+a"(acc[i][j]));
+#pragma unroll
+      for (int j = 0; j < HT; ++j) {
+        float c[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          c[e] = round_bf16(gate_of(decltype(kind)::value, round_bf16(acc[i][j][e]))) * round_bf16(acc[i][j + HT][e]);
+        *reinterpret_cast<uint2*>(ot + (i * 16 + fr) * OROWB + (j * 16 + 4 * kq) * 2) =
+            make_uint2(pack_bf16(c[0], c[1]), pack_bf16(c[2], c[3]));
+      }
+    }
+    };
+    if (pair.activation == 1) gated(std::integral_constant<int, 1>{});
+    else if (pair.activation == 2) gated(std::integral_constant<int, 2>{});
+    else gated(std::integral_constant<int, 3>{});
+    leave(C);
+    return;
+  }
   // Output through LDS: a wave lays its 128 x (16 NT) tile out row-major (rows padded by 16 bytes,
   // which spreads both the 8-byte writes below and the 16-byte reads over all banks) and stores
   // whole 16-byte pieces, so a row of the tile leaves as one contiguous segment.
@@ -2041,37 +2123,50 @@ __device__ __forceinline__ void gemm_nt16_pair_body(const bf16_t* __restrict__ A
             make_uint2(pack_bf16(accg[i][j][0], accg[i][j][1]), pack_bf16(accg[i][j][2], accg[i][j][3]));
     leave(G);
   }
+  auto gated = [&](auto kind) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float c[4];
+      for (int j = 0; j < 4; ++j) {
+        float c[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        c[e] = round_bf16(gate_of(activation, round_bf16(accg[i][j][e]))) * round_bf16(accu[i][j][e]);
-      *reinterpret_cast<uint2*>(ot + (i * 16 + fr) * OROWB + (j * 16 + 4 * kq) * 2) =
-          make_uint2(pack_bf16(c[0], c[1]), pack_bf16(c[2], c[3]));
-    }
+        for (int e = 0; e < 4; ++e)
+          c[e] = round_bf16(gate_of(decltype(kind)::value, round_bf16(accg[i][j][e]))) * round_bf16(accu[i][j][e]);
+        *reinterpret_cast<uint2*>(ot + (i * 16 + fr) * OROWB + (j * 16 + 4 * kq) * 2) =
+            make_uint2(pack_bf16(c[0], c[1]), pack_bf16(c[2], c[3]));
+      }
+  };
+  // The kind of gate is chosen once: asked an element, its branches kept the matrix results of one wave a
+  // SIMD waiting for each other.
+  if (activation == 1) gated(std::integral_constant<int, 1>{});
+  else if (activation == 2) gated(std::integral_constant<int, 2>{});
+  else gated(std::integral_constant<int, 3>{});
   leave(C);
 }
 
-// A gated feed-forward's two first projections over many rows as ONE launch: a block computes its
-// tile of the gate's product and stores it (rounded, as the separate product stores it), then
-// computes the same tile of the second product, whose epilogue reads the gate tile back -- the one
-// this very block wrote, so nothing crosses between blocks -- and leaves bf16(bf16(act(g)) * bf16(u)).
-// What goes is a launch boundary: the second launch's start, its first stages' fill and the first
-// one's drain.  The tile size is chosen on the device by the row bound as in gemm_either_kernel.
+// A gated feed-forward's two first projections over many rows as ONE launch, the tile chosen on the
+// device by the row bound as in gemm_either_kernel.  Few rows: 64 x 64 tiles, a block's gate tile first,
+// then the same tile of the second product, whose epilogue reads the gate tile back -- the one this
+// very block wrote, so nothing crosses between blocks.  Up to one round of them, 128 x 128 tiles of
+// both products at once.  Past that 256 rows x (128 + 128) columns, a wave's 128 x 128 half gate and half up
+// projection: the bytes a CU draws from L2 per flop are those of a 256 x 256 tile, two thirds of the smaller pair's.
+// A round of the large tiles takes 1.5 rounds of the small ones and covers two (N = 8192, K = 2048: 2048
+// rows 161 -> 130 us, 1024 89 -> 65, 1281 118 -> 113; 512 rows, on the small tiles, 46.5 -> 41.8 by asking the kind of gate once).
 __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __restrict__ A,
                                                               const bf16_t* __restrict__ Bg,
                                                               const bf16_t* __restrict__ Bu, bf16_t* __restrict__ G,
                                                               bf16_t* __restrict__ C, int M, int N, int K,
-                                                              const int* __restrict__ valid, Tiling t128, Tiling t64,
-                                                              int few128, int activation) {
+                                                              const int* __restrict__ valid, Tiling t256, Tiling t128,
+                                                              Tiling t64, int few256, int few128, int activation) {
   const int Mv = bound_or(valid, M), bid = blockIdx.x;
   QkvTail none{}, gate{};
   gate.residual = G;
   gate.gated = activation;
-  if (Mv > few128) {
+  if (Mv > few256) {
+    if (bid >= t256.tiles_m * t256.tiles_n) return;
+    gemm_nt256_body<4, BIG_KB, false, false, true>(A, Bg, C, M, N, K, valid, t256.tiles_m, t256.tiles_n, t256.patched,
+                                                   GatedPair{Bu, G, activation});
+  } else if (Mv > few128) {
     if (bid >= t128.tiles_m * t128.tiles_n) return;
     gemm_nt16_pair_body(A, Bg, Bu, G, C, M, N, K, valid, t128.tiles_m, t128.tiles_n, t128.patched, activation);
   } else {
@@ -2085,15 +2180,19 @@ __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __re
 static int launch_gemm_gated_pair(const bf16_t* A, const bf16_t* Bg, const bf16_t* Bu, bf16_t* G, bf16_t* C, int M,
                                   int N, int K, const int* valid, int activation, hipStream_t s) {
   const int n128 = (N + 127) / 128, n64 = (N + 63) / 64;
-  // 64 x 64 tiles up to the rows below which 128 x 128 ones would leave half the CUs idle (as iron_gemm_bf16).
+  // 64 x 64 tiles up to the rows below which 128 x 128 ones would leave half the CUs idle (as iron_gemm_bf16),
+  // 256 x (128 + 128) ones past the rows that one round of 128 x 128 ones covers.
   int few128 = n128 >= 128 ? 0 : 128 * (127 / n128);
   if (few128 > M) few128 = M;
+  int few256 = n128 >= 256 ? 0 : 128 * (256 / n128);
+  if (few256 > M || M < BIG_BM || N % 128 != 0) few256 = M;
   auto tiling = [](int tile_rows, int tile_cols) {
     const int whole = (tile_rows + 7) & ~7;
     if (tile_rows >= 8 && !patched_order(tile_rows, tile_cols) && patched_order(whole, tile_cols)) tile_rows = whole;
     return Tiling{tile_rows, tile_cols, patched_order(tile_rows, tile_cols)};
   };
-  const Tiling t128 = tiling((M + 127) / 128, n128), t64 = tiling((few128 + 63) / 64, n64);
+  const Tiling t256 = few256 < M ? tiling((M + BIG_BM - 1) / BIG_BM, n128) : Tiling{0, 0, 0};
+  const Tiling t128 = tiling((few256 + 127) / 128, n128), t64 = tiling((few128 + 63) / 64, n64);
   constexpr size_t lds = (size_t)PAIR_STAGES * 3 * 128 * BK * 2;   // the two-product body's stages, more than the others'
   static_assert(lds >= (size_t)NT_STAGES * 256 * BK * 2, "the 64 x 64 body's stages fit too");
   static LdsOptIn opt_in;
@@ -2102,9 +2201,10 @@ static int launch_gemm_gated_pair(const bf16_t* A, const bf16_t* Bg, const bf16_
     return (int)e;
   }
   int blocks = t128.tiles_m * t128.tiles_n;
+  if (t256.tiles_m * t256.tiles_n > blocks) blocks = t256.tiles_m * t256.tiles_n;
   if (t64.tiles_m * t64.tiles_n > blocks) blocks = t64.tiles_m * t64.tiles_n;
-  hipLaunchKernelGGL(gemm_gated_pair_kernel, dim3(blocks), dim3(256), lds, s, A, Bg, Bu, G, C, M, N, K, valid, t128, t64,
-                     few128, activation);
+  hipLaunchKernelGGL(gemm_gated_pair_kernel, dim3(blocks), dim3(256), lds, s, A, Bg, Bu, G, C, M, N, K, valid, t256, t128, t64,
+                     few256, few128, activation);
   IRON_LAUNCH_CHECK();
 }
 

@@ -462,12 +462,15 @@ def test_gemm_gated_epilogue(cuda, M, Kdim, N, rows, activation):
 
 
 @pytest.mark.parametrize("M,Kdim,N,rows", [(2048, 2048, 8192, 512), (2048, 2048, 8192, 1281), (2048, 2048, 8192, 100),
-                                           (256, 512, 1024, None), (192, 128, 320, 70)])
+                                           (256, 512, 1024, None), (192, 128, 320, 70),
+                                           # 256-row tiles: one stage, two, the last tile moved back, a bound inside it
+                                           (2048, 64, 4096, None), (1300, 128, 4096, None), (1301, 192, 4096, 1100),
+                                           (257, 64, 16512, 257), (1300, 128, 4100, None)])
 @pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
 def test_gemm_gated_pair_is_the_two_launches_bit_for_bit(cuda, M, Kdim, N, rows, activation):
     """Both first projections of a gated feed-forward in one launch: the gate's product and the gated
     output against the two launches they replace (the gate's GEMM, then the gated GEMM) bit for bit --
-    under row bounds that pick the 128 x 128 tiles, the 64 x 64 ones and neither whole -- and the gate's
+    under row bounds that pick the 256-row tiles, the 128 x 128 ones, the 64 x 64 ones and none whole -- and the gate's
     product against the oracle's GEMM; rows past the bound are left as they were.  The first case is
     Llama-3.2-1B's prompt chunk."""
     rng = np.random.default_rng(M + N + 3)
