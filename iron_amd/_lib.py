@@ -191,6 +191,9 @@ def ptr(t) -> int | None:
 
 
 def current_stream() -> int:
+    """The HIP stream that PyTorch would launch on now, as an address.  Asked for as the address: the stream
+    object that ``torch.cuda.current_stream()`` builds around it costs 2.9 us a call against 0.3, a third of
+    what a small operator takes."""
     import torch
 
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())

@@ -19,6 +19,8 @@ GATES = {"silu": 1, "gelu_tanh": 2, "relu": 3}   # a gated feed-forward's activa
 
 
 def _dev(t, name, dtype=BF16):
+    if type(t) is torch.Tensor and t.is_cuda and t.dtype is dtype and t.is_contiguous():   # what a call nearly always brings
+        return t
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name}: expected a torch tensor, got {type(t).__name__}")
     if not t.is_cuda:
