@@ -36,6 +36,13 @@ const char* iron_last_error(void);
 int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K,
                    int b_col_maj, int c_col_maj, const int* valid, const int* valid_k,
                    void* stream);
+/* The same product where its tiles come out badly as rounds over the chip (a few tiles over a long K, or
+ * a last round nearly empty): some tiles' K is dealt over several blocks whose float32 sums meet in
+ * `workspace` (16-byte aligned, iron_gemm_workspace_bytes of it; what it holds does not matter).  0 bytes: the product
+ * shares no tiles, and iron_gemm_shared_bf16 refuses it. */
+int64_t iron_gemm_workspace_bytes(int M, int N, int K, int b_col_maj, int c_col_maj);
+int iron_gemm_shared_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K, int b_col_maj,
+                          int c_col_maj, void* workspace, void* stream);
 
 /* y[b] = W[b / repeat] @ x[b] for b in [0, batches): W (batches/repeat, M, K), x (batches, K),
  * y (batches, M); f32 accumulation, one rounding.  K % 8 == 0.

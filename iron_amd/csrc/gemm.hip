@@ -322,6 +322,8 @@ struct QkvTail {
   // kernel deals tiles itself instead of by the block's id.
   int k_begin, k_len, tile_plus1;
   float* partial;
+  // ... or the block's 128 x 128 float32 sums whole, as C's rows lie, at `tile_sums` (with C (N,M): C's).
+  float* tile_sums;
 };
 
 
@@ -586,7 +588,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
 // through LDS so that it leaves as whole 128-byte row segments (16 bytes a lane).  QKV: the fused
 // projections' per-tile choice of weight and output, RoPE on the accumulators.  Otherwise `qkv`
 // carries the optional residual epilogue.
-template <bool QKV, bool B_KN = false, bool C_NM = false>
+template <bool QKV, bool B_KN = false, bool C_NM = false, bool SHARED = false>
 __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B_,
                                                bf16_t* __restrict__ C_, int M, int N_, int K,
                                                const int* __restrict__ valid, int tiles_m, int tiles_n,
@@ -625,8 +627,8 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
     }
   }
   // (K,N): B's columns are read in whole tiles, so the last tile is moved back to end at N (what two
-  // tiles both cover comes out the same from both).
-  const int n0 = B_KN ? min(tn * NT_BN, N - NT_BN) : tn * NT_BN;
+  // tiles both cover comes out the same from both).  A matrix narrower than a tile is read to its last piece again.
+  const int n0 = B_KN ? max(min(tn * NT_BN, N - NT_BN), 0) : tn * NT_BN;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
@@ -646,14 +648,14 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
       // B (K,N) lands as stored: 64 k-rows of 128 columns (256 bytes a row, four rows an
       // instruction), a row's 16 chunks XORed with kn_swizzle(row) for the transposing reads below.
       const int kr = (wave * INST + i) * 4 + (lane >> 4);
-      b_voff[i] = (int)(((size_t)kr * N + ((lane & 15) ^ kn_swizzle(kr)) * 8) * 2);
+      b_voff[i] = (int)(((size_t)kr * N + min(((lane & 15) ^ kn_swizzle(kr)) * 8, N - 8 - n0)) * 2);
       b_head[i] = kr;
     }
   }
-  const int k_first = QKV || B_KN ? 0 : qkv.k_begin;
+  const int k_first = QKV || (B_KN && !SHARED) ? 0 : qkv.k_begin;
   const int pad = QKV ? 0 : k_pad(K);
   const bf16_t* a_tile = A + (size_t)m0 * K + k_first - pad;
-  const bf16_t* b_tile = B_KN ? B + n0 - (size_t)pad * N : B + (size_t)n0 * K + k_first - pad;
+  const bf16_t* b_tile = B_KN ? B + n0 + ((ptrdiff_t)k_first - pad) * N : B + (size_t)n0 * K + k_first - pad;
   auto issue_one = [&](char* st, int kt, int idx, bool head) {
     const int k0 = kt * BK;
     if (idx < INST) {
@@ -692,11 +694,11 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
     }
   }
 
-  const int nk = (!QKV && !B_KN && qkv.k_len > 0 ? qkv.k_len : K + pad) / BK;
+  const int nk = (!QKV && (!B_KN || SHARED) && qkv.k_len > 0 ? qkv.k_len : K + pad) / BK;
 #pragma unroll
   for (int s = 0; s < NT_STAGES - 1; ++s)
 #pragma unroll
-    for (int idx = 0; idx < LOADS; ++idx) issue_one(smem_nt + s * NT_STAGE_BYTES, min(s, nk - 1), idx, s == 0);
+    for (int idx = 0; idx < LOADS; ++idx) issue_one(smem_nt + s * NT_STAGE_BYTES, min(s, nk - 1), idx, s == 0 && (!SHARED || k_first == 0));
 
   // Fragments: lane -> row fr of a 16-row tile, 16-byte chunk kq of the k-step's four.
   const int fr = lane & 15, kq = lane >> 4;
@@ -887,6 +889,19 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
     }
   }
 
+  if constexpr (SHARED) {
+    if (qkv.tile_sums != nullptr) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int row = C_NM ? wn * 64 + j * 16 + fr : wm * 64 + i * 16 + fr;
+          const int at = C_NM ? wm * 64 + i * 16 + 4 * kq : wn * 64 + j * 16 + 4 * kq;
+          *reinterpret_cast<f32x4*>(qkv.tile_sums + row * NT_BN + at) = acc[i][j];
+        }
+      return;
+    }
+  }
   if constexpr (!QKV && !B_KN) {
     if (qkv.partial != nullptr) {
       // A slice of K: the float32 sums as they are, four columns of a row a lane and tile.
@@ -926,7 +941,7 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
     for (int r = 0; r < 8; ++r) {
       const int row = r * 8 + out_row;
       const uint4 v = *reinterpret_cast<const uint4*>(ot + row * OROWB + out_col * 2);
-      if (out_m >= M) continue;
+      if (out_m >= M || n0 + wn * 64 + row >= N) continue;
       bf16_t* p = C + (size_t)(n0 + wn * 64 + row) * M + out_m;
       if (whole_m) {
         *reinterpret_cast<uint4*>(p) = v;
@@ -2263,6 +2278,82 @@ int launch_grouped(const bf16_t* A, const bf16_t* B, bf16_t* C, int N, int K, co
   IRON_LAUNCH_CHECK();
 }
 
+// Products whose 128 x 128 tiles come out badly as rounds over the chip: the last `shared` tiles' K is dealt over
+// `slices` blocks each, which leave float32 sums in a workspace; a second launch adds them up and
+// rounds once.  A few tiles over a long K share all of them (one block's chain of stages is what the
+// product takes: 383 x 1472 x 6520 36 tiles of 102 stages), tiles that just miss a whole number of rounds share the
+// last, nearly empty round's.
+struct TileShares {
+  int whole, shared, slices;
+};
+
+template <bool B_KN, bool C_NM>
+__global__ __launch_bounds__(256) void gemm_shared_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
+                                                          bf16_t* __restrict__ C, int M, int N, int K, int tiles_m,
+                                                          int tiles_n, TileShares deal, float* __restrict__ sums) {
+  QkvTail tail{};
+  int tile = blockIdx.x;
+  if (tile >= deal.whole) {
+    const int at = tile - deal.whole, slice = at / deal.shared, nth = at - slice * deal.shared;
+    const int stages = (K + k_pad(K)) / BK, from = slice * stages / deal.slices, to = (slice + 1) * stages / deal.slices;
+    tile = deal.whole + nth;
+    tail.k_begin = from * BK;
+    tail.k_len = (to - from) * BK;
+    tail.tile_sums = sums + (size_t)at * (128 * 128);
+  }
+  int tm, tn;
+  tile_of_block(tile, tiles_m, tiles_n, 0, tm, tn);
+  tail.tile_plus1 = tm * tiles_n + tn + 1;
+  gemm_nt16_body<false, B_KN, C_NM, true>(A, B, C, M, N, K, nullptr, tiles_m, tiles_n, 0, tail);
+}
+
+// The shared tiles' sums added up in the order of k, eight columns a thread, eight blocks a tile.
+template <bool B_KN, bool C_NM>
+__global__ __launch_bounds__(256) void gemm_shared_finish_kernel(const float* __restrict__ sums, bf16_t* __restrict__ C,
+                                                                 int M, int N, int tiles_m, int tiles_n, TileShares deal) {
+  const int nth = blockIdx.x >> 3, at = ((blockIdx.x & 7) * 256 + threadIdx.x) * 8;
+  const float* from = sums + (size_t)nth * (128 * 128) + at;
+  const size_t slice = (size_t)deal.shared * (128 * 128);
+  f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+#pragma unroll 4
+  for (int p = 0; p < deal.slices; ++p) {
+    lo += *reinterpret_cast<const f32x4*>(from + p * slice);
+    hi += *reinterpret_cast<const f32x4*>(from + p * slice + 4);
+  }
+  int tm, tn;
+  tile_of_block(deal.whole + nth, tiles_m, tiles_n, 0, tm, tn);
+  const int m0 = tm * 128, n0 = B_KN ? max(min(tn * 128, N - 128), 0) : tn * 128;
+  const int row = (C_NM ? n0 : m0) + (at >> 7), col = (C_NM ? m0 : n0) + (at & 127);
+  const int rows = C_NM ? N : M, cols = C_NM ? M : N;
+  if (row >= rows || col >= cols) return;
+  bf16_t* to = C + (size_t)row * cols + col;
+  const uint32_t w[4] = {pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3])};
+  if ((cols & 7) == 0) {
+    *reinterpret_cast<uint4*>(to) = make_uint4(w[0], w[1], w[2], w[3]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (col + e < cols) to[e] = (bf16_t)((e & 1) ? (w[e >> 1] >> 16) : (w[e >> 1] & 0xffffu));
+  }
+}
+
+template <bool B_KN, bool C_NM>
+static int launch_gemm_shared(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, const TileShares& deal,
+                              float* sums, hipStream_t s) {
+  const int tiles_m = (M + 127) / 128, tiles_n = (N + 127) / 128;
+  constexpr size_t lds = (size_t)NT_STAGES * 256 * BK * 2;
+  static LdsOptIn opt_in;
+  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_shared_kernel<B_KN, C_NM>), lds); e != hipSuccess) {
+    set_error("gemm: %s", hipGetErrorString(e));
+    return (int)e;
+  }
+  hipLaunchKernelGGL((gemm_shared_kernel<B_KN, C_NM>), dim3(deal.whole + deal.shared * deal.slices), dim3(256), lds, s, A, B,
+                     C, M, N, K, tiles_m, tiles_n, deal, sums);
+  hipLaunchKernelGGL((gemm_shared_finish_kernel<B_KN, C_NM>), dim3(deal.shared * 8), dim3(256), 0, s, sums, C, M, N, tiles_m,
+                     tiles_n, deal);
+  IRON_LAUNCH_CHECK();
+}
+
 template <bool B_KN, bool STREAM_OUT>
 static int launch_gemm_nt256_as(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K,
                                 const int* valid, hipStream_t s) {
@@ -2293,9 +2384,7 @@ static int launch_gemm_nt256(const bf16_t* A, const bf16_t* B, bf16_t* C, int M,
 
 using namespace iron;
 
-extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K,
-                              int b_col_maj, int c_col_maj, const int* valid, const int* valid_k,
-                              void* stream) {
+static int check_gemm(const uint16_t* A, const uint16_t* B, const uint16_t* C, int M, int N, int K, int b_col_maj) {
   IRON_REQUIRE(A && B && C, "gemm: null operand");
   IRON_REQUIRE(M > 0 && N > 0 && K > 0, "gemm: M (%d), N (%d), K (%d) must be positive", M, N, K);
   IRON_REQUIRE(K % 8 == 0, "gemm: K (%d) must be a multiple of 8 (16-byte loads)", K);
@@ -2305,6 +2394,20 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
                "gemm: operands must be 16-byte aligned");
   IRON_REQUIRE(b_col_maj || N % 8 == 0,
                "gemm: N (%d) must be a multiple of 8 when B is (K,N) (16-byte loads along N)", N);
+  return 0;
+}
+
+// Whether the 256x256 tiles take a product (see iron_gemm_bf16).
+static bool gemm_on_big_tiles(int M, int N, int K) {
+  const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
+  const long tiles256 = (long)((M + BIG_BM - 1) / BIG_BM) * ((N + BIG_BN - 1) / BIG_BN);
+  return M >= BIG_BM && N >= BIG_BN && N % 8 == 0 && tiles256 >= (K % BK == 0 ? 192 : 144) && 5 * tiles128 >= 16 * tiles256;
+}
+
+extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K,
+                              int b_col_maj, int c_col_maj, const int* valid, const int* valid_k,
+                              void* stream) {
+  if (const int rc = check_gemm(A, B, C, M, N, K, b_col_maj); rc != 0) return rc;
   hipStream_t s = (hipStream_t)stream;
   // The (N,M) output of A and B (N,K) is the (M,N) output of B and A: both are rows of K (2048^3 41.5 ->
   // 19.4 us against the general kernel's strided stores).
@@ -2322,8 +2425,9 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
   // the general kernel below, which loads through registers: 2048 x 2048 x 2056 42.5 -> 26.0 us, 86 x 1728 x
   // 5560 59 -> 26.5, (K,N) 2048 x 2048 x 2040 65 -> 22.0, 300 x 1000 x 1000 33.6 -> 9.8.  (A K that is no
   // multiple of 64 stays dearer than its neighbour that is, 26.0 us against 19.4: its rows' 128-byte
-  // pieces straddle two cache lines.)  (K,N) wants a whole tile of columns.
-  if (valid_k == nullptr && K >= BK && (b_col_maj ? !c_col_maj : M >= 64 && N >= 128 && (!c_col_maj || valid == nullptr))) {
+  // pieces straddle two cache lines.)  Under a whole tile of (K,N) two stages of it are no gain (1 x 64 x 64 3.6 us
+  // against 4.3).
+  if (valid_k == nullptr && K >= BK && (b_col_maj ? !c_col_maj : (!c_col_maj || valid == nullptr) && ((M >= 64 && N >= 128) || K > 2 * BK))) {
     if (c_col_maj) return launch_gemm_nt<true, false, 2, 4, true>(A, B, C, M, N, K, valid, s);
     const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
     // Enough 256x256 tiles to fill the chip: the large-tile kernel (offsets are 32-bit).  A round of
@@ -2332,10 +2436,8 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
     // that waste more than a fifth of the large tiles stay with the smaller; where rows straddle cache
     // lines the large tile, which reads half as much, gains more (1500 x 6000 x 3000: 144 tiles 93 us
     // against 110).
-    const long tiles256 = (long)((M + BIG_BM - 1) / BIG_BM) * ((N + BIG_BN - 1) / BIG_BN);
     const bool whole = M % BIG_BM == 0 && N % BIG_BN == 0;
-    const bool big = M >= BIG_BM && N >= BIG_BN && N % 8 == 0 && tiles256 >= (K % BK == 0 ? 192 : 144) &&
-                     5 * tiles128 >= 16 * tiles256;
+    const bool big = gemm_on_big_tiles(M, N, K);
     if (b_col_maj && big && (valid == nullptr || whole)) {
       // Under a row bound read on the device the large tiles may cover too few rows to fill the
       // chip (512 valid rows of 2048 leave 64 of 256 tiles): the blocks of one launch then choose
@@ -2368,6 +2470,59 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
   if (tiles128 >= 128 || (M >= 128 && N >= 128))
     return launch_gemm<128, 128, 2, 2>(A, B, C, M, N, K, b_col_maj, c_col_maj, valid, valid_k, s);
   return launch_gemm<64, 64, 2, 2>(A, B, C, M, N, K, b_col_maj, c_col_maj, valid, valid_k, s);
+}
+
+// How a product's 128 x 128 tiles are shared (none: slices 0), M and N as the tiles see them, by what was
+// measured, in us.  Unshared: 3 a launch; a stage of 64 k 0.5 a round of 128 x 128 tiles; on the 64 x 64 tiles
+// that few tiles of B (N,K) take, 0.13 to 0.23 up to a block a CU, and 0.14 (a few blocks) to 0.34 where K is no multiple of 64.
+// Shared: the second launch and 0.028 a slice of a tile (its 64 KB out and back) on top, which the slices
+// are chosen against.  Both sides: 97 x 400 x 7392 with B (K,N) 48.8 -> 14.0, 383 x 1472 x 6520 50.7 -> 25.0, 86 x 1728 x
+// 5560 with B (N,K) 26.6 -> 16.0, 5300 x 864 x 7744 (294 tiles) 92 -> 74; not 1024 x 1024 x 4096, 15.5 against 21.2.
+static TileShares gemm_shares(int M, int N, int K, bool b_nk, bool c_nm) {
+  const TileShares none{0, 0, 0};
+  const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
+  if (K < BK || (b_nk && M < 64) || tiles > 3 * 256) return none;   // (fewer rows of B (N,K): iron_gemm_few_bf16)
+  if (!c_nm && gemm_on_big_tiles(M, N, K)) return none;
+  const int stages = (K + BK - 1) / BK, t = (int)tiles;
+  const int shared = t <= 128 ? t : (t > 256 ? t % 256 : 0);   // all tiles, or those of the last round
+  if (shared == 0 || shared > 128) return none;
+  const int by_cost = (int)(4.2f * sqrtf((float)stages / shared) + 0.5f);
+  int slices = 256 / shared < stages / 6 ? 256 / shared : stages / 6;
+  if (slices > by_cost) slices = by_cost;
+  if (slices < 2) return none;
+  const float fill = (float)((long)((M + 63) / 64) * ((N + 63) / 64)) / 256.f;
+  const float stage64 = K % BK == 0 ? 0.13f + 0.10f * fill : fminf(0.14f + 3.f * fill, 0.22f + 0.12f * fill);
+  const float now = 3.f + stages * (b_nk && t <= 128 ? stage64 : 0.5f * ((t + 255) / 256));
+  const float then = 7.f + 0.028f * slices * shared + 0.5f * ((stages + slices - 1) / slices + stages * ((t - shared) / 256));
+  return then < 0.9f * now ? TileShares{t - shared, shared, slices} : none;
+}
+
+extern "C" int64_t iron_gemm_workspace_bytes(int M, int N, int K, int b_col_maj, int c_col_maj) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 8 != 0) return 0;
+  const bool turned = b_col_maj && c_col_maj;
+  const TileShares deal = gemm_shares(turned ? N : M, turned ? M : N, K, b_col_maj, c_col_maj && !turned);
+  return (int64_t)deal.slices * deal.shared * 128 * 128 * sizeof(float);
+}
+
+extern "C" int iron_gemm_shared_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K,
+                                     int b_col_maj, int c_col_maj, void* workspace, void* stream) {
+  if (const int rc = check_gemm(A, B, C, M, N, K, b_col_maj); rc != 0) return rc;
+  IRON_REQUIRE(workspace != nullptr && ((uintptr_t)workspace & 15) == 0, "gemm_shared: a workspace, 16-byte aligned");
+  IRON_REQUIRE(M <= (1 << 22), "gemm_shared: M (%d) may be at most 2^22", M);
+  if (b_col_maj && c_col_maj) {   // (as iron_gemm_bf16)
+    const uint16_t* rows = A;
+    A = B, B = rows;
+    const int m = M;
+    M = N, N = m;
+    c_col_maj = 0;
+  }
+  const TileShares deal = gemm_shares(M, N, K, b_col_maj, c_col_maj);
+  IRON_REQUIRE(deal.slices > 0, "gemm_shared: a product of %d x %d over %d shares no tiles (iron_gemm_workspace_bytes is 0)", M, N, K);
+  hipStream_t s = (hipStream_t)stream;
+  float* sums = (float*)workspace;
+  if (b_col_maj) return launch_gemm_shared<false, false>(A, B, C, M, N, K, deal, sums, s);
+  if (c_col_maj) return launch_gemm_shared<true, true>(A, B, C, M, N, K, deal, sums, s);
+  return launch_gemm_shared<true, false>(A, B, C, M, N, K, deal, sums, s);
 }
 
 // A product over many rows whose epilogue reads a second (M, N) operand: the residual sum or the gate.

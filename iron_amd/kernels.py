@@ -8,6 +8,7 @@ raises ``IronHipError`` on refusal.  Nothing here computes.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 
 import torch
@@ -47,10 +48,22 @@ def _numel(t, n, name):
         raise ValueError(f"{name}: expected {n} elements, got {t.numel()} {tuple(t.shape)}")
 
 
+@functools.lru_cache(maxsize=4096)
+def _gemm_workspace(M, N, K, b_col_maj, c_col_maj) -> int:
+    return int(lib().iron_gemm_workspace_bytes(M, N, K, int(b_col_maj), int(c_col_maj)))
+
+
 def gemm(A, B, C, *, M, N, K, b_col_maj=False, c_col_maj=False, valid=None, valid_k=None):
     _numel(_dev(A, "A"), M * K, "A")
     _numel(_dev(B, "B"), K * N, "B")
     _numel(_dev(C, "C"), M * N, "C")
+    if valid is None and valid_k is None:
+        room = _gemm_workspace(M, N, K, bool(b_col_maj), bool(c_col_maj))
+        if room:
+            sums = torch.empty(room, dtype=torch.uint8, device=C.device)
+            check(lib().iron_gemm_shared_bf16(ptr(A), ptr(B), ptr(C), M, N, K, int(b_col_maj), int(c_col_maj), ptr(sums),
+                                              current_stream()), "iron_gemm_shared_bf16")
+            return
     check(
         lib().iron_gemm_bf16(
             ptr(A), ptr(B), ptr(C), M, N, K, int(b_col_maj), int(c_col_maj),

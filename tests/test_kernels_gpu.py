@@ -127,6 +127,45 @@ def test_gemm_at_the_edges_of_tiles_and_stages(cuda, M, Kdim, N, b_col_maj, c_co
     assert np.all(np.abs(from_torch(C) - want) <= ops.gemm_bound(A, B, b_col_maj=b_col_maj, c_col_maj=c_col_maj))
 
 
+@pytest.mark.parametrize("M,Kdim,N,b_col_maj,c_col_maj", [
+    (64, 8192, 64, True, False), (67, 3640, 872, True, False), (872, 3640, 67, True, True),   # all tiles shared, B (N,K)
+    (1, 4096, 400, False, False), (130, 2504, 72, False, False), (257, 4000, 264, False, False),   # ... and (K,N)
+    (123, 2856, 200, False, True), (2049, 2504, 2056, True, False), (2049, 2504, 2056, False, False),   # (N,M); the last round's tiles
+])
+def test_gemm_whose_tiles_are_shared(cuda, M, Kdim, N, b_col_maj, c_col_maj):
+    """Products whose tiles' K is dealt over several blocks, over a workspace of NaNs: against the oracle by the
+    layouts' bound, and the same bits from a recorded graph's replays, whatever ran in between."""
+    assert K._gemm_workspace(M, N, Kdim, b_col_maj, c_col_maj) > 0
+    rng = np.random.default_rng(M + N + Kdim)
+    A, B = bf(rng, M, Kdim), bf(rng, (N if b_col_maj else Kdim), (Kdim if b_col_maj else N), scale=0.05)
+    dA, dB = dev(A, cuda), dev(B, cuda)
+    kw = dict(M=M, N=N, K=Kdim, b_col_maj=b_col_maj, c_col_maj=c_col_maj)
+    torch.full((32 << 20,), 255, dtype=torch.uint8, device=cuda)   # what the allocator hands out next is bf16 and float32 NaN
+    C = out_like((N, M) if c_col_maj else (M, N), cuda, fill=float("nan"))
+    K.gemm(dA, dB, C, **kw)
+    want = ops.gemm(A, B, b_col_maj=b_col_maj, c_col_maj=c_col_maj)
+    assert np.all(np.abs(from_torch(C) - want) <= ops.gemm_bound(A, B, b_col_maj=b_col_maj, c_col_maj=c_col_maj))
+    again = torch.zeros_like(C)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        K.gemm(dA, dB, again, **kw)
+        K.gemm(dA, dB, again, **kw)
+    for _ in range(3):
+        again.fill_(7.0)
+        K.gemm(dA, dB, torch.empty_like(C), **kw)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(again, C)
+
+
+def test_gemm_that_shares_no_tiles_is_refused_a_workspace(cuda):
+    """Whole rounds, or too short a K: no workspace, and the shared entry point refuses before any launch."""
+    for M, N, Kdim, b, c in ((2048, 2048, 2048, 0, 0), (1024, 1024, 1024, 1, 0), (64, 64, 56, 1, 0), (64, 64, 12, 1, 0), (32, 4096, 8192, 1, 0)):
+        assert K.lib().iron_gemm_workspace_bytes(M, N, Kdim, b, c) == 0
+    t = out_like((1024 * 1024,), cuda, fill=0.0)
+    assert K.lib().iron_gemm_shared_bf16(t.data_ptr(), t.data_ptr(), t.data_ptr(), 1024, 1024, 1024, 1, 0, t.data_ptr(), 0) == 1
+
+
 @pytest.mark.parametrize("b_col_maj", [True, False])
 @pytest.mark.parametrize("n", [4096, 8192])
 def test_gemm_large_squares_on_sampled_rows(cuda, n, b_col_maj):
