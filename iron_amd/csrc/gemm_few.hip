@@ -324,25 +324,38 @@ static int launch_gemm_strips(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
   IRON_LAUNCH_CHECK();
 }
 
-// Which products go by strips.  Below 4 MB of B a launch is mostly its start, which gemm_few_kernel's is shorter (777 x 1000, 8 rows: 3.3 us
-// against 3.5).  K up to eight strips: up to 32 rows of A (33: 8192 x 2048 15.1 us against 12.6).  A longer K: the strips of A that come with
-// every tile cost as much as B's own, so up to eight rows of A, more only where a block has one tile (16 rows: 2048 x 8192 11.2 us against
-// 16.6, 4096 x 4096 11.0 against 9.9; 48 rows: 30.4 against 33.9, 23.3 against 15.2 at 3072 x 3072).  The loads go past the caches except
-// where a block has one tile over a long K (2048 x 8192, 8 rows: 9.3 us, past them 10.5; 4096 x 4096 10.1 and 9.4).
+// Which products go by strips, by what both kernels took over sixty shapes (us, gemm_few_kernel against strips).  Below 4 MB of B
+// a launch is mostly its start, which gemm_few_kernel's is shorter (777 x 1000, 8 rows: 3.3 against 3.5).
+// K up to eight strips: up to 16 rows of A (8 rows: 8192 x 2048 9.0 / 8.7, 16384 x 1024 12.1 / 10.4, 128256 x 2048 105 / 84), but not short
+// rows that straddle cache lines (16000 x 600 8.7 / 9.4) nor up to four rows where long rows make one round or two
+// (one row: 3072 x 2048 5.1 / 5.6, 4096 x 2048 5.4 / 5.9); more rows, whose sums take a second set of registers, only over a B of 64 MB
+// (20 rows: 128256 x 2048 137 / 87, 16384 x 1024 10.7 / 14.5).
+// A longer K: the strips of A that come with every tile cost as much as B's own.  Up to eight rows where a block has one tile or many
+// (2048 x 8192 13.9 / 8.9, 9048 x 8184 49 / 35, but 4096 x 14336 22.7 / 26.1 and 2728 x 6128 9.9 / 12.3); up to 16 where it
+// has one (2048 x 8192 16.7 / 10.2); more where that one's rows keep to their cache lines or are few (32 rows: 2048 x 4096 13.2 / 12.2,
+// 1024 x 8192 23.5 / 14.8; 20 rows of 1960 x 6512 13.8 / 15.1).  The loads go past the caches except where a block has
+// one tile over a long K (2048 x 8192, 8 rows: 9.3, past them 10.5; 4096 x 4096 10.1 and 9.4).
 // Returns -1 where it is not for them.
 static int strips_for(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s) {
-  if ((long long)N * K < (1 << 21)) return -1;
-  const bool one_tile = N <= 256 * STRIP_ROWS;
+  const long long size = (long long)N * K;
+  if (size < (1 << 21)) return -1;
+  const bool one_tile = N <= 256 * STRIP_ROWS, on_lines = K % 64 == 0;
   if (K <= STRIP * STRIP_WAVES) {
+    if (M > 32 || (M > 16 && size < (1 << 25)) || (!on_lines && K < 1024)) return -1;
+    if (M > 16) return launch_gemm_strips<2, 16, true, 2, true>(A, B, C, M, N, K, s);
+    if (M <= 4 && size <= (1 << 23) && K > 1024 && N > 1536) return -1;
     if (M <= 8) return launch_gemm_strips<1, 8, true, 2, true>(A, B, C, M, N, K, s);
-    if (M <= 16) return launch_gemm_strips<1, 16, true, 2, true>(A, B, C, M, N, K, s);
-    return M <= 32 ? launch_gemm_strips<2, 16, true, 2, true>(A, B, C, M, N, K, s) : -1;
+    return launch_gemm_strips<1, 16, true, 2, true>(A, B, C, M, N, K, s);
   }
   if ((long long)64 * K * 2 >= 0x7ffffff0ll) return -1;   // (offsets within 64 rows are 32 bits wide)
-  if (M <= 8)
-    return one_tile ? launch_gemm_strips<1, 8, false, 2, false>(A, B, C, M, N, K, s) : launch_gemm_strips<1, 8, false, 2, true>(A, B, C, M, N, K, s);
+  if (M <= 8) {
+    if (one_tile) return launch_gemm_strips<1, 8, false, 2, false>(A, B, C, M, N, K, s);
+    if (N >= 8192 || (N > 4096 && K < 4096)) return launch_gemm_strips<1, 8, false, 2, true>(A, B, C, M, N, K, s);
+    return -1;
+  }
   if (!one_tile) return -1;
   if (M <= 16) return launch_gemm_strips<1, 16, false, 1, false>(A, B, C, M, N, K, s);
+  if (!on_lines && N > 1280) return -1;
   return M <= 32 ? launch_gemm_strips<2, 16, false, 2, false>(A, B, C, M, N, K, s) : launch_gemm_strips<4, 16, false, 2, false>(A, B, C, M, N, K, s);
 }
 

@@ -128,7 +128,7 @@ def test_gemm_at_the_edges_of_tiles_and_stages(cuda, M, Kdim, N, b_col_maj, c_co
 
 
 @pytest.mark.parametrize("M,Kdim,N,b_col_maj,c_col_maj", [
-    (64, 8192, 64, True, False), (67, 3640, 872, True, False), (872, 3640, 67, True, True),   # all tiles shared, B (N,K)
+    (64, 8192, 64, True, False), (24, 6200, 200, True, False), (63, 8184, 136, True, True), (67, 3640, 872, True, False), (872, 3640, 67, True, True),   # all tiles shared, B (N,K)
     (1, 4096, 400, False, False), (130, 2504, 72, False, False), (257, 4000, 264, False, False),   # ... and (K,N)
     (123, 2856, 200, False, True), (2049, 2504, 2056, True, False), (2049, 2504, 2056, False, False),   # (N,M); the last round's tiles
 ])
@@ -160,7 +160,7 @@ def test_gemm_whose_tiles_are_shared(cuda, M, Kdim, N, b_col_maj, c_col_maj):
 
 def test_gemm_that_shares_no_tiles_is_refused_a_workspace(cuda):
     """Whole rounds, or too short a K: no workspace, and the shared entry point refuses before any launch."""
-    for M, N, Kdim, b, c in ((2048, 2048, 2048, 0, 0), (1024, 1024, 1024, 1, 0), (64, 64, 56, 1, 0), (64, 64, 12, 1, 0), (32, 4096, 8192, 1, 0)):
+    for M, N, Kdim, b, c in ((2048, 2048, 2048, 0, 0), (1024, 1024, 1024, 1, 0), (64, 64, 56, 1, 0), (64, 64, 12, 1, 0), (16, 4096, 8192, 1, 0)):
         assert K.lib().iron_gemm_workspace_bytes(M, N, Kdim, b, c) == 0
     t = out_like((1024 * 1024,), cuda, fill=0.0)
     assert K.lib().iron_gemm_shared_bf16(t.data_ptr(), t.data_ptr(), t.data_ptr(), 1024, 1024, 1024, 1, 0, t.data_ptr(), 0) == 1

@@ -93,8 +93,9 @@ def test_a_product_over_few_rows(cuda, M, N, K_):
 
 # Products that go by strips of K: a tile of B's rows and less, a block's first second tile, groups of eight tiles stored together and the
 # ninth, N no multiple of 8; K just over a strip, to eight strips and past them with waves that have none; the rows of A at every edge.
-@pytest.mark.parametrize("M,N,K_", [(1, 1024, 2048), (8, 2049, 1032), (9, 2056, 1960), (16, 16384 + 72, 264), (17, 18500, 136), (32, 4104, 2048),
-                                    (2, 1027, 2056), (8, 2048, 8192), (7, 2064, 4104), (16, 520, 5000), (29, 2040, 2304), (33, 600, 4096), (63, 999, 2816)])
+@pytest.mark.parametrize("M,N,K_", [(1, 1024, 2048), (8, 2049, 1032), (9, 2056, 1960), (16, 16384 + 72, 320), (17, 30011, 1160), (32, 16392, 2048),
+                                    (2, 1027, 2056), (8, 2048, 8192), (7, 4100, 2312), (8, 8200, 4104), (16, 520, 5000), (29, 2040, 2304),
+                                    (33, 600, 4096), (47, 999, 2816)])
 def test_a_product_over_few_rows_by_strips(cuda, M, N, K_):
     rng = np.random.default_rng(N)
     a, b = bf(rng, M, K_), bf(rng, N, K_, scale=0.1)
