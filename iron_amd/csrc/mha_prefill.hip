@@ -34,9 +34,213 @@ constexpr int BKV = 64;   // key rows per tile
 constexpr float kLazyBits = 8.f;        // how far a maximum may run ahead of the reference the exponents are taken against
 constexpr float kSumLow = 0x1p-60f, kSumHigh = 0x1p24f;   // a tile's sum of exponentials outside this range: take its maximum and redo it
 constexpr int kCUs = 256;                // compute units the block orders below assume
+// Whether queries that fill `live` blocks of the launch go 32 to a block instead, the keys dealt over its waves
+// (prefill_few_rows).  Four times the blocks each read all the keys, so it pays while the chip has CUs for them,
+// and from a few tiles a wave on.  us, 32 / 8 heads, tiles against few rows: 40 queries, d = 64, 512 / 2048 / 12043
+// keys 11.2 / 9.7, 23.8 / 14.5, 103 / 44; 512 queries 11.5 / 11.0, 25.3 / 22.0, 112 / 83; d = 128, 8000 keys, 256 queries 121 / 56, 512 queries over
+// 512 keys 18.3 / 21.8.
+template <int D>
+__host__ __device__ __forceinline__ bool few_rows_pay(int live, int keys) { return live <= (D == 64 ? 128 : 64) && keys >= 512; }
 constexpr int kFewBlocks = 512;          // launches of fewer blocks than this halve their blocks' queries (S = 1024 at 32 heads: 18.5 -> 13.9 us)
 constexpr int kWideBigBlocks = 512;     // wide heads: launches of at least this many 128-query blocks keep that size
 constexpr int kSplitMaxBlocks = 1024;   // launches of up to this many blocks split each block's tiles over two halves
+
+// Few live queries over many keys (a turn late in a conversation: 40 rows of a 2048-row launch, 12 000 keys): by the
+// tiles below, a block a head and 128 queries, most of the chip would idle behind a block's chain
+// of tiles.  Here a block takes 32 queries of one head and its NW waves deal the keys among them, wave w the 32-key
+// tiles w, w + NW, ...; their (max, sum, O) meet in LDS.  No wave waits for another before that: a
+// wave has a K and a V tile of its own in LDS, takes both into registers and sends for the next ones before it
+// computes.  S^T, the lanes' queries and O^T lie as in the
+// kernel below.
+template <int D, int NW>
+__device__ __forceinline__ void prefill_few_rows(
+    char* smem, const bf16_t* __restrict__ Qh, const bf16_t* __restrict__ Kh, const bf16_t* __restrict__ Vh,
+    bf16_t* __restrict__ Oh, int q0, int seq, int q_tokens, int kv_tokens, int offset, float scale_log2, int causal, int window,
+    long q_row_stride, long kv_row_stride) {
+  constexpr int ROWB = D * 2, KS = D / 16, DT = D / 32, CPR = D / 8;
+  constexpr int TK = 32, TILE = TK * ROWB, VINST = TILE / 1024, RPI = 1024 / ROWB;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));   // (what depends on the lane is made here: shared with the caller's, a value of it spilled)
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, g = lane >> 5;
+  const int my_q = q0 + col;
+  const bool q_live = my_q < q_tokens;
+  const int qpos = offset + my_q, wq_lo = offset + q0, wq_hi = offset + min(q0 + 31, q_tokens - 1);
+
+  // Keys the block's live queries can see, in tiles; this wave's are wave, wave + NW, ...
+  int kv_hi = kv_tokens;
+  if (causal) kv_hi = min(kv_hi, wq_hi + 1);
+  else if (window >= 0) kv_hi = min(kv_hi, wq_hi + window + 1);
+  const int kv_lo = window >= 0 ? max(0, wq_lo - window) / TK * TK : 0;
+  const int ntiles = (kv_hi - kv_lo + TK - 1) / TK;
+  const int steps = ntiles > wave ? (ntiles - wave + NW - 1) / NW : 0;
+
+  // The head's keys (values) from kv_lo's row to the last key's end are one buffer: rows past it read as zeros.
+  const int row_bytes = (int)kv_row_stride * 2;
+  const int reach = kv_hi > kv_lo ? (kv_tokens - kv_lo - 1) * row_bytes + ROWB : 0;
+  const __amdgpu_buffer_rsrc_t k_rows = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<bf16_t*>(Kh + (long)kv_lo * kv_row_stride), 0, reach, 0x00020000);
+  const __amdgpu_buffer_rsrc_t v_rows = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<bf16_t*>(Vh + (long)kv_lo * kv_row_stride), 0, reach, 0x00020000);
+  // Load i covers tile rows i RPI + l; chunks swizzled as below.  A row starts on a multiple of its head's bytes, so the part of K's
+  // swizzle that is the load's own is an XOR of the lane's offset.
+  static_assert(RPI % 4 == 0, "V's swizzle, 2 (row % 4), is the lane's alone");
+  const int l = lane / CPR;
+  const int k_lane = l * row_bytes + (((lane % CPR) ^ (l >> 1)) << 4), v_lane = l * row_bytes + (((lane % CPR) ^ ((l & 3) << 1)) << 4);
+  char* stage = smem + wave * (2 * TILE);   // the wave's K tile, then its V tile
+  auto issue = [&](int step) {
+    const int at = (wave + step * NW) * TK * row_bytes;
+#pragma unroll
+    for (int i = 0; i < VINST; ++i) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(k_rows, IRON_LDS_PTR(stage + i * 1024), 16,
+                                               (int)(k_lane ^ ((i * RPI / 2 & 7) << 4)) + at + i * RPI * row_bytes, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(v_rows, IRON_LDS_PTR(stage + TILE + i * 1024), 16,
+                                               (int)v_lane + at + i * RPI * row_bytes, 0, 0, 0);
+    }
+  };
+  if (steps > 0) issue(0);
+
+  bf16x8 qf[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (q_live) v = *reinterpret_cast<const uint4*>(Qh + (size_t)my_q * q_row_stride + 8 * g + 16 * s);
+    qf[s] = __builtin_bit_cast(bf16x8, v);
+  }
+  const int v_key = 4 * g + ((lane & 15) >> 2), v_swz = ((lane >> 2) & 3) << 1;
+  unsigned v_frag[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) {
+    const int chunk = dt * 4 + (((lane >> 4) & 1) << 1) + ((lane & 3) >> 1);
+    v_frag[dt] = (unsigned)(size_t)IRON_LDS_PTR(stage) + TILE + v_key * ROWB + ((chunk ^ v_swz) << 4) + ((lane & 1) << 3);
+  }
+  int see_hi = kv_tokens - 1, see_lo = 0;
+  if (causal) see_hi = min(see_hi, qpos);
+  else if (window >= 0) see_hi = min(see_hi, qpos + window);
+  if (window >= 0) see_lo = max(0, qpos - window);
+  const unsigned see_span = see_hi >= see_lo ? (unsigned)(see_hi - see_lo) : 0u;
+  if (see_hi < see_lo) see_lo = 1 << 30;
+
+  f32x16 oacc[DT];
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) oacc[t][e] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+
+  const unsigned k_frag = (unsigned)(size_t)IRON_LDS_PTR(stage) + col * ROWB;
+  const int k_swz = (col >> 1) & 7;
+  for (int step = 0; step < steps; ++step) {
+    const int kv0 = kv_lo + (wave + step * NW) * TK;
+    wait_vmcnt<0>();   // the wave's own tiles: nobody else's wait, no barrier
+    bf16x8 kf[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) kf[s] = lds_read_b128_at<0>(k_frag + (((2 * s + g) ^ k_swz) << 4));
+    TrFrag vf[DT][2];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      vf[dt][0].lo = lds_read_tr16_at<0>(v_frag[dt]);
+      vf[dt][0].hi = lds_read_tr16_at<8 * ROWB>(v_frag[dt]);
+      vf[dt][1].lo = lds_read_tr16_at<16 * ROWB>(v_frag[dt]);
+      vf[dt][1].hi = lds_read_tr16_at<24 * ROWB>(v_frag[dt]);
+    }
+#pragma unroll
+    for (int s = 0; s < KS; ++s) lds_wait_for<0>(kf[s]);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) lds_tr_wait(vf[dt][0], vf[dt][1]);
+    if (step + 1 < steps) issue(step + 1);   // the tiles are in registers: their buffers take the next ones
+    f32x16 sacc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sacc[e] = 0.f;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s], qf[s], sacc, 0, 0, 0);
+    // Element e is key kv0 + 8 (e / 4) + 4 g + e % 4, query `col`.
+    bool edge = kv0 + TK > kv_tokens;
+    if (causal) edge |= kv0 + TK - 1 > wq_lo;
+    else if (window >= 0) edge |= kv0 + TK - 1 > wq_lo + window;
+    if (window >= 0) edge |= kv0 < wq_hi - window;
+    if (edge) {
+      const int rel = kv0 + 4 * g - see_lo;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) sacc[e] = (unsigned)(rel + 8 * (e >> 2) + (e & 3)) > see_span ? -INFINITY : sacc[e];
+    }
+    // The reference follows the maxima lazily, as below.
+    float rmax = sacc[0];
+#pragma unroll
+    for (int e = 1; e < 16; ++e) rmax = fmaxf(rmax, sacc[e]);
+    if (__builtin_amdgcn_ballot_w64((rmax - m_run) * scale_log2 > kLazyBits || (m_run == -INFINITY && rmax != -INFINITY)) != 0) {
+      const float m_new = fmaxf(m_run, max_with_other_half(rmax));
+      const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m_run - m_new) * scale_log2);
+      l_run *= alpha;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) oacc[t][e] *= alpha;
+      m_run = m_new;
+    }
+    const float mc = m_run == -INFINITY ? 0.f : m_run * scale_log2;
+    bf16x8 pf[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float p[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        float e = __builtin_amdgcn_exp2f(fmaf(sacc[8 * h + j], scale_log2, -mc));
+        if (edge && sacc[8 * h + j] == -INFINITY) e = 0.f;   // also where the scale is 0 and -inf * 0 is no number
+        p[j] = e;
+        l_run += e;
+      }
+      pf[h] = __builtin_bit_cast(bf16x8, pack8(p));
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_join(vf[dt][h]), pf[h], oacc[dt], 0, 0, 0);
+  }
+
+  // The upper half of the waves hands over to the lower, until one is left: a value a lane a row.
+  constexpr int FIELDS = 2 + 16 * DT;
+  float* hand = reinterpret_cast<float*>(smem);
+#pragma unroll
+  for (int left = NW / 2; left >= 1; left >>= 1) {
+    __syncthreads();   // every wave is done with the stages, or with what the round before handed over
+    if (wave >= left && wave < 2 * left) {
+      float* to = hand + (wave - left) * FIELDS * 64 + lane;
+      to[0] = m_run;
+      to[64] = l_run;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) to[(2 + 16 * t + e) * 64] = oacc[t][e];
+    }
+    __syncthreads();
+    if (wave < left) {
+      const float* from = hand + wave * FIELDS * 64 + lane;
+      const float m_other = from[0], l_other = from[64];
+      const float m_new = fmaxf(m_run, m_other);
+      const float mc = (m_new == -INFINITY) ? 0.f : m_new * scale_log2;
+      const float a_mine = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(fmaf(m_run, scale_log2, -mc));   // a wave
+      const float a_other = m_other == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(fmaf(m_other, scale_log2, -mc));   // may have seen no key
+      m_run = m_new;
+      l_run = l_run * a_mine + l_other * a_other;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) oacc[t][e] = oacc[t][e] * a_mine + from[(2 + 16 * t + e) * 64] * a_other;
+    }
+  }
+  if (wave != 0 || my_q >= seq) return;
+  const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+  const float inv = (q_live && l_tot > 0.f) ? 1.0f / l_tot : 0.f;
+  bf16_t* op = Oh + (size_t)my_q * q_row_stride;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<uint2*>(op + 32 * dt + 8 * q + 4 * g) =
+          make_uint2(pack_bf16(oacc[dt][4 * q + 0] * inv, oacc[dt][4 * q + 1] * inv),
+                     pack_bf16(oacc[dt][4 * q + 2] * inv, oacc[dt][4 * q + 3] * inv));
+}
 
 // K and V tiles go straight from global memory into LDS (buffer loads with the LDS bit, no register staging), as
 // stored: [64 keys][D], STAGES tiles deep.  16-byte chunks of a row are XOR-swizzled so unpadded
@@ -58,7 +262,7 @@ constexpr int kSplitMaxBlocks = 1024;   // launches of up to this many blocks sp
 //
 // W: the waves that share a tile's loads, each with 32 of the block's 32 W queries.  Four; two
 // where four would leave CUs without a block (a short prompt), so that twice as many blocks go out.
-template <int D, int SPLIT, int W = 4>
+template <int D, int SPLIT, int W, bool FEW>
 __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(W == 4 ? (D == 64 && SPLIT == 2 ? 4 : 2) : (D == 64 && SPLIT == 2 ? 2 : 1)))) void mha_prefill_kernel(
     const bf16_t* __restrict__ Q, const bf16_t* __restrict__ K, const bf16_t* __restrict__ V,
     bf16_t* __restrict__ O, int heads, int group, int seq, int seq_len, int kv_len, float scale_log2,
@@ -104,6 +308,28 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
   const int kv_tokens = kv_valid ? bound_or(kv_valid, kv_len) : (kv_len - seq + q_tokens);
   const bool masked_any = causal || window >= 0;
   const int offset = masked_any ? (kv_tokens - q_tokens) : 0;
+
+  // Few live queries (FEW: the launch may have them; the code beside the tiles' costs those 1.5 % at d = 128): groups of 32 take the first blocks, all blocks the zeros of the rows past them.
+  const int groups = FEW ? (q_tokens + 31) >> 5 : 0;
+  if (FEW && groups > 0 && groups <= nqb && offset >= 0 &&
+      few_rows_pay<D>(heads * ((q_tokens + BQW - 1) / BQW), window < 0 ? kv_tokens : min(kv_tokens, window + q_tokens))) {
+    const int all = (seq + 31) >> 5;
+    for (int unit = blockIdx.x; unit < heads * (all - groups); unit += gridDim.x) {
+      const int h = unit % heads, r0 = (groups + unit / heads) * 32;
+      bf16_t* to = O + (size_t)h * q_head_stride;
+      for (int i = tid; i < 32 * CPR; i += 64 * W * SPLIT) {
+        const int r = r0 + i / CPR, c = (i % CPR) * 8;
+        if (r < seq) *reinterpret_cast<uint4*>(to + (size_t)r * q_row_stride + c) = make_uint4(0, 0, 0, 0);
+      }
+    }
+    if (at >= groups) return;
+    const long first_row = kv_first ? max(0, min(*kv_first, kv_rows - kv_len)) : 0;
+    const size_t kv_at = (size_t)kvh * kv_head_stride + first_row * kv_row_stride;
+    prefill_few_rows<D, W * SPLIT>(smem_all, Q + (size_t)head * q_head_stride, K + kv_at, V + kv_at, O + (size_t)head * q_head_stride,
+                                   (groups - 1 - at) * 32, seq, q_tokens, kv_tokens, offset, scale_log2, causal, window,
+                                   q_row_stride, kv_row_stride);
+    return;
+  }
 
   const int my_q = q0 + wave * 32 + col;            // this lane's query row
   const bool q_live = my_q < q_tokens;
@@ -736,19 +962,29 @@ struct PrefillArgs {
 };
 
 // The stage buffers are dynamic LDS (more than the 64 KB a kernel may declare statically).
-template <int D, int SPLIT, int W = 4>
-static int launch_prefill(const PrefillArgs& a, int blocks, void* stream) {
+template <int D, int SPLIT, int W, bool FEW>
+static int launch_prefill_as(const PrefillArgs& a, int blocks, void* stream) {
   constexpr int STAGES = D == 64 && SPLIT == 1 ? 3 : 2;
   constexpr size_t lds = (size_t)SPLIT * STAGES * 2 * BKV * D * 2;
   static LdsOptIn opt_in;
-  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&mha_prefill_kernel<D, SPLIT, W>), lds); e != hipSuccess) {
+  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&mha_prefill_kernel<D, SPLIT, W, FEW>), lds); e != hipSuccess) {
     set_error("mha_prefill: %s", hipGetErrorString(e));
     return (int)e;
   }
-  hipLaunchKernelGGL((mha_prefill_kernel<D, SPLIT, W>), dim3(blocks), dim3(64 * W * SPLIT), lds, (hipStream_t)stream, a.Q,
+  hipLaunchKernelGGL((mha_prefill_kernel<D, SPLIT, W, FEW>), dim3(blocks), dim3(64 * W * SPLIT), lds, (hipStream_t)stream, a.Q,
                      a.K, a.V, a.O, a.heads, a.group, a.seq, a.seq_len, a.kv_len, a.scale_log2, a.causal, a.window,
                      a.q_row, a.q_head, a.kv_row, a.kv_head, a.valid, a.kv_valid, a.kv_first, a.kv_rows);
   return 0;
+}
+
+// Bounds read on the device may leave few queries; else the sizes say whether there are.
+template <int D, int SPLIT, int W = 4>
+static int launch_prefill(const PrefillArgs& a, int blocks, void* stream) {
+  const bool bounded = a.valid != nullptr || a.kv_valid != nullptr || a.seq_len != a.seq;
+  if (a.kv_len < 512 || (!bounded && !few_rows_pay<D>(blocks, a.kv_len))) return launch_prefill_as<D, SPLIT, W, false>(a, blocks, stream);
+  // (a launch so short that all its queries may go 32 to a block has a block for each 32)
+  const int groups = ((a.seq + 31) / 32) * a.heads;
+  return launch_prefill_as<D, SPLIT, W, true>(a, few_rows_pay<D>(blocks, a.kv_len) && groups > blocks ? groups : blocks, stream);
 }
 
 template <int D, int QN, int W>

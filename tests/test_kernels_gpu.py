@@ -787,6 +787,39 @@ def test_mha_prefill_longest_shape_on_sampled_queries(cuda):
         close(got[r : r + 1], want)
 
 
+@pytest.mark.parametrize("H,G,d,S,rows,L,keys,window,causal", [
+    (32, 8, 64, 2048, 40, 4096, 3001, None, True),     # a turn behind a history: two groups of queries, keys that end inside a tile
+    (32, 8, 64, 2048, 1, 2048, 512, None, True), (32, 8, 64, 2048, 512, 2048, 1024, None, True),   # the fewest and the most of each
+    (32, 8, 64, 2048, 300, 2048, 1700, 600, True), (16, 4, 64, 128, 33, 4096, 2000, None, False),
+    (12, 4, 64, 65, 65, 900, 900, 700, False), (8, 2, 128, 2048, 96, 4096, 1333, None, True),
+    (32, 8, 128, 40, 40, 3000, 3000, None, True), (4, 4, 128, 256, 129, 1024, 1024, 500, True),
+])
+def test_mha_prefill_of_few_rows_over_many_keys(cuda, H, G, d, S, rows, L, keys, window, causal):
+    """Few live queries: 32 a block, the keys dealt over its waves.  Every head of a sample of rows against the
+    oracle's attention of that one query over the keys its mask leaves it; rows past the bound are zero, and NaN past
+    either bound reaches nothing."""
+    rng = np.random.default_rng(rows + keys)
+    Q, Kc, Vc = bf(rng, S, H, d), bf(rng, L, G, d), bf(rng, L, G, d)
+    Q[rows:], Kc[keys:], Vc[keys:] = np.nan, np.nan, np.nan
+    O = out_like(Q.shape, cuda, fill=float("nan"))
+    bounds = {} if (rows, keys) == (S, L) else dict(valid=word(rows, cuda), kv_valid=word(keys, cuda))
+    K.mha_prefill(dev(Q, cuda), dev(Kc, cuda), dev(Vc, cuda), O, heads=H, kv_heads=G, d=d, seq=S, kv_len=L, causal=causal,
+                  window=window, q_interleaved=True, kv_interleaved=True, **bounds)
+    got = from_torch(O)
+    assert np.all(got[rows:] == 0)
+    masked = causal or window is not None
+    for r in sorted({0, rows - 1, min(31, rows - 1), min(32, rows - 1), *rng.integers(0, rows, 6).tolist()}):
+        at = keys - rows + r   # the query's position
+        last = at + 1 if causal else (min(keys, at + window + 1) if window is not None else keys)
+        first = max(0, at - window) if window is not None else 0
+        if not masked:
+            first, last = 0, keys
+        n = last - first
+        want = ops.mha(Q[r : r + 1], Kc[first:last], Vc[first:last], num_heads=H, num_KV_heads=G, seq_len=1, kv_len=n, d=d,
+                       causal=False, scale=d**-0.5, heads_interleaved=True, kv_interleaved=True)
+        close(got[r : r + 1], want)
+
+
 @pytest.mark.parametrize("rows", [512, 1500])
 def test_mha_prefill_bounded_chunk_at_the_decoder_s_width(cuda, rows):
     """A 2048-row prompt chunk of 32 heads under row and key bounds read on the device (512 rows
