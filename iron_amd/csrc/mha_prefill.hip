@@ -42,6 +42,8 @@ constexpr int kCUs = 256;                // compute units the block orders below
 template <int D>
 __host__ __device__ __forceinline__ bool few_rows_pay(int live, int keys) { return live <= (D == 64 ? 128 : 64) && keys >= 512; }
 constexpr int kFewBlocks = 512;          // launches of fewer blocks than this halve their blocks' queries (S = 1024 at 32 heads: 18.5 -> 13.9 us)
+constexpr int kFewBlocks128 = 360;       // d = 128: up to this many blocks of 64 queries a launch takes those (one a CU; 32 heads, 512 / 700 / 777
+                                         // queries 15.2 -> 12.3, 18.3 -> 17.4, 19.0 -> 20.0 us; 8 heads, 3001 46.5 -> 40.0)
 constexpr int kWideBigBlocks = 512;     // wide heads: launches of at least this many 128-query blocks keep that size
 constexpr int kSplitMaxBlocks = 1024;   // launches of up to this many blocks split each block's tiles over two halves
 
@@ -263,7 +265,7 @@ __device__ __forceinline__ void prefill_few_rows(
 // W: the waves that share a tile's loads, each with 32 of the block's 32 W queries.  Four; two
 // where four would leave CUs without a block (a short prompt), so that twice as many blocks go out.
 template <int D, int SPLIT, int W, bool FEW>
-__global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(W == 4 ? (D == 64 && SPLIT == 2 ? 4 : 2) : (D == 64 && SPLIT == 2 ? 2 : 1)))) void mha_prefill_kernel(
+__global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(W == 4 ? (D == 64 && SPLIT == 2 ? 4 : 2) : 2))) void mha_prefill_kernel(
     const bf16_t* __restrict__ Q, const bf16_t* __restrict__ K, const bf16_t* __restrict__ V,
     bf16_t* __restrict__ O, int heads, int group, int seq, int seq_len, int kv_len, float scale_log2,
     int causal, int window, long q_row_stride, long q_head_stride, long kv_row_stride,
@@ -1054,6 +1056,7 @@ static int mha_prefill(const uint16_t* Q, const uint16_t* K, const uint16_t* V, 
   // Fewer blocks of 128 queries than two a CU (a short prompt): blocks of 64, two waves a part.
   else if (d == 64 && blocks < kFewBlocks) rc = launch_prefill<64, 2, 2>(a, ((seq + 63) / 64) * heads, stream);
   else if (d == 64) rc = split ? launch_prefill<64, 2>(a, blocks, stream) : launch_prefill<64, 1>(a, blocks, stream);
+  else if (const int halves = ((seq + 63) / 64) * heads; halves <= kFewBlocks128) rc = launch_prefill<128, 2, 2>(a, halves, stream);
   else if (split) rc = launch_prefill<128, 2>(a, blocks, stream);
   else rc = launch_prefill<128, 1>(a, blocks, stream);
   if (rc != 0) return rc;

@@ -787,6 +787,24 @@ def test_mha_prefill_longest_shape_on_sampled_queries(cuda):
         close(got[r : r + 1], want)
 
 
+@pytest.mark.parametrize("H,G,S,window,causal", [(4, 2, 65, None, True), (4, 1, 200, 40, True), (2, 2, 1, None, True), (8, 2, 130, None, False),
+                                                 (12, 4, 700, 300, True)])
+def test_mha_prefill_128_wide_heads_of_short_prompts(cuda, H, G, S, window, causal):
+    """d = 128 in blocks of 64 queries: one query past a block, a block of one, and masks, against the oracle."""
+    rng = np.random.default_rng(S + H)
+    Q, Kc, Vc = bf(rng, S, H, 128), bf(rng, S, G, 128), bf(rng, S, G, 128)
+    O = out_like(Q.shape, cuda, fill=float("nan"))
+    K.mha_prefill(dev(Q, cuda), dev(Kc, cuda), dev(Vc, cuda), O, heads=H, kv_heads=G, d=128, seq=S, kv_len=S, causal=causal, window=window,
+                  q_interleaved=True, kv_interleaved=True)
+    got = from_torch(O)
+    for r in sorted({0, S - 1, min(63, S - 1), min(64, S - 1), *rng.integers(0, S, 8).tolist()}):
+        last = r + 1 if causal else S
+        first = max(0, r - window) if window is not None else 0
+        want = ops.mha(Q[r : r + 1], Kc[first:last], Vc[first:last], num_heads=H, num_KV_heads=G, seq_len=1, kv_len=last - first, d=128,
+                       causal=False, scale=128**-0.5, heads_interleaved=True, kv_interleaved=True)
+        close(got[r : r + 1], want)
+
+
 @pytest.mark.parametrize("H,G,d,S,rows,L,keys,window,causal", [
     (32, 8, 64, 2048, 40, 4096, 3001, None, True),     # a turn behind a history: two groups of queries, keys that end inside a tile
     (32, 8, 64, 2048, 1, 2048, 512, None, True), (32, 8, 64, 2048, 512, 2048, 1024, None, True),   # the fewest and the most of each
