@@ -201,6 +201,28 @@ def test_generation_through_the_entry_points():
     assert model.generate(prompts[0], 6) == model.generate_batch(prompts[:1], 6)[0]   # greedy again behind a sampler
 
 
+@pytest.mark.parametrize("lengths,slots,portions", [
+    ((3, 4, 1), 3, [8]),                       # all in one portion, to its last row
+    ((3, 6, 2), 3, [5, 6]),                    # a prompt that no longer fits waits for the next, a shorter one goes ahead
+    ((11, 5, 8), 3, [8, 8, 8]),                # whole portions of its own, and a rest that shares one
+    ((3, 4, 1), 2, [7, 1]),                    # as many at a time as there are slots
+])
+def test_prompts_of_a_batch_share_portions_uncut(lengths, slots, portions):
+    model, _ = host("mixed", slots=slots, prefill_chunk=8)
+    prompts = [tokens_of(model, n, seed=n) for n in lengths]
+    alone = [model.generate(p, 4) for p in prompts]
+    run, chunk = [], model.prompt_chunk
+
+    def counted(ids, **values):
+        run.append(values["rows"])
+        return chunk(ids, **values)
+
+    model.__dict__["prompt_chunk"] = counted
+    model.session.forget(0)
+    assert model.generate_batch(prompts, 4) == alone
+    assert run == portions
+
+
 def test_a_conversation_continues_and_starts_over():
     model, plain = host("odd")
     session, tokens = model.session, tokens_of(model, 20, seed=5)
