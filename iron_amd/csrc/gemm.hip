@@ -414,12 +414,14 @@ constexpr int NOWHERE = (int)0x80000000u;   // past stage_rows' 2^31 - 1 bytes, 
 // waits for the one before it).  Reading a k-step ahead, as the larger tiles do, left every MFMA
 // waiting for its operands: 600 cycles a stage.  STAGES = 4 (64 KB: a CU holds two blocks) where
 // the tiles outnumber the CUs, 8 (128 KB, more loads in flight) where a CU has one block anyway.
-// `qkv` carries only the optional residual epilogue here.
-template <int STAGES>
+// `qkv` carries only the optional residual epilogue here.  PAIR: both
+// first products of a gated feed-forward, 32 columns of each (`qkv` says the gate's kind).
+template <int STAGES, bool PAIR = false>
 __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
                                                bf16_t* __restrict__ C, int M, int N, int K,
                                                const int* __restrict__ valid, int tiles_m, int tiles_n,
-                                               int patched, const QkvTail& qkv) {
+                                               int patched, const QkvTail& qkv,
+                                               const bf16_t* __restrict__ up = nullptr, bf16_t* __restrict__ gate_out = nullptr) {
   constexpr int NT_BM = 64, NT_BN = 64;
   constexpr int NT_A_BYTES = NT_BM * BK * 2, NT_STAGE_BYTES = (NT_BM + NT_BN) * BK * 2;
   constexpr int INST = NT_BM / 8 / 4;  // 1 KB loads of A (and of B) a wave issues per stage
@@ -431,7 +433,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
 
   int tm, tn;
   if (!live_tile(blockIdx.x, tiles_m, tiles_n, patched, (Mv + NT_BM - 1) / NT_BM, tm, tn)) return;
-  const int m0 = tm * NT_BM, n0 = tn * NT_BN;
+  const int m0 = tm * NT_BM, n0 = tn * (PAIR ? NT_BN / 2 : NT_BN);
   if (m0 >= Mv) return;
 
   // The wave's number is uniform, so what depends on it (LDS destinations, the rows it loads) stays
@@ -447,11 +449,12 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
     head_ch[i] = lch * 8;
     // Rows past the end re-read the last row; what they produce is never stored.
     a_voff[i] = (int)(((size_t)(min(m0 + r, M - 1) - m0) * K + lch * 8) * 2);
-    b_voff[i] = (int)(((size_t)(min(n0 + r, N - 1) - n0) * K + lch * 8) * 2);
+    b_voff[i] = (int)(((size_t)(min(n0 + (PAIR ? r % (NT_BN / 2) : r), N - 1) - n0) * K + lch * 8) * 2);
   }
   const int pad = k_pad(K);
   const bf16_t* a_tile = A + (size_t)m0 * K - pad;
-  const bf16_t* b_tile = B + (size_t)n0 * K - pad;
+  // (PAIR: the tile's first 32 columns are the gate's, which waves 0 and 1 load and the waves wn = 0 compute, the rest the up projection's)
+  const bf16_t* b_tile = (PAIR && wave >= 2 ? up : B) + (size_t)n0 * K - pad;
   // One load of the 2*INST a wave issues per stage (A's first, then B's).
   auto issue_one = [&](char* st, int kt, int idx, bool head) {
     const int k0 = kt * BK;
@@ -474,11 +477,11 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
 
   // acc[e]: row fr of the wave's tile, column 8 (e/4) + 4 kh + e%4.
   const int fr = lane & 31, kh = lane >> 5;
-  const int m = m0 + wm * 32 + fr, nb = n0 + wn * 32 + 4 * kh;
+  const int m = m0 + wm * 32 + fr, nb = n0 + (PAIR ? 0 : wn * 32) + 4 * kh;
   // A residual's pieces this lane will add in the epilogue are requested now, so that their
   // latency passes under the whole product instead of at its end (N a multiple of 4: 8-byte pieces).
   uint2 res[4];
-  const bool res_ahead = qkv.residual != nullptr && (N & 3) == 0;
+  const bool res_ahead = !PAIR && qkv.residual != nullptr && (N & 3) == 0;
   if (res_ahead) {
 #pragma unroll
     for (int q = 0; q < 4; ++q)
@@ -538,13 +541,34 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
   wait_vmcnt<0>();  // the idle fetches of the last iterations land before the block's LDS is released
 #pragma unroll
   for (int e = 0; e < 16; ++e) acc[0][e] += acc[1][e];
+  if constexpr (PAIR) {
+    // The gate's waves leave their product, rounded as it is stored, in LDS for the others and store it; those make
+    // bf16(bf16(act(bf16 g)) * bf16 u) of it.
+    float* gates = reinterpret_cast<float*>(smem_nt) + (wm * 64 + lane) * 17;
+    block_barrier();   // every wave is done with the stages
+    if (wn == 0) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) gates[e] = acc[0][e] = round_bf16(acc[0][e]);
+    }
+    __syncthreads();
+    if (wn == 0) {
+      C = gate_out;
+    } else {
+      float x[16], g[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) x[e] = round_bf16(acc[0][e]), g[e] = gates[e];
+      tail_of(qkv, x, g);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[0][e] = x[e];
+    }
+  }
   const bool vec = (N & 3) == 0;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int n = nb + 8 * q;
     if (m >= Mv || n >= N) continue;
     bf16_t* p = C + (size_t)m * N + n;
-    if (qkv.residual != nullptr) {   // the product rounded as it would be stored, then scale * it + residual
+    if (!PAIR && qkv.residual != nullptr) {   // the product rounded as it would be stored, then scale * it + residual
       const bf16_t* r = qkv.residual + (size_t)m * N + n;
       float rf[4] = {0.f, 0.f, 0.f, 0.f};
       if (vec && n + 4 <= N) {
@@ -1819,13 +1843,16 @@ static int launch_gemm_either(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
 // down projection: 512 live rows x 2048 columns over K = 8192, then the next layer's input norm).
 // 128 x 128 tiles would occupy a quarter of the CUs and the 64 x 64 ones that fill the chip fetch
 // every operand row twice as often, so a tile's K is dealt over `splits` blocks -- chosen on the
-// device by the row bound: 4 while the live tiles fill a quarter of the chip, 2 up to half, else
+// device by the row bound: 16, 8 and 4 while the live tiles fill that part of the chip, 2 up to half, else
 // whole K -- each leaving its float32 sums in a workspace slice.  A second launch, a block a row,
 // adds a row's slices in slice order (the same sums whatever ran first), rounds once, adds the
 // residual, stores the row and norms it as rmsnorm_kernel does: that launch stands where the
 // norm's own stood, so the slices' sum costs no launch of its own.
-constexpr int kSplitKMax = 4;
-__device__ __host__ inline int splitk_for(int live_tiles) {
+constexpr int kSplitKMax = 4;    // slices the second launch asks for at a time, and every K can be cut into
+__device__ __host__ inline int splitk_for(int live_tiles, int K) {
+  // Past four slices while the chip would idle and a slice keeps eight stages (29 rows x 2048 x 8192 with the norm 17.4 -> 14.0 us, 128 rows 19.8 -> 17.9).
+  if (live_tiles * 16 <= 256 && K % (16 * 8 * BK) == 0) return 16;
+  if (live_tiles * 8 <= 256 && K % (8 * 8 * BK) == 0) return 8;
   return live_tiles * 4 <= 256 ? 4 : (live_tiles * 2 <= 256 ? 2 : 1);
 }
 // Rows a slice of the workspace holds when K is dealt `splits` ways: the most that split count runs for.
@@ -1839,7 +1866,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_kernel(const bf16_t* __restri
                                                           float* __restrict__ partial) {
   const int Mv = bound_or(valid, M);
   const int tiles_n = whole.tiles_n, live_tiles = ((Mv + 127) / 128) * tiles_n;
-  const int splits = splitk_for(live_tiles), id = blockIdx.x;
+  const int splits = splitk_for(live_tiles, K), id = blockIdx.x;
   if (splits == 1) {   // whole K a block, the residual in its epilogue: iron_gemm_residual_bf16's 128 x 128 launch
     if (id < whole.tiles_m * whole.tiles_n)
       gemm_nt16_body<false>(A, B, C, M, N, K, valid, whole.tiles_m, whole.tiles_n, whole.patched, tail);
@@ -1851,7 +1878,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_kernel(const bf16_t* __restri
   const int live = live_tiles * splits;
   if (id >= live) return;
   int tile, split;
-  if (live % 8 == 0) {
+  if (live % 8 == 0 && splits <= 8) {
     const int xcd = id & 7, per = 8 / splits;
     split = xcd % splits;
     tile = (id >> 3) * per + xcd / splits;
@@ -1877,7 +1904,7 @@ __global__ __launch_bounds__(256) void gemm_finish_rows_kernel(const float* __re
                                                                const bf16_t* residual, float scale, bf16_t* C,
                                                                const bf16_t* __restrict__ gain,
                                                                bf16_t* __restrict__ Y, int M, int N, float eps,
-                                                               const int* __restrict__ valid, int tiles_n) {
+                                                               const int* __restrict__ valid, int tiles_n, int K) {
   const int row = blockIdx.x, nchunk = N >> 3;
   const __amdgpu_buffer_rsrc_t gain_bytes = bounded_bytes(gain, N * 2);
   uint4 gains[CHUNKS];
@@ -1885,7 +1912,7 @@ __global__ __launch_bounds__(256) void gemm_finish_rows_kernel(const float* __re
   for (int i = 0; i < CHUNKS; ++i) gains[i] = load_bounded(gain_bytes, 16 * (threadIdx.x + 256 * i));
   const int Mv = bound_or(valid, M);
   if (row >= Mv) return;
-  const int splits = splitk_for(((Mv + 127) / 128) * tiles_n);
+  const int splits = splitk_for(((Mv + 127) / 128) * tiles_n, K);
   uint4* c_row = reinterpret_cast<uint4*>(C + (size_t)row * N);
   uint4 held[CHUNKS];
   if (splits == 1) {
@@ -1896,30 +1923,47 @@ __global__ __launch_bounds__(256) void gemm_finish_rows_kernel(const float* __re
     const size_t slice = splitk_slice_rows(splits, tiles_n) * N;
     const __amdgpu_buffer_rsrc_t res_bytes = bounded_bytes(residual + (size_t)row * N, N * 2);
     uint4 added[CHUNKS], part[CHUNKS][kSplitKMax][2];
+    // Slices first .. first + 3 of every piece, all requested before any is used.
+    auto request = [&](int first) {
 #pragma unroll
-    for (int i = 0; i < CHUNKS; ++i) {
-      added[i] = load_bounded(res_bytes, 16 * (threadIdx.x + 256 * i));
+      for (int i = 0; i < CHUNKS; ++i)
 #pragma unroll
-      for (int sl = 0; sl < kSplitKMax; ++sl) {
-        // slices past the split count: an empty buffer, zeros
-        const __amdgpu_buffer_rsrc_t sums = bounded_bytes(partial + (sl < splits ? sl : 0) * slice + (size_t)row * N,
-                                                          sl < splits ? N * 4 : 0);
-        part[i][sl][0] = load_bounded(sums, 32 * (threadIdx.x + 256 * i));
-        part[i][sl][1] = load_bounded(sums, 32 * (threadIdx.x + 256 * i) + 16);
+        for (int sl = 0; sl < kSplitKMax; ++sl) {
+          // slices past the split count: an empty buffer, zeros
+          const bool there = first + sl < splits;
+          const __amdgpu_buffer_rsrc_t sums = bounded_bytes(partial + (there ? first + sl : 0) * slice + (size_t)row * N,
+                                                            there ? N * 4 : 0);
+          part[i][sl][0] = load_bounded(sums, 32 * (threadIdx.x + 256 * i));
+          part[i][sl][1] = load_bounded(sums, 32 * (threadIdx.x + 256 * i) + 16);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < CHUNKS; ++i) added[i] = load_bounded(res_bytes, 16 * (threadIdx.x + 256 * i));
+    request(0);
+    f32x4 sum[CHUNKS][2];
+#pragma unroll
+    for (int i = 0; i < CHUNKS; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        sum[i][h] = __builtin_bit_cast(f32x4, part[i][0][h]);
+#pragma unroll
+        for (int sl = 1; sl < kSplitKMax; ++sl)
+          if (sl < splits) sum[i][h] += __builtin_bit_cast(f32x4, part[i][sl][h]);
       }
+    for (int first = kSplitKMax; first < splits; first += kSplitKMax) {   // (past four, the split count is a multiple of it)
+      request(first);
+#pragma unroll
+      for (int i = 0; i < CHUNKS; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int sl = 0; sl < kSplitKMax; ++sl) sum[i][h] += __builtin_bit_cast(f32x4, part[i][sl][h]);
     }
 #pragma unroll
     for (int i = 0; i < CHUNKS; ++i) {
       float x[8], rf[8];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        f32x4 sum = __builtin_bit_cast(f32x4, part[i][0][h]);
-#pragma unroll
-        for (int sl = 1; sl < kSplitKMax; ++sl)
-          if (sl < splits) sum += __builtin_bit_cast(f32x4, part[i][sl][h]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) x[4 * h + e] = sum[e];
-      }
+      for (int e = 0; e < 8; ++e) x[e] = sum[i][e >> 2][e & 3];
       unpack8(added[i], rf);
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] = fmaf(scale, round_bf16(x[e]), rf[e]);
@@ -2160,10 +2204,9 @@ __device__ __forceinline__ void gemm_nt16_pair_body(const bf16_t* __restrict__ A
 }
 
 // A gated feed-forward's two first projections over many rows as ONE launch, the tile chosen on the
-// device by the row bound as in gemm_either_kernel.  Few rows: 64 x 64 tiles, a block's gate tile first,
-// then the same tile of the second product, whose epilogue reads the gate tile back -- the one this
-// very block wrote, so nothing crosses between blocks.  Up to one round of them, 128 x 128 tiles of
-// both products at once.  Past that 256 rows x (128 + 128) columns, a wave's 128 x 128 half gate and half up
+// device by the row bound as in gemm_either_kernel.  Few rows: 64 rows x (32 + 32) columns on the 64 x 64 tile's
+// loop, two waves a product (29 x 8192 x 2048 29.7 -> 20.5 us: as a gate tile and then an up tile a block made
+// two chains of stages).  Up to one round of them, 128 x 128 tiles of both products at once.  Past that 256 rows x (128 + 128) columns, a wave's 128 x 128 half gate and half up
 // projection: the bytes a CU draws from L2 per flop are those of a 256 x 256 tile, two thirds of the smaller pair's.
 // A round of the large tiles takes 1.5 rounds of the small ones and covers two (N = 8192, K = 2048: 2048
 // rows 161 -> 130 us, 1024 89 -> 65, 1281 118 -> 113; 512 rows, on the small tiles, 46.5 -> 41.8 by asking the kind of gate once).
@@ -2174,8 +2217,7 @@ __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __re
                                                               const int* __restrict__ valid, Tiling t256, Tiling t128,
                                                               Tiling t64, int few256, int few128, int activation) {
   const int Mv = bound_or(valid, M), bid = blockIdx.x;
-  QkvTail none{}, gate{};
-  gate.residual = G;
+  QkvTail gate{};
   gate.gated = activation;
   if (Mv > few256) {
     if (bid >= t256.tiles_m * t256.tiles_n) return;
@@ -2186,15 +2228,13 @@ __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __re
     gemm_nt16_pair_body(A, Bg, Bu, G, C, M, N, K, valid, t128.tiles_m, t128.tiles_n, t128.patched, activation);
   } else {
     if (bid >= t64.tiles_m * t64.tiles_n) return;
-    gemm_nt64_body<8>(A, Bg, G, M, N, K, valid, t64.tiles_m, t64.tiles_n, t64.patched, none);
-    __syncthreads();
-    gemm_nt64_body<8>(A, Bu, C, M, N, K, valid, t64.tiles_m, t64.tiles_n, t64.patched, gate);
+    gemm_nt64_body<8, true>(A, Bg, C, M, N, K, valid, t64.tiles_m, t64.tiles_n, t64.patched, gate, Bu, G);
   }
 }
 
 static int launch_gemm_gated_pair(const bf16_t* A, const bf16_t* Bg, const bf16_t* Bu, bf16_t* G, bf16_t* C, int M,
                                   int N, int K, const int* valid, int activation, hipStream_t s) {
-  const int n128 = (N + 127) / 128, n64 = (N + 63) / 64;
+  const int n128 = (N + 127) / 128, n32 = (N + 31) / 32;
   // 64 x 64 tiles up to the rows below which 128 x 128 ones would leave half the CUs idle (as iron_gemm_bf16),
   // 256 x (128 + 128) ones past the rows that one round of 128 x 128 ones covers.
   int few128 = n128 >= 128 ? 0 : 128 * (127 / n128);
@@ -2207,7 +2247,7 @@ static int launch_gemm_gated_pair(const bf16_t* A, const bf16_t* Bg, const bf16_
     return Tiling{tile_rows, tile_cols, patched_order(tile_rows, tile_cols)};
   };
   const Tiling t256 = few256 < M ? tiling((M + BIG_BM - 1) / BIG_BM, n128) : Tiling{0, 0, 0};
-  const Tiling t128 = tiling((few256 + 127) / 128, n128), t64 = tiling((few128 + 63) / 64, n64);
+  const Tiling t128 = tiling((few256 + 127) / 128, n128), t64 = tiling((few128 + 63) / 64, n32);
   constexpr size_t lds = (size_t)PAIR_STAGES * 3 * 128 * BK * 2;   // the two-product body's stages, more than the others'
   static_assert(lds >= (size_t)NT_STAGES * 256 * BK * 2, "the 64 x 64 body's stages fit too");
   static LdsOptIn opt_in;
@@ -2605,7 +2645,7 @@ extern "C" int iron_gemm_residual_norm_bf16(const uint16_t* A, const uint16_t* B
   const int chunks = (N / 8 + 255) / 256;
 #define IRON_FINISH(CH)                                                                                          \
   hipLaunchKernelGGL((gemm_finish_rows_kernel<CH>), dim3(M), dim3(256), 0, s, (const float*)workspace, R,        \
-                     residual_scale, C, gain, Y, M, N, eps, valid, tiles_n)
+                     residual_scale, C, gain, Y, M, N, eps, valid, tiles_n, K)
   if (chunks <= 1) IRON_FINISH(1);
   else if (chunks == 2) IRON_FINISH(2);
   else IRON_FINISH(4);
