@@ -838,6 +838,32 @@ def test_mha_prefill_of_few_rows_over_many_keys(cuda, H, G, d, S, rows, L, keys,
         close(got[r : r + 1], want)
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("interleaved", [True, False])
+def test_mha_prefill_of_few_rows_in_both_layouts_and_a_window_of_a_buffer(cuda, d, interleaved):
+    """The few-row form over keys stored head by head or row by row, and over a run of a longer buffer's rows: the same bits."""
+    rng = np.random.default_rng(d)
+    H, G, S, L, first, rows, keys = 8, 2, 512, 1024, 37, 45, 800
+    Q, Kc, Vc = (torch.from_numpy(x).to(cuda).bfloat16() for x in (bf(rng, S, H, d), bf(rng, L, G, d), bf(rng, L, G, d)))
+    kw = dict(heads=H, kv_heads=G, d=d, seq=S, kv_len=L, valid=word(rows, cuda), kv_valid=word(keys, cuda))
+    plain, other = torch.empty_like(Q), torch.empty_like(Q)
+    K.mha_prefill(Q, Kc, Vc, plain, q_interleaved=True, kv_interleaved=True, **kw)
+    want = ops.mha(from_torch(Q)[44:45], from_torch(Kc)[:keys], from_torch(Vc)[:keys], num_heads=H, num_KV_heads=G, seq_len=1, kv_len=keys, d=d,
+                   causal=False, scale=d**-0.5, heads_interleaved=True, kv_interleaved=True)
+    close(from_torch(plain)[44:45], want)
+    if interleaved:
+        held = [torch.full((L + 100, G, d), float("nan"), dtype=torch.bfloat16, device=cuda) for _ in range(2)]
+        for buf, x in zip(held, (Kc, Vc)):
+            buf[first : first + L] = x
+        K.mha_prefill(Q, *held, other, q_interleaved=True, kv_interleaved=True, kv_first=word(first, cuda), kv_rows=L + 100, **kw)
+    else:
+        by_head = torch.empty(H, S, d, dtype=torch.bfloat16, device=cuda)
+        K.mha_prefill(Q.transpose(0, 1).contiguous(), Kc.transpose(0, 1).contiguous(), Vc.transpose(0, 1).contiguous(), by_head,
+                      q_interleaved=False, kv_interleaved=False, **kw)
+        other = by_head.transpose(0, 1)
+    assert torch.equal(plain, other)
+
+
 @pytest.mark.parametrize("rows", [512, 1500])
 def test_mha_prefill_bounded_chunk_at_the_decoder_s_width(cuda, rows):
     """A 2048-row prompt chunk of 32 heads under row and key bounds read on the device (512 rows
