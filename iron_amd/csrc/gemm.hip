@@ -405,15 +405,16 @@ constexpr int NOWHERE = (int)0x80000000u;   // past stage_rows' 2^31 - 1 bytes, 
 
 // 64 x 64 tiles, B as (N,K), for problems -- or row bounds -- whose 128 x 128 tiles would leave CUs
 // idle (k/v projections, short chunks): the direct-to-LDS pipeline of the 128 x 128 kernel below
-// (buffer loads, XOR-swizzled chunks) with a wave owning one 32x32x16 MFMA tile.  A stage is four
+// (buffer loads, XOR-swizzled chunks) with a wave owning 2 x 2 tiles of 16x16x32 MFMAs.  A stage is eight
 // MFMAs of a wave, far less than an LDS read takes to return, so the fragments of a WHOLE stage
 // are read one stage ahead into a second register set: at the top of stage kt the stage's one
-// barrier (stage kt+1 has landed in every wave, and nobody reads stage kt-1 any more), then the
-// eight fragment reads of stage kt+1, the loads of stage kt+STAGES-1 into stage kt-1's buffer, and
-// stage kt's four MFMAs out of registers on two accumulators (even and odd k-steps, so that no MFMA
-// waits for the one before it).  Reading a k-step ahead, as the larger tiles do, left every MFMA
+// barrier (stage kt+1 has landed in every wave, and nobody reads stage kt-1 any more) behind its first two
+// MFMAs, then, between the others, the eight fragment reads of stage kt+1 and the loads of stage kt+STAGES-1 into stage
+// kt-1's buffer.  Reading a k-step ahead, as the larger tiles do, left every MFMA
 // waiting for its operands: 600 cycles a stage.  STAGES = 4 (64 KB: a CU holds two blocks) where
 // the tiles outnumber the CUs, 8 (128 KB, more loads in flight) where a CU has one block anyway.
+// An element's sum is the same chain of 32-wide k-steps as in the 128 x 128 and the 256 x 256 tiles: where a row bound chooses
+// the tile, a row's products are the same bits whatever rows share the launch.
 // `qkv` carries only the optional residual epilogue here.  PAIR: both
 // first products of a gated feed-forward, 32 columns of each (`qkv` says the gate's kind).
 template <int STAGES, bool PAIR = false>
@@ -426,8 +427,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
   constexpr int NT_A_BYTES = NT_BM * BK * 2, NT_STAGE_BYTES = (NT_BM + NT_BN) * BK * 2;
   constexpr int INST = NT_BM / 8 / 4;  // 1 KB loads of A (and of B) a wave issues per stage
   constexpr int LOADS = 2 * INST;
-  constexpr int KSTEPS = BK / 16;
-  static_assert(LOADS == KSTEPS && STAGES >= 4, "one load rides each k-step's MFMA");
+  static_assert(BK == 64 && LOADS == 4 && STAGES >= 4, "two 32-wide k-steps a stage, a load behind every second MFMA");
   extern __shared__ __align__(16) char smem_nt[];
   const int Mv = bound_or(valid, M);
 
@@ -469,23 +469,23 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
     }
   };
 
-  f32x16 acc[2];
+  f32x4 acc[2][2];
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[h][e] = 0.f;
+  for (int t = 0; t < 4; ++t) acc[t >> 1][t & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // acc[e]: row fr of the wave's tile, column 8 (e/4) + 4 kh + e%4.
-  const int fr = lane & 31, kh = lane >> 5;
-  const int m = m0 + wm * 32 + fr, nb = n0 + (PAIR ? 0 : wn * 32) + 4 * kh;
+  // acc[i][j][e]: row 16 i + fr of the wave's 32 x 32, column 16 j + 4 kq + e.
+  const int fr = lane & 15, kq = lane >> 4;
+  const int mb = m0 + wm * 32 + fr, nb = n0 + (PAIR ? 0 : wn * 32) + 4 * kq;
   // A residual's pieces this lane will add in the epilogue are requested now, so that their
   // latency passes under the whole product instead of at its end (N a multiple of 4: 8-byte pieces).
-  uint2 res[4];
+  uint2 res[2][2];
   const bool res_ahead = !PAIR && qkv.residual != nullptr && (N & 3) == 0;
   if (res_ahead) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      res[q] = *reinterpret_cast<const uint2*>(qkv.residual + (size_t)min(m, M - 1) * N + min(nb + 8 * q, N - 4));
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        res[i][j] = *reinterpret_cast<const uint2*>(qkv.residual + (size_t)min(mb + 16 * i, M - 1) * N + min(nb + 16 * j, N - 4));
   }
 
   const int nk = (K + pad) / BK;
@@ -496,38 +496,46 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
 #pragma unroll
     for (int idx = 0; idx < LOADS; ++idx) issue_one(smem_nt + s * NT_STAGE_BYTES, min(s, nk - 1), idx, s == 0);
 
-  const int ra = wm * 32 + fr, rb = wn * 32 + fr;
-  const int a_off = ra * 128, a_swz = (ra >> 1) & 7, b_off = NT_A_BYTES + rb * 128, b_swz = (rb >> 1) & 7;
-  auto a_frag = [&](const char* st, int ks) {
-    return *reinterpret_cast<const bf16x8*>(st + a_off + (((ks * 2 + kh) ^ a_swz) << 4));
+  // Fragments: lane -> row fr of a 16-row tile, 16-byte chunk kq of the k-step's four.
+  const int a_off = (wm * 32 + fr) * 128, b_off = NT_A_BYTES + (wn * 32 + fr) * 128, swz = (fr >> 1) & 7;
+  auto a_frag = [&](const char* st, int ks, int i) {
+    return *reinterpret_cast<const bf16x8*>(st + a_off + i * 16 * 128 + (((ks * 4 + kq) ^ swz) << 4));
   };
-  auto b_frag = [&](const char* st, int ks) {
-    return *reinterpret_cast<const bf16x8*>(st + b_off + (((ks * 2 + kh) ^ b_swz) << 4));
+  auto b_frag = [&](const char* st, int ks, int j) {
+    return *reinterpret_cast<const bf16x8*>(st + b_off + j * 16 * 128 + (((ks * 4 + kq) ^ swz) << 4));
   };
 
   wait_vmcnt<(STAGES - 2) * LOADS>();   // stage 0 has landed once only the younger ones are out
   block_barrier();
-  bf16x8 af[2][KSTEPS], bfr[2][KSTEPS];   // [stage parity][k-step]
+  bf16x8 af[2][2][2], bfr[2][2][2];   // [stage parity][k-step][tile]
 #pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks) { af[0][ks] = a_frag(smem_nt, ks); bfr[0][ks] = b_frag(smem_nt, ks); }
+  for (int t = 0; t < 4; ++t) {
+    af[0][t >> 1][t & 1] = a_frag(smem_nt, t >> 1, t & 1);
+    bfr[0][t >> 1][t & 1] = b_frag(smem_nt, t >> 1, t & 1);
+  }
   // Two stages an iteration, so that the register sets are named at compile time.
   auto stage = [&](int kt, auto parity) {
     constexpr int P = decltype(parity)::value;
-    // Of this wave's loads in flight the oldest LOADS are stage kt+1's; the STAGES-3 stages after it may stay out.
-    wait_vmcnt<(STAGES - 3) * LOADS>();
-    block_barrier();
     const char* st1 = smem_nt + ((kt + 1) % STAGES) * NT_STAGE_BYTES;     // past the end: a stage nobody needs
     char* nst = smem_nt + ((kt + STAGES - 1) % STAGES) * NT_STAGE_BYTES;  // stage kt-1's buffer
     const int kn = min(kt + STAGES - 1, nk - 1);   // past the end the last stage again: the wait counts stay exact
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-      acc[ks & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[P][ks], af[P][ks], acc[ks & 1], 0, 0, 0);
+    for (int t = 0; t < 4; ++t) {
+      const int ks = t >> 1, i = t & 1;
+      mfma_16x16x32_in_place(acc[i][0], bfr[P][ks][0], af[P][ks][i]);
+      mfma_16x16x32_in_place(acc[i][1], bfr[P][ks][1], af[P][ks][i]);
       __builtin_amdgcn_sched_barrier(0);
-      af[P ^ 1][ks] = a_frag(st1, ks);
-      bfr[P ^ 1][ks] = b_frag(st1, ks);
-      issue_one(nst, kn, ks, false);
-      __builtin_amdgcn_sched_barrier(0);
+      if (t == 0) {   // (behind the first products, which the waves wait under: 300 x 512 x 2048 8.1 -> 7.8 us)
+        // Of this wave's loads in flight the oldest LOADS are stage kt+1's; the STAGES-3 stages after it may stay out.
+        wait_vmcnt<(STAGES - 3) * LOADS>();
+        block_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      af[P ^ 1][ks][i] = a_frag(st1, ks, i);
+      bfr[P ^ 1][ks][i] = b_frag(st1, ks, i);
+      issue_one(nst, kn, t, false);
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
   // (Unrolled over all its stage buffers, so that a fragment's stage rides in its read's offset
   // field as in the 128 x 128 loop, this loop measured the same: it waits for L2, not for issue slots.)
@@ -539,8 +547,8 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
   if (kt < nk) stage(kt, std::integral_constant<int, 0>{});
 
   wait_vmcnt<0>();  // the idle fetches of the last iterations land before the block's LDS is released
-#pragma unroll
-  for (int e = 0; e < 16; ++e) acc[0][e] += acc[1][e];
+  // (the matrix cores' last results: the compiler does not know what the assembly's are)
+  asm volatile("s_nop 15\n\ts_nop 3" : "+a"(acc[0][0]), "+a"(acc[0][1]), "+a"(acc[1][0]), "+a"(acc[1][1]));
   if constexpr (PAIR) {
     // The gate's waves leave their product, rounded as it is stored, in LDS for the others and store it; those make
     // bf16(bf16(act(bf16 g)) * bf16 u) of it.
@@ -548,7 +556,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
     block_barrier();   // every wave is done with the stages
     if (wn == 0) {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) gates[e] = acc[0][e] = round_bf16(acc[0][e]);
+      for (int e = 0; e < 16; ++e) gates[e] = acc[e >> 3][(e >> 2) & 1][e & 3] = round_bf16(acc[e >> 3][(e >> 2) & 1][e & 3]);
     }
     __syncthreads();
     if (wn == 0) {
@@ -556,46 +564,47 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
     } else {
       float x[16], g[16];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) x[e] = round_bf16(acc[0][e]), g[e] = gates[e];
+      for (int e = 0; e < 16; ++e) x[e] = round_bf16(acc[e >> 3][(e >> 2) & 1][e & 3]), g[e] = gates[e];
       tail_of(qkv, x, g);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[0][e] = x[e];
+      for (int e = 0; e < 16; ++e) acc[e >> 3][(e >> 2) & 1][e & 3] = x[e];
     }
   }
   const bool vec = (N & 3) == 0;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int n = nb + 8 * q;
-    if (m >= Mv || n >= N) continue;
-    bf16_t* p = C + (size_t)m * N + n;
-    if (!PAIR && qkv.residual != nullptr) {   // the product rounded as it would be stored, then scale * it + residual
-      const bf16_t* r = qkv.residual + (size_t)m * N + n;
-      float rf[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int m = mb + 16 * i, n = nb + 16 * j;
+      if (m >= Mv || n >= N) continue;
+      bf16_t* p = C + (size_t)m * N + n;
+      if (!PAIR && qkv.residual != nullptr) {   // the product rounded as it would be stored, then scale * it + residual
+        const bf16_t* r = qkv.residual + (size_t)m * N + n;
+        float rf[4] = {0.f, 0.f, 0.f, 0.f};
+        if (vec && n + 4 <= N) {
+          const uint2 rv = res_ahead ? res[i][j] : *reinterpret_cast<const uint2*>(r);
+          rf[0] = __uint_as_float(rv.x << 16); rf[1] = __uint_as_float(rv.x & 0xffff0000u);
+          rf[2] = __uint_as_float(rv.y << 16); rf[3] = __uint_as_float(rv.y & 0xffff0000u);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) rf[e] = bf16_to_f32(r[e]);
+        }
+        float prod[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) prod[e] = round_bf16(acc[i][j][e]);
+        tail_of(qkv, prod, rf);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][j][e] = prod[e];
+      }
       if (vec && n + 4 <= N) {
-        const uint2 rv = res_ahead ? res[q] : *reinterpret_cast<const uint2*>(r);
-        rf[0] = __uint_as_float(rv.x << 16); rf[1] = __uint_as_float(rv.x & 0xffff0000u);
-        rf[2] = __uint_as_float(rv.y << 16); rf[3] = __uint_as_float(rv.y & 0xffff0000u);
+        *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16(acc[i][j][0], acc[i][j][1]), pack_bf16(acc[i][j][2], acc[i][j][3]));
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (n + e < N) rf[e] = bf16_to_f32(r[e]);
+          if (n + e < N) p[e] = f32_to_bf16(acc[i][j][e]);
       }
-      float prod[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) prod[e] = round_bf16(acc[0][4 * q + e]);
-      tail_of(qkv, prod, rf);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[0][4 * q + e] = prod[e];
     }
-    if (vec && n + 4 <= N) {
-      *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16(acc[0][4 * q], acc[0][4 * q + 1]),
-                                                pack_bf16(acc[0][4 * q + 2], acc[0][4 * q + 3]));
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (n + e < N) p[e] = f32_to_bf16(acc[0][4 * q + e]);
-    }
-  }
 }
 
 // 128 x 128 x 64 tiles, four stages of 32 KB fed straight from global memory into LDS (buffer loads:

@@ -153,8 +153,8 @@ class Batch:
         return [rows[[self.slots[e.key]] * len(e.want)] for e in entries]
 
     def _portions(self, entries, ids, whole: bool = False) -> list[np.ndarray]:
-        """``whole``: a request's tokens are cut only where they would be alone, so that what it is told does not depend
-        on what else is run."""
+        """``whole``: a request's tokens are cut only where they would be alone.  A portion's kernels make a row by the same
+        sums whatever rows are beside it, so what a request is told then does not depend, to the bit, on what else is run."""
         model, c = self.lm, self.lm.config
         done = [0] * len(entries)
         room = c.key_room

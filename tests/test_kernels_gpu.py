@@ -282,6 +282,34 @@ def test_gemm_small_tiles_at_every_depth(cuda, M, Kdim, N, rows, residual):
     assert np.all(got[lim:] == 5.0)
 
 
+@pytest.mark.parametrize("M,Kdim,N,form", [(*s, f) for s in ((2048, 2048, 2048), (2048, 1024, 8192), (1500, 320, 4160))
+                                           for f in ("plain", "residual", "gated", "pair")] + [(2048, 200, 8192, "plain")])
+def test_a_row_s_products_are_the_same_bits_under_every_bound(cuda, M, Kdim, N, form):
+    """A bound on the rows chooses the tile (64, 128 or 256 rows of it), and with it nothing about a row's sums: what a row
+    becomes does not depend on how many others there are."""
+    rng = np.random.default_rng(M + N)
+    A, B, B2, R = (dev(bf(rng, *s, scale=x), cuda) for s, x in (((M, Kdim), 1.0), ((N, Kdim), 0.05), ((N, Kdim), 0.05), ((M, N), 1.0)))
+    kw = dict(M=M, N=N, K=Kdim)
+
+    def run(rows):
+        C, G = out_like((M, N), cuda, fill=7.0), out_like((M, N), cuda, fill=7.0)
+        if form == "plain":
+            K.gemm(A, B, C, b_col_maj=True, valid=word(rows, cuda), **kw)
+        elif form == "residual":
+            K.gemm_residual(A, B, R, C, residual_scale=0.5, valid=word(rows, cuda), **kw)
+        elif form == "gated":
+            K.gemm_gated(A, B, R, C, activation="silu", valid=word(rows, cuda), **kw)
+        else:
+            K.gemm_gated_pair(A, B, B2, G, C, activation="silu", valid=word(rows, cuda), **kw)
+        return C, G
+
+    whole = run(M)
+    for rows in (5, 64, 128, 129, 256, 257, 384, 385, 513, 896, 897, 1025):
+        for got, want in zip(run(rows), whole):
+            assert torch.equal(got[:rows], want[:rows]), rows
+            assert (got[rows:] == 7).all(), rows
+
+
 @pytest.mark.parametrize("rows,bound,H,G", [(2048, None, 32, 8), (256, 150, 16, 4), (128, None, 2, 2),
                                             # bounds on either side of where the 192-wide tiles take over
                                             (2048, 1280, 32, 8), (2048, 1281, 32, 8), (2048, 1999, 32, 8),
