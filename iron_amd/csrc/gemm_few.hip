@@ -21,6 +21,7 @@ namespace iron {
 // gemm_few_kernel and with this: 2048 x 2048 5.1 / 4.1, 2048 x 8192 14.1 / 9.3, 4160 x 2048 8.0 / 6.0, 8192 x 2048 10.2 / 8.8,
 // 10240 x 2048 15.0 / 10.3, 128256 x 2048 106 / 86 (6.1 TB/s); thirty-two rows: 4160 x 2048 14.3 / 9.6, 128256 x 2048 163 / 92.
 constexpr int STRIP = 256, STRIP_BYTES = 512, STRIP_WAVES = 8, STRIP_ROWS = 8;
+constexpr unsigned STRIP_BLOCKS = 256;   // one a CU; fewer tiles: a block each
 constexpr int STRIP_OUT = 64;   // columns of C staged for a store of whole lines: 128256 x 2048 98 -> 86 us with the loads past the caches
 
 __device__ __forceinline__ void lds_write_b128(unsigned addr, const f32x4& v) { asm volatile("ds_write_b128 %0, %1" ::"v"(addr), "v"(v) : "memory"); }
@@ -48,8 +49,10 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l16 = lane & 15, quad = lane >> 4;
   const int strips = (K + STRIP - 1) / STRIP, mine = SINGLE ? 1 : (strips - wave + W - 1) / W, most = SINGLE ? 1 : (strips + W - 1) / W;
   // A block's tiles are neighbours, so that its columns of C leave as whole lines.
-  const unsigned tiles = (N + R - 1) / R;   // (up to 2^19, the blocks 256)
-  const int tile0 = blockIdx.x * tiles / gridDim.x, my_tiles = (blockIdx.x + 1) * tiles / gridDim.x - tile0, items = my_tiles * mine;
+  // (64 bits: 256 times the tiles of an N of 2^27 pass 32)
+  const unsigned tiles = ((unsigned)N + R - 1) / R;
+  auto first_tile = [&](unsigned block) { return (int)(tiles < STRIP_BLOCKS ? block : (unsigned long long)block * tiles / STRIP_BLOCKS); };
+  const int tile0 = first_tile(blockIdx.x), my_tiles = first_tile(blockIdx.x + 1) - tile0, items = my_tiles * mine;
   char* const own = lds + wave * S::WAVE;
   char* const held = own + (SINGLE ? S::A_BYTES : 0);
   const unsigned lds0 = (unsigned)(uintptr_t)IRON_LDS_PTR(lds), part0 = lds0 + W * S::WAVE, out0 = part0 + 2 * S::PART;
@@ -319,8 +322,8 @@ static int launch_gemm_strips(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
     set_error("gemm_few: %s", hipGetErrorString(e));
     return (int)e;
   }
-  const int tiles = (N + STRIP_ROWS - 1) / STRIP_ROWS;
-  hipLaunchKernelGGL(kernel, dim3(tiles < 256 ? tiles : 256), dim3(STRIP_WAVES * 64), S::LDS, s, A, B, C, M, N, K);
+  const unsigned tiles = ((unsigned)N + STRIP_ROWS - 1) / STRIP_ROWS;
+  hipLaunchKernelGGL(kernel, dim3(tiles < STRIP_BLOCKS ? tiles : STRIP_BLOCKS), dim3(STRIP_WAVES * 64), S::LDS, s, A, B, C, M, N, K);
   IRON_LAUNCH_CHECK();
 }
 

@@ -109,6 +109,20 @@ def test_a_product_over_few_rows_by_strips(cuda, M, N, K_):
     assert (got[M] == 7).all()
 
 
+def test_a_product_over_few_rows_of_more_columns_than_27_bits_count(cuda):
+    """One row against 2^27 + 1032 rows of 64: no column is left out, and those where a block's tiles begin and end are right."""
+    N, K_ = 2**27 + 1032, 64
+    a, B = torch.randn((1, K_), device=cuda).bfloat16(), torch.empty((N, K_), dtype=torch.bfloat16, device=cuda).normal_()
+    C = torch.full((1, N), float("nan"), dtype=torch.bfloat16, device=cuda)
+    assert K.lib().iron_gemm_few_bf16(a.data_ptr(), B.data_ptr(), None, C.data_ptr(), 1, N, K_, 0, torch.cuda.current_stream().cuda_stream) == 0
+    assert not C.isnan().any()
+    edges = torch.arange(0, 257, device=cuda) * (N // 8) // 256 * 8
+    rows = (edges[:, None] + torch.arange(-40, 40, device=cuda)).flatten().clamp(0, N - 1)
+    want = (B[rows].double() * a.double()).sum(1)
+    bound = 2.0**-8 * want.abs() + K_ * 2.0**-24 * (B[rows].double() * a.double()).abs().sum(1)   # as above
+    assert ((C[0, rows].double() - want).abs() <= 1.01 * bound).all()
+
+
 # ---------------------------------------------------------------- recurrences
 
 
