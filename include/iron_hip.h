@@ -378,7 +378,7 @@ int iron_eval_words(int* words, int n_words, const int* exprs, int n, void* stre
 
 /* C = A B^T for up to 64 rows of A, or with B2 C = act(A B^T) * (A B2^T) (activation 1 SiLU, 2 GELU by its
  * tanh form, 3 ReLU; rounded where the separate steps round): bound by streaming B.  A (M, K), B and B2
- * (N, K), C (M, N); K % 8 == 0.  What iron_gemm_gated_pair_bf16 launches for fewer
+ * (N, K), C (M, N); K % 8 == 0; A, B and B2 16-byte aligned, C as its elements are.  What iron_gemm_gated_pair_bf16 launches for fewer
  * than 64 rows without a bound (it needs no G then), and iron_gemm_bf16 where those are not too many for K. */
 int iron_gemm_few_bf16(const uint16_t* A, const uint16_t* B, const uint16_t* B2, uint16_t* C, int M, int N, int K,
                        int activation, void* stream);

@@ -112,7 +112,7 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
 #pragma unroll
     for (int k = 0; k < 8; ++k) lds_wait_for<0>(af[0][k]);
   }
-  const bool whole = N % 8 == 0;   // C's rows take 16-byte pieces
+  const bool whole = N % 8 == 0 && ((uintptr_t)C & 15) == 0;   // C's rows take 16-byte pieces
   // The columns of `count` tiles from `first` on, from half `half` of the out stage, by one wave.
   auto flush = [&](int first, int count, int half) {
     for (int e = lane; e < M * count; e += 64) {

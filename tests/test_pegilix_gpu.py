@@ -109,6 +109,21 @@ def test_a_product_over_few_rows_by_strips(cuda, M, N, K_):
     assert (got[M] == 7).all()
 
 
+@pytest.mark.parametrize("M,N,K_", [(8, 2056, 1960), (16, 16456, 320), (20, 16392, 2048), (8, 2048, 8192), (9, 2048, 4096), (3, 640, 64)])
+@pytest.mark.parametrize("at", [1, 4])
+def test_a_product_over_few_rows_into_an_output_between_pieces(cuda, M, N, K_, at):
+    """C need not begin on a 16-byte piece, and what lies around it stays."""
+    rng = np.random.default_rng(N + at)
+    a, b = bf(rng, M, K_), bf(rng, N, K_, scale=0.1)
+    A, B, C = device(a, BF16), device(b, BF16), torch.full((M * N + 16,), 7.0, dtype=torch.bfloat16, device=cuda)
+    into = C[at : at + M * N]
+    assert K.lib().iron_gemm_few_bf16(A.data_ptr(), B.data_ptr(), None, into.data_ptr(), M, N, K_, 0, torch.cuda.current_stream().cuda_stream) == 0
+    aligned = torch.empty((M, N), dtype=torch.bfloat16, device=cuda)
+    assert K.lib().iron_gemm_few_bf16(A.data_ptr(), B.data_ptr(), None, aligned.data_ptr(), M, N, K_, 0, torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(into.view(M, N), aligned)
+    assert (C[:at] == 7).all() and (C[at + M * N :] == 7).all()
+
+
 def test_a_product_over_few_rows_of_more_columns_than_27_bits_count(cuda):
     """One row against 2^27 + 1032 rows of 64: no column is left out, and those where a block's tiles begin and end are right."""
     N, K_ = 2**27 + 1032, 64
