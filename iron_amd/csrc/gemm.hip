@@ -2448,8 +2448,12 @@ static int check_gemm(const uint16_t* A, const uint16_t* B, const uint16_t* C, i
 
 // Whether the few-row kernels take a product of B (N,K).  Their blocks read all of A each, so they grow with rows x K
 // (2048 x 8192 16 / 33 / 63 rows 10.3 / 27.1 / 35.8 us, 5256 x 6192 27 / 44 / 64) where the tiles do not (17.3 and 27);
-// the line lies where the two met over twenty shapes, short K to the few rows (63 x 1304 x 1032 6.4 against 7.8).
-static bool gemm_of_few_rows(int M, int K) {
+// the line lies where the two met over twenty shapes, short K to the few rows (63 x 1304 x 1032 6.4 against 7.8).  Up to sixteen rows
+// of a matrix that the strips take a tile a block stay ahead of the tiles past that line (weights out of memory: 16 rows 2048 x 9216 13.3
+// against 18.2, 2048 x 16384 18.0 against 23.4, 1000 x 16384 15.3 against 17.7, 304 x 14336 13.3 against 13.5; not
+// 14 x 304 x 18944, 16.0 against 14.9).
+static bool gemm_of_few_rows(int M, int N, int K) {
+  if (M <= 16 && N <= 2048 && K <= 16384 && (long)N * K >= (1 << 21)) return true;
   return M < 64 && (long)M * K < 140000 && (M < 48 || K < 1408);
 }
 
@@ -2475,7 +2479,7 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
     c_col_maj = 0;
   }
   // Fewer rows than the smallest tile: bound by streaming B.
-  if (gemm_of_few_rows(M, K) && b_col_maj && !c_col_maj && valid == nullptr && valid_k == nullptr)
+  if (gemm_of_few_rows(M, N, K) && b_col_maj && !c_col_maj && valid == nullptr && valid_k == nullptr)
     return iron_gemm_few_bf16(A, B, nullptr, C, M, N, K, 0, stream);
   // The direct-to-LDS kernels take any K from one stage on (k_pad), any M, and any N of B (N,K); against
   // the general kernel below, which loads through registers: 2048 x 2048 x 2056 42.5 -> 26.0 us, 86 x 1728 x
@@ -2537,7 +2541,7 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
 static TileShares gemm_shares(int M, int N, int K, bool b_nk, bool c_nm) {
   const TileShares none{0, 0, 0};
   const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
-  if (K < BK || (b_nk && gemm_of_few_rows(M, K)) || tiles > 3 * 256) return none;
+  if (K < BK || (b_nk && gemm_of_few_rows(M, N, K)) || tiles > 3 * 256) return none;
   if (!c_nm && gemm_on_big_tiles(M, N, K)) return none;
   const int stages = (K + BK - 1) / BK, t = (int)tiles;
   const int shared = t <= 128 ? t : (t > 256 ? t % 256 : 0);   // all tiles, or those of the last round

@@ -52,6 +52,16 @@ def test_every_entry_point_refuses_null_operands():
         assert lib.iron_last_error(), name
 
 
+def test_few_rows_over_a_long_k_share_no_tiles():
+    """Up to sixteen rows against up to 2048 of a long K go by strips, whatever the product of rows and K; past that, and past
+    K = 16384, their tiles' K is dealt over blocks.  As (N,M) output the same with the operands' places changed."""
+    room = _lib.lib().iron_gemm_workspace_bytes
+    for M, N, K, shared in ((16, 2048, 9216, False), (9, 1536, 16384, False), (16, 304, 14336, False), (16, 128, 16384, False),
+                            (16, 120, 16384, True), (16, 2056, 9216, True), (17, 2048, 9216, True), (12, 2048, 16392, True)):
+        assert (room(M, N, K, 1, 0) > 0) == shared, (M, N, K)
+        assert (room(N, M, K, 1, 1) > 0) == shared, (N, M, K)
+
+
 def test_bench_refuses_more_than_one_gpu():
     """``bench.py --gpus N`` with N above 1 exits with a message: this build is the one-GPU path."""
     import subprocess

@@ -109,6 +109,12 @@ def test_a_product_over_few_rows_by_strips(cuda, M, N, K_):
     assert (got[M] == 7).all()
 
 
+# ... and sixteen rows and less whose product with K passes what other sizes go by strips to.
+@pytest.mark.parametrize("M,N,K_", [(16, 2048, 9216), (9, 1531, 16384), (13, 128, 16384), (16, 2041, 10008)])
+def test_a_product_over_sixteen_rows_of_a_long_k(cuda, M, N, K_):
+    test_a_product_over_few_rows_by_strips(cuda, M, N, K_)
+
+
 @pytest.mark.parametrize("M,N,K_", [(8, 2056, 1960), (16, 16456, 320), (20, 16392, 2048), (8, 2048, 8192), (9, 2048, 4096), (3, 640, 64)])
 @pytest.mark.parametrize("at", [1, 4])
 def test_a_product_over_few_rows_into_an_output_between_pieces(cuda, M, N, K_, at):
