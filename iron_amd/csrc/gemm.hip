@@ -1852,16 +1852,24 @@ static int launch_gemm_either(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
 // down projection: 512 live rows x 2048 columns over K = 8192, then the next layer's input norm).
 // 128 x 128 tiles would occupy a quarter of the CUs and the 64 x 64 ones that fill the chip fetch
 // every operand row twice as often, so a tile's K is dealt over `splits` blocks -- chosen on the
-// device by the row bound: 16, 8 and 4 while the live tiles fill that part of the chip, 2 up to half, else
+// device by the row bound and K: 16, 8 and 4 while the live tiles fill that part of the chip, 2 up to half, else
 // whole K -- each leaving its float32 sums in a workspace slice.  A second launch, a block a row,
 // adds a row's slices in slice order (the same sums whatever ran first), rounds once, adds the
 // residual, stores the row and norms it as rmsnorm_kernel does: that launch stands where the
 // norm's own stood, so the slices' sum costs no launch of its own.
 constexpr int kSplitKMax = 4;    // slices the second launch asks for at a time, and every K can be cut into
-__device__ __host__ inline int splitk_for(int live_tiles, int K) {
-  // Past four slices while the chip would idle and a slice keeps eight stages (29 rows x 2048 x 8192 with the norm 17.4 -> 14.0 us, 128 rows 19.8 -> 17.9).
-  if (live_tiles * 16 <= 256 && K % (16 * 8 * BK) == 0) return 16;
-  if (live_tiles * 8 <= 256 && K % (8 * 8 * BK) == 0) return 8;
+__device__ __host__ inline int splitk_for(int tile_rows, int tiles_n, int K) {
+  const int live_tiles = tile_rows * tiles_n;
+  // Past four slices while the chip would idle and a slice keeps eight stages; ten where the slices of several tile rows pass half
+  // the chip, whose sums cost the second launch more.  us with the norm, weights out of memory, N = 2048, fewer slices and more: K = 8192 29 rows
+  // 26.0 / 16.3 (16), 128 28.5 / 19.8, 256 29.5 / 23.0 (8); K = 14336 41.3 / 21.6, 43.5 / 24.9, 43.8 / 31.1; K = 4096 29 rows 15.8 / 12.9 (8), but 256 20.6 / 21.8,
+  // and 256 rows of N = 1024 over 8192 by 8 slices 20.1, by 16 21.6.
+  auto keeps = [=](int splits) {
+    const int stages = tile_rows > 1 && 2 * live_tiles * splits > 256 ? 10 : 8;
+    return live_tiles * splits <= 256 && K % (splits * BK) == 0 && K >= splits * stages * BK;
+  };
+  if (keeps(16)) return 16;
+  if (keeps(8)) return 8;
   return live_tiles * 4 <= 256 ? 4 : (live_tiles * 2 <= 256 ? 2 : 1);
 }
 // Rows a slice of the workspace holds when K is dealt `splits` ways: the most that split count runs for.
@@ -1874,8 +1882,8 @@ __global__ __launch_bounds__(256) void gemm_splitk_kernel(const bf16_t* __restri
                                                           const int* __restrict__ valid, Tiling whole, QkvTail tail,
                                                           float* __restrict__ partial) {
   const int Mv = bound_or(valid, M);
-  const int tiles_n = whole.tiles_n, live_tiles = ((Mv + 127) / 128) * tiles_n;
-  const int splits = splitk_for(live_tiles, K), id = blockIdx.x;
+  const int tiles_n = whole.tiles_n, tile_rows = (Mv + 127) / 128, live_tiles = tile_rows * tiles_n;
+  const int splits = splitk_for(tile_rows, tiles_n, K), id = blockIdx.x;
   if (splits == 1) {   // whole K a block, the residual in its epilogue: iron_gemm_residual_bf16's 128 x 128 launch
     if (id < whole.tiles_m * whole.tiles_n)
       gemm_nt16_body<false>(A, B, C, M, N, K, valid, whole.tiles_m, whole.tiles_n, whole.patched, tail);
@@ -1921,7 +1929,7 @@ __global__ __launch_bounds__(256) void gemm_finish_rows_kernel(const float* __re
   for (int i = 0; i < CHUNKS; ++i) gains[i] = load_bounded(gain_bytes, 16 * (threadIdx.x + 256 * i));
   const int Mv = bound_or(valid, M);
   if (row >= Mv) return;
-  const int splits = splitk_for(((Mv + 127) / 128) * tiles_n, K);
+  const int splits = splitk_for((Mv + 127) / 128, tiles_n, K);
   uint4* c_row = reinterpret_cast<uint4*>(C + (size_t)row * N);
   uint4 held[CHUNKS];
   if (splits == 1) {

@@ -474,6 +474,21 @@ def test_gemm_residual_then_rmsnorm_with_k_dealt_over_blocks(cuda, M, Kdim, N, r
     assert np.array_equal(from_torch(Rd)[lim:], R[lim:])
 
 
+# Sixteen slices: a 1B prompt's few rows and the most there are for it; K no power of two; tile columns that the tiles of sixteen do
+# not fill, two tile rows; a row of four pieces a thread.  Eight, of a K that sixteen cut too short or not whole.
+@pytest.mark.parametrize("M,Kdim,N,rows,slices", [(2048, 8192, 2048, 29, 16), (2048, 8192, 2048, 128, 16), (256, 14336, 384, 130, 16), (128, 9216, 1024, None, 16),
+                                                  (256, 8192, 1024, 256, 8), (256, 5632, 256, 200, 8), (128, 4608, 4096, 77, 8), (256, 4096, 2048, 200, 4)])
+def test_gemm_residual_then_rmsnorm_with_k_dealt_over_many_blocks(cuda, M, Kdim, N, rows, slices):
+    test_gemm_residual_then_rmsnorm_with_k_dealt_over_blocks(cuda, M, Kdim, N, rows, 1.0)
+    # ... and as many slices of sums as the rows and K call for: the workspace holds them one behind the other.
+    A, B, R = (torch.ones(s, dtype=torch.bfloat16, device=cuda) for s in ((M, Kdim), (N, Kdim), (M, N)))
+    ws = torch.full((K.gemm_residual_norm_workspace_bytes(M, N, Kdim) // 4,), float("nan"), dtype=torch.float32, device=cuda)
+    K.gemm_residual_norm(A, B, R, R[0], torch.empty_like(R), torch.empty_like(R), ws, M=M, N=N, K=Kdim, eps=1e-6,
+                         valid=None if rows is None else word(rows, cuda))
+    sums = ws[~ws.isnan()]
+    assert (sums == Kdim // slices).all() and sums.numel() == slices * (rows or M) * N
+
+
 def test_gemm_residual_then_rmsnorm_refuses_other_shapes(cuda):
     """Shapes whose K is too short to deal, or whose rows the second launch cannot hold, report no
     workspace and are refused with a reason before any launch."""
