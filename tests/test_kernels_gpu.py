@@ -282,6 +282,37 @@ def test_gemm_small_tiles_at_every_depth(cuda, M, Kdim, N, rows, residual):
     assert np.all(got[lim:] == 5.0)
 
 
+@pytest.mark.parametrize("M,Kdim,N,b_col_maj,bounds", [
+    (2048, 200, 8192, True, (1, 128, 129, 1024, 1025, 2047)),    # 64, 128 and 256 tiles by the bound
+    (1500, 328, 2056, True, (63, 895, 896, 897, 1500)),          # 64 and 128 ones, ragged
+    (256, 136, 320, True, (0, 100, 200)), (40, 1000, 4168, True, (17, 40)), (33, 4096, 520, True, (1, 32)),   # 64 ones whatever the bound
+    (2048, 328, 2056, False, (1, 129, 1999)), (300, 200, 136, False, (299,)), (40, 264, 72, False, (17,)),    # (K,N): the last column tile moved back
+    (64, 72, 128, False, (5,)), (2, 192, 4104, False, (1,))])
+def test_gemm_under_a_bound_at_the_edges_of_tiles_and_stages(cuda, M, Kdim, N, b_col_maj, bounds):
+    """A bound on the rows with a K that ends inside a stage or columns inside a tile: rows past the bound are NaN on the way in and
+    come out untouched, the operands lie between NaNs."""
+    rng = np.random.default_rng(M + N + Kdim)
+    A, B = bf(rng, M, Kdim), bf(rng, (N if b_col_maj else Kdim), (Kdim if b_col_maj else N), scale=0.05)
+    want, near = ops.gemm(A, B, b_col_maj=b_col_maj), ops.gemm_bound(A, B, b_col_maj=b_col_maj)
+
+    def between_nans(x):
+        room = 64 * max(x.shape)
+        buf = torch.full((x.size + 2 * room,), float("nan"), dtype=torch.bfloat16, device=cuda)
+        inside = buf[room:room + x.size].view(*x.shape)
+        inside.copy_(dev(x, cuda))
+        return inside
+
+    dB = between_nans(B)
+    for rows in bounds:
+        live = A.copy()
+        live[rows:] = np.nan
+        C = out_like((M, N), cuda, fill=7.0)
+        K.gemm(between_nans(live), dB, C, M=M, N=N, K=Kdim, b_col_maj=b_col_maj, valid=word(rows, cuda))
+        got = from_torch(C)
+        assert np.all(np.abs(got[:rows] - want[:rows]) <= near[:rows]), rows
+        assert np.all(got[rows:] == 7.0), rows
+
+
 @pytest.mark.parametrize("M,Kdim,N,form", [(*s, f) for s in ((2048, 2048, 2048), (2048, 1024, 8192), (1500, 320, 4160))
                                            for f in ("plain", "residual", "gated", "pair")] + [(2048, 200, 8192, "plain")])
 def test_a_row_s_products_are_the_same_bits_under_every_bound(cuda, M, Kdim, N, form):
