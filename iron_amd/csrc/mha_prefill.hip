@@ -34,16 +34,14 @@ constexpr int BKV = 64;   // key rows per tile
 constexpr float kLazyBits = 8.f;        // how far a maximum may run ahead of the reference the exponents are taken against
 constexpr float kSumLow = 0x1p-60f, kSumHigh = 0x1p24f;   // a tile's sum of exponentials outside this range: take its maximum and redo it
 constexpr int kCUs = 256;                // compute units the block orders below assume
-// Whether queries that fill `live` blocks of the launch go 32 to a block instead, the keys dealt over its waves
-// (prefill_few_rows).  Four times the blocks each read all the keys, so it pays while the chip has CUs for them,
-// and from a few tiles a wave on.  us, 32 / 8 heads, tiles against few rows: 40 queries, d = 64, 512 / 2048 / 12043
+// Whether `groups` blocks of 32 queries and a head, the keys dealt over a block's waves (prefill_few_rows), take the place of a launch's
+// blocks of 32 W queries.  Each of them reads all the keys, so it pays while the chip has CUs for them (at d = 64 with eight waves, where
+// a CU holds two blocks, twice as many), and from a few tiles a wave on.  us, 32 / 8 heads, tiles against few rows: 40 queries, d = 64, 512 / 2048 / 12043
 // keys 11.2 / 9.7, 23.8 / 14.5, 103 / 44; 512 queries 11.5 / 11.0, 25.3 / 22.0, 112 / 83; d = 128, 8000 keys, 256 queries 121 / 56, 512 queries over
 // 512 keys 18.3 / 21.8.
-template <int D>
-__host__ __device__ __forceinline__ bool few_rows_pay(int live, int keys) { return live <= (D == 64 ? 128 : 64) && keys >= 512; }
+template <int D, int W>
+__host__ __device__ __forceinline__ bool few_rows_pay(int groups, int keys) { return groups <= (D == 64 && W == 4 ? 512 : 256) && keys >= 512; }
 constexpr int kFewBlocks = 512;          // launches of fewer blocks than this halve their blocks' queries (S = 1024 at 32 heads: 18.5 -> 13.9 us)
-constexpr int kFewBlocks128 = 360;       // d = 128: up to this many blocks of 64 queries a launch takes those (one a CU; 32 heads, 512 / 700 / 777
-                                         // queries 15.2 -> 12.3, 18.3 -> 17.4, 19.0 -> 20.0 us; 8 heads, 3001 46.5 -> 40.0)
 constexpr int kWideBigBlocks = 512;     // wide heads: launches of at least this many 128-query blocks keep that size
 constexpr int kSplitMaxBlocks = 1024;   // launches of up to this many blocks split each block's tiles over two halves
 
@@ -314,7 +312,7 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
   // Few live queries (FEW: the launch may have them; the code beside the tiles' costs those 1.5 % at d = 128): groups of 32 take the first blocks, all blocks the zeros of the rows past them.
   const int groups = FEW ? (q_tokens + 31) >> 5 : 0;
   if (FEW && groups > 0 && groups <= nqb && offset >= 0 &&
-      few_rows_pay<D>(heads * ((q_tokens + BQW - 1) / BQW), window < 0 ? kv_tokens : min(kv_tokens, window + q_tokens))) {
+      few_rows_pay<D, W>(heads * groups, window < 0 ? kv_tokens : min(kv_tokens, window + q_tokens))) {
     const int all = (seq + 31) >> 5;
     for (int unit = blockIdx.x; unit < heads * (all - groups); unit += gridDim.x) {
       const int h = unit % heads, r0 = (groups + unit / heads) * 32;
@@ -983,10 +981,23 @@ static int launch_prefill_as(const PrefillArgs& a, int blocks, void* stream) {
 template <int D, int SPLIT, int W = 4>
 static int launch_prefill(const PrefillArgs& a, int blocks, void* stream) {
   const bool bounded = a.valid != nullptr || a.kv_valid != nullptr || a.seq_len != a.seq;
-  if (a.kv_len < 512 || (!bounded && !few_rows_pay<D>(blocks, a.kv_len))) return launch_prefill_as<D, SPLIT, W, false>(a, blocks, stream);
   // (a launch so short that all its queries may go 32 to a block has a block for each 32)
   const int groups = ((a.seq + 31) / 32) * a.heads;
-  return launch_prefill_as<D, SPLIT, W, true>(a, few_rows_pay<D>(blocks, a.kv_len) && groups > blocks ? groups : blocks, stream);
+  const bool few = few_rows_pay<D, W>(groups, a.kv_len);
+  if (a.kv_len < 512 || (!bounded && !few)) return launch_prefill_as<D, SPLIT, W, false>(a, blocks, stream);
+  return launch_prefill_as<D, SPLIT, W, true>(a, few && groups > blocks ? groups : blocks, stream);
+}
+
+// Whether a launch of 128-wide heads takes blocks of 64 queries (one a CU) and not of 128.  One round of them does: it is the shorter
+// for every length (32 heads, us by 128 and by 64: 512 queries 14.3 / 11.4, 300 over 4096 keys 60 / 52).  A second round as long as the first does not
+// (640 queries over 4000 keys 60 / 90), but under a causal mask over the queries' own keys the blocks go out longest first, so the second round's meet the
+// first's shortest: with L blocks a head, 256 / heads of them in the first round, those two in line, each with about 5 blocks' time of its start and end,
+// end before a longest one while 2 (L - 256 / heads) + 5 <= L.  Both sides of that line: 8 heads 3001 queries 46.1 / 39.8, 16 heads 1650 30.2 / 26.7,
+// 24 heads 1024 21.7 / 20.6, 32 heads 704 17.1 / 16.8; past it 24 heads 1100 22.7 / 23.5, 32 heads 777 18.3 / 19.6, 40 heads 576 15.3 / 17.0.
+static bool half_blocks_128(const PrefillArgs& a) {
+  const long levels = (a.seq + 63) / 64;
+  if (a.heads * levels <= kCUs) return true;
+  return a.causal && (a.window < 0 || a.window >= a.kv_len) && a.heads * (levels + 5 + (a.kv_len - a.seq) / 64) <= 2 * kCUs;
 }
 
 template <int D, int QN, int W>
@@ -1056,7 +1067,10 @@ static int mha_prefill(const uint16_t* Q, const uint16_t* K, const uint16_t* V, 
   // Fewer blocks of 128 queries than two a CU (a short prompt): blocks of 64, two waves a part.
   else if (d == 64 && blocks < kFewBlocks) rc = launch_prefill<64, 2, 2>(a, ((seq + 63) / 64) * heads, stream);
   else if (d == 64) rc = split ? launch_prefill<64, 2>(a, blocks, stream) : launch_prefill<64, 1>(a, blocks, stream);
-  else if (const int halves = ((seq + 63) / 64) * heads; halves <= kFewBlocks128) rc = launch_prefill<128, 2, 2>(a, halves, stream);
+  // (where the few-row form takes the whole launch, and the keys are many, its blocks have eight waves: 40 queries over 512 / 1024 / 2000 / 12043 keys
+  // with four 9.5 / 12.8 / 19.0 / 87 us, with eight 10.9 / 13.3 / 18.0 / 69)
+  else if (half_blocks_128(a) && !(kv_len >= 1536 && few_rows_pay<128, 4>(((seq + 31) / 32) * heads, kv_len)))
+    rc = launch_prefill<128, 2, 2>(a, ((seq + 63) / 64) * heads, stream);
   else if (split) rc = launch_prefill<128, 2>(a, blocks, stream);
   else rc = launch_prefill<128, 1>(a, blocks, stream);
   if (rc != 0) return rc;

@@ -912,6 +912,16 @@ def test_mha_prefill_of_few_rows_over_many_keys(cuda, H, G, d, S, rows, L, keys,
         close(got[r : r + 1], want)
 
 
+# 128-wide heads, more queries than a block of 64 has: all of a launch's in the few-row form, with four waves a block and with eight; one
+# more than that form takes; a second round of blocks that only a causal mask over the queries' own keys allows, and one it does not.
+@pytest.mark.parametrize("H,G,S,rows,L,keys,window,causal", [
+    (32, 8, 256, 256, 1000, 1000, None, True), (32, 8, 256, 230, 2500, 2100, None, True), (32, 8, 200, 200, 1600, 1600, None, False),
+    (32, 8, 257, 257, 1600, 1600, None, True), (32, 8, 300, 270, 2000, 400, None, True),
+    (32, 8, 700, 700, 700, 700, None, True), (32, 8, 640, 640, 1700, 1700, None, True), (8, 2, 2200, 2200, 2200, 2200, 1500, True)])
+def test_mha_prefill_128_wide_heads_at_the_lines_between_the_forms(cuda, H, G, S, rows, L, keys, window, causal):
+    test_mha_prefill_of_few_rows_over_many_keys(cuda, H, G, 128, S, rows, L, keys, window, causal)
+
+
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("interleaved", [True, False])
 def test_mha_prefill_of_few_rows_in_both_layouts_and_a_window_of_a_buffer(cuda, d, interleaved):
