@@ -282,6 +282,43 @@ def test_gemm_small_tiles_at_every_depth(cuda, M, Kdim, N, rows, residual):
     assert np.all(got[lim:] == 5.0)
 
 
+@pytest.mark.parametrize("cols", [2049, 2050, 2052, 2054, 2055, 2060])
+@pytest.mark.parametrize("form", ["plain", "turned", "(N,M)", "residual", "pair"])
+def test_gemm_rows_that_are_no_whole_pieces(cuda, cols, form):
+    """Output rows of every remainder of eight elements, through the 128 x 128 tiles' stores: the columns at a row's end, and
+    nothing past the output's."""
+    M, Kdim = 1200, 264 if form in ("plain", "turned", "(N,M)") else 256
+    rng = np.random.default_rng(cols)
+    if form == "(N,M)":   # rows of M elements, B (K,N)
+        A, B = bf(rng, cols, Kdim), bf(rng, Kdim, M, scale=0.05)
+        want, near = ops.gemm(A, B, c_col_maj=True), ops.gemm_bound(A, B, c_col_maj=True)
+    elif form == "turned":
+        A, B = bf(rng, cols, Kdim), bf(rng, M, Kdim, scale=0.05)
+        want, near = ops.gemm(A, B, b_col_maj=True, c_col_maj=True), ops.gemm_bound(A, B, b_col_maj=True, c_col_maj=True)
+    else:
+        A, B = bf(rng, M, Kdim), bf(rng, cols, Kdim, scale=0.05)
+        want, near = ops.gemm(A, B, b_col_maj=True), ops.gemm_bound(A, B, b_col_maj=True)
+    dA, dB, buf = dev(A, cuda), dev(B, cuda), out_like((M * cols + 64,), cuda, fill=3.0)
+    C = buf[: M * cols].view(M, cols)
+    if form in ("plain", "turned", "(N,M)"):
+        m, n = (M, cols) if form == "plain" else (cols, M)
+        K.gemm(dA, dB, C, M=m, N=n, K=Kdim, b_col_maj=form != "(N,M)", c_col_maj=form != "plain")
+    elif form == "residual":
+        R = bf(rng, M, cols)
+        K.gemm_residual(dA, dB, dev(R, cuda), C, M=M, N=cols, K=Kdim, residual_scale=0.5)
+        near = near + 2.0**-8 * np.abs(0.5 * want + R)   # the sum's own rounding
+        want = np.float32(0.5) * want + R
+    else:
+        B2, G = bf(rng, cols, Kdim, scale=0.05), out_like((M * cols + 64,), cuda, fill=3.0)
+        K.gemm_gated_pair(dA, dB, dev(B2, cuda), G[: M * cols].view(M, cols), C, M=M, N=cols, K=Kdim, activation="relu")
+        assert np.all(np.abs(from_torch(G[: M * cols].view(M, cols)) - want) <= near) and bool((G[M * cols:] == 3).all())
+        gate, up = np.maximum(want, 0), ops.gemm(A, B2, b_col_maj=True)
+        near = near * np.abs(up) + gate * ops.gemm_bound(A, B2, b_col_maj=True) + 2.0**-7 * np.abs(gate * up) + near * ops.gemm_bound(A, B2, b_col_maj=True)
+        want = gate * up
+    assert np.all(np.abs(from_torch(C) - want) <= near)
+    assert bool((buf[M * cols:] == 3).all())
+
+
 @pytest.mark.parametrize("M,Kdim,N,b_col_maj,bounds", [
     (2048, 200, 8192, True, (1, 128, 129, 1024, 1025, 2047)),    # 64, 128 and 256 tiles by the bound
     (1500, 328, 2056, True, (63, 895, 896, 897, 1500)),          # 64 and 128 ones, ragged
