@@ -588,41 +588,45 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
       for (int e = 0; e < 16; ++e) acc[e >> 3][(e >> 2) & 1][e & 3] = x[e];
     }
   }
-  const bool vec = (N & 3) == 0;
+  const bool vec = (N & 3) == 0;   // rows of 8-byte pieces
+  auto pieces = [&](auto residual) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i) {
+      const int m = mb + 16 * i;
+      if (m >= Mv) continue;
+      bf16_t* row = C + (size_t)m * N;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int m = mb + 16 * i, n = nb + 16 * j;
-      if (m >= Mv || n >= N) continue;
-      bf16_t* p = C + (size_t)m * N + n;
-      if (!PAIR && qkv.residual != nullptr) {   // the product rounded as it would be stored, then scale * it + residual
-        const bf16_t* r = qkv.residual + (size_t)m * N + n;
-        float rf[4] = {0.f, 0.f, 0.f, 0.f};
-        if (vec && n + 4 <= N) {
-          const uint2 rv = res_ahead ? res[i][j] : *reinterpret_cast<const uint2*>(r);
-          rf[0] = __uint_as_float(rv.x << 16); rf[1] = __uint_as_float(rv.x & 0xffff0000u);
-          rf[2] = __uint_as_float(rv.y << 16); rf[3] = __uint_as_float(rv.y & 0xffff0000u);
+      for (int j = 0; j < 2; ++j) {
+        const int n = nb + 16 * j;
+        if (n >= N) continue;
+        if constexpr (decltype(residual)::value) {   // the product rounded as it would be stored, then scale * it + residual
+          float rf[4] = {0.f, 0.f, 0.f, 0.f}, prod[4];
+          if (vec) {
+            rf[0] = __uint_as_float(res[i][j].x << 16); rf[1] = __uint_as_float(res[i][j].x & 0xffff0000u);
+            rf[2] = __uint_as_float(res[i][j].y << 16); rf[3] = __uint_as_float(res[i][j].y & 0xffff0000u);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (n + e < N) rf[e] = bf16_to_f32(qkv.residual[(size_t)m * N + n + e]);
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) prod[e] = round_bf16(acc[i][j][e]);
+          tail_of(qkv, prod, rf);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][j][e] = prod[e];
+        }
+        if (vec) {
+          *reinterpret_cast<uint2*>(row + n) = make_uint2(pack_bf16(acc[i][j][0], acc[i][j][1]), pack_bf16(acc[i][j][2], acc[i][j][3]));
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            if (n + e < N) rf[e] = bf16_to_f32(r[e]);
+            if (n + e < N) row[n + e] = f32_to_bf16(acc[i][j][e]);
         }
-        float prod[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) prod[e] = round_bf16(acc[i][j][e]);
-        tail_of(qkv, prod, rf);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[i][j][e] = prod[e];
-      }
-      if (vec && n + 4 <= N) {
-        *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16(acc[i][j][0], acc[i][j][1]), pack_bf16(acc[i][j][2], acc[i][j][3]));
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (n + e < N) p[e] = f32_to_bf16(acc[i][j][e]);
       }
     }
+  };
+  if (!PAIR && qkv.residual != nullptr) pieces(std::true_type());
+  else pieces(std::false_type());
 }
 
 // 128 x 128 x 64 tiles, four stages of 32 KB fed straight from global memory into LDS (buffer loads:
