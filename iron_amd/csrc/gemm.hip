@@ -2476,6 +2476,25 @@ static bool gemm_on_big_tiles(int M, int N, int K) {
   return M >= BIG_BM && N >= BIG_BN && N % 8 == 0 && tiles256 >= (K % BK == 0 ? 192 : 144) && 5 * tiles128 >= 16 * tiles256;
 }
 
+// Whether the direct-to-LDS kernels take a product, B (N,K) with C (N,M) turned round before.  They take any K from one stage on (k_pad),
+// any M, and any N of B (N,K); against the general kernel, which loads through registers: 2048 x 2048 x 2056 42.5 -> 26.0 us, 86 x 1728 x
+// 5560 59 -> 26.5, (K,N) 2048 x 2048 x 2040 65 -> 22.0, 300 x 1000 x 1000 33.6 -> 9.8.  (A K that is no
+// multiple of 64 stays dearer than its neighbour that is, 26.0 us against 19.4: its rows' 128-byte
+// pieces straddle two cache lines.)  The general kernel, of which a CU holds several blocks, keeps a short K where there is one row or column
+// of tiles, and such a K that straddles where the direct tiles' second round is a short one or their rows leave in pieces of eight bytes, over
+// very many tiles up to a K of 1536 (general against direct: (K,N) 107 x 240 x 64 3.7 / 4.6, 100 x 8008 x 64 4.4 / 4.9, but 200 x 240 x 64 5.8 / 4.6;
+// (N,M) of 3 x 3904 x 224 5.8 / 6.3; (N,K) 490 x 22 x 64 3.2 / 3.8, under a bound 63 x 424 x 64 3.2 / 3.8; 2048 x 2616 x 120 10.2 / 11.4, but 4000 x
+// 5000 x 120 24.0 / 20.4; 7137 x 6620 x 80 49.0 / 55.1 and x 1000 166.6 / 179.4, but 4000 x 3004 x 1000 49.9 / 42.7).
+static bool gemm_direct_to_lds(int M, int N, int K, int b_col_maj, int c_col_maj, bool bounded) {
+  if (K < BK || (c_col_maj && (b_col_maj || bounded))) return false;
+  if (!b_col_maj) return (M >= 128 && N >= 128) || K > (c_col_maj && M < 8 ? 4 : 2) * BK;
+  if (M < 64 || N < 64) return K > 2 * BK;
+  const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
+  if (K % BK == 0 || tiles128 <= 256) return true;
+  if (tiles128 <= 448) return K >= 6 * BK;
+  return N % 8 != 4 || K >= (tiles128 > 1024 ? 24 : 3) * BK;
+}
+
 extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K,
                               int b_col_maj, int c_col_maj, const int* valid, const int* valid_k,
                               void* stream) {
@@ -2493,13 +2512,7 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
   // Fewer rows than the smallest tile: bound by streaming B.
   if (gemm_of_few_rows(M, N, K) && b_col_maj && !c_col_maj && valid == nullptr && valid_k == nullptr)
     return iron_gemm_few_bf16(A, B, nullptr, C, M, N, K, 0, stream);
-  // The direct-to-LDS kernels take any K from one stage on (k_pad), any M, and any N of B (N,K); against
-  // the general kernel below, which loads through registers: 2048 x 2048 x 2056 42.5 -> 26.0 us, 86 x 1728 x
-  // 5560 59 -> 26.5, (K,N) 2048 x 2048 x 2040 65 -> 22.0, 300 x 1000 x 1000 33.6 -> 9.8.  (A K that is no
-  // multiple of 64 stays dearer than its neighbour that is, 26.0 us against 19.4: its rows' 128-byte
-  // pieces straddle two cache lines.)  Under a whole tile of (K,N) two stages of it are no gain (1 x 64 x 64 3.6 us
-  // against 4.3).
-  if (valid_k == nullptr && K >= BK && (b_col_maj ? !c_col_maj : (!c_col_maj || valid == nullptr) && ((M >= 64 && N >= 128) || K > 2 * BK))) {
+  if (valid_k == nullptr && gemm_direct_to_lds(M, N, K, b_col_maj, c_col_maj, valid != nullptr)) {
     if (c_col_maj) return launch_gemm_nt<true, false, 2, 4, true>(A, B, C, M, N, K, valid, s);
     const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
     // Enough 256x256 tiles to fill the chip: the large-tile kernel (offsets are 32-bit).  A round of
