@@ -364,8 +364,10 @@ __device__ __forceinline__ void tile_of_block(int bid, int tiles_m, int tiles_n,
 }
 
 // The same under a row bound read on the device: an order that is not patched is that of the live tile rows alone, or the few
-// there are would be a few XCDs'.  False: the block has none.
+// there are would be a few XCDs'; so is one whose patches of eight tile rows would be cut (3072 x 3072 columns and K, 300 rows 33.4 -> 18.6 us).
+// False: the block has none.
 __device__ __forceinline__ bool live_tile(int bid, int tiles_m, int tiles_n, int patched, int live_m, int& tm, int& tn) {
+  if (live_m < 8) patched = 0;
   if (!patched) {
     tiles_m = min(tiles_m, live_m);
     if (bid >= tiles_m * tiles_n) return false;
@@ -2227,24 +2229,38 @@ __device__ __forceinline__ void gemm_nt16_pair_body(const bf16_t* __restrict__ A
 // A gated feed-forward's two first projections over many rows as ONE launch, the tile chosen on the
 // device by the row bound as in gemm_either_kernel.  Few rows: 64 rows x (32 + 32) columns on the 64 x 64 tile's
 // loop, two waves a product (29 x 8192 x 2048 29.7 -> 20.5 us: as a gate tile and then an up tile a block made
-// two chains of stages).  Up to one round of them, 128 x 128 tiles of both products at once.  Past that 256 rows x (128 + 128) columns, a wave's 128 x 128 half gate and half up
+// two chains of stages).  Else 128 x 128 tiles of both products at once, or 256 rows x (128 + 128) columns, a wave's 128 x 128 half gate and half up
 // projection: the bytes a CU draws from L2 per flop are those of a 256 x 256 tile, two thirds of the smaller pair's.
 // A round of the large tiles takes 1.5 rounds of the small ones and covers two (N = 8192, K = 2048: 2048
-// rows 161 -> 130 us, 1024 89 -> 65, 1281 118 -> 113; 512 rows, on the small tiles, 46.5 -> 41.8 by asking the kind of gate once).
+// rows 161 -> 130 us, 1024 89 -> 65; 512 rows, on the small tiles, 46.5 -> 41.8 by asking the kind of gate once).
+enum class PairForm { ROWS64, ROWS128, ROWS256 };
+// `few`: the rows below which 128 x 128 tiles would leave half the CUs idle.  Up to those 64 rows x (32 + 32) columns, a round of which takes about
+// a third of one of 128 x 128 tiles, so three rounds of them, or however many where each weight is read for one row of tiles (us, 64 against 128 rows, weights
+// out of memory: 888 x 3392 1600 rows 50.6 / 52.7, 2048 65 / 52.5; 3648 x 4160 400 rows 95 / 66; but 104 rows of 14336 x 4096 88 / 132).
+// The large tiles where their rounds, at 1.5 of the small ones', come out as no more (5632 x 2048: 1281 rows, 264 blocks, 113 against 82 by the small
+// ones, 1000 rows 57.6 against 81; 11776 x 4672: 580 rows 237 against 181).
+__host__ __device__ __forceinline__ PairForm pair_form(int rows, int few, int n32, int n128, bool large) {
+  const int blocks64 = ((rows + 63) / 64) * n32;
+  if (rows <= few && (blocks64 <= 768 || rows <= 128)) return PairForm::ROWS64;
+  const int rounds128 = (((rows + 127) / 128) * n128 + 255) / 256, rounds256 = (((rows + 255) / 256) * n128 + 255) / 256;
+  return large && 3 * rounds256 <= 2 * rounds128 ? PairForm::ROWS256 : PairForm::ROWS128;
+}
+
 __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __restrict__ A,
                                                               const bf16_t* __restrict__ Bg,
                                                               const bf16_t* __restrict__ Bu, bf16_t* __restrict__ G,
                                                               bf16_t* __restrict__ C, int M, int N, int K,
                                                               const int* __restrict__ valid, Tiling t256, Tiling t128,
-                                                              Tiling t64, int few256, int few128, int activation) {
+                                                              Tiling t64, int few, int activation) {
   const int Mv = bound_or(valid, M), bid = blockIdx.x;
+  const PairForm form = pair_form(Mv, few, t64.tiles_n, t128.tiles_n, t256.tiles_m > 0);
   QkvTail gate{};
   gate.gated = activation;
-  if (Mv > few256) {
+  if (form == PairForm::ROWS256) {
     if (bid >= t256.tiles_m * t256.tiles_n) return;
     gemm_nt256_body<4, BIG_KB, false, false, true>(A, Bg, C, M, N, K, valid, t256.tiles_m, t256.tiles_n, t256.patched,
                                                    GatedPair{Bu, G, activation});
-  } else if (Mv > few128) {
+  } else if (form == PairForm::ROWS128) {
     if (bid >= t128.tiles_m * t128.tiles_n) return;
     gemm_nt16_pair_body(A, Bg, Bu, G, C, M, N, K, valid, t128.tiles_m, t128.tiles_n, t128.patched, activation);
   } else {
@@ -2255,20 +2271,24 @@ __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __re
 
 static int launch_gemm_gated_pair(const bf16_t* A, const bf16_t* Bg, const bf16_t* Bu, bf16_t* G, bf16_t* C, int M,
                                   int N, int K, const int* valid, int activation, hipStream_t s) {
-  const int n128 = (N + 127) / 128, n32 = (N + 31) / 32;
-  // 64 x 64 tiles up to the rows below which 128 x 128 ones would leave half the CUs idle (as iron_gemm_bf16),
-  // 256 x (128 + 128) ones past the rows that one round of 128 x 128 ones covers.
-  int few128 = n128 >= 128 ? 0 : 128 * (127 / n128);
-  if (few128 > M) few128 = M;
-  int few256 = n128 >= 256 ? 0 : 128 * (256 / n128);
-  if (few256 > M || M < BIG_BM || N % 128 != 0) few256 = M;
+  const int n128 = (N + 127) / 128, n32 = (N + 31) / 32, few = n128 >= 128 ? 0 : 128 * (127 / n128);
+  const bool large = M >= BIG_BM && N % 128 == 0;
+  // The most rows each form is chosen for: its grid covers those.
+  int most[3] = {0, 0, 0};
+  for (int rows = valid == nullptr ? M : 1; rows < M + 64; rows += 64) {   // (a form is the same within a run of 64 rows that ends on a multiple of them)
+    const int r = rows < M ? rows : M;
+    int& upto = most[(int)pair_form(r, few, n32, n128, large)];
+    const int end = ((r + 63) / 64) * 64 < M ? ((r + 63) / 64) * 64 : M;
+    if (end > upto) upto = end;
+  }
   auto tiling = [](int tile_rows, int tile_cols) {
     const int whole = (tile_rows + 7) & ~7;
     if (tile_rows >= 8 && !patched_order(tile_rows, tile_cols) && patched_order(whole, tile_cols)) tile_rows = whole;
     return Tiling{tile_rows, tile_cols, patched_order(tile_rows, tile_cols)};
   };
-  const Tiling t256 = few256 < M ? tiling((M + BIG_BM - 1) / BIG_BM, n128) : Tiling{0, 0, 0};
-  const Tiling t128 = tiling((few256 + 127) / 128, n128), t64 = tiling((few128 + 63) / 64, n32);
+  // (the 64-row tiles in the order of all the rows up to `few`: 580 of 1024 rows in patches of eight tile rows took 27.2 us at 1536 x 1536, not 22.4)
+  const Tiling t64 = tiling(most[0] > 0 ? ((few < M ? few : M) + 63) / 64 : 0, n32), t128 = tiling((most[1] + 127) / 128, n128);
+  const Tiling t256 = large ? tiling((M + BIG_BM - 1) / BIG_BM, n128) : Tiling{0, 0, 0};
   constexpr size_t lds = (size_t)PAIR_STAGES * 3 * 128 * BK * 2;   // the two-product body's stages, more than the others'
   static_assert(lds >= (size_t)NT_STAGES * 256 * BK * 2, "the 64 x 64 body's stages fit too");
   static LdsOptIn opt_in;
@@ -2277,10 +2297,10 @@ static int launch_gemm_gated_pair(const bf16_t* A, const bf16_t* Bg, const bf16_
     return (int)e;
   }
   int blocks = t128.tiles_m * t128.tiles_n;
-  if (t256.tiles_m * t256.tiles_n > blocks) blocks = t256.tiles_m * t256.tiles_n;
+  if (most[2] > 0 && t256.tiles_m * t256.tiles_n > blocks) blocks = t256.tiles_m * t256.tiles_n;
   if (t64.tiles_m * t64.tiles_n > blocks) blocks = t64.tiles_m * t64.tiles_n;
   hipLaunchKernelGGL(gemm_gated_pair_kernel, dim3(blocks), dim3(256), lds, s, A, Bg, Bu, G, C, M, N, K, valid, t256, t128, t64,
-                     few256, few128, activation);
+                     few, activation);
   IRON_LAUNCH_CHECK();
 }
 

@@ -351,7 +351,8 @@ def test_gemm_under_a_bound_at_the_edges_of_tiles_and_stages(cuda, M, Kdim, N, b
 
 
 @pytest.mark.parametrize("M,Kdim,N,form", [(*s, f) for s in ((2048, 2048, 2048), (2048, 1024, 8192), (1500, 320, 4160))
-                                           for f in ("plain", "residual", "gated", "pair")] + [(2048, 200, 8192, "plain")])
+                                           for f in ("plain", "residual", "gated", "pair")] +
+                         [(2048, 200, 8192, "plain"), (2048, 128, 5632, "pair"), (2000, 192, 888, "pair")])
 def test_a_row_s_products_are_the_same_bits_under_every_bound(cuda, M, Kdim, N, form):
     """A bound on the rows chooses the tile (64, 128 or 256 rows of it), and with it nothing about a row's sums: what a row
     becomes does not depend on how many others there are."""
@@ -372,7 +373,7 @@ def test_a_row_s_products_are_the_same_bits_under_every_bound(cuda, M, Kdim, N, 
         return C, G
 
     whole = run(M)
-    for rows in (5, 64, 128, 129, 256, 257, 384, 385, 513, 896, 897, 1025):
+    for rows in (5, 64, 128, 129, 256, 257, 384, 385, 513, 896, 897, 1025, 1281):
         for got, want in zip(run(rows), whole):
             assert torch.equal(got[:rows], want[:rows]), rows
             assert (got[rows:] == 7).all(), rows
