@@ -2478,15 +2478,49 @@ static int check_gemm(const uint16_t* A, const uint16_t* B, const uint16_t* C, i
   return 0;
 }
 
+// How a product's 128 x 128 tiles are shared (none: slices 0), M and N as the tiles see them, by what was
+// measured, in us.  Unshared: 3 a launch; a stage of 64 k 0.5 a round of 128 x 128 tiles; on the 64 x 64 tiles
+// that few tiles of B (N,K) take, 0.13 to 0.23 up to a block a CU, and 0.14 (a few blocks) to 0.34 where K is no multiple of 64.
+// Shared: the second launch and 0.028 a slice of a tile (its 64 KB out and back) on top, which the slices
+// are chosen against.  Both sides: 97 x 400 x 7392 with B (K,N) 48.8 -> 14.0, 383 x 1472 x 6520 50.7 -> 25.0, 86 x 1728 x
+// 5560 with B (N,K) 26.6 -> 16.0, 5300 x 864 x 7744 (294 tiles) 92 -> 74; not 1024 x 1024 x 4096, 15.5 against 21.2.
+static TileShares gemm_shares_of_tiles(int M, int N, int K, bool b_nk) {
+  const TileShares none{0, 0, 0};
+  const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
+  if (K < BK || tiles > 3 * 256) return none;
+  const int stages = (K + BK - 1) / BK, t = (int)tiles;
+  const int shared = t <= 128 ? t : (t > 256 ? t % 256 : 0);   // all tiles, or those of the last round
+  if (shared == 0 || shared > 128) return none;
+  const int by_cost = (int)(4.2f * sqrtf((float)stages / shared) + 0.5f);
+  int slices = 256 / shared < stages / 6 ? 256 / shared : stages / 6;
+  if (slices > by_cost) slices = by_cost;
+  if (slices < 2) return none;
+  const float fill = (float)((long)((M + 63) / 64) * ((N + 63) / 64)) / 256.f;
+  const float stage64 = K % BK == 0 ? 0.13f + 0.10f * fill : fminf(0.14f + 3.f * fill, 0.22f + 0.12f * fill);
+  const float now = 3.f + stages * (b_nk && t <= 128 ? stage64 : 0.5f * ((t + 255) / 256));
+  const float then = 7.f + 0.028f * slices * shared + 0.5f * ((stages + slices - 1) / slices + stages * ((t - shared) / 256));
+  return then < 0.9f * now ? TileShares{t - shared, shared, slices} : none;
+}
+
 // Whether the few-row kernels take a product of B (N,K).  Their blocks read all of A each, so they grow with rows x K
 // (2048 x 8192 16 / 33 / 63 rows 10.3 / 27.1 / 35.8 us, 5256 x 6192 27 / 44 / 64) where the tiles do not (17.3 and 27);
 // the line lies where the two met over twenty shapes, short K to the few rows (63 x 1304 x 1032 6.4 against 7.8).  Up to sixteen rows
 // of a matrix that the strips take a tile a block stay ahead of the tiles past that line (weights out of memory: 16 rows 2048 x 9216 13.3
 // against 18.2, 2048 x 16384 18.0 against 23.4, 1000 x 16384 15.3 against 17.7, 304 x 14336 13.3 against 13.5; not
-// 14 x 304 x 18944, 16.0 against 14.9).
+// 14 x 304 x 18944, 16.0 against 14.9).  Past the line the few rows stay where what they are measured to take, weights out of memory, is the less:
+// 2.6 us and, a thousand of K, what the rows and the rounds of blocks make of it; the tiles 11 and the matrix at 5 TB/s where they are shared,
+// else 3.3 and their chain of stages, dearer where rows straddle cache lines (few rows against tiles: 45 x 1928 x 3192 16.4 / 23.7, 48 x 3992 x 1424
+// 8.5 / 12.4, 63 x 2048 x 6144 28.9 / 32.7, 16 x 4096 x 10192 24.2 / 31.6, but 40 x 2048 x 8192 28.9 / 17.6, 56 x 6000 x 3192 36.4 / 28.0).
 static bool gemm_of_few_rows(int M, int N, int K) {
+  if (M >= 64) return false;
   if (M <= 16 && N <= 2048 && K <= 16384 && (long)N * K >= (1 << 21)) return true;
-  return M < 64 && (long)M * K < 140000 && (M < 48 || K < 1408);
+  if ((long)M * K < 140000 && (M < 48 || K < 1408)) return true;
+  if (N > 8192 || K < BK) return false;
+  const float rows = M <= 16 ? 1.1f + 0.045f * M : 1.55f + 0.0435f * M;
+  const float each = N < 8192 ? rows * ((N + 4095) / 4096) : (M <= 16 ? 3.5f : 4.15f + 0.028f * M);   // (N = 8192: 32 columns a block)
+  const float stage = K % BK == 0 ? 0.17f + 0.0018f * M : 0.2f + 0.0048f * M, few = 2.6f + 1e-3f * K * each;
+  const float tiles = gemm_shares_of_tiles(M, N, K, true).slices > 0 ? 11.f + 4e-7f * N * K : 3.3f + stage * ((K + BK - 1) / BK);
+  return 1.05f * few < tiles;
 }
 
 // Whether the 256x256 tiles take a product (see iron_gemm_bf16).
@@ -2577,29 +2611,9 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
   return launch_gemm<64, 64, 2, 2>(A, B, C, M, N, K, b_col_maj, c_col_maj, valid, valid_k, s);
 }
 
-// How a product's 128 x 128 tiles are shared (none: slices 0), M and N as the tiles see them, by what was
-// measured, in us.  Unshared: 3 a launch; a stage of 64 k 0.5 a round of 128 x 128 tiles; on the 64 x 64 tiles
-// that few tiles of B (N,K) take, 0.13 to 0.23 up to a block a CU, and 0.14 (a few blocks) to 0.34 where K is no multiple of 64.
-// Shared: the second launch and 0.028 a slice of a tile (its 64 KB out and back) on top, which the slices
-// are chosen against.  Both sides: 97 x 400 x 7392 with B (K,N) 48.8 -> 14.0, 383 x 1472 x 6520 50.7 -> 25.0, 86 x 1728 x
-// 5560 with B (N,K) 26.6 -> 16.0, 5300 x 864 x 7744 (294 tiles) 92 -> 74; not 1024 x 1024 x 4096, 15.5 against 21.2.
 static TileShares gemm_shares(int M, int N, int K, bool b_nk, bool c_nm) {
-  const TileShares none{0, 0, 0};
-  const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
-  if (K < BK || (b_nk && gemm_of_few_rows(M, N, K)) || tiles > 3 * 256) return none;
-  if (!c_nm && gemm_on_big_tiles(M, N, K)) return none;
-  const int stages = (K + BK - 1) / BK, t = (int)tiles;
-  const int shared = t <= 128 ? t : (t > 256 ? t % 256 : 0);   // all tiles, or those of the last round
-  if (shared == 0 || shared > 128) return none;
-  const int by_cost = (int)(4.2f * sqrtf((float)stages / shared) + 0.5f);
-  int slices = 256 / shared < stages / 6 ? 256 / shared : stages / 6;
-  if (slices > by_cost) slices = by_cost;
-  if (slices < 2) return none;
-  const float fill = (float)((long)((M + 63) / 64) * ((N + 63) / 64)) / 256.f;
-  const float stage64 = K % BK == 0 ? 0.13f + 0.10f * fill : fminf(0.14f + 3.f * fill, 0.22f + 0.12f * fill);
-  const float now = 3.f + stages * (b_nk && t <= 128 ? stage64 : 0.5f * ((t + 255) / 256));
-  const float then = 7.f + 0.028f * slices * shared + 0.5f * ((stages + slices - 1) / slices + stages * ((t - shared) / 256));
-  return then < 0.9f * now ? TileShares{t - shared, shared, slices} : none;
+  if ((b_nk && gemm_of_few_rows(M, N, K)) || (!c_nm && gemm_on_big_tiles(M, N, K))) return TileShares{0, 0, 0};
+  return gemm_shares_of_tiles(M, N, K, b_nk);
 }
 
 extern "C" int64_t iron_gemm_workspace_bytes(int M, int N, int K, int b_col_maj, int c_col_maj) {

@@ -331,7 +331,9 @@ static int launch_gemm_strips(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
 // a launch is mostly its start, which gemm_few_kernel's is shorter (777 x 1000, 8 rows: 3.3 against 3.5).
 // K up to eight strips: up to 16 rows of A (8 rows: 8192 x 2048 9.0 / 8.7, 16384 x 1024 12.1 / 10.4, 128256 x 2048 105 / 84), but not short
 // rows that straddle cache lines (16000 x 600 8.7 / 9.4) nor up to four rows where long rows make one round or two
-// (one row: 3072 x 2048 5.1 / 5.6, 4096 x 2048 5.4 / 5.9); more rows, whose sums take a second set of registers, only over a B of 64 MB
+// (one row: 3072 x 2048 5.1 / 5.6, 4096 x 2048 5.4 / 5.9), up to eight of a K under 1408 (eight rows, weights out of memory: 3000 x 1224 4.2 / 4.8), nor
+// where the strips make four tiles a block of what gemm_few_kernel does in two rounds (one row: 6483 x 1360 6.1 / 7.0, 7159 x 2048 7.7 / 8.4; but sixteen rows of
+// it 8.1 / 7.3); more rows, whose sums take a second set of registers, only over a B of 64 MB
 // (20 rows: 128256 x 2048 137 / 87, 16384 x 1024 10.7 / 14.5).
 // A longer K: the strips of A that come with every tile cost as much as B's own.  Up to eight rows where a block has one tile or many
 // (2048 x 8192 13.9 / 8.9, 9048 x 8184 49 / 35, but 4096 x 14336 22.7 / 26.1 and 2728 x 6128 9.9 / 12.3); up to 16 where it
@@ -347,6 +349,8 @@ static int strips_for(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N,
     if (M > 32 || (M > 16 && size < (1 << 25)) || (!on_lines && K < 1024)) return -1;
     if (M > 16) return launch_gemm_strips<2, 16, true, 2, true>(A, B, C, M, N, K, s);
     if (M <= 4 && size <= (1 << 23) && K > 1024 && N > 1536) return -1;
+    if (K > 1024 && N > 2048 && N <= 4096 && M <= 8 && K < 1408) return -1;
+    if (K > 1024 && N > 6144 && N < 8192 && (M <= 4 || (M <= 8 && K < 1280))) return -1;
     if (M <= 8) return launch_gemm_strips<1, 8, true, 2, true>(A, B, C, M, N, K, s);
     return launch_gemm_strips<1, 16, true, 2, true>(A, B, C, M, N, K, s);
   }

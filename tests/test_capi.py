@@ -54,10 +54,11 @@ def test_every_entry_point_refuses_null_operands():
 
 def test_few_rows_over_a_long_k_share_no_tiles():
     """Up to sixteen rows against up to 2048 of a long K go by strips, whatever the product of rows and K; past that, and past
-    K = 16384, their tiles' K is dealt over blocks.  As (N,M) output the same with the operands' places changed."""
+    K = 16384, their tiles' K is dealt over blocks where that takes less than the few rows would.  As (N,M) output the same with the operands' places changed."""
     room = _lib.lib().iron_gemm_workspace_bytes
     for M, N, K, shared in ((16, 2048, 9216, False), (9, 1536, 16384, False), (16, 304, 14336, False), (16, 128, 16384, False),
-                            (16, 120, 16384, True), (16, 2056, 9216, True), (17, 2048, 9216, True), (12, 2048, 16392, True)):
+                            (16, 120, 16384, True), (16, 2056, 9216, True), (17, 2048, 9216, True), (12, 2048, 16392, True),
+                            (16, 4096, 10192, False), (40, 2048, 8192, True), (45, 512, 8184, True)):
         assert (room(M, N, K, 1, 0) > 0) == shared, (M, N, K)
         assert (room(N, M, K, 1, 1) > 0) == shared, (N, M, K)
 
