@@ -44,7 +44,7 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
                                                                        bf16_t* __restrict__ C, int M, int N, int K) {
   typedef Strips<MT, MA, SINGLE, STAGES> S;
   constexpr int W = STRIP_WAVES, R = STRIP_ROWS, GROUP = STRIP_OUT / R;   // GROUP: tiles whose columns are stored together
-  constexpr int NOWHERE = 0x7ffffff0;   // an offset past the end of every run of rows (the entry point bounds M * K)
+  constexpr int NOWHERE = 0x7ffffff0;   // an offset past the end of every run of rows (64 rows of at most 2^22, the entry point's bound, are 2^29 bytes)
   extern __shared__ __align__(1024) char lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l16 = lane & 15, quad = lane >> 4;
   const int strips = (K + STRIP - 1) / STRIP, mine = SINGLE ? 1 : (strips - wave + W - 1) / W, most = SINGLE ? 1 : (strips + W - 1) / W;
@@ -354,7 +354,6 @@ static int strips_for(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N,
     if (M <= 8) return launch_gemm_strips<1, 8, true, 2, true>(A, B, C, M, N, K, s);
     return launch_gemm_strips<1, 16, true, 2, true>(A, B, C, M, N, K, s);
   }
-  if ((long long)64 * K * 2 >= 0x7ffffff0ll) return -1;   // (offsets within 64 rows are 32 bits wide)
   if (M <= 8) {
     if (one_tile) return launch_gemm_strips<1, 8, false, 2, false>(A, B, C, M, N, K, s);
     if (N >= 8192 || (N > 4096 && K < 4096)) return launch_gemm_strips<1, 8, false, 2, true>(A, B, C, M, N, K, s);
