@@ -265,7 +265,7 @@ class Batch:
         try:
             while waiting or running:
                 # All the prompts there are slots for go in together: a portion costs its weights' way through the chip
-                # whatever it holds (eight prompts of 96 to 640 tokens: eight portions of 2.5 ms each, or two; serving them 52 -> 41 ms).
+                # whatever it holds (eight prompts of 96 to 640 tokens: eight portions of 2.5 ms each, or two; serving them 52 -> 42 ms).
                 new = {("generate", id(out), i): i for i in waiting[: len(self._free)]}
                 if new:
                     del waiting[: len(new)]
