@@ -309,7 +309,7 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
   const bool masked_any = causal || window >= 0;
   const int offset = masked_any ? (kv_tokens - q_tokens) : 0;
 
-  // Few live queries (FEW: the launch may have them; the code beside the tiles' costs those 1.5 % at d = 128): groups of 32 take the first blocks, all blocks the zeros of the rows past them.
+  // Few live queries (FEW: the launch may have them; the code beside the tiles' costs those 1.5 to 2.5 % at d = 128): groups of 32 take the first blocks, all blocks the zeros of the rows past them.
   const int groups = FEW ? (q_tokens + 31) >> 5 : 0;
   if (FEW && groups > 0 && groups <= nqb && offset >= 0 &&
       few_rows_pay<D, W>(heads * groups, window < 0 ? kv_tokens : min(kv_tokens, window + q_tokens))) {
