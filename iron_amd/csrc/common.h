@@ -131,6 +131,31 @@ __device__ __forceinline__ void store_stream(uint4* p, const uint4& v) {
   __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(p));
 }
 
+// Four or eight elements to any row of bf16, whatever its alignment (an element's own): this hardware stores several words to
+// any address, and the compiler, told the type's alignment, makes one store of it.
+struct __attribute__((packed, aligned(2))) LooseWords2 {
+  uint32_t w[2];
+};
+struct __attribute__((packed, aligned(2))) LooseWords4 {
+  uint32_t w[4];
+};
+__device__ __forceinline__ void store_loose(bf16_t* p, uint32_t a, uint32_t b) { *reinterpret_cast<LooseWords2*>(p) = LooseWords2{{a, b}}; }
+__device__ __forceinline__ void store_loose(bf16_t* p, const uint4& v) { *reinterpret_cast<LooseWords4*>(p) = LooseWords4{{v.x, v.y, v.z, v.w}}; }
+
+// Up to 8 elements of an output row, `left` of them inside it.  A whole piece leaves by one store wherever its row begins; in pieces that every
+// row begins on, as small as an element where rows are odd, 2048 x 2047 x 2048 took 27.2 us instead of 19.9, 4000 x 4099 x 512 59.6 instead of 40.2,
+// 7137 x 6621 x 256 117 instead of 62 (and 4000 x 4100 x 512, in halves, 41.5 instead of 39.9).
+__device__ __forceinline__ void store_ragged(bf16_t* p, const uint4& v, int left) {
+  if (left >= 8) {
+    store_loose(p, v);
+    return;
+  }
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int e = 0; e < 7; ++e)   // (constant indices: a runtime trip count puts the array in scratch memory)
+    if (e < left) p[e] = (bf16_t)((e & 1) ? (w[e >> 1] >> 16) : (w[e >> 1] & 0xffffu));
+}
+
 // Wave-wide reductions on the DPP data path (no LDS traffic): within quads, half rows and
 // rows, then across rows with the row broadcasts; lane 63 ends with the total.
 #define IRON_DPP(old, v, ctrl, rows) \

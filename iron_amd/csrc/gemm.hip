@@ -249,8 +249,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(const bf16_t* __restrict__ A,
           const int m = mb + frag_row, n = nb + 8 * q + hi;
           if (m >= Mv || n >= N) continue;
           bf16_t* p = C + (size_t)m * N + n;
-          if (n + 4 <= N && (N & 3) == 0) {
-            *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16(v0, v1), pack_bf16(v2, v3));
+          if (n + 4 <= N) {
+            store_loose(p, pack_bf16(v0, v1), pack_bf16(v2, v3));
           } else {
             const float v[4] = {v0, v1, v2, v3};
 #pragma unroll
@@ -261,8 +261,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(const bf16_t* __restrict__ A,
           const int n = nb + frag_row, m = mb + 8 * q + hi;
           if (n >= N || m >= Mv) continue;
           bf16_t* p = C + (size_t)n * M + m;
-          if (m + 4 <= Mv && (M & 3) == 0) {
-            *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16(v0, v1), pack_bf16(v2, v3));
+          if (m + 4 <= Mv) {
+            store_loose(p, pack_bf16(v0, v1), pack_bf16(v2, v3));
           } else {
             const float v[4] = {v0, v1, v2, v3};
             for (int e = 0; e < 4 && m + e < Mv; ++e) p[e] = f32_to_bf16(v[e]);
@@ -394,24 +394,6 @@ __device__ __forceinline__ void tail_of(const QkvTail& qkv, float (&x)[COUNT], c
     gate(std::integral_constant<int, 2>{});
   } else {
     gate(std::integral_constant<int, 3>{});
-  }
-}
-
-// Up to 8 elements of an output row of `cols`, `left` of them inside it, in the widest pieces that every row of C begins on (C itself does on
-// 16 bytes, `p` is a multiple of 8 elements into its row).  An element at a time a 7137 x 6620 output took 104 us instead of 53.
-__device__ __forceinline__ void store_ragged(bf16_t* p, const uint4& v, int left, int cols) {
-  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-  if ((cols & 3) == 0) {
-    *reinterpret_cast<uint2*>(p) = make_uint2(w[0], w[1]);
-    if (left > 4) *reinterpret_cast<uint2*>(p + 4) = make_uint2(w[2], w[3]);
-  } else if ((cols & 1) == 0) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (2 * e < left) *reinterpret_cast<uint32_t*>(p + 2 * e) = w[e];
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e)   // (constant indices: a runtime trip count puts the array in scratch memory)
-      if (e < left) p[e] = (bf16_t)((e & 1) ? (w[e >> 1] >> 16) : (w[e >> 1] & 0xffffu));
   }
 }
 
@@ -617,8 +599,8 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
 #pragma unroll
           for (int e = 0; e < 4; ++e) acc[i][j][e] = prod[e];
         }
-        if (vec) {
-          *reinterpret_cast<uint2*>(row + n) = make_uint2(pack_bf16(acc[i][j][0], acc[i][j][1]), pack_bf16(acc[i][j][2], acc[i][j][3]));
+        if (n + 4 <= N) {
+          store_loose(row + n, pack_bf16(acc[i][j][0], acc[i][j][1]), pack_bf16(acc[i][j][2], acc[i][j][3]));
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
@@ -1001,7 +983,7 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
       if (out_m >= M || n0 + wn * 64 + row >= N) continue;
       bf16_t* p = C + (size_t)(n0 + wn * 64 + row) * M + out_m;
       if (whole_m) *reinterpret_cast<uint4*>(p) = v;
-      else store_ragged(p, v, M - out_m, M);
+      else store_ragged(p, v, M - out_m);
     }
     return;
   }
@@ -1028,7 +1010,7 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
       }
     }
     if (whole) *reinterpret_cast<uint4*>(p) = v;
-    else store_ragged(p, v, N - out_n, N);
+    else store_ragged(p, v, N - out_n);
   }
 }
 
@@ -2190,7 +2172,7 @@ __device__ __forceinline__ void gemm_nt16_pair_body(const bf16_t* __restrict__ A
       if (m >= Mv || out_n >= N) continue;
       bf16_t* p = to + (size_t)m * N + out_n;
       if (whole) *reinterpret_cast<uint4*>(p) = v;
-      else store_ragged(p, v, N - out_n, N);
+      else store_ragged(p, v, N - out_n);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();   // the rows are read before the next product overwrites them
@@ -2409,13 +2391,7 @@ __global__ __launch_bounds__(256) void gemm_shared_finish_kernel(const float* __
   if (row >= rows || col >= cols) return;
   bf16_t* to = C + (size_t)row * cols + col;
   const uint32_t w[4] = {pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3])};
-  if ((cols & 7) == 0) {
-    *reinterpret_cast<uint4*>(to) = make_uint4(w[0], w[1], w[2], w[3]);
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      if (col + e < cols) to[e] = (bf16_t)((e & 1) ? (w[e >> 1] >> 16) : (w[e >> 1] & 0xffffu));
-  }
+  store_ragged(to, make_uint4(w[0], w[1], w[2], w[3]), cols - col);
 }
 
 template <bool B_KN, bool C_NM>

@@ -319,6 +319,28 @@ def test_gemm_rows_that_are_no_whole_pieces(cuda, cols, form):
     assert bool((buf[M * cols:] == 3).all())
 
 
+@pytest.mark.parametrize("cols", [1, 2, 3, 5, 6, 7, 8])
+@pytest.mark.parametrize("M,Kdim,N,b_col_maj,c_col_maj", [
+    (8, 2048, 1032, True, False), (30, 4096, 808, True, False),     # strips, a tile a block
+    (5, 1024, 16384, True, False), (16, 2048, 4096, True, False),   # ... several
+    (40, 264, 72, True, False), (9, 64, 8200, True, False),         # few rows otherwise, 16 columns a block and 32
+    (200, 200, 328, True, False), (24, 6200, 200, True, False),     # 64 x 64 tiles, shared tiles
+    (136, 40, 200, True, False), (200, 40, 136, False, True),       # the general kernel, C as (M,N) and (N,M)
+])
+def test_gemm_rows_of_every_alignment(cuda, M, Kdim, N, b_col_maj, c_col_maj, cols):
+    """Rows of every remainder of eight elements through every other kernel's stores: each begins where it begins, the columns
+    at its end, and nothing past the output's."""
+    M, N = (M + cols, N) if c_col_maj else (M, N + cols)
+    rng = np.random.default_rng(M + N)
+    A, B = bf(rng, M, Kdim), bf(rng, (N if b_col_maj else Kdim), (Kdim if b_col_maj else N), scale=0.05)
+    buf = out_like((M * N + 64,), cuda, fill=3.0)
+    C = buf[: M * N].view(*((N, M) if c_col_maj else (M, N)))
+    K.gemm(dev(A, cuda), dev(B, cuda), C, M=M, N=N, K=Kdim, b_col_maj=b_col_maj, c_col_maj=c_col_maj)
+    kw = dict(b_col_maj=b_col_maj, c_col_maj=c_col_maj)
+    assert np.all(np.abs(from_torch(C) - ops.gemm(A, B, **kw)) <= ops.gemm_bound(A, B, **kw))
+    assert bool((buf[M * N:] == 3).all())
+
+
 @pytest.mark.parametrize("M,Kdim,N,b_col_maj,bounds", [
     (2048, 200, 8192, True, (1, 128, 129, 1024, 1025, 2047)),    # 64, 128 and 256 tiles by the bound
     (1500, 328, 2056, True, (63, 895, 896, 897, 1500)),          # 64 and 128 ones, ragged
