@@ -340,26 +340,27 @@ __device__ __forceinline__ void to_cache_rows(QkvTail& t, const int* __restrict_
 // Which tile a block computes.  Blocks are dispatched in id order and dealt round-robin over the 8
 // XCDs, each with an L2 of its own, so the order is chosen for what an XCD's blocks share:
 // `patched` (whole 8 x 4-tile patches, a multiple of 8 of them): an XCD owns patches, whose A and B
-// panels it re-reads from its own L2.  Few tile rows (under 8, and a multiple of 8 tile columns,
-// e.g. the 512 live rows of a prompt chunk): an XCD owns whole columns of tiles, so the weight tile
-// its blocks share crosses HBM once instead of once an XCD.  Otherwise bands of 8 tile rows.
+// panels it re-reads from its own L2.  Otherwise the tiles in bands of 8 tile rows, a band's columns one after the other, and an XCD
+// owns an eighth of that order in one piece: the weight tile that its blocks share crosses HBM once instead of once an XCD
+// (against tile rows dealt round-robin: 7058 x 12872 x 792 174 -> 157 us, 941 x 9386 x 5296 121 -> 112, 181 x 10780 x 272 8.5 -> 7.5).  A matrix more than
+// twice as tall as wide goes by columns for rows (2056 x 713 x 1136 12.9 -> 11.5).
 __device__ __forceinline__ void tile_of_block(int bid, int tiles_m, int tiles_n, int patched, int& tm, int& tn) {
+  const int xcd = bid & 7, loc = bid >> 3;
   if (patched) {
-    const int xcd = bid & 7, loc = bid >> 3;
     const int patch = (loc >> 5) * 8 + xcd, within = loc & 31;
     const int patches_n = tiles_n >> 2;
     tm = (patch / patches_n) * 8 + (within & 7);
     tn = (patch % patches_n) * 4 + (within >> 3);
-  } else if (tiles_m < 8 && (tiles_n & 7) == 0) {
-    const int xcd = bid & 7, loc = bid >> 3;
-    tm = loc % tiles_m;
-    tn = (loc / tiles_m) * 8 + xcd;
   } else {
-    constexpr int BAND = 8;
-    const int per_band = BAND * tiles_n, band = bid / per_band, first = band * BAND;
-    const int height = min(BAND, tiles_m - first), in_band = bid - band * per_band;
-    tm = first + in_band % height;
-    tn = in_band / height;
+    const int tiles = tiles_m * tiles_n, at = xcd * (tiles >> 3) + min(xcd, tiles & 7) + loc;
+    const bool tall = tiles_m > 2 * tiles_n;
+    const int across = tall ? tiles_n : tiles_m, along = tall ? tiles_m : tiles_n;
+    // (eight by four tiles are an XCD's CUs; up to three left over join the last band)
+    const int band = min(at / (8 * along), max(1, (across + 4) >> 3) - 1), first = band * 8;
+    const int width = first + 12 > across ? across - first : 8, in_band = at - first * along;
+    const int l = in_band / width, c = first + in_band - l * width;
+    tm = tall ? l : c;
+    tn = tall ? c : l;
   }
 }
 
@@ -1403,26 +1404,15 @@ static int launch_gemm(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N
 }
 
 
-// Large problems, B (N,K): 256x256x64 tiles, two 64 KB stages fed straight into LDS.  Against the
-// 128x128 kernel a CU pulls half as many global bytes per flop -- the 64 B/clk a CU can move from L2
-// into LDS is what bounds the smaller tile.  Eight waves, two a SIMD, each owning 128 x 64 of the
-// tile (32 accumulator tiles of 16 x 16, 128 accumulation registers): one's loads and fragment reads
-// issue under the other's MFMAs (2048 x 8192 x 2048 60.5 -> 56.5 us, 4096^3 111 -> 107.5 against four
-// waves of 128 x 128; 8192^3 the same).  Within a wave the instruction stream still interleaves the
-// next k-step's fragment reads and the next stages' loads with the MFMAs.  Where the blocks of one
-// launch choose their tile size by a row bound (gemm_either_kernel) the large tile is four waves of
+// Large problems: whole tiles of up to 256 x 256 outputs on eight waves (two a SIMD: one's loads and fragment reads issue under the
+// other's MFMAs; 2048 x 8192 x 2048 60.5 -> 56.5 us, 4096^3 111 -> 107.5 against four waves of 128 x 128; 8192^3 the same), stages of 64
+// k fed straight into LDS.  Against the 128x128 kernel a CU pulls half as many global bytes per flop -- the 64 B/clk a CU can move
+// from L2 into LDS is what bounds the smaller tile.  WM x WN waves, each owning MI x NT accumulator tiles of 16 x 16: the
+// tile's height and width are then chosen by how the product's rounds over the chip come out (see big_tiling).  Within a wave
+// the instruction stream still interleaves the next k-step's fragment reads and the next stages' loads with the MFMAs.  Where the
+// blocks of one launch choose their tile size by a row bound (gemm_either_kernel) the large tile is four waves of
 // 128 x 128, as every other tiling of that launch is four waves.
 constexpr int BIG_BM = 256, BIG_BN = 256;
-#ifndef IRON_BIG_WAVES
-#define IRON_BIG_WAVES 8   // the stand-alone launch: two waves a SIMD, each 128 x 64 of the tile (4: one, 128 x 128)
-#endif
-constexpr int BIG_WAVES = IRON_BIG_WAVES;
-#ifndef IRON_BIG_KB
-#define IRON_BIG_KB 64
-#endif
-constexpr int BIG_KB = IRON_BIG_KB;   // k per stage: 64 (2 stages); 32 (4 stages of half-line rows) measured 13 % slower
-#define BIG_OUT_ROW_BYTES(TN) ((TN) * 64 + 16)
-constexpr int BIG_STAGE_BYTES = (BIG_BM + BIG_BN) * BK * 2;
 
 // The operands of a gated feed-forward's two first projections beyond the gate's own.
 struct GatedPair {
@@ -1431,105 +1421,123 @@ struct GatedPair {
   int activation;
 };
 
-template <int WAVES, int KB, bool B_KN = false, bool STREAM_OUT = false, bool PAIR = false>
-__device__ __forceinline__ void gemm_nt256_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
-                                                bf16_t* __restrict__ C, int M, int N, int K,
-                                                const int* __restrict__ valid, int tiles_m, int tiles_n,
-                                                int patched, const GatedPair& pair = GatedPair{}) {
-  static_assert(KB == 64, "k per stage: 64 (32 with four stages of half-line rows measured 13 % slower)");
-  constexpr int ROWB = KB * 2;               // bytes of a tile row in LDS
-  constexpr int CPR = KB / 8;                // its 16-byte chunks
-  constexpr int RPI = 1024 / ROWB;           // rows one 1 KB load covers
-  constexpr int A_BYTES = BIG_BM * ROWB, STAGE_BYTES = (BIG_BM + BIG_BN) * ROWB;
-  constexpr int STAGES = KB == 64 ? 2 : 4;   // 128 KB either way
-  constexpr int INST = BIG_BM / RPI / WAVES; // 1 KB loads of A (and of B) a wave issues per stage
-  constexpr int TN = 8 / WAVES * 2;          // 32-column MFMA tiles a wave owns along n (4 or 2)
+template <int WM_, int WN_, int MI_, int NT_>
+struct BigTile {
+  static constexpr int WM = WM_, WN = WN_, MI = MI_, NT = NT_, WAVES = WM * WN, BM = WM * MI * 16, BN = WN * NT * 16;
+  static constexpr int STAGE_BYTES = (BM + BN) * BK * 2;
+  // Three stages where they fit beside the 1 KB that loads without rows go to: a stage's loads then have a whole stage's time to land.
+  static constexpr int STAGES = 3 * STAGE_BYTES + 1024 <= 160 * 1024 ? 3 : 2;
+  static constexpr int OUT_ROW_BYTES = NT * 32 + 16, OUT_BYTES = WAVES * MI * 16 * OUT_ROW_BYTES;
+  static constexpr int LDS_BYTES = STAGES * STAGE_BYTES + 1024 > OUT_BYTES ? STAGES * STAGE_BYTES + 1024 : OUT_BYTES;
+};
+
+template <class T, bool B_KN = false, bool STREAM_OUT = false, bool PAIR = false>
+__device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
+                                              bf16_t* __restrict__ C, int M, int N, int K,
+                                              const int* __restrict__ valid, int tiles_m, int tiles_n,
+                                              int patched, const GatedPair& pair = GatedPair{}) {
+  constexpr int WAVES = T::WAVES, MI = T::MI, NT = T::NT, STAGES = T::STAGES;
+  constexpr int ROWB = BK * 2;                                        // bytes of a tile row in LDS, eight 16-byte chunks
+  constexpr int A_BYTES = T::BM * ROWB, STAGE_BYTES = T::STAGE_BYTES;
+  constexpr int A_INST = T::BM / 8, B_INST = T::BN / 8;               // 1 KB loads of a stage: eight rows each
+  constexpr int A_EACH = (A_INST + WAVES - 1) / WAVES, B_EACH = (B_INST + WAVES - 1) / WAVES, LOADS = A_EACH + B_EACH;   // ... a wave's
+  constexpr int A_LAST = A_INST % WAVES, B_LAST = B_INST % WAVES;     // waves that have a last one (0: all)
   extern __shared__ __align__(16) char smem_big[];
   const int Mv = bound_or(valid, M);
 
   int tm, tn;
-  if (!live_tile(blockIdx.x, tiles_m, tiles_n, patched, (Mv + BIG_BM - 1) / BIG_BM, tm, tn)) return;
-  if (tm * BIG_BM >= Mv) return;
+  if (!live_tile(blockIdx.x, tiles_m, tiles_n, patched, (Mv + T::BM - 1) / T::BM, tm, tn)) return;
+  if (tm * T::BM >= Mv) return;
   // The last tile of each direction is moved back to end at the matrix's edge, so that every tile is
   // whole; what two tiles both cover comes out the same from both.
-  const int m0 = min(tm * BIG_BM, M - BIG_BM), n0 = PAIR ? tn * (BIG_BN / 2) : min(tn * BIG_BN, N - BIG_BN);
+  const int m0 = min(tm * T::BM, M - T::BM), n0 = PAIR ? tn * (T::BN / 2) : min(tn * T::BN, N - T::BN);
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // uniform: LDS and global bases stay in scalar registers
-  const int wm = wave / (WAVES / 2), wn = wave % (WAVES / 2);
-  // Loader: instruction i of a wave moves rows (wave*INST + i)*RPI .. ; lane -> (row, physical
-  // chunk); the logical chunk it fetches is the physical one swizzled by the row.
-  const int lrow = lane / CPR, pch = lane % CPR;
-  unsigned ld_off[2];   // byte offset of this lane's 16 bytes within an even / odd instruction's rows
-  int ld_head[2];       // ... and the k of a stage at which they begin
-#pragma unroll
-  for (int par = 0; par < 2; ++par) {
-    const int r = par * RPI + lrow;
-    ld_head[par] = (pch ^ ((r >> 1) & (CPR - 1))) * 8;
-    ld_off[par] = (unsigned)(((size_t)lrow * K + (pch ^ ((r >> 1) & (CPR - 1))) * 8) * 2);
-  }
-  // Loads go out as buffer loads straight into LDS: the rows a wave fetches are one buffer, the
-  // lane's place within an instruction's rows is the (constant) vector offset and the instruction's
-  // rows and the stage's k are the scalar offset, so a load costs two scalar adds and no vector ALU
-  // work between two MFMAs.
+  const int wm = wave / T::WN, wn = wave % T::WN;
+  // Loader: a wave's instruction i moves rows 8 (i WAVES + wave) .. + 7; lane -> (row, physical chunk); the logical chunk it
+  // fetches is the physical one swizzled by the row.  Loads go out as buffer loads straight into LDS: the lane's
+  // place within an instruction's rows is the (constant) vector offset, the instruction's rows and the
+  // stage's k are the scalar offset, so a load costs two scalar adds and no vector ALU work between two MFMAs.
+  const int lrow = lane >> 3, ld_head = ((lane & 7) ^ ((wave & 1) * 4 + (lrow >> 1))) * 8;   // ld_head: the k of a stage at which the lane's piece begins
+  static_assert(WAVES % 2 == 0, "a wave's instructions all begin on an even eight rows, or all on an odd");
+  const int ld_off = (int)(((size_t)lrow * K + ld_head) * 2);
   const int pad = k_pad(K);
-  const __amdgpu_buffer_rsrc_t a_rows = stage_rows(A + (size_t)(m0 + wave * INST * RPI) * K - pad);
-  // B as (K,N) lands as stored: the stage's 64 k-rows of 256 columns (512 bytes a row, two rows an
-  // instruction), a row's 32 chunks XORed with kn_swizzle(row) so that the transposing reads below
-  // find the four rows of a 16-lane group, and the groups of a pass, in different banks.
-  const __amdgpu_buffer_rsrc_t b_rows =
-      PAIR ? stage_rows(((wave & 1) ? pair.up : B) + (size_t)(n0 + (wave >> 1) * INST * RPI) * K - pad) :
-      stage_rows(B_KN ? B + n0 + ((ptrdiff_t)(wave * INST * 2) - pad) * N : B + (size_t)(n0 + wave * INST * RPI) * K - pad);
+  const __amdgpu_buffer_rsrc_t a_rows = stage_rows(A + (size_t)(m0 + wave * 8) * K - pad);
+  // B as (K,N) lands as stored: the stage's 64 k-rows of BN columns, a row's chunks XORed with kn_swizzle(row) so that the
+  // transposing reads below find the four rows of a 16-lane group, and the groups of a pass, in different banks.
+  constexpr int KN_CHUNKS = T::BN / 8, KN_ROWS = 64 / KN_CHUNKS;   // chunks of a k-row, k-rows of an instruction
+  static_assert(!B_KN || KN_CHUNKS == 32, "(K,N): rows of 256 columns");
   auto kn_swizzle = [](int k) { return ((k & 3) << 1) | (((k >> 3) & 3) << 3); };
-  int kn_off[INST];   // (K,N): this lane's 16 bytes within instruction idx's two rows
+  // (PAIR: 64 rows of the gate's weights, 64 of the up projection's, and so on.)
+  const __amdgpu_buffer_rsrc_t b_rows = stage_rows(B_KN ? B + n0 + ((ptrdiff_t)(wave * KN_ROWS) - pad) * N : B + (size_t)(n0 + wave * 8) * K - pad);
+  const __amdgpu_buffer_rsrc_t up_rows = PAIR ? stage_rows(pair.up + (size_t)(n0 + wave * 8) * K - pad) : b_rows;
+  int kn_off[B_EACH], kn_row[B_EACH];   // (K,N): this lane's 16 bytes within instruction idx's k-rows, and the k-row
 #pragma unroll
-  for (int idx = 0; idx < INST; ++idx) {
-    const int kr = (wave * INST + idx) * 2 + (lane >> 5);   // the lane's k-row of the stage
-    kn_off[idx] = (int)(((size_t)(lane >> 5) * N + ((lane & 31) ^ kn_swizzle(kr)) * 8) * 2);
+  for (int i = 0; i < B_EACH; ++i) {
+    kn_row[i] = (i * WAVES + wave) * KN_ROWS + lane / KN_CHUNKS;
+    kn_off[i] = (int)(((size_t)(lane / KN_CHUNKS) * N + ((lane % KN_CHUNKS) ^ kn_swizzle(kn_row[i])) * 8) * 2);
   }
-  const int inst_stride = RPI * K * 2;
+  const int inst_stride = WAVES * 8 * K * 2;
+  static_assert(!PAIR || WAVES == 4, "PAIR: the rows of an instruction below are four waves'");
   auto issue_one = [&](char* st, int kt, int idx, bool head) {
-    const int k_off = kt * KB * 2;
-    if (idx < INST)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rows, IRON_LDS_PTR(st + (wave * INST + idx) * 1024), 16,
-                                               head && ld_head[idx & 1] < pad ? NOWHERE : (int)ld_off[idx & 1],
-                                               idx * inst_stride + k_off, 0, 0);
+    const int k_off = kt * ROWB;
+    const bool is_a = idx < A_EACH;
+    const int i = is_a ? idx : idx - A_EACH;
+    const int last = is_a ? A_LAST : B_LAST;
+    // A wave without a last instruction issues it all the same, from past the buffer's end and to where nobody reads: every wave's
+    // loads are then as many, which the waits count.
+    const bool none = last != 0 && i == (is_a ? A_EACH : B_EACH) - 1 && wave >= last;
+    char* to = none ? smem_big + STAGES * STAGE_BYTES : st + (is_a ? 0 : A_BYTES) + (i * WAVES + wave) * 1024;
+    if (is_a)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rows, IRON_LDS_PTR(to), 16, none || (head && ld_head < pad) ? NOWHERE : ld_off,
+                                               i * inst_stride + k_off, 0, 0);
+    else if constexpr (PAIR)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds((i >> 1) & 1 ? up_rows : b_rows, IRON_LDS_PTR(to), 16, head && ld_head < pad ? NOWHERE : ld_off,
+                                               ((i >> 2) * 2 + (i & 1)) * inst_stride + k_off, 0, 0);
     else if constexpr (!B_KN)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rows, IRON_LDS_PTR(st + A_BYTES + (wave * INST + idx - INST) * 1024),
-                                               16, head && ld_head[idx & 1] < pad ? NOWHERE : (int)ld_off[idx & 1],
-                                               (idx - INST) * inst_stride + k_off, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rows, IRON_LDS_PTR(to), 16, none || (head && ld_head < pad) ? NOWHERE : ld_off,
+                                               i * inst_stride + k_off, 0, 0);
     else
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rows, IRON_LDS_PTR(st + A_BYTES + (wave * INST + idx - INST) * 1024),
-                                               16, head && (wave * INST + idx - INST) * 2 + (lane >> 5) < pad ? NOWHERE : kn_off[idx - INST],
-                                               ((idx - INST) * 2 + kt * KB) * N * 2, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rows, IRON_LDS_PTR(to), 16, head && kn_row[i] < pad ? NOWHERE : kn_off[i],
+                                               (i * WAVES * KN_ROWS + kt * BK) * N * 2, 0, 0);
   };
 
   // The product runs on 16x16x32 MFMAs (a k-step is 32 wide, two a stage): on random operands the
   // part sustains about a sixth more of them than of the 32x32x16 form, at the same registers and
-  // the same LDS reads per flop.  A wave's 128 x 128 is 8 x NT tiles of 16 x 16.
-  constexpr int NT = TN * 2;                 // 16-column tiles a wave owns along n
-  f32x4 acc[8][NT];
+  // the same LDS reads per flop.
+  f32x4 acc[MI][NT];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.f;
 
-  const int nk = (K + pad) / KB;
-  static_assert(KB == 64 && (WAVES == 4 || WAVES == 8), "the loop below is written for two 64-wide stages and four or eight waves");
-  // A stage's 2 INST loads go out in two halves of INST: the first under the last quarter of the
-  // stage two before it (right after that stage's barrier freed the buffer), the second under the
-  // first quarter of the stage before it; two quarters later, at that stage's barrier, all have landed.
-  auto issue_half = [&](char* st, int kt, int half, int slot) { issue_one(st, kt, half * INST + slot, false); };
+  const int nk = (K + pad) / BK;
+  // A stage is two k-steps of MI NT MFMAs; source order is issue order (nothing crosses a sched_barrier): after an MFMA one
+  // fragment read or one load goes out.  A k-step's first MFMAs need all of its B fragments and its first A fragment, so
+  // B's are read first.
+  //   first k-step: the second's B fragments from the start and its A fragments from the middle; loads in the slots between (EARLY of them)
+  //   second k-step: up to slot BARRIER nothing -- then the stage's one barrier: every wave's loads of stage kt + 1 have landed and
+  //     nobody reads stage kt any more (this k-step's fragments are in registers) -- then stage kt + 1's first fragments and LATE loads
+  // With two stages the late loads are the first of stage kt + 2, into this stage's buffer, the early ones the rest of stage kt + 1's; with three
+  // all are stage kt + 2's, into the buffer that the last barrier freed.
+  constexpr int SLOTS = MI * NT, A_FROM = NT > SLOTS / 2 ? NT : SLOTS / 2, FREE = SLOTS - NT - MI;
+  constexpr int EARLY = STAGES == 3 ? (LOADS < FREE ? LOADS : FREE) : LOADS - LOADS / 2, LATE = LOADS - EARLY;
+  constexpr int BARRIER = SLOTS - NT - MI - LATE < SLOTS / 2 ? SLOTS - NT - MI - LATE : SLOTS / 2;
+  static_assert(A_FROM + MI <= SLOTS && EARLY <= FREE && BARRIER >= 0, "a k-step has a slot for each of its reads and loads");
+  constexpr int GAP = A_FROM - NT, APART = EARLY > 0 && GAP / EARLY > 1 ? GAP / EARLY : 1;   // slots between the B and the A reads
+  constexpr int IN_GAP = EARLY < GAP / APART ? EARLY : GAP / APART;
+  constexpr int Q3_FIRST = BARRIER + NT + MI, Q3_EVERY = SLOTS - Q3_FIRST > 2 * LATE && LATE > 0 ? (SLOTS - Q3_FIRST) / (LATE > 0 ? LATE : 1) : 1;
 #pragma unroll
-  for (int idx = 0; idx < 2 * INST; ++idx) issue_one(smem_big, 0, idx, true);
+  for (int idx = 0; idx < LOADS; ++idx) issue_one(smem_big, 0, idx, true);
 #pragma unroll
-  for (int slot = 0; slot < INST; ++slot) issue_half(smem_big + STAGE_BYTES, min(1, nk - 1), 0, slot);
+  for (int idx = 0; idx < (STAGES == 3 ? LOADS : LATE); ++idx) issue_one(smem_big + STAGE_BYTES, min(1, nk - 1), idx, false);
 
   // Fragments: lane -> row fr of a 16-row tile, 16-byte chunk kq of the k-step's four.
   const int fr = lane & 15, kq = lane >> 4;
-  const int swz = (fr >> 1) & (CPR - 1);   // tile rows are multiples of 16 apart: one swizzle for all
-  const int a_row = (wm * 128 + fr) * ROWB, b_row = A_BYTES + (wn * NT * 16 + fr) * ROWB;
+  const int swz = fr >> 1;   // tile rows are multiples of 16 apart: one swizzle for all
+  const int a_row = (wm * MI * 16 + fr) * ROWB, b_row = A_BYTES + (wn * NT * 16 + fr) * ROWB;
   auto a_frag = [&](const char* st, int ks, int i) {
     return *reinterpret_cast<const bf16x8*>(st + a_row + i * 16 * ROWB + (((ks * 4 + kq) ^ swz) << 4));
   };
@@ -1551,16 +1559,16 @@ __device__ __forceinline__ void gemm_nt256_body(const bf16_t* __restrict__ A, co
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     const int n = tr_n + j * 16;
-    kn_lane[j] = kn_base + (((n >> 3) ^ kn_swizzle(tr_k)) << 4) + ((n & 4) << 1) + tr_k * 512;
+    kn_lane[j] = kn_base + (((n >> 3) ^ kn_swizzle(tr_k)) << 4) + ((n & 4) << 1) + tr_k * (T::BN * 2);
   }
   auto b_frag_kn = [&](int stage_bytes, int ks, int j, TrFrag& t) {
     const unsigned at = kn_lane[j] + stage_bytes;
     if (ks == 0) {
       t.lo = lds_read_tr16_at<0>(at);
-      t.hi = lds_read_tr16_at<4 * 512>(at);
+      t.hi = lds_read_tr16_at<4 * T::BN * 2>(at);
     } else {
-      t.lo = lds_read_tr16_at<32 * 512>(at);
-      t.hi = lds_read_tr16_at<36 * 512>(at);
+      t.lo = lds_read_tr16_at<32 * T::BN * 2>(at);
+      t.hi = lds_read_tr16_at<36 * T::BN * 2>(at);
     }
   };
   // (K,N): the A fragments are read by uncounted reads as well, so that every wait of the loop is
@@ -1580,34 +1588,27 @@ __device__ __forceinline__ void gemm_nt256_body(const bf16_t* __restrict__ A, co
     else out = lds_read_b128_at<7 * 16 * ROWB>(at);
   };
   TrFrag tfb[2][NT];
+  bf16x8 af[2][MI], bfr[2][NT];
   // The compiler does not count these reads: a k-step's fragments pass through this wait (every LDS
   // read issued so far) before they are used.
-  auto join_b = [&](int ks, bf16x8 (&b)[NT], bf16x8 (&a)[8]) {
-    i32x4 a0 = __builtin_bit_cast(i32x4, a[0]), a1 = __builtin_bit_cast(i32x4, a[1]), a2 = __builtin_bit_cast(i32x4, a[2]),
-          a3 = __builtin_bit_cast(i32x4, a[3]), a4 = __builtin_bit_cast(i32x4, a[4]), a5 = __builtin_bit_cast(i32x4, a[5]),
-          a6 = __builtin_bit_cast(i32x4, a[6]), a7 = __builtin_bit_cast(i32x4, a[7]);
-    if constexpr (NT == 4)
-      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(tfb[ks][0].lo), "+v"(tfb[ks][0].hi), "+v"(tfb[ks][1].lo), "+v"(tfb[ks][1].hi),
-                                             "+v"(tfb[ks][2].lo), "+v"(tfb[ks][2].hi), "+v"(tfb[ks][3].lo), "+v"(tfb[ks][3].hi),
-                                             "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(a4), "+v"(a5), "+v"(a6), "+v"(a7));
-    else
-      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(tfb[ks][0].lo), "+v"(tfb[ks][0].hi), "+v"(tfb[ks][1].lo), "+v"(tfb[ks][1].hi),
-                                             "+v"(tfb[ks][2].lo), "+v"(tfb[ks][2].hi), "+v"(tfb[ks][3].lo), "+v"(tfb[ks][3].hi),
-                                             "+v"(tfb[ks][4].lo), "+v"(tfb[ks][4].hi), "+v"(tfb[ks][5].lo), "+v"(tfb[ks][5].hi),
-                                             "+v"(tfb[ks][6].lo), "+v"(tfb[ks][6].hi), "+v"(tfb[ks][7].lo), "+v"(tfb[ks][7].hi),
-                                             "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(a4), "+v"(a5), "+v"(a6), "+v"(a7));
-    a[0] = __builtin_bit_cast(bf16x8, a0); a[1] = __builtin_bit_cast(bf16x8, a1); a[2] = __builtin_bit_cast(bf16x8, a2);
-    a[3] = __builtin_bit_cast(bf16x8, a3); a[4] = __builtin_bit_cast(bf16x8, a4); a[5] = __builtin_bit_cast(bf16x8, a5);
-    a[6] = __builtin_bit_cast(bf16x8, a6); a[7] = __builtin_bit_cast(bf16x8, a7);
+  auto join_kn = [&](int ks) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-    for (int j = 0; j < NT; ++j) b[j] = tr_join(tfb[ks][j]);
+    for (int j = 0; j < NT; ++j) asm volatile("" : "+v"(tfb[ks][j].lo), "+v"(tfb[ks][j].hi));
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      i32x4 a = __builtin_bit_cast(i32x4, af[ks][i]);
+      asm volatile("" : "+v"(a));
+      af[ks][i] = __builtin_bit_cast(bf16x8, a);
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) bfr[ks][j] = tr_join(tfb[ks][j]);
   };
 
-  wait_vmcnt<INST>();   // stage 0 has landed once only stage 1's first half is out
+  wait_vmcnt<STAGES == 3 ? LOADS : LATE>();   // stage 0 has landed once only what was issued of stage 1 is out
   block_barrier();
-  bf16x8 af[2][8], bfr[2][NT];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < MI; ++i) {
     if constexpr (B_KN) a_frag_kn(0, 0, i, af[0][i]);
     else af[0][i] = a_frag(smem_big, 0, i);
   }
@@ -1616,69 +1617,68 @@ __device__ __forceinline__ void gemm_nt256_body(const bf16_t* __restrict__ A, co
     if constexpr (B_KN) b_frag_kn(0, 0, j, tfb[0][j]);
     else bfr[0][j] = b_frag(smem_big, 0, j);
   }
+  int now = 0, next = 1;   // kt % STAGES and (kt + 1) % STAGES
   for (int kt = 0; kt < nk; ++kt) {
     // Past the end the last stage is fetched again (into buffers nobody reads any more) rather than
     // branch: a branch would end the scheduling region and undo the interleaving below.
     const int k1 = min(kt + 1, nk - 1), k2 = min(kt + 2, nk - 1);
-    char* st = smem_big + (kt % STAGES) * STAGE_BYTES;          // this stage; then stage kt+2's buffer
-    char* nst = smem_big + ((kt + 1) % STAGES) * STAGE_BYTES;   // stage kt+1's
-    // A stage is two k-steps of 8 NT MFMAs, scheduled as four quarters (tile rows 0..3 and 4..7 of
-    // a k-step).  Source order is issue order (nothing crosses a sched_barrier): after an MFMA one
-    // fragment read or one load goes out.  A k-step's first MFMAs need all of its B fragments and
-    // its first A fragment, so B's are read first.
-    //   quarter 0: the second k-step's B fragments, and the second half of stage kt+1's loads
-    //   quarter 1: the second k-step's A fragments
-    //   quarter 2: nothing -- then the stage's one barrier: every wave's loads of stage kt+1 have
-    //              landed and nobody reads stage kt any more (the last quarter's fragments are in registers)
-    //   quarter 3: stage kt+1's first fragments, and the first half of stage kt+2's loads
-    constexpr int SLOTS = 4 * NT;                              // MFMAs of a quarter
-    constexpr int Q0_EVERY = (SLOTS - NT) / INST;              // quarter 0: a load every so many slots once B is read
-    constexpr int Q3_FIRST = NT + 8, Q3_EVERY = (SLOTS - Q3_FIRST) / INST;
-    static_assert(Q0_EVERY >= 1 && Q3_EVERY >= 1, "a quarter has a slot for each of its reads and loads");
-    const int st_bytes = (kt % STAGES) * STAGE_BYTES, nst_bytes = ((kt + 1) % STAGES) * STAGE_BYTES;
+    const int st_bytes = now * STAGE_BYTES, nst_bytes = next * STAGE_BYTES;
+    char* st = smem_big + st_bytes;          // this stage
+    char* nst = smem_big + nst_bytes;        // stage kt+1's
+    const int after = STAGES == 2 ? now : 3 - now - next;
+    char* fill = smem_big + after * STAGE_BYTES;   // stage kt+2's buffer
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      if constexpr (B_KN) join_b(ks, bfr[ks], af[ks]);
+      if constexpr (B_KN) join_kn(ks);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int quarter = ks * 2 + (i >> 2), q = i & 3;   // q: the quarter's tile row
-        if (quarter == 3 && q == 0) {
-          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-          wait_vmcnt<0>();
-          block_barrier();
-        }
+      for (int i = 0; i < MI; ++i) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
+          const int slot = i * NT + j;
+          if (ks == 1 && slot == BARRIER) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            wait_vmcnt<STAGES == 3 ? EARLY : 0>();   // (three stages: all but what is out of stage kt+2's)
+            block_barrier();
+          }
           mfma_16x16x32_in_place(acc[i][j], bfr[ks][j], af[ks][i]);
           __builtin_amdgcn_sched_barrier(0);
-          const int slot = q * NT + j;
-          if (quarter == 0) {
+          if (ks == 0) {
             if (slot < NT) {
               if constexpr (B_KN) b_frag_kn(st_bytes, 1, slot, tfb[1][slot]);
               else bfr[1][slot] = b_frag(st, 1, slot);
-            } else if ((slot - NT) % Q0_EVERY == 0 && (slot - NT) / Q0_EVERY < INST) issue_half(nst, k1, 1, (slot - NT) / Q0_EVERY);
-          } else if (quarter == 1) {
-            if (slot < 8) {
-              if constexpr (B_KN) a_frag_kn(st_bytes, 1, slot, af[1][slot]);
-              else af[1][slot] = a_frag(st, 1, slot);
+            } else if (slot >= A_FROM && slot < A_FROM + MI) {
+              if constexpr (B_KN) a_frag_kn(st_bytes, 1, slot - A_FROM, af[1][slot - A_FROM]);
+              else af[1][slot - A_FROM] = a_frag(st, 1, slot - A_FROM);
+            } else {
+              const int nth = slot < A_FROM ? ((slot - NT) % APART == 0 && (slot - NT) / APART < IN_GAP ? (slot - NT) / APART : EARLY)
+                                            : IN_GAP + slot - A_FROM - MI;
+              if (nth < EARLY) {
+                if constexpr (STAGES == 3) issue_one(fill, k2, nth, false);
+                else issue_one(nst, k1, LATE + nth, false);
+              }
             }
-          } else if (quarter == 3) {
-            if (slot < NT) {
-              if constexpr (B_KN) b_frag_kn(nst_bytes, 0, slot, tfb[0][slot]);
-              else bfr[0][slot] = b_frag(nst, 0, slot);
+          } else if (slot >= BARRIER) {
+            if (slot < BARRIER + NT) {
+              if constexpr (B_KN) b_frag_kn(nst_bytes, 0, slot - BARRIER, tfb[0][slot - BARRIER]);
+              else bfr[0][slot - BARRIER] = b_frag(nst, 0, slot - BARRIER);
             } else if (slot < Q3_FIRST) {
-              if constexpr (B_KN) a_frag_kn(nst_bytes, 0, slot - NT, af[0][slot - NT]);
-              else af[0][slot - NT] = a_frag(nst, 0, slot - NT);
-            } else if ((slot - Q3_FIRST) % Q3_EVERY == 0 && (slot - Q3_FIRST) / Q3_EVERY < INST)
-              issue_half(st, k2, 0, (slot - Q3_FIRST) / Q3_EVERY);
+              if constexpr (B_KN) a_frag_kn(nst_bytes, 0, slot - BARRIER - NT, af[0][slot - BARRIER - NT]);
+              else af[0][slot - BARRIER - NT] = a_frag(nst, 0, slot - BARRIER - NT);
+            } else if ((slot - Q3_FIRST) % Q3_EVERY == 0 && (slot - Q3_FIRST) / Q3_EVERY < LATE) {
+              const int nth = (slot - Q3_FIRST) / Q3_EVERY;
+              issue_one(fill, k2, STAGES == 3 ? EARLY + nth : nth, false);
+            }
           }
           __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
+    now = next;
+    next = STAGES == 2 ? 1 - next : after;
   }
 
-  wait_vmcnt<0>();   // the last iteration's idle fetch must land before LDS is reused
+  if constexpr (B_KN) join_kn(0);   // the idle reads of the last iteration land while their registers are still theirs
+  wait_vmcnt<0>();   // ... and its idle fetch before LDS is reused
   block_barrier();   // every wave is done reading the stages
 
   if constexpr (PAIR) {
@@ -1686,6 +1686,7 @@ __device__ __forceinline__ void gemm_nt256_body(const bf16_t* __restrict__ A, co
     // the same 8 NT columns of the output: the gate's product leaves as it is stored, then, made in the
     // accumulators' own layout, bf16(bf16(act(bf16 g)) * bf16 u).
     constexpr int HT = NT / 2, OROWB = HT * 32 + 16, LPRW = HT * 2, ORPI = 64 / LPRW;
+    static_assert(MI == 8, "a wave's 128 rows");
     char* ot = smem_big + wave * (128 * OROWB);
     const int lr = lane / LPRW, lc = lane % LPRW;
     const size_t first = (size_t)(m0 + wm * 128) * N + n0 + wn * HT * 16 + lc * 8;
@@ -1735,14 +1736,14 @@ __device__ __forceinline__ void gemm_nt256_body(const bf16_t* __restrict__ A, co
     leave(C);
     return;
   }
-  // Output through LDS: a wave lays its 128 x (16 NT) tile out row-major (rows padded by 16 bytes,
+  // Output through LDS: a wave lays its (16 MI) x (16 NT) tile out row-major (rows padded by 16 bytes,
   // which spreads both the 8-byte writes below and the 16-byte reads over all banks) and stores
   // whole 16-byte pieces, so a row of the tile leaves as one contiguous segment.
   // acc[i][j][e]: row fr of A tile i, column 4*kq + e of B tile j.
-  constexpr int OROWB = BIG_OUT_ROW_BYTES(TN);
-  char* ot = smem_big + wave * (128 * OROWB);
+  constexpr int OROWB = T::OUT_ROW_BYTES;
+  char* ot = smem_big + wave * (MI * 16 * OROWB);
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < NT; ++j)
       *reinterpret_cast<uint2*>(ot + (i * 16 + fr) * OROWB + (j * 16 + 4 * kq) * 2) =
@@ -1752,36 +1753,45 @@ __device__ __forceinline__ void gemm_nt256_body(const bf16_t* __restrict__ A, co
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  constexpr int LPRW = TN * 4;        // lanes (16 bytes each) per tile row
-  constexpr int ORPI = 64 / LPRW;     // rows per instruction
+  constexpr int LPRW = NT * 2;        // lanes (16 bytes each) per tile row
+  constexpr int ORPI = 64 / LPRW;     // rows per instruction (of 96-byte rows ten: four lanes idle)
   const int lr = lane / LPRW, lc = lane % LPRW;
-  bf16_t* cbase = C + (size_t)(m0 + wm * 128) * N + n0 + wn * TN * 32 + lc * 8;
+  const int row0 = m0 + wm * MI * 16;
+  bf16_t* cbase = C + (size_t)row0 * N + n0 + wn * NT * 16 + lc * 8;
   // STREAM_OUT (the launch sets it over a long K): the tile leaves by non-temporal stores, so C's
   // lines do not stay in the XCD's L2 among the A and B panels its blocks re-read (8192^3: 790 ->
   // 750 us; 1 to 5 % from K = 4096 on, and 1.5 % slower at K = 2048, where a tile's stores are a
   // larger part of its time).  A template argument: as a branch on K the compiler merged the two
   // stores into one plain one.
-  typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+  typedef unsigned int u32x4_t __attribute__((ext_vector_type(4), aligned(2)));   // (rows begin where they begin, see store_loose)
 #pragma unroll 4
-  for (int r0 = 0; r0 < 128; r0 += ORPI) {
+  for (int r0 = 0; r0 < MI * 16; r0 += ORPI) {
     const int r = r0 + lr;
+    if (64 % LPRW != 0 && (lr >= ORPI || r >= MI * 16)) continue;
     const uint4 v = *reinterpret_cast<const uint4*>(ot + r * OROWB + lc * 16);
-    if (m0 + wm * 128 + r < Mv) {
+    if (row0 + r < Mv) {
       if constexpr (STREAM_OUT)
         __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, v), reinterpret_cast<u32x4_t*>(cbase + (size_t)r * N));
       else
-        *reinterpret_cast<uint4*>(cbase + (size_t)r * N) = v;
+        store_loose(cbase + (size_t)r * N, v);
     }
   }
 }
 
-template <int WAVES, int KB, bool B_KN = false, bool STREAM_OUT = false>
-__global__ __launch_bounds__(WAVES * 64) void gemm_nt256_kernel(const bf16_t* __restrict__ A,
-                                                         const bf16_t* __restrict__ B,
-                                                         bf16_t* __restrict__ C, int M, int N, int K,
-                                                         const int* __restrict__ valid, int tiles_m,
-                                                         int tiles_n, int patched) {
-  gemm_nt256_body<WAVES, KB, B_KN, STREAM_OUT>(A, B, C, M, N, K, valid, tiles_m, tiles_n, patched);
+typedef BigTile<2, 4, 8, 4> Tile256;       // 256 x 256, eight waves
+typedef BigTile<2, 4, 6, 4> Tile192x256;
+typedef BigTile<2, 4, 5, 4> Tile160x256;
+typedef BigTile<2, 4, 4, 4> Tile128x256;
+typedef BigTile<2, 4, 4, 3> Tile128x192;   // B (N,K) only
+typedef BigTile<2, 2, 8, 8> Tile256Four;   // 256 x 256 by four waves, for launches whose other tilings are four waves
+
+template <class T, bool B_KN = false, bool STREAM_OUT = false>
+__global__ __launch_bounds__(T::WAVES * 64) void gemm_big_kernel(const bf16_t* __restrict__ A,
+                                                                 const bf16_t* __restrict__ B,
+                                                                 bf16_t* __restrict__ C, int M, int N, int K,
+                                                                 const int* __restrict__ valid, int tiles_m,
+                                                                 int tiles_n, int patched) {
+  gemm_big_body<T, B_KN, STREAM_OUT>(A, B, C, M, N, K, valid, tiles_m, tiles_n, patched);
 }
 
 // A row bound read on the device decides which tile size fills the chip best (512 valid rows of
@@ -1800,7 +1810,7 @@ __global__ __launch_bounds__(256) void gemm_either_kernel(const bf16_t* __restri
   const int Mv = bound_or(valid, M), bid = blockIdx.x;
   if (BIG && Mv > few256) {
     if (bid < t256.tiles_m * t256.tiles_n)
-      gemm_nt256_body<4, BIG_KB>(A, B, C, M, N, K, valid, t256.tiles_m, t256.tiles_n, t256.patched);
+      gemm_big_body<Tile256Four>(A, B, C, M, N, K, valid, t256.tiles_m, t256.tiles_n, t256.patched);
   } else if (Mv > few128) {
     if (bid < t128.tiles_m * t128.tiles_n)
       gemm_nt16_body<false>(A, B, C, M, N, K, valid, t128.tiles_m, t128.tiles_n, t128.patched, tail);
@@ -1825,8 +1835,7 @@ static int launch_gemm_either(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
     return Tiling{tile_rows, tile_cols, patched_order(tile_rows, tile_cols)};
   };
   const Tiling t128 = tiling((rows128 + 127) / 128, n128), t64 = tiling((rows64 + 63) / 64, n64);
-  constexpr size_t out_bytes = (size_t)4 * 128 * BIG_OUT_ROW_BYTES(4);   // this launch's large tiles are four waves'
-  constexpr size_t lds256 = out_bytes > (size_t)2 * BIG_STAGE_BYTES ? out_bytes : (size_t)2 * BIG_STAGE_BYTES;
+  constexpr size_t lds256 = Tile256Four::LDS_BYTES;
   constexpr size_t lds128 = (size_t)NT_STAGES * 256 * BK * 2;
   constexpr size_t lds = BIG ? (lds256 > lds128 ? lds256 : lds128) : lds128;
   static LdsOptIn opt_in;
@@ -2240,7 +2249,7 @@ __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __re
   gate.gated = activation;
   if (form == PairForm::ROWS256) {
     if (bid >= t256.tiles_m * t256.tiles_n) return;
-    gemm_nt256_body<4, BIG_KB, false, false, true>(A, Bg, C, M, N, K, valid, t256.tiles_m, t256.tiles_n, t256.patched,
+    gemm_big_body<Tile256Four, false, false, true>(A, Bg, C, M, N, K, valid, t256.tiles_m, t256.tiles_n, t256.patched,
                                                    GatedPair{Bu, G, activation});
   } else if (form == PairForm::ROWS128) {
     if (bid >= t128.tiles_m * t128.tiles_n) return;
@@ -2411,30 +2420,65 @@ static int launch_gemm_shared(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
   IRON_LAUNCH_CHECK();
 }
 
-template <bool B_KN, bool STREAM_OUT>
-static int launch_gemm_nt256_as(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K,
-                                const int* valid, hipStream_t s) {
-  const int tiles_m = (M + BIG_BM - 1) / BIG_BM, tiles_n = (N + BIG_BN - 1) / BIG_BN;
-  constexpr size_t out_bytes = (size_t)BIG_WAVES * 128 * BIG_OUT_ROW_BYTES(8 / BIG_WAVES * 2);
-  const size_t lds = out_bytes > (size_t)2 * BIG_STAGE_BYTES ? out_bytes : (size_t)2 * BIG_STAGE_BYTES;
+template <class T, bool B_KN, bool STREAM_OUT>
+static int launch_gemm_big_as(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, const int* valid, hipStream_t s) {
+  const int tiles_m = (M + T::BM - 1) / T::BM, tiles_n = (N + T::BN - 1) / T::BN;
   static LdsOptIn opt_in;
-  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_nt256_kernel<BIG_WAVES, BIG_KB, B_KN, STREAM_OUT>), lds);
+  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_big_kernel<T, B_KN, STREAM_OUT>), T::LDS_BYTES);
       e != hipSuccess) {
     set_error("gemm: %s", hipGetErrorString(e));
     return (int)e;
   }
-  const int patched = (tiles_m % 8 == 0 && tiles_n % 4 == 0 && ((tiles_m / 8) * (tiles_n / 4)) % 8 == 0) ? 1 : 0;
-  hipLaunchKernelGGL((gemm_nt256_kernel<BIG_WAVES, BIG_KB, B_KN, STREAM_OUT>), dim3(tiles_m * tiles_n), dim3(BIG_WAVES * 64), lds, s,
-                     A, B, C, M, N, K, valid, tiles_m, tiles_n, patched);
+  hipLaunchKernelGGL((gemm_big_kernel<T, B_KN, STREAM_OUT>), dim3(tiles_m * tiles_n), dim3(T::WAVES * 64), T::LDS_BYTES, s,
+                     A, B, C, M, N, K, valid, tiles_m, tiles_n, patched_order(tiles_m, tiles_n));
   IRON_LAUNCH_CHECK();
 }
 
-// Over a long K the tiles leave by non-temporal stores (see the body's epilogue).
-template <bool B_KN = false>
-static int launch_gemm_nt256(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K,
-                             const int* valid, hipStream_t s) {
-  if (K >= 4096) return launch_gemm_nt256_as<B_KN, true>(A, B, C, M, N, K, valid, s);
-  return launch_gemm_nt256_as<B_KN, false>(A, B, C, M, N, K, valid, s);
+// Whole tiles larger than 128 x 128, by how the rounds they make over the chip's 256 CUs come out: a round of a tile was measured
+// to take `start` us (its entry, first loads and stores) and `stage` for each 64 of K, `loose` where rows straddle cache lines; [0] with B (N,K), [1] (K,N).
+// The stage grows with the tile's area, so what a product gains is the part of its rounds that is not filled (us, by 128 x 128 or 256 x 256 tiles
+// alone and by the tile chosen here): 777 x 10240 x 2560 59 -> 47, 2012 x 3008 x 1608 34.4 -> 24.4, 2856 x 2325 x 3176 77 -> 51, 1636 x 5256 x 6200 with
+// B (K,N) 153 -> 119, 908 x 5328 x 344 with B (K,N) 14.8 -> 9.9, 3000 x 3000 x 3000 74 -> 54.
+enum BigForm { BIG_NONE, BIG_256, BIG_192X256, BIG_160X256, BIG_128X256, BIG_128X192, BIG_FORMS };
+struct BigPrice {
+  int bm, bn;
+  float start, stage[2], loose[2];
+};
+constexpr BigPrice BIG_PRICES[BIG_FORMS] = {
+    {128, 128, 2.8f, {0.415f, 0.426f}, {0.615f, 0.49f}},   // (the 128 x 128 kernel)
+    {256, 256, 7.5f, {1.36f, 1.42f}, {1.63f, 1.48f}},  {192, 256, 5.9f, {1.10f, 1.16f}, {1.38f, 1.22f}},
+    {160, 256, 4.9f, {0.92f, 0.955f}, {1.08f, 1.00f}}, {128, 256, 4.4f, {0.76f, 0.80f}, {0.95f, 0.835f}},
+    {128, 192, 3.2f, {0.595f, 0.f}, {0.76f, 0.f}},     // (a stage of (K,N) rows of 192 columns is no whole number of loads)
+};
+static float big_price(BigForm form, int M, int N, int K, bool b_nk) {
+  const BigPrice& p = BIG_PRICES[form];
+  const long tiles = (long)((M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
+  return (float)((tiles + 255) / 256) * (p.start + (K % BK == 0 ? p.stage : p.loose)[!b_nk] * ((K + BK - 1) / BK));
+}
+// The form for a product without a row bound, and what it and the 128 x 128 tiles are expected to take.
+static BigForm big_form(int M, int N, int K, bool b_nk, float& price, float& price128) {
+  const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
+  BigForm best = BIG_NONE;
+  price = price128 = big_price(BIG_NONE, M, N, K, b_nk);
+  if (!b_nk && (long)(K + BK) * N * 2 >= (1L << 31)) return best;   // (a (K,N) matrix is addressed with 32-bit byte offsets)
+  for (int form = BIG_256; form < BIG_FORMS; ++form) {
+    if (M < BIG_PRICES[form].bm || N < BIG_PRICES[form].bn || (form == BIG_128X192 && !b_nk)) continue;
+    const float p = big_price((BigForm)form, M, N, K, b_nk);
+    // (past four rounds of 256 x 256 tiles the smaller ones' traffic tells: 5540 x 12392 x 7728 1011 us by those, 1024 by 160 x 256, 881 by its price)
+    if (p < (best == BIG_256 && tiles256 > 3 * 256 ? 0.9f : 0.97f) * price) best = (BigForm)form, price = p;
+  }
+  return best;
+}
+template <bool B_KN>
+static int launch_gemm_big(BigForm form, const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, const int* valid, hipStream_t s) {
+  // Over a long K the tiles leave by non-temporal stores (see the body's epilogue).
+  if (form == BIG_256 && K >= 4096) return launch_gemm_big_as<Tile256, B_KN, true>(A, B, C, M, N, K, valid, s);
+  if (form == BIG_256) return launch_gemm_big_as<Tile256, B_KN, false>(A, B, C, M, N, K, valid, s);
+  if (form == BIG_192X256) return launch_gemm_big_as<Tile192x256, B_KN, false>(A, B, C, M, N, K, valid, s);
+  if (form == BIG_160X256) return launch_gemm_big_as<Tile160x256, B_KN, false>(A, B, C, M, N, K, valid, s);
+  if constexpr (!B_KN)
+    if (form == BIG_128X192) return launch_gemm_big_as<Tile128x192, false, false>(A, B, C, M, N, K, valid, s);
+  return launch_gemm_big_as<Tile128x256, B_KN, false>(A, B, C, M, N, K, valid, s);
 }
 
 }  // namespace iron
@@ -2460,7 +2504,7 @@ static int check_gemm(const uint16_t* A, const uint16_t* B, const uint16_t* C, i
 // Shared: the second launch and 0.028 a slice of a tile (its 64 KB out and back) on top, which the slices
 // are chosen against.  Both sides: 97 x 400 x 7392 with B (K,N) 48.8 -> 14.0, 383 x 1472 x 6520 50.7 -> 25.0, 86 x 1728 x
 // 5560 with B (N,K) 26.6 -> 16.0, 5300 x 864 x 7744 (294 tiles) 92 -> 74; not 1024 x 1024 x 4096, 15.5 against 21.2.
-static TileShares gemm_shares_of_tiles(int M, int N, int K, bool b_nk) {
+static TileShares gemm_shares_of_tiles(int M, int N, int K, bool b_nk, float* price = nullptr) {
   const TileShares none{0, 0, 0};
   const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
   if (K < BK || tiles > 3 * 256) return none;
@@ -2475,6 +2519,7 @@ static TileShares gemm_shares_of_tiles(int M, int N, int K, bool b_nk) {
   const float stage64 = K % BK == 0 ? 0.13f + 0.10f * fill : fminf(0.14f + 3.f * fill, 0.22f + 0.12f * fill);
   const float now = 3.f + stages * (b_nk && t <= 128 ? stage64 : 0.5f * ((t + 255) / 256));
   const float then = 7.f + 0.028f * slices * shared + 0.5f * ((stages + slices - 1) / slices + stages * ((t - shared) / 256));
+  if (price != nullptr) *price = then;
   return then < 0.9f * now ? TileShares{t - shared, shared, slices} : none;
 }
 
@@ -2499,30 +2544,17 @@ static bool gemm_of_few_rows(int M, int N, int K) {
   return 1.05f * few < tiles;
 }
 
-// Whether the 256x256 tiles take a product (see iron_gemm_bf16).
-static bool gemm_on_big_tiles(int M, int N, int K) {
-  const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-  const long tiles256 = (long)((M + BIG_BM - 1) / BIG_BM) * ((N + BIG_BN - 1) / BIG_BN);
-  return M >= BIG_BM && N >= BIG_BN && N % 8 == 0 && tiles256 >= (K % BK == 0 ? 192 : 144) && 5 * tiles128 >= 16 * tiles256;
-}
-
 // Whether the direct-to-LDS kernels take a product, B (N,K) with C (N,M) turned round before.  They take any K from one stage on (k_pad),
 // any M, and any N of B (N,K); against the general kernel, which loads through registers: 2048 x 2048 x 2056 42.5 -> 26.0 us, 86 x 1728 x
-// 5560 59 -> 26.5, (K,N) 2048 x 2048 x 2040 65 -> 22.0, 300 x 1000 x 1000 33.6 -> 9.8.  (A K that is no
-// multiple of 64 stays dearer than its neighbour that is, 26.0 us against 19.4: its rows' 128-byte
+// 5560 59 -> 26.5, (K,N) 2048 x 2048 x 2040 65 -> 22.0, 300 x 1000 x 1000 33.6 -> 9.8, 2048 x 2616 x 72 9.8 -> 6.9, 7137 x 6620 x 80 49.0 -> 30.8.
+// (A K that is no multiple of 64 stays dearer than its neighbour that is, 26.0 us against 19.4: its rows' 128-byte
 // pieces straddle two cache lines.)  The general kernel, of which a CU holds several blocks, keeps a short K where there is one row or column
-// of tiles, and such a K that straddles where the direct tiles' second round is a short one or their rows leave in pieces of eight bytes, over
-// very many tiles up to a K of 1536 (general against direct: (K,N) 107 x 240 x 64 3.7 / 4.6, 100 x 8008 x 64 4.4 / 4.9, but 200 x 240 x 64 5.8 / 4.6;
-// (N,M) of 3 x 3904 x 224 5.8 / 6.3; (N,K) 490 x 22 x 64 3.2 / 3.8, under a bound 63 x 424 x 64 3.2 / 3.8; 2048 x 2616 x 120 10.2 / 11.4, but 4000 x
-// 5000 x 120 24.0 / 20.4; 7137 x 6620 x 80 49.0 / 55.1 and x 1000 166.6 / 179.4, but 4000 x 3004 x 1000 49.9 / 42.7).
+// of tiles (general against direct: (K,N) 107 x 240 x 64 3.7 / 4.6, 100 x 8008 x 64 4.4 / 4.9, but 200 x 240 x 64 5.8 / 4.6;
+// (N,M) of 3 x 3904 x 224 5.8 / 6.3; (N,K) 490 x 22 x 64 3.2 / 3.8, under a bound 63 x 424 x 64 3.2 / 3.8).
 static bool gemm_direct_to_lds(int M, int N, int K, int b_col_maj, int c_col_maj, bool bounded) {
   if (K < BK || (c_col_maj && (b_col_maj || bounded))) return false;
   if (!b_col_maj) return (M >= 128 && N >= 128) || K > (c_col_maj && M < 8 ? 4 : 2) * BK;
-  if (M < 64 || N < 64) return K > 2 * BK;
-  const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-  if (K % BK == 0 || tiles128 <= 256) return true;
-  if (tiles128 <= 448) return K >= 6 * BK;
-  return N % 8 != 4 || K >= (tiles128 > 1024 ? 24 : 3) * BK;
+  return (M >= 64 && N >= 64) || K > 2 * BK;
 }
 
 extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K,
@@ -2545,25 +2577,23 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
   if (valid_k == nullptr && gemm_direct_to_lds(M, N, K, b_col_maj, c_col_maj, valid != nullptr)) {
     if (c_col_maj) return launch_gemm_nt<true, false, 2, 4, true>(A, B, C, M, N, K, valid, s);
     const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-    // Enough 256x256 tiles to fill the chip: the large-tile kernel (offsets are 32-bit).  A round of
-    // them takes as long as about 3.2 rounds of 128x128 ones (4000 x 4096 x 4096: 256 tiles 129 us, 1024 smaller
-    // ones 158; 777 x 10240 x 2560: 160 tiles 69 us, 560 smaller ones 61), so 192 it is, and edges
-    // that waste more than a fifth of the large tiles stay with the smaller; where rows straddle cache
-    // lines the large tile, which reads half as much, gains more (1500 x 6000 x 3000: 144 tiles 93 us
-    // against 110).
-    const bool whole = M % BIG_BM == 0 && N % BIG_BN == 0;
-    const bool big = gemm_on_big_tiles(M, N, K);
-    if (b_col_maj && big && (valid == nullptr || whole)) {
-      // Under a row bound read on the device the large tiles may cover too few rows to fill the
-      // chip (512 valid rows of 2048 leave 64 of 256 tiles): the blocks of one launch then choose
-      // the tile size where the bound is known, on the device.
-      const int tiles_n256 = N / BIG_BN, tiles_n128 = N / 128;
-      const int few256 = tiles_n256 >= 128 ? 0 : BIG_BM * (128 / tiles_n256);   // rows up to which 128x128 tiles win
-      const int few128 = tiles_n128 >= 128 ? 0 : 128 * (127 / tiles_n128);      // ... and 64x64 ones
-      if (valid == nullptr || few256 == 0 || few256 >= M) return launch_gemm_nt256(A, B, C, M, N, K, valid, s);
-      return launch_gemm_either<true>(A, B, C, M, N, K, valid, s, few256, few128);
+    if (valid == nullptr && tiles128 >= 128) {
+      float price, price128;
+      const BigForm form = big_form(M, N, K, b_col_maj, price, price128);
+      if (form != BIG_NONE)
+        return b_col_maj ? launch_gemm_big<false>(form, A, B, C, M, N, K, nullptr, s) : launch_gemm_big<true>(form, A, B, C, M, N, K, nullptr, s);
     }
     if (b_col_maj) {
+      if (valid != nullptr && M % BIG_BM == 0 && N % BIG_BN == 0 && (long)(M / BIG_BM) * (N / BIG_BN) >= (K % BK == 0 ? 192 : 144)) {
+        // Under a row bound read on the device the large tiles may cover too few rows to fill the
+        // chip (512 valid rows of 2048 leave 64 of 256 tiles): the blocks of one launch then choose
+        // the tile size where the bound is known, on the device.
+        const int tiles_n256 = N / BIG_BN, tiles_n128 = N / 128;
+        const int few256 = tiles_n256 >= 128 ? 0 : BIG_BM * (128 / tiles_n256);   // rows up to which 128x128 tiles win
+        const int few128 = tiles_n128 >= 128 ? 0 : 128 * (127 / tiles_n128);      // ... and 64x64 ones
+        if (few256 == 0 || few256 >= M) return launch_gemm_big<false>(BIG_256, A, B, C, M, N, K, valid, s);
+        return launch_gemm_either<true>(A, B, C, M, N, K, valid, s, few256, few128);
+      }
       // 128x128 tiles that would occupy under half the CUs give way to 64x64 ones: always, where
       // the shape says so; under a row bound, the blocks of one launch choose where the bound is
       // known (the few-row 64x64 tiles run the eight-stage pipeline, a block a CU, so nothing is
@@ -2575,9 +2605,6 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
       if (valid == nullptr || few == 0 || few >= M) return launch_gemm_nt<false>(A, B, C, M, N, K, valid, s);
       return launch_gemm_either<false>(A, B, C, M, N, K, valid, s, 0, few);
     }
-    // (K,N): the same line, for a matrix a 32-bit byte offset spans.
-    if (valid == nullptr && big && (long)(K + BK) * N * 2 < (1L << 31))
-      return launch_gemm_nt256<true>(A, B, C, M, N, K, valid, s);
     return launch_gemm_nt<true>(A, B, C, M, N, K, valid, s);
   }
   // 128x128 tiles fill the 256 CUs once at 2048x2048; narrower problems take 64-wide tiles.
@@ -2588,8 +2615,13 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
 }
 
 static TileShares gemm_shares(int M, int N, int K, bool b_nk, bool c_nm) {
-  if ((b_nk && gemm_of_few_rows(M, N, K)) || (!c_nm && gemm_on_big_tiles(M, N, K))) return TileShares{0, 0, 0};
-  return gemm_shares_of_tiles(M, N, K, b_nk);
+  if (b_nk && gemm_of_few_rows(M, N, K)) return TileShares{0, 0, 0};
+  float then = 0.f, big, price128;
+  const TileShares deal = gemm_shares_of_tiles(M, N, K, b_nk, &then);
+  // (whole tiles of another size, where they take no more)
+  if (deal.slices > 0 && !c_nm && deal.whole + deal.shared >= 128 && big_form(M, N, K, b_nk, big, price128) != BIG_NONE && big + 3.f <= then)
+    return TileShares{0, 0, 0};
+  return deal;
 }
 
 extern "C" int64_t iron_gemm_workspace_bytes(int M, int N, int K, int b_col_maj, int c_col_maj) {

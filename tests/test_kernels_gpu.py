@@ -128,6 +128,38 @@ def test_gemm_at_the_edges_of_tiles_and_stages(cuda, M, Kdim, N, b_col_maj, c_co
 
 
 @pytest.mark.parametrize("M,Kdim,N,b_col_maj,c_col_maj", [
+    (3329, 128, 3593, True, False), (3329, 192, 3592, False, False),                                   # 256 x 256 tiles
+    (192, 136, 48000, True, False), (3840, 264, 2819, True, False), (1290, 200, 8200, False, False),   # 192 x 256
+    (160, 200, 40963, True, False), (1025, 64, 7169, True, False), (1025, 72, 7176, False, False),     # 160 x 256
+    (641, 264, 8067, True, False), (777, 64, 6915, True, False), (641, 136, 5384, False, False),       # 128 x 256
+    (128, 328, 33000, True, False), (641, 64, 5377, True, False), (3585, 200, 1025, True, True),       # 128 x 192
+])
+def test_gemm_large_tiles_of_every_size(cuda, M, Kdim, N, b_col_maj, c_col_maj):
+    """Each size of tile a launch without a row bound may take, down to one tile row, one stage of K and a K that ends inside
+    one, the last tiles moved back to the edges; the operands lie between NaNs.  B (N,K): the bits of the launch under a bound, whose
+    tiles are of other sizes."""
+    rng = np.random.default_rng(M + N + Kdim)
+    A, B = bf(rng, M, Kdim), bf(rng, (N if b_col_maj else Kdim), (Kdim if b_col_maj else N), scale=0.05)
+
+    def between_nans(x):
+        buf = torch.full((x.size + 256 * x.shape[1],), float("nan"), dtype=torch.bfloat16, device=cuda)
+        inside = buf[128 * x.shape[1]:128 * x.shape[1] + x.size].view(*x.shape)
+        inside.copy_(dev(x, cuda))
+        return inside
+
+    dA, dB, buf = between_nans(A), between_nans(B), out_like((M * N + 64,), cuda, fill=3.0)
+    C = buf[: M * N].view(*((N, M) if c_col_maj else (M, N)))
+    K.gemm(dA, dB, C, M=M, N=N, K=Kdim, b_col_maj=b_col_maj, c_col_maj=c_col_maj)
+    kw = dict(b_col_maj=b_col_maj, c_col_maj=c_col_maj)
+    assert np.all(np.abs(from_torch(C) - ops.gemm(A, B, **kw)) <= ops.gemm_bound(A, B, **kw))
+    assert bool((buf[M * N:] == 3).all())
+    if b_col_maj and not c_col_maj:
+        bounded = torch.empty_like(C)
+        K.gemm(dA, dB, bounded, M=M, N=N, K=Kdim, b_col_maj=True, valid=word(M, cuda))
+        assert torch.equal(bounded, C)
+
+
+@pytest.mark.parametrize("M,Kdim,N,b_col_maj,c_col_maj", [
     (64, 8192, 64, True, False), (24, 6200, 200, True, False), (63, 8184, 136, True, True), (67, 3640, 872, True, False), (872, 3640, 67, True, True),   # all tiles shared, B (N,K)
     (1, 4096, 400, False, False), (130, 2504, 72, False, False), (257, 4000, 264, False, False),   # ... and (K,N)
     (123, 2856, 200, False, True), (2049, 2504, 2056, True, False), (2049, 2504, 2056, False, False),   # (N,M); the last round's tiles
