@@ -1424,11 +1424,15 @@ struct GatedPair {
 template <int WM_, int WN_, int MI_, int NT_>
 struct BigTile {
   static constexpr int WM = WM_, WN = WN_, MI = MI_, NT = NT_, WAVES = WM * WN, BM = WM * MI * 16, BN = WN * NT * 16;
-  static constexpr int STAGE_BYTES = (BM + BN) * BK * 2;
-  // Three stages where they fit beside the 1 KB that loads without rows go to: a stage's loads then have a whole stage's time to land.
-  static constexpr int STAGES = 3 * STAGE_BYTES + 1024 <= 160 * 1024 ? 3 : 2;
+  static constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2, LDS_MOST = 160 * 1024;
+  // B, which comes from memory where a weight is used once, is held three stages deep, A too where that fits, else two (weights out of memory,
+  // us with two and with three stages of B: 2048 x 16384 x 2048 120 / 109, 2048 x 8192 x 2048 60.4 / 54.9, 4096^3 105 / 98; the same weights
+  // again 105 either way, 8192^3 733 / 729).  Where the waves' loads do not come out even, those without rows go to 1 KB behind the stages.
+  static constexpr int SPARE = BM / 8 % WAVES == 0 && BN / 8 % WAVES == 0 ? 0 : 1024;
+  static constexpr int A_STAGES = 3 * (A_BYTES + B_BYTES) + SPARE <= LDS_MOST ? 3 : 2, STAGES_BYTES = A_STAGES * A_BYTES + 3 * B_BYTES;
   static constexpr int OUT_ROW_BYTES = NT * 32 + 16, OUT_BYTES = WAVES * MI * 16 * OUT_ROW_BYTES;
-  static constexpr int LDS_BYTES = STAGES * STAGE_BYTES + 1024 > OUT_BYTES ? STAGES * STAGE_BYTES + 1024 : OUT_BYTES;
+  static constexpr int LDS_BYTES = STAGES_BYTES + SPARE > OUT_BYTES ? STAGES_BYTES + SPARE : OUT_BYTES;
+  static_assert(LDS_BYTES <= LDS_MOST, "a CU's LDS");
 };
 
 template <class T, bool B_KN = false, bool STREAM_OUT = false, bool PAIR = false>
@@ -1436,9 +1440,9 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
                                               bf16_t* __restrict__ C, int M, int N, int K,
                                               const int* __restrict__ valid, int tiles_m, int tiles_n,
                                               int patched, const GatedPair& pair = GatedPair{}) {
-  constexpr int WAVES = T::WAVES, MI = T::MI, NT = T::NT, STAGES = T::STAGES;
+  constexpr int WAVES = T::WAVES, MI = T::MI, NT = T::NT, A_STAGES = T::A_STAGES;
   constexpr int ROWB = BK * 2;                                        // bytes of a tile row in LDS, eight 16-byte chunks
-  constexpr int A_BYTES = T::BM * ROWB, STAGE_BYTES = T::STAGE_BYTES;
+  constexpr int A_BYTES = T::A_BYTES, B_BYTES = T::B_BYTES, B_BASE = A_STAGES * A_BYTES;   // A's stages, then B's
   constexpr int A_INST = T::BM / 8, B_INST = T::BN / 8;               // 1 KB loads of a stage: eight rows each
   constexpr int A_EACH = (A_INST + WAVES - 1) / WAVES, B_EACH = (B_INST + WAVES - 1) / WAVES, LOADS = A_EACH + B_EACH;   // ... a wave's
   constexpr int A_LAST = A_INST % WAVES, B_LAST = B_INST % WAVES;     // waves that have a last one (0: all)
@@ -1479,7 +1483,7 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
   }
   const int inst_stride = WAVES * 8 * K * 2;
   static_assert(!PAIR || WAVES == 4, "PAIR: the rows of an instruction below are four waves'");
-  auto issue_one = [&](char* st, int kt, int idx, bool head) {
+  auto issue_one = [&](int a_at, int b_at, int kt, int idx, bool head) {
     const int k_off = kt * ROWB;
     const bool is_a = idx < A_EACH;
     const int i = is_a ? idx : idx - A_EACH;
@@ -1487,7 +1491,7 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
     // A wave without a last instruction issues it all the same, from past the buffer's end and to where nobody reads: every wave's
     // loads are then as many, which the waits count.
     const bool none = last != 0 && i == (is_a ? A_EACH : B_EACH) - 1 && wave >= last;
-    char* to = none ? smem_big + STAGES * STAGE_BYTES : st + (is_a ? 0 : A_BYTES) + (i * WAVES + wave) * 1024;
+    char* to = smem_big + (none ? T::STAGES_BYTES : (is_a ? a_at : B_BASE + b_at) + (i * WAVES + wave) * 1024);
     if (is_a)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rows, IRON_LDS_PTR(to), 16, none || (head && ld_head < pad) ? NOWHERE : ld_off,
                                                i * inst_stride + k_off, 0, 0);
@@ -1520,36 +1524,37 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
   //   first k-step: the second's B fragments from the start and its A fragments from the middle; loads in the slots between (EARLY of them)
   //   second k-step: up to slot BARRIER nothing -- then the stage's one barrier: every wave's loads of stage kt + 1 have landed and
   //     nobody reads stage kt any more (this k-step's fragments are in registers) -- then stage kt + 1's first fragments and LATE loads
-  // With two stages the late loads are the first of stage kt + 2, into this stage's buffer, the early ones the rest of stage kt + 1's; with three
-  // all are stage kt + 2's, into the buffer that the last barrier freed.
+  // All loads are stage kt + 2's.  The early ones go into a buffer that the last barrier freed: B's, and A's where A has three stages; with two
+  // A's are the late ones, into this stage's buffer.
   constexpr int SLOTS = MI * NT, A_FROM = NT > SLOTS / 2 ? NT : SLOTS / 2, FREE = SLOTS - NT - MI;
-  constexpr int EARLY = STAGES == 3 ? (LOADS < FREE ? LOADS : FREE) : LOADS - LOADS / 2, LATE = LOADS - EARLY;
+  constexpr int EARLY = A_STAGES == 2 ? B_EACH : (LOADS < FREE ? LOADS : FREE), LATE = LOADS - EARLY;
+  constexpr int EARLY_FROM = A_STAGES == 2 ? A_EACH : 0, LATE_FROM = A_STAGES == 2 ? 0 : EARLY;   // their numbers
   constexpr int BARRIER = SLOTS - NT - MI - LATE < SLOTS / 2 ? SLOTS - NT - MI - LATE : SLOTS / 2;
   static_assert(A_FROM + MI <= SLOTS && EARLY <= FREE && BARRIER >= 0, "a k-step has a slot for each of its reads and loads");
   constexpr int GAP = A_FROM - NT, APART = EARLY > 0 && GAP / EARLY > 1 ? GAP / EARLY : 1;   // slots between the B and the A reads
   constexpr int IN_GAP = EARLY < GAP / APART ? EARLY : GAP / APART;
   constexpr int Q3_FIRST = BARRIER + NT + MI, Q3_EVERY = SLOTS - Q3_FIRST > 2 * LATE && LATE > 0 ? (SLOTS - Q3_FIRST) / (LATE > 0 ? LATE : 1) : 1;
 #pragma unroll
-  for (int idx = 0; idx < LOADS; ++idx) issue_one(smem_big, 0, idx, true);
+  for (int idx = 0; idx < LOADS; ++idx) issue_one(0, 0, 0, idx, true);
 #pragma unroll
-  for (int idx = 0; idx < (STAGES == 3 ? LOADS : LATE); ++idx) issue_one(smem_big + STAGE_BYTES, min(1, nk - 1), idx, false);
+  for (int idx = 0; idx < LOADS; ++idx) issue_one(A_BYTES, B_BYTES, min(1, nk - 1), idx, false);
 
   // Fragments: lane -> row fr of a 16-row tile, 16-byte chunk kq of the k-step's four.
   const int fr = lane & 15, kq = lane >> 4;
   const int swz = fr >> 1;   // tile rows are multiples of 16 apart: one swizzle for all
-  const int a_row = (wm * MI * 16 + fr) * ROWB, b_row = A_BYTES + (wn * NT * 16 + fr) * ROWB;
-  auto a_frag = [&](const char* st, int ks, int i) {
-    return *reinterpret_cast<const bf16x8*>(st + a_row + i * 16 * ROWB + (((ks * 4 + kq) ^ swz) << 4));
+  const int a_row = (wm * MI * 16 + fr) * ROWB, b_row = B_BASE + (wn * NT * 16 + fr) * ROWB;
+  auto a_frag = [&](int at, int ks, int i) {
+    return *reinterpret_cast<const bf16x8*>(smem_big + at + a_row + i * 16 * ROWB + (((ks * 4 + kq) ^ swz) << 4));
   };
-  auto b_frag = [&](const char* st, int ks, int j) {
-    return *reinterpret_cast<const bf16x8*>(st + b_row + j * 16 * ROWB + (((ks * 4 + kq) ^ swz) << 4));
+  auto b_frag = [&](int at, int ks, int j) {
+    return *reinterpret_cast<const bf16x8*>(smem_big + at + b_row + j * 16 * ROWB + (((ks * 4 + kq) ^ swz) << 4));
   };
   // (K,N): the B operand of tile j wants, for column n = 16 j + fr, the k-step's k = 8 kq .. + 7.  A
   // transposing read hands a 16-lane group the 4 x 16 block its lanes point at (4 k-rows, each
   // lane 4 columns) turned round: the lane gets 4 k of one column.  Rows 8 kq .. + 3 and 8 kq + 4 .. + 7.
   const int tr_k = 8 * kq + ((lane & 15) >> 2), tr_n = wn * NT * 16 + 4 * (lane & 3);
   const unsigned lds_base_big = (unsigned)(size_t)IRON_LDS_PTR(smem_big);
-  const unsigned kn_base = lds_base_big + A_BYTES;
+  const unsigned kn_base = lds_base_big + B_BASE;
   // The lane's place in a stage's B tile for tile j (k-step 0, low half) is fixed before the loop; the
   // k-step (32 rows on) and the high half (4 rows on) leave the swizzle as it is and ride in the
   // reads' offset fields, so a k-step's reads cost one vector add a tile (the stage) and no more.
@@ -1605,28 +1610,24 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
     for (int j = 0; j < NT; ++j) bfr[ks][j] = tr_join(tfb[ks][j]);
   };
 
-  wait_vmcnt<STAGES == 3 ? LOADS : LATE>();   // stage 0 has landed once only what was issued of stage 1 is out
+  wait_vmcnt<LOADS>();   // stage 0 has landed once only stage 1 is out
   block_barrier();
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
     if constexpr (B_KN) a_frag_kn(0, 0, i, af[0][i]);
-    else af[0][i] = a_frag(smem_big, 0, i);
+    else af[0][i] = a_frag(0, 0, i);
   }
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     if constexpr (B_KN) b_frag_kn(0, 0, j, tfb[0][j]);
-    else bfr[0][j] = b_frag(smem_big, 0, j);
+    else bfr[0][j] = b_frag(0, 0, j);
   }
-  int now = 0, next = 1;   // kt % STAGES and (kt + 1) % STAGES
+  // Where this stage's, the next one's and stage kt + 2's A and B lie.
+  int a_now = 0, a_next = A_BYTES, a_fill = A_STAGES == 2 ? 0 : 2 * A_BYTES, b_now = 0, b_next = B_BYTES, b_fill = 2 * B_BYTES;
   for (int kt = 0; kt < nk; ++kt) {
     // Past the end the last stage is fetched again (into buffers nobody reads any more) rather than
     // branch: a branch would end the scheduling region and undo the interleaving below.
-    const int k1 = min(kt + 1, nk - 1), k2 = min(kt + 2, nk - 1);
-    const int st_bytes = now * STAGE_BYTES, nst_bytes = next * STAGE_BYTES;
-    char* st = smem_big + st_bytes;          // this stage
-    char* nst = smem_big + nst_bytes;        // stage kt+1's
-    const int after = STAGES == 2 ? now : 3 - now - next;
-    char* fill = smem_big + after * STAGE_BYTES;   // stage kt+2's buffer
+    const int k2 = min(kt + 2, nk - 1);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       if constexpr (B_KN) join_kn(ks);
@@ -1637,44 +1638,45 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
           const int slot = i * NT + j;
           if (ks == 1 && slot == BARRIER) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            wait_vmcnt<STAGES == 3 ? EARLY : 0>();   // (three stages: all but what is out of stage kt+2's)
+            wait_vmcnt<EARLY>();   // all but what is out of stage kt + 2's
             block_barrier();
           }
           mfma_16x16x32_in_place(acc[i][j], bfr[ks][j], af[ks][i]);
           __builtin_amdgcn_sched_barrier(0);
           if (ks == 0) {
             if (slot < NT) {
-              if constexpr (B_KN) b_frag_kn(st_bytes, 1, slot, tfb[1][slot]);
-              else bfr[1][slot] = b_frag(st, 1, slot);
+              if constexpr (B_KN) b_frag_kn(b_now, 1, slot, tfb[1][slot]);
+              else bfr[1][slot] = b_frag(b_now, 1, slot);
             } else if (slot >= A_FROM && slot < A_FROM + MI) {
-              if constexpr (B_KN) a_frag_kn(st_bytes, 1, slot - A_FROM, af[1][slot - A_FROM]);
-              else af[1][slot - A_FROM] = a_frag(st, 1, slot - A_FROM);
+              if constexpr (B_KN) a_frag_kn(a_now, 1, slot - A_FROM, af[1][slot - A_FROM]);
+              else af[1][slot - A_FROM] = a_frag(a_now, 1, slot - A_FROM);
             } else {
               const int nth = slot < A_FROM ? ((slot - NT) % APART == 0 && (slot - NT) / APART < IN_GAP ? (slot - NT) / APART : EARLY)
                                             : IN_GAP + slot - A_FROM - MI;
-              if (nth < EARLY) {
-                if constexpr (STAGES == 3) issue_one(fill, k2, nth, false);
-                else issue_one(nst, k1, LATE + nth, false);
-              }
+              if (nth < EARLY) issue_one(a_fill, b_fill, k2, EARLY_FROM + nth, false);
             }
           } else if (slot >= BARRIER) {
             if (slot < BARRIER + NT) {
-              if constexpr (B_KN) b_frag_kn(nst_bytes, 0, slot - BARRIER, tfb[0][slot - BARRIER]);
-              else bfr[0][slot - BARRIER] = b_frag(nst, 0, slot - BARRIER);
+              if constexpr (B_KN) b_frag_kn(b_next, 0, slot - BARRIER, tfb[0][slot - BARRIER]);
+              else bfr[0][slot - BARRIER] = b_frag(b_next, 0, slot - BARRIER);
             } else if (slot < Q3_FIRST) {
-              if constexpr (B_KN) a_frag_kn(nst_bytes, 0, slot - BARRIER - NT, af[0][slot - BARRIER - NT]);
-              else af[0][slot - BARRIER - NT] = a_frag(nst, 0, slot - BARRIER - NT);
+              if constexpr (B_KN) a_frag_kn(a_next, 0, slot - BARRIER - NT, af[0][slot - BARRIER - NT]);
+              else af[0][slot - BARRIER - NT] = a_frag(a_next, 0, slot - BARRIER - NT);
             } else if ((slot - Q3_FIRST) % Q3_EVERY == 0 && (slot - Q3_FIRST) / Q3_EVERY < LATE) {
-              const int nth = (slot - Q3_FIRST) / Q3_EVERY;
-              issue_one(fill, k2, STAGES == 3 ? EARLY + nth : nth, false);
+              issue_one(a_fill, b_fill, k2, LATE_FROM + (slot - Q3_FIRST) / Q3_EVERY, false);
             }
           }
           __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
-    now = next;
-    next = STAGES == 2 ? 1 - next : after;
+    const int a_was = a_now, b_was = b_now;
+    a_now = a_next;
+    a_next = A_STAGES == 2 ? a_was : a_fill;
+    a_fill = A_STAGES == 2 ? a_now : a_was;
+    b_now = b_next;
+    b_next = b_fill;
+    b_fill = b_was;
   }
 
   if constexpr (B_KN) join_kn(0);   // the idle reads of the last iteration land while their registers are still theirs
@@ -2280,8 +2282,8 @@ static int launch_gemm_gated_pair(const bf16_t* A, const bf16_t* Bg, const bf16_
   // (the 64-row tiles in the order of all the rows up to `few`: 580 of 1024 rows in patches of eight tile rows took 27.2 us at 1536 x 1536, not 22.4)
   const Tiling t64 = tiling(most[0] > 0 ? ((few < M ? few : M) + 63) / 64 : 0, n32), t128 = tiling((most[1] + 127) / 128, n128);
   const Tiling t256 = large ? tiling((M + BIG_BM - 1) / BIG_BM, n128) : Tiling{0, 0, 0};
-  constexpr size_t lds = (size_t)PAIR_STAGES * 3 * 128 * BK * 2;   // the two-product body's stages, more than the others'
-  static_assert(lds >= (size_t)NT_STAGES * 256 * BK * 2, "the 64 x 64 body's stages fit too");
+  constexpr size_t lds = Tile256Four::LDS_BYTES;   // the large tile's, more than the others'
+  static_assert(lds >= (size_t)PAIR_STAGES * 3 * 128 * BK * 2 && lds >= (size_t)NT_STAGES * 256 * BK * 2, "the other bodies' stages fit too");
   static LdsOptIn opt_in;
   if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_gated_pair_kernel), lds); e != hipSuccess) {
     set_error("gemm_gated_pair: %s", hipGetErrorString(e));
