@@ -1429,7 +1429,8 @@ struct BigTile {
   // us with two and with three stages of B: 2048 x 16384 x 2048 120 / 109, 2048 x 8192 x 2048 60.4 / 54.9, 4096^3 105 / 98; the same weights
   // again 105 either way, 8192^3 733 / 729).  Where the waves' loads do not come out even, those without rows go to 1 KB behind the stages.
   static constexpr int SPARE = BM / 8 % WAVES == 0 && BN / 8 % WAVES == 0 ? 0 : 1024;
-  static constexpr int A_STAGES = 3 * (A_BYTES + B_BYTES) + SPARE <= LDS_MOST ? 3 : 2, STAGES_BYTES = A_STAGES * A_BYTES + 3 * B_BYTES;
+  static constexpr int FIT = (LDS_MOST - SPARE) / (A_BYTES + B_BYTES);   // (tiles of four waves with room for more take four)
+  static constexpr int B_STAGES = FIT >= 4 ? 4 : 3, A_STAGES = FIT >= 3 ? B_STAGES : 2, STAGES_BYTES = A_STAGES * A_BYTES + B_STAGES * B_BYTES;
   static constexpr int OUT_ROW_BYTES = NT * 32 + 16, OUT_BYTES = WAVES * MI * 16 * OUT_ROW_BYTES;
   static constexpr int LDS_BYTES = STAGES_BYTES + SPARE > OUT_BYTES ? STAGES_BYTES + SPARE : OUT_BYTES;
   static_assert(LDS_BYTES <= LDS_MOST, "a CU's LDS");
@@ -1440,7 +1441,7 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
                                               bf16_t* __restrict__ C, int M, int N, int K,
                                               const int* __restrict__ valid, int tiles_m, int tiles_n,
                                               int patched, const GatedPair& pair = GatedPair{}) {
-  constexpr int WAVES = T::WAVES, MI = T::MI, NT = T::NT, A_STAGES = T::A_STAGES;
+  constexpr int WAVES = T::WAVES, MI = T::MI, NT = T::NT, A_STAGES = T::A_STAGES, B_STAGES = T::B_STAGES;
   constexpr int ROWB = BK * 2;                                        // bytes of a tile row in LDS, eight 16-byte chunks
   constexpr int A_BYTES = T::A_BYTES, B_BYTES = T::B_BYTES, B_BASE = A_STAGES * A_BYTES;   // A's stages, then B's
   constexpr int A_INST = T::BM / 8, B_INST = T::BN / 8;               // 1 KB loads of a stage: eight rows each
@@ -1472,7 +1473,7 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
   constexpr int KN_CHUNKS = T::BN / 8, KN_ROWS = 64 / KN_CHUNKS;   // chunks of a k-row, k-rows of an instruction
   static_assert(!B_KN || KN_CHUNKS == 32, "(K,N): rows of 256 columns");
   auto kn_swizzle = [](int k) { return ((k & 3) << 1) | (((k >> 3) & 3) << 3); };
-  // (PAIR: 64 rows of the gate's weights, 64 of the up projection's, and so on.)
+  // (PAIR: 8 NT rows of the gate's weights, as many of the up projection's, and so on.)
   const __amdgpu_buffer_rsrc_t b_rows = stage_rows(B_KN ? B + n0 + ((ptrdiff_t)(wave * KN_ROWS) - pad) * N : B + (size_t)(n0 + wave * 8) * K - pad);
   const __amdgpu_buffer_rsrc_t up_rows = PAIR ? stage_rows(pair.up + (size_t)(n0 + wave * 8) * K - pad) : b_rows;
   int kn_off[B_EACH], kn_row[B_EACH];   // (K,N): this lane's 16 bytes within instruction idx's k-rows, and the k-row
@@ -1482,7 +1483,7 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
     kn_off[i] = (int)(((size_t)(lane / KN_CHUNKS) * N + ((lane % KN_CHUNKS) ^ kn_swizzle(kn_row[i])) * 8) * 2);
   }
   const int inst_stride = WAVES * 8 * K * 2;
-  static_assert(!PAIR || WAVES == 4, "PAIR: the rows of an instruction below are four waves'");
+  static_assert(!PAIR || (WAVES == 4 && NT % 4 == 0), "PAIR: the rows of an instruction below are four waves'");
   auto issue_one = [&](int a_at, int b_at, int kt, int idx, bool head) {
     const int k_off = kt * ROWB;
     const bool is_a = idx < A_EACH;
@@ -1495,9 +1496,9 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
     if (is_a)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rows, IRON_LDS_PTR(to), 16, none || (head && ld_head < pad) ? NOWHERE : ld_off,
                                                i * inst_stride + k_off, 0, 0);
-    else if constexpr (PAIR)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds((i >> 1) & 1 ? up_rows : b_rows, IRON_LDS_PTR(to), 16, head && ld_head < pad ? NOWHERE : ld_off,
-                                               ((i >> 2) * 2 + (i & 1)) * inst_stride + k_off, 0, 0);
+    else if constexpr (PAIR)   // (NT / 4 of four waves' instructions are a wave's columns of one weight)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(i / (NT / 4) % 2 ? up_rows : b_rows, IRON_LDS_PTR(to), 16, head && ld_head < pad ? NOWHERE : ld_off,
+                                               (i / (NT / 2) * (NT / 4) + i % (NT / 4)) * inst_stride + k_off, 0, 0);
     else if constexpr (!B_KN)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rows, IRON_LDS_PTR(to), 16, none || (head && ld_head < pad) ? NOWHERE : ld_off,
                                                i * inst_stride + k_off, 0, 0);
@@ -1524,8 +1525,9 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
   //   first k-step: the second's B fragments from the start and its A fragments from the middle; loads in the slots between (EARLY of them)
   //   second k-step: up to slot BARRIER nothing -- then the stage's one barrier: every wave's loads of stage kt + 1 have landed and
   //     nobody reads stage kt any more (this k-step's fragments are in registers) -- then stage kt + 1's first fragments and LATE loads
-  // All loads are stage kt + 2's.  The early ones go into a buffer that the last barrier freed: B's, and A's where A has three stages; with two
-  // A's are the late ones, into this stage's buffer.
+  // B's loads, and with as many stages A's, are stage kt + B_STAGES - 1's and begin in the first k-step: the last barrier freed their buffer.  A's,
+  // with two stages, are stage kt + 2's and the late ones, into this stage's buffer.
+  static_assert(A_STAGES == B_STAGES || (A_STAGES == 2 && B_STAGES == 3), "stages alike, or two of A and three of B");
   constexpr int SLOTS = MI * NT, A_FROM = NT > SLOTS / 2 ? NT : SLOTS / 2, FREE = SLOTS - NT - MI;
   constexpr int EARLY = A_STAGES == 2 ? B_EACH : (LOADS < FREE ? LOADS : FREE), LATE = LOADS - EARLY;
   constexpr int EARLY_FROM = A_STAGES == 2 ? A_EACH : 0, LATE_FROM = A_STAGES == 2 ? 0 : EARLY;   // their numbers
@@ -1535,9 +1537,9 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
   constexpr int IN_GAP = EARLY < GAP / APART ? EARLY : GAP / APART;
   constexpr int Q3_FIRST = BARRIER + NT + MI, Q3_EVERY = SLOTS - Q3_FIRST > 2 * LATE && LATE > 0 ? (SLOTS - Q3_FIRST) / (LATE > 0 ? LATE : 1) : 1;
 #pragma unroll
-  for (int idx = 0; idx < LOADS; ++idx) issue_one(0, 0, 0, idx, true);
+  for (int st = 0; st < B_STAGES - 1; ++st)
 #pragma unroll
-  for (int idx = 0; idx < LOADS; ++idx) issue_one(A_BYTES, B_BYTES, min(1, nk - 1), idx, false);
+    for (int idx = 0; idx < LOADS; ++idx) issue_one(st * A_BYTES, st * B_BYTES, min(st, nk - 1), idx, st == 0);
 
   // Fragments: lane -> row fr of a 16-row tile, 16-byte chunk kq of the k-step's four.
   const int fr = lane & 15, kq = lane >> 4;
@@ -1610,7 +1612,7 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
     for (int j = 0; j < NT; ++j) bfr[ks][j] = tr_join(tfb[ks][j]);
   };
 
-  wait_vmcnt<LOADS>();   // stage 0 has landed once only stage 1 is out
+  wait_vmcnt<(B_STAGES - 2) * LOADS>();   // stage 0 has landed once only the younger ones are out
   block_barrier();
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
@@ -1622,12 +1624,12 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
     if constexpr (B_KN) b_frag_kn(0, 0, j, tfb[0][j]);
     else bfr[0][j] = b_frag(0, 0, j);
   }
-  // Where this stage's, the next one's and stage kt + 2's A and B lie.
-  int a_now = 0, a_next = A_BYTES, a_fill = A_STAGES == 2 ? 0 : 2 * A_BYTES, b_now = 0, b_next = B_BYTES, b_fill = 2 * B_BYTES;
+  // Where this stage's A and B lie, the next one's, and what the loads fill.
+  int a_now = 0, a_next = A_BYTES, a_fill = A_STAGES == 2 ? 0 : (A_STAGES - 1) * A_BYTES, b_now = 0, b_next = B_BYTES, b_fill = (B_STAGES - 1) * B_BYTES;
   for (int kt = 0; kt < nk; ++kt) {
     // Past the end the last stage is fetched again (into buffers nobody reads any more) rather than
     // branch: a branch would end the scheduling region and undo the interleaving below.
-    const int k2 = min(kt + 2, nk - 1);
+    const int k2 = min(kt + B_STAGES - 1, nk - 1);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       if constexpr (B_KN) join_kn(ks);
@@ -1638,7 +1640,7 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
           const int slot = i * NT + j;
           if (ks == 1 && slot == BARRIER) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            wait_vmcnt<EARLY>();   // all but what is out of stage kt + 2's
+            wait_vmcnt<(B_STAGES - 3) * LOADS + EARLY>();   // all but the stages behind the next one
             block_barrier();
           }
           mfma_16x16x32_in_place(acc[i][j], bfr[ks][j], af[ks][i]);
@@ -1670,13 +1672,12 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
         }
       }
     }
-    const int a_was = a_now, b_was = b_now;
+    b_fill = b_now;
+    a_fill = A_STAGES == 2 ? a_next : a_now;
     a_now = a_next;
-    a_next = A_STAGES == 2 ? a_was : a_fill;
-    a_fill = A_STAGES == 2 ? a_now : a_was;
     b_now = b_next;
-    b_next = b_fill;
-    b_fill = b_was;
+    a_next = a_now == (A_STAGES - 1) * A_BYTES ? 0 : a_now + A_BYTES;
+    b_next = b_now == (B_STAGES - 1) * B_BYTES ? 0 : b_now + B_BYTES;
   }
 
   if constexpr (B_KN) join_kn(0);   // the idle reads of the last iteration land while their registers are still theirs
@@ -1688,19 +1689,19 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
     // the same 8 NT columns of the output: the gate's product leaves as it is stored, then, made in the
     // accumulators' own layout, bf16(bf16(act(bf16 g)) * bf16 u).
     constexpr int HT = NT / 2, OROWB = HT * 32 + 16, LPRW = HT * 2, ORPI = 64 / LPRW;
-    static_assert(MI == 8, "a wave's 128 rows");
-    char* ot = smem_big + wave * (128 * OROWB);
+    constexpr int ROWS = MI * 16;   // of a wave
+    char* ot = smem_big + wave * (ROWS * OROWB);
     const int lr = lane / LPRW, lc = lane % LPRW;
-    const size_t first = (size_t)(m0 + wm * 128) * N + n0 + wn * HT * 16 + lc * 8;
+    const size_t first = (size_t)(m0 + wm * ROWS) * N + n0 + wn * HT * 16 + lc * 8;
     auto leave = [&](bf16_t* to) {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll 4
-      for (int r0 = 0; r0 < 128; r0 += ORPI) {
+      for (int r0 = 0; r0 < ROWS; r0 += ORPI) {
         const int r = r0 + lr;
         const uint4 v = *reinterpret_cast<const uint4*>(ot + r * OROWB + lc * 16);
-        if (m0 + wm * 128 + r < Mv) *reinterpret_cast<uint4*>(to + first + (size_t)r * N) = v;
+        if (m0 + wm * ROWS + r < Mv) *reinterpret_cast<uint4*>(to + first + (size_t)r * N) = v;
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();   // the rows are read before the next product overwrites them
@@ -1709,7 +1710,7 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
     // (The kind of gate is chosen once: asked an element, its branches made the lone wave of a SIMD wait 128 times over, and a
     // 2048 x 8192 x 2048 pair take 143 us instead of 130.)
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int j = 0; j < HT; ++j)
         *reinterpret_cast<uint2*>(ot + (i * 16 + fr) * OROWB + (j * 16 + 4 * kq) * 2) =
@@ -1717,7 +1718,7 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
     leave(pair.gate_out);
     auto gated = [&](auto kind) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < MI; ++i) {
       // A tile row at a time leaves the accumulation registers: all at once they would not fit.
 #pragma unroll
       for (int j = 0; j < NT; ++j) asm volatile("" : "+a"(acc[i][j]));
@@ -2219,81 +2220,115 @@ __device__ __forceinline__ void gemm_nt16_pair_body(const bf16_t* __restrict__ A
   leave(C);
 }
 
-// A gated feed-forward's two first projections over many rows as ONE launch, the tile chosen on the
-// device by the row bound as in gemm_either_kernel.  Few rows: 64 rows x (32 + 32) columns on the 64 x 64 tile's
-// loop, two waves a product (29 x 8192 x 2048 29.7 -> 20.5 us: as a gate tile and then an up tile a block made
-// two chains of stages).  Else 128 x 128 tiles of both products at once, or 256 rows x (128 + 128) columns, a wave's 128 x 128 half gate and half up
-// projection: the bytes a CU draws from L2 per flop are those of a 256 x 256 tile, two thirds of the smaller pair's.
-// A round of the large tiles takes 1.5 rounds of the small ones and covers two (N = 8192, K = 2048: 2048
-// rows 161 -> 130 us, 1024 89 -> 65; 512 rows, on the small tiles, 46.5 -> 41.8 by asking the kind of gate once).
-enum class PairForm { ROWS64, ROWS128, ROWS256 };
-// `few`: the rows below which 128 x 128 tiles would leave half the CUs idle.  Up to those 64 rows x (32 + 32) columns, a round of which takes about
-// a third of one of 128 x 128 tiles, so three rounds of them, or however many where each weight is read for one row of tiles (us, 64 against 128 rows, weights
-// out of memory: 888 x 3392 1600 rows 50.6 / 52.7, 2048 65 / 52.5; 3648 x 4160 400 rows 95 / 66; but 104 rows of 14336 x 4096 88 / 132).
-// The large tiles where their rounds, at 1.5 of the small ones', come out as no more (5632 x 2048: 1281 rows, 264 blocks, 113 against 82 by the small
-// ones, 1000 rows 57.6 against 81; 11776 x 4672: 580 rows 237 against 181).
-__host__ __device__ __forceinline__ PairForm pair_form(int rows, int few, int n32, int n128, bool large) {
-  const int blocks64 = ((rows + 63) / 64) * n32;
-  if (rows <= few && (blocks64 <= 768 || rows <= 128)) return PairForm::ROWS64;
-  const int rounds128 = (((rows + 127) / 128) * n128 + 255) / 256, rounds256 = (((rows + 255) / 256) * n128 + 255) / 256;
-  return large && 3 * rounds256 <= 2 * rounds128 ? PairForm::ROWS256 : PairForm::ROWS128;
+// Which form a launch under a row bound takes: the price list's, read by the bound where it is known, on the device.  Four bits for each run of
+// 64 << shift rows (the words are chosen by tests: by an index they would be another trip to memory behind the bound's), and a bit for each
+// form whose tiles come in patches.
+struct FormTable {
+  uint64_t w[4];
+  int shift, patched;
+};
+__device__ __forceinline__ int form_of_rows(const FormTable& t, int rows) {
+  const int run = max(rows - 1, 0) >> (6 + t.shift);
+  const uint64_t w = run < 32 ? (run < 16 ? t.w[0] : t.w[1]) : (run < 48 ? t.w[2] : t.w[3]);
+  return (int)(w >> ((run & 15) * 4)) & 15;
+}
+// `best(rows)` for the most rows of every run up to M; `upto[form]`: the most rows a form is taken for.
+template <class Best>
+static FormTable form_table(int M, Best best, int* upto) {
+  FormTable t{};
+  while ((64L << t.shift) * 64 < M) ++t.shift;
+  const long run = 64L << t.shift;
+  for (long rows = run, i = 0; rows < M + run; rows += run, ++i) {
+    const int r = rows < M ? (int)rows : M, form = best(r);
+    t.w[i >> 4] |= (uint64_t)form << ((i & 15) * 4);
+    if (r > upto[form]) upto[form] = r;
+  }
+  return t;
 }
 
+// A gated feed-forward's two first projections over many rows as ONE launch, the tile chosen on the
+// device by the row bound as in gemm_either_kernel.  Tiles of BN / 2 columns of both weights: a wave's columns are half gate and half up projection, so
+// the gated product is made in its registers (64 rows: on the 64 x 64 tile's loop, two waves a product; 29 x 8192 x 2048 29.7 -> 20.5 us).
+// Which tile: by rounds of blocks over the CUs, as big_form, at what a round was measured to take with weights out of memory.  8192 columns over
+// K = 2048, us, by 64 x (32 + 32), 128 x (128 + 128) and 256 x (128 + 128) tiles alone and by these: 128 rows 27.9 / 25.9, 256 38.5 / 27.4, 384 39.6 /
+// 33.2, 500 41.3 / 38.6, 640 58.5 / 45.7, 768 59.1 / 48.8, 1280 111 / 87, 1536 113 / 93, 1792 114 / 105.
+enum PairForm { PAIR_64X32, PAIR_EDGED, PAIR_128X64, PAIR_160X64, PAIR_192X64, PAIR_128X128, PAIR_160X128, PAIR_192X128, PAIR_224X128, PAIR_256X128, PAIR_FORMS };
+struct PairPrice {
+  int bm, bn;   // rows and columns of each product
+  float start, stage;
+};
+constexpr PairPrice PAIR_PRICES[PAIR_FORMS] = {
+    {64, 32, 3.f, 0.28f},    {128, 128, 7.f, 0.95f},    // (a product whose columns are no whole tiles: 128 rows at the edges' cost)
+    {128, 64, 4.f, 0.58f},   {160, 64, 4.5f, 0.64f},  {192, 64, 5.f, 0.73f},   {128, 128, 6.f, 0.90f},
+    {160, 128, 6.5f, 1.12f}, {192, 128, 7.5f, 1.2f},  {224, 128, 8.5f, 1.36f}, {256, 128, 9.5f, 1.5f},
+};
+static PairForm pair_form(int rows, int M, int N, int K) {
+  PairForm best = PAIR_64X32;
+  float price = 0.f;
+  for (int form = PAIR_64X32; form < PAIR_FORMS; ++form) {
+    const PairPrice& p = PAIR_PRICES[form];
+    if (form > PAIR_EDGED && (M < p.bm || N % p.bn != 0)) continue;
+    const long tiles = (long)((rows + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
+    const float us = (float)((tiles + 255) / 256) * (p.start + p.stage * (K / BK));
+    if (form == PAIR_64X32 || us < price) best = (PairForm)form, price = us;
+  }
+  return best;
+}
 __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __restrict__ A,
                                                               const bf16_t* __restrict__ Bg,
                                                               const bf16_t* __restrict__ Bu, bf16_t* __restrict__ G,
                                                               bf16_t* __restrict__ C, int M, int N, int K,
-                                                              const int* __restrict__ valid, Tiling t256, Tiling t128,
-                                                              Tiling t64, int few, int activation) {
-  const int Mv = bound_or(valid, M), bid = blockIdx.x;
-  const PairForm form = pair_form(Mv, few, t64.tiles_n, t128.tiles_n, t256.tiles_m > 0);
-  QkvTail gate{};
-  gate.gated = activation;
-  if (form == PairForm::ROWS256) {
-    if (bid >= t256.tiles_m * t256.tiles_n) return;
-    gemm_big_body<Tile256Four, false, false, true>(A, Bg, C, M, N, K, valid, t256.tiles_m, t256.tiles_n, t256.patched,
-                                                   GatedPair{Bu, G, activation});
-  } else if (form == PairForm::ROWS128) {
-    if (bid >= t128.tiles_m * t128.tiles_n) return;
-    gemm_nt16_pair_body(A, Bg, Bu, G, C, M, N, K, valid, t128.tiles_m, t128.tiles_n, t128.patched, activation);
-  } else {
-    if (bid >= t64.tiles_m * t64.tiles_n) return;
-    gemm_nt64_body<8, true>(A, Bg, C, M, N, K, valid, t64.tiles_m, t64.tiles_n, t64.patched, gate, Bu, G);
+                                                              const int* __restrict__ valid, FormTable forms, int activation) {
+  const int form = form_of_rows(forms, bound_or(valid, M)), patched = forms.patched >> form & 1;
+  const GatedPair pair{Bu, G, activation};
+#define IRON_PAIR(FORM, MI, NT) \
+  case FORM: \
+    static_assert(PAIR_PRICES[FORM].bm == 32 * MI && PAIR_PRICES[FORM].bn == 16 * NT, "the tile that was priced"); \
+    gemm_big_body<BigTile<2, 2, MI, NT>, false, false, true>(A, Bg, C, M, N, K, valid, (M + 32 * MI - 1) / (32 * MI), N / (16 * NT), patched, pair); \
+    break
+  switch (form) {
+    IRON_PAIR(PAIR_128X64, 4, 4);
+    IRON_PAIR(PAIR_160X64, 5, 4);
+    IRON_PAIR(PAIR_192X64, 6, 4);
+    IRON_PAIR(PAIR_128X128, 4, 8);
+    IRON_PAIR(PAIR_160X128, 5, 8);
+    IRON_PAIR(PAIR_192X128, 6, 8);
+    IRON_PAIR(PAIR_224X128, 7, 8);
+    IRON_PAIR(PAIR_256X128, 8, 8);
+    case PAIR_EDGED:
+      gemm_nt16_pair_body(A, Bg, Bu, G, C, M, N, K, valid, (M + 127) / 128, (N + 127) / 128, patched, activation);
+      break;
+    default: {
+      QkvTail gate{};
+      gate.gated = activation;
+      gemm_nt64_body<8, true>(A, Bg, C, M, N, K, valid, (M + 63) / 64, (N + 31) / 32, patched, gate, Bu, G);
+    }
   }
+#undef IRON_PAIR
 }
 
 static int launch_gemm_gated_pair(const bf16_t* A, const bf16_t* Bg, const bf16_t* Bu, bf16_t* G, bf16_t* C, int M,
                                   int N, int K, const int* valid, int activation, hipStream_t s) {
-  const int n128 = (N + 127) / 128, n32 = (N + 31) / 32, few = n128 >= 128 ? 0 : 128 * (127 / n128);
-  const bool large = M >= BIG_BM && N % 128 == 0;
-  // The most rows each form is chosen for: its grid covers those.
-  int most[3] = {0, 0, 0};
-  for (int rows = valid == nullptr ? M : 1; rows < M + 64; rows += 64) {   // (a form is the same within a run of 64 rows that ends on a multiple of them)
-    const int r = rows < M ? rows : M;
-    int& upto = most[(int)pair_form(r, few, n32, n128, large)];
-    const int end = ((r + 63) / 64) * 64 < M ? ((r + 63) / 64) * 64 : M;
-    if (end > upto) upto = end;
-  }
-  auto tiling = [](int tile_rows, int tile_cols) {
-    const int whole = (tile_rows + 7) & ~7;
+  int upto[PAIR_FORMS] = {};   // each form's grid covers the rows it is chosen for
+  FormTable forms = form_table(M, [&](int rows) { return (int)pair_form(valid == nullptr ? M : rows, M, N, K); }, upto);
+  int blocks = 1;
+  for (int form = 0; form < PAIR_FORMS; ++form) {
+    // Tile rows rounded up to whole patches where that lets the XCD-aware order apply: the added
+    // tiles lie past the bound any block of that tiling runs for, and leave at once.
+    int tile_rows = (upto[form] + PAIR_PRICES[form].bm - 1) / PAIR_PRICES[form].bm;
+    const int tile_cols = (N + PAIR_PRICES[form].bn - 1) / PAIR_PRICES[form].bn, whole = (tile_rows + 7) & ~7;
     if (tile_rows >= 8 && !patched_order(tile_rows, tile_cols) && patched_order(whole, tile_cols)) tile_rows = whole;
-    return Tiling{tile_rows, tile_cols, patched_order(tile_rows, tile_cols)};
-  };
-  // (the 64-row tiles in the order of all the rows up to `few`: 580 of 1024 rows in patches of eight tile rows took 27.2 us at 1536 x 1536, not 22.4)
-  const Tiling t64 = tiling(most[0] > 0 ? ((few < M ? few : M) + 63) / 64 : 0, n32), t128 = tiling((most[1] + 127) / 128, n128);
-  const Tiling t256 = large ? tiling((M + BIG_BM - 1) / BIG_BM, n128) : Tiling{0, 0, 0};
-  constexpr size_t lds = Tile256Four::LDS_BYTES;   // the large tile's, more than the others'
+    forms.patched |= (tile_rows >= 8 && patched_order(tile_rows, tile_cols)) << form;
+    if (tile_rows * tile_cols > blocks) blocks = tile_rows * tile_cols;
+  }
+  constexpr size_t lds = Tile256Four::LDS_BYTES;   // the largest tile's, more than the others'
   static_assert(lds >= (size_t)PAIR_STAGES * 3 * 128 * BK * 2 && lds >= (size_t)NT_STAGES * 256 * BK * 2, "the other bodies' stages fit too");
   static LdsOptIn opt_in;
   if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_gated_pair_kernel), lds); e != hipSuccess) {
     set_error("gemm_gated_pair: %s", hipGetErrorString(e));
     return (int)e;
   }
-  int blocks = t128.tiles_m * t128.tiles_n;
-  if (most[2] > 0 && t256.tiles_m * t256.tiles_n > blocks) blocks = t256.tiles_m * t256.tiles_n;
-  if (t64.tiles_m * t64.tiles_n > blocks) blocks = t64.tiles_m * t64.tiles_n;
-  hipLaunchKernelGGL(gemm_gated_pair_kernel, dim3(blocks), dim3(256), lds, s, A, Bg, Bu, G, C, M, N, K, valid, t256, t128, t64,
-                     few, activation);
+  hipLaunchKernelGGL(gemm_gated_pair_kernel, dim3(blocks), dim3(256), lds, s, A, Bg, Bu, G, C, M, N, K, valid, forms, activation);
   IRON_LAUNCH_CHECK();
 }
 

@@ -670,7 +670,10 @@ def test_gemm_gated_epilogue(cuda, M, Kdim, N, rows, activation):
                                            (256, 512, 1024, None), (192, 128, 320, 70),
                                            # 256-row tiles: one stage, two, the last tile moved back, a bound inside it
                                            (2048, 64, 4096, None), (1300, 128, 4096, None), (1301, 192, 4096, 1100),
-                                           (257, 64, 16512, 257), (1300, 128, 4100, None)])
+                                           (257, 64, 16512, 257), (1300, 128, 4100, None),
+                                           # every form by the bound: 64 x 32 (of each), 128 x 64, 160 x 64, 192 x 64, 128 x 128, 160, 192, 224, 256 x 128
+                                           *[(2000, 128, 8192, rows) for rows in (1, 64, 65, 256, 257, 320, 321, 449, 513, 641, 769, 1600, 1793, 2000)],
+                                           (1999, 192, 4160, 1100), (4500, 64, 1088, 3000), (160, 64, 2048, 159)])
 @pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
 def test_gemm_gated_pair_is_the_two_launches_bit_for_bit(cuda, M, Kdim, N, rows, activation):
     """Both first projections of a gated feed-forward in one launch: the gate's product and the gated
