@@ -418,21 +418,20 @@ constexpr int NOWHERE = (int)0x80000000u;   // past stage_rows' 2^31 - 1 bytes, 
 // the tiles outnumber the CUs, 8 (128 KB, more loads in flight) where a CU has one block anyway.
 // An element's sum is the same chain of 32-wide k-steps as in the 128 x 128 and the 256 x 256 tiles: where a row bound chooses
 // the tile, a row's products are the same bits whatever rows share the launch.
-// `qkv` carries only the optional residual epilogue here.  PAIR: both
+// `qkv` carries only the optional residual epilogue here.  MI: 16-row tiles a wave owns; 4 make 128 x 64 tiles.  PAIR: both
 // first products of a gated feed-forward, 32 columns of each (`qkv` says the gate's kind).
-template <int STAGES, bool PAIR = false>
+template <int STAGES, bool PAIR = false, int MI = 2>
 __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
                                                bf16_t* __restrict__ C, int M, int N, int K,
-                                               const int* __restrict__ valid, int tiles_m, int tiles_n,
+                                               int Mv, int tiles_m, int tiles_n,
                                                int patched, const QkvTail& qkv,
                                                const bf16_t* __restrict__ up = nullptr, bf16_t* __restrict__ gate_out = nullptr) {
-  constexpr int NT_BM = 64, NT_BN = 64;
+  constexpr int NT_BM = 32 * MI, NT_BN = 64;
   constexpr int NT_A_BYTES = NT_BM * BK * 2, NT_STAGE_BYTES = (NT_BM + NT_BN) * BK * 2;
-  constexpr int INST = NT_BM / 8 / 4;  // 1 KB loads of A (and of B) a wave issues per stage
-  constexpr int LOADS = 2 * INST;
-  static_assert(BK == 64 && LOADS == 4 && STAGES >= 4, "two 32-wide k-steps a stage, a load behind every second MFMA");
+  constexpr int INST = NT_BM / 8 / 4, B_INST = NT_BN / 8 / 4;  // 1 KB loads of A and of B a wave issues per stage
+  constexpr int LOADS = INST + B_INST;
+  static_assert(BK == 64 && LOADS <= 2 * MI && STAGES >= 4 && (MI == 2 || !PAIR), "two 32-wide k-steps a stage, a load behind every second MFMA");
   extern __shared__ __align__(16) char smem_nt[];
-  const int Mv = bound_or(valid, M);
 
   int tm, tn;
   if (!live_tile(blockIdx.x, tiles_m, tiles_n, patched, (Mv + NT_BM - 1) / NT_BM, tm, tn)) return;
@@ -444,7 +443,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const int lrow = lane >> 3, pch = lane & 7;
-  int a_voff[INST], b_voff[INST], head_ch[INST];
+  int a_voff[4], b_voff[2], head_ch[4];   // (instruction i of A and of B begin on rows that are 16 i apart or all alike: one swizzle)
 #pragma unroll
   for (int i = 0; i < INST; ++i) {
     const int r = (wave * INST + i) * 8 + lrow;
@@ -452,12 +451,17 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
     head_ch[i] = lch * 8;
     // Rows past the end re-read the last row; what they produce is never stored.
     a_voff[i] = (int)(((size_t)(min(m0 + r, M - 1) - m0) * K + lch * 8) * 2);
-    b_voff[i] = (int)(((size_t)(min(n0 + (PAIR ? r % (NT_BN / 2) : r), N - 1) - n0) * K + lch * 8) * 2);
+  }
+#pragma unroll
+  for (int i = 0; i < B_INST; ++i) {
+    const int r = (wave * B_INST + i) * 8 + lrow;
+    b_voff[i] = (int)(((size_t)(min(n0 + (PAIR ? r % (NT_BN / 2) : r), N - 1) - n0) * K + (pch ^ ((r >> 1) & 7)) * 8) * 2);
   }
   const int pad = k_pad(K);
   const bf16_t* a_tile = A + (size_t)m0 * K - pad;
   // (PAIR: the tile's first 32 columns are the gate's, which waves 0 and 1 load and the waves wn = 0 compute, the rest the up projection's)
   const bf16_t* b_tile = (PAIR && wave >= 2 ? up : B) + (size_t)n0 * K - pad;
+  const int b_first = NT_A_BYTES + wave * B_INST * 1024;   // where a wave's part of B begins in a stage
   // One load of the 2*INST a wave issues per stage (A's first, then B's).
   auto issue_one = [&](char* st, int kt, int idx, bool head) {
     const int k0 = kt * BK;
@@ -467,25 +471,25 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
                                                head && head_ch[idx] < pad ? NOWHERE : a_voff[idx], 0, 0, 0);
     } else {
       const __amdgpu_buffer_rsrc_t rows = stage_rows(b_tile + k0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, IRON_LDS_PTR(st + NT_A_BYTES + (wave * INST + idx - INST) * 1024),
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, IRON_LDS_PTR(st + b_first + (idx - INST) * 1024),
                                                16, head && head_ch[idx - INST] < pad ? NOWHERE : b_voff[idx - INST], 0, 0, 0);
     }
   };
 
-  f32x4 acc[2][2];
+  f32x4 acc[MI][2];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t >> 1][t & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < 2 * MI; ++t) acc[t >> 1][t & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // acc[i][j][e]: row 16 i + fr of the wave's 32 x 32, column 16 j + 4 kq + e.
+  // acc[i][j][e]: row 16 i + fr of the wave's 16 MI x 32, column 16 j + 4 kq + e.
   const int fr = lane & 15, kq = lane >> 4;
-  const int mb = m0 + wm * 32 + fr, nb = n0 + (PAIR ? 0 : wn * 32) + 4 * kq;
+  const int mb = m0 + wm * (16 * MI) + fr, nb = n0 + (PAIR ? 0 : wn * 32) + 4 * kq;
   // A residual's pieces this lane will add in the epilogue are requested now, so that their
   // latency passes under the whole product instead of at its end (N a multiple of 4: 8-byte pieces).
-  uint2 res[2][2];
+  uint2 res[MI][2];
   const bool res_ahead = !PAIR && qkv.residual != nullptr && (N & 3) == 0;
   if (res_ahead) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
         res[i][j] = *reinterpret_cast<const uint2*>(qkv.residual + (size_t)min(mb + 16 * i, M - 1) * N + min(nb + 16 * j, N - 4));
@@ -500,7 +504,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
     for (int idx = 0; idx < LOADS; ++idx) issue_one(smem_nt + s * NT_STAGE_BYTES, min(s, nk - 1), idx, s == 0);
 
   // Fragments: lane -> row fr of a 16-row tile, 16-byte chunk kq of the k-step's four.
-  const int a_off = (wm * 32 + fr) * 128, b_off = NT_A_BYTES + (wn * 32 + fr) * 128, swz = (fr >> 1) & 7;
+  const int a_off = (wm * (16 * MI) + fr) * 128, b_off = NT_A_BYTES + (wn * 32 + fr) * 128, swz = (fr >> 1) & 7;
   auto a_frag = [&](const char* st, int ks, int i) {
     return *reinterpret_cast<const bf16x8*>(st + a_off + i * 16 * 128 + (((ks * 4 + kq) ^ swz) << 4));
   };
@@ -510,11 +514,11 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
 
   wait_vmcnt<(STAGES - 2) * LOADS>();   // stage 0 has landed once only the younger ones are out
   block_barrier();
-  bf16x8 af[2][2][2], bfr[2][2][2];   // [stage parity][k-step][tile]
+  bf16x8 af[2][2][MI], bfr[2][2][2];   // [stage parity][k-step][tile]
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    af[0][t >> 1][t & 1] = a_frag(smem_nt, t >> 1, t & 1);
-    bfr[0][t >> 1][t & 1] = b_frag(smem_nt, t >> 1, t & 1);
+  for (int t = 0; t < 2 * MI; ++t) {
+    af[0][t / MI][t % MI] = a_frag(smem_nt, t / MI, t % MI);
+    if (t % MI < 2) bfr[0][t / MI][t % MI] = b_frag(smem_nt, t / MI, t % MI);
   }
   // Two stages an iteration, so that the register sets are named at compile time.
   auto stage = [&](int kt, auto parity) {
@@ -523,8 +527,8 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
     char* nst = smem_nt + ((kt + STAGES - 1) % STAGES) * NT_STAGE_BYTES;  // stage kt-1's buffer
     const int kn = min(kt + STAGES - 1, nk - 1);   // past the end the last stage again: the wait counts stay exact
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int ks = t >> 1, i = t & 1;
+    for (int t = 0; t < 2 * MI; ++t) {
+      const int ks = t / MI, i = t % MI;
       mfma_16x16x32_in_place(acc[i][0], bfr[P][ks][0], af[P][ks][i]);
       mfma_16x16x32_in_place(acc[i][1], bfr[P][ks][1], af[P][ks][i]);
       __builtin_amdgcn_sched_barrier(0);
@@ -535,8 +539,8 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
         __builtin_amdgcn_sched_barrier(0);
       }
       af[P ^ 1][ks][i] = a_frag(st1, ks, i);
-      bfr[P ^ 1][ks][i] = b_frag(st1, ks, i);
-      issue_one(nst, kn, t, false);
+      if (i < 2) bfr[P ^ 1][ks][i] = b_frag(st1, ks, i);
+      if (t < LOADS) issue_one(nst, kn, t, false);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -551,7 +555,9 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
 
   wait_vmcnt<0>();  // the idle fetches of the last iterations land before the block's LDS is released
   // (the matrix cores' last results: the compiler does not know what the assembly's are)
-  asm volatile("s_nop 15\n\ts_nop 3" : "+a"(acc[0][0]), "+a"(acc[0][1]), "+a"(acc[1][0]), "+a"(acc[1][1]));
+  asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");
+#pragma unroll
+  for (int t = 0; t < 2 * MI; ++t) asm volatile("" : "+a"(acc[t >> 1][t & 1]));
   if constexpr (PAIR) {
     // The gate's waves leave their product, rounded as it is stored, in LDS for the others and store it; those make
     // bf16(bf16(act(bf16 g)) * bf16 u) of it.
@@ -576,7 +582,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
   const bool vec = (N & 3) == 0;   // rows of 8-byte pieces
   auto pieces = [&](auto residual) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < MI; ++i) {
       const int m = mb + 16 * i;
       if (m >= Mv) continue;
       bf16_t* row = C + (size_t)m * N;
@@ -631,7 +637,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
 template <bool QKV, bool B_KN = false, bool C_NM = false, bool SHARED = false>
 __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B_,
                                                bf16_t* __restrict__ C_, int M, int N_, int K,
-                                               const int* __restrict__ valid, int tiles_m, int tiles_n,
+                                               int Mv, int tiles_m, int tiles_n,
                                                int patched, const QkvTail& qkv) {
   constexpr int NT_BM = 128, NT_BN = 128;
   constexpr int NT_A_BYTES = NT_BM * BK * 2, NT_STAGE_BYTES = (NT_BM + NT_BN) * BK * 2;
@@ -641,7 +647,6 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
   static_assert(!(B_KN && QKV), "the fused projections read weights as stored, (N,K)");
   static_assert(B_KN || !C_NM, "with B (N,K) the (N,M) output is the product of B and A");
   extern __shared__ __align__(16) char smem_nt[];
-  const int Mv = bound_or(valid, M);
 
   int tm, tn;
   const bool given = !QKV && qkv.tile_plus1 > 0;
@@ -1025,9 +1030,9 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(const bf16_t* __restrict__
   if constexpr (QKV) to_cache_rows(qkv, valid, M);
   static_assert(T == 2 || (T == 1 && !B_KN && !QKV), "64x64 tiles: B (N,K), plain or residual output");
   if constexpr (T == 2)
-    gemm_nt16_body<QKV, B_KN, C_NM>(A, B, C, M, N, K, valid, tiles_m, tiles_n, patched, qkv);
+    gemm_nt16_body<QKV, B_KN, C_NM>(A, B, C, M, N, K, bound_or(valid, M), tiles_m, tiles_n, patched, qkv);
   else
-    gemm_nt64_body<STAGES64>(A, B, C, M, N, K, valid, tiles_m, tiles_n, patched, qkv);
+    gemm_nt64_body<STAGES64>(A, B, C, M, N, K, bound_or(valid, M), tiles_m, tiles_n, patched, qkv);
 }
 
 template <bool B_KN, bool QKV = false, int T = 2, int STAGES64 = 4, bool C_NM = false>
@@ -1318,7 +1323,7 @@ __global__ __launch_bounds__(256) void qkv_either_kernel(const bf16_t* __restric
       qkv_heads_body<3>(A, Bq, Cq, M, heads, kv_heads, K, valid, wide.tiles_m, wide.tiles_n, wide.patched, qkv);
   } else {
     if ((int)blockIdx.x < narrow.tiles_m * narrow.tiles_n)
-      gemm_nt16_body<true>(A, Bq, Cq, M, heads * 64, K, valid, narrow.tiles_m, narrow.tiles_n, narrow.patched, qkv);
+      gemm_nt16_body<true>(A, Bq, Cq, M, heads * 64, K, Mv, narrow.tiles_m, narrow.tiles_n, narrow.patched, qkv);
   }
 }
 
@@ -1410,9 +1415,8 @@ static int launch_gemm(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N
 // from L2 into LDS is what bounds the smaller tile.  WM x WN waves, each owning MI x NT accumulator tiles of 16 x 16: the
 // tile's height and width are then chosen by how the product's rounds over the chip come out (see big_tiling).  Within a wave
 // the instruction stream still interleaves the next k-step's fragment reads and the next stages' loads with the MFMAs.  Where the
-// blocks of one launch choose their tile size by a row bound (gemm_either_kernel) the large tile is four waves of
+// blocks of one launch choose their tile size by a row bound (gemm_rows_kernel) the large tile is four waves of
 // 128 x 128, as every other tiling of that launch is four waves.
-constexpr int BIG_BM = 256, BIG_BN = 256;
 
 // The operands of a gated feed-forward's two first projections beyond the gate's own.
 struct GatedPair {
@@ -1436,11 +1440,12 @@ struct BigTile {
   static_assert(LDS_BYTES <= LDS_MOST, "a CU's LDS");
 };
 
-template <class T, bool B_KN = false, bool STREAM_OUT = false, bool PAIR = false>
+// PAIR: both first products of a gated feed-forward.  TAIL: a residual sum or a gate in the epilogue (N a multiple of 8).
+template <class T, bool B_KN = false, bool STREAM_OUT = false, bool PAIR = false, bool TAIL = false>
 __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
                                               bf16_t* __restrict__ C, int M, int N, int K,
-                                              const int* __restrict__ valid, int tiles_m, int tiles_n,
-                                              int patched, const GatedPair& pair = GatedPair{}) {
+                                              int Mv, int tiles_m, int tiles_n,
+                                              int patched, const GatedPair& pair = GatedPair{}, const QkvTail& tail = QkvTail{}) {
   constexpr int WAVES = T::WAVES, MI = T::MI, NT = T::NT, A_STAGES = T::A_STAGES, B_STAGES = T::B_STAGES;
   constexpr int ROWB = BK * 2;                                        // bytes of a tile row in LDS, eight 16-byte chunks
   constexpr int A_BYTES = T::A_BYTES, B_BYTES = T::B_BYTES, B_BASE = A_STAGES * A_BYTES;   // A's stages, then B's
@@ -1448,7 +1453,6 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
   constexpr int A_EACH = (A_INST + WAVES - 1) / WAVES, B_EACH = (B_INST + WAVES - 1) / WAVES, LOADS = A_EACH + B_EACH;   // ... a wave's
   constexpr int A_LAST = A_INST % WAVES, B_LAST = B_INST % WAVES;     // waves that have a last one (0: all)
   extern __shared__ __align__(16) char smem_big[];
-  const int Mv = bound_or(valid, M);
 
   int tm, tn;
   if (!live_tile(blockIdx.x, tiles_m, tiles_n, patched, (Mv + T::BM - 1) / T::BM, tm, tn)) return;
@@ -1517,6 +1521,18 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.f;
+
+  // Where a lane stores: lanes of 16 bytes a tile row, rows an instruction (of 96-byte rows ten: four lanes idle).
+  constexpr int LPRW = NT * 2, ORPI = 64 / LPRW, PIECES = (MI * 16 + ORPI - 1) / ORPI;
+  const int lr = lane / LPRW, lc = lane % LPRW;
+  const int row0 = m0 + wm * MI * 16;
+  // A residual's pieces this lane will add in the epilogue are requested now, so that their latency passes under the product.
+  uint4 res[TAIL ? PIECES : 1];
+  if constexpr (TAIL) {
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i)
+      res[i] = *reinterpret_cast<const uint4*>(tail.residual + (size_t)min(row0 + i * ORPI + lr, M - 1) * N + n0 + wn * NT * 16 + lc * 8);
+  }
 
   const int nk = (K + pad) / BK;
   // A stage is two k-steps of MI NT MFMAs; source order is issue order (nothing crosses a sched_barrier): after an MFMA one
@@ -1688,7 +1704,7 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
     // Columns 0 .. NT / 2 - 1 of the wave's tiles are the gate's product, the rest the up projection's, of
     // the same 8 NT columns of the output: the gate's product leaves as it is stored, then, made in the
     // accumulators' own layout, bf16(bf16(act(bf16 g)) * bf16 u).
-    constexpr int HT = NT / 2, OROWB = HT * 32 + 16, LPRW = HT * 2, ORPI = 64 / LPRW;
+    constexpr int HT = NT / 2, OROWB = HT * 32 + 16, LPRW = HT * 2, ORPI = 64 / LPRW;   // (half a tile's columns at a time)
     constexpr int ROWS = MI * 16;   // of a wave
     char* ot = smem_big + wave * (ROWS * OROWB);
     const int lr = lane / LPRW, lc = lane % LPRW;
@@ -1756,10 +1772,6 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  constexpr int LPRW = NT * 2;        // lanes (16 bytes each) per tile row
-  constexpr int ORPI = 64 / LPRW;     // rows per instruction (of 96-byte rows ten: four lanes idle)
-  const int lr = lane / LPRW, lc = lane % LPRW;
-  const int row0 = m0 + wm * MI * 16;
   bf16_t* cbase = C + (size_t)row0 * N + n0 + wn * NT * 16 + lc * 8;
   // STREAM_OUT (the launch sets it over a long K): the tile leaves by non-temporal stores, so C's
   // lines do not stay in the XCD's L2 among the A and B panels its blocks re-read (8192^3: 790 ->
@@ -1767,12 +1779,20 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
   // larger part of its time).  A template argument: as a branch on K the compiler merged the two
   // stores into one plain one.
   typedef unsigned int u32x4_t __attribute__((ext_vector_type(4), aligned(2)));   // (rows begin where they begin, see store_loose)
-#pragma unroll 4
+#pragma unroll TAIL ? PIECES : 4
   for (int r0 = 0; r0 < MI * 16; r0 += ORPI) {
     const int r = r0 + lr;
     if (64 % LPRW != 0 && (lr >= ORPI || r >= MI * 16)) continue;
-    const uint4 v = *reinterpret_cast<const uint4*>(ot + r * OROWB + lc * 16);
-    if (row0 + r < Mv) {
+    uint4 v = *reinterpret_cast<const uint4*>(ot + r * OROWB + lc * 16);
+    if constexpr (TAIL) {   // the product rounded as it would be stored, then scale * it + residual, or its gate
+      float x[8], rf[8];
+      unpack8(v, x);
+      unpack8(res[r0 / ORPI], rf);
+      tail_of(tail, x, rf);
+      v = pack8(x);
+    }
+    // (TAIL: C may be the residual itself, so what two tiles both cover is one's to store)
+    if (row0 + r < Mv && (!TAIL || (row0 + r >= tm * T::BM && n0 + wn * NT * 16 + lc * 8 >= tn * T::BN))) {
       if constexpr (STREAM_OUT)
         __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, v), reinterpret_cast<u32x4_t*>(cbase + (size_t)r * N));
       else
@@ -1794,63 +1814,132 @@ __global__ __launch_bounds__(T::WAVES * 64) void gemm_big_kernel(const bf16_t* _
                                                                  bf16_t* __restrict__ C, int M, int N, int K,
                                                                  const int* __restrict__ valid, int tiles_m,
                                                                  int tiles_n, int patched) {
-  gemm_big_body<T, B_KN, STREAM_OUT>(A, B, C, M, N, K, valid, tiles_m, tiles_n, patched);
+  gemm_big_body<T, B_KN, STREAM_OUT>(A, B, C, M, N, K, bound_or(valid, M), tiles_m, tiles_n, patched);
 }
 
-// A row bound read on the device decides which tile size fills the chip best (512 valid rows of
-// 2048 leave 64 of 256 large tiles), so under one the blocks of ONE launch choose: 256 x 256 tiles
-// past `few256` rows (BIG: the shape takes them), 128 x 128 past `few128`, 64 x 64 below.  Each
-// tiling's grid covers only the rows it can be chosen for; the launch's grid is the largest of
-// them and a block past its tiling's tiles leaves at once.  LDS is the largest tiling's, so a CU
-// holds one block whatever the choice.
-template <bool BIG>
-__global__ __launch_bounds__(256) void gemm_either_kernel(const bf16_t* __restrict__ A,
-                                                          const bf16_t* __restrict__ B, bf16_t* __restrict__ C,
-                                                          int M, int N, int K, const int* __restrict__ valid,
-                                                          Tiling t256, Tiling t128, Tiling t64, int few256,
-                                                          int few128, QkvTail tail) {
-  // The blocks of this launch are four waves whatever the stand-alone large-tile launch uses.
-  const int Mv = bound_or(valid, M), bid = blockIdx.x;
-  if (BIG && Mv > few256) {
-    if (bid < t256.tiles_m * t256.tiles_n)
-      gemm_big_body<Tile256Four>(A, B, C, M, N, K, valid, t256.tiles_m, t256.tiles_n, t256.patched);
-  } else if (Mv > few128) {
-    if (bid < t128.tiles_m * t128.tiles_n)
-      gemm_nt16_body<false>(A, B, C, M, N, K, valid, t128.tiles_m, t128.tiles_n, t128.patched, tail);
-  } else {
-    if (bid < t64.tiles_m * t64.tiles_n)
-      gemm_nt64_body<8>(A, B, C, M, N, K, valid, t64.tiles_m, t64.tiles_n, t64.patched, tail);
+// Which form a launch under a row bound takes: the price list's, read by the bound where it is known, on the device.  Four bits for each run of
+// 64 << shift rows (the words are chosen by tests, not by an index: that would be another trip to memory behind the bound's), and a bit for each
+// form whose tiles come in patches.
+struct FormTable {
+  uint64_t w[4];
+  int shift, patched;
+};
+struct FormOfRows {
+  int rows, form, patched;
+};
+__device__ __forceinline__ FormOfRows form_of_rows(const FormTable& t, const int* __restrict__ valid, int M) {
+  uint64_t w0 = t.w[0], w1 = t.w[1], w2 = t.w[2], w3 = t.w[3];
+  int shift = t.shift, patched = t.patched, bound = valid == nullptr ? M : *valid;
+  asm volatile("" : "+s"(w0), "+s"(w1), "+s"(w2), "+s"(w3), "+s"(shift), "+s"(patched), "+s"(bound));   // (one wait for the bound and the table)
+  const int rows = max(0, min(bound, M)), run = max(rows - 1, 0) >> (6 + shift);
+  const uint64_t w = run < 32 ? (run < 16 ? w0 : w1) : (run < 48 ? w2 : w3);
+  const int form = (int)(w >> ((run & 15) * 4)) & 15;
+  return FormOfRows{rows, form, patched >> form & 1};
+}
+// `best(rows)` for the most rows of every run up to M; `upto[form]`: the most rows a form is taken for.
+template <class Best>
+static FormTable form_table(int M, Best best, int* upto) {
+  FormTable t{};
+  while ((64L << t.shift) * 64 < M) ++t.shift;
+  const long run = 64L << t.shift;
+  for (long rows = run, i = 0; rows < M + run; rows += run, ++i) {
+    const int r = rows < M ? (int)rows : M, form = best(r);
+    t.w[i >> 4] |= (uint64_t)form << ((i & 15) * 4);
+    if (r > upto[form]) upto[form] = r;
   }
+  return t;
 }
 
-template <bool BIG>
-static int launch_gemm_either(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, const int* valid,
-                              hipStream_t s, int few256, int few128, QkvTail tail = QkvTail{}) {
-  // Rows a tiling can be chosen for: the large one all of them, the others up to the next one's bound.
-  const int rows128 = BIG ? (few256 < M ? few256 : M) : M, rows64 = few128 < M ? few128 : M;
-  const int n128 = (N + 127) / 128, n64 = (N + 63) / 64;
-  const Tiling t256{BIG ? M / BIG_BM : 0, BIG ? N / BIG_BN : 0, BIG ? patched_order(M / BIG_BM, N / BIG_BN) : 0};
-  // Tile rows rounded up to whole patches where that lets the XCD-aware order apply: the added
-  // tiles lie past the bound any block of that tiling runs for, and leave at once.
-  auto tiling = [](int tile_rows, int tile_cols) {
-    const int whole = (tile_rows + 7) & ~7;
+// A product under a row bound that is read on the device: the blocks of ONE launch take the form that is the cheapest at the bound (512 valid rows of
+// 2048 leave 64 of 256 large tiles).  Each form's grid covers only the rows it can be chosen for; the launch's grid is the largest of
+// them and a block past its tiling's tiles leaves at once.  LDS is the largest tiling's, so a CU
+// holds one block whatever the choice, and four waves are a block whatever the stand-alone launch of a form uses.
+// The prices: rounds of blocks, as big_form, at what a round was measured to take with weights out of memory behind the launch's own 4.5 us (by 64 x 64,
+// 128 x 128 and 256 x 256 tiles alone and by these, us: 2048 columns over 2048 with a residual, 640 rows 19.9 / 17.7, 1024 23.7 / 18.4; over 8192, 900
+// rows 68 / 52; 8192 over 2048, 256 rows 22.9 / 18.6, 640 42 / 26, 1024 43 / 34, 1280 50 / 39; 6144 over 2048, 1200 rows 54 / 32).
+enum RowsForm { ROWS_64X64, ROWS_128X64, ROWS_128X128, ROWS_160X128, ROWS_192X128, ROWS_256X128, ROWS_160X256, ROWS_192X256, ROWS_256X256, ROWS_FORMS };
+struct RowsPrice {
+  int bm, bn;
+  float start, stage;
+};
+constexpr RowsPrice ROWS_PRICES[ROWS_FORMS] = {
+    {64, 64, 0.8f, 0.28f},   {128, 64, 2.f, 0.34f},   {128, 128, 4.f, 0.45f}, {160, 128, 3.4f, 0.52f}, {192, 128, 5.f, 0.57f},
+    {256, 128, 6.5f, 0.69f}, {160, 256, 8.f, 0.8f},   {192, 256, 9.f, 0.85f}, {256, 256, 15.f, 1.f},
+};
+// `whole`: the output's rows are pieces of 8 or the product has no second operand.
+static RowsForm rows_form(int rows, int M, int N, int K, bool whole) {
+  RowsForm best = ROWS_64X64;
+  float price = 0.f;
+  for (int form = ROWS_64X64; form < ROWS_FORMS; ++form) {
+    const RowsPrice& p = ROWS_PRICES[form];
+    if (form > ROWS_128X128 && (M < p.bm || N < p.bn || !whole)) continue;
+    const long tiles = (long)((rows + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
+    const float us = (float)((tiles + 255) / 256) * (p.start + p.stage * ((K + BK - 1) / BK));
+    if (form == ROWS_64X64 || us < price) best = (RowsForm)form, price = us;
+  }
+  return best;
+}
+template <bool TAIL>
+__global__ __launch_bounds__(256) void gemm_rows_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, bf16_t* __restrict__ C,
+                                                        int M, int N, int K, const int* __restrict__ valid, FormTable forms, QkvTail tail) {
+  const FormOfRows chosen = form_of_rows(forms, valid, M);
+  const int Mv = chosen.rows, patched = chosen.patched;
+#define IRON_ROWS(FORM, MI, NT) \
+  case FORM: \
+    static_assert(ROWS_PRICES[FORM].bm == 32 * MI && ROWS_PRICES[FORM].bn == 32 * NT, "the tile that was priced"); \
+    gemm_big_body<BigTile<2, 2, MI, NT>, false, false, false, TAIL>(A, B, C, M, N, K, Mv, (M + 32 * MI - 1) / (32 * MI), (N + 32 * NT - 1) / (32 * NT), \
+                                                                    patched, GatedPair{}, tail); \
+    break
+  switch (chosen.form) {
+    IRON_ROWS(ROWS_160X128, 5, 4);
+    IRON_ROWS(ROWS_192X128, 6, 4);
+    IRON_ROWS(ROWS_256X128, 8, 4);
+    IRON_ROWS(ROWS_160X256, 5, 8);
+    IRON_ROWS(ROWS_192X256, 6, 8);
+    IRON_ROWS(ROWS_256X256, 8, 8);
+    case ROWS_128X128:
+      gemm_nt16_body<false>(A, B, C, M, N, K, Mv, (M + 127) / 128, (N + 127) / 128, patched, tail);
+      break;
+    case ROWS_128X64:
+      gemm_nt64_body<5, false, 4>(A, B, C, M, N, K, Mv, (M + 127) / 128, (N + 63) / 64, patched, tail);
+      break;
+    default:
+      gemm_nt64_body<8>(A, B, C, M, N, K, Mv, (M + 63) / 64, (N + 63) / 64, patched, tail);
+  }
+#undef IRON_ROWS
+}
+
+// The blocks of a launch whose forms are chosen by `forms`, up to the rows of `upto` each; sets the forms' orders.
+template <class Price, int FORMS>
+static int blocks_of_forms(const Price (&prices)[FORMS], const int (&upto)[FORMS], int N, FormTable& forms) {
+  int blocks = 1;
+  for (int form = 0; form < FORMS; ++form) {
+    // Tile rows rounded up to whole patches where that lets the XCD-aware order apply: the added
+    // tiles lie past the bound any block of that tiling runs for, and leave at once.
+    int tile_rows = (upto[form] + prices[form].bm - 1) / prices[form].bm;
+    const int tile_cols = (N + prices[form].bn - 1) / prices[form].bn, whole = (tile_rows + 7) & ~7;
     if (tile_rows >= 8 && !patched_order(tile_rows, tile_cols) && patched_order(whole, tile_cols)) tile_rows = whole;
-    return Tiling{tile_rows, tile_cols, patched_order(tile_rows, tile_cols)};
-  };
-  const Tiling t128 = tiling((rows128 + 127) / 128, n128), t64 = tiling((rows64 + 63) / 64, n64);
-  constexpr size_t lds256 = Tile256Four::LDS_BYTES;
-  constexpr size_t lds128 = (size_t)NT_STAGES * 256 * BK * 2;
-  constexpr size_t lds = BIG ? (lds256 > lds128 ? lds256 : lds128) : lds128;
-  static LdsOptIn opt_in;
-  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_either_kernel<BIG>), lds); e != hipSuccess) {
+    forms.patched |= (tile_rows >= 8 && patched_order(tile_rows, tile_cols)) << form;
+    if (tile_rows * tile_cols > blocks) blocks = tile_rows * tile_cols;
+  }
+  return blocks;
+}
+
+static int launch_gemm_rows(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, const int* valid, hipStream_t s,
+                            const QkvTail& tail = QkvTail{}) {
+  int upto[ROWS_FORMS] = {};
+  const bool whole = tail.residual == nullptr || N % 8 == 0;
+  FormTable forms = form_table(M, [&](int rows) { return (int)rows_form(valid == nullptr ? M : rows, M, N, K, whole); }, upto);
+  const int blocks = blocks_of_forms(ROWS_PRICES, upto, N, forms);
+  constexpr size_t lds = Tile256Four::LDS_BYTES;
+  static_assert(lds >= (size_t)NT_STAGES * 256 * BK * 2, "the other bodies' stages fit too");
+  static LdsOptIn opt_in[2];
+  const auto kernel = tail.residual != nullptr ? &gemm_rows_kernel<true> : &gemm_rows_kernel<false>;
+  if (hipError_t e = opt_in[tail.residual != nullptr].ensure(reinterpret_cast<const void*>(kernel), lds); e != hipSuccess) {
     set_error("gemm: %s", hipGetErrorString(e));
     return (int)e;
   }
-  int blocks = t128.tiles_m * t128.tiles_n;
-  if (t256.tiles_m * t256.tiles_n > blocks) blocks = t256.tiles_m * t256.tiles_n;
-  if (t64.tiles_m * t64.tiles_n > blocks) blocks = t64.tiles_m * t64.tiles_n;
-  hipLaunchKernelGGL((gemm_either_kernel<BIG>), dim3(blocks), dim3(256), lds, s, A, B, C, M, N, K, valid, t256, t128, t64,
-                     few256, few128, tail);
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), lds, s, A, B, C, M, N, K, valid, forms, tail);
   IRON_LAUNCH_CHECK();
 }
 
@@ -1892,7 +1981,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_kernel(const bf16_t* __restri
   const int splits = splitk_for(tile_rows, tiles_n, K), id = blockIdx.x;
   if (splits == 1) {   // whole K a block, the residual in its epilogue: iron_gemm_residual_bf16's 128 x 128 launch
     if (id < whole.tiles_m * whole.tiles_n)
-      gemm_nt16_body<false>(A, B, C, M, N, K, valid, whole.tiles_m, whole.tiles_n, whole.patched, tail);
+      gemm_nt16_body<false>(A, B, C, M, N, K, Mv, whole.tiles_m, whole.tiles_n, whole.patched, tail);
     return;
   }
   // The live (tile, slice) pairs are the first ids, so that they go out one a CU whatever the
@@ -1914,7 +2003,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_kernel(const bf16_t* __restri
   tail.k_begin = split * tail.k_len;
   tail.partial = partial + (size_t)split * splitk_slice_rows(splits, tiles_n) * N;
   tail.tile_plus1 = tile + 1;
-  gemm_nt16_body<false>(A, B, C, M, N, K, valid, (Mv + 127) / 128, tiles_n, 0, tail);
+  gemm_nt16_body<false>(A, B, C, M, N, K, Mv, (Mv + 127) / 128, tiles_n, 0, tail);
 }
 
 // The second launch: row `blockIdx.x` of C finished (from the slices, or as the first launch left
@@ -2036,7 +2125,7 @@ template <bool GROUPED = false>
 __device__ __forceinline__ void gemm_nt16_pair_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ Bg,
                                                     const bf16_t* __restrict__ Bu, bf16_t* __restrict__ G,
                                                     bf16_t* __restrict__ C, int M, int N, int K,
-                                                    const int* __restrict__ valid, int tiles_m, int tiles_n,
+                                                    int Mv, int tiles_m, int tiles_n,
                                                     int patched, int activation, const int* __restrict__ a_rows = nullptr) {
   constexpr int NT_BM = 128, NT_BN = 128;
   constexpr int PART = NT_BM * BK * 2;             // a 128 x 64 tile's 16 KB: A, then the gate's, then the up projection's
@@ -2045,7 +2134,6 @@ __device__ __forceinline__ void gemm_nt16_pair_body(const bf16_t* __restrict__ A
   constexpr int LOADS = 3 * INST;
   static_assert(BK == 64 && INST == 4, "two 32-wide k-steps a stage, twelve loads a wave");
   extern __shared__ __align__(16) char smem_nt[];
-  const int Mv = bound_or(valid, M);
 
   int tm = tiles_m, tn = tiles_n;
   if constexpr (!GROUPED) {
@@ -2220,34 +2308,8 @@ __device__ __forceinline__ void gemm_nt16_pair_body(const bf16_t* __restrict__ A
   leave(C);
 }
 
-// Which form a launch under a row bound takes: the price list's, read by the bound where it is known, on the device.  Four bits for each run of
-// 64 << shift rows (the words are chosen by tests: by an index they would be another trip to memory behind the bound's), and a bit for each
-// form whose tiles come in patches.
-struct FormTable {
-  uint64_t w[4];
-  int shift, patched;
-};
-__device__ __forceinline__ int form_of_rows(const FormTable& t, int rows) {
-  const int run = max(rows - 1, 0) >> (6 + t.shift);
-  const uint64_t w = run < 32 ? (run < 16 ? t.w[0] : t.w[1]) : (run < 48 ? t.w[2] : t.w[3]);
-  return (int)(w >> ((run & 15) * 4)) & 15;
-}
-// `best(rows)` for the most rows of every run up to M; `upto[form]`: the most rows a form is taken for.
-template <class Best>
-static FormTable form_table(int M, Best best, int* upto) {
-  FormTable t{};
-  while ((64L << t.shift) * 64 < M) ++t.shift;
-  const long run = 64L << t.shift;
-  for (long rows = run, i = 0; rows < M + run; rows += run, ++i) {
-    const int r = rows < M ? (int)rows : M, form = best(r);
-    t.w[i >> 4] |= (uint64_t)form << ((i & 15) * 4);
-    if (r > upto[form]) upto[form] = r;
-  }
-  return t;
-}
-
 // A gated feed-forward's two first projections over many rows as ONE launch, the tile chosen on the
-// device by the row bound as in gemm_either_kernel.  Tiles of BN / 2 columns of both weights: a wave's columns are half gate and half up projection, so
+// device by the row bound as in gemm_rows_kernel.  Tiles of BN / 2 columns of both weights: a wave's columns are half gate and half up projection, so
 // the gated product is made in its registers (64 rows: on the 64 x 64 tile's loop, two waves a product; 29 x 8192 x 2048 29.7 -> 20.5 us).
 // Which tile: by rounds of blocks over the CUs, as big_form, at what a round was measured to take with weights out of memory.  8192 columns over
 // K = 2048, us, by 64 x (32 + 32), 128 x (128 + 128) and 256 x (128 + 128) tiles alone and by these: 128 rows 27.9 / 25.9, 256 38.5 / 27.4, 384 39.6 /
@@ -2279,14 +2341,15 @@ __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __re
                                                               const bf16_t* __restrict__ Bu, bf16_t* __restrict__ G,
                                                               bf16_t* __restrict__ C, int M, int N, int K,
                                                               const int* __restrict__ valid, FormTable forms, int activation) {
-  const int form = form_of_rows(forms, bound_or(valid, M)), patched = forms.patched >> form & 1;
+  const FormOfRows chosen = form_of_rows(forms, valid, M);
+  const int Mv = chosen.rows, patched = chosen.patched;
   const GatedPair pair{Bu, G, activation};
 #define IRON_PAIR(FORM, MI, NT) \
   case FORM: \
     static_assert(PAIR_PRICES[FORM].bm == 32 * MI && PAIR_PRICES[FORM].bn == 16 * NT, "the tile that was priced"); \
-    gemm_big_body<BigTile<2, 2, MI, NT>, false, false, true>(A, Bg, C, M, N, K, valid, (M + 32 * MI - 1) / (32 * MI), N / (16 * NT), patched, pair); \
+    gemm_big_body<BigTile<2, 2, MI, NT>, false, false, true>(A, Bg, C, M, N, K, Mv, (M + 32 * MI - 1) / (32 * MI), N / (16 * NT), patched, pair); \
     break
-  switch (form) {
+  switch (chosen.form) {
     IRON_PAIR(PAIR_128X64, 4, 4);
     IRON_PAIR(PAIR_160X64, 5, 4);
     IRON_PAIR(PAIR_192X64, 6, 4);
@@ -2296,12 +2359,12 @@ __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __re
     IRON_PAIR(PAIR_224X128, 7, 8);
     IRON_PAIR(PAIR_256X128, 8, 8);
     case PAIR_EDGED:
-      gemm_nt16_pair_body(A, Bg, Bu, G, C, M, N, K, valid, (M + 127) / 128, (N + 127) / 128, patched, activation);
+      gemm_nt16_pair_body(A, Bg, Bu, G, C, M, N, K, Mv, (M + 127) / 128, (N + 127) / 128, patched, activation);
       break;
     default: {
       QkvTail gate{};
       gate.gated = activation;
-      gemm_nt64_body<8, true>(A, Bg, C, M, N, K, valid, (M + 63) / 64, (N + 31) / 32, patched, gate, Bu, G);
+      gemm_nt64_body<8, true>(A, Bg, C, M, N, K, Mv, (M + 63) / 64, (N + 31) / 32, patched, gate, Bu, G);
     }
   }
 #undef IRON_PAIR
@@ -2311,16 +2374,7 @@ static int launch_gemm_gated_pair(const bf16_t* A, const bf16_t* Bg, const bf16_
                                   int N, int K, const int* valid, int activation, hipStream_t s) {
   int upto[PAIR_FORMS] = {};   // each form's grid covers the rows it is chosen for
   FormTable forms = form_table(M, [&](int rows) { return (int)pair_form(valid == nullptr ? M : rows, M, N, K); }, upto);
-  int blocks = 1;
-  for (int form = 0; form < PAIR_FORMS; ++form) {
-    // Tile rows rounded up to whole patches where that lets the XCD-aware order apply: the added
-    // tiles lie past the bound any block of that tiling runs for, and leave at once.
-    int tile_rows = (upto[form] + PAIR_PRICES[form].bm - 1) / PAIR_PRICES[form].bm;
-    const int tile_cols = (N + PAIR_PRICES[form].bn - 1) / PAIR_PRICES[form].bn, whole = (tile_rows + 7) & ~7;
-    if (tile_rows >= 8 && !patched_order(tile_rows, tile_cols) && patched_order(whole, tile_cols)) tile_rows = whole;
-    forms.patched |= (tile_rows >= 8 && patched_order(tile_rows, tile_cols)) << form;
-    if (tile_rows * tile_cols > blocks) blocks = tile_rows * tile_cols;
-  }
+  const int blocks = blocks_of_forms(PAIR_PRICES, upto, N, forms);
   constexpr size_t lds = Tile256Four::LDS_BYTES;   // the largest tile's, more than the others'
   static_assert(lds >= (size_t)PAIR_STAGES * 3 * 128 * BK * 2 && lds >= (size_t)NT_STAGES * 256 * BK * 2, "the other bodies' stages fit too");
   static LdsOptIn opt_in;
@@ -2353,7 +2407,7 @@ __global__ __launch_bounds__(256) void gemm_grouped_pair_kernel(const bf16_t* __
                                                                 GroupedTiles g, const int* __restrict__ a_rows, int activation) {
   int tm, tn, e;
   if (!grouped_tile(g, (N + 127) / 128, tm, tn, e)) return;
-  gemm_nt16_pair_body<true>(A, Bg + (size_t)e * N * K, Bu + (size_t)e * N * K, nullptr, C, g.most * 128, N, K, nullptr, tm, tn, 0, activation, a_rows);
+  gemm_nt16_pair_body<true>(A, Bg + (size_t)e * N * K, Bu + (size_t)e * N * K, nullptr, C, g.most * 128, N, K, g.most * 128, tm, tn, 0, activation, a_rows);
 }
 __global__ __launch_bounds__(256) void gemm_grouped_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, bf16_t* __restrict__ C,
                                                            int N, int K, GroupedTiles g) {
@@ -2362,7 +2416,7 @@ __global__ __launch_bounds__(256) void gemm_grouped_kernel(const bf16_t* __restr
   if (!grouped_tile(g, tiles_n, tm, tn, e)) return;
   QkvTail tail{};
   tail.tile_plus1 = tm * tiles_n + tn + 1;
-  gemm_nt16_body<false>(A, B + (size_t)e * N * K, C, g.most * 128, N, K, nullptr, g.most, tiles_n, 0, tail);
+  gemm_nt16_body<false>(A, B + (size_t)e * N * K, C, g.most * 128, N, K, g.most * 128, g.most, tiles_n, 0, tail);
 }
 
 int launch_grouped_pair(const bf16_t* A, const bf16_t* Bg, const bf16_t* Bu, bf16_t* C, int N, int K, const GroupedTiles& g,
@@ -2413,7 +2467,7 @@ __global__ __launch_bounds__(256) void gemm_shared_kernel(const bf16_t* __restri
   int tm, tn;
   tile_of_block(tile, tiles_m, tiles_n, 0, tm, tn);
   tail.tile_plus1 = tm * tiles_n + tn + 1;
-  gemm_nt16_body<false, B_KN, C_NM, true>(A, B, C, M, N, K, nullptr, tiles_m, tiles_n, 0, tail);
+  gemm_nt16_body<false, B_KN, C_NM, true>(A, B, C, M, N, K, M, tiles_m, tiles_n, 0, tail);
 }
 
 // The shared tiles' sums added up in the order of k, eight columns a thread, eight blocks a tile.
@@ -2621,26 +2675,11 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
         return b_col_maj ? launch_gemm_big<false>(form, A, B, C, M, N, K, nullptr, s) : launch_gemm_big<true>(form, A, B, C, M, N, K, nullptr, s);
     }
     if (b_col_maj) {
-      if (valid != nullptr && M % BIG_BM == 0 && N % BIG_BN == 0 && (long)(M / BIG_BM) * (N / BIG_BN) >= (K % BK == 0 ? 192 : 144)) {
-        // Under a row bound read on the device the large tiles may cover too few rows to fill the
-        // chip (512 valid rows of 2048 leave 64 of 256 tiles): the blocks of one launch then choose
-        // the tile size where the bound is known, on the device.
-        const int tiles_n256 = N / BIG_BN, tiles_n128 = N / 128;
-        const int few256 = tiles_n256 >= 128 ? 0 : BIG_BM * (128 / tiles_n256);   // rows up to which 128x128 tiles win
-        const int few128 = tiles_n128 >= 128 ? 0 : 128 * (127 / tiles_n128);      // ... and 64x64 ones
-        if (few256 == 0 || few256 >= M) return launch_gemm_big<false>(BIG_256, A, B, C, M, N, K, valid, s);
-        return launch_gemm_either<true>(A, B, C, M, N, K, valid, s, few256, few128);
-      }
-      // 128x128 tiles that would occupy under half the CUs give way to 64x64 ones: always, where
-      // the shape says so; under a row bound, the blocks of one launch choose where the bound is
-      // known (the few-row 64x64 tiles run the eight-stage pipeline, a block a CU, so nothing is
-      // lost to the launch's 128 KB of LDS and the second, empty launch is saved).  So do tiles that
+      if (valid != nullptr) return launch_gemm_rows(A, B, C, M, N, K, valid, s);
+      // 128x128 tiles that would occupy under half the CUs give way to 64x64 ones, and so do tiles that
       // up to 64 rows would half fill at most (64 x 16384 x 8184: 93 -> 68 us).
-      const int tiles_n128 = (N + 127) / 128;
       if (tiles128 < 128 || M <= 64) return launch_gemm_nt<false, false, 1>(A, B, C, M, N, K, valid, s);
-      const int few = tiles_n128 >= 128 ? 0 : 128 * (127 / tiles_n128);   // rows up to which 64x64 tiles win
-      if (valid == nullptr || few == 0 || few >= M) return launch_gemm_nt<false>(A, B, C, M, N, K, valid, s);
-      return launch_gemm_either<false>(A, B, C, M, N, K, valid, s, 0, few);
+      return launch_gemm_nt<false>(A, B, C, M, N, K, valid, s);
     }
     return launch_gemm_nt<true>(A, B, C, M, N, K, valid, s);
   }
@@ -2700,13 +2739,7 @@ static int gemm_with_tail(const char* what, const uint16_t* A, const uint16_t* B
   IRON_REQUIRE((((uintptr_t)A | (uintptr_t)B | (uintptr_t)R | (uintptr_t)C) & 15) == 0,
                "%s: operands must be 16-byte aligned", what);
   hipStream_t s = (hipStream_t)stream;
-  // The tile sizes of iron_gemm_bf16's (N,K) path below the 256-wide ones.
-  const int tiles_n128 = (N + 127) / 128;
-  const long tiles128 = (long)((M + 127) / 128) * tiles_n128;
-  if (tiles128 < 128) return launch_gemm_nt<false, false, 1>(A, B, C, M, N, K, valid, s, tail);
-  const int few = tiles_n128 >= 128 ? 0 : 128 * (127 / tiles_n128);
-  if (valid == nullptr || few == 0 || few >= M) return launch_gemm_nt<false>(A, B, C, M, N, K, valid, s, tail);
-  return launch_gemm_either<false>(A, B, C, M, N, K, valid, s, 0, few, tail);
+  return launch_gemm_rows(A, B, C, M, N, K, valid, s, tail);
 }
 
 extern "C" int iron_gemm_residual_bf16(const uint16_t* A, const uint16_t* B, const uint16_t* R, uint16_t* C, int M,

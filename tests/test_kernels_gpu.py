@@ -374,6 +374,7 @@ def test_gemm_rows_of_every_alignment(cuda, M, Kdim, N, b_col_maj, c_col_maj, co
 
 
 @pytest.mark.parametrize("M,Kdim,N,b_col_maj,bounds", [
+    (2000, 136, 8195, True, (130, 257, 513, 641, 769, 1025, 1281, 1537, 1999)),   # every form by the bound, the last tiles moved back
     (2048, 200, 8192, True, (1, 128, 129, 1024, 1025, 2047)),    # 64, 128 and 256 tiles by the bound
     (1500, 328, 2056, True, (63, 895, 896, 897, 1500)),          # 64 and 128 ones, ragged
     (256, 136, 320, True, (0, 100, 200)), (40, 1000, 4168, True, (17, 40)), (33, 4096, 520, True, (1, 32)),   # 64 ones whatever the bound
@@ -520,7 +521,9 @@ def test_prefill_qkv_writes_k_and_v_into_the_cache_rows(cuda, rows, bound, start
 
 @pytest.mark.parametrize("M,Kdim,N,rows,scale", [(2048, 512, 2048, None, 1.0), (2048, 256, 2048, 512, 1.0),
                                                  (2048, 256, 2048, 1500, 0.22), (256, 128, 512, 100, 1.0),
-                                                 (128, 64, 64, None, -0.5), (4096, 192, 1024, 3000, 1.0)])
+                                                 (128, 64, 64, None, -0.5), (4096, 192, 1024, 3000, 1.0),
+                                                 # tiles of 128, 160, 192 and 256 rows and columns, the last moved back over its neighbour
+                                                 *[(2000, 128, 8200, rows, 1.0) for rows in (200, 641, 769, 1025, 1281, 1537, 2000, None)]])
 def test_gemm_residual_epilogue(cuda, M, Kdim, N, rows, scale):
     """A projection over many rows with its residual in the epilogue: the product rounded as the
     separate step would store it, then one fused multiply-add with the residual (the sum, or AXPY)."""
