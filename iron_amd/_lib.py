@@ -7,6 +7,7 @@ raises, and every operator call goes through here.
 from __future__ import annotations
 
 import ctypes
+import functools
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p
 from pathlib import Path
 
@@ -178,6 +179,21 @@ def lib() -> ctypes.CDLL:
             fn.restype, fn.argtypes = restype, argtypes
         _lib = handle
     return _lib
+
+
+@functools.lru_cache(maxsize=None)
+def native():
+    """``_calls``, which checks and launches the plain case of an operator in one native call, on the entry points of
+    ``lib()``; its functions return the entry point's code, or None for what is not that case.  A caller to whom
+    that is not 0 goes the long way, which does the work or raises."""
+    if not (LIB_PATH.parent / "_calls.so").exists():
+        raise IronHipError(f"{LIB_PATH.parent / '_calls.so'} is missing: build it with `python -m iron_amd.build`")
+    lib()
+    from . import _calls
+
+    _calls.bind(*(ctypes.cast(getattr(_lib, name), c_void_p).value for name in (
+        "iron_gemm_bf16", "iron_gemm_workspace_bytes", "iron_gemm_shared_bf16", "iron_gemv_bf16_tuned", "iron_mha_prefill_bf16")))
+    return _calls
 
 
 def check(code: int, what: str) -> None:

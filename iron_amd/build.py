@@ -1,4 +1,4 @@
-"""Build ``libiron_hip.so``: every HIP source of ``csrc/`` compiled for gfx950.
+"""Build ``libiron_hip.so``: every HIP source of ``csrc/`` compiled for gfx950; and ``_calls.so``, its host calls' shortcut.
 
 ``python -m iron_amd.build`` or ``build()``; hipcc cross-compiles without a GPU.
 The library is written beside this file so it travels with the source tree.
@@ -10,12 +10,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 LIB = HERE / "libiron_hip.so"
+CALLS = HERE / "_calls.so"
 ARCH = "gfx950"
 # -packed-fp32-ops off: the compiler is not to form v_pk_*_f32 from float code.
 FLAGS = [
@@ -59,6 +61,21 @@ def _run(cmd: list[str]) -> None:
         print(err, file=sys.stderr)
 
 
+def _build_calls(objdir: Path) -> None:
+    """The Python module of ``calls.cpp``: host code over torch's tensors, no kernel."""
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    libs = Path(torch.__file__).parent / "lib"
+    flags = ["-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    dirs = [*include_paths(), str(Path(_hipcc()).resolve().parent.parent / "include"), sysconfig.get_paths()["include"]]
+    part = objdir / CALLS.name
+    _run(["g++", *flags, *(f"-isystem{d}" for d in dirs), str(CSRC / "calls.cpp"), "-o", str(part), f"-L{libs}",
+          "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"])
+    os.replace(part, CALLS)
+
+
 def build(verbose: bool = False) -> Path:
     """Compile every source and link the shared library; always recompiles."""
     hipcc = _hipcc()
@@ -69,13 +86,15 @@ def build(verbose: bool = False) -> Path:
 
     def compile_one(pair):
         src, obj = pair
+        if src is None:
+            return _build_calls(objdir)
         if verbose:
             print(f"hipcc {src.name}")
         _run([hipcc, *FLAGS, "-c", str(src), "-o", str(obj)])
 
     jobs = min(len(srcs), int(os.environ.get("MAX_JOBS", "8")))
     with ThreadPoolExecutor(max_workers=jobs) as pool:
-        list(pool.map(compile_one, zip(srcs, objs)))
+        list(pool.map(compile_one, [(None, CALLS), *zip(srcs, objs)]))
     # Linked beside its place and moved there whole: a build that is cut short leaves no half library.
     part = objdir / LIB.name
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(part), *map(str, objs)])

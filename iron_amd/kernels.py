@@ -13,7 +13,7 @@ import math
 
 import torch
 
-from ._lib import check, current_stream, lib, ptr
+from ._lib import check, current_stream, lib, native, ptr
 
 BF16 = torch.bfloat16
 GATES = {"silu": 1, "gelu_tanh": 2, "relu": 3}   # a gated feed-forward's activation, by the C ABI's number
@@ -54,6 +54,10 @@ def _gemm_workspace(M, N, K, b_col_maj, c_col_maj) -> int:
 
 
 def gemm(A, B, C, *, M, N, K, b_col_maj=False, c_col_maj=False, valid=None, valid_k=None):
+    if valid is None and valid_k is None:
+        code = native().gemm(A, B, C, M, N, K, b_col_maj, c_col_maj)
+        if code == 0:
+            return
     _numel(_dev(A, "A"), M * K, "A")
     _numel(_dev(B, "B"), K * N, "B")
     _numel(_dev(C, "C"), M * N, "C")
@@ -74,6 +78,8 @@ def gemm(A, B, C, *, M, N, K, b_col_maj=False, c_col_maj=False, valid=None, vali
 
 
 def gemv(W, x, y, *, M, K, batches=1, repeat=1, valid=None, rows_per_wave=0, k_split=0):
+    if batches == 1 and repeat == 1 and valid is None and rows_per_wave == 0 and k_split == 0 and native().gemv(W, x, y, M, K) == 0:
+        return
     _numel(_dev(W, "A"), (batches // repeat) * M * K, "A")
     _numel(_dev(x, "B"), batches * K, "B")
     _numel(_dev(y, "C"), batches * M, "C")
@@ -391,6 +397,11 @@ def mha_prefill(
     least; ``kv_interleaved``) of which the ``kv_len`` from row ``*kv_first`` on are the keys."""
     seq_len = seq if seq_len is None else seq_len
     scale = 1.0 / math.sqrt(d) if scale is None else scale
+    if valid is None and kv_valid is None and kv_first is None:
+        code = native().mha_prefill(Q, K, V, O, scale, heads, kv_heads, d, seq, seq_len, kv_len, causal, -1 if window is None else window,
+                                    q_interleaved, kv_interleaved)
+        if code == 0:
+            return
     _numel(_dev(Q, "Q"), seq * heads * d, "Q")
     _numel(_dev(O, "O"), seq * heads * d, "O")
     if kv_first is not None:

@@ -4,6 +4,8 @@ import ctypes
 import re
 from pathlib import Path
 
+import pytest
+
 from iron_amd import _lib
 
 ROOT = Path(__file__).resolve().parent.parent
@@ -72,3 +74,23 @@ def test_bench_refuses_more_than_one_gpu():
     bench = Path(__file__).resolve().parent.parent / "bench.py"
     done = subprocess.run([sys.executable, str(bench), "--gpus", "2"], capture_output=True, text=True, timeout=120)
     assert done.returncode != 0 and "one-GPU" in done.stderr and done.stdout.strip() == ""
+
+
+def test_native_calls_leave_what_is_not_plain_to_the_caller():
+    """The one-call shortcut answers None, and raises nothing, for tensors off the GPU, other types of number and of argument, and
+    counts past 32 bits; the operators' own words are then what a caller reads."""
+    import torch
+
+    from iron_amd import kernels as K
+    from iron_amd._lib import native
+
+    a = torch.zeros(8, 8, dtype=torch.bfloat16)
+    for args in ((a, a, a, 8, 8, 8, True, False), (None, a, a, 8, 8, 8, 0, 0), (a, a, a, 8.0, 8, 8, 0, 0), (a, a, a, 1 << 40, 8, 8, 0, 0),
+                 (a, a, a, 8, 8, 8, "x", 0), (a, a, a, 8, 8)):
+        assert native().gemm(*args) is None
+    assert native().gemv(a, a, a, 8, 8) is None and native().gemv(a) is None
+    assert native().mha_prefill(a, a, a, a, 1.0, 1, 1, 64, -8, 8, 8, 1, -1, 0, 0) is None and native().mha_prefill(a) is None
+    with pytest.raises(TypeError, match="A: expected a tensor on the GPU"):
+        K.gemm(a, a, a, M=8, N=8, K=8)
+    with pytest.raises(TypeError, match="expected a torch tensor"):
+        K.gemv([1.0], a, a, M=8, K=8)

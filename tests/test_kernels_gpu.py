@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 import torch
 
-from iron_amd import kernels as K
+from iron_amd import _lib, kernels as K
 from iron_amd.bf16 import from_torch, round_bf16, to_torch
 from oracle import ops
 
@@ -98,6 +98,32 @@ def test_gemm_layouts(cuda, b_col_maj, c_col_maj):
     # And by the reference's own bound: 2 units of 2^-8 |A|@|B| (gemm.py:704-735).
     bound = ops.gemm_bound(A, B, b_col_maj=b_col_maj, c_col_maj=c_col_maj)
     assert np.all(np.abs(from_torch(C) - want) <= bound)
+
+
+def test_native_calls_refuse_what_the_long_way_refuses_and_follow_the_stream(cuda):
+    """What the one-call shortcut is not for -- another dtype, strides, count, a refused size -- raises as the long way does; a call inside a
+    stream's block runs on that stream, behind what was queued there."""
+    x = torch.zeros(64, 64, dtype=torch.bfloat16, device=cuda)
+    for bad, error in ((x.float(), TypeError), (x.t()[:, :32], ValueError), (x[:32], ValueError), (torch.zeros(64, 64, dtype=torch.bfloat16), TypeError)):
+        with pytest.raises(error):
+            K.gemm(x, bad, x.clone(), M=64, N=64, K=64)
+        with pytest.raises(error):
+            K.mha_prefill(x, bad, x, x.clone(), heads=1, kv_heads=1, d=64, seq=64, kv_len=64)
+    with pytest.raises(_lib.IronHipError, match="iron_gemm_bf16 refused.*multiple of 8"):
+        K.gemm(x.view(-1)[: 64 * 63], x.view(-1)[: 64 * 63], x.clone(), M=64, N=64, K=63)
+    with pytest.raises(_lib.IronHipError, match="refused"):
+        K.gemv(x.view(-1)[: 64 * 63], x.view(-1)[:63], x.view(-1)[:64].clone(), M=64, K=63)
+    big, one, side = torch.randn(4096, 4096, device=cuda), torch.ones(64, 64, dtype=torch.bfloat16, device=cuda), torch.cuda.Stream()
+    y = torch.empty_like(x)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(8):
+            big = big @ big * 1e-3
+        late = one + big[0, 0].to(torch.bfloat16) * 0
+        K.gemm(late, one, y, M=64, N=64, K=64)
+        out = y.clone()
+    side.synchronize()
+    assert bool((out == 64).all())
 
 
 @pytest.mark.parametrize("b_col_maj", [False, True])
