@@ -34,6 +34,13 @@ constexpr int BKV = 64;   // key rows per tile
 constexpr float kLazyBits = 8.f;        // how far a maximum may run ahead of the reference the exponents are taken against
 constexpr float kSumLow = 0x1p-60f, kSumHigh = 0x1p24f;   // a tile's sum of exponentials outside this range: take its maximum and redo it
 constexpr int kCUs = 256;                // compute units the block orders below assume
+// Which 16-byte chunk of a key's (value's) row in LDS holds its first one: the others are XORed by it.  A row of 64 elements is half the banks, so sixteen
+// rows' fragments at one chunk, and four rows' at four, meet no bank twice by these; a row of 128 is all of them and takes the row itself
+// (with the narrow rows' swizzle its reads took every bank twice: 32 heads of 128, 3001 queries 100.3 -> 94.6 us, 8192 542 -> 523).
+template <int D>
+__device__ __forceinline__ int k_swizzle(int row) { return D == 64 ? (row >> 1) & 7 : row & 15; }
+template <int D>
+__device__ __forceinline__ int v_swizzle(int row) { return (row & 3) << (D == 64 ? 1 : 2); }
 // Whether `groups` blocks of 32 queries and a head, the keys dealt over a block's waves (prefill_few_rows), take the place of a launch's
 // blocks of 32 W queries.  Each of them reads all the keys, so it pays while the chip has CUs for them (at d = 64 with eight waves, where
 // a CU holds two blocks, twice as many), and from a few tiles a wave on.  us, 32 / 8 heads, tiles against few rows: 40 queries, d = 64, 512 / 2048 / 12043
@@ -82,18 +89,18 @@ __device__ __forceinline__ void prefill_few_rows(
       const_cast<bf16_t*>(Kh + (long)kv_lo * kv_row_stride), 0, reach, 0x00020000);
   const __amdgpu_buffer_rsrc_t v_rows = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<bf16_t*>(Vh + (long)kv_lo * kv_row_stride), 0, reach, 0x00020000);
-  // Load i covers tile rows i RPI + l; chunks swizzled as below.  A row starts on a multiple of its head's bytes, so the part of K's
+  // Load i covers tile rows i RPI + l.  A row starts on a multiple of its head's bytes, so the part of K's
   // swizzle that is the load's own is an XOR of the lane's offset.
   static_assert(RPI % 4 == 0, "V's swizzle, 2 (row % 4), is the lane's alone");
   const int l = lane / CPR;
-  const int k_lane = l * row_bytes + (((lane % CPR) ^ (l >> 1)) << 4), v_lane = l * row_bytes + (((lane % CPR) ^ ((l & 3) << 1)) << 4);
+  const int k_lane = l * row_bytes + (((lane % CPR) ^ k_swizzle<D>(l)) << 4), v_lane = l * row_bytes + (((lane % CPR) ^ v_swizzle<D>(l)) << 4);
   char* stage = smem + wave * (2 * TILE);   // the wave's K tile, then its V tile
   auto issue = [&](int step) {
     const int at = (wave + step * NW) * TK * row_bytes;
 #pragma unroll
     for (int i = 0; i < VINST; ++i) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(k_rows, IRON_LDS_PTR(stage + i * 1024), 16,
-                                               (int)(k_lane ^ ((i * RPI / 2 & 7) << 4)) + at + i * RPI * row_bytes, 0, 0, 0);
+                                               (int)(k_lane ^ (k_swizzle<D>(i * RPI) << 4)) + at + i * RPI * row_bytes, 0, 0, 0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(v_rows, IRON_LDS_PTR(stage + TILE + i * 1024), 16,
                                                (int)v_lane + at + i * RPI * row_bytes, 0, 0, 0);
     }
@@ -107,7 +114,7 @@ __device__ __forceinline__ void prefill_few_rows(
     if (q_live) v = *reinterpret_cast<const uint4*>(Qh + (size_t)my_q * q_row_stride + 8 * g + 16 * s);
     qf[s] = __builtin_bit_cast(bf16x8, v);
   }
-  const int v_key = 4 * g + ((lane & 15) >> 2), v_swz = ((lane >> 2) & 3) << 1;
+  const int v_key = 4 * g + ((lane & 15) >> 2), v_swz = v_swizzle<D>(lane >> 2);
   unsigned v_frag[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) {
@@ -129,7 +136,7 @@ __device__ __forceinline__ void prefill_few_rows(
   float m_run = -INFINITY, l_run = 0.f;
 
   const unsigned k_frag = (unsigned)(size_t)IRON_LDS_PTR(stage) + col * ROWB;
-  const int k_swz = (col >> 1) & 7;
+  const int k_swz = k_swizzle<D>(col);
   for (int step = 0; step < steps; ++step) {
     const int kv0 = kv_lo + (wave + step * NW) * TK;
     wait_vmcnt<0>();   // the wave's own tiles: nobody else's wait, no barrier
@@ -244,8 +251,8 @@ __device__ __forceinline__ void prefill_few_rows(
 
 // K and V tiles go straight from global memory into LDS (buffer loads with the LDS bit, no register staging), as
 // stored: [64 keys][D], STAGES tiles deep.  16-byte chunks of a row are XOR-swizzled so unpadded
-// rows read without bank conflicts: K by (key >> 1) & 7 for its 16-byte fragment reads, V by
-// 2 * (key & 3) for the transposing reads (ds_read_b64_tr_b16) that deliver V^T fragments.  A bare
+// rows read without bank conflicts: K by k_swizzle for its 16-byte fragment reads, V by
+// v_swizzle for the transposing reads (ds_read_b64_tr_b16) that deliver V^T fragments.  A bare
 // s_barrier and counted s_waitcnt vmcnt keep the younger tiles' loads in flight across the barrier.
 //
 // At least two waves a SIMD caps the register budget at 256, which makes the compiler keep MFMA
@@ -398,8 +405,8 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
     for (int i = 0; i < INST; ++i) {
       const int r = (wave * INST + i) * RPI + l_row;
-      k_voff[i] = r * row_bytes + (l_pch ^ ((r >> 1) & 7)) * 16;
-      v_voff[i] = r * row_bytes + (l_pch ^ ((r & 3) << 1)) * 16;
+      k_voff[i] = r * row_bytes + (l_pch ^ k_swizzle<D>(r)) * 16;
+      v_voff[i] = r * row_bytes + (l_pch ^ v_swizzle<D>(r)) * 16;
     }
     // The keys (and values) of the head that this block can see, from row kv_lo's start to the
     // last key's row end, are one buffer for the whole loop; a tile's place in it goes into the
@@ -427,12 +434,12 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
     for (int s = 0; s < STAGES - 1; ++s) issue(min(s * SPLIT + half, ntiles - 1), s);
 
     // Fragment addressing.  K (A operand of S^T): lane reads key t*32 + col, chunk 2s + g.
-    const int k_frag = col * ROWB, k_swz = (col >> 1) & 7;
+    const int k_frag = col * ROWB, k_swz = k_swizzle<D>(col);
     // V^T (A operand of O^T): for (t, h) a lane group g needs keys 32t + 16h + 4g + 0..3 (low
     // half of its k slots) and the same + 8 (high half) of column d = 32 dt + col.  In the
     // transposing read a lane points at 4 consecutive d of the key row 4g + (lane & 15) / 4 ...
     const int v_key = 4 * g + ((lane & 15) >> 2);
-    const int v_swz = ((lane >> 2) & 3) << 1;           // 2 * (key & 3), the same for every (t, h)
+    const int v_swz = v_swizzle<D>(lane >> 2);           // the same for every (t, h)
     int v_frag[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
