@@ -50,7 +50,11 @@ template <int D, int W>
 __host__ __device__ __forceinline__ bool few_rows_pay(int groups, int keys) { return groups <= (D == 64 && W == 4 ? 512 : 256) && keys >= 512; }
 constexpr int kFewBlocks = 512;          // launches of fewer blocks than this halve their blocks' queries (S = 1024 at 32 heads: 18.5 -> 13.9 us)
 constexpr int kWideBigBlocks = 512;     // wide heads: launches of at least this many 128-query blocks keep that size
-constexpr int kSplitMaxBlocks = 1024;   // launches of up to this many blocks split each block's tiles over two halves
+// Launches of up to this many blocks split each block's tiles over two halves of eight waves, which halves a block's chain of tiles; more fill the chip better
+// four waves each.  64-wide heads (two eight-wave blocks share a CU): S = 8192 at 32 heads 365 -> 353-360 us split, S = 16384 not.  128-wide ones (two
+// four-wave blocks, which read a tile's keys ahead): 32 heads, split against not, 2048 queries 45.4 / 52.4, 2305 63.6 / 59.8, 3001 90.4 / 81.8, 4096
+// 147 / 135, a window of 1024 of those 90 / 76; 24 heads, 3000 74.4 / 73.4; 16 heads, 5000 120 / 122, 6000 159 / 155.
+constexpr int kSplitMaxBlocks64 = 4096, kSplitMaxBlocks128 = 560;
 
 // Few live queries over many keys (a turn late in a conversation: 40 rows of a 2048-row launch, 12 000 keys): by the
 // tiles below, a block a head and 128 queries, most of the chip would idle behind a block's chain
@@ -281,6 +285,11 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
   constexpr int DT = D / 32;             // 32-row tiles of O^T
   constexpr int CPR = D / 8;             // 16-byte chunks a row has
   constexpr int STAGES = D == 64 && SPLIT == 1 ? 3 : 2;
+  // 128-wide heads by four waves: a tile's K fragments are read under the softmax of the tile before, and a tile's loads have a whole step to land (one
+  // barrier a step as without; 8192 queries 521 -> 501 us, and it makes this form the faster one from 560 blocks on).  Not with eight waves, one block
+  // a CU, where the 32 more registers bought nothing (3001 queries 93.9 / 95.2; halves half a step apart, one's products under the
+  // other's softmax, 102), nor with 64-wide heads, whose four waves a SIMD cover the reads.
+  constexpr bool PIPED = D == 128 && SPLIT == 1;
   constexpr int TILE = BKV * ROWB;       // bytes of a K (or V) tile
   constexpr int STAGE = 2 * TILE;
   constexpr int BQW = 32 * W;            // query rows of this block
@@ -417,21 +426,35 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
     const __amdgpu_buffer_rsrc_t v_rows = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<bf16_t*>(Vh + (long)kv_lo * kv_row_stride), 0, reach, 0x00020000);
     const int tile_bytes = BKV * row_bytes;
-    auto issue = [&](int tile, int buf) {
+    auto issue_k = [&](int tile, int buf) {
       char* st = smem + buf * STAGE;
       const int at = tile * tile_bytes;
 #pragma unroll
-      for (int i = 0; i < INST; ++i) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(k_rows, IRON_LDS_PTR(st + (wave * INST + i) * 1024), 16,
-                                                 (int)k_voff[i] + at, 0, 0, 0);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(v_rows, IRON_LDS_PTR(st + TILE + (wave * INST + i) * 1024), 16,
-                                                 (int)v_voff[i] + at, 0, 0, 0);
-      }
+      for (int i = 0; i < INST; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(k_rows, IRON_LDS_PTR(st + (wave * INST + i) * 1024), 16, (int)k_voff[i] + at, 0, 0, 0);
     };
+    auto issue_v = [&](int tile, int buf) {
+      char* st = smem + buf * STAGE;
+      const int at = tile * tile_bytes;
+#pragma unroll
+      for (int i = 0; i < INST; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(v_rows, IRON_LDS_PTR(st + TILE + (wave * INST + i) * 1024), 16, (int)v_voff[i] + at, 0, 0, 0);
+    };
+    auto issue = [&](int tile, int buf) {
+      issue_k(tile, buf);
+      issue_v(tile, buf);
+    };
+    auto tile_of = [&](int step) { return min(step * SPLIT + half, ntiles - 1); };
     // Always STAGES-1 tiles in flight before the loop and one more each iteration (past the end
     // the last tile again, into a buffer nobody reads), so the wait counts below are exact.
+    if constexpr (PIPED) {
+      issue_k(tile_of(0), 0);
+      issue_v(tile_of(0), 0);
+      issue_k(tile_of(1), 1);
+    } else {
 #pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s) issue(min(s * SPLIT + half, ntiles - 1), s);
+      for (int s = 0; s < STAGES - 1; ++s) issue(tile_of(s), s);
+    }
 
     // Fragment addressing.  K (A operand of S^T): lane reads key t*32 + col, chunk 2s + g.
     const int k_frag = col * ROWB, k_swz = k_swizzle<D>(col);
@@ -456,46 +479,29 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
     const unsigned see_span = see_hi >= see_lo ? (unsigned)(see_hi - see_lo) : 0u;
     if (see_hi < see_lo) see_lo = 1 << 30;
 
-    // A step of the loop on stage buffer `buf`.
-    auto tile_step = [&](int step, const int buf) {
-      const int ahead_buf = (buf + STAGES - 1) % STAGES;
-      const int tile = step * SPLIT + half;
-      const int kv0 = kv_lo + tile * BKV;
-      wait_vmcnt<(STAGES - 2) * 2 * INST>();   // this wave's share of the tile has landed
-      block_barrier();                          // everyone's has; everyone is done with the step before
-      if constexpr (SPLIT > 1) {
-        if (tile >= ntiles) {   // past this half's last tile: keep the loads (and the wait counts) going
-          issue(ntiles - 1, ahead_buf);
-          return;
-        }
+    // A tile's K fragments, a 32-key half's all requested together (one wait, not one a fragment).
+    auto k_half = [&](int buf, int t, bf16x8 (&kf)[KS]) {
+      const char* kt = smem + buf * STAGE + t * 32 * ROWB;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) kf[s] = *reinterpret_cast<const bf16x8*>(kt + k_frag + (((2 * s + g) ^ k_swz) << 4));
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // S^T = K Q^T for the two 32-key halves of the tile.
+    auto scores = [&](const bf16x8 (&kf)[2][KS], f32x16 (&sacc)[2]) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sacc[t][e] = 0.f;
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+          sacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[t][s], qf[s], sacc[t], 0, 0, 0);
       }
+    };
+    // The softmax and O^T += V^T P^T of a tile on stage buffer `buf`.
+    auto rest = [&](int tile, int buf, f32x16 (&sacc)[2]) __attribute__((always_inline)) {
+      const int kv0 = kv_lo + tile * BKV;
+      const unsigned vt = lds_base + buf * STAGE + TILE;
       {
-        const char* kt = smem + buf * STAGE;
-        const unsigned vt = lds_base + buf * STAGE + TILE;
-        // S^T = K Q^T for the two 32-key halves of the tile.
-        f32x16 sacc[2];
-        // A half's K fragments are all requested before its MFMAs (one wait, not one a fragment),
-        // and the second half's while the first half's MFMAs run.
-        bf16x8 kf[2][KS];
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
-          kf[0][s] = *reinterpret_cast<const bf16x8*>(kt + k_frag + (((2 * s + g) ^ k_swz) << 4));
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
-          kf[1][s] = *reinterpret_cast<const bf16x8*>(kt + 32 * ROWB + k_frag + (((2 * s + g) ^ k_swz) << 4));
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-#pragma unroll
-          for (int e = 0; e < 16; ++e) sacc[t][e] = 0.f;
-#pragma unroll
-          for (int s = 0; s < KS; ++s)
-            sacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[t][s], qf[s], sacc[t], 0, 0, 0);
-        }
-        // The prefetch goes out while the score MFMAs run (its buffer, tile - 1's, is free since
-        // the barrier above).
-        issue(min(tile + (STAGES - 1) * SPLIT, ntiles - 1), ahead_buf);
         // Only tiles that touch a bound or the mask's edge pay for masking.  Element e of half t
         // is key kv0 + 32 t + 8 (e/4) + 4 g + e%4, query `col`.
         bool edge = kv0 + BKV > kv_tokens;
@@ -591,7 +597,50 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
         pv_half(std::integral_constant<int, 1>{});
       }
     };
-    if constexpr (SPLIT > 1) {
+    // A step of the loop on stage buffer `buf`.
+    auto tile_step = [&](int step, const int buf) {
+      const int ahead_buf = (buf + STAGES - 1) % STAGES;
+      const int tile = step * SPLIT + half;
+      wait_vmcnt<(STAGES - 2) * 2 * INST>();   // this wave's share of the tile has landed
+      block_barrier();                          // everyone's has; everyone is done with the step before
+      if constexpr (SPLIT > 1) {
+        if (tile >= ntiles) {   // past this half's last tile: keep the loads (and the wait counts) going
+          issue(ntiles - 1, ahead_buf);
+          return;
+        }
+      }
+      bf16x8 kf[2][KS];
+      f32x16 sacc[2];
+      k_half(buf, 0, kf[0]);
+      k_half(buf, 1, kf[1]);   // (while the first half's MFMAs run)
+      scores(kf, sacc);
+      // The prefetch goes out while the score MFMAs run (its buffer, tile - 1's, is free since
+      // the barrier above).
+      issue(tile_of(step + STAGES - 1), ahead_buf);
+      rest(tile, buf, sacc);
+    };
+    if constexpr (PIPED) {
+      bf16x8 kf[2][KS];
+      wait_vmcnt<2 * INST>();   // the first tile's keys have landed
+      block_barrier();
+      k_half(0, 0, kf[0]);
+      k_half(0, 1, kf[1]);
+      auto piped_step = [&](int step, const int buf) {
+        f32x16 sacc[2];
+        scores(kf, sacc);
+        wait_vmcnt<0>();   // this tile's values and the next one's keys: sent for a step ago
+        block_barrier();   // everyone's have landed; everyone has this tile's keys in registers and is done with the values before
+        k_half(buf ^ 1, 0, kf[0]);
+        k_half(buf ^ 1, 1, kf[1]);
+        issue_k(tile_of(step + 2), buf);
+        issue_v(tile_of(step + 1), buf ^ 1);
+        if (step < ntiles) rest(step, buf, sacc);
+      };
+      for (int step = 0; step < steps; step += 2) {
+        piped_step(step, 0);
+        piped_step(step + 1, 1);
+      }
+    } else if constexpr (SPLIT > 1) {
       // Few, long blocks (a short sequence): the loop unrolled over the stage buffers, so that a
       // fragment's place in its stage is an immediate of the read and the buffer arithmetic goes
       // (S = 2048: 3.5 % faster).  Where a CU holds several blocks at different places of the loop
@@ -1056,9 +1105,8 @@ static int mha_prefill(const uint16_t* Q, const uint16_t* K, const uint16_t* V, 
   const float scale_log2 = scale * 1.4426950408889634f;
   const int blocks = ((seq + BQ - 1) / BQ) * heads;
   // Few blocks (a short sequence): the longest block's chain of tiles bounds the launch, so its
-  // tiles are split over two halves of eight waves.  Many blocks fill the chip better four waves each
-  // (at d = 64, where two eight-wave blocks share a CU, only from S = 16384 at 32 heads on: S = 8192 365 -> 353-360 us).
-  const bool split = blocks <= (d == 64 ? 4 * kSplitMaxBlocks : kSplitMaxBlocks);
+  // tiles are split over two halves of eight waves.  Many blocks fill the chip better four waves each.
+  const bool split = blocks <= (d == 64 ? kSplitMaxBlocks64 : kSplitMaxBlocks128);
   PrefillArgs a{Q, K, V, O, heads, heads / kv_heads, seq, seq_len, kv_len, scale_log2, causal, window,
                 q_row, q_head, kv_row, kv_head, valid, kv_valid, kv_first, kv_rows};
   int rc;

@@ -1041,7 +1041,11 @@ def test_mha_prefill_of_few_rows_over_many_keys(cuda, H, G, d, S, rows, L, keys,
 @pytest.mark.parametrize("H,G,S,rows,L,keys,window,causal", [
     (32, 8, 256, 256, 1000, 1000, None, True), (32, 8, 256, 230, 2500, 2100, None, True), (32, 8, 200, 200, 1600, 1600, None, False),
     (32, 8, 257, 257, 1600, 1600, None, True), (32, 8, 300, 270, 2000, 400, None, True),
-    (32, 8, 700, 700, 700, 700, None, True), (32, 8, 640, 640, 1700, 1700, None, True), (8, 2, 2200, 2200, 2200, 2200, 1500, True)])
+    (32, 8, 700, 700, 700, 700, None, True), (32, 8, 640, 640, 1700, 1700, None, True), (8, 2, 2200, 2200, 2200, 2200, 1500, True),
+    # many blocks of four waves, keys read a tile ahead: one key, one tile, two, three of them, a window, no mask, rows past the bounds
+    (576, 64, 1, 1, 1, 1, None, True), (576, 64, 64, 64, 64, 64, None, False), (576, 64, 65, 65, 65, 65, None, True),
+    (256, 64, 300, 300, 300, 300, None, True), (288, 32, 129, 129, 190, 190, None, False), (288, 32, 129, 129, 700, 700, 200, True),
+    (288, 32, 200, 131, 500, 400, None, True)])
 def test_mha_prefill_128_wide_heads_at_the_lines_between_the_forms(cuda, H, G, S, rows, L, keys, window, causal):
     test_mha_prefill_of_few_rows_over_many_keys(cuda, H, G, 128, S, rows, L, keys, window, causal)
 
