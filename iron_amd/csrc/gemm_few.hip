@@ -44,10 +44,11 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
                                                                        bf16_t* __restrict__ C, int M, int N, int K) {
   typedef Strips<MT, MA, SINGLE, STAGES> S;
   constexpr int W = STRIP_WAVES, R = STRIP_ROWS, GROUP = STRIP_OUT / R;   // GROUP: tiles whose columns are stored together
+  static_assert(STAGES <= 2, "the last item's wait is for all that is out");
   constexpr int NOWHERE = 0x7ffffff0;   // an offset past the end of every run of rows (64 rows of at most 2^22, the entry point's bound, are 2^29 bytes)
   extern __shared__ __align__(1024) char lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l16 = lane & 15, quad = lane >> 4;
-  const int strips = (K + STRIP - 1) / STRIP, mine = SINGLE ? 1 : (strips - wave + W - 1) / W, most = SINGLE ? 1 : (strips + W - 1) / W;
+  const int strips = (K + STRIP - 1) / STRIP, mine = SINGLE ? wave < strips : (strips - wave + W - 1) / W, most = SINGLE ? 1 : (strips + W - 1) / W;
   // A block's tiles are neighbours, so that its columns of C leave as whole lines.
   // (64 bits: 256 times the tiles of an N of 2^27 pass 32)
   const unsigned tiles = ((unsigned)N + R - 1) / R;
@@ -59,10 +60,11 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
 
   // `count` loads of two rows each, `past` the caches or not: a lane's place in LDS is fixed, so the row's pieces are chosen by it.  Past the
   // rows or K: zeros.
-  auto fetch_rows = [&](const bf16_t* base, int rows, int strip, char* to, auto count, auto past) {
+  auto fetch_rows = [&](const bf16_t* base, int rows, int strip, char* to, auto count, auto past, int most_rows = 64) {
     const __amdgpu_buffer_rsrc_t run = bounded_bytes(base, rows * K * 2);
 #pragma unroll
     for (int i = 0; i < decltype(count)::value; ++i) {
+      if (2 * i >= most_rows) break;
       const int r = 2 * i + (lane >> 5), col = strip * STRIP + (((lane & 31) ^ (r & 15)) << 3);
       const int offset = col < K && r < rows ? (r * K + col) * 2 : NOWHERE;
       if (decltype(past)::value) __builtin_amdgcn_raw_ptr_buffer_load_lds(run, IRON_LDS_PTR(to + i * 1024), 16, offset, 0, 0, 2);   // non-temporal
@@ -72,12 +74,12 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
   auto fetch = [&](int item) {
     char* to = held + item % STAGES * S::ITEM;
     const int t = SINGLE ? item : item / max(mine, 1), strip = wave + W * (SINGLE ? 0 : item - t * mine), row0 = (tile0 + t) * R;
-    const int rows = item < items ? min(R, N - row0) : 0;   // past the last item: as many loads, of nothing
+    const int rows = min(R, N - row0);
     if (!SINGLE && S::A_BY_LDS) {
-      fetch_rows(A, rows > 0 ? M : 0, strip, to, std::integral_constant<int, S::A_INST>(), std::false_type());
+      fetch_rows(A, M, strip, to, std::integral_constant<int, S::A_INST>(), std::false_type());
       to += S::A_BYTES;
     }
-    fetch_rows(B + (rows > 0 ? (size_t)row0 * K : 0), rows, strip, to, std::integral_constant<int, S::B_INST>(), std::integral_constant<bool, STREAM>());
+    fetch_rows(B + (size_t)row0 * K, rows, strip, to, std::integral_constant<int, S::B_INST>(), std::integral_constant<bool, STREAM>());
   };
   // Fragments: lane (quad, l16) has columns 32 k + 8 quad .. + 7 of row l16 (of B's eight rows l16 % 8; of a row of A past the last whatever
   // is there, for columns of the product that are not stored).
@@ -99,15 +101,16 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
 #pragma unroll
     for (int k = 0; k < 8; ++k) af[0][k] = lds_read_b128_at<0>((at + a_at) ^ (k << 6));
   };
-  if (SINGLE) {
-    if (S::A_BY_LDS) fetch_rows(A, M, wave, own, std::integral_constant<int, S::A_INST>(), std::false_type());
+  if (SINGLE && items > 0) {
+    if (S::A_BY_LDS) fetch_rows(A, M, wave, own, std::integral_constant<int, S::A_INST>(), std::false_type(), M);
     else a_from_memory(wave);
   }
 #pragma unroll
-  for (int i = 0; i < STAGES - 1; ++i) fetch(i);
-  if (SINGLE && S::A_BY_LDS) {
+  for (int i = 0; i < STAGES - 1; ++i)
+    if (i < items) fetch(i);
+  if (SINGLE && S::A_BY_LDS && items > 0) {
     __builtin_amdgcn_sched_barrier(0);
-    wait_vmcnt<(STAGES - 1) * S::INST>();
+    wait_vmcnt<(STAGES - 1) * S::INST>();   // (the first item's loads stay out)
     a_from_lds(lds0 + (unsigned)(own - lds));
 #pragma unroll
     for (int k = 0; k < 8; ++k) lds_wait_for<0>(af[0][k]);
@@ -131,9 +134,13 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
     for (int s = 0; s < most; ++s) {
       if (s >= mine) continue;   // (the other waves' last strips)
       if (!SINGLE && !S::A_BY_LDS) a_from_memory(wave + W * s);
-      fetch(item + STAGES - 1);
-      __builtin_amdgcn_sched_barrier(0);
-      wait_vmcnt<(STAGES - 1) * S::INST>();
+      if (STAGES == 1 || item + STAGES - 1 < items) {
+        fetch(item + STAGES - 1);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vmcnt<(STAGES - 1) * S::INST>();
+      } else {
+        wait_vmcnt<0>();
+      }
       __builtin_amdgcn_sched_barrier(0);
       const unsigned at = lds0 + (unsigned)(held - lds) + item % STAGES * S::ITEM;
       if (!SINGLE && S::A_BY_LDS) a_from_lds(at);
@@ -338,40 +345,41 @@ static int launch_gemm_strips(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
   IRON_LAUNCH_CHECK();
 }
 
-// Which products go by strips, by what both kernels took over sixty shapes (us, gemm_few_kernel against strips).  Below 4 MB of B
-// a launch is mostly its start, which gemm_few_kernel's is shorter (777 x 1000, 8 rows: 3.3 against 3.5).
-// K up to eight strips: up to 16 rows of A (8 rows: 8192 x 2048 9.0 / 8.7, 16384 x 1024 12.1 / 10.4, 128256 x 2048 105 / 84), but not short
-// rows that straddle cache lines (16000 x 600 8.7 / 9.4) nor up to four rows where long rows make one round or two
-// (one row: 3072 x 2048 5.1 / 5.6, 4096 x 2048 5.4 / 5.9), up to eight of a K under 1408 (eight rows, weights out of memory: 3000 x 1224 4.2 / 4.8), nor
-// where the strips make four tiles a block of what gemm_few_kernel does in two rounds (one row: 6483 x 1360 6.1 / 7.0, 7159 x 2048 7.7 / 8.4; but sixteen rows of
-// it 8.1 / 7.3); more rows, whose sums take a second set of registers, only over a B of 64 MB
-// (20 rows: 128256 x 2048 137 / 87, 16384 x 1024 10.7 / 14.5).
-// A longer K: the strips of A that come with every tile cost as much as B's own.  Up to eight rows where a block has one tile or many
-// (2048 x 8192 13.9 / 8.9, 9048 x 8184 49 / 35, but 4096 x 14336 22.7 / 26.1 and 2728 x 6128 9.9 / 12.3); up to 16 where it
-// has one (2048 x 8192 16.7 / 10.2); more where that one's rows keep to their cache lines or are few (32 rows: 2048 x 4096 13.2 / 12.2,
-// 1024 x 8192 23.5 / 14.8; 20 rows of 1960 x 6512 13.8 / 15.1).  The loads go past the caches except where a block has
+// Which products go by strips, by what both kernels took over three hundred shapes with weights out of memory (us, gemm_few_kernel against strips).
+// K up to eight strips: up to 16 rows of A (8 rows: 64 x 384 3.9 / 2.6, 1024 x 1024 4.4 / 2.9, 8192 x 2048 9.0 / 8.2, 16000 x 600 8.8 / 7.4, 128256 x 2048
+// 105 / 82; one row: 2048 x 2048 4.5 / 3.6, 7159 x 2048 8.1 / 7.7), but not many rows of B that are a cache line or less (6 rows: 3440 x 40 2.8 / 3.4)
+// nor, short of 1408 columns that straddle lines, those that make two tiles a block of gemm_few_kernel's one round (3000 x 1224 4.2 / 4.4, 2656 x 136
+// 3.1 / 3.5); up to 32 rows, whose sums take a second set of registers, over long rows
+// that keep to their lines (32 rows: 1024 x 2048 7.8 / 6.6, 4160 x 2048 13.8 / 9.5; but 2400 x 192 3.5 / 5.2) or a B of 64 MB (20 rows: 128256 x 2048 137 / 87).
+// A longer K: the strips of A that come with every tile cost as much as B's own.  Up to eight rows (2048 x 8192 13.9 / 8.9, 6000 x 6000 21.8 / 18.5,
+// 4096 x 14336 25.0 / 24.0, 4560 x 4416 19.5 / 12.6) but where they make two tiles a block of one round (3669 x 3168 8.0 / 8.3, 4096 x 4096 8.9 / 9.2);
+// up to 16 where a block has one tile (2048 x 8192 16.7 / 10.2) or three and more (4788 x 6848 28.6 / 21.2, 9762 x 9056 60.9 / 46.7; but 6576 x 5160
+// 21.5 / 22.3 and 3488 x 2696 7.4 / 8.5); more where that one's rows keep to their cache lines or are few (32 rows: 2048 x 4096
+// 13.2 / 12.2, 1024 x 8192 23.5 / 14.8; 20 rows of 1960 x 6512 13.8 / 15.1).  The loads go past the caches except where a block has
 // one tile over a long K (2048 x 8192, 8 rows: 9.3, past them 10.5; 4096 x 4096 10.1 and 9.4).
 // Returns -1 where it is not for them.
 static int strips_for(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s) {
-  const long long size = (long long)N * K;
-  if (size < (1 << 21)) return -1;
-  const bool one_tile = N <= 256 * STRIP_ROWS, on_lines = K % 64 == 0;
+  const bool one_tile = N <= 256 * STRIP_ROWS, two_tiles = !one_tile && N <= 512 * STRIP_ROWS, on_lines = K % 64 == 0;
   if (K <= STRIP * STRIP_WAVES) {
-    if (M > 32 || (M > 16 && size < (1 << 25)) || (!on_lines && K < 1024)) return -1;
+    const bool long_rows = K >= 1600 && on_lines && !two_tiles, large = (long long)N * K >= (1 << 25) && (on_lines || K >= 1024);
+    if (M > 32 || (M > 16 && !long_rows && !large)) return -1;
     if (M > 16) return launch_gemm_strips<2, 16, true, 2, true>(A, B, C, M, N, K, s);
-    if (M <= 4 && size <= (1 << 23) && K > 1024 && N > 1536) return -1;
-    if (K > 1024 && N > 2048 && N <= 4096 && M <= 8 && K < 1408) return -1;
-    if (K > 1024 && N > 6144 && N < 8192 && (M <= 4 || (M <= 8 && K < 1280))) return -1;
+    if (!one_tile && K < 64) return -1;
+    if (two_tiles && !on_lines && K < 1408) return -1;
     if (M <= 8) return launch_gemm_strips<1, 8, true, 2, true>(A, B, C, M, N, K, s);
     return launch_gemm_strips<1, 16, true, 2, true>(A, B, C, M, N, K, s);
   }
   if (M <= 8) {
     if (one_tile) return launch_gemm_strips<1, 8, false, 2, false>(A, B, C, M, N, K, s);
-    if (N >= 8192 || (N > 4096 && K < 4096)) return launch_gemm_strips<1, 8, false, 2, true>(A, B, C, M, N, K, s);
-    return -1;
+    if (two_tiles && K >= 3072 && K < 4608) return -1;
+    return launch_gemm_strips<1, 8, false, 2, true>(A, B, C, M, N, K, s);
+  }
+  if (M <= 16) {
+    if (one_tile) return launch_gemm_strips<1, 16, false, 1, false>(A, B, C, M, N, K, s);
+    if (two_tiles || (!on_lines && N > 6144 && N < 8192 && K < 5632)) return -1;
+    return launch_gemm_strips<1, 16, false, 1, true>(A, B, C, M, N, K, s);
   }
   if (!one_tile) return -1;
-  if (M <= 16) return launch_gemm_strips<1, 16, false, 1, false>(A, B, C, M, N, K, s);
   if (!on_lines && N > 1280) return -1;
   return M <= 32 ? launch_gemm_strips<2, 16, false, 2, false>(A, B, C, M, N, K, s) : launch_gemm_strips<4, 16, false, 2, false>(A, B, C, M, N, K, s);
 }

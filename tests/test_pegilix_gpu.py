@@ -109,6 +109,13 @@ def test_a_product_over_few_rows_by_strips(cuda, M, N, K_):
     assert (got[M] == 7).all()
 
 
+# ... the smallest sizes that go by strips, with waves that have none, and the others at the lines between the two kernels.
+@pytest.mark.parametrize("M,N,K_", [(1, 1, 8), (5, 40, 24), (16, 2047, 56), (3, 13, 264), (12, 3000, 1416), (6, 2048, 1400), (2, 3001, 2560), (9, 4104, 2056),
+                                    (16, 8200, 5640), (30, 1032, 1600), (20, 4200, 1664)])
+def test_a_product_over_few_rows_between_the_kernels(cuda, M, N, K_):
+    test_a_product_over_few_rows_by_strips(cuda, M, N, K_)
+
+
 # ... and sixteen rows and less whose product with K passes what other sizes go by strips to.
 @pytest.mark.parametrize("M,N,K_", [(16, 2048, 9216), (9, 1531, 16384), (13, 128, 16384), (16, 2041, 10008)])
 def test_a_product_over_sixteen_rows_of_a_long_k(cuda, M, N, K_):
