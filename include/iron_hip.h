@@ -628,6 +628,14 @@ int iron_stream_product_bf16(int input, const void* x, const uint16_t* gain, con
                              float* state, const int* spans, float eps, float unit, const uint16_t* W, int M,
                              int K, uint16_t* y, float* stream_row, const uint16_t* y_bias, const uint16_t* gate, const uint16_t* gate_bias,
                              void* stream);
+/* Products of up to eight rows around the stream, W (N, K), each what the entry points above compute in turn.
+ * norm_strips: y (rows, N) = W times the float rows x (K up to 2048), RMS-normed with unit + gain.
+ * gated_strips: iron_stream_gated_rows of W times the bf16 rows x, plus y_bias (may be NULL), on stream_rows (rows, N), by gates
+ * `gate_stride` apart. */
+int iron_norm_strips_bf16(const float* x, const uint16_t* gain, float eps, float unit, const uint16_t* W, uint16_t* y, int rows, int N,
+                          int K, void* stream);
+int iron_gated_strips_bf16(const uint16_t* x, const uint16_t* W, const uint16_t* y_bias, const uint16_t* gate, int gate_stride,
+                           const uint16_t* gate_bias, float* stream_rows, int rows, int N, int K, void* stream);
 /* norm_product: y = W (M, K) times h, the float row x normed in `groups` parts (iron_stream_groups); h (may be NULL) as well, and
  * with a router (logits, K) its logits in float to z.  product_sum: the stream's row += W (M, K) times x, plus also (may be NULL). */
 int iron_norm_product_bf16(const float* x, const uint16_t* gain, int groups, float eps, float unit, const uint16_t* W, int M, int K,

@@ -32,6 +32,8 @@ in a batched decoder's decode step (bf16; a float32 stream, layers with a state)
   GEMV gate, GEMV up, SiLU / GELU (tanh) / ReLU, Mul     => iron_gemv_fused_bf16 (epilogue 2 / 3 / 6)
   StreamNorm, GEMV (one slot, as the rest here)          => iron_stream_product_bf16 (input 1)
   [MinGRU / PolyNorm,] GEMV, StreamGatedAdd              => iron_stream_product_bf16 (input 0 / 3 / 4)
+  StreamNorm, GEMM (two to eight slots, as the next)     => iron_norm_strips_bf16
+  GEMM, StreamGatedAdd                                   => iron_gated_strips_bf16
   LatentRows, GEMV (the queries)                         => iron_latent_query_bf16
   StreamNorm (groups), GEMV                              => iron_norm_product_bf16
   Hgrn2, HeadGate [, GatedColumns] (any slots)           => iron_decode_hgrn2_bf16
@@ -357,6 +359,33 @@ def plan(recording, tensor: Callable[[Any], Any], word: Callable[[Any], Any],
             args["x"] = tensor(s.inputs["B"]).reshape(-1)
             return Fused("gated_product", j, 2, lambda a=args, kw=kw: kernels.stream_product(input="row", **a, **kw))
         return None
+
+    def stream_strips_at(j):
+        """The launch for a few rows' product (a batch's step) with the stream's norm ahead of it, which every block then takes for itself, or
+        with its sum into the stream behind it; streams as wide as one strip a wave makes up (the norm of a wider one is a launch,
+        which then takes the sum ahead of it too: 12.4 us with a product over K = 8192, 9.5 and 2.2 apart) -- or None."""
+        s = steps[j]
+        normed = _name(s) == "StreamNorm"
+        if j + 1 >= len(steps):
+            return None
+        g, o = (steps[j + 1], s) if normed else (s, steps[j + 1])   # the product, and the step around the stream
+        if not (_name(g) == "GEMM" and g.op.b_col_maj and not g.op.c_col_maj and 2 <= g.op.M <= 8 and g.op.K % 8 == 0
+                and o.op.rows == g.op.M and o.op.cols <= 2048 and o.op.dtype is bfloat16 and bare(g) and bare(o)):
+            return None
+        kw = dict(rows=g.op.M, N=g.op.N, K=g.op.K)
+        if normed:
+            h = s.outputs["y"]
+            if not (s.op.groups == 1 and s.op.cols == g.op.K and _same(g.inputs["A"], h) and once(h)):
+                return None
+            args = dict(x=tensor(s.inputs["x"]), gain=tensor(s.inputs["weight"]), W=tensor(g.inputs["B"]), y=tensor(g.outputs["C"]))
+            kw |= dict(eps=float(s.op.epsilon), unit=float(s.op.unit))
+            return Fused("norm_strips", j, 2, lambda: kernels.norm_strips(**args, **kw))
+        y, at = g.outputs["C"], o.op.gate_at
+        if not (o.op.cols == g.op.N and g.op.N % 4 == 0 and o.op.gate_width % 4 == 0 and at % 4 == 0 and _same(o.inputs["y"], y) and once(y)):
+            return None
+        args = dict(x=tensor(g.inputs["A"]), W=tensor(g.inputs["B"]), stream=tensor(o.inputs["x"]), gate=tensor(o.inputs["gate"]).reshape(-1)[at:],
+                    gate_bias=tensor(o.inputs["gate_bias"]), y_bias=tensor(o.inputs["y_bias"]) if "y_bias" in o.inputs else None)
+        return Fused("gated_strips", j, 2, lambda: kernels.gated_strips(**args, **kw, gate_stride=o.op.gate_width))
 
     def depth_rows_at(j):
         """The launch for a block's output into the stream, the average over what it was behind every layer and the row a
@@ -876,6 +905,9 @@ def plan(recording, tensor: Callable[[Any], Any], word: Callable[[Any], Any],
                 kw = dict(rows=s.op.rows, cols=s.op.cols, eps=float(s.op.epsilon), unit=float(s.op.unit), valid=word(s.values.get("valid")))
                 got = Fused("stream_add_norm", i, 2, lambda a=args, kw=kw: kernels.stream_rows(**a, **kw))
         elif (_name(s) in ("StreamNorm", "MinGRU", "PolyNorm") or gemv_row(s)) and (got := stream_product_at(i)) is not None:
+            pass
+        elif ((_name(s) == "StreamNorm" or (_name(s) == "GEMM" and i + 1 < len(steps) and _name(steps[i + 1]) == "StreamGatedAdd"))
+              and (got := stream_strips_at(i)) is not None):
             pass
         elif _name(s) == "LatentRows" and (got := latent_query_at(i)) is not None:
             pass

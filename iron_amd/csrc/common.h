@@ -169,6 +169,15 @@ __device__ __forceinline__ float wave_sum(float v) {
   v += IRON_DPP(0.f, v, 0x143, 0xC);  // row_bcast31 into rows 2 and 3
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
+// Each half of the wave's sum, in its last lane.
+__device__ __forceinline__ float half_wave_sum(float v) {
+  v += IRON_DPP(0.f, v, 0xB1, 0xF);
+  v += IRON_DPP(0.f, v, 0x4E, 0xF);
+  v += IRON_DPP(0.f, v, 0x141, 0xF);
+  v += IRON_DPP(0.f, v, 0x140, 0xF);
+  v += IRON_DPP(0.f, v, 0x142, 0xA);
+  return v;
+}
 __device__ __forceinline__ float wave_max(float v) {
   v = fmaxf(v, IRON_DPP(v, v, 0xB1, 0xF));
   v = fmaxf(v, IRON_DPP(v, v, 0x4E, 0xF));

@@ -3,6 +3,8 @@
 // Two kernels.  `gemm_strips_kernel` takes B eight rows at a time through LDS; `gemm_few_kernel` takes sixteen straight into the
 // MFMA's registers and stands where the first's operands do not fit.  With GATED a second matrix is streamed beside the first and
 // the output is act(A B^T) * (A B2^T), rounded where the separate steps round.
+//
+// Around a float32 stream A may be its normed rows (iron_norm_strips_bf16), and C may join it through a gate (iron_gated_strips_bf16).
 #include "../../include/iron_hip.h"
 #include "common.h"
 
@@ -39,10 +41,77 @@ struct Strips {
   static constexpr int A_INST = A_BYTES / 1024, B_INST = B_BYTES / 1024, INST = ITEM / 1024;
 };
 
-template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM>
+// A's rows are rows of the stream, RMS-normed (as in stream.hip), up to eight of them and K up to eight strips: every block makes all of A for
+// its own tiles, a wave its strip of K while the first of B is on its way.  The launch of a norm between two of 256 blocks takes 2.2 us, and making
+// the rows here 1.0: twice A's bytes out of L2, and a chain of sums, root and scale.  Eight rows over K = 2048, weights out of memory, a norm and a
+// product against both here: 2048 columns 6.1 / 5.1 us, 4160 8.2 / 6.7, 10240 11.6 / 10.3, 128256 86.2 / 85.4.  (A recurrence's step made the same
+// way was not the faster one, 8.9 / 9.3 with its product and sum: three exponentials an element, 8 x 2048 of them a block.)
+struct StripsNorm {
+  const bf16_t* gain;
+  float eps, unit;
+};
+// C joins the stream: stream += (C + y_bias) * sigmoid(gate + gate_bias), C rounded as it would be stored, by the lanes that hold its sums, which ask
+// for what they add them to ahead of everything else: 0.4 us where a launch for it took 2.9 with the next norm (2048 columns: K = 2048 6.9 / 4.4,
+// K = 8192 12.4 / 9.5).
+struct StripsOut {
+  float* stream;              // rows of N
+  const bf16_t *y_bias, *gate, *gate_bias;   // y_bias may be null
+  int gate_stride;
+};
+struct Joined {   // ... what four columns of it need
+  float4 held;
+  uint2 gate, gate_bias, y_bias;
+};
+
+// A lane's eight columns of rows 2 i + lane / 32 of the stream, normed.  `sums`: LDS, 64 floats.
+__device__ __forceinline__ void norm_strips(const StripsNorm& norm, int K, int lane, int wave, unsigned sums, const float4 (&f)[4][2], const uint4& gain,
+                                            uint4 (&out)[4]) {
+  float ss[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float4 a = f[i][0], b = f[i][1];
+    const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    ss[i] = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss[i] = fmaf(x[j], x[j], ss[i]);
+    ss[i] = half_wave_sum(ss[i]);
+  }
+  if ((lane & 31) == 31) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) asm volatile("ds_write_b32 %0, %1" ::"v"(sums + ((2 * i + (lane >> 5)) * STRIP_WAVES + wave) * 4), "v"(ss[i]) : "memory");
+  }
+  lds_barrier();
+  // Lane l has row l % 8's: a root and a quotient a lane, and not one a lane and row.
+  bf16x8 part[2];
+  part[0] = lds_read_b128_at<0>(sums + (lane & 7) * STRIP_WAVES * 4);
+  part[1] = lds_read_b128_at<16>(sums + (lane & 7) * STRIP_WAVES * 4);
+  float total = 0.f;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    lds_wait_for<0>(part[h]);
+    const f32x4 p = __builtin_bit_cast(f32x4, part[h]);
+    total += p[0] + p[1] + p[2] + p[3];
+  }
+  const int inverse = __builtin_bit_cast(int, 1.0f / sqrtf(total / (float)K + norm.eps));
+  float g[8];
+  unpack8(gain, g);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int even = __builtin_amdgcn_readlane(inverse, 2 * i), odd = __builtin_amdgcn_readlane(inverse, 2 * i + 1);
+    const float inv = __builtin_bit_cast(float, lane < 32 ? even : odd);
+    const float4 a = f[i][0], b = f[i][1];
+    float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = x[j] * inv * (norm.unit + g[j]);
+    out[i] = pack8(x);
+  }
+}
+
+template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM, bool NORMED = false, bool JOINS = false>
 __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
-                                                                       bf16_t* __restrict__ C, int M, int N, int K) {
+                                                                       bf16_t* __restrict__ C, int M, int N, int K, StripsNorm norm, StripsOut out) {
   typedef Strips<MT, MA, SINGLE, STAGES> S;
+  static_assert(!NORMED || (SINGLE && MT == 1 && MA == 8), "a wave norms its own strip of eight rows");
   constexpr int W = STRIP_WAVES, R = STRIP_ROWS, GROUP = STRIP_OUT / R;   // GROUP: tiles whose columns are stored together
   static_assert(STAGES <= 2, "the last item's wait is for all that is out");
   constexpr int NOWHERE = 0x7ffffff0;   // an offset past the end of every run of rows (64 rows of at most 2^22, the entry point's bound, are 2^29 bytes)
@@ -101,21 +170,70 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
 #pragma unroll
     for (int k = 0; k < 8; ++k) af[0][k] = lds_read_b128_at<0>((at + a_at) ^ (k << 6));
   };
-  if (SINGLE && items > 0) {
+  // What the stream's columns need of a tile, asked for ahead of everything for the first.
+  const bool joins = JOINS && lane < 32 && l16 < M;
+  auto join_loads = [&](int t) {
+    Joined j{};
+    const int n = (tile0 + t) * R + quad * 4;
+    if (joins && n < N) {
+      j.held = *reinterpret_cast<const float4*>(out.stream + (size_t)l16 * N + n);
+      j.gate = *reinterpret_cast<const uint2*>(out.gate + (size_t)l16 * out.gate_stride + n);
+      j.gate_bias = *reinterpret_cast<const uint2*>(out.gate_bias + n);
+      if (out.y_bias != nullptr) j.y_bias = *reinterpret_cast<const uint2*>(out.y_bias + n);
+    }
+    return j;
+  };
+  Joined first_joined{};
+  if (JOINS && wave == 0) first_joined = join_loads(0);
+  if (!NORMED && SINGLE && items > 0) {
     if (S::A_BY_LDS) fetch_rows(A, M, wave, own, std::integral_constant<int, S::A_INST>(), std::false_type(), M);
     else a_from_memory(wave);
   }
+  if constexpr (!NORMED) {
 #pragma unroll
-  for (int i = 0; i < STAGES - 1; ++i)
-    if (i < items) fetch(i);
-  if (SINGLE && S::A_BY_LDS && items > 0) {
+    for (int i = 0; i < STAGES - 1; ++i)
+      if (i < items) fetch(i);
+  } else {
+    // Rows as they are fetched: row 2 i + lane / 32, eight columns a lane (past the rows or K: zeros).
+    const int col = wave * STRIP + ((lane & 31) << 3), hi = lane >> 5;
+    const __amdgpu_buffer_rsrc_t rows = bounded_bytes(A, M * K * 4);
+    float4 f[4][2];
+    uint4 made[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int r = 2 * i + hi;
+        f[i][h] = __builtin_bit_cast(float4, load_bounded(rows, col < K && r < M ? (r * K + col) * 4 + 16 * h : NOWHERE));
+      }
+    const uint4 gain = load_bounded(bounded_bytes(norm.gain, K * 2), col * 2);
+    __builtin_amdgcn_sched_barrier(0);
+    // (of a wave without a strip too, for whom it is nothing: behind a branch the compiler, which then counts none of its loads, would wait for B
+    // before the norm)
+#pragma unroll
+    for (int i = 0; i < STAGES - 1; ++i) fetch(i);
+    __builtin_amdgcn_sched_barrier(0);
+    norm_strips(norm, K, lane, wave, part0 + S::PART, f, gain, made);
+    // (the strip is the wave's alone: no barrier)
+    const unsigned mine_at = lds0 + (unsigned)(own - lds);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 2 * i + hi;
+      lds_write_b128(mine_at + r * STRIP_BYTES + (((lane & 31) ^ r) << 4), __builtin_bit_cast(f32x4, made[i]));
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    a_from_lds(mine_at);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) lds_wait_for<0>(af[0][k]);
+  }
+  if (!NORMED && SINGLE && S::A_BY_LDS && items > 0) {
     __builtin_amdgcn_sched_barrier(0);
     wait_vmcnt<(STAGES - 1) * S::INST>();   // (the first item's loads stay out)
     a_from_lds(lds0 + (unsigned)(own - lds));
 #pragma unroll
     for (int k = 0; k < 8; ++k) lds_wait_for<0>(af[0][k]);
   }
-  const bool staged = my_tiles > 1;   // (a lone tile's columns leave as they are: by way of LDS and another barrier 8 rows of 2048 x 2048 took 4.44 us instead of 4.24)
+  const bool staged = !JOINS && my_tiles > 1;   // (a lone tile's columns leave as they are: by way of LDS and another barrier 8 rows of 2048 x 2048 took 4.44 us instead of 4.24)
   // The columns of `count` tiles from `first` on, from half `half` of the out stage, by one wave.
   auto flush = [&](int first, int count, int half) {
     for (int e = lane; e < M * count; e += 64) {
@@ -167,8 +285,9 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
       lds_write_b128(pa + ((wave * MT + m) * 64 + lane) * 16, v);
     }
     lds_barrier();
-    if (t > 0 && t % GROUP == 0 && wave == (t + W / 2) % W) flush(t - GROUP, GROUP, (t / GROUP - 1) & 1);
+    if (!JOINS && t > 0 && t % GROUP == 0 && wave == (t + W / 2) % W) flush(t - GROUP, GROUP, (t / GROUP - 1) & 1);
     // Tile t's sums by wave t % 8: lane (quad, l16) of the first two quads has columns 4 quad .. + 3 of row l16.
+    const Joined joined = JOINS ? (t == 0 ? first_joined : (wave == t % W ? join_loads(t) : Joined{})) : Joined{};
     if (wave == t % W && lane < 32) {
       const int n = (tile0 + t) * R + quad * 4;
 #pragma unroll
@@ -184,7 +303,17 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
 #pragma unroll
           for (int j = 0; j < 4; ++j) v[j] += __builtin_bit_cast(f32x4, p[q])[j];
         const int r = m * 16 + l16;
-        if (staged) {
+        if (JOINS) {
+          if (r < M && n < N) {
+            float h[4] = {joined.held.x, joined.held.y, joined.held.z, joined.held.w};
+            const float g[4] = {bf16_lo(joined.gate.x), bf16_hi(joined.gate.x), bf16_lo(joined.gate.y), bf16_hi(joined.gate.y)};
+            const float gb[4] = {bf16_lo(joined.gate_bias.x), bf16_hi(joined.gate_bias.x), bf16_lo(joined.gate_bias.y), bf16_hi(joined.gate_bias.y)};
+            const float yb[4] = {bf16_lo(joined.y_bias.x), bf16_hi(joined.y_bias.x), bf16_lo(joined.y_bias.y), bf16_hi(joined.y_bias.y)};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) h[j] += (round_bf16(v[j]) + yb[j]) * (1.0f / (1.0f + expf(-(g[j] + gb[j]))));
+            *reinterpret_cast<float4*>(out.stream + (size_t)r * N + n) = make_float4(h[0], h[1], h[2], h[3]);
+          }
+        } else if (staged) {
           const unsigned to = out0 + (t / GROUP & 1) * S::OUT + (r * STRIP_OUT + t % GROUP * R + quad * 4) * 2;
           const uint64_t four = (uint64_t)pack_bf16(v[2], v[3]) << 32 | pack_bf16(v[0], v[1]);
           asm volatile("ds_write_b64 %0, %1" ::"v"(to), "v"(four) : "memory");
@@ -329,19 +458,20 @@ static int launch_gemm_few(const bf16_t* A, const bf16_t* B, const bf16_t* B2, b
   IRON_LAUNCH_CHECK();
 }
 
-template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM>
-static int launch_gemm_strips(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s) {
+template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM, bool NORMED = false, bool JOINS = false>
+static int launch_gemm_strips(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s, const StripsNorm& norm = {},
+                              const StripsOut& out = {}) {
   typedef Strips<MT, MA, SINGLE, STAGES> S;
   static_assert(S::LDS <= 163840, "a CU's LDS");
   static LdsOptIn opt;
-  auto kernel = &gemm_strips_kernel<MT, MA, SINGLE, STAGES, STREAM>;
+  auto kernel = &gemm_strips_kernel<MT, MA, SINGLE, STAGES, STREAM, NORMED, JOINS>;
   const hipError_t e = opt.ensure(reinterpret_cast<const void*>(kernel), S::LDS);
   if (e != hipSuccess) {
     set_error("gemm_few: %s", hipGetErrorString(e));
     return (int)e;
   }
   const unsigned tiles = ((unsigned)N + STRIP_ROWS - 1) / STRIP_ROWS;
-  hipLaunchKernelGGL(kernel, dim3(tiles < STRIP_BLOCKS ? tiles : STRIP_BLOCKS), dim3(STRIP_WAVES * 64), S::LDS, s, A, B, C, M, N, K);
+  hipLaunchKernelGGL(kernel, dim3(tiles < STRIP_BLOCKS ? tiles : STRIP_BLOCKS), dim3(STRIP_WAVES * 64), S::LDS, s, A, B, C, M, N, K, norm, out);
   IRON_LAUNCH_CHECK();
 }
 
@@ -404,4 +534,28 @@ extern "C" int iron_gemm_few_bf16(const uint16_t* A, const uint16_t* B, const ui
   if (B2 != nullptr) return launch_gemm_few<FEW_GATED>(A, B, B2, C, M, N, K, activation, s);
   if (N >= 8192) return launch_gemm_few<FEW_TWO>(A, B, nullptr, C, M, N, K, 0, s);
   return launch_gemm_few<FEW_ONE>(A, B, nullptr, C, M, N, K, 0, s);
+}
+
+// x of a norm: float rows.
+extern "C" int iron_norm_strips_bf16(const float* x, const uint16_t* gain, float eps, float unit, const uint16_t* W, uint16_t* y, int rows, int N, int K,
+                                     void* stream) {
+  IRON_REQUIRE(x && gain && W && y, "norm_strips: null operand");
+  IRON_REQUIRE(rows > 0 && rows <= 8 && N > 0, "norm_strips: rows (%d) from 1 to 8, N (%d) positive", rows, N);
+  IRON_REQUIRE(K >= 8 && K % 8 == 0 && K <= STRIP * STRIP_WAVES, "norm_strips: K (%d) is a positive multiple of 8 up to %d", K, STRIP * STRIP_WAVES);
+  IRON_REQUIRE((((uintptr_t)x | (uintptr_t)gain | (uintptr_t)W) & 15) == 0, "norm_strips: operands must be 16-byte aligned");
+  return launch_gemm_strips<1, 8, true, 2, true, true>(reinterpret_cast<const bf16_t*>(x), W, y, rows, N, K, (hipStream_t)stream, StripsNorm{gain, eps, unit});
+}
+
+extern "C" int iron_gated_strips_bf16(const uint16_t* x, const uint16_t* W, const uint16_t* y_bias, const uint16_t* gate, int gate_stride,
+                                      const uint16_t* gate_bias, float* stream_rows, int rows, int N, int K, void* stream) {
+  IRON_REQUIRE(x && W && gate && gate_bias && stream_rows, "gated_strips: null operand");
+  IRON_REQUIRE(rows > 0 && rows <= 8 && N > 0 && N % 4 == 0, "gated_strips: rows (%d) from 1 to 8, N (%d) a positive multiple of 4", rows, N);
+  IRON_REQUIRE(K >= 8 && K % 8 == 0 && K <= (1 << 22), "gated_strips: K (%d) is a positive multiple of 8 up to 2^22", K);
+  IRON_REQUIRE(gate_stride >= N && gate_stride % 4 == 0, "gated_strips: gates %d apart, a multiple of 4, for N (%d)", gate_stride, N);
+  IRON_REQUIRE((((uintptr_t)x | (uintptr_t)W | (uintptr_t)stream_rows) & 15) == 0 && (((uintptr_t)y_bias | (uintptr_t)gate | (uintptr_t)gate_bias) & 7) == 0,
+               "gated_strips: operands must be 16-byte aligned, a gate and the output's biases 8-byte");
+  const StripsOut out{stream_rows, y_bias, gate, gate_bias, gate_stride};
+  hipStream_t s = (hipStream_t)stream;
+  if (K <= STRIP * STRIP_WAVES) return launch_gemm_strips<1, 8, true, 2, true, false, true>(x, W, nullptr, rows, N, K, s, {}, out);
+  return launch_gemm_strips<1, 8, false, 2, false, false, true>(x, W, nullptr, rows, N, K, s, {}, out);
 }

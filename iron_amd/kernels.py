@@ -1171,6 +1171,30 @@ def stream_product(W, x, *, input, M, K, y=None, stream=None, y_bias=None, gate=
                                          ptr(gate), ptr(gate_bias), current_stream()), "iron_stream_product_bf16")
 
 
+def norm_strips(x, gain, W, y, *, rows, N, K, eps, unit=0.0):
+    """Up to eight rows of the stream, normed, and their product, one launch."""
+    _f32(x, rows * K, "x")
+    _bf16(gain, K, "gain")
+    _bf16(W, N * K, "W")
+    _bf16(y, rows * N, "y")
+    check(lib().iron_norm_strips_bf16(ptr(x), ptr(gain), float(eps), float(unit), ptr(W), ptr(y), rows, N, K, current_stream()), "iron_norm_strips_bf16")
+
+
+def gated_strips(x, W, stream, gate, gate_bias, *, rows, N, K, gate_stride, y_bias=None):
+    """Up to eight rows' product, joining the rows ``stream`` through ``gate`` (its rows ``gate_stride`` apart, from its first
+    column on), one launch."""
+    _bf16(x, rows * K, "x")
+    _bf16(W, N * K, "W")
+    _f32(stream, rows * N, "stream")
+    _bf16(gate_bias, N, "gate_bias")
+    if y_bias is not None:
+        _bf16(y_bias, N, "y_bias")
+    if _dev(gate, "gate").numel() < (rows - 1) * gate_stride + N:
+        raise ValueError(f"gated_strips: a gate of {gate.numel()} elements for {rows} rows of {N}, {gate_stride} apart")
+    check(lib().iron_gated_strips_bf16(ptr(x), ptr(W), ptr(y_bias), ptr(gate), gate_stride, ptr(gate_bias), ptr(stream), rows, N, K,
+                                       current_stream()), "iron_gated_strips_bf16")
+
+
 def latent_query(x, q_gain, c_gain, spans, W, q, latents, *, M, stride, q_rank, rank, ring, eps, rot=0, turned=0, angle_rows=0,
                  angles=None, shared_keys=None):
     """A single slot's row: its latents normed, stored and turned, and the queries' product."""

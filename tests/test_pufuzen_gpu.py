@@ -303,6 +303,53 @@ def test_a_row_s_product_joins_the_stream(cuda, M, K_):
                 assert np.array_equal(new[(start - 1) % 2], state[(start - 1) % 2]) and np.abs(new[start % 2] - S).max() <= 1e-5 * np.abs(S).max()
 
 
+# Few columns and many, more tiles than blocks, strips that end in a piece, waves without a strip, one row and all eight.
+@pytest.mark.parametrize("rows,N,K_", [(1, 64, 8), (3, 71, 264), (8, 2048, 2048), (5, 4103, 2040), (7, 20001, 1000)])
+def test_normed_rows_products(cuda, rows, N, K_):
+    rng = np.random.default_rng(N)
+    W, gain, x = bf(rng, N, K_, scale=1 / np.sqrt(K_)), bf(rng, K_), rng.standard_normal((rows, K_)).astype(F32) * 3
+    x[0] *= 100   # (a row's own root mean square)
+    y = torch.empty((rows, N), dtype=torch.bfloat16, device="cuda")
+    K.norm_strips(device(x, F32), device(gain, BF16), device(W, BF16), y, rows=rows, N=N, K=K_, eps=1e-3, unit=0.5)
+    h = round_bf16((x / np.sqrt((x.astype(np.float64) ** 2).mean(1, keepdims=True) + 1e-3) * (0.5 + gain)).astype(F32))
+    want = h.astype(np.float64) @ W.astype(np.float64).T
+    assert (np.abs(from_torch(y) - want).max(1) <= 6e-3 * np.abs(want).max(1)).all()
+
+
+@pytest.mark.parametrize("rows,N,K_", [(1, 64, 8), (3, 76, 264), (8, 2048, 2048), (6, 2100, 2040), (8, 2048, 8192), (5, 4104, 2064), (7, 6008, 1000)])
+def test_rows_products_join_the_stream(cuda, rows, N, K_):
+    rng = np.random.default_rng(N + K_)
+    W, x, gate_bias, stream = bf(rng, N, K_, scale=1 / np.sqrt(K_)), bf(rng, rows, K_), bf(rng, N), rng.standard_normal((rows, N)).astype(F32)
+    gates = bf(rng, rows, N + 12, scale=2)
+    opened = 1 / (1 + np.exp(-(gates[:, 4 : 4 + N].astype(np.float64) + gate_bias)))
+    for bias in (None, bf(rng, N)):
+        to = device(stream, F32)
+        K.gated_strips(device(x, BF16), device(W, BF16), to, device(gates, BF16).reshape(-1)[4:], device(gate_bias, BF16), rows=rows, N=N, K=K_,
+                       gate_stride=N + 12, y_bias=None if bias is None else device(bias, BF16))
+        want = stream + (x.astype(np.float64) @ W.astype(np.float64).T + (0 if bias is None else bias)) * opened
+        assert np.abs(from_torch(to) - want).max() <= 8e-3 * np.abs(want).max()
+
+
+def test_a_batch_s_steps_in_few_launches(cuda):
+    """Steps of two to eight slots: the stream's norms and sums in the products' launches, with what the steps alone give."""
+    for slots in (2, 8):
+        rows = {}
+        for fuse in (True, False):
+            model, _ = built("mixed", Pufuzen, slots=slots, max_seq_len=200, prefill_chunk=32)
+            model.load_versions(fuse=fuse)
+            kinds = {f.kind for f in model.decode_step._fused.values()}
+            assert not fuse or {"norm_strips", "gated_strips"} <= kinds
+            prompts = [tokens_of(model, 5 + 3 * i, seed=i) for i in range(slots)]
+            model.batch.step([Entry(i, p) for i, p in enumerate(prompts)])
+            steps = []
+            for t in range(6):   # (a slot is idle every other step)
+                live = [i for i in range(slots) if t % 2 or i != 1]
+                steps += [r[0] for r in model.batch.step([Entry(i, [int(prompts[i][t % 5])], [0]) for i in live])]
+            rows[fuse] = np.stack(steps)
+            model.release()
+        assert far_off(rows[True], rows[False], rows[False].std()) < LIMIT["bf16"]
+
+
 # ---------------------------------------------------------------- whole models
 
 
