@@ -418,44 +418,55 @@ constexpr int NOWHERE = (int)0x80000000u;   // past stage_rows' 2^31 - 1 bytes, 
 // the tiles outnumber the CUs, 8 (128 KB, more loads in flight) where a CU has one block anyway.
 // An element's sum is the same chain of 32-wide k-steps as in the 128 x 128 and the 256 x 256 tiles: where a row bound chooses
 // the tile, a row's products are the same bits whatever rows share the launch.
-// `qkv` carries only the optional residual epilogue here.  MI: 16-row tiles a wave owns; 4 make 128 x 64 tiles.  PAIR: both
-// first products of a gated feed-forward, 32 columns of each (`qkv` says the gate's kind).
-template <int STAGES, bool PAIR = false, int MI = 2>
+// `qkv` carries only the optional residual epilogue here, or (QKV) the fused projections'.  WM x 4 / WM waves of MI x NJ tiles: <2, 2, 2> are 64 x 64, <4>
+// 128 x 64.  PAIR: both first products of a gated feed-forward, 32 columns of each (`qkv` says the gate's kind).
+// A few rows' tiles wait for what a CU can draw of operands that are 128 bytes of a row here and there, some 60 GB/s of weights out of memory, whatever the
+// stages in flight (8 or 10 of 16 KB the same): where the tiles leave CUs without one, smaller tiles have more CUs draw less each.  2048 columns over 2048
+// with a residual, us by 64 x 64 tiles, 64 x 32 <1, 4, 2> and 32 x 32 <1, 2, 1>: 12.5 / 10.4 / 8.6 (256 blocks: up to 640, 256 and 128 rows); over 8192
+// 36 / 28.7 / 21.3.
+template <int STAGES, bool PAIR = false, int MI = 2, int WM = 2, int NJ = 2, bool QKV = false>
 __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
                                                bf16_t* __restrict__ C, int M, int N, int K,
                                                int Mv, int tiles_m, int tiles_n,
                                                int patched, const QkvTail& qkv,
                                                const bf16_t* __restrict__ up = nullptr, bf16_t* __restrict__ gate_out = nullptr) {
-  constexpr int NT_BM = 32 * MI, NT_BN = 64;
+  constexpr int NT_BM = 16 * MI * WM, NT_BN = 16 * NJ * (4 / WM);
   constexpr int NT_A_BYTES = NT_BM * BK * 2, NT_STAGE_BYTES = (NT_BM + NT_BN) * BK * 2;
   constexpr int INST = NT_BM / 8 / 4, B_INST = NT_BN / 8 / 4;  // 1 KB loads of A and of B a wave issues per stage
-  constexpr int LOADS = INST + B_INST;
-  static_assert(BK == 64 && LOADS <= 2 * MI && STAGES >= 4 && (MI == 2 || !PAIR), "two 32-wide k-steps a stage, a load behind every second MFMA");
+  constexpr int LOADS = INST + B_INST, PER = (LOADS + 2 * MI - 1) / (2 * MI);   // PER: loads behind every second MFMA
+  static_assert(BK == 64 && STAGES >= 4 && ((MI == 2 && WM == 2 && NJ == 2) || !PAIR) && (!QKV || (NJ == 2 && NT_BN <= 64)),
+                "two 32-wide k-steps a stage");
   extern __shared__ __align__(16) char smem_nt[];
 
   int tm, tn;
   if (!live_tile(blockIdx.x, tiles_m, tiles_n, patched, (Mv + NT_BM - 1) / NT_BM, tm, tn)) return;
-  const int m0 = tm * NT_BM, n0 = tn * (PAIR ? NT_BN / 2 : NT_BN);
+  const int m0 = tm * NT_BM, n0 = QKV ? 0 : tn * (PAIR ? NT_BN / 2 : NT_BN);
   if (m0 >= Mv) return;
+  // QKV: a tile is columns first .. + NT_BN / 2 and 32 + first .. of one 64-wide head of the list q | k | v (C's rows of N columns hold q), a wave's two
+  // accumulators the two halves that RoPE turns.
+  const int q_heads = N >> 6, kv_heads = QKV ? qkv.kv_n >> 6 : 0, head = tn / (64 / NT_BN), first = tn % (64 / NT_BN) * (NT_BN / 2);
+  const int which = !QKV || head < q_heads ? 0 : (head < q_heads + kv_heads ? 1 : 2), own = head - (which == 0 ? 0 : q_heads + (which - 1) * kv_heads);
+  if constexpr (QKV) B = (which == 0 ? B : (which == 1 ? qkv.Bk : qkv.Bv)) + (size_t)own * 64 * K;
 
   // The wave's number is uniform, so what depends on it (LDS destinations, the rows it loads) stays
   // in scalar registers.
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave / (4 / WM), wn = wave % (4 / WM);
   const int lrow = lane >> 3, pch = lane & 7;
-  int a_voff[4], b_voff[2], head_ch[4];   // (instruction i of A and of B begin on rows that are 16 i apart or all alike: one swizzle)
+  int a_voff[4], b_voff[2], a_head[4], b_head[2];
 #pragma unroll
   for (int i = 0; i < INST; ++i) {
     const int r = (wave * INST + i) * 8 + lrow;
     const int lch = pch ^ ((r >> 1) & 7);
-    head_ch[i] = lch * 8;
+    a_head[i] = lch * 8;
     // Rows past the end re-read the last row; what they produce is never stored.
     a_voff[i] = (int)(((size_t)(min(m0 + r, M - 1) - m0) * K + lch * 8) * 2);
   }
 #pragma unroll
   for (int i = 0; i < B_INST; ++i) {
     const int r = (wave * B_INST + i) * 8 + lrow;
-    b_voff[i] = (int)(((size_t)(min(n0 + (PAIR ? r % (NT_BN / 2) : r), N - 1) - n0) * K + (pch ^ ((r >> 1) & 7)) * 8) * 2);
+    b_head[i] = (pch ^ ((r >> 1) & 7)) * 8;
+    b_voff[i] = (int)(((size_t)(QKV ? first + (r >> 4 & 1) * 32 + (r >> 5) * 16 + (r & 15) : min(n0 + (PAIR ? r % (NT_BN / 2) : r), N - 1) - n0) * K + b_head[i]) * 2);
   }
   const int pad = k_pad(K);
   const bf16_t* a_tile = A + (size_t)m0 * K - pad;
@@ -468,30 +479,30 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
     if (idx < INST) {
       const __amdgpu_buffer_rsrc_t rows = stage_rows(a_tile + k0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, IRON_LDS_PTR(st + (wave * INST + idx) * 1024), 16,
-                                               head && head_ch[idx] < pad ? NOWHERE : a_voff[idx], 0, 0, 0);
+                                               head && a_head[idx] < pad ? NOWHERE : a_voff[idx], 0, 0, 0);
     } else {
       const __amdgpu_buffer_rsrc_t rows = stage_rows(b_tile + k0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, IRON_LDS_PTR(st + b_first + (idx - INST) * 1024),
-                                               16, head && head_ch[idx - INST] < pad ? NOWHERE : b_voff[idx - INST], 0, 0, 0);
+                                               16, head && b_head[idx - INST] < pad ? NOWHERE : b_voff[idx - INST], 0, 0, 0);
     }
   };
 
-  f32x4 acc[MI][2];
+  f32x4 acc[MI][NJ];
 #pragma unroll
-  for (int t = 0; t < 2 * MI; ++t) acc[t >> 1][t & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < NJ * MI; ++t) acc[t / NJ][t % NJ] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // acc[i][j][e]: row 16 i + fr of the wave's 16 MI x 32, column 16 j + 4 kq + e.
+  // acc[i][j][e]: row 16 i + fr of the wave's 16 MI x 16 NJ, column 16 j + 4 kq + e.
   const int fr = lane & 15, kq = lane >> 4;
-  const int mb = m0 + wm * (16 * MI) + fr, nb = n0 + (PAIR ? 0 : wn * 32) + 4 * kq;
+  const int mb = m0 + wm * (16 * MI) + fr, nb = n0 + (PAIR ? 0 : wn * (16 * NJ)) + 4 * kq;
   // A residual's pieces this lane will add in the epilogue are requested now, so that their
   // latency passes under the whole product instead of at its end (N a multiple of 4: 8-byte pieces).
-  uint2 res[MI][2];
-  const bool res_ahead = !PAIR && qkv.residual != nullptr && (N & 3) == 0;
+  uint2 res[MI][NJ];
+  const bool res_ahead = !PAIR && !QKV && qkv.residual != nullptr && (N & 3) == 0;
   if (res_ahead) {
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < NJ; ++j)
         res[i][j] = *reinterpret_cast<const uint2*>(qkv.residual + (size_t)min(mb + 16 * i, M - 1) * N + min(nb + 16 * j, N - 4));
   }
 
@@ -504,7 +515,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
     for (int idx = 0; idx < LOADS; ++idx) issue_one(smem_nt + s * NT_STAGE_BYTES, min(s, nk - 1), idx, s == 0);
 
   // Fragments: lane -> row fr of a 16-row tile, 16-byte chunk kq of the k-step's four.
-  const int a_off = (wm * (16 * MI) + fr) * 128, b_off = NT_A_BYTES + (wn * 32 + fr) * 128, swz = (fr >> 1) & 7;
+  const int a_off = (wm * (16 * MI) + fr) * 128, b_off = NT_A_BYTES + (wn * (16 * NJ) + fr) * 128, swz = (fr >> 1) & 7;
   auto a_frag = [&](const char* st, int ks, int i) {
     return *reinterpret_cast<const bf16x8*>(st + a_off + i * 16 * 128 + (((ks * 4 + kq) ^ swz) << 4));
   };
@@ -514,11 +525,13 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
 
   wait_vmcnt<(STAGES - 2) * LOADS>();   // stage 0 has landed once only the younger ones are out
   block_barrier();
-  bf16x8 af[2][2][MI], bfr[2][2][2];   // [stage parity][k-step][tile]
+  bf16x8 af[2][2][MI], bfr[2][2][NJ];   // [stage parity][k-step][tile]
 #pragma unroll
   for (int t = 0; t < 2 * MI; ++t) {
     af[0][t / MI][t % MI] = a_frag(smem_nt, t / MI, t % MI);
-    if (t % MI < 2) bfr[0][t / MI][t % MI] = b_frag(smem_nt, t / MI, t % MI);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      if (j % MI == t % MI) bfr[0][t / MI][j] = b_frag(smem_nt, t / MI, j);
   }
   // Two stages an iteration, so that the register sets are named at compile time.
   auto stage = [&](int kt, auto parity) {
@@ -529,8 +542,8 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
 #pragma unroll
     for (int t = 0; t < 2 * MI; ++t) {
       const int ks = t / MI, i = t % MI;
-      mfma_16x16x32_in_place(acc[i][0], bfr[P][ks][0], af[P][ks][i]);
-      mfma_16x16x32_in_place(acc[i][1], bfr[P][ks][1], af[P][ks][i]);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) mfma_16x16x32_in_place(acc[i][j], bfr[P][ks][j], af[P][ks][i]);
       __builtin_amdgcn_sched_barrier(0);
       if (t == 0) {   // (behind the first products, which the waves wait under: 300 x 512 x 2048 8.1 -> 7.8 us)
         // Of this wave's loads in flight the oldest LOADS are stage kt+1's; the STAGES-3 stages after it may stay out.
@@ -539,8 +552,11 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
         __builtin_amdgcn_sched_barrier(0);
       }
       af[P ^ 1][ks][i] = a_frag(st1, ks, i);
-      if (i < 2) bfr[P ^ 1][ks][i] = b_frag(st1, ks, i);
-      if (t < LOADS) issue_one(nst, kn, t, false);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        if (j % MI == i) bfr[P ^ 1][ks][j] = b_frag(st1, ks, j);
+#pragma unroll
+      for (int idx = t * PER; idx < t * PER + PER && idx < LOADS; ++idx) issue_one(nst, kn, idx, false);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -557,7 +573,30 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
   // (the matrix cores' last results: the compiler does not know what the assembly's are)
   asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");
 #pragma unroll
-  for (int t = 0; t < 2 * MI; ++t) asm volatile("" : "+a"(acc[t >> 1][t & 1]));
+  for (int t = 0; t < NJ * MI; ++t) asm volatile("" : "+a"(acc[t / NJ][t % NJ]));
+  if constexpr (QKV) {
+    const int row_len = which == 0 ? N : qkv.kv_n, c = first + wn * 16 + 4 * kq;   // ... of the head's first half
+    bf16_t* to = (which == 0 ? C : (which == 1 ? qkv.Ck : qkv.Cv)) + own * 64 + c;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const int m = mb + 16 * i;
+      if (m >= Mv) continue;
+      if (which < 2) {   // rounded as the projection would store them, turned, rounded again
+        float cs[8];
+        unpack8(*reinterpret_cast<const uint4*>(qkv.angles + (size_t)m * 64 + 2 * c), cs);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float x1 = round_bf16(acc[i][0][e]), x2 = round_bf16(acc[i][NJ - 1][e]);
+          acc[i][0][e] = x1 * cs[2 * e] - x2 * cs[2 * e + 1];
+          acc[i][NJ - 1][e] = x2 * cs[2 * e] + x1 * cs[2 * e + 1];
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        store_loose(to + (size_t)m * row_len + 32 * j, pack_bf16(acc[i][j][0], acc[i][j][1]), pack_bf16(acc[i][j][2], acc[i][j][3]));
+    }
+    return;
+  }
   if constexpr (PAIR) {
     // The gate's waves leave their product, rounded as it is stored, in LDS for the others and store it; those make
     // bf16(bf16(act(bf16 g)) * bf16 u) of it.
@@ -587,7 +626,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
       if (m >= Mv) continue;
       bf16_t* row = C + (size_t)m * N;
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < NJ; ++j) {
         const int n = nb + 16 * j;
         if (n >= N) continue;
         if constexpr (decltype(residual)::value) {   // the product rounded as it would be stored, then scale * it + residual
@@ -1311,11 +1350,15 @@ __global__ __launch_bounds__(256) void qkv_either_kernel(const bf16_t* __restric
                                                          int M, int heads, int kv_heads, int K,
                                                          const int* __restrict__ valid, Tiling narrow, Tiling wide,
                                                          Tiling thin, int above, int wide_top, int thin_upto,
-                                                         QkvTail qkv) {
+                                                         int half_upto, int low_upto, QkvTail qkv) {
   const int Mv = bound_or(valid, M);
   const bool past = Mv > above;
   to_cache_rows(qkv, valid, M);
-  if (Mv <= thin_upto) {   // so few rows that one-head tiles still fit one round over the chip
+  if (Mv <= half_upto) {   // ... or half-head ones of 64 rows
+    gemm_nt64_body<10, false, 1, 4, 2, true>(A, Bq, Cq, M, heads * 64, K, Mv, (M + 63) / 64, (heads + 2 * kv_heads) * 2, 0, qkv);
+  } else if (Mv <= low_upto) {
+    gemm_nt64_body<8, false, 2, 2, 2, true>(A, Bq, Cq, M, heads * 64, K, Mv, (M + 63) / 64, heads + 2 * kv_heads, 0, qkv);
+  } else if (Mv <= thin_upto) {   // so few rows that one-head tiles still fit one round over the chip
     if ((int)blockIdx.x < thin.tiles_m * thin.tiles_n)
       qkv_heads_body<1>(A, Bq, Cq, M, heads, kv_heads, K, valid, thin.tiles_m, thin.tiles_n, thin.patched, qkv);
   } else if (wide.tiles_n > 0 && past == (wide_top != 0)) {
@@ -1331,6 +1374,10 @@ static int patched_order(int tiles_m, int tiles_n) {
   return (tiles_m % 8 == 0 && tiles_n % 4 == 0 && ((tiles_m / 8) * (tiles_n / 4)) % 8 == 0) ? 1 : 0;
 }
 
+// The rows up to which 64-row tiles of `columns` (a whole head's 64 or 32, q | k | v of `total` heads) are one round over the chip: few rows wait
+// for what a CU draws, so a tile of fewer operand rows is the faster one as long as each has a CU of its own.  Hidden 2048, 32 + 8 + 8 heads,
+// weights out of memory, us by 128 x 64 tiles and by these: 8 rows 15.8 / 10.0, 45 15.9 / 10.1, 128 16.5 / 10.2, 200 16.2 / 12.4, 320 16.4 / 13.0.
+static int few_qkv_rows(int total, int K, int columns) { return K < 8 * BK ? 0 : 256 / (total * 64 / columns) * 64; }
 // wide_ok: the head count comes in threes (else the 192-wide tiling is never chosen).  thin_upto: the
 // row bound up to which the one-head tiles run (0: never).
 static int launch_qkv_either(const bf16_t* A, const bf16_t* Bq, bf16_t* Cq, int M, int heads, int kv_heads, int K,
@@ -1350,8 +1397,10 @@ static int launch_qkv_either(const bf16_t* A, const bf16_t* Bq, bf16_t* Cq, int 
   }
   int blocks = tiles_m * (narrow.tiles_n > wide.tiles_n ? narrow.tiles_n : wide.tiles_n);
   if (thin.tiles_m * thin.tiles_n > blocks) blocks = thin.tiles_m * thin.tiles_n;
+  const int half_upto = few_qkv_rows(total, K, 32), low_upto = few_qkv_rows(total, K, 64);
+  if (blocks < 256 && low_upto > 0) blocks = 256;
   hipLaunchKernelGGL(qkv_either_kernel, dim3(blocks), dim3(256), lds, s, A, Bq, Cq, M, heads, kv_heads, K, valid, narrow,
-                     wide, thin, above, wide_top ? 1 : 0, thin_upto, qkv);
+                     wide, thin, above, wide_top ? 1 : 0, thin_upto, half_upto, low_upto, qkv);
   IRON_LAUNCH_CHECK();
 }
 
@@ -1855,27 +1904,28 @@ static FormTable form_table(int M, Best best, int* upto) {
 // them and a block past its tiling's tiles leaves at once.  LDS is the largest tiling's, so a CU
 // holds one block whatever the choice, and four waves are a block whatever the stand-alone launch of a form uses.
 // The prices: rounds of blocks, as big_form, at what a round was measured to take with weights out of memory behind the launch's own 4.5 us (by 64 x 64,
-// 128 x 128 and 256 x 256 tiles alone and by these, us: 2048 columns over 2048 with a residual, 640 rows 19.9 / 17.7, 1024 23.7 / 18.4; over 8192, 900
+// 128 x 128 and 256 x 256 tiles alone and by all these, us: 2048 columns over 2048 with a residual, 640 rows 19.9 / 17.7, 1024 23.7 / 18.4; over 8192, 900
 // rows 68 / 52; 8192 over 2048, 256 rows 22.9 / 18.6, 640 42 / 26, 1024 43 / 34, 1280 50 / 39; 6144 over 2048, 1200 rows 54 / 32).
-enum RowsForm { ROWS_64X64, ROWS_128X64, ROWS_128X128, ROWS_160X128, ROWS_192X128, ROWS_256X128, ROWS_160X256, ROWS_192X256, ROWS_256X256, ROWS_FORMS };
+enum RowsForm { ROWS_32X32, ROWS_64X32, ROWS_64X64, ROWS_128X64, ROWS_128X128, ROWS_160X128, ROWS_192X128, ROWS_256X128, ROWS_160X256, ROWS_192X256, ROWS_256X256, ROWS_FORMS };
 struct RowsPrice {
   int bm, bn;
   float start, stage;
 };
 constexpr RowsPrice ROWS_PRICES[ROWS_FORMS] = {
-    {64, 64, 0.8f, 0.28f},   {128, 64, 2.f, 0.34f},   {128, 128, 4.f, 0.45f}, {160, 128, 3.4f, 0.52f}, {192, 128, 5.f, 0.57f},
+    {32, 32, 0.8f, 0.15f},   {64, 32, 0.8f, 0.2f},    {64, 64, 0.8f, 0.28f},   {128, 64, 2.f, 0.34f},   {128, 128, 4.f, 0.45f}, {160, 128, 3.4f, 0.52f}, {192, 128, 5.f, 0.57f},
     {256, 128, 6.5f, 0.69f}, {160, 256, 8.f, 0.8f},   {192, 256, 9.f, 0.85f}, {256, 256, 15.f, 1.f},
 };
 // `whole`: the output's rows are pieces of 8 or the product has no second operand.
 static RowsForm rows_form(int rows, int M, int N, int K, bool whole) {
-  RowsForm best = ROWS_64X64;
+  const RowsForm first = K < 8 * BK ? ROWS_64X64 : ROWS_32X32;   // (a short K does not fill the small tiles' many stages)
+  RowsForm best = first;
   float price = 0.f;
-  for (int form = ROWS_64X64; form < ROWS_FORMS; ++form) {
+  for (int form = first; form < ROWS_FORMS; ++form) {
     const RowsPrice& p = ROWS_PRICES[form];
     if (form > ROWS_128X128 && (M < p.bm || N < p.bn || !whole)) continue;
     const long tiles = (long)((rows + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
     const float us = (float)((tiles + 255) / 256) * (p.start + p.stage * ((K + BK - 1) / BK));
-    if (form == ROWS_64X64 || us < price) best = (RowsForm)form, price = us;
+    if (form == first || us < price) best = (RowsForm)form, price = us;
   }
   return best;
 }
@@ -1903,8 +1953,14 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const bf16_t* __restrict
     case ROWS_128X64:
       gemm_nt64_body<5, false, 4>(A, B, C, M, N, K, Mv, (M + 127) / 128, (N + 63) / 64, patched, tail);
       break;
-    default:
+    case ROWS_64X64:
       gemm_nt64_body<8>(A, B, C, M, N, K, Mv, (M + 63) / 64, (N + 63) / 64, patched, tail);
+      break;
+    case ROWS_64X32:
+      gemm_nt64_body<13, false, 1, 4>(A, B, C, M, N, K, Mv, (M + 63) / 64, (N + 31) / 32, patched, tail);
+      break;
+    default:
+      gemm_nt64_body<20, false, 1, 2, 1>(A, B, C, M, N, K, Mv, (M + 31) / 32, (N + 31) / 32, patched, tail);
   }
 #undef IRON_ROWS
 }
@@ -2869,13 +2925,13 @@ static int prefill_qkv(const uint16_t* x, const uint16_t* Wq, const uint16_t* Wk
   int thin_upto = 0;
   for (int live = 128; live <= ((rows + 127) / 128) * 128; live += 128)
     if (thin_wins(live)) thin_upto = live;
-  if (thin_upto >= rows) return launch_qkv64(x, Wq, q_out, rows, heads, kv_heads, hidden, valid, s, tail);
+  if (thin_upto >= rows && (valid == nullptr ? rows : 1) > few_qkv_rows(total, hidden, 64)) return launch_qkv64(x, Wq, q_out, rows, heads, kv_heads, hidden, valid, s, tail);
   // The bound above which the winner at `rows` wins, if the two ever change places below `rows`.
   int above = -1;
   if (valid != nullptr)
     for (int live = 128; live <= rows; live += 128)
       if (wide_wins(live) != wide_wins(rows)) above = live;
-  if (valid == nullptr) thin_upto = 0;
+  if (valid == nullptr && rows > few_qkv_rows(total, hidden, 64)) thin_upto = 0;
   if (above < 0 && thin_upto == 0) {
     if (wide_wins(rows)) return launch_qkv192(x, Wq, q_out, rows, heads, kv_heads, hidden, valid, s, tail);
     return launch_gemm_nt<false, true>(x, Wq, q_out, rows, heads * d, hidden, valid, s, tail);

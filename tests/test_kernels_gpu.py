@@ -403,6 +403,7 @@ def test_gemm_rows_of_every_alignment(cuda, M, Kdim, N, b_col_maj, c_col_maj, co
     (2000, 136, 8195, True, (130, 257, 513, 641, 769, 1025, 1281, 1537, 1999)),   # every form by the bound, the last tiles moved back
     (2048, 200, 8192, True, (1, 128, 129, 1024, 1025, 2047)),    # 64, 128 and 256 tiles by the bound
     (1500, 328, 2056, True, (63, 895, 896, 897, 1500)),          # 64 and 128 ones, ragged
+    (2048, 1032, 2056, True, (1, 32, 33, 65, 128, 129, 200, 257, 400)), (300, 584, 200, True, (31, 64, 97, 299)),   # 32-column ones, ragged
     (256, 136, 320, True, (0, 100, 200)), (40, 1000, 4168, True, (17, 40)), (33, 4096, 520, True, (1, 32)),   # 64 ones whatever the bound
     (2048, 328, 2056, False, (1, 129, 1999)), (300, 200, 136, False, (299,)), (40, 264, 72, False, (17,)),    # (K,N): the last column tile moved back
     (64, 72, 128, False, (5,)), (2, 192, 4104, False, (1,))])
@@ -454,7 +455,7 @@ def test_a_row_s_products_are_the_same_bits_under_every_bound(cuda, M, Kdim, N, 
         return C, G
 
     whole = run(M)
-    for rows in (5, 64, 128, 129, 256, 257, 384, 385, 513, 896, 897, 1025, 1281):
+    for rows in (5, 32, 33, 64, 65, 128, 129, 256, 257, 384, 385, 513, 896, 897, 1025, 1281):
         for got, want in zip(run(rows), whole):
             assert torch.equal(got[:rows], want[:rows]), rows
             assert (got[rows:] == 7).all(), rows
@@ -464,6 +465,8 @@ def test_a_row_s_products_are_the_same_bits_under_every_bound(cuda, M, Kdim, N, 
                                             # bounds on either side of where the 192-wide tiles take over
                                             (2048, 1280, 32, 8), (2048, 1281, 32, 8), (2048, 1999, 32, 8),
                                             (2048, 2048, 32, 8), (2048, 70, 32, 8),
+                                            # ... and of 64-row tiles' half and whole heads
+                                            (2048, 1, 32, 8), (2048, 129, 32, 8), (2048, 320, 32, 8), (2048, 321, 32, 8), (256, 31, 16, 4), (130, None, 4, 2),
                                             # heads that do not come in threes keep the 128-wide tiles
                                             (2048, None, 32, 4), (1024, None, 8, 2), (4096, 3000, 16, 4)])
 def test_prefill_qkv_equals_three_projections_then_rope(cuda, rows, bound, H, G):
@@ -488,11 +491,11 @@ def test_prefill_qkv_equals_three_projections_then_rope(cuda, rows, bound, H, G)
         assert np.all(got[lim:] == 7.0)
 
 
-@pytest.mark.parametrize("E", [64, 192, 320])
-@pytest.mark.parametrize("rows,bound", [(512, None), (2048, 600)])
+@pytest.mark.parametrize("E", [64, 192, 320, 576])
+@pytest.mark.parametrize("rows,bound", [(512, None), (2048, 600), (2048, 100), (2048, 300), (300, None)])
 def test_prefill_qkv_one_head_tiles_at_short_hidden(cuda, E, rows, bound):
     """The one-head tiles a short chunk takes (whole-stage-ahead pipeline, five stages) with fewer
-    k-stages than are in flight and an odd count of them."""
+    k-stages than are in flight and an odd count of them; the 64-row tiles of few rows likewise."""
     rng = np.random.default_rng(E + rows)
     H, G, D = 32, 8, 64
     x = bf(rng, rows, E)
