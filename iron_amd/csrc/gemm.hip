@@ -1097,6 +1097,25 @@ static int launch_gemm_nt(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, in
   IRON_LAUNCH_CHECK();
 }
 
+template <int STAGES, int MI, int WM, int NJ>
+__global__ __launch_bounds__(256) void gemm_small_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, bf16_t* __restrict__ C, int M, int N,
+                                                         int K, int tiles_m, int tiles_n) {
+  gemm_nt64_body<STAGES, false, MI, WM, NJ>(A, B, C, M, N, K, M, tiles_m, tiles_n, 0, QkvTail{});
+}
+template <int STAGES, int MI, int WM, int NJ>
+static int launch_gemm_small(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s) {
+  constexpr int BM = 16 * MI * WM, BN = 16 * NJ * (4 / WM);
+  constexpr size_t lds = (size_t)STAGES * (BM + BN) * BK * 2;
+  static LdsOptIn opt_in;
+  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_small_kernel<STAGES, MI, WM, NJ>), lds); e != hipSuccess) {
+    set_error("gemm: %s", hipGetErrorString(e));
+    return (int)e;
+  }
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  hipLaunchKernelGGL((gemm_small_kernel<STAGES, MI, WM, NJ>), dim3(tiles_m * tiles_n), dim3(256), lds, s, A, B, C, M, N, K, tiles_m, tiles_n);
+  IRON_LAUNCH_CHECK();
+}
+
 // The fused projections at 128 x 192 tiles: three 64-wide heads of the concatenated q | k | v head
 // list a tile, so a 2048-row chunk of a 32 + 8 + 8-head layer is 16 x 16 = 256 tiles -- one a CU in
 // one round, where 128 x 128 tiles make 384 (a round and a half, run as two).  Four waves stacked
@@ -2645,6 +2664,23 @@ static int check_gemm(const uint16_t* A, const uint16_t* B, const uint16_t* C, i
   return 0;
 }
 
+// Tiles of 32 columns by 32 or 64 rows (rows 0: neither), while they are one round over the chip: a CU then draws a half or three
+// quarters of what it draws for a 64 x 64 tile (see gemm_nt64_body), which is what a product without a full round of those takes; and what they were
+// measured to take (a twentieth off over 270 shapes). us, weights out of memory, by the kernels chosen before and by these: 97 x 711 x 1936 10.9 / 6.8,
+// 250 x 232 x 2584 13.9 / 7.8, 163 x 2113 x 4088 26.1 / 16.4; against shared K 112 x 886 x 2704 18.7 / 9.1, 58 x 411 x 4416 19.5 / 10.4; out of the
+// last-level cache 510 x 331 x 2232 9.3 / 7.1, 41 x 4827 x 3112 21.2 / 11.0. Two stages are too few for them to pay.
+struct SmallTiles {
+  int rows;
+  float us;
+};
+static SmallTiles small_tiles(int M, int N, int K) {
+  const long low = (long)((M + 31) / 32) * ((N + 31) / 32), high = (long)((M + 63) / 64) * ((N + 31) / 32);
+  const float stages = (float)((K + BK - 1) / BK);
+  if (K < 3 * BK || high > 256) return {0, 0.f};
+  if (low <= 256) return {32, 3.05f + stages * (0.108f + (K % BK == 0 ? 0.02f : 0.034f) * low / 256)};
+  return {64, 3.2f + stages * (0.14f + 0.035f * high / 256)};
+}
+
 // How a product's 128 x 128 tiles are shared (none: slices 0), M and N as the tiles see them, by what was
 // measured, in us.  Unshared: 3 a launch; a stage of 64 k 0.5 a round of 128 x 128 tiles; on the 64 x 64 tiles
 // that few tiles of B (N,K) take, 0.13 to 0.23 up to a block a CU, and 0.14 (a few blocks) to 0.34 where K is no multiple of 64.
@@ -2679,14 +2715,18 @@ static TileShares gemm_shares_of_tiles(int M, int N, int K, bool b_nk, float* pr
 // 2.6 us and, a thousand of K, what the rows and the rounds of blocks make of it; the tiles 11 and the matrix at 5 TB/s where they are shared,
 // else 3.3 and their chain of stages, dearer where rows straddle cache lines (few rows against tiles: 45 x 1928 x 3192 16.4 / 23.7, 48 x 3992 x 1424
 // 8.5 / 12.4, 63 x 2048 x 6144 28.9 / 32.7, 16 x 4096 x 10192 24.2 / 31.6, but 40 x 2048 x 8192 28.9 / 17.6, 56 x 6000 x 3192 36.4 / 28.0).
+// More than 32 rows give way to tiles of 32 columns that take a good deal less (few rows against those: 34 x 7452 x 2312 19.0 / 11.7, 40 x 3208 x 3744
+// 17.2 / 12.1, 35 x 1828 x 2512 11.2 / 8.3; but 59 x 344 x 480 3.1 / 3.9).
 static bool gemm_of_few_rows(int M, int N, int K) {
   if (M >= 64) return false;
+  const float rows = M <= 16 ? 1.1f + 0.045f * M : 1.55f + 0.0435f * M;
+  const float each = N < 8192 ? rows * ((N + 4095) / 4096) : (M <= 16 ? 3.5f : 4.15f + 0.028f * M);   // (N = 8192: 32 columns a block)
+  const float few = 2.6f + 1e-3f * K * each;
+  if (const SmallTiles small = small_tiles(M, N, K); M > 32 && small.rows > 0 && small.us < 0.72f * few) return false;
   if (M <= 16 && N <= 2048 && K <= 16384 && (long)N * K >= (1 << 21)) return true;
   if ((long)M * K < 140000 && (M < 48 || K < 1408)) return true;
   if (N > 8192 || K < BK) return false;
-  const float rows = M <= 16 ? 1.1f + 0.045f * M : 1.55f + 0.0435f * M;
-  const float each = N < 8192 ? rows * ((N + 4095) / 4096) : (M <= 16 ? 3.5f : 4.15f + 0.028f * M);   // (N = 8192: 32 columns a block)
-  const float stage = K % BK == 0 ? 0.17f + 0.0018f * M : 0.2f + 0.0048f * M, few = 2.6f + 1e-3f * K * each;
+  const float stage = K % BK == 0 ? 0.17f + 0.0018f * M : 0.2f + 0.0048f * M;
   const float tiles = gemm_shares_of_tiles(M, N, K, true).slices > 0 ? 11.f + 4e-7f * N * K : 3.3f + stage * ((K + BK - 1) / BK);
   return 1.05f * few < tiles;
 }
@@ -2734,7 +2774,12 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
       if (valid != nullptr) return launch_gemm_rows(A, B, C, M, N, K, valid, s);
       // 128x128 tiles that would occupy under half the CUs give way to 64x64 ones, and so do tiles that
       // up to 64 rows would half fill at most (64 x 16384 x 8184: 93 -> 68 us).
-      if (tiles128 < 128 || M <= 64) return launch_gemm_nt<false, false, 1>(A, B, C, M, N, K, valid, s);
+      if (tiles128 < 128 || M <= 64) {
+        const SmallTiles small = small_tiles(M, N, K);
+        if (small.rows == 32) return launch_gemm_small<20, 1, 2, 1>(A, B, C, M, N, K, s);
+        if (small.rows == 64) return launch_gemm_small<13, 1, 4, 2>(A, B, C, M, N, K, s);
+        return launch_gemm_nt<false, false, 1>(A, B, C, M, N, K, valid, s);
+      }
       return launch_gemm_nt<false>(A, B, C, M, N, K, valid, s);
     }
     return launch_gemm_nt<true>(A, B, C, M, N, K, valid, s);
@@ -2750,6 +2795,7 @@ static TileShares gemm_shares(int M, int N, int K, bool b_nk, bool c_nm) {
   if (b_nk && gemm_of_few_rows(M, N, K)) return TileShares{0, 0, 0};
   float then = 0.f, big, price128;
   const TileShares deal = gemm_shares_of_tiles(M, N, K, b_nk, &then);
+  if (const SmallTiles small = small_tiles(M, N, K); b_nk && deal.slices > 0 && small.rows > 0 && small.us < 0.78f * then) return TileShares{0, 0, 0};
   // (whole tiles of another size, where they take no more)
   if (deal.slices > 0 && !c_nm && deal.whole + deal.shared >= 128 && big_form(M, N, K, b_nk, big, price128) != BIG_NONE && big + 3.f <= then)
     return TileShares{0, 0, 0};
