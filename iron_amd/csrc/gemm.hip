@@ -419,12 +419,12 @@ constexpr int NOWHERE = (int)0x80000000u;   // past stage_rows' 2^31 - 1 bytes, 
 // An element's sum is the same chain of 32-wide k-steps as in the 128 x 128 and the 256 x 256 tiles: where a row bound chooses
 // the tile, a row's products are the same bits whatever rows share the launch.
 // `qkv` carries only the optional residual epilogue here, or (QKV) the fused projections'.  WM x 4 / WM waves of MI x NJ tiles: <2, 2, 2> are 64 x 64, <4>
-// 128 x 64.  PAIR: both first products of a gated feed-forward, 32 columns of each (`qkv` says the gate's kind).
+// 128 x 64.  PAIR: both first products of a gated feed-forward, 32 columns of each (`qkv` says the gate's kind).  B_KN: B is (K,N), 64 columns a tile.
 // A few rows' tiles wait for what a CU can draw of operands that are 128 bytes of a row here and there, some 60 GB/s of weights out of memory, whatever the
 // stages in flight (8 or 10 of 16 KB the same): where the tiles leave CUs without one, smaller tiles have more CUs draw less each.  2048 columns over 2048
 // with a residual, us by 64 x 64 tiles, 64 x 32 <1, 4, 2> and 32 x 32 <1, 2, 1>: 12.5 / 10.4 / 8.6 (256 blocks: up to 640, 256 and 128 rows); over 8192
 // 36 / 28.7 / 21.3.
-template <int STAGES, bool PAIR = false, int MI = 2, int WM = 2, int NJ = 2, bool QKV = false>
+template <int STAGES, bool PAIR = false, int MI = 2, int WM = 2, int NJ = 2, bool QKV = false, bool B_KN = false>
 __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
                                                bf16_t* __restrict__ C, int M, int N, int K,
                                                int Mv, int tiles_m, int tiles_n,
@@ -434,13 +434,14 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
   constexpr int NT_A_BYTES = NT_BM * BK * 2, NT_STAGE_BYTES = (NT_BM + NT_BN) * BK * 2;
   constexpr int INST = NT_BM / 8 / 4, B_INST = NT_BN / 8 / 4;  // 1 KB loads of A and of B a wave issues per stage
   constexpr int LOADS = INST + B_INST, PER = (LOADS + 2 * MI - 1) / (2 * MI);   // PER: loads behind every second MFMA
-  static_assert(BK == 64 && STAGES >= 4 && ((MI == 2 && WM == 2 && NJ == 2) || !PAIR) && (!QKV || (NJ == 2 && NT_BN <= 64)),
+  static_assert(BK == 64 && STAGES >= 4 && ((MI == 2 && WM == 2 && NJ == 2) || !PAIR) && (!QKV || (NJ == 2 && NT_BN <= 64)) &&
+                    (!B_KN || (NT_BN == 64 && NJ == 2 && !PAIR && !QKV)),
                 "two 32-wide k-steps a stage");
   extern __shared__ __align__(16) char smem_nt[];
 
   int tm, tn;
   if (!live_tile(blockIdx.x, tiles_m, tiles_n, patched, (Mv + NT_BM - 1) / NT_BM, tm, tn)) return;
-  const int m0 = tm * NT_BM, n0 = QKV ? 0 : tn * (PAIR ? NT_BN / 2 : NT_BN);
+  const int m0 = tm * NT_BM, n0 = QKV ? 0 : (B_KN ? max(min(tn * NT_BN, N - NT_BN), 0) : tn * (PAIR ? NT_BN / 2 : NT_BN));
   if (m0 >= Mv) return;
   // QKV: a tile is columns first .. + NT_BN / 2 and 32 + first .. of one 64-wide head of the list q | k | v (C's rows of N columns hold q), a wave's two
   // accumulators the two halves that RoPE turns.
@@ -454,6 +455,8 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
   const int wm = wave / (4 / WM), wn = wave % (4 / WM);
   const int lrow = lane >> 3, pch = lane & 7;
   int a_voff[4], b_voff[2], a_head[4], b_head[2];
+  // (K,N): a row of 64 columns is half the banks; what sixteen lanes' transposing read takes, four rows of 32 bytes, and its neighbours' eight rows on meet none twice.
+  auto kn_swizzle = [](int k) { return (k & 2) | ((k >> 1) & 4); };
 #pragma unroll
   for (int i = 0; i < INST; ++i) {
     const int r = (wave * INST + i) * 8 + lrow;
@@ -465,13 +468,18 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
 #pragma unroll
   for (int i = 0; i < B_INST; ++i) {
     const int r = (wave * B_INST + i) * 8 + lrow;
+    if constexpr (B_KN) {   // as stored, a row a k: 64 columns, the last tile moved back to end at N
+      b_head[i] = r;
+      b_voff[i] = (int)(((size_t)r * N + min((pch ^ kn_swizzle(r)) * 8, N - 8 - n0)) * 2);
+      continue;
+    }
     b_head[i] = (pch ^ ((r >> 1) & 7)) * 8;
     b_voff[i] = (int)(((size_t)(QKV ? first + (r >> 4 & 1) * 32 + (r >> 5) * 16 + (r & 15) : min(n0 + (PAIR ? r % (NT_BN / 2) : r), N - 1) - n0) * K + b_head[i]) * 2);
   }
   const int pad = k_pad(K);
   const bf16_t* a_tile = A + (size_t)m0 * K - pad;
   // (PAIR: the tile's first 32 columns are the gate's, which waves 0 and 1 load and the waves wn = 0 compute, the rest the up projection's)
-  const bf16_t* b_tile = (PAIR && wave >= 2 ? up : B) + (size_t)n0 * K - pad;
+  const bf16_t* b_tile = B_KN ? B + n0 - (ptrdiff_t)pad * N : (PAIR && wave >= 2 ? up : B) + (size_t)n0 * K - pad;
   const int b_first = NT_A_BYTES + wave * B_INST * 1024;   // where a wave's part of B begins in a stage
   // One load of the 2*INST a wave issues per stage (A's first, then B's).
   auto issue_one = [&](char* st, int kt, int idx, bool head) {
@@ -481,7 +489,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, IRON_LDS_PTR(st + (wave * INST + idx) * 1024), 16,
                                                head && a_head[idx] < pad ? NOWHERE : a_voff[idx], 0, 0, 0);
     } else {
-      const __amdgpu_buffer_rsrc_t rows = stage_rows(b_tile + k0);
+      const __amdgpu_buffer_rsrc_t rows = stage_rows(b_tile + (B_KN ? (size_t)k0 * N : (size_t)k0));
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, IRON_LDS_PTR(st + b_first + (idx - INST) * 1024),
                                                16, head && b_head[idx - INST] < pad ? NOWHERE : b_voff[idx - INST], 0, 0, 0);
     }
@@ -526,8 +534,48 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
   wait_vmcnt<(STAGES - 2) * LOADS>();   // stage 0 has landed once only the younger ones are out
   block_barrier();
   bf16x8 af[2][2][MI], bfr[2][2][NJ];   // [stage parity][k-step][tile]
+  // (K,N): reads that the compiler does not count, A's too, so that every wait is this code's own (as in the 128 x 128 tiles).
+  TrFrag tfb[2][2][NJ];
+  const unsigned lds_base = (unsigned)(size_t)IRON_LDS_PTR(smem_nt);
+  unsigned a_lane[2], kn_lane[NJ];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) a_lane[ks] = lds_base + a_off + (((ks * 4 + kq) ^ swz) << 4);
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int k = 8 * kq + ((lane & 15) >> 2), n = wn * (16 * NJ) + j * 16 + 4 * (lane & 3);
+    kn_lane[j] = lds_base + NT_A_BYTES + k * 128 + (((n >> 3) ^ kn_swizzle(k)) << 4) + ((n & 4) << 1);
+  }
+  auto kn_reads = [&](unsigned at, int parity, int ks, int i) {   // at: the stage's place; what slot (ks, i) reads
+    if (i == 0) af[parity][ks][0] = lds_read_b128_at<0>(a_lane[ks] + at);
+    else af[parity][ks][MI - 1] = lds_read_b128_at<(MI - 1) * 16 * 128>(a_lane[ks] + at);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      if (j % MI == i) {
+        TrFrag& t = tfb[parity][ks][j];
+        if (ks == 0) {
+          t.lo = lds_read_tr16_at<0>(kn_lane[j] + at);
+          t.hi = lds_read_tr16_at<4 * 128>(kn_lane[j] + at);
+        } else {
+          t.lo = lds_read_tr16_at<32 * 128>(kn_lane[j] + at);
+          t.hi = lds_read_tr16_at<36 * 128>(kn_lane[j] + at);
+        }
+      }
+  };
+  // A k-step's fragments are there once at most the next k-step's are outstanding.
+  auto kn_wait = [&](int parity, int ks) {
+    asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(tfb[parity][ks][0].lo), "+v"(tfb[parity][ks][0].hi), "+v"(tfb[parity][ks][NJ - 1].lo), "+v"(tfb[parity][ks][NJ - 1].hi) : "n"(MI + 2 * NJ));
+#pragma unroll
+    for (int i = 0; i < MI; ++i) lds_wait_for<MI + 2 * NJ>(af[parity][ks][i]);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) bfr[parity][ks][j] = tr_join(tfb[parity][ks][j]);
+  };
+  static_assert(!B_KN || MI <= 2, "two rows of tiles a wave");
 #pragma unroll
   for (int t = 0; t < 2 * MI; ++t) {
+    if constexpr (B_KN) {
+      kn_reads(0, 0, t / MI, t % MI);
+      continue;
+    }
     af[0][t / MI][t % MI] = a_frag(smem_nt, t / MI, t % MI);
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
@@ -542,6 +590,10 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
 #pragma unroll
     for (int t = 0; t < 2 * MI; ++t) {
       const int ks = t / MI, i = t % MI;
+      if constexpr (B_KN) {
+        if (i == 0) kn_wait(P, ks);
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
       for (int j = 0; j < NJ; ++j) mfma_16x16x32_in_place(acc[i][j], bfr[P][ks][j], af[P][ks][i]);
       __builtin_amdgcn_sched_barrier(0);
@@ -551,10 +603,15 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
         block_barrier();
         __builtin_amdgcn_sched_barrier(0);
       }
-      af[P ^ 1][ks][i] = a_frag(st1, ks, i);
+      if constexpr (B_KN) {
+        kn_reads((unsigned)(st1 - smem_nt), P ^ 1, ks, i);
+        __builtin_amdgcn_sched_barrier(0);
+      } else {
+        af[P ^ 1][ks][i] = a_frag(st1, ks, i);
 #pragma unroll
-      for (int j = 0; j < NJ; ++j)
-        if (j % MI == i) bfr[P ^ 1][ks][j] = b_frag(st1, ks, j);
+        for (int j = 0; j < NJ; ++j)
+          if (j % MI == i) bfr[P ^ 1][ks][j] = b_frag(st1, ks, j);
+      }
 #pragma unroll
       for (int idx = t * PER; idx < t * PER + PER && idx < LOADS; ++idx) issue_one(nst, kn, idx, false);
     }
@@ -569,6 +626,16 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
   }
   if (kt < nk) stage(kt, std::integral_constant<int, 0>{});
 
+  if constexpr (B_KN) {   // the fragments read past the end, before their registers are given away
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        lds_tr_wait(tfb[p][ks][0], tfb[p][ks][NJ - 1]);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) lds_wait_for<0>(af[p][ks][i]);
+      }
+  }
   wait_vmcnt<0>();  // the idle fetches of the last iterations land before the block's LDS is released
   // (the matrix cores' last results: the compiler does not know what the assembly's are)
   asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");
@@ -1097,22 +1164,22 @@ static int launch_gemm_nt(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, in
   IRON_LAUNCH_CHECK();
 }
 
-template <int STAGES, int MI, int WM, int NJ>
+template <int STAGES, int MI, int WM, int NJ, bool B_KN = false>
 __global__ __launch_bounds__(256) void gemm_small_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, bf16_t* __restrict__ C, int M, int N,
                                                          int K, int tiles_m, int tiles_n) {
-  gemm_nt64_body<STAGES, false, MI, WM, NJ>(A, B, C, M, N, K, M, tiles_m, tiles_n, 0, QkvTail{});
+  gemm_nt64_body<STAGES, false, MI, WM, NJ, false, B_KN>(A, B, C, M, N, K, M, tiles_m, tiles_n, 0, QkvTail{});
 }
-template <int STAGES, int MI, int WM, int NJ>
+template <int STAGES, int MI, int WM, int NJ, bool B_KN = false>
 static int launch_gemm_small(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s) {
   constexpr int BM = 16 * MI * WM, BN = 16 * NJ * (4 / WM);
   constexpr size_t lds = (size_t)STAGES * (BM + BN) * BK * 2;
   static LdsOptIn opt_in;
-  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_small_kernel<STAGES, MI, WM, NJ>), lds); e != hipSuccess) {
+  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_small_kernel<STAGES, MI, WM, NJ, B_KN>), lds); e != hipSuccess) {
     set_error("gemm: %s", hipGetErrorString(e));
     return (int)e;
   }
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  hipLaunchKernelGGL((gemm_small_kernel<STAGES, MI, WM, NJ>), dim3(tiles_m * tiles_n), dim3(256), lds, s, A, B, C, M, N, K, tiles_m, tiles_n);
+  hipLaunchKernelGGL((gemm_small_kernel<STAGES, MI, WM, NJ, B_KN>), dim3(tiles_m * tiles_n), dim3(256), lds, s, A, B, C, M, N, K, tiles_m, tiles_n);
   IRON_LAUNCH_CHECK();
 }
 
@@ -2664,19 +2731,24 @@ static int check_gemm(const uint16_t* A, const uint16_t* B, const uint16_t* C, i
   return 0;
 }
 
-// Tiles of 32 columns by 32 or 64 rows (rows 0: neither), while they are one round over the chip: a CU then draws a half or three
+// Tiles of 32 columns (B (N,K)) by 32 or 64 rows (rows 0: neither), while they are one round over the chip: a CU then draws a half or three
 // quarters of what it draws for a 64 x 64 tile (see gemm_nt64_body), which is what a product without a full round of those takes; and what they were
 // measured to take (a twentieth off over 270 shapes). us, weights out of memory, by the kernels chosen before and by these: 97 x 711 x 1936 10.9 / 6.8,
 // 250 x 232 x 2584 13.9 / 7.8, 163 x 2113 x 4088 26.1 / 16.4; against shared K 112 x 886 x 2704 18.7 / 9.1, 58 x 411 x 4416 19.5 / 10.4; out of the
 // last-level cache 510 x 331 x 2232 9.3 / 7.1, 41 x 4827 x 3112 21.2 / 11.0. Two stages are too few for them to pay.
+// With B (K,N) the columns are 64, a cache line of a row of B; 128 x 128 tiles and those: 521 x 416 x 1320 12.3 / 7.5, 50 x 6672 x 1880 21.6 / 13.1,
+// 130 x 88 x 1008 8.9 / 5.8; a long K shared stays so, 135 x 440 x 8096 14.8 / 36.
 struct SmallTiles {
   int rows;
   float us;
 };
-static SmallTiles small_tiles(int M, int N, int K) {
-  const long low = (long)((M + 31) / 32) * ((N + 31) / 32), high = (long)((M + 63) / 64) * ((N + 31) / 32);
+static SmallTiles small_tiles(int M, int N, int K, bool b_nk) {
+  const int columns = b_nk ? 32 : 64;
+  const long low = (long)((M + 31) / 32) * ((N + columns - 1) / columns), high = (long)((M + 63) / 64) * ((N + columns - 1) / columns);
   const float stages = (float)((K + BK - 1) / BK);
   if (K < 3 * BK || high > 256) return {0, 0.f};
+  if (!b_nk && low <= 256) return {32, 3.f + stages * (0.165f + 0.02f * low / 256)};
+  if (!b_nk) return {64, 3.2f + stages * (0.19f + 0.02f * high / 256)};
   if (low <= 256) return {32, 3.05f + stages * (0.108f + (K % BK == 0 ? 0.02f : 0.034f) * low / 256)};
   return {64, 3.2f + stages * (0.14f + 0.035f * high / 256)};
 }
@@ -2722,7 +2794,7 @@ static bool gemm_of_few_rows(int M, int N, int K) {
   const float rows = M <= 16 ? 1.1f + 0.045f * M : 1.55f + 0.0435f * M;
   const float each = N < 8192 ? rows * ((N + 4095) / 4096) : (M <= 16 ? 3.5f : 4.15f + 0.028f * M);   // (N = 8192: 32 columns a block)
   const float few = 2.6f + 1e-3f * K * each;
-  if (const SmallTiles small = small_tiles(M, N, K); M > 32 && small.rows > 0 && small.us < 0.72f * few) return false;
+  if (const SmallTiles small = small_tiles(M, N, K, true); M > 32 && small.rows > 0 && small.us < 0.72f * few) return false;
   if (M <= 16 && N <= 2048 && K <= 16384 && (long)N * K >= (1 << 21)) return true;
   if ((long)M * K < 140000 && (M < 48 || K < 1408)) return true;
   if (N > 8192 || K < BK) return false;
@@ -2775,12 +2847,17 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
       // 128x128 tiles that would occupy under half the CUs give way to 64x64 ones, and so do tiles that
       // up to 64 rows would half fill at most (64 x 16384 x 8184: 93 -> 68 us).
       if (tiles128 < 128 || M <= 64) {
-        const SmallTiles small = small_tiles(M, N, K);
+        const SmallTiles small = small_tiles(M, N, K, true);
         if (small.rows == 32) return launch_gemm_small<20, 1, 2, 1>(A, B, C, M, N, K, s);
         if (small.rows == 64) return launch_gemm_small<13, 1, 4, 2>(A, B, C, M, N, K, s);
         return launch_gemm_nt<false, false, 1>(A, B, C, M, N, K, valid, s);
       }
       return launch_gemm_nt<false>(A, B, C, M, N, K, valid, s);
+    }
+    if (valid == nullptr && tiles128 < 128) {
+      const SmallTiles small = small_tiles(M, N, K, false);
+      if (small.rows == 32) return launch_gemm_small<13, 1, 2, 2, true>(A, B, C, M, N, K, s);
+      if (small.rows == 64) return launch_gemm_small<10, 2, 2, 2, true>(A, B, C, M, N, K, s);
     }
     return launch_gemm_nt<true>(A, B, C, M, N, K, valid, s);
   }
@@ -2795,7 +2872,8 @@ static TileShares gemm_shares(int M, int N, int K, bool b_nk, bool c_nm) {
   if (b_nk && gemm_of_few_rows(M, N, K)) return TileShares{0, 0, 0};
   float then = 0.f, big, price128;
   const TileShares deal = gemm_shares_of_tiles(M, N, K, b_nk, &then);
-  if (const SmallTiles small = small_tiles(M, N, K); b_nk && deal.slices > 0 && small.rows > 0 && small.us < 0.78f * then) return TileShares{0, 0, 0};
+  if (const SmallTiles small = small_tiles(M, N, K, b_nk); !c_nm && deal.slices > 0 && small.rows > 0 && small.us < (b_nk || N % BK == 0 ? 0.78f : 0.68f) * then)
+    return TileShares{0, 0, 0};   // (rows of B (K,N) that straddle cache lines cost the small tiles more, out of memory: 30 x 2776 x 3248 shared 16.1, by those 21.0)
   // (whole tiles of another size, where they take no more)
   if (deal.slices > 0 && !c_nm && deal.whole + deal.shared >= 128 && big_form(M, N, K, b_nk, big, price128) != BIG_NONE && big + 3.f <= then)
     return TileShares{0, 0, 0};

@@ -293,8 +293,9 @@ def test_gemm_weight_layout_fast_paths(cuda, M, Kdim, N, rows):
     assert np.all(got[lim:] == 5.0)
 
 
-# (the first six: tiles of 32 columns by 32 and by 64 rows, a single round of them and one tile, K of three stages and more, whole and ragged)
-@pytest.mark.parametrize("M,Kdim,N", [(97, 192, 65), (65, 200, 2042), (510, 1096, 333), (1000, 576, 509), (33, 4160, 2000), (129, 2344, 1364), (130, 128, 264), (200, 192, 136), (1000, 256, 1000), (65, 64, 65), (2047, 320, 2050), (333, 128, 384)])
+# (the first eight: tiles of 32 or 64 columns by 32 and by 64 rows, a single round of them and one tile, K of three stages and more, whole and ragged)
+@pytest.mark.parametrize("M,Kdim,N", [(97, 192, 65), (65, 200, 2042), (510, 1096, 333), (1000, 576, 509), (33, 4160, 2000), (129, 2344, 1364), (1000, 584, 640), (70, 264, 24),
+                                       (130, 128, 264), (200, 192, 136), (1000, 256, 1000), (65, 64, 65), (2047, 320, 2050), (333, 128, 384)])
 @pytest.mark.parametrize("b_col_maj", [False, True])
 def test_gemm_direct_to_lds_tiles_at_ragged_edges(cuda, M, Kdim, N, b_col_maj):
     """K a multiple of 64 takes the direct-to-LDS tiles whatever M and N are: rows and columns past
