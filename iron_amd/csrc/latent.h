@@ -30,9 +30,10 @@ __device__ __forceinline__ void latent_row(const T* __restrict__ xr, const Laten
   float f[CH][8], gain[CH][8], qs = 0.f, cs = 0.f;
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
-    const int e = t + 256 * i;
-    if (e < n) load_vec<8>(xr + e * 8, f[i]);
-    if (e < cn) load_vec<8>(QUERY && e < qn ? g.q_gain + e * 8 : g.c_gain + (e - qn) * 8, gain[i]);
+    // (the last piece again past the end: behind a test each load would be waited for by itself)
+    const int e = min(t + 256 * i, n - 1), ge = min(e, cn - 1);
+    load_vec<8>(xr + e * 8, f[i]);
+    load_vec<8>(QUERY && ge < qn ? g.q_gain + ge * 8 : g.c_gain + (ge - qn) * 8, gain[i]);
   }
 #pragma unroll
   for (int i = 0; i < CH; ++i) {

@@ -105,13 +105,9 @@ __global__ __launch_bounds__(256) void latent_rows_wide_kernel(const T* __restri
                                                                T* __restrict__ shared_keys, LatentShape a, int stride) {
   __shared__ float part[2][4];
   const int row = blockIdx.x;
-  for (int slot = 0; slot < a.slots; ++slot) {
-    const Span s = span_of(spans, slot, a.rows);
-    if (row >= s.row0 && row < s.row0 + s.rows) {
-      latent_row<T, CH, true>(x + (size_t)row * stride, g, a, slot, s.start + row - s.row0, q_out + (size_t)row * g.q_rank, latents, shared_keys, part);
-      return;
-    }
-  }
+  Span s;
+  const int slot = slot_of_row(spans, a.slots, a.rows, row, s);
+  if (slot >= 0) latent_row<T, CH, true>(x + (size_t)row * stride, g, a, slot, s.start + row - s.row0, q_out + (size_t)row * g.q_rank, latents, shared_keys, part);
 }
 // --------------------------------------------------------------- expansion
 // The latents a portion attends, slot after slot, with their shared key parts, and behind the last a tile's rows of
