@@ -630,10 +630,15 @@ int iron_stream_product_bf16(int input, const void* x, const uint16_t* gain, con
                              void* stream);
 /* Products of up to eight rows around the stream, W (N, K), each what the entry points above compute in turn.
  * norm_strips: y (rows, N) = W times the float rows x (K up to 2048), RMS-normed with unit + gain.
+ * norm_gru_strips: norm_strips by W (4 width, K), the row [zx | ux | gx | gate], of which packed (rows, 4 width) gets the gate alone, and
+ * iron_min_gru of the rest, spans of one row at the most.
  * gated_strips: iron_stream_gated_rows of W times the bf16 rows x, plus y_bias (may be NULL), on stream_rows (rows, N), by gates
  * `gate_stride` apart. */
 int iron_norm_strips_bf16(const float* x, const uint16_t* gain, float eps, float unit, const uint16_t* W, uint16_t* y, int rows, int N,
                           int K, void* stream);
+int iron_norm_gru_strips_bf16(const float* x, const uint16_t* gain, float eps, float unit, const uint16_t* W, const uint16_t* z_bias,
+                              const uint16_t* x_bias, float* state, const int* spans, uint16_t* packed, uint16_t* y, int slots, int rows,
+                              int width, int K, void* stream);
 int iron_gated_strips_bf16(const uint16_t* x, const uint16_t* W, const uint16_t* y_bias, const uint16_t* gate, int gate_stride,
                            const uint16_t* gate_bias, float* stream_rows, int rows, int N, int K, void* stream);
 /* norm_product: y = W (M, K) times h, the float row x normed in `groups` parts (iron_stream_groups); h (may be NULL) as well, and

@@ -33,6 +33,7 @@ in a batched decoder's decode step (bf16; a float32 stream, layers with a state)
   StreamNorm, GEMV (one slot, as the rest here)          => iron_stream_product_bf16 (input 1)
   [MinGRU / PolyNorm,] GEMV, StreamGatedAdd              => iron_stream_product_bf16 (input 0 / 3 / 4)
   StreamNorm, GEMM (two to eight slots, as the next)     => iron_norm_strips_bf16
+  ... and MinGRU, beside the gate its output joins by    => iron_norm_gru_strips_bf16
   GEMM, StreamGatedAdd                                   => iron_gated_strips_bf16
   LatentRows, GEMV (the queries)                         => iron_latent_query_bf16
   StreamNorm (groups), GEMV                              => iron_norm_product_bf16
@@ -379,6 +380,18 @@ def plan(recording, tensor: Callable[[Any], Any], word: Callable[[Any], Any],
                 return None
             args = dict(x=tensor(s.inputs["x"]), gain=tensor(s.inputs["weight"]), W=tensor(g.inputs["B"]), y=tensor(g.outputs["C"]))
             kw |= dict(eps=float(s.op.epsilon), unit=float(s.op.unit))
+            c = g.outputs["C"]
+            gru, add = (steps[j + 2], steps[j + 4]) if j + 4 < len(steps) else (None, None)
+            # (the packed row is read by the recurrence, and its gate by the sum behind the product that follows)
+            if (gru is not None and _name(gru) == "MinGRU" and gru.op.single and gru.op.dtype is bfloat16 and bare(gru) and _same(gru.inputs["x"], c)
+                    and once(c, 2) and gru.op.rows == g.op.M and gru.op.slots <= 64 and g.op.N == gru.op.stride == 4 * gru.op.width
+                    and gru.op.width % 8 == 0 and gru.op.width <= 2048 and _name(add) == "StreamGatedAdd" and _same(add.inputs["gate"], c)
+                    and add.op.gate_at == 3 * gru.op.width and add.op.cols == gru.op.width):
+                args |= dict(packed=args.pop("y"), y=tensor(gru.outputs["y"]), z_bias=tensor(gru.inputs["z_bias"]), x_bias=tensor(gru.inputs["x_bias"]),
+                             state=tensor(gru.inputs["state"]), spans=tensor(gru.inputs["spans"]))
+                kw |= dict(slots=gru.op.slots, width=gru.op.width)
+                del kw["N"]
+                return Fused("norm_gru_strips", j, 3, lambda: kernels.norm_gru_strips(**args, **kw))
             return Fused("norm_strips", j, 2, lambda: kernels.norm_strips(**args, **kw))
         y, at = g.outputs["C"], o.op.gate_at
         if not (o.op.cols == g.op.N and g.op.N % 4 == 0 and o.op.gate_width % 4 == 0 and at % 4 == 0 and _same(o.inputs["y"], y) and once(y)):

@@ -6,7 +6,7 @@
 //
 // Around a float32 stream A may be its normed rows (iron_norm_strips_bf16), and C may join it through a gate (iron_gated_strips_bf16).
 #include "../../include/iron_hip.h"
-#include "common.h"
+#include "rows.h"
 
 #include <type_traits>
 
@@ -45,7 +45,7 @@ struct Strips {
 // its own tiles, a wave its strip of K while the first of B is on its way.  The launch of a norm between two of 256 blocks takes 2.2 us, and making
 // the rows here 1.0: twice A's bytes out of L2, and a chain of sums, root and scale.  Eight rows over K = 2048, weights out of memory, a norm and a
 // product against both here: 2048 columns 6.1 / 5.1 us, 4160 8.2 / 6.7, 10240 11.6 / 10.3, 128256 86.2 / 85.4.  (A recurrence's step made the same
-// way was not the faster one, 8.9 / 9.3 with its product and sum: three exponentials an element, 8 x 2048 of them a block.)
+// way ahead of the product behind it was not the faster one, 8.9 / 9.3: three exponentials an element, 8 x 2048 of them a block.)
 struct StripsNorm {
   const bf16_t* gain;
   float eps, unit;
@@ -57,6 +57,17 @@ struct StripsOut {
   float* stream;              // rows of N
   const bf16_t *y_bias, *gate, *gate_bias;   // y_bias may be null
   int gate_stride;
+};
+// C's columns are [zx | ux | gx | gate] of N / 4 each and the first three a gated recurrence's (min_gru.hip), its spans of one row at the most: a block has
+// the same eight columns of each, and a row's step and state are the lanes' that hold their sums; y gets its output, C the gates alone.
+// The launch of eight blocks that this was took 2.1 us behind the product, and costs 0.1 here (8192 columns over 2048, with the norm: 2 rows 11.0 -> 8.8
+// us, 8 rows 11.25 -> 9.3).
+struct StripsGru {
+  const bf16_t *z_bias, *x_bias;
+  float* state;
+  const int* spans;
+  bf16_t* y;
+  int slots;
 };
 struct Joined {   // ... what four columns of it need
   float4 held;
@@ -107,10 +118,11 @@ __device__ __forceinline__ void norm_strips(const StripsNorm& norm, int K, int l
   }
 }
 
-template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM, bool NORMED = false, bool JOINS = false>
+template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM, bool NORMED = false, bool JOINS = false, bool GRU = false>
 __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
-                                                                       bf16_t* __restrict__ C, int M, int N, int K, StripsNorm norm, StripsOut out) {
+                                                                       bf16_t* __restrict__ C, int M, int N, int K, StripsNorm norm, StripsOut out, StripsGru gru) {
   typedef Strips<MT, MA, SINGLE, STAGES> S;
+  static_assert(!GRU || (MT == 1 && MA == 8 && !JOINS), "one lane a row and four columns");
   static_assert(!NORMED || (SINGLE && MT == 1 && MA == 8), "a wave norms its own strip of eight rows");
   constexpr int W = STRIP_WAVES, R = STRIP_ROWS, GROUP = STRIP_OUT / R;   // GROUP: tiles whose columns are stored together
   static_assert(STAGES <= 2, "the last item's wait is for all that is out");
@@ -122,7 +134,8 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
   // (64 bits: 256 times the tiles of an N of 2^27 pass 32)
   const unsigned tiles = ((unsigned)N + R - 1) / R;
   auto first_tile = [&](unsigned block) { return (int)(tiles < STRIP_BLOCKS ? block : (unsigned long long)block * tiles / STRIP_BLOCKS); };
-  const int tile0 = first_tile(blockIdx.x), my_tiles = first_tile(blockIdx.x + 1) - tile0, items = my_tiles * mine;
+  const int tile0 = GRU ? 0 : first_tile(blockIdx.x), my_tiles = GRU ? 4 : first_tile(blockIdx.x + 1) - tile0, items = my_tiles * mine;
+  auto column_of = [&](int t) { return GRU ? t * (N >> 2) + (int)blockIdx.x * R : (tile0 + t) * R; };   // tile t's first
   char* const own = lds + wave * S::WAVE;
   char* const held = own + (SINGLE ? S::A_BYTES : 0);
   const unsigned lds0 = (unsigned)(uintptr_t)IRON_LDS_PTR(lds), part0 = lds0 + W * S::WAVE, out0 = part0 + 2 * S::PART;
@@ -142,7 +155,7 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
   };
   auto fetch = [&](int item) {
     char* to = held + item % STAGES * S::ITEM;
-    const int t = SINGLE ? item : item / max(mine, 1), strip = wave + W * (SINGLE ? 0 : item - t * mine), row0 = (tile0 + t) * R;
+    const int t = SINGLE ? item : item / max(mine, 1), strip = wave + W * (SINGLE ? 0 : item - t * mine), row0 = column_of(t);
     const int rows = min(R, N - row0);
     if (!SINGLE && S::A_BY_LDS) {
       fetch_rows(A, M, strip, to, std::integral_constant<int, S::A_INST>(), std::false_type());
@@ -174,7 +187,7 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
   const bool joins = JOINS && lane < 32 && l16 < M;
   auto join_loads = [&](int t) {
     Joined j{};
-    const int n = (tile0 + t) * R + quad * 4;
+    const int n = column_of(t) + quad * 4;
     if (joins && n < N) {
       j.held = *reinterpret_cast<const float4*>(out.stream + (size_t)l16 * N + n);
       j.gate = *reinterpret_cast<const uint2*>(out.gate + (size_t)l16 * out.gate_stride + n);
@@ -183,6 +196,19 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
     }
     return j;
   };
+  // ... and what a recurrence's step needs: lane (quad, l16) of the first wave's first two quads, four columns of row l16.
+  int start = -1, state_at = 0;   // the row's position (none: no span has it), and its slot's first state
+  float4 old_state = make_float4(0.f, 0.f, 0.f, 0.f);
+  uint2 z_bias = make_uint2(0, 0), x_bias = make_uint2(0, 0);
+  float gru_z[4] = {}, gru_u[4] = {};
+  const int gru_col = (int)blockIdx.x * R + (quad & 1) * 4;
+  Span mine_span{};
+  if (GRU && wave == 0) {
+    const int col = gru_col;
+    z_bias = *reinterpret_cast<const uint2*>(gru.z_bias + col);
+    x_bias = *reinterpret_cast<const uint2*>(gru.x_bias + col);
+    mine_span = span_of(gru.spans, min(lane, gru.slots - 1), M);
+  }
   Joined first_joined{};
   if (JOINS && wave == 0) first_joined = join_loads(0);
   if (!NORMED && SINGLE && items > 0) {
@@ -233,7 +259,17 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
 #pragma unroll
     for (int k = 0; k < 8; ++k) lds_wait_for<0>(af[0][k]);
   }
-  const bool staged = !JOINS && my_tiles > 1;   // (a lone tile's columns leave as they are: by way of LDS and another barrier 8 rows of 2048 x 2048 took 4.44 us instead of 4.24)
+  if (GRU && wave == 0) {   // (the spans' trip passed under the norm, this one passes under the products)
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const unsigned long long holds = __builtin_amdgcn_ballot_w64(lane < gru.slots && mine_span.rows > 0 && mine_span.row0 == r);
+      if (holds == 0) continue;
+      const int slot = __builtin_ctzll(holds), at = __builtin_amdgcn_readlane(mine_span.start, slot);
+      if (l16 == r) start = at, state_at = slot * (N >> 1) + gru_col;
+    }
+    if (lane < 32 && start > 0) old_state = *reinterpret_cast<const float4*>(gru.state + state_at + ((start - 1) & 1) * (N >> 2));
+  }
+  const bool staged = !JOINS && !GRU && my_tiles > 1;   // (a lone tile's columns leave as they are: by way of LDS and another barrier 8 rows of 2048 x 2048 took 4.44 us instead of 4.24)
   // The columns of `count` tiles from `first` on, from half `half` of the out stage, by one wave.
   auto flush = [&](int first, int count, int half) {
     for (int e = lane; e < M * count; e += 64) {
@@ -285,11 +321,11 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
       lds_write_b128(pa + ((wave * MT + m) * 64 + lane) * 16, v);
     }
     lds_barrier();
-    if (!JOINS && t > 0 && t % GROUP == 0 && wave == (t + W / 2) % W) flush(t - GROUP, GROUP, (t / GROUP - 1) & 1);
+    if (!JOINS && !GRU && t > 0 && t % GROUP == 0 && wave == (t + W / 2) % W) flush(t - GROUP, GROUP, (t / GROUP - 1) & 1);
     // Tile t's sums by wave t % 8: lane (quad, l16) of the first two quads has columns 4 quad .. + 3 of row l16.
     const Joined joined = JOINS ? (t == 0 ? first_joined : (wave == t % W ? join_loads(t) : Joined{})) : Joined{};
-    if (wave == t % W && lane < 32) {
-      const int n = (tile0 + t) * R + quad * 4;
+    if (wave == (GRU ? 0 : t % W) && lane < 32) {
+      const int n = column_of(t) + quad * 4;
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
         bf16x8 p[W];
@@ -312,6 +348,30 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
 #pragma unroll
             for (int j = 0; j < 4; ++j) h[j] += (round_bf16(v[j]) + yb[j]) * (1.0f / (1.0f + expf(-(g[j] + gb[j]))));
             *reinterpret_cast<float4*>(out.stream + (size_t)r * N + n) = make_float4(h[0], h[1], h[2], h[3]);
+          }
+        } else if (GRU && t < 3) {
+          // (zx and ux are kept, rounded as they would be stored, until gx is there)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float rounded = round_bf16(v[j]);
+            if (t == 0) gru_z[j] = rounded;
+            else if (t == 1) gru_u[j] = rounded;
+            else v[j] = rounded;
+          }
+          if (t == 2 && r < M && start >= 0) {
+            const float zb[4] = {bf16_lo(z_bias.x), bf16_hi(z_bias.x), bf16_lo(z_bias.y), bf16_hi(z_bias.y)};
+            const float ub[4] = {bf16_lo(x_bias.x), bf16_hi(x_bias.x), bf16_lo(x_bias.y), bf16_hi(x_bias.y)};
+            float S[4] = {old_state.x, old_state.y, old_state.z, old_state.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const float share = __builtin_amdgcn_rcpf(1.0f + __expf(-(gru_z[j] + zb[j]))), u = gru_u[j] + ub[j];
+              const float c = u >= 0.f ? u + 0.5f : __builtin_amdgcn_rcpf(1.0f + __expf(-u));
+              S[j] = fmaf(1.0f - share, S[j], share * c);
+              v[j] = S[j] * (v[j] * __builtin_amdgcn_rcpf(1.0f + __expf(-v[j])));
+            }
+            const int width = N >> 2, col = (int)blockIdx.x * R + quad * 4;
+            *reinterpret_cast<float4*>(gru.state + state_at + (start & 1) * width) = make_float4(S[0], S[1], S[2], S[3]);
+            *reinterpret_cast<uint2*>(gru.y + (size_t)r * width + col) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
           }
         } else if (staged) {
           const unsigned to = out0 + (t / GROUP & 1) * S::OUT + (r * STRIP_OUT + t % GROUP * R + quad * 4) * 2;
@@ -458,20 +518,20 @@ static int launch_gemm_few(const bf16_t* A, const bf16_t* B, const bf16_t* B2, b
   IRON_LAUNCH_CHECK();
 }
 
-template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM, bool NORMED = false, bool JOINS = false>
+template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM, bool NORMED = false, bool JOINS = false, bool GRU = false>
 static int launch_gemm_strips(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s, const StripsNorm& norm = {},
-                              const StripsOut& out = {}) {
+                              const StripsOut& out = {}, const StripsGru& gru = {}) {
   typedef Strips<MT, MA, SINGLE, STAGES> S;
   static_assert(S::LDS <= 163840, "a CU's LDS");
   static LdsOptIn opt;
-  auto kernel = &gemm_strips_kernel<MT, MA, SINGLE, STAGES, STREAM, NORMED, JOINS>;
+  auto kernel = &gemm_strips_kernel<MT, MA, SINGLE, STAGES, STREAM, NORMED, JOINS, GRU>;
   const hipError_t e = opt.ensure(reinterpret_cast<const void*>(kernel), S::LDS);
   if (e != hipSuccess) {
     set_error("gemm_few: %s", hipGetErrorString(e));
     return (int)e;
   }
   const unsigned tiles = ((unsigned)N + STRIP_ROWS - 1) / STRIP_ROWS;
-  hipLaunchKernelGGL(kernel, dim3(tiles < STRIP_BLOCKS ? tiles : STRIP_BLOCKS), dim3(STRIP_WAVES * 64), S::LDS, s, A, B, C, M, N, K, norm, out);
+  hipLaunchKernelGGL(kernel, dim3(GRU ? tiles / 4 : (tiles < STRIP_BLOCKS ? tiles : STRIP_BLOCKS)), dim3(STRIP_WAVES * 64), S::LDS, s, A, B, C, M, N, K, norm, out, gru);
   IRON_LAUNCH_CHECK();
 }
 
@@ -544,6 +604,21 @@ extern "C" int iron_norm_strips_bf16(const float* x, const uint16_t* gain, float
   IRON_REQUIRE(K >= 8 && K % 8 == 0 && K <= STRIP * STRIP_WAVES, "norm_strips: K (%d) is a positive multiple of 8 up to %d", K, STRIP * STRIP_WAVES);
   IRON_REQUIRE((((uintptr_t)x | (uintptr_t)gain | (uintptr_t)W) & 15) == 0, "norm_strips: operands must be 16-byte aligned");
   return launch_gemm_strips<1, 8, true, 2, true, true>(reinterpret_cast<const bf16_t*>(x), W, y, rows, N, K, (hipStream_t)stream, StripsNorm{gain, eps, unit});
+}
+
+extern "C" int iron_norm_gru_strips_bf16(const float* x, const uint16_t* gain, float eps, float unit, const uint16_t* W, const uint16_t* z_bias,
+                                         const uint16_t* x_bias, float* state, const int* spans, uint16_t* packed, uint16_t* y, int slots, int rows,
+                                         int width, int K, void* stream) {
+  IRON_REQUIRE(x && gain && W && z_bias && x_bias && state && spans && packed && y, "norm_gru_strips: null operand");
+  IRON_REQUIRE(rows > 0 && rows <= 8 && slots > 0 && slots <= 64, "norm_gru_strips: rows (%d) from 1 to 8, slots (%d) from 1 to 64", rows, slots);
+  IRON_REQUIRE(width > 0 && width % 8 == 0 && width <= 8 * (int)STRIP_BLOCKS, "norm_gru_strips: width (%d) is a positive multiple of 8 up to %d", width,
+               8 * (int)STRIP_BLOCKS);
+  IRON_REQUIRE(K >= 8 && K % 8 == 0 && K <= STRIP * STRIP_WAVES, "norm_gru_strips: K (%d) is a positive multiple of 8 up to %d", K, STRIP * STRIP_WAVES);
+  IRON_REQUIRE((((uintptr_t)x | (uintptr_t)gain | (uintptr_t)W | (uintptr_t)z_bias | (uintptr_t)x_bias | (uintptr_t)state | (uintptr_t)spans |
+                 (uintptr_t)packed | (uintptr_t)y) & 15) == 0, "norm_gru_strips: operands must be 16-byte aligned");
+  const StripsGru gru{z_bias, x_bias, state, spans, y, slots};
+  return launch_gemm_strips<1, 8, true, 2, true, true, false, true>(reinterpret_cast<const bf16_t*>(x), W, packed, rows, 4 * width, K, (hipStream_t)stream,
+                                                                    StripsNorm{gain, eps, unit}, {}, gru);
 }
 
 extern "C" int iron_gated_strips_bf16(const uint16_t* x, const uint16_t* W, const uint16_t* y_bias, const uint16_t* gate, int gate_stride,

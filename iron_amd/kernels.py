@@ -1180,6 +1180,20 @@ def norm_strips(x, gain, W, y, *, rows, N, K, eps, unit=0.0):
     check(lib().iron_norm_strips_bf16(ptr(x), ptr(gain), float(eps), float(unit), ptr(W), ptr(y), rows, N, K, current_stream()), "iron_norm_strips_bf16")
 
 
+def norm_gru_strips(x, gain, W, z_bias, x_bias, state, spans, packed, y, *, slots, rows, width, K, eps, unit=0.0):
+    """Up to eight rows of the stream, normed, a gated recurrence's packed projection (its gates alone are stored) and its step, one launch."""
+    _f32(x, rows * K, "x")
+    _bf16(gain, K, "gain")
+    _bf16(W, 4 * width * K, "W")
+    _bf16(z_bias, width, "z_bias")
+    _bf16(x_bias, width, "x_bias")
+    _f32(state, slots * 2 * width, "state")
+    _bf16(packed, rows * 4 * width, "packed")
+    _bf16(y, rows * width, "y")
+    check(lib().iron_norm_gru_strips_bf16(ptr(x), ptr(gain), float(eps), float(unit), ptr(W), ptr(z_bias), ptr(x_bias), ptr(state), _spans(spans, slots),
+                                          ptr(packed), ptr(y), slots, rows, width, K, current_stream()), "iron_norm_gru_strips_bf16")
+
+
 def gated_strips(x, W, stream, gate, gate_bias, *, rows, N, K, gate_stride, y_bias=None):
     """Up to eight rows' product, joining the rows ``stream`` through ``gate`` (its rows ``gate_stride`` apart, from its first
     column on), one launch."""

@@ -248,7 +248,8 @@ class GatedRecurrence(iron.Graph):
         return {"memory": iron.state((slots, 2, self.inner), np.float32)}
 
     def body(self, x, call, state):
-        return self.out(MinGRU.step(x, self.z_bias, self.x_bias, state["memory"], call.spans, dtype=self.dtype)[1])
+        return self.out(MinGRU.step(x, self.z_bias, self.x_bias, state["memory"], call.spans, single=not call.prompt,
+                                    dtype=self.dtype)[1])
 
 
 class LatentAttention(iron.Graph):

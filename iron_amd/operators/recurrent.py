@@ -151,6 +151,7 @@ class MinGRU(_Spanned):
     rows: int = param()
     stride: int = param()
     width: int = param()
+    single: bool = param(default=False, repr=False)   # no span has more than one row
     dtype: Any = param(default=bfloat16, repr=False)
     x = In(rows, stride, dtype=dtype)
     z_bias = In(width)

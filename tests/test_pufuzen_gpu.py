@@ -330,15 +330,39 @@ def test_rows_products_join_the_stream(cuda, rows, N, K_):
         assert np.abs(from_torch(to) - want).max() <= 8e-3 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("rows,width,K_", [(1, 8, 64), (3, 264, 136), (8, 2048, 2048), (5, 1000, 2040)])
+def test_a_recurrence_s_step_in_its_projection_s_launch(cuda, rows, width, K_):
+    rng = np.random.default_rng(width)
+    slots = rows + 3
+    W, gain, x = bf(rng, 4 * width, K_, scale=1 / np.sqrt(K_)), bf(rng, K_), rng.standard_normal((rows, K_)).astype(F32) * 3
+    b0, b1, state = bf(rng, width), bf(rng, width), rng.standard_normal((slots, 2, width)).astype(F32)
+    # the rows' slots in another order, some idle, at positions of either parity and at none
+    spans, order, starts = table(slots=slots), rng.permutation(slots)[:rows], [(0, 5, 6, 1)[r % 4] for r in range(rows)]
+    for r, (slot, start) in enumerate(zip(order, starts)):
+        spans[slot] = (r, 1, start, 0)
+    packed, y = (torch.full((rows, n), 7.0, dtype=torch.bfloat16, device="cuda") for n in (4 * width, width))
+    kept = device(state, F32)
+    K.norm_gru_strips(device(x, F32), device(gain, BF16), device(W, BF16), device(b0, BF16), device(b1, BF16), kept, device(spans, np.int32), packed, y,
+                      slots=slots, rows=rows, width=width, K=K_, eps=1e-3, unit=0.5)
+    # against the separate launches: the products' bits, and the recurrence of them
+    p = torch.empty_like(packed)
+    K.norm_strips(device(x, F32), device(gain, BF16), device(W, BF16), p, rows=rows, N=4 * width, K=K_, eps=1e-3, unit=0.5)
+    alone, out = device(state, F32), torch.empty_like(y)
+    K.min_gru(p, device(b0, BF16), device(b1, BF16), alone, device(spans, np.int32), out, slots=slots, rows=rows, stride=4 * width, width=width)
+    assert torch.equal(packed[:, 3 * width :], p[:, 3 * width :]) and (packed[:, : 3 * width] == 7).all()
+    assert np.abs(from_torch(kept) - from_torch(alone)).max() <= 1e-6 * np.abs(state).max()
+    assert np.abs(from_torch(y) - from_torch(out)).max() <= 2**-8 * np.abs(from_torch(out)).max()
+
+
 def test_a_batch_s_steps_in_few_launches(cuda):
     """Steps of two to eight slots: the stream's norms and sums in the products' launches, with what the steps alone give."""
-    for slots in (2, 8):
+    for name, slots in (("mixed", 2), ("mixed", 8), ("wide", 3), ("wide", 8)):   # (recurrences of other widths than the stream's, and of its width)
         rows = {}
         for fuse in (True, False):
-            model, _ = built("mixed", Pufuzen, slots=slots, max_seq_len=200, prefill_chunk=32)
+            model, _ = built(name, Pufuzen, slots=slots, max_seq_len=200, prefill_chunk=32)
             model.load_versions(fuse=fuse)
             kinds = {f.kind for f in model.decode_step._fused.values()}
-            assert not fuse or {"norm_strips", "gated_strips"} <= kinds
+            assert not fuse or {"norm_strips", "gated_strips", *(("norm_gru_strips",) if name == "wide" else ())} <= kinds
             prompts = [tokens_of(model, 5 + 3 * i, seed=i) for i in range(slots)]
             model.batch.step([Entry(i, p) for i, p in enumerate(prompts)])
             steps = []
