@@ -11,6 +11,7 @@ import pytest
 import oracle
 from iron_amd.applications import Pufuzen, PufuzenConfig, model_class
 from iron_amd.applications.pufuzen import module_weights
+from iron_amd.common import fusion
 from iron_amd.lm import Sampler, write_safetensors
 from iron_amd.lm.batched import BatchedOnHost, Entry
 from iron_amd.operators.mha_latent import EVERYTHING
@@ -251,3 +252,35 @@ def test_a_conversation_continues_and_starts_over():
         assert far_off(session.logits(tokens[:n]), want[n - 1], want.std()) < 2e-5
     other = np.concatenate([tokens[:4], tokens[10:14]])
     assert far_off(session.logits(other), plain(other)[-1], want.std()) < 2e-5   # a state is not rewound: from the start
+
+
+# ---------------------------------------------------------------- what a batch's step is recorded as, and launched as
+
+STRIPS = {"norm_strips", "norm_gru_strips", "gated_strips"}
+
+
+@pytest.mark.parametrize("slots,name,kinds", [(1, "wide", set()), (2, "wide", STRIPS), (8, "wide", STRIPS), (9, "wide", set()),   # two to eight rows
+                                              (3, "mixed", STRIPS - {"norm_gru_strips"}),   # recurrences of other widths than the stream's
+                                              (3, "odd", set())])                           # columns that are no whole pieces
+def test_the_steps_that_products_take_in(slots, name, kinds):
+    model, _ = built(name, Pufuzen, slots=slots, max_seq_len=64, prefill_chunk=16)
+    found = fusion.match(model.record())
+    assert {f.kind for f in found} & STRIPS == kinds
+    if kinds:   # no norm, gated sum or (of the stream's width) recurrence is left beside them
+        recording = model.record()
+        hidden = {i for f in found for i in range(f.first, f.first + f.count)}
+        left = [type(s.op).__name__ for i, s in enumerate(recording.steps) if i not in hidden]
+        assert not {"StreamNorm", "StreamGatedAdd", *(("MinGRU",) if "norm_gru_strips" in kinds else ())} & set(left)
+    # a prompt's portion is bounded by its rows and keeps its launches, but for the head's over its spans' last rows
+    prompt = [f.kind for f in fusion.match(model.record(ids=((16,), np.int32))) if f.kind in STRIPS]
+    assert prompt == (["norm_strips"] if kinds else [])
+
+
+@pytest.mark.parametrize("options", [{"activations": np.float32}, {"hidden_size": 2056}], ids=["float32", "a wide stream"])
+def test_the_steps_that_products_leave(options):
+    """In 32 bits, and of a stream wider than a block's strips make up, every step is its own or as it was."""
+    layers = document([gru(options.get("hidden_size", 192))], vocab=64, width=options.get("hidden_size", 192), scale=1.0)
+    config = dataclasses.replace(PufuzenConfig.from_json(layers), slots=3, max_seq_len=64, prefill_chunk=16,
+                                 **{k: v for k, v in options.items() if k == "activations"})
+    model = Pufuzen(config, weights_of(config))
+    assert not {f.kind for f in fusion.match(model.record())} & STRIPS
