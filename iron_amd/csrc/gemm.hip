@@ -419,12 +419,12 @@ constexpr int NOWHERE = (int)0x80000000u;   // past stage_rows' 2^31 - 1 bytes, 
 // An element's sum is the same chain of 32-wide k-steps as in the 128 x 128 and the 256 x 256 tiles: where a row bound chooses
 // the tile, a row's products are the same bits whatever rows share the launch.
 // `qkv` carries only the optional residual epilogue here, or (QKV) the fused projections'.  WM x 4 / WM waves of MI x NJ tiles: <2, 2, 2> are 64 x 64, <4>
-// 128 x 64.  PAIR: both first products of a gated feed-forward, 32 columns of each (`qkv` says the gate's kind).  B_KN: B is (K,N), 64 columns a tile.
+// 128 x 64.  PAIR: both first products of a gated feed-forward, 32 columns of each (`qkv` says the gate's kind).  B_KN: B is (K,N), 64 columns a tile; C_NM: and C (N,M).
 // A few rows' tiles wait for what a CU can draw of operands that are 128 bytes of a row here and there, some 60 GB/s of weights out of memory, whatever the
 // stages in flight (8 or 10 of 16 KB the same): where the tiles leave CUs without one, smaller tiles have more CUs draw less each.  2048 columns over 2048
 // with a residual, us by 64 x 64 tiles, 64 x 32 <1, 4, 2> and 32 x 32 <1, 2, 1>: 12.5 / 10.4 / 8.6 (256 blocks: up to 640, 256 and 128 rows); over 8192
 // 36 / 28.7 / 21.3.
-template <int STAGES, bool PAIR = false, int MI = 2, int WM = 2, int NJ = 2, bool QKV = false, bool B_KN = false>
+template <int STAGES, bool PAIR = false, int MI = 2, int WM = 2, int NJ = 2, bool QKV = false, bool B_KN = false, bool C_NM = false>
 __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
                                                bf16_t* __restrict__ C, int M, int N, int K,
                                                int Mv, int tiles_m, int tiles_n,
@@ -435,7 +435,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
   constexpr int INST = NT_BM / 8 / 4, B_INST = NT_BN / 8 / 4;  // 1 KB loads of A and of B a wave issues per stage
   constexpr int LOADS = INST + B_INST, PER = (LOADS + 2 * MI - 1) / (2 * MI);   // PER: loads behind every second MFMA
   static_assert(BK == 64 && STAGES >= 4 && ((MI == 2 && WM == 2 && NJ == 2) || !PAIR) && (!QKV || (NJ == 2 && NT_BN <= 64)) &&
-                    (!B_KN || (NT_BN == 64 && NJ == 2 && !PAIR && !QKV)),
+                    (!B_KN || (NT_BN == 64 && NJ == 2 && !PAIR && !QKV)) && (B_KN || !C_NM),
                 "two 32-wide k-steps a stage");
   extern __shared__ __align__(16) char smem_nt[];
 
@@ -595,7 +595,11 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) mfma_16x16x32_in_place(acc[i][j], bfr[P][ks][j], af[P][ks][i]);
+      for (int j = 0; j < NJ; ++j) {
+        // (the operands' order decides whether a lane owns four columns of a row or four rows of a column)
+        if constexpr (C_NM) mfma_16x16x32_in_place(acc[i][j], af[P][ks][i], bfr[P][ks][j]);
+        else mfma_16x16x32_in_place(acc[i][j], bfr[P][ks][j], af[P][ks][i]);
+      }
       __builtin_amdgcn_sched_barrier(0);
       if (t == 0) {   // (behind the first products, which the waves wait under: 300 x 512 x 2048 8.1 -> 7.8 us)
         // Of this wave's loads in flight the oldest LOADS are stage kt+1's; the STAGES-3 stages after it may stay out.
@@ -641,6 +645,24 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
   asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");
 #pragma unroll
   for (int t = 0; t < NJ * MI; ++t) asm volatile("" : "+a"(acc[t / NJ][t % NJ]));
+  if constexpr (C_NM) {   // C (N,M), no bound: acc[i][j][e] is row 16 i + 4 kq + e, column 16 j + fr of the wave's
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int m = m0 + wm * (16 * MI) + 16 * i + 4 * kq, n = n0 + wn * (16 * NJ) + 16 * j + fr;
+        if (n >= N || m >= M) continue;
+        bf16_t* to = C + (size_t)n * M + m;
+        if (m + 4 <= M) {
+          store_loose(to, pack_bf16(acc[i][j][0], acc[i][j][1]), pack_bf16(acc[i][j][2], acc[i][j][3]));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 3; ++e)
+            if (m + e < M) to[e] = f32_to_bf16(acc[i][j][e]);
+        }
+      }
+    return;
+  }
   if constexpr (QKV) {
     const int row_len = which == 0 ? N : qkv.kv_n, c = first + wn * 16 + 4 * kq;   // ... of the head's first half
     bf16_t* to = (which == 0 ? C : (which == 1 ? qkv.Ck : qkv.Cv)) + own * 64 + c;
@@ -1164,22 +1186,22 @@ static int launch_gemm_nt(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, in
   IRON_LAUNCH_CHECK();
 }
 
-template <int STAGES, int MI, int WM, int NJ, bool B_KN = false>
+template <int STAGES, int MI, int WM, int NJ, bool B_KN = false, bool C_NM = false>
 __global__ __launch_bounds__(256) void gemm_small_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, bf16_t* __restrict__ C, int M, int N,
                                                          int K, int tiles_m, int tiles_n) {
-  gemm_nt64_body<STAGES, false, MI, WM, NJ, false, B_KN>(A, B, C, M, N, K, M, tiles_m, tiles_n, 0, QkvTail{});
+  gemm_nt64_body<STAGES, false, MI, WM, NJ, false, B_KN, C_NM>(A, B, C, M, N, K, M, tiles_m, tiles_n, 0, QkvTail{});
 }
-template <int STAGES, int MI, int WM, int NJ, bool B_KN = false>
+template <int STAGES, int MI, int WM, int NJ, bool B_KN = false, bool C_NM = false>
 static int launch_gemm_small(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s) {
   constexpr int BM = 16 * MI * WM, BN = 16 * NJ * (4 / WM);
   constexpr size_t lds = (size_t)STAGES * (BM + BN) * BK * 2;
   static LdsOptIn opt_in;
-  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_small_kernel<STAGES, MI, WM, NJ, B_KN>), lds); e != hipSuccess) {
+  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_small_kernel<STAGES, MI, WM, NJ, B_KN, C_NM>), lds); e != hipSuccess) {
     set_error("gemm: %s", hipGetErrorString(e));
     return (int)e;
   }
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  hipLaunchKernelGGL((gemm_small_kernel<STAGES, MI, WM, NJ, B_KN>), dim3(tiles_m * tiles_n), dim3(256), lds, s, A, B, C, M, N, K, tiles_m, tiles_n);
+  hipLaunchKernelGGL((gemm_small_kernel<STAGES, MI, WM, NJ, B_KN, C_NM>), dim3(tiles_m * tiles_n), dim3(256), lds, s, A, B, C, M, N, K, tiles_m, tiles_n);
   IRON_LAUNCH_CHECK();
 }
 
@@ -2737,7 +2759,8 @@ static int check_gemm(const uint16_t* A, const uint16_t* B, const uint16_t* C, i
 // 250 x 232 x 2584 13.9 / 7.8, 163 x 2113 x 4088 26.1 / 16.4; against shared K 112 x 886 x 2704 18.7 / 9.1, 58 x 411 x 4416 19.5 / 10.4; out of the
 // last-level cache 510 x 331 x 2232 9.3 / 7.1, 41 x 4827 x 3112 21.2 / 11.0. Two stages are too few for them to pay.
 // With B (K,N) the columns are 64, a cache line of a row of B; 128 x 128 tiles and those: 521 x 416 x 1320 12.3 / 7.5, 50 x 6672 x 1880 21.6 / 13.1,
-// 130 x 88 x 1008 8.9 / 5.8; a long K shared stays so, 135 x 440 x 8096 14.8 / 36.
+// 130 x 88 x 1008 8.9 / 5.8; a long K shared stays so, 135 x 440 x 8096 14.8 / 36.  C (N,M) of it likewise: 248 x 1472 x 1480 12.7 / 7.6, 883 x 160 x 1032
+// 10.8 / 6.8, 110 x 176 x 248 6.2 / 3.9.
 struct SmallTiles {
   int rows;
   float us;
@@ -2834,8 +2857,13 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
   if (gemm_of_few_rows(M, N, K) && b_col_maj && !c_col_maj && valid == nullptr && valid_k == nullptr)
     return iron_gemm_few_bf16(A, B, nullptr, C, M, N, K, 0, stream);
   if (valid_k == nullptr && gemm_direct_to_lds(M, N, K, b_col_maj, c_col_maj, valid != nullptr)) {
-    if (c_col_maj) return launch_gemm_nt<true, false, 2, 4, true>(A, B, C, M, N, K, valid, s);
     const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
+    if (c_col_maj) {
+      const SmallTiles small = tiles128 < 128 ? small_tiles(M, N, K, false) : SmallTiles{0, 0.f};
+      if (small.rows == 32) return launch_gemm_small<13, 1, 2, 2, true, true>(A, B, C, M, N, K, s);
+      if (small.rows == 64) return launch_gemm_small<10, 2, 2, 2, true, true>(A, B, C, M, N, K, s);
+      return launch_gemm_nt<true, false, 2, 4, true>(A, B, C, M, N, K, valid, s);
+    }
     if (valid == nullptr && tiles128 >= 128) {
       float price, price128;
       const BigForm form = big_form(M, N, K, b_col_maj, price, price128);
@@ -2872,7 +2900,7 @@ static TileShares gemm_shares(int M, int N, int K, bool b_nk, bool c_nm) {
   if (b_nk && gemm_of_few_rows(M, N, K)) return TileShares{0, 0, 0};
   float then = 0.f, big, price128;
   const TileShares deal = gemm_shares_of_tiles(M, N, K, b_nk, &then);
-  if (const SmallTiles small = small_tiles(M, N, K, b_nk); !c_nm && deal.slices > 0 && small.rows > 0 && small.us < (b_nk || N % BK == 0 ? 0.78f : 0.68f) * then)
+  if (const SmallTiles small = small_tiles(M, N, K, b_nk); deal.slices > 0 && small.rows > 0 && small.us < (b_nk || N % BK == 0 ? 0.78f : 0.68f) * then)
     return TileShares{0, 0, 0};   // (rows of B (K,N) that straddle cache lines cost the small tiles more, out of memory: 30 x 2776 x 3248 shared 16.1, by those 21.0)
   // (whole tiles of another size, where they take no more)
   if (deal.slices > 0 && !c_nm && deal.whole + deal.shared >= 128 && big_form(M, N, K, b_nk, big, price128) != BIG_NONE && big + 3.f <= then)

@@ -85,6 +85,17 @@ def test_gemv_batches_repeat_and_bound(cuda):
 
 
 # ------------------------------------------------------------------------ GEMM
+@pytest.mark.parametrize("M,Kdim,N", [(5, 648, 8), (33, 264, 72), (97, 192, 136), (130, 1096, 600), (1003, 584, 640), (70, 520, 24)])
+def test_gemm_turned_over_small_tiles(cuda, M, Kdim, N):
+    """B (K,N) into C (N,M), less than a round of tiles of 32 and of 64 rows: edges of both, ragged K, nothing beyond C."""
+    rng = np.random.default_rng(M + N)
+    A, B = bf(rng, M, Kdim), bf(rng, Kdim, N, scale=0.05)
+    C = out_like((N * M + 64,), cuda, fill=3.0)
+    K.gemm(dev(A, cuda), dev(B, cuda), C[: N * M].view(N, M), M=M, N=N, K=Kdim, c_col_maj=True)
+    got = from_torch(C)
+    assert np.all(np.abs(got[: N * M].reshape(N, M).T - ops.gemm(A, B)) <= ops.gemm_bound(A, B)) and np.all(got[N * M :] == 3.0)
+
+
 @pytest.mark.parametrize("b_col_maj", [False, True])
 @pytest.mark.parametrize("c_col_maj", [False, True])
 def test_gemm_layouts(cuda, b_col_maj, c_col_maj):
