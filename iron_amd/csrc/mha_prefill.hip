@@ -52,11 +52,11 @@ constexpr int kFewBlocks = 512;          // launches of fewer blocks than this h
 constexpr int kWideBigBlocks = 512;     // wide heads: launches of at least this many 128-query blocks keep that size
 // Launches of up to this many blocks split each block's tiles over two halves of eight waves, which halves a block's chain of tiles; more fill the chip better
 // four waves each.  64-wide heads (two eight-wave blocks share a CU): S = 8192 at 32 heads 365 -> 353-360 us split, S = 16384 not.  128-wide ones (two
-// four-wave blocks, which read a tile's keys ahead): 32 heads, split against not, 2048 queries 45.4 / 52.4, 2305 63.6 / 59.8, 3001 90.4 / 81.8, 4096
-// 147 / 135, a window of 1024 of those 90 / 76; 24 heads, 3000 74.4 / 73.4; 16 heads, 5000 120 / 122, 6000 159 / 155.
-// (Both take their weights to bf16 and everything else in float; split, a query has a reference a half instead of one. Against 64 bits 3001 queries are
-// 0.00208 off split and 0.00211 not, of which the output's own rounding is 0.00166.)
-constexpr int kSplitMaxBlocks64 = 4096, kSplitMaxBlocks128 = 560;
+// four-wave blocks, which read a tile's keys ahead) would be the faster unsplit from 560 blocks on (32 heads, split against not, 2048 queries 45.4 / 52.4, 2305
+// 63.6 / 59.8, 3001 90.4 / 81.8, 4096 147 / 135; 16 heads, 6000 159 / 155), but split, a query has a reference for each half of its tiles, so that the
+// largest weight of either is 1, which bf16 holds exactly: 3001 queries are 0.00208 from 64 bits split and 0.00211 not (the output's own rounding
+// is 0.00166), and up to 1024 blocks the nearer one stays.
+constexpr int kSplitMaxBlocks64 = 4096, kSplitMaxBlocks128 = 1024;
 
 // Few live queries over many keys (a turn late in a conversation: 40 rows of a 2048-row launch, 12 000 keys): by the
 // tiles below, a block a head and 128 queries, most of the chip would idle behind a block's chain
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
   constexpr int CPR = D / 8;             // 16-byte chunks a row has
   constexpr int STAGES = D == 64 && SPLIT == 1 ? 3 : 2;
   // 128-wide heads by four waves: a tile's K fragments are read under the softmax of the tile before, and a tile's loads have a whole step to land (one
-  // barrier a step as without; 8192 queries 521 -> 501 us, and it makes this form the faster one from 560 blocks on).  Not with eight waves, one block
+  // barrier a step as without; 8192 queries 521 -> 501 us).  Not with eight waves, one block
   // a CU, where the 32 more registers bought nothing (3001 queries 93.9 / 95.2; halves half a step apart, one's products under the
   // other's softmax, 102), nor with 64-wide heads, whose four waves a SIMD cover the reads.
   constexpr bool PIPED = D == 128 && SPLIT == 1;

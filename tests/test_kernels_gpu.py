@@ -1058,12 +1058,36 @@ def test_mha_prefill_of_few_rows_over_many_keys(cuda, H, G, d, S, rows, L, keys,
     (32, 8, 256, 256, 1000, 1000, None, True), (32, 8, 256, 230, 2500, 2100, None, True), (32, 8, 200, 200, 1600, 1600, None, False),
     (32, 8, 257, 257, 1600, 1600, None, True), (32, 8, 300, 270, 2000, 400, None, True),
     (32, 8, 700, 700, 700, 700, None, True), (32, 8, 640, 640, 1700, 1700, None, True), (8, 2, 2200, 2200, 2200, 2200, 1500, True),
-    # many blocks of four waves, keys read a tile ahead: one key, one tile, two, three of them, a window, no mask, rows past the bounds
+    # more blocks than two a CU, keys dealt over two halves: one key, one tile, two, three of them, a window, no mask, rows past the bounds
     (576, 64, 1, 1, 1, 1, None, True), (576, 64, 64, 64, 64, 64, None, False), (576, 64, 65, 65, 65, 65, None, True),
     (256, 64, 300, 300, 300, 300, None, True), (288, 32, 129, 129, 190, 190, None, False), (288, 32, 129, 129, 700, 700, 200, True),
     (288, 32, 200, 131, 500, 400, None, True)])
 def test_mha_prefill_128_wide_heads_at_the_lines_between_the_forms(cuda, H, G, S, rows, L, keys, window, causal):
     test_mha_prefill_of_few_rows_over_many_keys(cuda, H, G, 128, S, rows, L, keys, window, causal)
+
+
+@pytest.mark.parametrize("H,G,S", [(32, 8, 2305), (16, 4, 5000), (32, 32, 4096)])   # 608, 640 and 1024 blocks of 128 queries
+def test_mha_prefill_128_wide_heads_keep_a_reference_for_each_half_of_the_tiles(cuda, H, G, S):
+    """Every query sees one key of the first tile at a score of 0 and a value of 0, one of the second at a score of its own and a value of
+    1, and others out of sight of both.  With a reference for the even tiles and one for the odd, both weights are exactly 1 in the products and the
+    sums join in float32, so the answer w / (1 + w) is off by its own rounding alone (half a step of bf16, 2^-8 of its power of
+    two) and float32's; with one reference w itself is rounded to bf16 first, half a step more."""
+    rng = np.random.default_rng(S)
+    Q, Kc, Vc = np.zeros((S, H, 128), np.float32), np.zeros((S, G, 128), np.float32), np.zeros((S, G, 128), np.float32)
+    Q[..., 0] = round_bf16(rng.uniform(0.1, 3.0, (S, H)).astype(np.float32))
+    Q[..., 1] = 1.0
+    Kc[..., 1] = -300.0
+    Kc[5, :, 1] = 0.0
+    Kc[70, :, 0], Kc[70, :, 1] = -1.0, 0.0
+    Vc[70] = 1.0
+    O = out_like(Q.shape, cuda, fill=float("nan"))
+    K.mha_prefill(dev(Q, cuda), dev(Kc, cuda), dev(Vc, cuda), O, heads=H, kv_heads=G, d=128, seq=S, kv_len=S, scale=1.0, causal=True,
+                  q_interleaved=True, kv_interleaved=True)
+    w = np.exp(-Q[71:, :, 0].astype(np.float64))
+    want = w / (1 + w)
+    err = np.abs(from_torch(O)[71:].astype(np.float64) - want[..., None])
+    step = 2.0 ** (np.floor(np.log2(want)) - 7)
+    assert np.all(err <= (0.5 * step + 2.0**-18 * want)[..., None]), f"{(err > (0.5 * step + 2.0**-18 * want)[..., None]).mean():.3f} are off by more"
 
 
 @pytest.mark.parametrize("d", [64, 128])
