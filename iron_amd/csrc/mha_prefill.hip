@@ -627,6 +627,9 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
       block_barrier();
       k_half(0, 0, kf[0]);
       k_half(0, 1, kf[1]);
+      // The first tile's keys are in registers before this wave meets the barrier behind which their place is refilled: the products, which would wait for
+      // them, may be scheduled past it.  (Every later tile's are there once the values read behind them are, which `rest` waits for.)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       auto piped_step = [&](int step, const int buf) {
         f32x16 sacc[2];
         scores(kf, sacc);

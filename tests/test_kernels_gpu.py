@@ -1090,6 +1090,16 @@ def test_mha_prefill_128_wide_heads_keep_a_reference_for_each_half_of_the_tiles(
     assert np.all(err <= (0.5 * step + 2.0**-18 * want)[..., None]), f"{(err > (0.5 * step + 2.0**-18 * want)[..., None]).mean():.3f} are off by more"
 
 
+# Launches of more than 1024 blocks, four waves each, which read a tile's keys ahead and refill their place at the next step: one key, one tile and one
+# key more, two tiles, three and four (the first refill, the last step's reads past the end), a window, no mask, rows past the bounds.
+@pytest.mark.parametrize("H,G,S,rows,L,keys,window,causal", [
+    (1088, 64, 1, 1, 1, 1, None, True), (1088, 64, 64, 64, 64, 64, None, False), (1088, 64, 65, 65, 65, 65, None, True),
+    (1088, 32, 128, 128, 128, 128, None, True), (1088, 32, 97, 97, 192, 192, None, False), (1088, 32, 100, 100, 250, 250, None, True),
+    (544, 32, 300, 300, 300, 300, 100, True), (544, 32, 200, 131, 450, 400, None, True)])
+def test_mha_prefill_128_wide_heads_whose_keys_are_read_a_tile_ahead(cuda, H, G, S, rows, L, keys, window, causal):
+    test_mha_prefill_of_few_rows_over_many_keys(cuda, H, G, 128, S, rows, L, keys, window, causal)
+
+
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("interleaved", [True, False])
 def test_mha_prefill_of_few_rows_in_both_layouts_and_a_window_of_a_buffer(cuda, d, interleaved):
