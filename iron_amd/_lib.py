@@ -22,6 +22,7 @@ SIGNATURES = {
     "iron_gemm_bf16": (c_int, [_P, _P, _P, c_int, c_int, c_int, c_int, c_int, _P, _P, _P]),
     "iron_gemm_workspace_bytes": (c_int64, [c_int, c_int, c_int, c_int, c_int]),
     "iron_gemm_shared_bf16": (c_int, [_P, _P, _P, c_int, c_int, c_int, c_int, c_int, _P, _P]),
+    "iron_gemm_tile": (c_int, [c_int] * 7),
     "iron_gemv_bf16": (c_int, [_P, _P, _P, c_int, c_int, c_int, c_int, _P, _P]),
     "iron_gemv_bf16_tuned": (c_int, [_P, _P, _P, c_int, c_int, c_int, c_int, _P, c_int, c_int, _P]),
     "iron_gemm_residual_bf16": (c_int, [_P, _P, _P, _P, c_int, c_int, c_int, c_float, _P, _P]),

@@ -1993,6 +1993,10 @@ __device__ __forceinline__ FormOfRows form_of_rows(const FormTable& t, const int
   const int form = (int)(w >> ((run & 15) * 4)) & 15;
   return FormOfRows{rows, form, patched >> form & 1};
 }
+static int form_of_rows(const FormTable& t, int rows) {
+  const int run = (rows < 1 ? 0 : rows - 1) >> (6 + t.shift);
+  return (int)(t.w[run >> 4] >> ((run & 15) * 4)) & 15;
+}
 // `best(rows)` for the most rows of every run up to M; `upto[form]`: the most rows a form is taken for.
 template <class Best>
 static FormTable form_table(int M, Best best, int* upto) {
@@ -2036,6 +2040,9 @@ static RowsForm rows_form(int rows, int M, int N, int K, bool whole) {
     if (form == first || us < price) best = (RowsForm)form, price = us;
   }
   return best;
+}
+static FormTable rows_forms(int M, int N, int K, bool bounded, bool whole, int* upto) {
+  return form_table(M, [&](int rows) { return (int)rows_form(bounded ? rows : M, M, N, K, whole); }, upto);
 }
 template <bool TAIL>
 __global__ __launch_bounds__(256) void gemm_rows_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, bf16_t* __restrict__ C,
@@ -2093,7 +2100,7 @@ static int launch_gemm_rows(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, 
                             const QkvTail& tail = QkvTail{}) {
   int upto[ROWS_FORMS] = {};
   const bool whole = tail.residual == nullptr || N % 8 == 0;
-  FormTable forms = form_table(M, [&](int rows) { return (int)rows_form(valid == nullptr ? M : rows, M, N, K, whole); }, upto);
+  FormTable forms = rows_forms(M, N, K, valid != nullptr, whole, upto);
   const int blocks = blocks_of_forms(ROWS_PRICES, upto, N, forms);
   constexpr size_t lds = Tile256Four::LDS_BYTES;
   static_assert(lds >= (size_t)NT_STAGES * 256 * BK * 2, "the other bodies' stages fit too");
@@ -2500,6 +2507,9 @@ static PairForm pair_form(int rows, int M, int N, int K) {
   }
   return best;
 }
+static FormTable pair_forms(int M, int N, int K, bool bounded, int* upto) {
+  return form_table(M, [&](int rows) { return (int)pair_form(bounded ? rows : M, M, N, K); }, upto);
+}
 __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __restrict__ A,
                                                               const bf16_t* __restrict__ Bg,
                                                               const bf16_t* __restrict__ Bu, bf16_t* __restrict__ G,
@@ -2537,7 +2547,7 @@ __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __re
 static int launch_gemm_gated_pair(const bf16_t* A, const bf16_t* Bg, const bf16_t* Bu, bf16_t* G, bf16_t* C, int M,
                                   int N, int K, const int* valid, int activation, hipStream_t s) {
   int upto[PAIR_FORMS] = {};   // each form's grid covers the rows it is chosen for
-  FormTable forms = form_table(M, [&](int rows) { return (int)pair_form(valid == nullptr ? M : rows, M, N, K); }, upto);
+  FormTable forms = pair_forms(M, N, K, valid != nullptr, upto);
   const int blocks = blocks_of_forms(PAIR_PRICES, upto, N, forms);
   constexpr size_t lds = Tile256Four::LDS_BYTES;   // the largest tile's, more than the others'
   static_assert(lds >= (size_t)PAIR_STAGES * 3 * 128 * BK * 2 && lds >= (size_t)NT_STAGES * 256 * BK * 2, "the other bodies' stages fit too");
@@ -2839,6 +2849,39 @@ static bool gemm_direct_to_lds(int M, int N, int K, int b_col_maj, int c_col_maj
   return (M >= 64 && N >= 64) || K > 2 * BK;
 }
 
+// What a product without a bound takes, B (N,K) with C (N,M) turned round before: one answer for the launch, for the workspace and for whoever asks.
+// `deal`: how its tiles' K is shared where the caller brings a workspace.  Small tiles are the cheaper wherever they are one round, 128 tiles of 128 x 128
+// with a dimension of at most 64 among them (us, weights out of memory, half-empty 128 x 128 tiles / shared / small: 64 x 16384 x 8192 with B (K,N) 70 / 58 / 54,
+// 16384 x 64 71 / 87 / 59; 64 x 16320 x 200 6.0 unshared, 5.0 small).
+enum class GemmForm { FEW_ROWS, SMALL, BIG, TILES_64, TILES_128, GENERAL };
+struct GemmPlan {
+  GemmForm form;
+  SmallTiles small;
+  BigForm big;
+  TileShares deal;
+};
+static GemmPlan gemm_plan(int M, int N, int K, bool b_nk, bool c_nm) {
+  GemmPlan plan{GemmForm::GENERAL, {0, 0.f}, BIG_NONE, {0, 0, 0}};
+  if (b_nk && !c_nm && gemm_of_few_rows(M, N, K)) {   // fewer rows than the smallest tile: bound by streaming B
+    plan.form = GemmForm::FEW_ROWS;
+    return plan;
+  }
+  if (!gemm_direct_to_lds(M, N, K, b_nk, c_nm, false)) return plan;
+  const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
+  float big = 0.f, price128 = 0.f, shared = 0.f;
+  plan.small = small_tiles(M, N, K, b_nk);
+  if (!c_nm && tiles128 >= 128) plan.big = big_form(M, N, K, b_nk, big, price128);
+  // 128 x 128 tiles that would occupy under half the CUs give way to 64 x 64 ones, and so do tiles that up to 64 rows would half fill at
+  // most (64 x 16384 x 8184: 93 -> 68 us).
+  plan.form = plan.small.rows > 0 ? GemmForm::SMALL : (plan.big != BIG_NONE ? GemmForm::BIG : (b_nk && (tiles128 < 128 || M <= 64) ? GemmForm::TILES_64 : GemmForm::TILES_128));
+  const TileShares deal = gemm_shares_of_tiles(M, N, K, b_nk, &shared);
+  // (rows of B (K,N) that straddle cache lines cost the small tiles more, out of memory: 30 x 2776 x 3248 shared 16.1, by those 21.0; whole tiles of
+  // another size where they take no more)
+  const bool alone = plan.form == GemmForm::SMALL ? plan.small.us < (b_nk || N % BK == 0 ? 0.78f : 0.68f) * shared : plan.form == GemmForm::BIG && big + 3.f <= shared;
+  if (!alone) plan.deal = deal;
+  return plan;
+}
+
 extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K,
                               int b_col_maj, int c_col_maj, const int* valid, const int* valid_k,
                               void* stream) {
@@ -2853,41 +2896,28 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
     M = N, N = m;
     c_col_maj = 0;
   }
-  // Fewer rows than the smallest tile: bound by streaming B.
-  if (gemm_of_few_rows(M, N, K) && b_col_maj && !c_col_maj && valid == nullptr && valid_k == nullptr)
-    return iron_gemm_few_bf16(A, B, nullptr, C, M, N, K, 0, stream);
-  if (valid_k == nullptr && gemm_direct_to_lds(M, N, K, b_col_maj, c_col_maj, valid != nullptr)) {
-    const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-    if (c_col_maj) {
-      const SmallTiles small = tiles128 < 128 ? small_tiles(M, N, K, false) : SmallTiles{0, 0.f};
-      if (small.rows == 32) return launch_gemm_small<13, 1, 2, 2, true, true>(A, B, C, M, N, K, s);
-      if (small.rows == 64) return launch_gemm_small<10, 2, 2, 2, true, true>(A, B, C, M, N, K, s);
-      return launch_gemm_nt<true, false, 2, 4, true>(A, B, C, M, N, K, valid, s);
+  if (valid == nullptr && valid_k == nullptr) {
+    const GemmPlan plan = gemm_plan(M, N, K, b_col_maj, c_col_maj);
+    const bool high = plan.small.rows == 64;
+    switch (plan.form) {
+      case GemmForm::FEW_ROWS:
+        return iron_gemm_few_bf16(A, B, nullptr, C, M, N, K, 0, stream);
+      case GemmForm::SMALL:
+        if (b_col_maj) return high ? launch_gemm_small<13, 1, 4, 2>(A, B, C, M, N, K, s) : launch_gemm_small<20, 1, 2, 1>(A, B, C, M, N, K, s);
+        if (c_col_maj) return high ? launch_gemm_small<10, 2, 2, 2, true, true>(A, B, C, M, N, K, s) : launch_gemm_small<13, 1, 2, 2, true, true>(A, B, C, M, N, K, s);
+        return high ? launch_gemm_small<10, 2, 2, 2, true>(A, B, C, M, N, K, s) : launch_gemm_small<13, 1, 2, 2, true>(A, B, C, M, N, K, s);
+      case GemmForm::BIG:
+        return b_col_maj ? launch_gemm_big<false>(plan.big, A, B, C, M, N, K, nullptr, s) : launch_gemm_big<true>(plan.big, A, B, C, M, N, K, nullptr, s);
+      case GemmForm::TILES_64:
+        return launch_gemm_nt<false, false, 1>(A, B, C, M, N, K, nullptr, s);
+      case GemmForm::TILES_128:
+        if (b_col_maj) return launch_gemm_nt<false>(A, B, C, M, N, K, nullptr, s);
+        return c_col_maj ? launch_gemm_nt<true, false, 2, 4, true>(A, B, C, M, N, K, nullptr, s) : launch_gemm_nt<true>(A, B, C, M, N, K, nullptr, s);
+      case GemmForm::GENERAL:
+        break;
     }
-    if (valid == nullptr && tiles128 >= 128) {
-      float price, price128;
-      const BigForm form = big_form(M, N, K, b_col_maj, price, price128);
-      if (form != BIG_NONE)
-        return b_col_maj ? launch_gemm_big<false>(form, A, B, C, M, N, K, nullptr, s) : launch_gemm_big<true>(form, A, B, C, M, N, K, nullptr, s);
-    }
-    if (b_col_maj) {
-      if (valid != nullptr) return launch_gemm_rows(A, B, C, M, N, K, valid, s);
-      // 128x128 tiles that would occupy under half the CUs give way to 64x64 ones, and so do tiles that
-      // up to 64 rows would half fill at most (64 x 16384 x 8184: 93 -> 68 us).
-      if (tiles128 < 128 || M <= 64) {
-        const SmallTiles small = small_tiles(M, N, K, true);
-        if (small.rows == 32) return launch_gemm_small<20, 1, 2, 1>(A, B, C, M, N, K, s);
-        if (small.rows == 64) return launch_gemm_small<13, 1, 4, 2>(A, B, C, M, N, K, s);
-        return launch_gemm_nt<false, false, 1>(A, B, C, M, N, K, valid, s);
-      }
-      return launch_gemm_nt<false>(A, B, C, M, N, K, valid, s);
-    }
-    if (valid == nullptr && tiles128 < 128) {
-      const SmallTiles small = small_tiles(M, N, K, false);
-      if (small.rows == 32) return launch_gemm_small<13, 1, 2, 2, true>(A, B, C, M, N, K, s);
-      if (small.rows == 64) return launch_gemm_small<10, 2, 2, 2, true>(A, B, C, M, N, K, s);
-    }
-    return launch_gemm_nt<true>(A, B, C, M, N, K, valid, s);
+  } else if (valid_k == nullptr && gemm_direct_to_lds(M, N, K, b_col_maj, c_col_maj, true)) {
+    return b_col_maj ? launch_gemm_rows(A, B, C, M, N, K, valid, s) : launch_gemm_nt<true>(A, B, C, M, N, K, valid, s);
   }
   // 128x128 tiles fill the 256 CUs once at 2048x2048; narrower problems take 64-wide tiles.
   const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
@@ -2896,22 +2926,10 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
   return launch_gemm<64, 64, 2, 2>(A, B, C, M, N, K, b_col_maj, c_col_maj, valid, valid_k, s);
 }
 
-static TileShares gemm_shares(int M, int N, int K, bool b_nk, bool c_nm) {
-  if (b_nk && gemm_of_few_rows(M, N, K)) return TileShares{0, 0, 0};
-  float then = 0.f, big, price128;
-  const TileShares deal = gemm_shares_of_tiles(M, N, K, b_nk, &then);
-  if (const SmallTiles small = small_tiles(M, N, K, b_nk); deal.slices > 0 && small.rows > 0 && small.us < (b_nk || N % BK == 0 ? 0.78f : 0.68f) * then)
-    return TileShares{0, 0, 0};   // (rows of B (K,N) that straddle cache lines cost the small tiles more, out of memory: 30 x 2776 x 3248 shared 16.1, by those 21.0)
-  // (whole tiles of another size, where they take no more)
-  if (deal.slices > 0 && !c_nm && deal.whole + deal.shared >= 128 && big_form(M, N, K, b_nk, big, price128) != BIG_NONE && big + 3.f <= then)
-    return TileShares{0, 0, 0};
-  return deal;
-}
-
 extern "C" int64_t iron_gemm_workspace_bytes(int M, int N, int K, int b_col_maj, int c_col_maj) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 8 != 0) return 0;
   const bool turned = b_col_maj && c_col_maj;
-  const TileShares deal = gemm_shares(turned ? N : M, turned ? M : N, K, b_col_maj, c_col_maj && !turned);
+  const TileShares deal = gemm_plan(turned ? N : M, turned ? M : N, K, b_col_maj, c_col_maj && !turned).deal;
   return (int64_t)deal.slices * deal.shared * 128 * 128 * sizeof(float);
 }
 
@@ -2927,13 +2945,33 @@ extern "C" int iron_gemm_shared_bf16(const uint16_t* A, const uint16_t* B, uint1
     M = N, N = m;
     c_col_maj = 0;
   }
-  const TileShares deal = gemm_shares(M, N, K, b_col_maj, c_col_maj);
+  const TileShares deal = gemm_plan(M, N, K, b_col_maj, c_col_maj).deal;
   IRON_REQUIRE(deal.slices > 0, "gemm_shared: a product of %d x %d over %d shares no tiles (iron_gemm_workspace_bytes is 0)", M, N, K);
   hipStream_t s = (hipStream_t)stream;
   float* sums = (float*)workspace;
   if (b_col_maj) return launch_gemm_shared<false, false>(A, B, C, M, N, K, deal, sums, s);
   if (c_col_maj) return launch_gemm_shared<true, true>(A, B, C, M, N, K, deal, sums, s);
   return launch_gemm_shared<true, false>(A, B, C, M, N, K, deal, sums, s);
+}
+
+// What the launches above and below decide on the host, for whoever asks without a launch.
+extern "C" int iron_gemm_tile(int kind, int M, int N, int K, int b_col_maj, int c_col_maj, int rows) {
+  if (kind < 0 || kind > 3 || M <= 0 || N <= 0 || K <= 0 || K % 8 != 0 || K > (1 << 22) || N > (1 << 22)) return 0;
+  auto tile = [](int bm, int bn) { return bm << 16 | bn; };
+  if (kind > 0) {
+    int upto[16] = {};
+    const int live = rows < M ? rows : M, form = form_of_rows(kind == 3 ? pair_forms(M, N, K, true, upto) : rows_forms(M, N, K, true, kind == 1 || N % 8 == 0, upto), live);
+    return kind == 3 ? tile(PAIR_PRICES[form].bm, PAIR_PRICES[form].bn) : tile(ROWS_PRICES[form].bm, ROWS_PRICES[form].bn);
+  }
+  const bool turned = b_col_maj && c_col_maj;
+  const GemmPlan plan = gemm_plan(turned ? N : M, turned ? M : N, K, b_col_maj, c_col_maj && !turned);
+  switch (plan.form) {
+    case GemmForm::SMALL: return tile(plan.small.rows, b_col_maj ? 32 : 64);
+    case GemmForm::BIG: return tile(BIG_PRICES[plan.big].bm, BIG_PRICES[plan.big].bn);
+    case GemmForm::TILES_64: return tile(64, 64);
+    case GemmForm::TILES_128: return tile(128, 128);
+    default: return 0;
+  }
 }
 
 // A product over many rows whose epilogue reads a second (M, N) operand: the residual sum or the gate.

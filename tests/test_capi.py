@@ -65,6 +65,19 @@ def test_few_rows_over_a_long_k_share_no_tiles():
         assert (room(N, M, K, 1, 1) > 0) == shared, (N, M, K)
 
 
+def test_a_product_of_one_round_of_small_tiles_takes_them_or_shares_its_k():
+    """Up to 64 rows or columns against as many of the other as make 128 tiles of 128 x 128: where sharing a long K is given up because
+    small tiles are the cheaper, the launch takes small tiles, in every layout and up to the last column."""
+    lib = _lib.lib()
+    for K in (1024, 4096, 6200, 8192, 12288):
+        for few in (33, 64):
+            for many in (8192, 16256, 16264, 16320, 16384):
+                for M, N, b, c in ((few, many, 0, 0), (many, few // 8 * 8, 0, 0), (few, many, 0, 1), (many, few // 8 * 8, 0, 1), (many, 32, 1, 0), (32, many, 1, 1)):
+                    tile, room = lib.iron_gemm_tile(0, M, N, K, b, c, 0), lib.iron_gemm_workspace_bytes(M, N, K, b, c)
+                    assert tile in (32 << 16 | 64, 64 << 16 | 64, 64 << 16 | 32, 32 << 16 | 32, 0), (M, N, K, b, c, tile >> 16, tile & 65535, room)
+    assert lib.iron_gemm_workspace_bytes(64, 16384, 8192, 0, 0) == 0 and lib.iron_gemm_tile(0, 64, 16384, 8192, 0, 0, 0) == 64 << 16 | 64
+
+
 def test_bench_refuses_more_than_one_gpu():
     """``bench.py --gpus N`` with N above 1 exits with a message: this build is the one-GPU path."""
     import subprocess

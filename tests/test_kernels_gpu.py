@@ -165,6 +165,15 @@ def test_gemm_at_the_edges_of_tiles_and_stages(cuda, M, Kdim, N, b_col_maj, c_co
 
 
 @pytest.mark.parametrize("M,Kdim,N,b_col_maj,c_col_maj", [
+    (64, 200, 16384, False, False), (33, 264, 16264, False, False), (16384, 192, 64, False, True), (16321, 264, 40, False, False), (16384, 200, 32, True, False),
+    (31, 1096, 16383, True, True)])
+def test_gemm_small_tiles_of_one_whole_round(cuda, M, Kdim, N, b_col_maj, c_col_maj):
+    """As many small tiles as there are CUs, a row or a column of tiles long: 128 tiles of 128 x 128 would be half empty."""
+    assert K.lib().iron_gemm_tile(0, M, N, Kdim, b_col_maj, c_col_maj, 0) >> 16 in (32, 64)
+    test_gemm_at_the_edges_of_tiles_and_stages(cuda, M, Kdim, N, b_col_maj, c_col_maj)
+
+
+@pytest.mark.parametrize("M,Kdim,N,b_col_maj,c_col_maj", [
     (3329, 128, 3593, True, False), (3329, 192, 3592, False, False),                                   # 256 x 256 tiles
     (192, 136, 48000, True, False), (3840, 264, 2819, True, False), (1290, 200, 8200, False, False),   # 192 x 256
     (160, 200, 40963, True, False), (1025, 64, 7169, True, False), (1025, 72, 7176, False, False),     # 160 x 256
