@@ -1997,15 +1997,16 @@ static int form_of_rows(const FormTable& t, int rows) {
   const int run = (rows < 1 ? 0 : rows - 1) >> (6 + t.shift);
   return (int)(t.w[run >> 4] >> ((run & 15) * 4)) & 15;
 }
-// `best(rows)` for the most rows of every run up to M; `upto[form]`: the most rows a form is taken for.
+// `best(rows)` for the most rows of every run up to M, without a bound for M alone; `upto[form]`: the most rows a form is taken for.
 template <class Best>
-static FormTable form_table(int M, Best best, int* upto) {
+static FormTable form_table(int M, bool bounded, Best best, int* upto) {
   FormTable t{};
   while ((64L << t.shift) * 64 < M) ++t.shift;
   const long run = 64L << t.shift;
-  for (long rows = run, i = 0; rows < M + run; rows += run, ++i) {
+  for (long rows = bounded ? run : M, i = 0; rows < M + run; rows += run, ++i) {
     const int r = rows < M ? (int)rows : M, form = best(r);
-    t.w[i >> 4] |= (uint64_t)form << ((i & 15) * 4);
+    if (bounded) t.w[i >> 4] |= (uint64_t)form << ((i & 15) * 4);
+    else for (uint64_t& w : t.w) w = (uint64_t)form * 0x1111111111111111u;
     if (r > upto[form]) upto[form] = r;
   }
   return t;
@@ -2040,9 +2041,6 @@ static RowsForm rows_form(int rows, int M, int N, int K, bool whole) {
     if (form == first || us < price) best = (RowsForm)form, price = us;
   }
   return best;
-}
-static FormTable rows_forms(int M, int N, int K, bool bounded, bool whole, int* upto) {
-  return form_table(M, [&](int rows) { return (int)rows_form(bounded ? rows : M, M, N, K, whole); }, upto);
 }
 template <bool TAIL>
 __global__ __launch_bounds__(256) void gemm_rows_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, bf16_t* __restrict__ C,
@@ -2080,28 +2078,48 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const bf16_t* __restrict
 #undef IRON_ROWS
 }
 
-// The blocks of a launch whose forms are chosen by `forms`, up to the rows of `upto` each; sets the forms' orders.
-template <class Price, int FORMS>
-static int blocks_of_forms(const Price (&prices)[FORMS], const int (&upto)[FORMS], int N, FormTable& forms) {
-  int blocks = 1;
+// A launch whose blocks choose their form: the table that they choose by, and how many there are.
+struct FormPlan {
+  FormTable table;
+  int blocks;
+};
+template <class Price, int FORMS, class Best>
+static FormPlan form_plan(const Price (&prices)[FORMS], int M, int N, bool bounded, Best best) {
+  int upto[FORMS] = {};   // each form's grid covers the rows it is chosen for
+  FormPlan plan{form_table(M, bounded, best, upto), 1};
   for (int form = 0; form < FORMS; ++form) {
     // Tile rows rounded up to whole patches where that lets the XCD-aware order apply: the added
     // tiles lie past the bound any block of that tiling runs for, and leave at once.
     int tile_rows = (upto[form] + prices[form].bm - 1) / prices[form].bm;
     const int tile_cols = (N + prices[form].bn - 1) / prices[form].bn, whole = (tile_rows + 7) & ~7;
     if (tile_rows >= 8 && !patched_order(tile_rows, tile_cols) && patched_order(whole, tile_cols)) tile_rows = whole;
-    forms.patched |= (tile_rows >= 8 && patched_order(tile_rows, tile_cols)) << form;
-    if (tile_rows * tile_cols > blocks) blocks = tile_rows * tile_cols;
+    plan.table.patched |= (tile_rows >= 8 && patched_order(tile_rows, tile_cols)) << form;
+    if (tile_rows * tile_cols > plan.blocks) plan.blocks = tile_rows * tile_cols;
   }
-  return blocks;
+  return plan;
+}
+// Under a bound the plan is a price for every form and run of rows, 1.5 us of the host's time at 2048 rows and 3 at 4096 (asked for again 0.02), and follows
+// from the sizes alone: a thread keeps the last ones it made (a decoder layer has up to five).
+constexpr int PLANS_HELD = 16;
+struct HeldPlan {
+  int M, N, K, variant;   // M 0: none
+  FormPlan plan;
+};
+template <class Make>
+static FormPlan held_plan(HeldPlan (&held)[PLANS_HELD], int M, int N, int K, int variant, Make make) {
+  HeldPlan& h = held[((uint32_t)M * 31 + (uint32_t)N * 17 + (uint32_t)K / 8 * 7 + variant) % 251 % PLANS_HELD];
+  if (h.M != M || h.N != N || h.K != K || h.variant != variant) h = HeldPlan{M, N, K, variant, make()};
+  return h.plan;
+}
+static FormPlan rows_plan(int M, int N, int K, bool bounded, bool whole) {
+  auto make = [&] { return form_plan(ROWS_PRICES, M, N, bounded, [&](int rows) { return (int)rows_form(rows, M, N, K, whole); }); };
+  static thread_local HeldPlan held[PLANS_HELD];
+  return bounded ? held_plan(held, M, N, K, whole, make) : make();
 }
 
 static int launch_gemm_rows(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, const int* valid, hipStream_t s,
                             const QkvTail& tail = QkvTail{}) {
-  int upto[ROWS_FORMS] = {};
-  const bool whole = tail.residual == nullptr || N % 8 == 0;
-  FormTable forms = rows_forms(M, N, K, valid != nullptr, whole, upto);
-  const int blocks = blocks_of_forms(ROWS_PRICES, upto, N, forms);
+  const FormPlan plan = rows_plan(M, N, K, valid != nullptr, tail.residual == nullptr || N % 8 == 0);
   constexpr size_t lds = Tile256Four::LDS_BYTES;
   static_assert(lds >= (size_t)NT_STAGES * 256 * BK * 2, "the other bodies' stages fit too");
   static LdsOptIn opt_in[2];
@@ -2110,7 +2128,7 @@ static int launch_gemm_rows(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, 
     set_error("gemm: %s", hipGetErrorString(e));
     return (int)e;
   }
-  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), lds, s, A, B, C, M, N, K, valid, forms, tail);
+  hipLaunchKernelGGL(kernel, dim3(plan.blocks), dim3(256), lds, s, A, B, C, M, N, K, valid, plan.table, tail);
   IRON_LAUNCH_CHECK();
 }
 
@@ -2507,9 +2525,6 @@ static PairForm pair_form(int rows, int M, int N, int K) {
   }
   return best;
 }
-static FormTable pair_forms(int M, int N, int K, bool bounded, int* upto) {
-  return form_table(M, [&](int rows) { return (int)pair_form(bounded ? rows : M, M, N, K); }, upto);
-}
 __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __restrict__ A,
                                                               const bf16_t* __restrict__ Bg,
                                                               const bf16_t* __restrict__ Bu, bf16_t* __restrict__ G,
@@ -2544,11 +2559,14 @@ __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __re
 #undef IRON_PAIR
 }
 
+static FormPlan pair_plan(int M, int N, int K, bool bounded) {
+  auto make = [&] { return form_plan(PAIR_PRICES, M, N, bounded, [&](int rows) { return (int)pair_form(rows, M, N, K); }); };
+  static thread_local HeldPlan held[PLANS_HELD];
+  return bounded ? held_plan(held, M, N, K, 0, make) : make();
+}
 static int launch_gemm_gated_pair(const bf16_t* A, const bf16_t* Bg, const bf16_t* Bu, bf16_t* G, bf16_t* C, int M,
                                   int N, int K, const int* valid, int activation, hipStream_t s) {
-  int upto[PAIR_FORMS] = {};   // each form's grid covers the rows it is chosen for
-  FormTable forms = pair_forms(M, N, K, valid != nullptr, upto);
-  const int blocks = blocks_of_forms(PAIR_PRICES, upto, N, forms);
+  const FormPlan plan = pair_plan(M, N, K, valid != nullptr);
   constexpr size_t lds = Tile256Four::LDS_BYTES;   // the largest tile's, more than the others'
   static_assert(lds >= (size_t)PAIR_STAGES * 3 * 128 * BK * 2 && lds >= (size_t)NT_STAGES * 256 * BK * 2, "the other bodies' stages fit too");
   static LdsOptIn opt_in;
@@ -2556,7 +2574,7 @@ static int launch_gemm_gated_pair(const bf16_t* A, const bf16_t* Bg, const bf16_
     set_error("gemm_gated_pair: %s", hipGetErrorString(e));
     return (int)e;
   }
-  hipLaunchKernelGGL(gemm_gated_pair_kernel, dim3(blocks), dim3(256), lds, s, A, Bg, Bu, G, C, M, N, K, valid, forms, activation);
+  hipLaunchKernelGGL(gemm_gated_pair_kernel, dim3(plan.blocks), dim3(256), lds, s, A, Bg, Bu, G, C, M, N, K, valid, plan.table, activation);
   IRON_LAUNCH_CHECK();
 }
 
@@ -2959,8 +2977,8 @@ extern "C" int iron_gemm_tile(int kind, int M, int N, int K, int b_col_maj, int 
   if (kind < 0 || kind > 3 || M <= 0 || N <= 0 || K <= 0 || K % 8 != 0 || K > (1 << 22) || N > (1 << 22)) return 0;
   auto tile = [](int bm, int bn) { return bm << 16 | bn; };
   if (kind > 0) {
-    int upto[16] = {};
-    const int live = rows < M ? rows : M, form = form_of_rows(kind == 3 ? pair_forms(M, N, K, true, upto) : rows_forms(M, N, K, true, kind == 1 || N % 8 == 0, upto), live);
+    const FormPlan plan = kind == 3 ? pair_plan(M, N, K, true) : rows_plan(M, N, K, true, kind == 1 || N % 8 == 0);
+    const int form = form_of_rows(plan.table, rows < M ? rows : M);
     return kind == 3 ? tile(PAIR_PRICES[form].bm, PAIR_PRICES[form].bn) : tile(ROWS_PRICES[form].bm, ROWS_PRICES[form].bn);
   }
   const bool turned = b_col_maj && c_col_maj;

@@ -78,6 +78,33 @@ def test_a_product_of_one_round_of_small_tiles_takes_them_or_shares_its_k():
     assert lib.iron_gemm_workspace_bytes(64, 16384, 8192, 0, 0) == 0 and lib.iron_gemm_tile(0, 64, 16384, 8192, 0, 0, 0) == 64 << 16 | 64
 
 
+def test_what_a_bound_chooses_is_decided_once_for_the_same_sizes():
+    """A launch under a row bound prices every form for every run of rows: the same sizes again cost no more than a launch without a bound,
+    and more sizes than are held, or another thread, change no answer."""
+    import threading
+    import time
+
+    tile = _lib.lib().iron_gemm_tile
+
+    def best(*args):
+        times = []
+        for _ in range(9):
+            start = time.perf_counter()
+            for _ in range(300):
+                tile(*args)
+            times.append(time.perf_counter() - start)
+        return min(times)
+
+    assert best(1, 4096, 2048, 2048, 1, 0, 1000) < 2 * best(0, 4096, 2048, 2048, 1, 0, 0)
+    asked = [(kind, M, N, K, 1, 0, rows) for kind in (1, 2, 3) for M in (300, 2048, 4096, 5000) for N in (2048, 2056, 8192) for K in (448, 2048)
+             for rows in (1, 130, 300, 2048)]
+    first, again = [tile(*a) for a in asked], []
+    other = threading.Thread(target=lambda: again.extend(tile(*a) for a in reversed(asked)))
+    other.start()
+    other.join()
+    assert first == again[::-1] == [tile(*a) for a in asked] and len(set(first)) > 6
+
+
 def test_bench_refuses_more_than_one_gpu():
     """``bench.py --gpus N`` with N above 1 exits with a message: this build is the one-GPU path."""
     import subprocess
