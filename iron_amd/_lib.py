@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import warnings
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p
 from pathlib import Path
 
@@ -185,16 +186,29 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+class _LongWay:
+    """In the place of ``_calls`` where it does not load: every operator is checked and launched from Python."""
+
+    @staticmethod
+    def gemm(*_):
+        return None
+
+    gemv = mha_prefill = gemm
+
+
 @functools.lru_cache(maxsize=None)
 def native():
     """``_calls``, which checks and launches the plain case of an operator in one native call, on the entry points of
     ``lib()``; its functions return the entry point's code, or None for what is not that case.  A caller to whom
-    that is not 0 goes the long way, which does the work or raises."""
-    if not (LIB_PATH.parent / "_calls.so").exists():
-        raise IronHipError(f"{LIB_PATH.parent / '_calls.so'} is missing: build it with `python -m iron_amd.build`")
+    that is not 0 goes the long way, which does the work or raises; so does every call, 2 us the slower, where the module was not built
+    or was built for another torch, after a warning."""
     lib()
-    from . import _calls
-
+    try:
+        from . import _calls
+    except ImportError as why:
+        warnings.warn(f"iron_amd._calls does not load ({why}); operators are launched from Python, which takes the host 2 us a call more: "
+                      "build it for this torch with `python -m iron_amd.build`", RuntimeWarning, stacklevel=3)
+        return _LongWay
     _calls.bind(*(ctypes.cast(getattr(_lib, name), c_void_p).value for name in (
         "iron_gemm_bf16", "iron_gemm_workspace_bytes", "iron_gemm_shared_bf16", "iron_gemv_bf16_tuned", "iron_mha_prefill_bf16")))
     return _calls

@@ -62,22 +62,28 @@ def _run(cmd: list[str]) -> None:
 
 
 def _build_calls(objdir: Path) -> None:
-    """The Python module of ``calls.cpp``: host code over torch's tensors, no kernel."""
-    import torch
-    from torch.utils.cpp_extension import include_paths
-
-    libs = Path(torch.__file__).parent / "lib"
-    flags = ["-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1",
-             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
-    dirs = [*include_paths(), str(Path(_hipcc()).resolve().parent.parent / "include"), sysconfig.get_paths()["include"]]
+    """The Python module of ``calls.cpp``: host code over torch's tensors, no kernel; it takes torch's C++ headers.  Where it is not built
+    none is left from before: it calls the library's entry points by address."""
     part = objdir / CALLS.name
-    _run(["g++", *flags, *(f"-isystem{d}" for d in dirs), str(CSRC / "calls.cpp"), "-o", str(part), f"-L{libs}",
-          "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"])
-    os.replace(part, CALLS)
+    try:
+        import torch
+        from torch.utils.cpp_extension import include_paths
+
+        libs = Path(torch.__file__).parent / "lib"
+        flags = ["-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1",
+                 f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+        dirs = [*include_paths(), str(Path(_hipcc()).resolve().parent.parent / "include"), sysconfig.get_paths()["include"]]
+        _run([_hipcc(), *flags, *(f"-isystem{d}" for d in dirs), str(CSRC / "calls.cpp"), "-o", str(part), f"-L{libs}",
+              "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"])
+        os.replace(part, CALLS)
+    except BaseException:
+        CALLS.unlink(missing_ok=True)
+        raise
 
 
 def build(verbose: bool = False) -> Path:
-    """Compile every source and link the shared library; always recompiles."""
+    """Compile every source and link the shared library; always recompiles.  The library is in its place also where its host calls'
+    shortcut, which it works without, could not be built; that then raises."""
     hipcc = _hipcc()
     objdir = HERE / "build"
     objdir.mkdir(exist_ok=True)
@@ -86,19 +92,19 @@ def build(verbose: bool = False) -> Path:
 
     def compile_one(pair):
         src, obj = pair
-        if src is None:
-            return _build_calls(objdir)
         if verbose:
             print(f"hipcc {src.name}")
         _run([hipcc, *FLAGS, "-c", str(src), "-o", str(obj)])
 
     jobs = min(len(srcs), int(os.environ.get("MAX_JOBS", "8")))
     with ThreadPoolExecutor(max_workers=jobs) as pool:
-        list(pool.map(compile_one, [(None, CALLS), *zip(srcs, objs)]))
+        calls = pool.submit(_build_calls, objdir)
+        list(pool.map(compile_one, zip(srcs, objs)))
     # Linked beside its place and moved there whole: a build that is cut short leaves no half library.
     part = objdir / LIB.name
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(part), *map(str, objs)])
     os.replace(part, LIB)
+    calls.result()
     return LIB
 
 

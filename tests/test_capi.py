@@ -134,3 +134,54 @@ def test_native_calls_leave_what_is_not_plain_to_the_caller():
         K.gemm(a, a, a, M=8, N=8, K=8)
     with pytest.raises(TypeError, match="expected a torch tensor"):
         K.gemv([1.0], a, a, M=8, K=8)
+
+
+def test_operators_go_the_long_way_where_the_native_calls_do_not_load(monkeypatch):
+    """A tree without ``_calls``, or with one built for another torch: one warning, and the operators' own words for what they refuse."""
+    import sys
+    import warnings
+
+    import torch
+
+    import iron_amd
+    from iron_amd import kernels as K
+
+    monkeypatch.setitem(sys.modules, "iron_amd._calls", None)   # an import of it raises ImportError
+    monkeypatch.delattr(iron_amd, "_calls", raising=False)
+    _lib.native.cache_clear()
+    try:
+        a = torch.zeros(8, 8, dtype=torch.bfloat16)
+        with pytest.warns(RuntimeWarning, match="iron_amd._calls does not load"), pytest.raises(TypeError, match="A: expected a tensor on the GPU"):
+            K.gemm(a, a, a, M=8, N=8, K=8)
+        with warnings.catch_warnings():
+            warnings.simplefilter("error")
+            for call in (lambda: K.gemv(a, a, a, M=8, K=8), lambda: K.mha_prefill(a, a, a, a, heads=1, kv_heads=1, d=64, seq=1, kv_len=1)):
+                with pytest.raises(TypeError, match="expected a tensor on the GPU"):
+                    call()
+    finally:
+        _lib.native.cache_clear()
+
+
+def test_the_library_is_linked_where_the_native_calls_are_not_built(monkeypatch, tmp_path):
+    """A build whose native calls fail leaves the library, leaves no native calls of another build beside it, and says what failed."""
+    from iron_amd import build
+
+    (tmp_path / "csrc").mkdir()
+    (tmp_path / "csrc" / "calls.cpp").write_text("#error no headers")
+    (tmp_path / "csrc" / "one.hip").write_text("")
+    (tmp_path / "_calls.so").write_text("another build's")
+    ran = []
+
+    def run(cmd):
+        ran.append(cmd)
+        if any(str(c).endswith("calls.cpp") for c in cmd):
+            raise RuntimeError("no headers")
+        Path(cmd[cmd.index("-o") + 1]).write_text("built")
+
+    for name, value in (("HERE", tmp_path), ("CSRC", tmp_path / "csrc"), ("LIB", tmp_path / "lib.so"), ("CALLS", tmp_path / "_calls.so"), ("_run", run),
+                        ("_hipcc", lambda: "hipcc")):
+        monkeypatch.setattr(build, name, value)
+    with pytest.raises(RuntimeError, match="no headers"):
+        build.build()
+    assert (tmp_path / "lib.so").read_text() == "built" and not (tmp_path / "_calls.so").exists()
+    assert all(cmd[0] == "hipcc" for cmd in ran)

@@ -137,6 +137,25 @@ def test_native_calls_refuse_what_the_long_way_refuses_and_follow_the_stream(cud
     assert bool((out == 64).all())
 
 
+def test_the_native_calls_and_the_long_way_are_the_same_launches(cuda, monkeypatch):
+    """A product alone, one whose tiles are shared, a matrix-vector product and prompt attention, with the native calls and without: the same bits."""
+    rng = np.random.default_rng(17)
+    x = {n: dev(bf(rng, n), cuda) for n in (64 * 8192, 192 * 384, 384 * 64, 8192, 300 * 4 * 64)}
+
+    def run():
+        outs = [out_like((64, 64), cuda, fill=5.0), out_like((192, 64), cuda, fill=5.0), out_like((64,), cuda, fill=5.0), out_like((300 * 4 * 64,), cuda, fill=5.0)]
+        K.gemm(x[64 * 8192], x[64 * 8192], outs[0], M=64, N=64, K=8192, b_col_maj=True)
+        K.gemm(x[192 * 384], x[384 * 64], outs[1], M=192, N=64, K=384)
+        K.gemv(x[64 * 8192], x[8192], outs[2], M=64, K=8192)
+        K.mha_prefill(*(x[300 * 4 * 64],) * 3, outs[3], heads=4, kv_heads=4, d=64, seq=300, kv_len=300)
+        return outs
+
+    assert _lib.native().__name__ == "iron_amd._calls"
+    native = run()
+    monkeypatch.setattr(K, "native", lambda: _lib._LongWay)
+    assert all(torch.equal(a, b) and not bool((a == 5).all()) for a, b in zip(native, run()))
+
+
 @pytest.mark.parametrize("b_col_maj", [False, True])
 @pytest.mark.parametrize("c_col_maj", [False, True])
 @pytest.mark.parametrize("M,Kdim,N", [
