@@ -2019,26 +2019,42 @@ static FormTable form_table(int M, bool bounded, Best best, int* upto) {
 // The prices: rounds of blocks, as big_form, at what a round was measured to take with weights out of memory behind the launch's own 4.5 us (by 64 x 64,
 // 128 x 128 and 256 x 256 tiles alone and by all these, us: 2048 columns over 2048 with a residual, 640 rows 19.9 / 17.7, 1024 23.7 / 18.4; over 8192, 900
 // rows 68 / 52; 8192 over 2048, 256 rows 22.9 / 18.6, 640 42 / 26, 1024 43 / 34, 1280 50 / 39; 6144 over 2048, 1200 rows 54 / 32).
+// Up to K = 1024 a round is mostly its start and its end, which tiles with a second operand pay twice: prices of their own, [0] without one and [1] with, fitted to 1800
+// launches of every form, of which the cheapest by them takes 1.0002 of the best on average and 1.03 at the most (by the long K's prices 1.08 below
+// K = 512, 1.02 from there on, and up to 2.1: 2048 x 2560 x 64 by 64 x 64 tiles 15.5, by 192 x 128 7.2; 2048 x 6144 x 512 27.3 / 20.0).
 enum RowsForm { ROWS_32X32, ROWS_64X32, ROWS_64X64, ROWS_128X64, ROWS_128X128, ROWS_160X128, ROWS_192X128, ROWS_256X128, ROWS_160X256, ROWS_192X256, ROWS_256X256, ROWS_FORMS };
-struct RowsPrice {
-  int bm, bn;
+constexpr int SHORT_STAGES = 16;
+struct RoundPrice {
   float start, stage;
 };
-constexpr RowsPrice ROWS_PRICES[ROWS_FORMS] = {
-    {32, 32, 0.8f, 0.15f},   {64, 32, 0.8f, 0.2f},    {64, 64, 0.8f, 0.28f},   {128, 64, 2.f, 0.34f},   {128, 128, 4.f, 0.45f}, {160, 128, 3.4f, 0.52f}, {192, 128, 5.f, 0.57f},
-    {256, 128, 6.5f, 0.69f}, {160, 256, 8.f, 0.8f},   {192, 256, 9.f, 0.85f}, {256, 256, 15.f, 1.f},
+struct RowsPrice {
+  int bm, bn;
+  RoundPrice long_k, short_k[2];
 };
-// `whole`: the output's rows are pieces of 8 or the product has no second operand.
-static RowsForm rows_form(int rows, int M, int N, int K, bool whole) {
+constexpr RowsPrice ROWS_PRICES[ROWS_FORMS] = {
+    {32, 32, {0.8f, 0.15f}, {{2.f, 0.142f}, {2.2f, 0.146f}}},     {64, 32, {0.8f, 0.2f}, {{2.45f, 0.171f}, {2.85f, 0.17f}}},
+    {64, 64, {0.8f, 0.28f}, {{2.5f, 0.235f}, {3.3f, 0.235f}}},    {128, 64, {2.f, 0.34f}, {{3.05f, 0.357f}, {4.55f, 0.362f}}},
+    {128, 128, {4.f, 0.45f}, {{3.4f, 0.515f}, {5.1f, 0.53f}}},    {160, 128, {3.4f, 0.52f}, {{3.4f, 0.583f}, {5.4f, 0.6f}}},
+    {192, 128, {5.f, 0.57f}, {{3.9f, 0.645f}, {6.f, 0.665f}}},    {256, 128, {6.5f, 0.69f}, {{4.3f, 0.743f}, {9.f, 0.76f}}},
+    {160, 256, {8.f, 0.8f}, {{4.85f, 0.872f}, {10.5f, 0.93f}}},   {192, 256, {9.f, 0.85f}, {{5.5f, 0.9f}, {13.f, 0.96f}}},
+    {256, 256, {15.f, 1.f}, {{6.7f, 1.1f}, {20.f, 1.19f}}},
+};
+struct RowsChoice {
+  RowsForm form;
+  float us;
+};
+// `second`: the product has a second operand.
+static RowsChoice rows_form(int rows, int M, int N, int K, bool second) {
+  const int stages = (K + BK - 1) / BK;
   const RowsForm first = K < 8 * BK ? ROWS_64X64 : ROWS_32X32;   // (a short K does not fill the small tiles' many stages)
-  RowsForm best = first;
-  float price = 0.f;
+  RowsChoice best{first, 0.f};
   for (int form = first; form < ROWS_FORMS; ++form) {
     const RowsPrice& p = ROWS_PRICES[form];
-    if (form > ROWS_128X128 && (M < p.bm || N < p.bn || !whole)) continue;
+    if (form > ROWS_128X128 && (M < p.bm || N < p.bn || (second && N % 8 != 0))) continue;
+    const RoundPrice& of = stages > SHORT_STAGES ? p.long_k : p.short_k[second];
     const long tiles = (long)((rows + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
-    const float us = (float)((tiles + 255) / 256) * (p.start + p.stage * ((K + BK - 1) / BK));
-    if (form == first || us < price) best = (RowsForm)form, price = us;
+    const float us = (float)((tiles + 255) / 256) * (of.start + of.stage * stages);
+    if (form == first || us < best.us) best = {(RowsForm)form, us};
   }
   return best;
 }
@@ -2111,15 +2127,14 @@ static FormPlan held_plan(HeldPlan (&held)[PLANS_HELD], int M, int N, int K, int
   if (h.M != M || h.N != N || h.K != K || h.variant != variant) h = HeldPlan{M, N, K, variant, make()};
   return h.plan;
 }
-static FormPlan rows_plan(int M, int N, int K, bool bounded, bool whole) {
-  auto make = [&] { return form_plan(ROWS_PRICES, M, N, bounded, [&](int rows) { return (int)rows_form(rows, M, N, K, whole); }); };
+static FormPlan rows_plan(int M, int N, int K, bool bounded, bool second) {
+  auto make = [&] { return form_plan(ROWS_PRICES, M, N, bounded, [&](int rows) { return (int)rows_form(rows, M, N, K, second).form; }); };
   static thread_local HeldPlan held[PLANS_HELD];
-  return bounded ? held_plan(held, M, N, K, whole, make) : make();
+  return bounded ? held_plan(held, M, N, K, second, make) : make();
 }
-
 static int launch_gemm_rows(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, const int* valid, hipStream_t s,
                             const QkvTail& tail = QkvTail{}) {
-  const FormPlan plan = rows_plan(M, N, K, valid != nullptr, tail.residual == nullptr || N % 8 == 0);
+  const FormPlan plan = rows_plan(M, N, K, valid != nullptr, tail.residual != nullptr);
   constexpr size_t lds = Tile256Four::LDS_BYTES;
   static_assert(lds >= (size_t)NT_STAGES * 256 * BK * 2, "the other bodies' stages fit too");
   static LdsOptIn opt_in[2];
@@ -2977,7 +2992,7 @@ extern "C" int iron_gemm_tile(int kind, int M, int N, int K, int b_col_maj, int 
   if (kind < 0 || kind > 3 || M <= 0 || N <= 0 || K <= 0 || K % 8 != 0 || K > (1 << 22) || N > (1 << 22)) return 0;
   auto tile = [](int bm, int bn) { return bm << 16 | bn; };
   if (kind > 0) {
-    const FormPlan plan = kind == 3 ? pair_plan(M, N, K, true) : rows_plan(M, N, K, true, kind == 1 || N % 8 == 0);
+    const FormPlan plan = kind == 3 ? pair_plan(M, N, K, true) : rows_plan(M, N, K, true, kind == 2);
     const int form = form_of_rows(plan.table, rows < M ? rows : M);
     return kind == 3 ? tile(PAIR_PRICES[form].bm, PAIR_PRICES[form].bn) : tile(ROWS_PRICES[form].bm, ROWS_PRICES[form].bn);
   }

@@ -78,6 +78,20 @@ def test_a_product_of_one_round_of_small_tiles_takes_them_or_shares_its_k():
     assert lib.iron_gemm_workspace_bytes(64, 16384, 8192, 0, 0) == 0 and lib.iron_gemm_tile(0, 64, 16384, 8192, 0, 0, 0) == 64 << 16 | 64
 
 
+def test_short_products_under_a_bound_take_large_tiles_for_many_rows():
+    """Up to K = 1024 a round of tiles is mostly its start and its end: rows that make several rounds of 64 x 64 tiles take larger ones, fewer
+    of a product whose second operand its epilogue reads than of a plain one."""
+    tile = _lib.lib().iron_gemm_tile
+    for kind, M, N, K, want in ((1, 2048, 2560, 64, (192, 128)), (1, 2048, 3064, 64, (256, 128)), (1, 2048, 6144, 512, (256, 256)), (1, 2048, 1280, 128, (128, 128)),
+                                (2, 2048, 2560, 64, (192, 128)), (2, 2048, 1256, 128, (128, 128)), (2, 2048, 6144, 512, (128, 128)), (2, 256, 8376, 64, (128, 128)),
+                                (1, 1024, 4552, 192, (160, 128))):
+        got = tile(kind, M, N, K, 1, 0, M)
+        assert (got >> 16, got & 65535) == want, (kind, M, N, K, got >> 16, got & 65535)
+    for kind in (1, 2):   # (and few rows small ones)
+        for K in (64, 448, 512, 1024):
+            assert tile(kind, 2048, 1024, K, 1, 0, 40) in (64 << 16 | 64, 64 << 16 | 32, 32 << 16 | 32)
+
+
 def test_what_a_bound_chooses_is_decided_once_for_the_same_sizes():
     """A launch under a row bound prices every form for every run of rows: the same sizes again cost no more than a launch without a bound,
     and more sizes than are held, or another thread, change no answer."""
