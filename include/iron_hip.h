@@ -45,7 +45,7 @@ int iron_gemm_shared_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C, int
                           int c_col_maj, void* workspace, void* stream);
 /* The tile a product is made of, rows << 16 | columns of what a block computes (0: the few-row and the general kernels), as the launches decide
  * it on the host; for tests.  kind 0: M rows, no bound, no workspace; 1: under a bound of `rows` (B (N,K)); 2: iron_gemm_residual_bf16 and
- * iron_gemm_gated_bf16 under it; 3: iron_gemm_gated_pair_bf16 under it, columns of each product. */
+ * iron_gemm_gated_bf16 under it (0: without one); 3: iron_gemm_gated_pair_bf16 under it, columns of each product. */
 int iron_gemm_tile(int kind, int M, int N, int K, int b_col_maj, int c_col_maj, int rows);
 
 /* y[b] = W[b / repeat] @ x[b] for b in [0, batches): W (batches/repeat, M, K), x (batches, K),

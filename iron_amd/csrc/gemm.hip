@@ -2132,8 +2132,21 @@ static FormPlan rows_plan(int M, int N, int K, bool bounded, bool second) {
   static thread_local HeldPlan held[PLANS_HELD];
   return bounded ? held_plan(held, M, N, K, second, make) : make();
 }
+// Fewer than 128 tiles of 128 x 128 are 64 x 64 ones on 64 KB of LDS, two blocks a CU and their whole register file of 256 each, which the forms above leave to one
+// block: over a short K always (us, one a CU / two, with a second operand: 2048 x 528 x 256 6.6 / 5.5, 1024 x 1160 x 192 6.5 / 5.7, 2 rows of 256 x 4568 x 64 4.1 /
+// 3.6, which is the table's trip); over a longer one, where few rows have smaller tiles, without a bound and while there are more than one a CU and little of B for each
+// to wait for (2048 x 528 x 512 8.9 / 7.9, 2048 x 624 x 1024 11.7 / 11.0, 2048 x 960 x 1536 16.2 / 15.6; but 1024 x 1904 x 1024 13.0 / 13.9, 2048 x 960 x 4096
+// 30.2 / 31.3).  Under a bound and K of 512 and more the forms above stay: at the bound's most rows they take 0.5 to 1 us longer than two a CU,
+// at few rows 1 to 2 less (2048 x 568 x 960 under 119 rows 7.0 / 5.7).
+static bool two_a_cu(int M, int N, int K, bool bounded) {
+  const long tiles64 = (long)((M + 63) / 64) * ((N + 63) / 64);
+  if ((long)((M + 127) / 128) * ((N + 127) / 128) >= 128) return false;
+  return K < 8 * BK || (!bounded && tiles64 > 256 && tiles64 <= 512 && (long)N * K <= 3 << 19);
+}
+
 static int launch_gemm_rows(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, const int* valid, hipStream_t s,
                             const QkvTail& tail = QkvTail{}) {
+  if (two_a_cu(M, N, K, valid != nullptr)) return launch_gemm_nt<false, false, 1>(A, B, C, M, N, K, valid, s, tail);
   const FormPlan plan = rows_plan(M, N, K, valid != nullptr, tail.residual != nullptr);
   constexpr size_t lds = Tile256Four::LDS_BYTES;
   static_assert(lds >= (size_t)NT_STAGES * 256 * BK * 2, "the other bodies' stages fit too");
@@ -2992,8 +3005,9 @@ extern "C" int iron_gemm_tile(int kind, int M, int N, int K, int b_col_maj, int 
   if (kind < 0 || kind > 3 || M <= 0 || N <= 0 || K <= 0 || K % 8 != 0 || K > (1 << 22) || N > (1 << 22)) return 0;
   auto tile = [](int bm, int bn) { return bm << 16 | bn; };
   if (kind > 0) {
+    if (kind < 3 && two_a_cu(M, N, K, rows > 0)) return tile(64, 64);
     const FormPlan plan = kind == 3 ? pair_plan(M, N, K, true) : rows_plan(M, N, K, true, kind == 2);
-    const int form = form_of_rows(plan.table, rows < M ? rows : M);
+    const int form = form_of_rows(plan.table, rows > 0 && rows < M ? rows : M);
     return kind == 3 ? tile(PAIR_PRICES[form].bm, PAIR_PRICES[form].bn) : tile(ROWS_PRICES[form].bm, ROWS_PRICES[form].bn);
   }
   const bool turned = b_col_maj && c_col_maj;
