@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256) void poly_norm_kernel(const T* __restrict__ x,
   auto pieces = [&](const auto* p, float (&f)[CH][VEC]) {
     if constexpr (VEC == 8) {
       constexpr int SIZE = sizeof(*p), PARTS = SIZE / 2;
-      const __amdgpu_buffer_rsrc_t run = bounded_bytes(p, p != nullptr ? cols * SIZE : 0);
+      const __amdgpu_buffer_rsrc_t run = bounded_bytes(p, p != nullptr ? min(cols, CH * STEP) * SIZE : 0);   // (a whole row's bytes need not fit 32 bits)
       uint4 raw[CH][PARTS];
 #pragma unroll
       for (int i = 0; i < CH; ++i)

@@ -50,6 +50,19 @@ def test_a_gated_row_joins_the_stream(cuda, dtype, rows, cols, width, at):
         assert np.array_equal(from_torch(xd), added) and np.array_equal(from_torch(hd), want)
 
 
+def test_a_polynomial_over_a_row_of_more_bytes_than_32_bits_count(cuda):
+    """2^30 + 8 columns of float32, 32 bytes past 4 GiB, all but the first zero: those are read, and normed over the whole row."""
+    cols, held = (1 << 30) + 8, 9000
+    z = torch.from_numpy(np.random.default_rng(1).standard_normal(held).astype(F32))
+    x, y = torch.zeros(cols, device=cuda), torch.empty(cols, device=cuda)
+    x[:held] = z.to(cuda)
+    K.poly_norm(x, torch.tensor([0.5, -1.25, 0.75, 0.25], device=cuda).bfloat16(), y, rows=1, cols=cols, stride=cols, at=0, eps=1e-2)
+    z = z.numpy().astype(np.float64)
+    want = sum(c * z**n / np.sqrt((z ** (2 * n)).sum() / cols + 1e-2) for c, n in ((0.5, 1), (-1.25, 2), (0.75, 3))) + 0.25
+    got = y[:held].cpu().numpy()
+    assert np.abs(got - want).max() <= 2e-6 * np.abs(want).max() and bool((y[held:] == 0.25).all())
+
+
 @BOTH
 @pytest.mark.parametrize("rows,cols,stride,at", [(4, 96, 160, 0), (3, 37, 97, 5), (2, 2048, 4096, 2048), (2, 3000, 3000, 0), (1, 8200, 8208, 8), (1, 9001, 9001, 0)])
 def test_a_polynomial_of_normed_powers(cuda, dtype, rows, cols, stride, at):
