@@ -542,9 +542,12 @@ static int launch_gemm_strips(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
 // 3.1 / 3.5); up to 32 rows, whose sums take a second set of registers, over long rows
 // that keep to their lines (32 rows: 1024 x 2048 7.8 / 6.6, 4160 x 2048 13.8 / 9.5; but 2400 x 192 3.5 / 5.2) or a B of 64 MB (20 rows: 128256 x 2048 137 / 87).
 // A longer K: the strips of A that come with every tile cost as much as B's own.  Up to eight rows (2048 x 8192 13.9 / 8.9, 6000 x 6000 21.8 / 18.5,
-// 4096 x 14336 25.0 / 24.0, 4560 x 4416 19.5 / 12.6) but where they make two tiles a block of one round (3669 x 3168 8.0 / 8.3, 4096 x 4096 8.9 / 9.2);
-// up to 16 where a block has one tile (2048 x 8192 16.7 / 10.2) or three and more (4788 x 6848 28.6 / 21.2, 9762 x 9056 60.9 / 46.7; but 6576 x 5160
-// 21.5 / 22.3 and 3488 x 2696 7.4 / 8.5); more where that one's rows keep to their cache lines or are few (32 rows: 2048 x 4096
+// 4096 x 14336 25.0 / 24.0, 4560 x 4416 19.5 / 12.6; two tiles a block of one round too: 3904 x 3072 10.7 / 7.2, 3656 x 4160 12.9 / 8.9, and the same weights
+// again, out of the last-level cache, 8.8 / 8.4 and 11.5 / 10.1);
+// up to 16 where a block has one tile (2048 x 8192 16.7 / 10.2) or three and more (4788 x 6848 28.6 / 21.2, 9762 x 9056 60.9 / 46.7).  With
+// two tiles a block, or three and a half whose rows straddle lines, strips take the less of weights out of memory and gemm_few_kernel of the same weights again (3016 x
+// 4520 14.1 / 11.8 and 10.3 / 12.9, 2448 x 7456 17.8 / 16.3 and 12.5 / 17.4, 7562 x 2888 17.7 / 15.7 and 13.2 / 16.8): that kernel, which gains
+// more than it loses; more rows where that one's rows keep to their cache lines or are few (32 rows: 2048 x 4096
 // 13.2 / 12.2, 1024 x 8192 23.5 / 14.8; 20 rows of 1960 x 6512 13.8 / 15.1).  The loads go past the caches except where a block has
 // one tile over a long K (2048 x 8192, 8 rows: 9.3, past them 10.5; 4096 x 4096 10.1 and 9.4).
 // Returns -1 where it is not for them.
@@ -561,7 +564,6 @@ static int strips_for(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N,
   }
   if (M <= 8) {
     if (one_tile) return launch_gemm_strips<1, 8, false, 2, false>(A, B, C, M, N, K, s);
-    if (two_tiles && K >= 3072 && K < 4608) return -1;
     return launch_gemm_strips<1, 8, false, 2, true>(A, B, C, M, N, K, s);
   }
   if (M <= 16) {
