@@ -97,6 +97,18 @@ def test_short_products_under_a_bound_take_large_tiles_for_many_rows():
             assert tile(kind, 2048, 1024, K, 1, 0, 40) in (64 << 16 | 64, 64 << 16 | 32, 32 << 16 | 32)
 
 
+def test_large_products_without_a_bound_reach_every_size_of_tile():
+    """The sizes at which the GPU's tests take each large tile for their own, by what the launch chooses."""
+    tile = _lib.lib().iron_gemm_tile
+    for want, sizes in {(256, 256): [(3329, 128, 3593, 1, 0), (3329, 192, 3592, 0, 0)], (192, 256): [(192, 136, 48000, 1, 0), (3840, 264, 2819, 1, 0), (1290, 200, 8200, 0, 0)],
+                        (160, 256): [(160, 200, 40963, 1, 0), (1025, 64, 7169, 1, 0), (1025, 72, 7176, 0, 0)],
+                        (128, 256): [(641, 264, 8067, 1, 0), (777, 64, 6915, 1, 0), (641, 136, 5384, 0, 0)],
+                        (128, 192): [(128, 328, 33000, 1, 0), (641, 64, 5377, 1, 0), (3585, 200, 1025, 1, 1)]}.items():
+        for M, K, N, b, c in sizes:
+            got = tile(0, M, N, K, b, c, 0)
+            assert (got >> 16, got & 65535) == want, (M, K, N, b, c)
+
+
 def test_what_a_bound_chooses_is_decided_once_for_the_same_sizes():
     """A launch under a row bound prices every form for every run of rows: the same sizes again cost no more than a launch without a bound,
     and more sizes than are held, or another thread, change no answer."""

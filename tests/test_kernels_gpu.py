@@ -283,7 +283,7 @@ def test_gemm_large_squares_on_sampled_rows(cuda, n, b_col_maj):
 
 @pytest.mark.parametrize("M,Kdim,N", [(2048, 192, 6144), (4096, 64, 3072), (3072, 1152, 4096)])
 def test_gemm_large_tiles_with_b_as_stored_by_default(cuda, M, Kdim, N):
-    """B (K, N) through the 256 x 256 tiles (192 whole tiles or more): one stage, three, and
+    """B (K, N) through the 256 x 256 tiles and the 192 x 256 ones: one stage, three, and
     eighteen of them, every element against the oracle."""
     rng = np.random.default_rng(M + N + Kdim)
     A, B = bf(rng, M, Kdim), bf(rng, Kdim, N)
@@ -316,8 +316,8 @@ def test_gemm_ragged_shapes(cuda, M, Kdim, N, b_col_maj):
 @pytest.mark.parametrize("M,Kdim,N,rows", [(2048, 512, 8192, None), (2048, 64, 6144, None), (4096, 192, 4096, 1000), (4096, 192, 4096, 3000), (2048, 128, 2048, 512), (2048, 128, 2048, 1500), (2048, 192, 512, 700),
                                            (128, 64, 128, None), (256, 128, 192, None)])
 def test_gemm_weight_layout_fast_paths(cuda, M, Kdim, N, rows):
-    """B (N,K): the 256x256-tile kernel (>= 192 whole tiles) and the 128x128 one, down to a single
-    k stage, with a row bound that cuts through a tile."""
+    """B (N,K): tiles from 64 x 64 to 256 x 256, down to a single k stage, with a row bound that cuts
+    through a tile."""
     rng = np.random.default_rng(55)
     A, B = bf(rng, M, Kdim), bf(rng, N, Kdim, scale=0.1)
     want = ops.gemm(A, B, b_col_maj=True)
@@ -352,11 +352,11 @@ def test_gemm_direct_to_lds_tiles_at_ragged_edges(cuda, M, Kdim, N, b_col_maj):
 
 
 @pytest.mark.parametrize("M,Kdim,N,rows", [
-    # 64 x 64 tiles, eight stages (no more tiles than CUs): fewer k-stages than the pipeline is deep, an odd count, many
+    # 64 x 64 tiles, eight stages (no more tiles than CUs): fewer k-stages than the pipeline is deep, an odd count; 64 x 32 ones, many
     (512, 64, 2048, None), (512, 192, 2048, None), (512, 576, 2048, None), (448, 1024, 1024, None),
-    # 64 x 64 tiles, four stages (more tiles than CUs, too few for 128 x 128 ones): one stage, odd, even
+    # 64 x 64 tiles, four stages (more tiles than CUs, too few for 128 x 128 ones): one stage, odd; under a bound 128 x 64 ones, even
     (1024, 64, 1536, None), (1024, 320, 1536, None), (1024, 512, 1536, 1000),
-    # a row bound under which the blocks of one launch pick 64 x 64 tiles, short and odd in k
+    # a row bound under which the blocks of one launch pick 64 x 64 and 128 x 64 tiles, short and odd in k
     (2048, 64, 2048, 512), (2048, 192, 2048, 300), (2048, 576, 2048, 896), (2048, 576, 2048, 897)])
 @pytest.mark.parametrize("residual", [False, True])
 def test_gemm_small_tiles_at_every_depth(cuda, M, Kdim, N, rows, residual):
@@ -441,11 +441,11 @@ def test_gemm_rows_of_every_alignment(cuda, M, Kdim, N, b_col_maj, c_col_maj, co
 
 
 @pytest.mark.parametrize("M,Kdim,N,b_col_maj,bounds", [
-    (2000, 136, 8195, True, (130, 257, 513, 641, 769, 1025, 1281, 1537, 1999)),   # every form by the bound, the last tiles moved back
-    (2048, 200, 8192, True, (1, 128, 129, 1024, 1025, 2047)),    # 64, 128 and 256 tiles by the bound
+    (2000, 136, 8195, True, (130, 257, 513, 641, 769, 1025, 1281, 1537, 1999)),   # 128 x 128 to 256 x 256 by the bound, the last tiles moved back
+    (2048, 200, 8192, True, (1, 128, 129, 1024, 1025, 2047)),    # 64 x 64 to 256 x 256 by the bound
     (1500, 328, 2056, True, (63, 895, 896, 897, 1500)),          # 64 and 128 ones, ragged
-    (2048, 1032, 2056, True, (1, 32, 33, 65, 128, 129, 200, 257, 400)), (300, 584, 200, True, (31, 64, 97, 299)),   # 32-column ones, ragged
-    (256, 136, 320, True, (0, 100, 200)), (40, 1000, 4168, True, (17, 40)), (33, 4096, 520, True, (1, 32)),   # 64 ones whatever the bound
+    (2048, 1032, 2056, True, (1, 32, 33, 65, 128, 129, 200, 257, 400)), (300, 584, 200, True, (31, 64, 97, 299)),   # 32-column ones and 64 x 64, ragged
+    (256, 136, 320, True, (0, 100, 200)), (40, 1000, 4168, True, (17, 40)), (33, 4096, 520, True, (1, 32)),   # 64 x 64, 64 x 32 and 32 x 32 ones whatever the bound
     (2048, 328, 2056, False, (1, 129, 1999)), (300, 200, 136, False, (299,)), (40, 264, 72, False, (17,)),    # (K,N): the last column tile moved back
     (64, 72, 128, False, (5,)), (2, 192, 4104, False, (1,))])
 def test_gemm_under_a_bound_at_the_edges_of_tiles_and_stages(cuda, M, Kdim, N, b_col_maj, bounds):
@@ -473,11 +473,71 @@ def test_gemm_under_a_bound_at_the_edges_of_tiles_and_stages(cuda, M, Kdim, N, b
         assert np.all(got[rows:] == 7.0), rows
 
 
+# Each form that a launch under a bound may take (K decides the price, so the sizes are each form's own), with a last row and column of tiles
+# that are no whole ones, which the larger forms move back over their neighbours'.
+ROWS_FORMS = {(32, 32): (75, 512, 80), (64, 32): (67, 512, 2808), (64, 64): (74, 64, 80), (128, 64): (132, 64, 8080), (128, 128): (131, 64, 8232),
+              (160, 128): (389, 64, 8200), (160, 256): (771, 64, 8256), (192, 128): (482, 64, 8200), (192, 256): (965, 64, 9224), (256, 128): (579, 64, 8208),
+              (256, 256): (1156, 64, 9224)}
+TAIL_FORMS = {(32, 32): (73, 512, 72), (64, 32): (67, 512, 2736), (64, 64): (68, 64, 72), (128, 64): (131, 64, 8088), (128, 128): (131, 64, 8208),
+              (160, 128): (387, 64, 8240), (160, 256): (774, 64, 9424), (192, 128): (481, 64, 8208), (192, 256): (966, 192, 9352), (256, 128): (579, 64, 8216),
+              (256, 256): (1413, 512, 8216)}
+PAIR_FORMS = [((64, 32), (81, 64, 80)), ((128, 64), (134, 64, 2752)), ((128, 128), (67, 64, 8320)), ((128, 128), (68, 64, 8232)), ((160, 64), (259, 64, 5504)),
+              ((160, 128), (387, 64, 8320)), ((192, 64), (323, 64, 5504)), ((192, 128), (481, 64, 8320)), ((224, 128), (579, 64, 8320)), ((256, 128), (674, 64, 8320))]
+
+
+@pytest.mark.parametrize("kind,tile,size", [*((k, *f) for k in ("plain", "residual", "gated") for f in (ROWS_FORMS if k == "plain" else TAIL_FORMS).items()),
+                                            *(("pair", *f) for f in PAIR_FORMS)])
+def test_every_form_of_a_launch_under_a_bound(cuda, kind, tile, size):
+    """Each size of tile, named by the launch's own choice, under a bound a few rows short of its last tile's end: against the oracle, rows
+    past the bound untouched; with a second operand also in place, where a tile moved back reads what its neighbour has
+    perhaps stored already, three times over the same bits."""
+    M, Kdim, N = size
+    rows = M - 2
+    code = K.lib().iron_gemm_tile({"plain": 1, "residual": 2, "gated": 2, "pair": 3}[kind], M, N, Kdim, 1, 0, rows)
+    assert (code >> 16, code & 65535) == tile
+    rng = np.random.default_rng(M + N)
+    A, B, B2, R = bf(rng, M, Kdim), bf(rng, N, Kdim, scale=0.05), bf(rng, N, Kdim, scale=0.05), bf(rng, M, N)
+    want, near = ops.gemm(A, B, b_col_maj=True), ops.gemm_bound(A, B, b_col_maj=True)
+    A[rows:] = np.nan
+    dA, dB, dR, bound = dev(A, cuda), dev(B, cuda), dev(R, cuda), word(rows, cuda)
+    kw = dict(M=M, N=N, K=Kdim, valid=bound)
+    C, G = out_like((M, N), cuda, fill=7.0), out_like((M, N), cuda, fill=7.0)
+    if kind == "plain":
+        K.gemm(dA, dB, C, b_col_maj=True, **kw)
+        product = C
+    elif kind == "pair":
+        K.gemm_gated_pair(dA, dB, dev(B2, cuda), G, C, activation="relu", **kw)
+        product = G
+    else:
+        product = out_like((M, N), cuda, fill=7.0)
+        K.gemm(dA, dB, product, b_col_maj=True, **kw)
+    assert np.all(np.abs(from_torch(product)[:rows] - want[:rows]) <= near[:rows]) and bool((product[rows:] == 7).all())
+    if kind == "pair":
+        up = out_like((M, N), cuda, fill=7.0)
+        K.gemm_gated(dA, dev(B2, cuda), G, up, activation="relu", **kw)
+        assert torch.equal(C[:rows], up[:rows]) and bool((C[rows:] == 7).all())
+    elif kind != "plain":
+        def run(to, R_):
+            if kind == "residual":
+                K.gemm_residual(dA, dB, R_, to, residual_scale=0.5, **kw)
+            else:
+                K.gemm_gated(dA, dB, R_, to, activation="relu", **kw)
+            return to
+
+        run(C, dR)
+        p = from_torch(product)[:rows]   # the product as the separate launch rounds it
+        link = round_bf16(np.float32(0.5) * p + R[:rows]) if kind == "residual" else ops.mul(np.maximum(R[:rows], 0), p)
+        assert np.array_equal(from_torch(C)[:rows], link) and bool((C[rows:] == 7).all())
+        for _ in range(3):
+            held = dR.clone()
+            assert torch.equal(run(held, held)[:rows], C[:rows]) and torch.equal(held[rows:], dR[rows:])
+
+
 @pytest.mark.parametrize("M,Kdim,N,form", [(*s, f) for s in ((2048, 2048, 2048), (2048, 1024, 8192), (1500, 320, 4160))
                                            for f in ("plain", "residual", "gated", "pair")] +
                          [(2048, 200, 8192, "plain"), (2048, 128, 5632, "pair"), (2000, 192, 888, "pair")])
 def test_a_row_s_products_are_the_same_bits_under_every_bound(cuda, M, Kdim, N, form):
-    """A bound on the rows chooses the tile (64, 128 or 256 rows of it), and with it nothing about a row's sums: what a row
+    """A bound on the rows chooses the tile (from 32 x 32 to 256 x 256), and with it nothing about a row's sums: what a row
     becomes does not depend on how many others there are."""
     rng = np.random.default_rng(M + N)
     A, B, B2, R = (dev(bf(rng, *s, scale=x), cuda) for s, x in (((M, Kdim), 1.0), ((N, Kdim), 0.05), ((N, Kdim), 0.05), ((M, N), 1.0)))
@@ -592,7 +652,7 @@ def test_prefill_qkv_writes_k_and_v_into_the_cache_rows(cuda, rows, bound, start
 @pytest.mark.parametrize("M,Kdim,N,rows,scale", [(2048, 512, 2048, None, 1.0), (2048, 256, 2048, 512, 1.0),
                                                  (2048, 256, 2048, 1500, 0.22), (256, 128, 512, 100, 1.0),
                                                  (128, 64, 64, None, -0.5), (4096, 192, 1024, 3000, 1.0),
-                                                 # tiles of 128, 160, 192 and 256 rows and columns, the last moved back over its neighbour
+                                                 # tiles of 128, 160, 192 and 256 rows by 128 and 256 columns, the last moved back over its neighbour
                                                  *[(2000, 128, 8200, rows, 1.0) for rows in (200, 641, 769, 1025, 1281, 1537, 2000, None)]])
 def test_gemm_residual_epilogue(cuda, M, Kdim, N, rows, scale):
     """A projection over many rows with its residual in the epilogue: the product rounded as the
@@ -751,7 +811,7 @@ def test_gemm_gated_epilogue(cuda, M, Kdim, N, rows, activation):
 def test_gemm_gated_pair_is_the_two_launches_bit_for_bit(cuda, M, Kdim, N, rows, activation):
     """Both first projections of a gated feed-forward in one launch: the gate's product and the gated
     output against the two launches they replace (the gate's GEMM, then the gated GEMM) bit for bit --
-    under row bounds that pick the 256-row tiles, the 128 x 128 ones, the 64 x 64 ones and none whole -- and the gate's
+    under row bounds that pick every size of tile, and none whole -- and the gate's
     product against the oracle's GEMM; rows past the bound are left as they were.  The first case is
     Llama-3.2-1B's prompt chunk."""
     rng = np.random.default_rng(M + N + 3)
