@@ -71,7 +71,7 @@ int iron_gemm_residual_bf16(const uint16_t* A, const uint16_t* B, const uint16_t
  * C = bf16(residual_scale * bf16(A B^T) + R), Y = RMSNorm(C) * gain as iron_rmsnorm_bf16 computes it
  * (Y is bit for bit what that call makes of C), for the rows under *valid (or M), in two launches.
  * While the bound leaves 128 x 128 tiles for no more than half the chip (512 live rows of a 2048-row
- * prompt chunk at N = 2048), each tile's K is dealt over 4 or 2 blocks that leave float32 sums in
+ * prompt chunk at N = 2048), each tile's K is dealt over 16, 8, 4 or 2 blocks that leave float32 sums in
  * `workspace`, and the second launch adds a row's slices in slice order before it rounds: the sums
  * are the same whatever ran first, and differ from iron_gemm_residual_bf16's in the last bits of the
  * float32 sum only.  A (M,K), B (N,K), R and C (M,N), gain (N), Y (M,N); C may be R, Y neither.

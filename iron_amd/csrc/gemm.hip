@@ -7,8 +7,8 @@
 // double-buffered; a wave owns a (BM/WM) x (BN/WN) sub-tile as 32x32x16 MFMA tiles; B as (K,N) is
 // transposed on its way into LDS (a thread loads a 4(k) x 8(n) patch and writes eight 8-byte
 // k-runs).  The fast ones (K at least 64, no bound on K) feed LDS straight from global memory
-// and come in four tile sizes: 64 x 64, 128 x 128, 128 x 192 / 128 x 64 for the fused projections,
-// and 256 x 256; each is described where it stands.
+// and come in tiles from 32 x 32 to 256 x 256, each described where it stands: gemm_plan says which a product takes,
+// by small_tiles' and BIG_PRICES; a launch under a row bound chooses by ROWS_PRICES, a gated pair by PAIR_PRICES.
 //
 // For a row-major C the MFMA is issued with the operands swapped (B tile as the "A" operand), so a
 // lane ends up holding 4 consecutive columns of one row of C and stores them as 8 bytes.
@@ -274,7 +274,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(const bf16_t* __restrict__ A,
 
 
 // ---------------------------------------------------------------------------
-// Fast paths: A (M,K) K-contiguous, K a multiple of 64, row-major C.
+// Fast paths: A (M,K) K-contiguous, K a multiple of 8 from 64 on, C (M,N) or, of B (K,N), (N,M).
 //
 // Tiles stream global -> LDS directly (buffer loads with the LDS bit: no VGPR staging, and the
 // L2 -> CU path delivers more per clock to LDS than to registers), several stages deep.  A wave
@@ -2748,7 +2748,7 @@ static int launch_gemm_big_as(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
 // Whole tiles larger than 128 x 128, by how the rounds they make over the chip's 256 CUs come out: a round of a tile was measured
 // to take `start` us (its entry, first loads and stores) and `stage` for each 64 of K, `loose` where rows straddle cache lines; [0] with B (N,K), [1] (K,N).
 // The stage grows with the tile's area, so what a product gains is the part of its rounds that is not filled (us, by 128 x 128 or 256 x 256 tiles
-// alone and by the tile chosen here): 777 x 10240 x 2560 59 -> 47, 2012 x 3008 x 1608 34.4 -> 24.4, 2856 x 2325 x 3176 77 -> 51, 1636 x 5256 x 6200 with
+// alone and by the tile chosen here): 777 x 10240 x 2560 53 -> 37 (weights out of memory 63 -> 50), 2012 x 3008 x 1608 34.4 -> 24.4, 2856 x 2325 x 3176 77 -> 51, 1636 x 5256 x 6200 with
 // B (K,N) 153 -> 119, 908 x 5328 x 344 with B (K,N) 14.8 -> 9.9, 3000 x 3000 x 3000 74 -> 54.
 enum BigForm { BIG_NONE, BIG_256, BIG_192X256, BIG_160X256, BIG_128X256, BIG_128X192, BIG_FORMS };
 struct BigPrice {

@@ -51,7 +51,7 @@ __host__ __device__ __forceinline__ bool few_rows_pay(int groups, int keys) { re
 constexpr int kFewBlocks = 512;          // launches of fewer blocks than this halve their blocks' queries (S = 1024 at 32 heads: 18.5 -> 13.9 us)
 constexpr int kWideBigBlocks = 512;     // wide heads: launches of at least this many 128-query blocks keep that size
 // Launches of up to this many blocks split each block's tiles over two halves of eight waves, which halves a block's chain of tiles; more fill the chip better
-// four waves each.  64-wide heads (two eight-wave blocks share a CU): S = 8192 at 32 heads 365 -> 353-360 us split, S = 16384 not.  128-wide ones (two
+// four waves each.  64-wide heads (two eight-wave blocks share a CU): S = 8192 at 32 heads 365 -> 353-360 us split, past S = 16384 not.  128-wide ones (two
 // four-wave blocks, which read a tile's keys ahead) would be the faster unsplit from 560 blocks on (32 heads, split against not, 2048 queries 45.4 / 52.4, 2305
 // 63.6 / 59.8, 3001 90.4 / 81.8, 4096 147 / 135; 16 heads, 6000 159 / 155), but split, a query has a reference for each half of its tiles, so that the
 // largest weight of either is 1, which bf16 holds exactly: 3001 queries are 0.00208 from 64 bits split and 0.00211 not (the output's own rounding
@@ -97,7 +97,7 @@ __device__ __forceinline__ void prefill_few_rows(
       const_cast<bf16_t*>(Vh + (long)kv_lo * kv_row_stride), 0, reach, 0x00020000);
   // Load i covers tile rows i RPI + l.  A row starts on a multiple of its head's bytes, so the part of K's
   // swizzle that is the load's own is an XOR of the lane's offset.
-  static_assert(RPI % 4 == 0, "V's swizzle, 2 (row % 4), is the lane's alone");
+  static_assert(RPI % 4 == 0, "V's swizzle is by row % 4: the lane's alone");
   const int l = lane / CPR;
   const int k_lane = l * row_bytes + (((lane % CPR) ^ k_swizzle<D>(l)) << 4), v_lane = l * row_bytes + (((lane % CPR) ^ v_swizzle<D>(l)) << 4);
   char* stage = smem + wave * (2 * TILE);   // the wave's K tile, then its V tile
