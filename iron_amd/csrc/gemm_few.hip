@@ -538,18 +538,19 @@ static int launch_gemm_strips(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
 // Which products go by strips, by what both kernels took over three hundred shapes with weights out of memory (us, gemm_few_kernel against strips).
 // K up to eight strips: up to 16 rows of A (8 rows: 64 x 384 3.9 / 2.6, 1024 x 1024 4.4 / 2.9, 8192 x 2048 9.0 / 8.2, 16000 x 600 8.8 / 7.4, 128256 x 2048
 // 105 / 82; one row: 2048 x 2048 4.5 / 3.6, 7159 x 2048 8.1 / 7.7), but not many rows of B that are a cache line or less (6 rows: 3440 x 40 2.8 / 3.4)
-// nor, short of 1408 columns that straddle lines, those that make two tiles a block of gemm_few_kernel's one round (3000 x 1224 4.2 / 4.4, 2656 x 136
-// 3.1 / 3.5); up to 32 rows, whose sums take a second set of registers, over long rows
+// nor rows that straddle lines where they make two tiles a block of gemm_few_kernel's one round (212 shapes of K 1280 to 2047: strips take 1.07 to 1.24 of
+// its time; 2656 x 136 3.1 / 3.5); up to 32 rows, whose sums take a second set of registers, over long rows
 // that keep to their lines (32 rows: 1024 x 2048 7.8 / 6.6, 4160 x 2048 13.8 / 9.5; but 2400 x 192 3.5 / 5.2) or a B of 64 MB (20 rows: 128256 x 2048 137 / 87).
 // A longer K: the strips of A that come with every tile cost as much as B's own.  Up to eight rows (2048 x 8192 13.9 / 8.9, 6000 x 6000 21.8 / 18.5,
 // 4096 x 14336 25.0 / 24.0, 4560 x 4416 19.5 / 12.6; two tiles a block of one round too: 3904 x 3072 10.7 / 7.2, 3656 x 4160 12.9 / 8.9, and the same weights
-// again, out of the last-level cache, 8.8 / 8.4 and 11.5 / 10.1);
+// again, out of the last-level cache, 8.8 / 8.4 and 11.5 / 10.1; there rows that straddle lines from K = 8192 on: of 210 shapes short of it strips take 1.02 to 1.08 of the
+// other's time, one row of 2382 x 2488 5.4 / 6.0, past it 0.97, and go through the caches, which with the same weights again is 0.87 to 0.96 of going past them);
 // up to 16 where a block has one tile (2048 x 8192 16.7 / 10.2) or three and more (4788 x 6848 28.6 / 21.2, 9762 x 9056 60.9 / 46.7).  With
 // two tiles a block, or three and a half whose rows straddle lines, strips take the less of weights out of memory and gemm_few_kernel of the same weights again (3016 x
 // 4520 14.1 / 11.8 and 10.3 / 12.9, 2448 x 7456 17.8 / 16.3 and 12.5 / 17.4, 7562 x 2888 17.7 / 15.7 and 13.2 / 16.8): that kernel, which gains
 // more than it loses; more rows where that one's rows keep to their cache lines or are few (32 rows: 2048 x 4096
-// 13.2 / 12.2, 1024 x 8192 23.5 / 14.8; 20 rows of 1960 x 6512 13.8 / 15.1).  The loads go past the caches except where a block has
-// one tile over a long K (2048 x 8192, 8 rows: 9.3, past them 10.5; 4096 x 4096 10.1 and 9.4).
+// 13.2 / 12.2, 1024 x 8192 23.5 / 14.8; 20 rows of 1960 x 6512 13.8 / 15.1), and are not three or less (22 rows of 2 x 2688 6.2 / 6.9).  The loads go past the caches except where a block has
+// one tile over a long K (2048 x 8192, 8 rows: 9.3, past them 10.5; 4096 x 4096 10.1 and 9.4), or two of rows that straddle lines.
 // Returns -1 where it is not for them.
 static int strips_for(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s) {
   const bool one_tile = N <= 256 * STRIP_ROWS, two_tiles = !one_tile && N <= 512 * STRIP_ROWS, on_lines = K % 64 == 0;
@@ -558,12 +559,13 @@ static int strips_for(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N,
     if (M > 32 || (M > 16 && !long_rows && !large)) return -1;
     if (M > 16) return launch_gemm_strips<2, 16, true, 2, true>(A, B, C, M, N, K, s);
     if (!one_tile && K < 64) return -1;
-    if (two_tiles && !on_lines && K < 1408) return -1;
+    if (two_tiles && !on_lines) return -1;
     if (M <= 8) return launch_gemm_strips<1, 8, true, 2, true>(A, B, C, M, N, K, s);
     return launch_gemm_strips<1, 16, true, 2, true>(A, B, C, M, N, K, s);
   }
   if (M <= 8) {
-    if (one_tile) return launch_gemm_strips<1, 8, false, 2, false>(A, B, C, M, N, K, s);
+    if (two_tiles && !on_lines && K < 8192) return -1;
+    if (one_tile || (two_tiles && !on_lines)) return launch_gemm_strips<1, 8, false, 2, false>(A, B, C, M, N, K, s);
     return launch_gemm_strips<1, 8, false, 2, true>(A, B, C, M, N, K, s);
   }
   if (M <= 16) {
@@ -571,7 +573,7 @@ static int strips_for(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N,
     if (two_tiles || (!on_lines && N > 6144 && N < 8192 && K < 5632)) return -1;
     return launch_gemm_strips<1, 16, false, 1, true>(A, B, C, M, N, K, s);
   }
-  if (!one_tile) return -1;
+  if (!one_tile || N < STRIP_ROWS / 2) return -1;
   if (!on_lines && N > 1280) return -1;
   return M <= 32 ? launch_gemm_strips<2, 16, false, 2, false>(A, B, C, M, N, K, s) : launch_gemm_strips<4, 16, false, 2, false>(A, B, C, M, N, K, s);
 }
