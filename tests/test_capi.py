@@ -78,6 +78,15 @@ def test_a_product_of_one_round_of_small_tiles_takes_them_or_shares_its_k():
     assert lib.iron_gemm_workspace_bytes(64, 16384, 8192, 0, 0) == 0 and lib.iron_gemm_tile(0, 64, 16384, 8192, 0, 0, 0) == 64 << 16 | 64
 
 
+def test_few_rows_of_a_matrix_from_memory_share_its_k():
+    """With B (K,N) of more than 16 MB a tile of 64 columns draws a line of each row out of memory: too few of them to fill the chip share K instead, in
+    either order of C; a matrix that the caches hold, or one of more columns over a shorter K, stays on small tiles."""
+    room = _lib.lib().iron_gemm_workspace_bytes
+    for M, N, K, c, shared in ((59, 6144, 4712, 0, True), (1, 5120, 4336, 1, True), (9, 6144, 3824, 0, True), (1, 5120, 4088, 0, True), (10, 4096, 3776, 0, True),
+                               (10, 12288, 2736, 0, False), (16, 6144, 1024, 0, False), (29, 6144, 2040, 0, False), (8, 1024, 4096, 0, True)):
+        assert (room(M, N, K, 0, c) > 0) == shared, (M, N, K)
+
+
 def test_short_products_under_a_bound_take_large_tiles_for_many_rows():
     """Up to K = 1024 a round of tiles is mostly its start and its end: rows that make several rounds of 64 x 64 tiles take larger ones, fewer
     of a product whose second operand its epilogue reads than of a plain one."""
