@@ -2019,11 +2019,12 @@ static FormTable form_table(int M, bool bounded, Best best, int* upto) {
 // The prices: rounds of blocks, as big_form, at what a round was measured to take with weights out of memory behind the launch's own 4.5 us (by 64 x 64,
 // 128 x 128 and 256 x 256 tiles alone and by all these, us: 2048 columns over 2048 with a residual, 640 rows 19.9 / 17.7, 1024 23.7 / 18.4; over 8192, 900
 // rows 68 / 52; 8192 over 2048, 256 rows 22.9 / 18.6, 640 42 / 26, 1024 43 / 34, 1280 50 / 39; 6144 over 2048, 1200 rows 54 / 32).
-// Up to K = 1024 a round is mostly its start and its end, which tiles with a second operand pay twice: prices of their own, [0] without one and [1] with, fitted to 1800
-// launches of every form, of which the cheapest by them takes 1.0002 of the best on average and 1.03 at the most (by the long K's prices 1.08 below
-// K = 512, 1.02 from there on, and up to 2.1: 2048 x 2560 x 64 by 64 x 64 tiles 15.5, by 192 x 128 7.2; 2048 x 6144 x 512 27.3 / 20.0).
+// Up to K = 1536 a round is mostly its start and its end, which tiles with a second operand pay twice: prices of their own, [0] without one and [1] with, fitted to 1800
+// launches of every form up to 1024, of which the cheapest by them takes 1.0002 of the best on average and 1.03 at the most (by the long K's prices 1.08 below
+// K = 512, 1.02 from there on, and up to 2.1: 2048 x 2560 x 64 by 64 x 64 tiles 15.5, by 192 x 128 7.2; 2048 x 6144 x 512 27.3 / 20.0; from 1088 to 1536
+// 87 launches of few rows by many columns 1.002 and 1.11: 3 rows of 64 x 26574 x 1152 with a second operand by two rounds of 64 x 64 tiles 21.2, by one of 128 x 128 15.9).
 enum RowsForm { ROWS_32X32, ROWS_64X32, ROWS_64X64, ROWS_128X64, ROWS_128X128, ROWS_160X128, ROWS_192X128, ROWS_256X128, ROWS_160X256, ROWS_192X256, ROWS_256X256, ROWS_FORMS };
-constexpr int SHORT_STAGES = 16;
+constexpr int SHORT_STAGES = 24;
 struct RoundPrice {
   float start, stage;
 };

@@ -88,12 +88,12 @@ def test_few_rows_of_a_matrix_from_memory_share_its_k():
 
 
 def test_short_products_under_a_bound_take_large_tiles_for_many_rows():
-    """Up to K = 1024 a round of tiles is mostly its start and its end: rows that make several rounds of 64 x 64 tiles take larger ones, fewer
+    """Up to K = 1536 a round of tiles is mostly its start and its end: rows that make several rounds of 64 x 64 tiles take larger ones, fewer
     of a product whose second operand its epilogue reads than of a plain one."""
     tile = _lib.lib().iron_gemm_tile
     for kind, M, N, K, want in ((1, 2048, 2560, 64, (192, 128)), (1, 2048, 3064, 64, (256, 128)), (1, 2048, 6144, 512, (256, 256)), (1, 2048, 1280, 128, (128, 128)),
                                 (2, 2048, 2560, 64, (192, 128)), (2, 2048, 1256, 128, (128, 128)), (2, 2048, 6144, 512, (128, 128)), (2, 256, 8376, 64, (128, 128)),
-                                (1, 1024, 4552, 192, (160, 128))):
+                                (1, 1024, 4552, 192, (160, 128)), (2, 64, 26574, 1152, (128, 128)), (2, 64, 32000, 1216, (128, 128)), (1, 4, 20111, 1056, (128, 128))):
         got = tile(kind, M, N, K, 1, 0, M)
         assert (got >> 16, got & 65535) == want, (kind, M, N, K, got >> 16, got & 65535)
     # (two 64 x 64 tiles a CU: few tiles of a short K whatever the bound, of a longer one without a bound)
