@@ -2138,9 +2138,12 @@ static FormPlan rows_plan(int M, int N, int K, bool bounded, bool second) {
 // 3.6, which is the table's trip); over a longer one, where few rows have smaller tiles, without a bound and while there are more than one a CU and little of B for each
 // to wait for (2048 x 528 x 512 8.9 / 7.9, 2048 x 624 x 1024 11.7 / 11.0, 2048 x 960 x 1536 16.2 / 15.6; but 1024 x 1904 x 1024 13.0 / 13.9, 2048 x 960 x 4096
 // 30.2 / 31.3).  Under a bound and K of 512 and more the forms above stay: at the bound's most rows they take 0.5 to 1 us longer than two a CU,
-// at few rows 1 to 2 less (2048 x 568 x 960 under 119 rows 7.0 / 5.7).
+// at few rows 1 to 2 less (2048 x 568 x 960 under 119 rows 7.0 / 5.7).  Up to 64 rows, whose tiles are 64 x 64 whatever the bound, of more columns: over a short K as well
+// (one a CU / two: 2 x 32000 x 168 6.3 / 5.2, 64 x 19760 x 128 with a second operand 6.9 / 6.0; over 328 drawn ones 1.09), and to K = 1024 where there are more than two a CU
+// (19 drawn ones 1.13; up to two, K from 512 on, 70 of them 0.94).
 static bool two_a_cu(int M, int N, int K, bool bounded) {
   const long tiles64 = (long)((M + 63) / 64) * ((N + 63) / 64);
+  if (M <= 64 && (K < 8 * BK || (K < 16 * BK && tiles64 > 512))) return true;
   if ((long)((M + 127) / 128) * ((N + 127) / 128) >= 128) return false;
   return K < 8 * BK || (!bounded && tiles64 > 256 && tiles64 <= 512 && (long)N * K <= 3 << 19);
 }

@@ -98,7 +98,8 @@ def test_short_products_under_a_bound_take_large_tiles_for_many_rows():
         assert (got >> 16, got & 65535) == want, (kind, M, N, K, got >> 16, got & 65535)
     # (two 64 x 64 tiles a CU: few tiles of a short K whatever the bound, of a longer one without a bound)
     for kind, M, N, K, rows, want in ((1, 2048, 672, 192, 670, (64, 64)), (2, 2048, 528, 256, 0, (64, 64)), (2, 2048, 528, 512, 0, (64, 64)), (2, 2048, 624, 1024, 0, (64, 64)),
-                                      (2, 2048, 528, 512, 2048, (128, 64)), (2, 1024, 1904, 1024, 0, (128, 64)), (2, 2048, 568, 960, 119, (32, 32))):
+                                      (2, 2048, 528, 512, 2048, (128, 64)), (2, 1024, 1904, 1024, 0, (128, 64)), (2, 2048, 568, 960, 119, (32, 32)),
+                                      (1, 64, 28672, 192, 3, (64, 64)), (2, 64, 19760, 128, 64, (64, 64)), (1, 40, 36000, 960, 33, (64, 64))):
         got = tile(kind, M, N, K, 1, 0, rows)
         assert (got >> 16, got & 65535) == want, (kind, M, N, K, rows, got >> 16, got & 65535)
     for kind in (1, 2):   # (and few rows small ones)
