@@ -2825,13 +2825,14 @@ struct SmallTiles {
   int rows;
   float us;
 };
+// B (K,N) past 16 MB comes from memory, a line of a row at a time.
+static bool kn_from_memory(int N, int K) { return (long)N * K > 8000000; }
 static SmallTiles small_tiles(int M, int N, int K, bool b_nk) {
   const int columns = b_nk ? 32 : 64;
   const long low = (long)((M + 31) / 32) * ((N + columns - 1) / columns), high = (long)((M + 63) / 64) * ((N + columns - 1) / columns);
   const float stages = (float)((K + BK - 1) / BK);
   if (K < 3 * BK || high > 256) return {0, 0.f};
-  // (K,N): past 16 MB of B its rows come from memory, a line of each at a time.
-  const float from_memory = !b_nk && (long)N * K > 8000000 ? 0.08f : 0.f;
+  const float from_memory = !b_nk && kn_from_memory(N, K) ? 0.08f : 0.f;
   if (!b_nk && low <= 256) return {32, 3.f + stages * (0.165f + 0.02f * low / 256 + from_memory)};
   if (!b_nk) return {64, 3.2f + stages * (0.19f + 0.02f * high / 256 + from_memory)};
   if (low <= 256) return {32, 3.05f + stages * (0.108f + (K % BK == 0 ? 0.02f : 0.034f) * low / 256)};
@@ -2928,9 +2929,10 @@ static GemmPlan gemm_plan(int M, int N, int K, bool b_nk, bool c_nm) {
   plan.form = plan.small.rows > 0 ? GemmForm::SMALL : (plan.big != BIG_NONE ? GemmForm::BIG : (b_nk && (tiles128 < 128 || M <= 64) ? GemmForm::TILES_64 : GemmForm::TILES_128));
   const TileShares deal = gemm_shares_of_tiles(M, N, K, b_nk, &shared);
   // (small tiles against shared ones, us out of memory and with the same weights again: with B (K,N) 59 x 6144 x 4712 28.0 / 21.3 and 18.6 / 19.8, 9 x 6144 x 3824
-  // 21.5 / 18.8 and 14.1 / 17.9, 30 x 2776 x 3248 21.0 / 16.1, but 10 x 12288 x 2736 18.7 / 21.9 and 14.5 / 19.6: over 547 drawn shapes the form taken is within 0.4 % and 0.9 % of
-  // the better one on average, before the price from memory 1.3 % and 1.6 %; whole tiles of another size where they take no more)
-  const bool alone = plan.form == GemmForm::SMALL ? plan.small.us < (b_nk ? 0.78f : 0.9f) * shared : plan.form == GemmForm::BIG && big + 3.f <= shared;
+  // 21.5 / 18.8 and 14.1 / 17.9, but 10 x 12288 x 2736 18.7 / 21.9 and 14.5 / 19.6; rows of a smaller B (K,N) that straddle cache lines cost the small tiles more,
+  // 30 x 2776 x 3248 shared 16.1, by those 21.0; whole tiles of another size where they take no more)
+  const float line = !b_nk && kn_from_memory(N, K) ? 0.9f : (b_nk || N % BK == 0 ? 0.78f : 0.68f);
+  const bool alone = plan.form == GemmForm::SMALL ? plan.small.us < line * shared : plan.form == GemmForm::BIG && big + 3.f <= shared;
   if (!alone) plan.deal = deal;
   return plan;
 }

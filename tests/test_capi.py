@@ -83,7 +83,7 @@ def test_few_rows_of_a_matrix_from_memory_share_its_k():
     either order of C; a matrix that the caches hold, or one of more columns over a shorter K, stays on small tiles."""
     room = _lib.lib().iron_gemm_workspace_bytes
     for M, N, K, c, shared in ((59, 6144, 4712, 0, True), (1, 5120, 4336, 1, True), (9, 6144, 3824, 0, True), (1, 5120, 4088, 0, True), (10, 4096, 3776, 0, True),
-                               (10, 12288, 2736, 0, False), (16, 6144, 1024, 0, False), (29, 6144, 2040, 0, False), (8, 1024, 4096, 0, True)):
+                               (10, 12288, 2736, 0, False), (16, 6144, 1024, 0, False), (130, 72, 2504, 0, True), (29, 6144, 2040, 0, False), (8, 1024, 4096, 0, True)):
         assert (room(M, N, K, 0, c) > 0) == shared, (M, N, K)
 
 
