@@ -440,6 +440,33 @@ def test_gemm_rows_of_every_alignment(cuda, M, Kdim, N, b_col_maj, c_col_maj, co
     assert bool((buf[M * N:] == 3).all())
 
 
+@pytest.mark.parametrize("M,Kdim,N,form", [(8190, 136, 140, "plain"), (348, 168, 464, "(N,M)"), (12, 176, 1000, "(N,M)"), (1004, 64, 264, "(N,M)"), (131, 64, 8212, "residual"),
+                                           (131, 64, 8236, "bounded")])
+def test_gemm_rows_of_whole_pieces_and_a_half_of_one_round(cuda, M, Kdim, N, form):
+    """Output rows of four elements more than whole pieces, from 128 x 128 tiles that are one round: each leaves by halves, its last one alone, nothing past
+    the output's end and no row past the bound."""
+    c_col_maj, rows = form == "(N,M)", M - 2 if form in ("residual", "bounded") else M
+    code = K.lib().iron_gemm_tile({"residual": 2, "bounded": 1}.get(form, 0), M, N, Kdim, not c_col_maj, c_col_maj, rows if rows < M else 0)
+    assert code == 128 << 16 | 128 and (M if c_col_maj else N) % 8 == 4
+    rng = np.random.default_rng(M + N)
+    A, B, R = bf(rng, M, Kdim), bf(rng, *((Kdim, N) if c_col_maj else (N, Kdim)), scale=0.05), bf(rng, M, N)
+    kw = dict(b_col_maj=not c_col_maj, c_col_maj=c_col_maj)
+    want, near = ops.gemm(A, B, **kw), ops.gemm_bound(A, B, **kw)
+    buf = out_like((M * N + 64,), cuda, fill=3.0)
+    C = buf[: M * N].view(*((N, M) if c_col_maj else (M, N)))
+    bound = word(rows, cuda) if rows < M else None
+    if form == "residual":
+        K.gemm_residual(dev(A, cuda), dev(B, cuda), dev(R, cuda), C, M=M, N=N, K=Kdim, residual_scale=0.5, valid=bound)
+        near = near + 2.0**-8 * np.abs(0.5 * want + R)   # the sum's own rounding
+        want = np.float32(0.5) * want + R
+    else:
+        K.gemm(dev(A, cuda), dev(B, cuda), C, M=M, N=N, K=Kdim, valid=bound, **kw)
+    got = from_torch(C)
+    live = slice(None) if c_col_maj else slice(rows)
+    assert np.all(np.abs(got[live] - want[live]) <= near[live])
+    assert bool((buf[M * N:] == 3).all()) and (c_col_maj or np.all(got[rows:] == 3))
+
+
 @pytest.mark.parametrize("M,Kdim,N,b_col_maj,bounds", [
     (2000, 136, 8195, True, (130, 257, 513, 641, 769, 1025, 1281, 1537, 1999)),   # 128 x 128 to 256 x 256 by the bound, the last tiles moved back
     (2048, 200, 8192, True, (1, 128, 129, 1024, 1025, 2047)),    # 64 x 64 to 256 x 256 by the bound
