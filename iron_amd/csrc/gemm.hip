@@ -343,7 +343,10 @@ __device__ __forceinline__ void to_cache_rows(QkvTail& t, const int* __restrict_
 // panels it re-reads from its own L2.  Otherwise the tiles in bands of 8 tile rows, a band's columns one after the other, and an XCD
 // owns an eighth of that order in one piece: the weight tile that its blocks share crosses HBM once instead of once an XCD
 // (against tile rows dealt round-robin: 7058 x 12872 x 792 174 -> 157 us, 941 x 9386 x 5296 121 -> 112, 181 x 10780 x 272 8.5 -> 7.5).  A matrix more than
-// twice as tall as wide goes by columns for rows (2056 x 713 x 1136 12.9 -> 11.5).
+// twice as tall as wide goes by columns for rows (2056 x 713 x 1136 12.9 -> 11.5), and so does one of two bands or more that is more than a round of tiles: the tiles of
+// the last round, which few CUs share, then meet weights that the round before has read, where by rows they are the first to ask memory for theirs (K from 1024 on, weights out of
+// memory, 300 to 420 tiles: 2048 x 2560 x 8448 with the next norm dealt round-robin 142 us, by rows 163, by columns 140; over 870 drawn products of 128 x 128 tiles by columns 0.96
+// of by rows, with the same weights again 1.00).
 __device__ __forceinline__ void tile_of_block(int bid, int tiles_m, int tiles_n, int patched, int& tm, int& tn) {
   const int xcd = bid & 7, loc = bid >> 3;
   if (patched) {
@@ -353,7 +356,7 @@ __device__ __forceinline__ void tile_of_block(int bid, int tiles_m, int tiles_n,
     tn = (patch % patches_n) * 4 + (within >> 3);
   } else {
     const int tiles = tiles_m * tiles_n, at = xcd * (tiles >> 3) + min(xcd, tiles & 7) + loc;
-    const bool tall = tiles_m > 2 * tiles_n;
+    const bool tall = tiles_m > 2 * tiles_n || (tiles_m >= 12 && tiles > 288);
     const int across = tall ? tiles_n : tiles_m, along = tall ? tiles_m : tiles_n;
     // (eight by four tiles are an XCD's CUs; up to three left over join the last band)
     const int band = min(at / (8 * along), max(1, (across + 4) >> 3) - 1), first = band * 8;

@@ -192,6 +192,18 @@ def test_gemm_small_tiles_of_one_whole_round(cuda, M, Kdim, N, b_col_maj, c_col_
     test_gemm_at_the_edges_of_tiles_and_stages(cuda, M, Kdim, N, b_col_maj, c_col_maj)
 
 
+# tiles 14 x 24 and 17 x 21 of 128 x 128 (19 x 16 without a band left over), 17 x 24 of 256 x 256, 24 x 16 and 29 x 13 of 64 x 64
+@pytest.mark.parametrize("M,Kdim,N,b_col_maj,c_col_maj", [
+    (1700, 136, 3000, False, True), (2050, 72, 2600, False, True), (2400, 64, 2048, False, True), (4100, 64, 6000, True, False), (1536, 192, 1000, True, False),
+    (1850, 136, 780, True, False)])
+def test_gemm_of_more_than_a_round_of_tiles_by_columns(cuda, M, Kdim, N, b_col_maj, c_col_maj):
+    """Twelve rows of tiles and more, and more of them than a round: an XCD's tiles go by bands of columns, each tile computed and none left out."""
+    code = K.lib().iron_gemm_tile(0, M, N, Kdim, b_col_maj, c_col_maj, 0)
+    rows, cols = -(-M // (code >> 16)), -(-N // (code & 65535))
+    assert rows >= 12 and rows * cols > 288
+    test_gemm_at_the_edges_of_tiles_and_stages(cuda, M, Kdim, N, b_col_maj, c_col_maj)
+
+
 @pytest.mark.parametrize("M,Kdim,N,b_col_maj,c_col_maj", [
     (3329, 128, 3593, True, False), (3329, 192, 3592, False, False),                                   # 256 x 256 tiles
     (192, 136, 48000, True, False), (3840, 264, 2819, True, False), (1290, 200, 8200, False, False),   # 192 x 256
