@@ -2557,11 +2557,15 @@ constexpr PairPrice PAIR_PRICES[PAIR_FORMS] = {
     {128, 64, 4.f, 0.58f},   {160, 64, 4.5f, 0.64f},  {192, 64, 5.f, 0.73f},   {128, 128, 6.f, 0.90f},
     {160, 128, 6.5f, 1.12f}, {192, 128, 7.5f, 1.2f},  {224, 128, 8.5f, 1.36f}, {256, 128, 9.5f, 1.5f},
 };
+// Whole tiles of 128 x (128 + 128) are made by the body that takes edges up to K = 2048 (us, by gemm_big_body and by that, weights out of memory: 2048 x 2048 x 1920 33.5 / 29.6, x 960 20.9 /
+// 19.3, 1024 x 4096 x 512 15.4 / 14.2; 330 drawn ones 0.95, with the same weights again 0.93), past it by gemm_big_body (150 drawn ones 1.03 and 0.90).
 static PairForm pair_form(int rows, int M, int N, int K) {
   PairForm best = PAIR_64X32;
   float price = 0.f;
+  const bool edged = K < 32 * BK && M >= 128 && N % 128 == 0;
   for (int form = PAIR_64X32; form < PAIR_FORMS; ++form) {
-    const PairPrice& p = PAIR_PRICES[form];
+    if (edged && form == PAIR_128X128) continue;
+    const PairPrice& p = PAIR_PRICES[edged && form == PAIR_EDGED ? PAIR_128X128 : form];
     if (form > PAIR_EDGED && (M < p.bm || N % p.bn != 0)) continue;
     const long tiles = (long)((rows + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
     const float us = (float)((tiles + 255) / 256) * (p.start + p.stage * (K / BK));

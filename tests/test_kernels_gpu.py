@@ -520,7 +520,7 @@ ROWS_FORMS = {(32, 32): (75, 512, 80), (64, 32): (67, 512, 2808), (64, 64): (74,
 TAIL_FORMS = {(32, 32): (73, 512, 72), (64, 32): (67, 512, 2736), (64, 64): (68, 64, 72), (128, 64): (131, 64, 8088), (128, 128): (131, 64, 8208),
               (160, 128): (387, 64, 8240), (160, 256): (774, 64, 9424), (192, 128): (481, 64, 8208), (192, 256): (966, 192, 9352), (256, 128): (579, 64, 8216),
               (256, 256): (1413, 512, 8216)}
-PAIR_FORMS = [((64, 32), (81, 64, 80)), ((128, 64), (134, 64, 2752)), ((128, 128), (67, 64, 8320)), ((128, 128), (68, 64, 8232)), ((160, 64), (259, 64, 5504)),
+PAIR_FORMS = [((64, 32), (81, 64, 80)), ((128, 64), (134, 64, 2752)), ((128, 128), (67, 64, 8320)), ((128, 128), (68, 64, 8232)), ((128, 128), (131, 64, 8320)), ((128, 128), (131, 2048, 8320)), ((160, 64), (259, 64, 5504)),
               ((160, 128), (387, 64, 8320)), ((192, 64), (323, 64, 5504)), ((192, 128), (481, 64, 8320)), ((224, 128), (579, 64, 8320)), ((256, 128), (674, 64, 8320))]
 
 
