@@ -2557,8 +2557,8 @@ constexpr PairPrice PAIR_PRICES[PAIR_FORMS] = {
     {128, 64, 4.f, 0.58f},   {160, 64, 4.5f, 0.64f},  {192, 64, 5.f, 0.73f},   {128, 128, 6.f, 0.90f},
     {160, 128, 6.5f, 1.12f}, {192, 128, 7.5f, 1.2f},  {224, 128, 8.5f, 1.36f}, {256, 128, 9.5f, 1.5f},
 };
-// Whole tiles of 128 x (128 + 128) are made by the body that takes edges up to K = 2048 (us, by gemm_big_body and by that, weights out of memory: 2048 x 2048 x 1920 33.5 / 29.6, x 960 20.9 /
-// 19.3, 1024 x 4096 x 512 15.4 / 14.2; 330 drawn ones 0.95, with the same weights again 0.93), past it by gemm_big_body (150 drawn ones 1.03 and 0.90).
+// Whole tiles of 128 x (128 + 128) are made by the body that takes edges up to K = 2048 (us, by gemm_big_body and by that: 2048 x 2048 x 1920 33.5 / 29.6, x 960 20.9 / 19.3,
+// 1024 x 4096 x 512 15.4 / 14.2; 430 drawn ones 0.90 to 0.95 with weights that the last-level cache holds, 0.98 to 1.02 out of memory), past it by gemm_big_body (0.91 and 1.03).
 static PairForm pair_form(int rows, int M, int N, int K) {
   PairForm best = PAIR_64X32;
   float price = 0.f;
