@@ -117,6 +117,8 @@ def test_large_products_without_a_bound_reach_every_size_of_tile():
         for M, K, N, b, c in sizes:
             got = tile(0, M, N, K, b, c, 0)
             assert (got >> 16, got & 65535) == want, (M, K, N, b, c)
+    for M, N, K in ((8192, 1400, 1608), (32000, 1040, 3904), (749, 26520, 4912), (17071, 1384, 1384), (1274, 19568, 1976)):   # B (K,N), where 128 x 128 tiles take more than their price
+        assert tile(0, M, N, K, 0, 0, 0) != 128 << 16 | 128, (M, N, K)
 
 
 def test_what_a_bound_chooses_is_decided_once_for_the_same_sizes():
