@@ -551,7 +551,8 @@ static int launch_gemm_strips(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
 // more than it loses; more rows where that one's rows keep to their cache lines or are few (32 rows: 2048 x 4096
 // 13.2 / 12.2, 1024 x 8192 23.5 / 14.8; 20 rows of 1960 x 6512 13.8 / 15.1), and are not three or less (22 rows of 2 x 2688 6.2 / 6.9), past 32 rows from K = 2560 on,
 // or 3072 of rows that straddle lines (38 rows of 9 x 2200 7.1 / 8.9, 51 of 32 x 2080 8.3 / 9.5; of 110 drawn ones short of there strips take 1.05 to 1.29 of the other's time).  The loads go past the caches except where a block has
-// one tile over a long K (2048 x 8192, 8 rows: 9.3, past them 10.5; 4096 x 4096 10.1 and 9.4), or two of rows that straddle lines.
+// one tile over a long K (2048 x 8192, 8 rows: 9.3, past them 10.5; 4096 x 4096 10.1 and 9.4), or two of rows that straddle lines, or of more
+// than eight rows any number of these (309 drawn ones: through them 0.93 of gemm_few_kernel's time and 0.91 with the same weights again, past them 0.92 and 1.15).
 // Returns -1 where it is not for them.
 static int strips_for(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s) {
   const bool one_tile = N <= 256 * STRIP_ROWS, two_tiles = !one_tile && N <= 512 * STRIP_ROWS, on_lines = K % 64 == 0;
@@ -572,6 +573,7 @@ static int strips_for(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N,
   if (M <= 16) {
     if (one_tile) return launch_gemm_strips<1, 16, false, 1, false>(A, B, C, M, N, K, s);
     if (two_tiles || (!on_lines && N > 6144 && N < 8192 && K < 5632)) return -1;
+    if (!on_lines) return launch_gemm_strips<1, 16, false, 1, false>(A, B, C, M, N, K, s);
     return launch_gemm_strips<1, 16, false, 1, true>(A, B, C, M, N, K, s);
   }
   if (!one_tile || N < STRIP_ROWS / 2 || (M > 32 && K < (on_lines ? 2560 : 3072))) return -1;

@@ -433,7 +433,7 @@ def test_gemm_rows_that_are_no_whole_pieces(cuda, cols, form):
 @pytest.mark.parametrize("cols", [1, 2, 3, 5, 6, 7, 8])
 @pytest.mark.parametrize("M,Kdim,N,b_col_maj,c_col_maj", [
     (8, 2048, 1032, True, False), (30, 4096, 808, True, False),     # strips, a tile a block
-    (5, 1024, 16384, True, False), (16, 2048, 4096, True, False), (8, 3584, 2600, True, False), (5, 8200, 2600, True, False),   # ... several, also over a long K
+    (5, 1024, 16384, True, False), (16, 2048, 4096, True, False), (8, 3584, 2600, True, False), (5, 8200, 2600, True, False), (13, 2056, 6152, True, False),   # ... several, also over a long K
     (40, 264, 72, True, False), (9, 64, 8200, True, False), (7, 2056, 2600, True, False), (38, 2200, 8, True, False),   # few rows otherwise, 16 columns a block and 32
     (200, 200, 328, True, False), (24, 6200, 200, True, False),     # 64 x 64 tiles, shared tiles
     (136, 40, 200, True, False), (200, 40, 136, False, True),       # the general kernel, C as (M,N) and (N,M)
