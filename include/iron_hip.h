@@ -101,6 +101,9 @@ int iron_gemm_gated_bf16(const uint16_t* A, const uint16_t* B, const uint16_t* G
 int iron_gemm_gated_pair_bf16(const uint16_t* A, const uint16_t* Bg, const uint16_t* Bu, uint16_t* G,
                               uint16_t* C, int M, int N, int K, int activation, const int* valid,
                               void* stream);
+/* The same with the gate's product stored nowhere. */
+int iron_gemm_gated_product_bf16(const uint16_t* A, const uint16_t* Bg, const uint16_t* Bu, uint16_t* C,
+                                 int M, int N, int K, int activation, const int* valid, void* stream);
 
 /* One-row fusions of a decoder layer (no single counterpart in the reference: each replaces a run
  * of its steps, iron/lm/blocks.py:627-648,697-699,723-733, and rounds where those steps round).

@@ -18,7 +18,7 @@ in a prompt chunk's version (several rows, 64-wide heads),
 
   GEMM q/k/v (one input), RoPE q/k                       => iron_prefill_qkv_bf16
   ... and Copy k/v -> the chunk's cache rows             => iron_prefill_qkv_cache_bf16
-  GEMM (gate), GEMM (up), SiLU or GELU (tanh), Mul       => iron_gemm_gated_pair_bf16
+  GEMM (gate), GEMM (up), SiLU or GELU (tanh), Mul       => iron_gemm_gated_product_bf16
   GEMM (up), SiLU or GELU (tanh) of the gate, Mul        => iron_gemm_gated_bf16
   SiLU, ElementwiseMul (no such product before them)     => iron_silu_mul_bf16
   GEMM, ElementwiseAdd / AXPY (the residual)             => iron_gemm_residual_bf16
@@ -843,10 +843,11 @@ def plan(recording, tensor: Callable[[Any], Any], word: Callable[[Any], Any],
                                 launches=2, scratch_bytes=need)
         elif _name(s) == "GEMM" and (gated := gated_at(i + 1, s)) is not None:
             # a gated feed-forward's two first projections over many rows: one launch computes both
-            # products tile by tile, the activated gate riding the second one's epilogue
+            # products tile by tile, the activated gate riding the second one's epilogue; the gate's own, which
+            # nothing else reads, stays in the registers
             args, kw = gated
-            args = dict(A=args["A"], Bg=tensor(s.inputs["B"]), Bu=args["B"], G=args["G"], C=args["C"])
-            got = Fused("gemm_gated_pair", i, 4, lambda a=args, kw=kw: kernels.gemm_gated_pair(**a, **kw))
+            args = dict(A=args["A"], Bg=tensor(s.inputs["B"]), Bu=args["B"], C=args["C"])
+            got = Fused("gemm_gated_pair", i, 4, lambda a=args, kw=kw: kernels.gemm_gated_product(**a, **kw))
         elif _name(s) == "GEMM" and (gated := gated_at(i)) is not None:
             # a gated feed-forward's second projection over many rows: the activated gate rides its epilogue
             args, kw = gated

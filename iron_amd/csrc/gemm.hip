@@ -690,7 +690,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
     return;
   }
   if constexpr (PAIR) {
-    // The gate's waves leave their product, rounded as it is stored, in LDS for the others and store it; those make
+    // The gate's waves leave their product, rounded as it is stored, in LDS for the others and store it where it is asked for; those make
     // bf16(bf16(act(bf16 g)) * bf16 u) of it.
     float* gates = reinterpret_cast<float*>(smem_nt) + (wm * 64 + lane) * 17;
     block_barrier();   // every wave is done with the stages
@@ -700,6 +700,7 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
     }
     __syncthreads();
     if (wn == 0) {
+      if (gate_out == nullptr) return;
       C = gate_out;
     } else {
       float x[16], g[16];
@@ -1590,7 +1591,7 @@ static int launch_gemm(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N
 // The operands of a gated feed-forward's two first projections beyond the gate's own.
 struct GatedPair {
   const bf16_t* up;      // the up projection's weights, (N,K) as the gate's
-  bf16_t* gate_out;      // where the gate's product goes
+  bf16_t* gate_out;      // where the gate's product goes, if anywhere
   int activation;
 };
 
@@ -1871,7 +1872,7 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
 
   if constexpr (PAIR) {
     // Columns 0 .. NT / 2 - 1 of the wave's tiles are the gate's product, the rest the up projection's, of
-    // the same 8 NT columns of the output: the gate's product leaves as it is stored, then, made in the
+    // the same 8 NT columns of the output: the gate's product leaves as it is stored, where it is asked for, then, made in the
     // accumulators' own layout, bf16(bf16(act(bf16 g)) * bf16 u).
     constexpr int HT = NT / 2, OROWB = HT * 32 + 16, LPRW = HT * 2, ORPI = 64 / LPRW;   // (half a tile's columns at a time)
     constexpr int ROWS = MI * 16;   // of a wave
@@ -1894,13 +1895,15 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
     };
     // (The kind of gate is chosen once: asked an element, its branches made the lone wave of a SIMD wait 128 times over, and a
     // 2048 x 8192 x 2048 pair take 143 us instead of 130.)
+    if (pair.gate_out != nullptr) {
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
+      for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < HT; ++j)
-        *reinterpret_cast<uint2*>(ot + (i * 16 + fr) * OROWB + (j * 16 + 4 * kq) * 2) =
-            make_uint2(pack_bf16(acc[i][j][0], acc[i][j][1]), pack_bf16(acc[i][j][2], acc[i][j][3]));
-    leave(pair.gate_out);
+        for (int j = 0; j < HT; ++j)
+          *reinterpret_cast<uint2*>(ot + (i * 16 + fr) * OROWB + (j * 16 + 4 * kq) * 2) =
+              make_uint2(pack_bf16(acc[i][j][0], acc[i][j][1]), pack_bf16(acc[i][j][2], acc[i][j][3]));
+      leave(pair.gate_out);
+    }
     auto gated = [&](auto kind) {
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
@@ -2487,7 +2490,7 @@ __device__ __forceinline__ void gemm_nt16_pair_body(const bf16_t* __restrict__ A
 
   // Output through LDS, a product at a time: the wave lays its 64 x 64 out row-major (rows padded by
   // 16 bytes) and each lane then owns 8 consecutive columns of a row, so a row of the tile leaves as
-  // one 128-byte segment.  First the gate's product as it is stored; then, made in the accumulators'
+  // one 128-byte segment.  First the gate's product as it is stored, where it is asked for; then, made in the accumulators'
   // own layout, bf16(bf16(act(bf16 g)) * bf16 u).
   constexpr int OROWB = 64 * 2 + 16;
   char* ot = smem_nt + wave * (64 * OROWB);
@@ -2511,7 +2514,7 @@ __device__ __forceinline__ void gemm_nt16_pair_body(const bf16_t* __restrict__ A
     __builtin_amdgcn_wave_barrier();   // the rows are read before the next product overwrites them
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
-  if constexpr (!GROUPED) {
+  if (!GROUPED && G != nullptr) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -3134,10 +3137,12 @@ extern "C" int iron_gemm_gated_bf16(const uint16_t* A, const uint16_t* B, const 
   return gemm_with_tail("gemm_gated", A, B, G, C, M, N, K, tail, valid, stream);
 }
 
-extern "C" int iron_gemm_gated_pair_bf16(const uint16_t* A, const uint16_t* Bg, const uint16_t* Bu, uint16_t* G,
-                                         uint16_t* C, int M, int N, int K, int activation, const int* valid,
-                                         void* stream) {
-  IRON_REQUIRE(A && Bg && Bu && C && (G || M < 64), "gemm_gated_pair: null operand");
+// G may be null: the gate's product is then stored nowhere.  It is as many bytes as the output, behind each tile's last product, where nothing is left to
+// hide them under (weights out of memory, us with and without: 2048 x 8192 x 2048 111 / 107, 857 rows 52 / 50, 4096 x 14336 x 4096 699 / 677, 1024 x 4096 x 1024
+// 23.4 / 21.5, 200 rows of 2048 x 512 8.0 / 7.65).
+static int gemm_gated_pair(const uint16_t* A, const uint16_t* Bg, const uint16_t* Bu, uint16_t* G, uint16_t* C, int M, int N, int K, int activation,
+                           const int* valid, void* stream) {
+  IRON_REQUIRE(A && Bg && Bu && C, "gemm_gated_pair: null operand");
   IRON_REQUIRE(activation >= 1 && activation <= 3, "gemm_gated_pair: activation (%d) is 1 (SiLU), 2 (GELU, tanh form) or 3 (ReLU)",
                activation);
   if (M < 64 && valid == nullptr) return iron_gemm_few_bf16(A, Bg, Bu, C, M, N, K, activation, stream);
@@ -3149,6 +3154,18 @@ extern "C" int iron_gemm_gated_pair_bf16(const uint16_t* A, const uint16_t* Bg, 
   IRON_REQUIRE((((uintptr_t)A | (uintptr_t)Bg | (uintptr_t)Bu | (uintptr_t)G | (uintptr_t)C) & 15) == 0,
                "gemm_gated_pair: operands must be 16-byte aligned");
   return launch_gemm_gated_pair(A, Bg, Bu, G, C, M, N, K, valid, activation, (hipStream_t)stream);
+}
+
+extern "C" int iron_gemm_gated_pair_bf16(const uint16_t* A, const uint16_t* Bg, const uint16_t* Bu, uint16_t* G,
+                                         uint16_t* C, int M, int N, int K, int activation, const int* valid,
+                                         void* stream) {
+  IRON_REQUIRE(G || M < 64, "gemm_gated_pair: null operand");
+  return gemm_gated_pair(A, Bg, Bu, G, C, M, N, K, activation, valid, stream);
+}
+
+extern "C" int iron_gemm_gated_product_bf16(const uint16_t* A, const uint16_t* Bg, const uint16_t* Bu, uint16_t* C, int M, int N, int K, int activation,
+                                            const int* valid, void* stream) {
+  return gemm_gated_pair(A, Bg, Bu, nullptr, C, M, N, K, activation, valid, stream);
 }
 
 static int prefill_qkv(const uint16_t* x, const uint16_t* Wq, const uint16_t* Wk, const uint16_t* Wv,

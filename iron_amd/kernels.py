@@ -154,6 +154,19 @@ def gemm_gated_pair(A, Bg, Bu, G, C, *, M, N, K, activation="silu", valid=None):
                                           ptr(_word(valid, "valid")), current_stream()), "iron_gemm_gated_pair_bf16")
 
 
+def gemm_gated_product(A, Bg, Bu, C, *, M, N, K, activation="silu", valid=None):
+    """``gemm_gated_pair`` with the gate's product stored nowhere."""
+    kinds = GATES
+    if activation not in kinds:
+        raise ValueError(f"gemm_gated_product: activation {activation!r} is none of {sorted(kinds)}")
+    _numel(_dev(A, "A"), M * K, "A")
+    _numel(_dev(Bg, "Bg"), N * K, "Bg")
+    _numel(_dev(Bu, "Bu"), N * K, "Bu")
+    _numel(_dev(C, "C"), M * N, "C")
+    check(lib().iron_gemm_gated_product_bf16(ptr(A), ptr(Bg), ptr(Bu), ptr(C), M, N, K, kinds[activation], ptr(_word(valid, "valid")),
+                                             current_stream()), "iron_gemm_gated_product_bf16")
+
+
 def gemv_fused(W, x, y, *, M, K, W2=None, norm_w=None, eps=0.0, residual=None, residual_scale=1.0, epilogue=0):
     """One-row fusion: ``[RMSNorm ->] GEMV [-> + residual | gate/up -> SiLU -> Mul]``."""
     _numel(_dev(W, "W"), M * K, "W")

@@ -870,6 +870,19 @@ def test_gemm_gated_pair_is_the_two_launches_bit_for_bit(cuda, M, Kdim, N, rows,
     assert np.all(from_torch(C1)[lim:] == 7.0) and np.all(from_torch(G1)[lim:] == 7.0)
 
 
+# few rows; 64 x 32, edged, 128 x 64, 128 x 128 by both bodies and 256 x 128 tiles; a bound inside a tile
+@pytest.mark.parametrize("M,Kdim,N,rows", [(40, 128, 320, None), (192, 128, 320, 70), (1300, 128, 4100, None), (2000, 128, 8192, 200), (1024, 512, 4096, None),
+                                           (1024, 2048, 4096, 1000), (2048, 128, 8192, 1999)])
+def test_gemm_gated_product_is_the_pair_without_the_gate_s_own(cuda, M, Kdim, N, rows):
+    rng = np.random.default_rng(M + N)
+    A, Bg, Bu = (dev(bf(rng, *shape, scale=0.1), cuda) for shape in ((M, Kdim), (N, Kdim), (N, Kdim)))
+    G, want, got = (out_like((M, N), cuda, fill=7.0) for _ in range(3))
+    kw = dict(M=M, N=N, K=Kdim, activation="silu", valid=None if rows is None else word(rows, cuda))
+    K.gemm_gated_pair(A, Bg, Bu, G, want, **kw)
+    K.gemm_gated_product(A, Bg, Bu, got, **kw)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("bound", [None, 512, 1281])
 @pytest.mark.parametrize("cache", [False, True])
 def test_prefill_qkv_at_the_decoder_s_width(cuda, bound, cache):
