@@ -640,7 +640,12 @@ int iron_stream_product_bf16(int input, const void* x, const uint16_t* gain, con
  * norm_gru_strips: norm_strips by W (4 width, K), the row [zx | ux | gx | gate], of which packed (rows, 4 width) gets the gate alone, and
  * iron_min_gru of the rest, spans of one row at the most.
  * gated_strips: iron_stream_gated_rows of W times the bf16 rows x, plus y_bias (may be NULL), on stream_rows (rows, N), by gates
- * `gate_stride` apart. */
+ * `gate_stride` apart.
+ * latent_strips: iron_latent_rows of the rows x (whole 16-byte pieces; q_rank up to 2048, rank + rot up to 4096, up to 64 slots), and q (rows, N) =
+ * W (N, q_rank) times the queries' latents. */
+int iron_latent_strips_bf16(const uint16_t* x, const uint16_t* q_gain, const uint16_t* c_gain, const float* angles, const int* spans,
+                            const uint16_t* W, uint16_t* q, uint16_t* latents, uint16_t* shared_keys, int slots, int rows, int N, int stride,
+                            int q_rank, int rank, int rot, int turned, int angle_rows, int ring, float eps, void* stream);
 int iron_norm_strips_bf16(const float* x, const uint16_t* gain, float eps, float unit, const uint16_t* W, uint16_t* y, int rows, int N,
                           int K, void* stream);
 int iron_norm_gru_strips_bf16(const float* x, const uint16_t* gain, float eps, float unit, const uint16_t* W, const uint16_t* z_bias,

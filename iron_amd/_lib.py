@@ -153,6 +153,7 @@ SIGNATURES = {
     "iron_decode_delta_bf16": (c_int, [_P] * 9 + [c_int] * 11 + [c_float, _P]),
     "iron_norm_strips_bf16": (c_int, [_P, _P, c_float, c_float, _P, _P, c_int, c_int, c_int, _P]),
     "iron_norm_gru_strips_bf16": (c_int, [_P, _P, c_float, c_float] + [_P] * 7 + [c_int, c_int, c_int, c_int, _P]),
+    "iron_latent_strips_bf16": (c_int, [_P] * 9 + [c_int] * 10 + [c_float, _P]),
     "iron_gated_strips_bf16": (c_int, [_P] * 4 + [c_int, _P, _P, c_int, c_int, c_int, _P]),
     "iron_stream_product_bf16": (c_int, [c_int] + [_P] * 6 + [c_float, c_float, _P, c_int, c_int] + [_P] * 6),
     "iron_latent_query_bf16": (c_int, [_P] * 9 + [c_int] * 8 + [c_float, _P]),

@@ -35,7 +35,8 @@ in a batched decoder's decode step (bf16; a float32 stream, layers with a state)
   StreamNorm, GEMM (two to eight slots, as the next)     => iron_norm_strips_bf16
   ... and MinGRU, beside the gate its output joins by    => iron_norm_gru_strips_bf16
   GEMM, StreamGatedAdd                                   => iron_gated_strips_bf16
-  LatentRows, GEMV (the queries)                         => iron_latent_query_bf16
+  LatentRows, GEMM (the queries)                         => iron_latent_strips_bf16
+  LatentRows, GEMV (one slot)                            => iron_latent_query_bf16
   StreamNorm (groups), GEMV                              => iron_norm_product_bf16
   Hgrn2, HeadGate [, GatedColumns] (any slots)           => iron_decode_hgrn2_bf16
   CachedHeads, GlobalMHA [, GatedColumns] (any slots)    => iron_decode_heads_global_bf16, iron_mha_global
@@ -551,20 +552,27 @@ def plan(recording, tensor: Callable[[Any], Any], word: Callable[[Any], Any],
         return Fused("experts_tail", j, 3, lambda: kernels.experts_tail(**args, **kw), launches=2)
 
     def latent_query_at(j):
-        """The launch for a single slot's latents and the product of its queries -- or None."""
+        """The launch for up to eight rows' latents and the product of their queries -- or None."""
         s = steps[j]
         g = steps[j + 1] if j + 1 < len(steps) else None
         o, q = s.op, s.outputs["q"]
-        if not (g is not None and o.rows == 1 and o.slots == 1 and o.dtype is bfloat16 and bare(s) and gemv_row(g, q) and once(q)
-                and not any(n % 8 for n in (o.stride, o.q_rank, o.rank, o.rot, o.turned)) and o.rank + o.rot <= 4096
-                and o.q_rank + o.rank + o.rot <= 8192):
+        if not (g is not None and o.dtype is bfloat16 and bare(s) and once(q) and not any(n % 8 for n in (o.stride, o.q_rank, o.rank, o.rot, o.turned))):
+            return None
+        one = o.rows == 1 and o.slots == 1 and gemv_row(g, q) and o.rank + o.rot <= 4096 and o.q_rank + o.rank + o.rot <= 8192
+        few = (2 <= o.rows <= 8 and o.slots <= 64 and o.q_rank <= 2048 and o.rank + o.rot <= 4096 and _name(g) == "GEMM" and bare(g) and g.op.b_col_maj
+               and not g.op.c_col_maj and _same(g.inputs["A"], q) and g.op.M == o.rows and g.op.K == o.q_rank)
+        if not (one or few):
             return None
         args = dict(x=tensor(s.inputs["x"]).reshape(-1), q_gain=tensor(s.inputs["q_gain"]), c_gain=tensor(s.inputs["c_gain"]),
-                    spans=tensor(s.inputs["spans"]), W=tensor(g.inputs["A"]), q=tensor(g.outputs["C"]).reshape(-1),
+                    spans=tensor(s.inputs["spans"]), W=tensor(g.inputs["A" if one else "B"]), q=tensor(g.outputs["C"]).reshape(-1),
                     latents=tensor(s.inputs["latents"]))
         args |= {n: tensor(s.inputs[n]) for n in ("shared_keys", "angles") if n in s.inputs}
         kw = {n: getattr(o, n) for n in ("stride", "q_rank", "rank", "rot", "turned", "angle_rows", "ring")}
-        kw |= dict(M=g.op.M, eps=float(o.epsilon))
+        kw["eps"] = float(o.epsilon)
+        if few:
+            kw |= dict(slots=o.slots, rows=o.rows, N=g.op.N)
+            return Fused("latent_strips", j, 2, lambda a=args, kw=kw: kernels.latent_strips(**a, **kw))
+        kw["M"] = g.op.M
         return Fused("latent_query", j, 2, lambda a=args, kw=kw: kernels.latent_query(**a, **kw))
 
     def same_data(a, b) -> bool:

@@ -4,9 +4,10 @@
 // MFMA's registers and stands where the first's operands do not fit.  With GATED a second matrix is streamed beside the first and
 // the output is act(A B^T) * (A B2^T), rounded where the separate steps round.
 //
-// Around a float32 stream A may be its normed rows (iron_norm_strips_bf16), and C may join it through a gate (iron_gated_strips_bf16).
+// Around a float32 stream A may be its normed rows (iron_norm_strips_bf16), and C may join it through a gate (iron_gated_strips_bf16); or A is
+// the query latents of rows whose other latents go into caches (iron_latent_strips_bf16).
 #include "../../include/iron_hip.h"
-#include "rows.h"
+#include "latent.h"
 
 #include <type_traits>
 
@@ -69,12 +70,25 @@ struct StripsGru {
   bf16_t* y;
   int slots;
 };
+// A's rows are the query latents at the head of rows [query latent | latent | shared key part | ..] (mha_latent.hip), over their root mean squares as
+// in NORMED; the rest of row i goes into the caches by block i, a 16-byte piece a thread.
+// The launch of a block a row that this was takes 2.7 us between two others; here the norm costs 1.2 and the rest 0.3, because all of a block's waves
+// share it (by one wave 0.9: cold code for several pieces, which the norm's barrier waits for).  Behind another product, weights out of memory: 2048
+// columns over 1536, latents of 512, 2 rows 5.7 -> 4.6 us, 8 rows 6.4 -> 4.9; 3072 columns, 512 + 64, 8 rows 7.4 -> 5.75.
+struct StripsLatent {
+  LatentRow row;
+  LatentShape a;
+  const int* spans;
+  bf16_t *latents, *shared_keys;
+  int stride;
+};
 struct Joined {   // ... what four columns of it need
   float4 held;
   uint2 gate, gate_bias, y_bias;
 };
 
-// A lane's eight columns of rows 2 i + lane / 32 of the stream, normed.  `sums`: LDS, 64 floats.
+// A lane's eight columns of rows 2 i + lane / 32 of the stream, normed.  `sums`: LDS, 64 floats.  LATENT: rounded as latent_row does.
+template <bool LATENT>
 __device__ __forceinline__ void norm_strips(const StripsNorm& norm, int K, int lane, int wave, unsigned sums, const float4 (&f)[4][2], const uint4& gain,
                                             uint4 (&out)[4]) {
   float ss[4];
@@ -113,17 +127,68 @@ __device__ __forceinline__ void norm_strips(const StripsNorm& norm, int K, int l
     const float4 a = f[i][0], b = f[i][1];
     float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = x[j] * inv * (norm.unit + g[j]);
+    for (int j = 0; j < 8; ++j) x[j] = LATENT ? x[j] * (inv * g[j]) : x[j] * inv * (norm.unit + g[j]);
     out[i] = pack8(x);
   }
 }
 
-template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM, bool NORMED = false, bool JOINS = false, bool GRU = false>
+// A lane's 16-byte piece of a row's latent and shared key part.
+struct LatentPiece {
+  uint4 x, gain;
+  Span span;   // lane s: slot s's
+  float f[8];
+  __device__ __forceinline__ void ask(const StripsLatent& o, const bf16_t* __restrict__ rows, int row, int M, int piece) {
+    const int cn = o.a.rank >> 3, e = min(piece, cn + (o.a.rot >> 3) - 1);   // (the last again past the end)
+    x = reinterpret_cast<const uint4*>(rows + (size_t)row * o.stride + o.row.q_rank)[e];
+    gain = reinterpret_cast<const uint4*>(o.row.c_gain)[min(e, cn - 1)];
+    span = span_of(o.spans, min((int)threadIdx.x & 63, o.a.slots - 1), M);
+  }
+  // The wave's part of the latent's sum of squares.
+  __device__ __forceinline__ float squares(const StripsLatent& o, int piece) {
+    unpack8(x, f);
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sum = fmaf(f[j], f[j], sum);
+    return wave_sum(piece < o.a.rank >> 3 ? sum : 0.f);
+  }
+  __device__ __forceinline__ void store(const StripsLatent& o, int row, int piece, float squares) {
+    const int cn = o.a.rank >> 3, n = cn + (o.a.rot >> 3), c = (piece - cn) * 8;
+    const unsigned long long holds = __builtin_amdgcn_ballot_w64(((int)threadIdx.x & 63) < o.a.slots && row >= span.row0 && row < span.row0 + span.rows);
+    if (holds == 0) return;
+    const int slot = __builtin_ctzll(holds), pos = __builtin_amdgcn_readlane(span.start, slot) + row - __builtin_amdgcn_readlane(span.row0, slot);
+    const size_t at = (size_t)slot * o.a.ring + pos % o.a.ring;
+    if (piece < cn) {
+      const float inv = 1.0f / sqrtf(squares / (float)o.a.rank + o.row.eps);
+      float g[8];
+      unpack8(gain, g);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] *= inv * g[j];
+      *reinterpret_cast<uint4*>(o.latents + at * o.a.rank + piece * 8) = pack8(f);
+    } else if (piece < n) {
+      if (c < o.a.turned) {
+        const float4* turn = reinterpret_cast<const float4*>(o.row.angles + (size_t)min(pos, o.a.angle_rows - 1) * o.a.turned + c);
+        const float4 a = turn[0], b = turn[1];
+        const float by[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+          const float u = f[j], v = f[j + 1];
+          f[j] = u * by[j] - v * by[j + 1];
+          f[j + 1] = v * by[j] + u * by[j + 1];
+        }
+      }
+      *reinterpret_cast<uint4*>(o.shared_keys + at * o.a.rot + c) = pack8(f);
+    }
+  }
+};
+
+template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM, bool NORMED = false, bool JOINS = false, bool GRU = false, bool LATENT = false>
 __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
-                                                                       bf16_t* __restrict__ C, int M, int N, int K, StripsNorm norm, StripsOut out, StripsGru gru) {
+                                                                       bf16_t* __restrict__ C, int M, int N, int K, StripsNorm norm, StripsOut out, StripsGru gru,
+                                                                       StripsLatent latent) {
   typedef Strips<MT, MA, SINGLE, STAGES> S;
   static_assert(!GRU || (MT == 1 && MA == 8 && !JOINS), "one lane a row and four columns");
   static_assert(!NORMED || (SINGLE && MT == 1 && MA == 8), "a wave norms its own strip of eight rows");
+  static_assert(!LATENT || (NORMED && !JOINS && !GRU), "the query latents are normed rows");
   constexpr int W = STRIP_WAVES, R = STRIP_ROWS, GROUP = STRIP_OUT / R;   // GROUP: tiles whose columns are stored together
   static_assert(STAGES <= 2, "the last item's wait is for all that is out");
   constexpr int NOWHERE = 0x7ffffff0;   // an offset past the end of every run of rows (64 rows of at most 2^22, the entry point's bound, are 2^29 bytes)
@@ -134,11 +199,13 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
   // (64 bits: 256 times the tiles of an N of 2^27 pass 32)
   const unsigned tiles = ((unsigned)N + R - 1) / R;
   auto first_tile = [&](unsigned block) { return (int)(tiles < STRIP_BLOCKS ? block : (unsigned long long)block * tiles / STRIP_BLOCKS); };
-  const int tile0 = GRU ? 0 : first_tile(blockIdx.x), my_tiles = GRU ? 4 : first_tile(blockIdx.x + 1) - tile0, items = my_tiles * mine;
+  const bool idle = LATENT && blockIdx.x >= tiles;   // (a block for its row's latent alone; the tile that it fetches all the same is the first)
+  const int tile0 = GRU || idle ? 0 : first_tile(blockIdx.x), my_tiles = GRU ? 4 : (idle ? 0 : first_tile(blockIdx.x + 1) - tile0), items = my_tiles * mine;
   auto column_of = [&](int t) { return GRU ? t * (N >> 2) + (int)blockIdx.x * R : (tile0 + t) * R; };   // tile t's first
   char* const own = lds + wave * S::WAVE;
   char* const held = own + (SINGLE ? S::A_BYTES : 0);
   const unsigned lds0 = (unsigned)(uintptr_t)IRON_LDS_PTR(lds), part0 = lds0 + W * S::WAVE, out0 = part0 + 2 * S::PART;
+  const unsigned rest_sums = part0 + S::PART + 64 * 4;   // behind the norm's
 
   // `count` loads of two rows each, `past` the caches or not: a lane's place in LDS is fixed, so the row's pieces are chosen by it.  Past the
   // rows or K: zeros.
@@ -209,6 +276,13 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
     x_bias = *reinterpret_cast<const uint2*>(gru.x_bias + col);
     mine_span = span_of(gru.spans, min(lane, gru.slots - 1), M);
   }
+  // ... and a row's latent (the first blocks' waves, as many as its pieces fill).
+  const int piece = (int)threadIdx.x;
+  const bool rest_here = LATENT && (int)blockIdx.x < M && wave * 64 < (latent.a.rank + latent.a.rot) >> 3;
+  LatentPiece rest;
+  if constexpr (LATENT) {
+    if (rest_here) rest.ask(latent, A, blockIdx.x, M, piece);
+  }
   Joined first_joined{};
   if (JOINS && wave == 0) first_joined = join_loads(0);
   if (!NORMED && SINGLE && items > 0) {
@@ -222,16 +296,19 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
   } else {
     // Rows as they are fetched: row 2 i + lane / 32, eight columns a lane (past the rows or K: zeros).
     const int col = wave * STRIP + ((lane & 31) << 3), hi = lane >> 5;
-    const __amdgpu_buffer_rsrc_t rows = bounded_bytes(A, M * K * 4);
+    const __amdgpu_buffer_rsrc_t rows = bounded_bytes(A, LATENT ? M * latent.stride * 2 : M * K * 4);
     float4 f[4][2];
-    uint4 made[4];
+    uint4 made[4], halves[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 4; ++i) {
+      const int r = 2 * i + hi;
+      if (LATENT) {
+        halves[i] = load_bounded(rows, col < K && r < M ? (r * latent.stride + col) * 2 : NOWHERE);
+      } else {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int r = 2 * i + hi;
-        f[i][h] = __builtin_bit_cast(float4, load_bounded(rows, col < K && r < M ? (r * K + col) * 4 + 16 * h : NOWHERE));
+        for (int h = 0; h < 2; ++h) f[i][h] = __builtin_bit_cast(float4, load_bounded(rows, col < K && r < M ? (r * K + col) * 4 + 16 * h : NOWHERE));
       }
+    }
     const uint4 gain = load_bounded(bounded_bytes(norm.gain, K * 2), col * 2);
     __builtin_amdgcn_sched_barrier(0);
     // (of a wave without a strip too, for whom it is nothing: behind a branch the compiler, which then counts none of its loads, would wait for B
@@ -239,7 +316,22 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
 #pragma unroll
     for (int i = 0; i < STAGES - 1; ++i) fetch(i);
     __builtin_amdgcn_sched_barrier(0);
-    norm_strips(norm, K, lane, wave, part0 + S::PART, f, gain, made);
+    if (LATENT) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float x[8];
+        unpack8(halves[i], x);
+        f[i][0] = make_float4(x[0], x[1], x[2], x[3]);
+        f[i][1] = make_float4(x[4], x[5], x[6], x[7]);
+      }
+    }
+    if constexpr (LATENT) {   // (the norm's barrier is this sum's too)
+      if (rest_here) {
+        const float sum = rest.squares(latent, piece);
+        if (lane == 0) asm volatile("ds_write_b32 %0, %1" ::"v"(rest_sums + wave * 4), "v"(sum) : "memory");
+      }
+    }
+    norm_strips<LATENT>(norm, K, lane, wave, part0 + S::PART, f, gain, made);
     // (the strip is the wave's alone: no barrier)
     const unsigned mine_at = lds0 + (unsigned)(own - lds);
 #pragma unroll
@@ -258,6 +350,22 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
     a_from_lds(lds0 + (unsigned)(own - lds));
 #pragma unroll
     for (int k = 0; k < 8; ++k) lds_wait_for<0>(af[0][k]);
+  }
+  if constexpr (LATENT) {
+    if (rest_here) {
+      bf16x8 part[2];
+      part[0] = lds_read_b128_at<0>(rest_sums);
+      part[1] = lds_read_b128_at<16>(rest_sums);
+      float total = 0.f;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        lds_wait_for<0>(part[h]);
+        const f32x4 p = __builtin_bit_cast(f32x4, part[h]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) total += (4 * h + q) * 64 < latent.a.rank >> 3 ? p[q] : 0.f;   // (waves that have none left nothing)
+      }
+      rest.store(latent, blockIdx.x, piece, total);
+    }
   }
   if (GRU && wave == 0) {   // (the spans' trip passed under the norm, this one passes under the products)
 #pragma unroll
@@ -518,20 +626,23 @@ static int launch_gemm_few(const bf16_t* A, const bf16_t* B, const bf16_t* B2, b
   IRON_LAUNCH_CHECK();
 }
 
-template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM, bool NORMED = false, bool JOINS = false, bool GRU = false>
+template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM, bool NORMED = false, bool JOINS = false, bool GRU = false,
+          bool LATENT = false>
 static int launch_gemm_strips(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s, const StripsNorm& norm = {},
-                              const StripsOut& out = {}, const StripsGru& gru = {}) {
+                              const StripsOut& out = {}, const StripsGru& gru = {}, const StripsLatent& latent = {}) {
   typedef Strips<MT, MA, SINGLE, STAGES> S;
   static_assert(S::LDS <= 163840, "a CU's LDS");
   static LdsOptIn opt;
-  auto kernel = &gemm_strips_kernel<MT, MA, SINGLE, STAGES, STREAM, NORMED, JOINS, GRU>;
+  auto kernel = &gemm_strips_kernel<MT, MA, SINGLE, STAGES, STREAM, NORMED, JOINS, GRU, LATENT>;
   const hipError_t e = opt.ensure(reinterpret_cast<const void*>(kernel), S::LDS);
   if (e != hipSuccess) {
     set_error("gemm_few: %s", hipGetErrorString(e));
     return (int)e;
   }
   const unsigned tiles = ((unsigned)N + STRIP_ROWS - 1) / STRIP_ROWS;
-  hipLaunchKernelGGL(kernel, dim3(GRU ? tiles / 4 : (tiles < STRIP_BLOCKS ? tiles : STRIP_BLOCKS)), dim3(STRIP_WAVES * 64), S::LDS, s, A, B, C, M, N, K, norm, out, gru);
+  unsigned blocks = GRU ? tiles / 4 : (tiles < STRIP_BLOCKS ? tiles : STRIP_BLOCKS);
+  if (LATENT && blocks < (unsigned)M) blocks = M;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(STRIP_WAVES * 64), S::LDS, s, A, B, C, M, N, K, norm, out, gru, latent);
   IRON_LAUNCH_CHECK();
 }
 
@@ -626,6 +737,27 @@ extern "C" int iron_norm_gru_strips_bf16(const float* x, const uint16_t* gain, f
   const StripsGru gru{z_bias, x_bias, state, spans, y, slots};
   return launch_gemm_strips<1, 8, true, 2, true, true, false, true>(reinterpret_cast<const bf16_t*>(x), W, packed, rows, 4 * width, K, (hipStream_t)stream,
                                                                     StripsNorm{gain, eps, unit}, {}, gru);
+}
+
+extern "C" int iron_latent_strips_bf16(const uint16_t* x, const uint16_t* q_gain, const uint16_t* c_gain, const float* angles, const int* spans,
+                                       const uint16_t* W, uint16_t* q, uint16_t* latents, uint16_t* shared_keys, int slots, int rows, int N, int stride,
+                                       int q_rank, int rank, int rot, int turned, int angle_rows, int ring, float eps, void* stream) {
+  IRON_REQUIRE(x && q_gain && c_gain && spans && W && q && latents && (rot == 0 || shared_keys), "latent_strips: null operand");
+  IRON_REQUIRE(rows > 0 && rows <= 8 && slots > 0 && slots <= 64 && N > 0, "latent_strips: rows (%d) from 1 to 8, slots (%d) from 1 to 64, N (%d) positive",
+               rows, slots, N);
+  IRON_REQUIRE(q_rank >= 8 && q_rank % 8 == 0 && q_rank <= STRIP * STRIP_WAVES, "latent_strips: the query latent (%d) is a positive multiple of 8 up to %d",
+               q_rank, STRIP * STRIP_WAVES);
+  IRON_REQUIRE(rank > 0 && rot >= 0 && ring > 0 && (rank | rot | stride) % 8 == 0 && rank <= 4096 && rot <= 4096 - rank,
+               "latent_strips: latents of %d + %d columns, whole 16-byte pieces and 4096 together at the most, a ring (%d) of at least 1", rank, rot, ring);
+  IRON_REQUIRE(stride >= q_rank + rank + rot && stride <= (1 << 22), "latent_strips: a row of %d holds no latents of %d and %d + %d", stride, q_rank, rank, rot);
+  IRON_REQUIRE(turned >= 0 && turned <= rot && turned % 8 == 0 && (turned == 0 || (angles && angle_rows > 0)),
+               "latent_strips: %d of %d shared columns turn, whole 16-byte pieces, by a table of %d rows", turned, rot, angle_rows);
+  IRON_REQUIRE((((uintptr_t)x | (uintptr_t)q_gain | (uintptr_t)c_gain | (uintptr_t)angles | (uintptr_t)spans | (uintptr_t)W | (uintptr_t)latents |
+                 (uintptr_t)shared_keys) & 15) == 0, "latent_strips: operands must be 16-byte aligned");
+  const StripsLatent latent{LatentRow{q_gain, c_gain, angles, q_rank, eps}, LatentShape{slots, rows, 1, 1, rot, 1, rank, turned, angle_rows, 1, ring, 0, 1.f},
+                            spans, latents, shared_keys, stride};
+  return launch_gemm_strips<1, 8, true, 2, true, true, false, false, true>(x, W, q, rows, N, q_rank, (hipStream_t)stream, StripsNorm{q_gain, eps, 0.f}, {}, {},
+                                                                           latent);
 }
 
 extern "C" int iron_gated_strips_bf16(const uint16_t* x, const uint16_t* W, const uint16_t* y_bias, const uint16_t* gate, int gate_stride,

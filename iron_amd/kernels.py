@@ -1238,6 +1238,22 @@ def latent_query(x, q_gain, c_gain, spans, W, q, latents, *, M, stride, q_rank, 
                                        current_stream()), "iron_latent_query_bf16")
 
 
+def latent_strips(x, q_gain, c_gain, spans, W, q, latents, *, slots, rows, N, stride, q_rank, rank, ring, eps, rot=0, turned=0, angle_rows=0,
+                  angles=None, shared_keys=None):
+    """Up to eight rows: their latents normed, stored and turned, and the queries' product, one launch."""
+    _bf16(x, rows * stride, "x")
+    _bf16(q_gain, q_rank, "q_gain")
+    _bf16(c_gain, rank, "c_gain")
+    _bf16(W, N * q_rank, "W")
+    _bf16(q, rows * N, "q")
+    _bf16(latents, slots * ring * rank, "latents")
+    if rot:
+        _bf16(shared_keys, slots * ring * rot, "shared_keys")
+    check(lib().iron_latent_strips_bf16(ptr(x), ptr(q_gain), ptr(c_gain), _turned(angles, angle_rows, turned), _spans(spans, slots), ptr(W), ptr(q),
+                                        ptr(latents), ptr(shared_keys), slots, rows, N, stride, q_rank, rank, rot, turned, angle_rows, ring,
+                                        float(eps), current_stream()), "iron_latent_strips_bf16")
+
+
 def decode_mixed(h, carry, spans, products, *, k):
     """A token shift and the projections of its blends, one row, one launch.  ``products``: (weight, output,
     mu row or None) each."""

@@ -367,6 +367,40 @@ def test_a_recurrence_s_step_in_its_projection_s_launch(cuda, rows, width, K_):
     assert np.abs(from_torch(y) - from_torch(out)).max() <= 2**-8 * np.abs(from_torch(out)).max()
 
 
+# One row and eight, fewer blocks than rows, latents of a piece and of as many as a wave holds, a waves' strip that ends in a piece, parts that turn whole, half and not.
+@pytest.mark.parametrize("rows,N,q_rank,rank,rot,turn", [(8, 3072, 1536, 512, 64, 64), (2, 2048, 1536, 512, 0, 0), (8, 24, 264, 8, 0, 0), (5, 8, 8, 40, 64, 32),
+                                                         (3, 4103, 2048, 4056, 40, 40), (1, 64, 2040, 520, 1528, 8)])
+def test_rows_latents_in_their_queries_launch(cuda, rows, N, q_rank, rank, rot, turn):
+    rng = np.random.default_rng(N)
+    slots, ring, stride = rows + 2, 64, q_rank + rank + rot + 24
+    W, x = bf(rng, N, q_rank, scale=1 / np.sqrt(q_rank)), bf(rng, rows, stride, scale=3)
+    x[0] *= 16   # (a row's own root mean square)
+    # the rows' slots in another order, some idle, at positions that wrap around the ring; the last row is nobody's where there are several
+    spans, order = table(slots=slots), rng.permutation(slots)[: max(1, rows - 1)]
+    for r, slot in enumerate(order):
+        spans[slot] = (r, 1, (0, 70, 63, 9)[r % 4], 0)
+    spans, x, W = device(spans, np.int32), device(x, BF16), device(W, BF16)
+    q_gain, c_gain = device(bf(rng, q_rank), BF16), device(bf(rng, rank), BF16)
+    sizes = dict(slots=slots, rows=rows, stride=stride, q_rank=q_rank, rank=rank, rot=rot, turned=turn, angle_rows=128 if turn else 0, ring=ring, eps=1e-3)
+    angles = device(rope_angles(turn, 128, 400.0), F32) if turn else None
+    kept = {}
+    for launch in ("apart", "one"):
+        latents, keys = (torch.full((slots, ring, n), 7.0, dtype=torch.bfloat16, device="cuda") for n in (rank, max(rot, 8)))
+        q, h = (torch.full((rows, n), 7.0, dtype=torch.bfloat16, device="cuda") for n in (N, q_rank))
+        parts = dict(angles=angles, shared_keys=keys[..., :rot].contiguous() if rot else None)
+        if launch == "one":
+            K.latent_strips(x, q_gain, c_gain, spans, W, q, latents, N=N, **sizes, **parts)
+        else:
+            K.latent_rows(x, q_gain, c_gain, spans, h, latents, **sizes, **parts)
+            live = len(order)
+            want = from_torch(h)[:live].astype(np.float64) @ from_torch(W).astype(np.float64).T
+        kept[launch] = (from_torch(latents), from_torch(parts["shared_keys"]) if rot else None)
+    got = from_torch(q)[:live]
+    assert (np.abs(got - want).max(1) <= 6e-3 * np.abs(want).max(1)).all()
+    for a, b in zip(kept["apart"], kept["one"]):   # (the sums of squares in another order: a value may round the other way)
+        assert a is None or (np.abs(a - b) <= 2**-7 * np.abs(a)).all() and (a != b).mean() < 1e-2
+
+
 def test_a_batch_s_steps_in_few_launches(cuda):
     """Steps of two to eight slots: the stream's norms and sums in the products' launches, with what the steps alone give."""
     for name, slots in (("mixed", 2), ("mixed", 8), ("wide", 3), ("wide", 8)):   # (recurrences of other widths than the stream's, and of its width)
@@ -375,7 +409,7 @@ def test_a_batch_s_steps_in_few_launches(cuda):
             model, _ = built(name, Pufuzen, slots=slots, max_seq_len=200, prefill_chunk=32)
             model.load_versions(fuse=fuse)
             kinds = {f.kind for f in model.decode_step._fused.values()}
-            assert not fuse or {"norm_strips", "gated_strips", *(("norm_gru_strips",) if name == "wide" else ())} <= kinds
+            assert not fuse or {"norm_strips", "gated_strips", "latent_strips", *(("norm_gru_strips",) if name == "wide" else ())} <= kinds
             prompts = [tokens_of(model, 5 + 3 * i, seed=i) for i in range(slots)]
             model.batch.step([Entry(i, p) for i, p in enumerate(prompts)])
             steps = []
