@@ -21,24 +21,38 @@ namespace iron {
 // What bounds it is the way to the memory, so the shape follows that: eight rows a tile and not the MFMA's sixteen (half of each product is
 // dropped; the matrix cores idle anyway), because 2048 rows of B then occupy all 256 CUs; up to sixteen rows of A as contiguous runs, because
 // rows a power of two apart, read a fragment at a time by every block, meet on one L2 channel.  Eight rows of A over cold weights, us with
-// gemm_few_kernel and with this: 2048 x 2048 5.1 / 4.1, 2048 x 8192 14.1 / 9.3, 4160 x 2048 8.0 / 6.0, 8192 x 2048 10.2 / 8.8,
-// 10240 x 2048 15.0 / 10.3, 128256 x 2048 106 / 86 (6.1 TB/s); thirty-two rows: 4160 x 2048 14.3 / 9.6, 128256 x 2048 163 / 92.
+// gemm_few_kernel and with this: 2048 x 2048 5.1 / 4.0, 2048 x 8192 14.1 / 9.2, 4160 x 2048 8.0 / 5.5, 8192 x 2048 10.2 / 7.7,
+// 10240 x 2048 15.0 / 9.1, 128256 x 2048 106 / 79 (6.6 TB/s); thirty-two rows: 4160 x 2048 14.3 / 9.5, 128256 x 2048 163 / 90.
 constexpr int STRIP = 256, STRIP_BYTES = 512, STRIP_WAVES = 8, STRIP_ROWS = 8;
 constexpr unsigned STRIP_BLOCKS = 256;   // one a CU; fewer tiles: a block each
-constexpr int STRIP_OUT = 64;   // columns of C staged for a store of whole lines: 128256 x 2048 98 -> 86 us with the loads past the caches
+// The blocks take rounds of 256 neighbouring tiles, so that all of them together read one run of B at a time; the blocks of a chiplet (every eighth) have
+// eight neighbours, whose columns make a line of C in its L2.  Where a block's own tiles were neighbours the blocks read 256 places that are the same
+// power of two apart, and a stream alone took 6.6 us for 33 MB and 12.1 for 67 that takes 6.4 and 11.4 so (weights out of memory, us: 8 rows of 3072 x 1536 4.75 -> 4.1,
+// 4160 x 2048 5.95 -> 5.5, 8192 x 2048 8.0 -> 7.7, 50257 x 768 19.4 -> 15.9, 128256 x 2048 81.5 -> 79; 16 rows of 32000 x 1024 14.6 -> 12.5).  More than sixteen rows keep
+// neighbours, and STRIP_OUT columns of C leave as whole lines: a C that its chiplets do not hold until its lines are whole costs more than that (32 rows of
+// 128256 x 2048 90, in rounds 104).
+constexpr int STRIP_OUT = 64;
+__device__ __forceinline__ unsigned strip_place(unsigned block) { return (block >> 6 << 6) + ((block & 7) << 3) + (block >> 3 & 7); }
 
 __device__ __forceinline__ void lds_write_b128(unsigned addr, const f32x4& v) { asm volatile("ds_write_b128 %0, %1" ::"v"(addr), "v"(v) : "memory"); }
 // A barrier behind the wave's own LDS accesses that leaves its loads from memory in flight.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // MT: tiles of sixteen rows of A; one of them has MA rows at the most and comes by LDS, more come straight into registers.
-template <int MT, int MA, bool SINGLE, int STAGES>
+// MEET: tiles whose sums meet at one barrier, instead of one a tile at which every wave waited for the slowest (with the same weights out of the last-level
+// cache, where that is most of it: 8 rows of 4096 x 2048 4.55 -> 3.95 us, 16000 x 600 7.0 -> 6.0).
+template <int MT, int MA, bool SINGLE, int STAGES, int MEET = 1>
 struct Strips {
   static constexpr bool A_BY_LDS = MT == 1;
   static constexpr int A_BYTES = A_BY_LDS ? MA * STRIP_BYTES : 0, B_BYTES = STRIP_ROWS * STRIP_BYTES;
   static constexpr int ITEM = (SINGLE ? 0 : A_BYTES) + B_BYTES, WAVE = ITEM * STAGES + (SINGLE ? A_BYTES : 0);
-  static constexpr int PART = STRIP_WAVES * MT * 1024, OUT = MT * 16 * STRIP_OUT * 2;
-  static constexpr int LDS = STRIP_WAVES * WAVE + 2 * PART + 2 * OUT;
+  static constexpr int PART = STRIP_WAVES * MT * 1024;
+  // LDS: the waves' strips (with MEET A's strips first, whose place every other meeting's sums take: A is in registers by then), one
+  // meeting's sums or two, a norm's, columns of C.
+  static constexpr bool OVER_A = MEET > 1;
+  static constexpr int SUMS = STRIP_WAVES * WAVE, NORM = SUMS + (OVER_A ? 1 : 2) * MEET * PART, OUT0 = NORM + 512, OUT = MT * 16 * STRIP_OUT * 2;
+  static constexpr int LDS = OUT0 + (MT > 1 ? 2 * OUT : 0);
+  static_assert(!OVER_A || (SINGLE && MT == 1 && MEET * PART <= STRIP_WAVES * A_BYTES), "the sums fit where A's strips were");
   static constexpr int A_INST = A_BYTES / 1024, B_INST = B_BYTES / 1024, INST = ITEM / 1024;
 };
 
@@ -181,31 +195,42 @@ struct LatentPiece {
   }
 };
 
-template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM, bool NORMED = false, bool JOINS = false, bool GRU = false, bool LATENT = false>
+template <int MT, int MA, bool SINGLE, bool JOINS, bool GRU>   // (what LDS has room for)
+__host__ __device__ constexpr int strips_meet() { return MT > 1 || !SINGLE || JOINS || GRU ? 1 : (MA == 8 ? 4 : 2); }
+
+template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM, bool NORMED = false, bool JOINS = false, bool GRU = false, bool LATENT = false,
+          bool MANY = false>
 __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
                                                                        bf16_t* __restrict__ C, int M, int N, int K, StripsNorm norm, StripsOut out, StripsGru gru,
                                                                        StripsLatent latent) {
-  typedef Strips<MT, MA, SINGLE, STAGES> S;
+  constexpr int MEET = strips_meet<MT, MA, SINGLE, JOINS, GRU>();
+  typedef Strips<MT, MA, SINGLE, STAGES, MEET> S;
   static_assert(!GRU || (MT == 1 && MA == 8 && !JOINS), "one lane a row and four columns");
   static_assert(!NORMED || (SINGLE && MT == 1 && MA == 8), "a wave norms its own strip of eight rows");
+  static_assert(!MANY || (SINGLE && STAGES == 2 && MT == 1 && !JOINS && !GRU && !LATENT), "a block's tiles follow each other strip by strip");
   static_assert(!LATENT || (NORMED && !JOINS && !GRU), "the query latents are normed rows");
-  constexpr int W = STRIP_WAVES, R = STRIP_ROWS, GROUP = STRIP_OUT / R;   // GROUP: tiles whose columns are stored together
+  constexpr int W = STRIP_WAVES, R = STRIP_ROWS;
+  constexpr bool LINED = MT > 1 && !JOINS && !GRU;   // a block's tiles are neighbours, and the columns of GROUP of them are stored together
+  constexpr int GROUP = STRIP_OUT / R;
   static_assert(STAGES <= 2, "the last item's wait is for all that is out");
   constexpr int NOWHERE = 0x7ffffff0;   // an offset past the end of every run of rows (64 rows of at most 2^22, the entry point's bound, are 2^29 bytes)
   extern __shared__ __align__(1024) char lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l16 = lane & 15, quad = lane >> 4;
   const int strips = (K + STRIP - 1) / STRIP, mine = SINGLE ? wave < strips : (strips - wave + W - 1) / W, most = SINGLE ? 1 : (strips + W - 1) / W;
-  // A block's tiles are neighbours, so that its columns of C leave as whole lines.
-  // (64 bits: 256 times the tiles of an N of 2^27 pass 32)
   const unsigned tiles = ((unsigned)N + R - 1) / R;
-  auto first_tile = [&](unsigned block) { return (int)(tiles < STRIP_BLOCKS ? block : (unsigned long long)block * tiles / STRIP_BLOCKS); };
+  // (64 bits: 256 times the tiles of an N of 2^27 pass 32)
+  auto neighbours = [&](unsigned block) { return (unsigned)((unsigned long long)block * tiles / STRIP_BLOCKS); };
+  const unsigned first = GRU || tiles <= STRIP_BLOCKS ? blockIdx.x : (LINED ? neighbours(blockIdx.x) : strip_place(blockIdx.x));
+  const unsigned end = LINED && tiles > STRIP_BLOCKS ? neighbours(blockIdx.x + 1) : tiles;
+  constexpr int STEP = LINED ? 1 : (int)STRIP_BLOCKS;
   const bool idle = LATENT && blockIdx.x >= tiles;   // (a block for its row's latent alone; the tile that it fetches all the same is the first)
-  const int tile0 = GRU || idle ? 0 : first_tile(blockIdx.x), my_tiles = GRU ? 4 : (idle ? 0 : first_tile(blockIdx.x + 1) - tile0), items = my_tiles * mine;
-  auto column_of = [&](int t) { return GRU ? t * (N >> 2) + (int)blockIdx.x * R : (tile0 + t) * R; };   // tile t's first
-  char* const own = lds + wave * S::WAVE;
-  char* const held = own + (SINGLE ? S::A_BYTES : 0);
-  const unsigned lds0 = (unsigned)(uintptr_t)IRON_LDS_PTR(lds), part0 = lds0 + W * S::WAVE, out0 = part0 + 2 * S::PART;
-  const unsigned rest_sums = part0 + S::PART + 64 * 4;   // behind the norm's
+  const int tile0 = GRU || idle ? 0 : (int)first;
+  const int my_tiles = GRU ? 4 : (idle ? 0 : (tiles <= STRIP_BLOCKS ? 1 : (int)((end - first + STEP - 1) / STEP))), items = my_tiles * mine;
+  auto column_of = [&](int t) { return GRU ? t * (N >> 2) + (int)blockIdx.x * R : (tile0 + t * STEP) * R; };   // tile t's first
+  char* const own = lds + wave * (S::OVER_A ? S::A_BYTES : S::WAVE);   // (with SINGLE A's strip)
+  char* const held = S::OVER_A ? lds + W * S::A_BYTES + wave * (STAGES * S::ITEM) : own + (SINGLE ? S::A_BYTES : 0);
+  const unsigned lds0 = (unsigned)(uintptr_t)IRON_LDS_PTR(lds), part0 = lds0 + S::SUMS;
+  const unsigned norm_sums = lds0 + S::NORM, rest_sums = norm_sums + 64 * 4;
 
   // `count` loads of two rows each, `past` the caches or not: a lane's place in LDS is fixed, so the row's pieces are chosen by it.  Past the
   // rows or K: zeros.
@@ -222,8 +247,8 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
   };
   auto fetch = [&](int item) {
     char* to = held + item % STAGES * S::ITEM;
-    const int t = SINGLE ? item : item / max(mine, 1), strip = wave + W * (SINGLE ? 0 : item - t * mine), row0 = column_of(t);
-    const int rows = min(R, N - row0);
+    const int t = SINGLE ? item : item / max(mine, 1), strip = wave + W * (SINGLE ? 0 : item - t * mine);
+    const int row0 = column_of(t), rows = min(R, N - row0);
     if (!SINGLE && S::A_BY_LDS) {
       fetch_rows(A, M, strip, to, std::integral_constant<int, S::A_INST>(), std::false_type());
       to += S::A_BYTES;
@@ -331,7 +356,7 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
         if (lane == 0) asm volatile("ds_write_b32 %0, %1" ::"v"(rest_sums + wave * 4), "v"(sum) : "memory");
       }
     }
-    norm_strips<LATENT>(norm, K, lane, wave, part0 + S::PART, f, gain, made);
+    norm_strips<LATENT>(norm, K, lane, wave, norm_sums, f, gain, made);
     // (the strip is the wave's alone: no barrier)
     const unsigned mine_at = lds0 + (unsigned)(own - lds);
 #pragma unroll
@@ -377,14 +402,13 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
     }
     if (lane < 32 && start > 0) old_state = *reinterpret_cast<const float4*>(gru.state + state_at + ((start - 1) & 1) * (N >> 2));
   }
-  const bool staged = !JOINS && !GRU && my_tiles > 1;   // (a lone tile's columns leave as they are: by way of LDS and another barrier 8 rows of 2048 x 2048 took 4.44 us instead of 4.24)
-  // The columns of `count` tiles from `first` on, from half `half` of the out stage, by one wave.
-  auto flush = [&](int first, int count, int half) {
+  const bool staged = LINED && my_tiles > 1;
+  // The columns of `count` tiles from `from` on, from half `half` of the out stage, by one wave.
+  auto flush = [&](int from, int count, int half) {
     for (int e = lane; e < M * count; e += 64) {
-      const int r = e / count, p = e - r * count, n = (tile0 + first + p) * R;
-      bf16x8 v = lds_read_b128_at<0>(out0 + half * S::OUT + (r * STRIP_OUT + p * R) * 2);
+      const int r = e / count, p = e - r * count, n = (tile0 + from + p) * R;
+      bf16x8 v = lds_read_b128_at<0>(lds0 + S::OUT0 + half * S::OUT + (r * STRIP_OUT + p * R) * 2);
       lds_wait_for<0>(v);
-      // (wherever C's rows begin: an element at a time 8 rows of 16001 x 2048 took 15.1 us instead of 12.8)
       if (n < N) store_ragged(C + (size_t)r * N + n, __builtin_bit_cast(uint4, v), N - n);
     }
   };
@@ -397,7 +421,7 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
       if (s >= mine) continue;   // (the other waves' last strips)
       if (!SINGLE && !S::A_BY_LDS) a_from_memory(wave + W * s);
       if (STAGES == 1 || item + STAGES - 1 < items) {
-        fetch(item + STAGES - 1);
+        if (!MANY || item == 0) fetch(item + STAGES - 1);
         __builtin_amdgcn_sched_barrier(0);
         wait_vmcnt<(STAGES - 1) * S::INST>();
       } else {
@@ -414,6 +438,12 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
         if (!SINGLE && S::A_BY_LDS) lds_wait_for<0>(af[0][k]);
         lds_wait_for<0>(bf[k]);
       }
+      if (MANY && item + STAGES < items) {
+        asm volatile("" ::: "memory");   // (behind the reads)
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(item + STAGES);
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
       for (int k = 0; k < 8; ++k)
 #pragma unroll
@@ -421,19 +451,24 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
       ++item;
     }
     // The waves' sums meet, through assembly: the compiler would wait for every strip in flight before each access to LDS.
-    const unsigned pa = part0 + (t & 1) * S::PART;
+    const int meeting = t / MEET;
+    const unsigned sums0 = S::OVER_A ? (meeting & 1 ? lds0 : part0) : part0 + (meeting & 1) * S::PART;
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       f32x4 v = acc[m];
       asm volatile("s_nop 15\n\ts_nop 3" : "+v"(v));   // (the matrix cores' results, which assembly is not waited for with)
-      lds_write_b128(pa + ((wave * MT + m) * 64 + lane) * 16, v);
+      lds_write_b128(sums0 + t % MEET * S::PART + ((wave * MT + m) * 64 + lane) * 16, v);
     }
+    if (MEET > 1 && (t + 1) % MEET != 0 && t + 1 < my_tiles) continue;
     lds_barrier();
-    if (!JOINS && !GRU && t > 0 && t % GROUP == 0 && wave == (t + W / 2) % W) flush(t - GROUP, GROUP, (t / GROUP - 1) & 1);
-    // Tile t's sums by wave t % 8: lane (quad, l16) of the first two quads has columns 4 quad .. + 3 of row l16.
+    const int met = meeting * MEET;   // the first tile of this meeting; tile met + i's sums by wave (met + i) % 8
+    if (LINED && t > 0 && t % GROUP == 0 && wave == (t + W / 2) % W) flush(t - GROUP, GROUP, (t / GROUP - 1) & 1);
+    const int u = GRU ? t : met + ((wave - met) & (W - 1));
+    const unsigned pa = sums0 + (u - met) * S::PART;
+    // Lane (quad, l16) of the first two quads has columns 4 quad .. + 3 of row l16.
     const Joined joined = JOINS ? (t == 0 ? first_joined : (wave == t % W ? join_loads(t) : Joined{})) : Joined{};
-    if (wave == (GRU ? 0 : t % W) && lane < 32) {
-      const int n = column_of(t) + quad * 4;
+    if ((GRU ? wave == 0 : u <= t) && lane < 32) {
+      const int n = column_of(u) + quad * 4;
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
         bf16x8 p[W];
@@ -482,7 +517,7 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
             *reinterpret_cast<uint2*>(gru.y + (size_t)r * width + col) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
           }
         } else if (staged) {
-          const unsigned to = out0 + (t / GROUP & 1) * S::OUT + (r * STRIP_OUT + t % GROUP * R + quad * 4) * 2;
+          const unsigned to = lds0 + S::OUT0 + (u / GROUP & 1) * S::OUT + (r * STRIP_OUT + u % GROUP * R + quad * 4) * 2;
           const uint64_t four = (uint64_t)pack_bf16(v[2], v[3]) << 32 | pack_bf16(v[0], v[1]);
           asm volatile("ds_write_b64 %0, %1" ::"v"(to), "v"(four) : "memory");
         } else if (r < M && n < N) {
@@ -500,8 +535,8 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
   }
   if (staged) {
     lds_barrier();
-    const int first = (my_tiles - 1) / GROUP * GROUP;
-    if (wave == 0) flush(first, my_tiles - first, first / GROUP & 1);
+    const int from = (my_tiles - 1) / GROUP * GROUP;
+    if (wave == 0) flush(from, my_tiles - from, from / GROUP & 1);
   }
   wait_vmcnt<0>();   // (loads of nothing may still be on their way into LDS)
 }
@@ -627,13 +662,13 @@ static int launch_gemm_few(const bf16_t* A, const bf16_t* B, const bf16_t* B2, b
 }
 
 template <int MT, int MA, bool SINGLE, int STAGES, bool STREAM, bool NORMED = false, bool JOINS = false, bool GRU = false,
-          bool LATENT = false>
+          bool LATENT = false, bool MANY = false>
 static int launch_gemm_strips(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s, const StripsNorm& norm = {},
                               const StripsOut& out = {}, const StripsGru& gru = {}, const StripsLatent& latent = {}) {
-  typedef Strips<MT, MA, SINGLE, STAGES> S;
+  typedef Strips<MT, MA, SINGLE, STAGES, strips_meet<MT, MA, SINGLE, JOINS, GRU>()> S;
   static_assert(S::LDS <= 163840, "a CU's LDS");
   static LdsOptIn opt;
-  auto kernel = &gemm_strips_kernel<MT, MA, SINGLE, STAGES, STREAM, NORMED, JOINS, GRU, LATENT>;
+  auto kernel = &gemm_strips_kernel<MT, MA, SINGLE, STAGES, STREAM, NORMED, JOINS, GRU, LATENT, MANY>;
   const hipError_t e = opt.ensure(reinterpret_cast<const void*>(kernel), S::LDS);
   if (e != hipSuccess) {
     set_error("gemm_few: %s", hipGetErrorString(e));
@@ -645,6 +680,11 @@ static int launch_gemm_strips(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(STRIP_WAVES * 64), S::LDS, s, A, B, C, M, N, K, norm, out, gru, latent);
   IRON_LAUNCH_CHECK();
 }
+
+// Eight tiles a block and more: a stage is filled again as soon as it is in registers, not behind its tile's sums (8 rows, weights out of memory: 128256 x 2048
+// 79.6 -> 78.6 us, 32000 x 1024 12.8 -> 12.5; but 10240 x 2048 with the norm 9.9 -> 10.4: there is little to overlap, and the memory takes longer with
+// more out).
+static bool strips_many(int N) { return N >= 8 * (int)STRIP_BLOCKS * STRIP_ROWS; }
 
 // Which products go by strips, by what both kernels took over three hundred shapes with weights out of memory (us, gemm_few_kernel against strips).
 // K up to eight strips: up to 16 rows of A (8 rows: 64 x 384 3.9 / 2.6, 1024 x 1024 4.4 / 2.9, 8192 x 2048 9.0 / 8.2, 16000 x 600 8.8 / 7.4, 128256 x 2048
@@ -673,6 +713,10 @@ static int strips_for(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N,
     if (M > 16) return launch_gemm_strips<2, 16, true, 2, true>(A, B, C, M, N, K, s);
     if (!one_tile && K < 64) return -1;
     if (two_tiles && !on_lines) return -1;
+    if (strips_many(N)) {
+      if (M <= 8) return launch_gemm_strips<1, 8, true, 2, true, false, false, false, false, true>(A, B, C, M, N, K, s);
+      return launch_gemm_strips<1, 16, true, 2, true, false, false, false, false, true>(A, B, C, M, N, K, s);
+    }
     if (M <= 8) return launch_gemm_strips<1, 8, true, 2, true>(A, B, C, M, N, K, s);
     return launch_gemm_strips<1, 16, true, 2, true>(A, B, C, M, N, K, s);
   }
@@ -721,7 +765,10 @@ extern "C" int iron_norm_strips_bf16(const float* x, const uint16_t* gain, float
   IRON_REQUIRE(rows > 0 && rows <= 8 && N > 0, "norm_strips: rows (%d) from 1 to 8, N (%d) positive", rows, N);
   IRON_REQUIRE(K >= 8 && K % 8 == 0 && K <= STRIP * STRIP_WAVES, "norm_strips: K (%d) is a positive multiple of 8 up to %d", K, STRIP * STRIP_WAVES);
   IRON_REQUIRE((((uintptr_t)x | (uintptr_t)gain | (uintptr_t)W) & 15) == 0, "norm_strips: operands must be 16-byte aligned");
-  return launch_gemm_strips<1, 8, true, 2, true, true>(reinterpret_cast<const bf16_t*>(x), W, y, rows, N, K, (hipStream_t)stream, StripsNorm{gain, eps, unit});
+  const StripsNorm norm{gain, eps, unit};
+  if (strips_many(N))
+    return launch_gemm_strips<1, 8, true, 2, true, true, false, false, false, true>(reinterpret_cast<const bf16_t*>(x), W, y, rows, N, K, (hipStream_t)stream, norm);
+  return launch_gemm_strips<1, 8, true, 2, true, true>(reinterpret_cast<const bf16_t*>(x), W, y, rows, N, K, (hipStream_t)stream, norm);
 }
 
 extern "C" int iron_norm_gru_strips_bf16(const float* x, const uint16_t* gain, float eps, float unit, const uint16_t* W, const uint16_t* z_bias,
