@@ -492,27 +492,36 @@ __device__ __forceinline__ StepKeys step_keys(const Span& s, const LatentShape& 
   StepKeys k;
   k.count = min(s.start + 1, a.window);
   k.first = s.start + 1 - k.count;
-  const int tiles = (k.count + STEP_KEYS - 1) / STEP_KEYS, each = (tiles + splits - 1) / splits;
+  // (the divisions, a tenth of a microsecond each ahead of the first load, only where one is due)
+  const int tiles = (k.count + STEP_KEYS - 1) / STEP_KEYS, each = tiles <= splits ? 1 : (tiles + splits - 1) / splits;
   k.per = each * STEP_KEYS;
-  k.live = (tiles + each - 1) / each;
+  k.live = each == 1 ? tiles : (tiles + each - 1) / each;
   return k;
 }
 
-// A head's query in the latents' space, q_h U_h, and its turned columns behind it.
-template <typename T, typename OUT, int VEC>
+// A head's query in the latents' space, q_h U_h, and its turned columns behind it.  A chain of trips to memory, so the first AHEAD
+// rows of a thread's weights, which wait for nothing, are asked for behind the span and ahead of the row that it names, whose values a
+// thread reads for itself (by way of LDS they waited for another barrier: weights to sums 1.3 us of the launch's 2.7, now 0.8).
+template <typename T, typename OUT, int VEC, int AHEAD>
 __global__ __launch_bounds__(256) void latent_absorb_kernel(const T* __restrict__ q, const bf16_t* __restrict__ up,
                                                             const float* __restrict__ angles, const int* __restrict__ spans,
                                                             OUT* __restrict__ out, LatentShape a) {
   constexpr int COLUMNS = 16 * VEC;
-  extern __shared__ float lds[];            // the query's unturned columns, then 16 partial sums a column
-  float* red = lds + ((a.dim + 3) & ~3);
+  __shared__ float red[16 * COLUMNS];       // 16 partial sums a column
   const int head = blockIdx.x, slot = blockIdx.y, t = threadIdx.x, wide = a.dim + a.rot;
+  const int col = blockIdx.z * COLUMNS + (t & 15) * VEC, group = t >> 4;
   const Span s = span_of(spans, slot, a.rows);
-  if (s.rows == 0) return;
-  const T* qr = q + ((size_t)s.row0 * a.heads + head) * wide;
+  const bf16_t* w = up + (size_t)head * a.dim * a.rank + min(col, a.rank - VEC);
+  uint4 ahead[AHEAD > 0 ? AHEAD : 1];
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i) ahead[i] = *reinterpret_cast<const uint4*>(w + (size_t)min(group + 16 * i, a.dim - 1) * a.rank);
+  // (an idle slot's loads are some row's, and nothing of it is stored: behind a branch the loads would wait for the span)
+  const T* qr = q + ((size_t)min(s.row0, a.rows - 1) * a.heads + head) * wide;
+  float x[AHEAD > 0 ? AHEAD : 1];
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i) x[i] = load_one(qr + min(group + 16 * i, a.dim - 1));
   OUT* to = out + ((size_t)slot * a.heads + head) * (a.rank + a.rot);
-  for (int c = t; c < a.dim; c += 256) lds[c] = load_one(qr + c);
-  if (blockIdx.z == 0) {
+  if (blockIdx.z == 0 && s.rows > 0) {
     const float* turn = angles + (size_t)min(s.start, a.angle_rows - 1) * a.turned;
     for (int c = t; c < a.rot; c += 256) {
       float v = load_one(qr + a.dim + c);
@@ -523,25 +532,31 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(const T* __restrict_
       store_one(to + a.rank + c, v);
     }
   }
-  __syncthreads();
-  const int col = blockIdx.z * COLUMNS + (t & 15) * VEC, group = t >> 4;
   float acc[VEC];
 #pragma unroll
   for (int j = 0; j < VEC; ++j) acc[j] = 0.f;
-  if (col < a.rank) {
-    const bf16_t* w = up + (size_t)head * a.dim * a.rank + col;
-#pragma unroll 4
-    for (int d = group; d < a.dim; d += 16) {
-      float f[VEC];
-      load_vec<VEC>(w + (size_t)d * a.rank, f);
+  if constexpr (AHEAD > 0) {
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) acc[j] = fmaf(lds[d], f[j], acc[j]);
+    for (int i = 0; i < AHEAD; ++i) {
+      float f[8];
+      unpack8(ahead[i], f);
+      const float q_at = group + 16 * i < a.dim ? x[i] : 0.f;   // (past the last: a finite weight of the last row)
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) acc[j] = fmaf(q_at, f[j], acc[j]);
     }
+  }
+#pragma unroll 4
+  for (int d = group + 16 * AHEAD; d < a.dim; d += 16) {
+    float f[VEC];
+    const float q_at = load_one(qr + d);
+    load_vec<VEC>(w + (size_t)d * a.rank, f);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) acc[j] = fmaf(q_at, f[j], acc[j]);
   }
 #pragma unroll
   for (int j = 0; j < VEC; ++j) red[group * COLUMNS + (t & 15) * VEC + j] = acc[j];
   __syncthreads();
-  if (t < COLUMNS && blockIdx.z * COLUMNS + t < a.rank) {
+  if (s.rows > 0 && t < COLUMNS && blockIdx.z * COLUMNS + t < a.rank) {
     float sum = 0.f;
 #pragma unroll
     for (int g = 0; g < 16; ++g) sum += red[g * COLUMNS + t];
@@ -614,45 +629,54 @@ __global__ __launch_bounds__(256) void latent_step_kernel(const float* __restric
 // time each.  A team's keys lie in LDS as [latent, padded to 64s | shared part, padded to 32s]; its waves deal the
 // columns of the scores' product, add their parts up in LDS, and deal the columns of the weighted sum.  Heads are
 // an MFMA's columns throughout.  NG: groups of 64 latent columns a wave sums.
+//
+// The grid is (head groups x STEP_RUN splits, slots, runs of splits): the slots' first splits, which are the ones with keys, are
+// dealt out ahead of all others, and STEP_RUN neighbours, one a chiplet, read one slot's keys (slots fastest, so that a
+// chiplet has one slot's, 4 slots of 4000 keys take 25.2 us instead of 23.9).
+constexpr int STEP_RUN = 8;
 constexpr int TEAM_KEYS = 32, TEAM_PARTS = 4 * 2 * 64 * 16;   // keys, and bytes of scores in parts
 template <int NG>
 __global__ __launch_bounds__(512) void latent_step_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ latents,
                                                                const bf16_t* __restrict__ shared_keys, const int* __restrict__ spans,
-                                                               StepParts to, LatentShape a, int splits, unsigned each_inverse) {
-  constexpr int PIECES = 5 * NG;              // 16-byte pieces of a tile a thread stages
-  constexpr int STEPS = (10 * NG + 3) / 4;    // 32-column steps of the scores' product a wave takes
+                                                               StepParts to, LatentShape a, int splits, unsigned lat_inverse, unsigned rot_inverse) {
+  constexpr int LATENTS = 4 * NG, SHARED = NG;   // 16-byte pieces of a tile's latents and of its shared parts a thread stages
+  constexpr int STEPS = (10 * NG + 3) / 4;       // 32-column steps of the scores' product a wave takes
   extern __shared__ __align__(16) unsigned char dyn[];
-  const int head0 = blockIdx.x * 16, split = blockIdx.y, slot = blockIdx.z;
+  const int split = blockIdx.z * STEP_RUN + blockIdx.x % STEP_RUN, slot = blockIdx.y, head0 = blockIdx.x / STEP_RUN * 16;
   const int team = threadIdx.x >> 8, t = threadIdx.x & 255, lane = t & 63, wave = t >> 6, lo16 = lane & 15, quad = lane >> 4;
   const Span s = span_of(spans, slot, a.rows);
-  if (s.rows == 0) return;
   const StepKeys k = step_keys(s, a, splits);
-  if (split >= k.live) return;
+  if (s.rows == 0 || split >= k.live) return;
   const int rank_pad = (a.rank + 63) & ~63, rot_pad = (a.rot + 31) & ~31, pitch = rank_pad + rot_pad + 8, wide = a.rank + a.rot;
   unsigned char* mine = dyn + team * (TEAM_PARTS + TEAM_KEYS * pitch * 2);
   f32x4* parts = reinterpret_cast<f32x4*>(mine);                  // [wave][key tile][lane]
   bf16_t* tile = reinterpret_cast<bf16_t*>(mine + TEAM_PARTS);    // [32][pitch]
 
-  const int hi = min(k.count, (split + 1) * k.per), each = wide / 8;
-  int p_row[PIECES], p_col[PIECES];
-#pragma unroll
-  for (int i = 0; i < PIECES; ++i) {
-    const int e = t + 256 * i;
-    const int row = (int)__umulhi((unsigned)e, each_inverse);   // e / each
-    p_row[i] = e < TEAM_KEYS * each ? row : -1;
-    p_col[i] = (e - row * each) * 8;
-  }
-  u32x4 held[PIECES];
-  const int wrap = k.first % a.ring;
+  const int hi = min(k.count, (split + 1) * k.per), lat_each = a.rank / 8, rot_each = a.rot / 8;
+  const int wrap = k.first < a.ring ? k.first : k.first % a.ring;
+  const bf16_t* const lat0 = latents + (size_t)slot * a.ring * a.rank;
+  const bf16_t* const rot0 = shared_keys + (size_t)slot * a.ring * a.rot;
+  u32x4 held[LATENTS], held_rot[SHARED];
+  // Piece e of a tile is piece e % each of its row e / each (each 0: nobody asks).  Loads past a tile's end are its last piece again, and past the
+  // last key the last key's: behind tests, a branch a load, the first tile came 1.5 us later.
+  auto row_of = [](int e, int each, unsigned inverse) { return each == 1 ? e : (int)__umulhi((unsigned)e, inverse); };
+  auto place = [&](int row) {
+    const int in_ring = wrap + row;
+    return (size_t)(in_ring < a.ring ? in_ring : in_ring - a.ring);
+  };
   auto fetch = [&](int base) {
 #pragma unroll
-    for (int i = 0; i < PIECES; ++i)
-      if (p_row[i] >= 0) {
-        const int in_ring = wrap + min(base + p_row[i], hi - 1);   // past the last: the last again
-        const size_t at = (size_t)slot * a.ring + (in_ring < a.ring ? in_ring : in_ring - a.ring);
-        const bf16_t* from = p_col[i] < a.rank ? latents + at * a.rank + p_col[i] : shared_keys + at * a.rot + p_col[i] - a.rank;
-        held[i] = *reinterpret_cast<const u32x4*>(from);
+    for (int i = 0; i < LATENTS; ++i) {
+      const int e = min(t + 256 * i, TEAM_KEYS * lat_each - 1), row = row_of(e, lat_each, lat_inverse);
+      held[i] = *reinterpret_cast<const u32x4*>(lat0 + place(min(base + row, hi - 1)) * a.rank + (e - row * lat_each) * 8);
+    }
+    if (a.rot > 0) {
+#pragma unroll
+      for (int i = 0; i < SHARED; ++i) {
+        const int e = min(t + 256 * i, TEAM_KEYS * rot_each - 1), row = row_of(e, rot_each, rot_inverse);
+        held_rot[i] = *reinterpret_cast<const u32x4*>(rot0 + place(min(base + row, hi - 1)) * a.rot + (e - row * rot_each) * 8);
       }
+    }
   };
   int base = split * k.per + team * TEAM_KEYS;
   fetch(base);
@@ -681,9 +705,15 @@ __global__ __launch_bounds__(512) void latent_step_mfma_kernel(const bf16_t* __r
   for (; base - team * TEAM_KEYS < hi; base += STEP_KEYS) {   // (a team past the last key: weights of zero)
     __syncthreads();   // the last tile's readers are done
 #pragma unroll
-    for (int i = 0; i < PIECES; ++i)
-      if (p_row[i] >= 0)
-        *reinterpret_cast<u32x4*>(tile + p_row[i] * pitch + (p_col[i] < a.rank ? p_col[i] : rank_pad + p_col[i] - a.rank)) = held[i];
+    for (int i = 0; i < LATENTS; ++i) {
+      const int e = t + 256 * i, row = row_of(e, lat_each, lat_inverse);
+      if (e < TEAM_KEYS * lat_each) *reinterpret_cast<u32x4*>(tile + row * pitch + (e - row * lat_each) * 8) = held[i];
+    }
+#pragma unroll
+    for (int i = 0; i < SHARED; ++i) {
+      const int e = t + 256 * i, row = row_of(e, rot_each, rot_inverse);
+      if (e < TEAM_KEYS * rot_each) *reinterpret_cast<u32x4*>(tile + row * pitch + rank_pad + (e - row * rot_each) * 8) = held_rot[i];
+    }
     __syncthreads();
     if (base - team * TEAM_KEYS + STEP_KEYS < hi) fetch(base + STEP_KEYS);
     f32x4 sc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
@@ -826,14 +856,14 @@ __global__ __launch_bounds__(256) void latent_values_kernel(StepParts from, cons
   auto piece = [&](int i, int c) {
     return *reinterpret_cast<const piece_t*>(from.sums + (part + (size_t)min(i, k.live - 1) * a.heads) * a.rank + c);
   };
+  auto stat = [&](int i) { return *reinterpret_cast<const float2*>(from.stats + 2 * (part + (size_t)min(i, k.live - 1) * a.heads)); };
+  const float2 held = stat(lane);
   const int mine = min(t * COLUMNS, a.rank - COLUMNS);
   piece_t ahead[VALUE_AHEAD];
   if (CH > 0) {
 #pragma unroll
     for (int j = 0; j < VALUE_AHEAD; ++j) ahead[j] = piece(j, mine);
   }
-  auto stat = [&](int i) { return *reinterpret_cast<const float2*>(from.stats + 2 * (part + (size_t)min(i, k.live - 1) * a.heads)); };
-  const float2 held = stat(lane);
   const float sunk = sink != nullptr ? bf16_to_f32(sink[head]) * LATENT_LOG2E : -1e30f;
   float top = fmaxf(sunk, held.x), total = 0.f;
   for (int i = lane + 64; i < k.live; i += 64) top = fmaxf(top, stat(i).x);
@@ -915,12 +945,17 @@ static size_t step_mfma_lds(const LatentShape& a) {
   const size_t bytes = 2 * (TEAM_PARTS + (size_t)TEAM_KEYS * (((a.rank + 63) & ~63) + ((a.rot + 31) & ~31) + 8) * 2);
   return bytes <= 163840 ? bytes : 0;
 }
+// Splits for a block a CU: each leaves a float32 sum of the rank a head, which is more than its keys' bytes under 64 keys a
+// split, and blocks whose runs hold no keys yet still have to be dealt out (16 heads over 512 + 64 columns, with the launches
+// around it, 512 blocks -> 256: 8 slots of 4000 keys 35.1 -> 29.8 us, 16 slots of 30 27.2 -> 20.2, of 4000 49.9 -> 44.4, 32 slots
+// of 30 33.0 -> 27.2).  No fewer than 8: 64 slots of 4000 keys take 135 us by 8 and 218 by 4.
 static int step_splits(const LatentShape& a) {
   const int most = a.window < a.ring ? a.window : a.ring, tiles = (most + STEP_KEYS - 1) / STEP_KEYS;
-  int splits = 512 / (a.slots * ((a.heads + 15) / 16));
+  int splits = 256 / (a.slots * ((a.heads + 15) / 16));
   splits = splits < 8 ? 8 : (splits > 64 ? 64 : splits);
   return tiles < splits ? tiles : splits;
 }
+static unsigned inverse_of(int n) { return n > 0 ? (unsigned)((1ull << 32) / (unsigned)n + 1) : 0; }   // (1's does not fit)
 static size_t rounded16(size_t n) { return (n + 15) & ~(size_t)15; }
 
 static int check_latent(const char* what, const LatentShape& a, const void* spans, const void* shared_keys, const void* angles) {
@@ -1000,18 +1035,17 @@ extern "C" int iron_mha_latent(const void* q, const void* latents, const void* s
     parts.stats = (float*)((unsigned char*)parts.sums + rounded16((size_t)slots * splits * heads * rank * 4));
     const bool vec = rank % 8 == 0;
     const dim3 ag(heads, slots, vec ? (rank + 127) / 128 : (rank + 15) / 16);
-    const size_t alds = (size_t)(((dim + 3) & ~3) + 16 * (vec ? 128 : 16)) * 4;
 #define IRON_ABSORB(T, OUT)                                                                                                              \
   {                                                                                                                                      \
-    if (vec) hipLaunchKernelGGL((latent_absorb_kernel<T, OUT, 8>), ag, dim3(256), alds, s, (const T*)q, up, angles, spans, (OUT*)absorbed, a); \
-    else hipLaunchKernelGGL((latent_absorb_kernel<T, OUT, 1>), ag, dim3(256), alds, s, (const T*)q, up, angles, spans, (OUT*)absorbed, a);     \
+    if (vec) hipLaunchKernelGGL((latent_absorb_kernel<T, OUT, 8, 8>), ag, dim3(256), 0, s, (const T*)q, up, angles, spans, (OUT*)absorbed, a); \
+    else hipLaunchKernelGGL((latent_absorb_kernel<T, OUT, 1, 0>), ag, dim3(256), 0, s, (const T*)q, up, angles, spans, (OUT*)absorbed, a);     \
   }
     if (is_float) IRON_ABSORB(float, float)
     else if (mfma_lds) IRON_ABSORB(bf16_t, bf16_t)
     else IRON_ABSORB(bf16_t, float)
 #undef IRON_ABSORB
     if (mfma_lds) {
-      const dim3 grid((heads + 15) / 16, splits, slots);
+      const dim3 grid((heads + 15) / 16 * STEP_RUN, slots, (splits + STEP_RUN - 1) / STEP_RUN);
 #define IRON_STEP(NG)                                                                                                        \
   static LdsOptIn opted##NG;                                                                                                 \
   if (const hipError_t e = opted##NG.ensure((const void*)latent_step_mfma_kernel<NG>, 163840)) {                             \
@@ -1019,7 +1053,7 @@ extern "C" int iron_mha_latent(const void* q, const void* latents, const void* s
     return (int)e;                                                                                                           \
   }                                                                                                                          \
   hipLaunchKernelGGL((latent_step_mfma_kernel<NG>), grid, dim3(512), mfma_lds, s, (const bf16_t*)absorbed, (const bf16_t*)latents, \
-                     (const bf16_t*)shared_keys, spans, parts, a, splits, (unsigned)((1ull << 32) / (unsigned)((rank + rot) / 8) + 1))
+                     (const bf16_t*)shared_keys, spans, parts, a, splits, inverse_of(rank / 8), inverse_of(rot / 8))
       if (rank <= 256) { IRON_STEP(1); }
       else if (rank <= 512) { IRON_STEP(2); }
       else { IRON_STEP(4); }

@@ -246,6 +246,34 @@ def test_latent_rows(cuda, dtype, q_rank, rank, rot, turn):
     agrees(op, given, 3e-6 if dtype is F32 else 5e-3, rows_of(spans))
 
 
+# A row a slot in the latents' space: latents and shared parts of one piece, none, several a thread; heads past a group of sixteen; keys wider than the weights
+# asked for ahead, no whole sixteens; fewer keys than splits and more, splits no multiple of the grid's runs, a ring that wraps.
+@pytest.mark.parametrize("H,D,rot,V,R,window,slots,T", [(3, 16, 8, 16, 8, None, 2, 90), (20, 32, 0, 24, 40, 300, 5, 400), (17, 20, 64, 8, 512, None, 12, 700),
+                                                        (2, 200, 24, 16, 96, 130, 3, 260), (1, 128, 16, 40, 264, None, 9, 1300), (2, 9, 40, 8, 520, 70, 4, 200)])
+def test_steps_of_several_slots_in_the_latents_space(cuda, H, D, rot, V, R, window, slots, T):
+    rng = np.random.default_rng(R)
+    base, scale, ring = 300.0, 1 / np.sqrt(D + rot), min(T, (window or T) + 1)
+    spans, order = table(slots=slots), rng.permutation(slots)[1:]   # one is idle
+    latents, keys, q = np.full((slots, ring, R), 5.0, F32), np.full((slots, ring, rot), 5.0, F32), np.zeros((slots, H * (D + rot)), F32)
+    want, up = {}, None
+    for row, slot in enumerate(order):
+        n = (T, 1, 65, T // 2, 64, T - 1)[row % 6]   # its keys, this step's among them
+        qs, c, r, u, _ = latent_case(rng, H, D, rot, V, R, window, n, False)
+        up = u if up is None else up
+        want[row] = plain_latent(qs, c, r, up, None, H, D, rot, V, R, window, scale, base)[-1]
+        ring_rows(latents[slot], ring, c, 0)
+        if rot:
+            ring_rows(keys[slot], ring, round_bf16(turned(r, base, rot).astype(F32)), 0)
+        q[row], spans[slot] = qs[-1], (row, 1, n - 1, 0)
+    given = dict(q=q, latents=latents, up=up, spans=spans) | (dict(shared_keys=keys, angles=rope_angles(rot, T, base)) if rot else {})
+    op = LatentMHA(slots=slots, rows=slots, heads=H, dim=D, rot=rot, vdim=V, rank=R, turned=rot, angle_rows=T if rot else 0, sunk=False,
+                   window=window or EVERYTHING, ring=ring, cap=T, scale=scale, single=True)
+    y = ran(op, workspace=True, **given)["y"]
+    for row in range(len(order)):
+        assert np.abs(y[row] - want[row]).max() <= 2e-2 * np.abs(want[row]).max(), row
+    assert (y[len(order) :] == 7).all()
+
+
 def test_a_long_step_over_many_splits(cuda):
     """A step far from the sequence's start: every split of the keys has several tiles, and the loudest key is in
     the first, a middle or the last one."""
