@@ -20,11 +20,11 @@ constexpr int kMaxSplits = 128;      // what the workspace holds per head
 constexpr int kScanMaxSplits = 128;  // the lane-scan kernels' own limit
 constexpr int kSingleMaxKeys = 2048;  // lane-scan kernels: caches up to this many rows take the one-launch kernel
 // One-shape launch: up to this many live keys one block a query head writes O itself.  Where the two
-// forms cost the same inside that launch shape (32 / 8 heads of 64, an 8192-row cache, us at 1024 /
-// 1280 / 1536 / 2048 live keys: one block a head 8.0 / 8.8 / 9.7 / 12.1, split + merge 9.0 / 9.0 /
-// 9.0 / 9.5).
-constexpr int kShortKeys = 1408;
+// forms cost the same inside that launch shape (an 8192-row cache, us, one block a head / split + merge: 32 / 8 heads
+// of 64, 400 live keys 5.8 / 6.0, 500 5.9 / 6.1, 600 6.5 / 6.3, 1000 8.1 / 6.45; of 128, 300 6.4 / 7.2, 400 7.4 / 7.3, 600 8.1 / 7.4).
+constexpr int short_keys_of(int d) { return d == 64 ? 512 : 384; }
 constexpr int kComputeUnits = 256;    // MI355X: what the split count is sized for
+constexpr int EITHER_WAVES = 8;       // waves a block of the one-shape launch
 
 // 2^x for x <= 0 by the hardware's own instruction: a softmax weight small enough to be a denormal
 // counts as 0, which saves the library routine's rescaling around every call.
@@ -336,41 +336,38 @@ __global__ __launch_bounds__(1024) void mha_decode_single_kernel(
   }
 }
 
-// The run of keys a block of the split scan takes: an equal share of the live keys, in whole
-// 16-key tiles for each of the 2^share_log2 waves that work on one KV head.  The scan and the merge
-// both derive it from the same words.
-__device__ __forceinline__ int decode_chunk(int live, int nsplit, int share_log2) {
-  const int unit = 16 << share_log2;
-  return ((live + nsplit - 1) / nsplit + unit - 1) & ~(unit - 1);
-}
-
 // ---- one query, one launch shape whatever the cache's length
 //
-// grid = (sets, nsplit) blocks of WAVES waves, as many as the chip has CUs; the blocks choose what to
+// grid = (sets, nsplit) blocks of eight waves, as many as the chip has CUs; the blocks choose what to
 // do by the live keys n = *kv_valid (less what a window drops), so the work and its spread over the
 // chip follow the context and the cache only sizes the buffers.
 //
 // n <= short_keys: the first `heads` blocks each scan all keys for one query head with the
-// lane-per-column scan above (16 waves a head: the launch is latency-bound, and this is the shortest
-// chain) and write the output row; the others leave at once, and so does the merge launch behind.
+// lane-per-column scan above and write the output row; the others leave at once, and so does the merge launch behind.
 //
-// Otherwise the keys are dealt over the nsplit blocks of a set of KV heads in equal runs sized by n,
+// Otherwise the keys are dealt over the nsplit blocks of a set of KV heads, 32 at a time in turn -- all blocks
+// together read one run of them at a time, and no wave has two steps more than another --
 // and a block leaves (max, sum, O) per head for the merge.  Here the G query heads that share a KV
 // head are the columns of a 16-wide MFMA tile (G <= 16; the rest are zero columns), so a key row is
-// multiplied with all of them by one instruction stream whatever G is.  A wave works through its own
-// run of keys 32 at a time.  S^T = K Q^T (M = keys, N = heads): the K rows are the A operand exactly
+// multiplied with all of them by one instruction stream whatever G is.  S^T = K Q^T (M = keys, N = heads): the K rows are the A operand exactly
 // as they lie in memory (lane -> key row lane % 16, 16-byte piece lane / 16 of a 32-wide k-step), so
 // they go from global memory straight into registers.  A lane then owns one head column: the softmax
 // is in-lane but for the maximum over the four lanes of a column, which is only exchanged on the
 // (rare) steps where some lane's own maximum passes the column's reference.  The probabilities,
-// rounded to bf16, are already the B operand of O^T = V^T P^T; V^T comes from the transposing LDS read
+// in two bf16 terms (their distance from 64 bits is then that of the form that keeps them in 32; rounded to one, 2000 to 16384 keys
+// were 1.06 to 1.09 times as far off), are already the B operand of O^T = V^T P^T; V^T comes from the transposing LDS read
 // of the wave's own 32-row V tile, which buffer loads put there as stored (16-byte chunks
 // XOR-swizzled by 2 (row & 3), as the prompt kernel's).  Rows past the last live key lie outside the
 // buffers and read as zeros.
-template <int D, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void mha_decode_either_kernel(
+//
+// At a few thousand keys the launch is as long as its instructions, which the waves of a SIMD take in turn, so there
+// are eight a block and not sixteen, and nothing of a block's shape is a variable.  32 / 8 heads of 64 with the merge, us: runs of whole steps of
+// sixteen waves a block, then of eight, then keys in turn: 1420 keys 8.65 / 6.55 / 6.4, 4000 8.75 / 7.4 / 7.3, 8000 9.65 / 8.8 / 8.55, 12003
+// 11.9 / 11.0 / 10.2, 16300 13.4 / 12.9 / 12.0 (the second term of the probabilities 0.05 to 0.1 more).
+template <int D, int HPB_LOG2>
+__global__ __launch_bounds__(64 * EITHER_WAVES) void mha_decode_either_kernel(
     const bf16_t* __restrict__ Q, const bf16_t* __restrict__ K, const bf16_t* __restrict__ V,
-    bf16_t* __restrict__ O, float* __restrict__ part, int kv_heads, int group, int hpb_log2, int kv_len,
+    bf16_t* __restrict__ O, float* __restrict__ part, int kv_heads, int group, int kv_len,
     float scale_log2, int window, long row_stride, long head_stride, const int* __restrict__ kv_valid,
     const int* __restrict__ kv_first, int kv_rows, int short_keys) {
   constexpr int ROWB = D * 2;            // bytes of a V row in LDS
@@ -381,8 +378,7 @@ __global__ __launch_bounds__(64 * WAVES) void mha_decode_either_kernel(
   constexpr int TILE = TK * ROWB;        // bytes of a V tile
   constexpr int VINST = TILE / 1024;     // 1 KB loads into LDS a tile
   constexpr int RPI = 1024 / ROWB;       // rows one of them covers
-  constexpr int WAVES_LOG2 = WAVES == 16 ? 4 : 3;
-  static_assert(WAVES == 16 || WAVES == 8, "waves a block");
+  constexpr int WAVES = EITHER_WAVES, HPB = 1 << HPB_LOG2, SHARE = WAVES >> HPB_LOG2;   // KV heads a block, waves a head
   extern __shared__ __align__(1024) char smem_dec[];   // WAVES x 2 x TILE bytes
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -435,27 +431,22 @@ __global__ __launch_bounds__(64 * WAVES) void mha_decode_either_kernel(
     return;
   }
 
-  // ---- many keys: the block takes one run of them for 2^hpb_log2 KV heads at once, wave w on head
-  // w % hpb (with the heads interleaved in a cache row, the block's loads then cover longer pieces of it).
+  // ---- many keys: the block takes its share of them for HPB KV heads at once, wave w on head
+  // w % HPB (with the heads interleaved in a cache row, the block's loads then cover longer pieces of it).
   const int n = lane & 15, q = lane >> 4;   // head column, quarter of the k slots
-  const int hpb = 1 << hpb_log2, share_log2 = WAVES_LOG2 - hpb_log2;
   const int split = blockIdx.y;
-  const int kvh = (blockIdx.x << hpb_log2) + (wave & (hpb - 1));
-  const int sub = wave >> hpb_log2;          // this wave's place among the 2^share_log2 on its head
-  const int chunk = decode_chunk(live, nsplit, share_log2);
-  const int blo = first + split * chunk, bhi = min(blo + chunk, kv_tokens);
-  if (blo >= kv_tokens) return;   // the merge reads the splits that hold keys, no more
-  // The wave's run of keys, in whole 16-key MFMA tiles.
-  const int per = ((((bhi - blo) + (1 << share_log2) - 1) >> share_log2) + 15) & ~15;
-  const int wlo = blo + sub * per, whi = min(wlo + per, bhi);
-  const int steps = wlo < whi ? (whi - wlo + TK - 1) / TK : 0;
+  const int kvh = (blockIdx.x << HPB_LOG2) + (wave & (HPB - 1));
+  const int sub = wave >> HPB_LOG2;          // this wave's place among the SHARE on its head
+  if (split * TK >= live) return;   // the merge reads the splits that hold keys, no more
+  // The wave's steps, SHARE * nsplit tiles of keys apart.
+  const int k_first = first + (sub * nsplit + split) * TK, k_step = SHARE * nsplit * TK;
+  auto has = [=](int step) { return k_first + step * k_step < kv_tokens; };
 
   const bf16_t* Kh = K + (size_t)kvh * head_stride + first_row * row_stride;
   const bf16_t* Vh = V + (size_t)kvh * head_stride + first_row * row_stride;
   const int row_bytes = (int)row_stride * 2;
-  // The head's keys (values) up to the last of this wave's run are one buffer: rows past it -- the
-  // next wave's, or past the last live key -- read as zeros and cost no traffic.
-  const int reach = wlo < whi ? (whi - 1) * row_bytes + ROWB : 0;
+  // The head's live keys (values) are one buffer: rows past the last read as zeros and cost no traffic.
+  const int reach = (kv_tokens - 1) * row_bytes + ROWB;
   const __amdgpu_buffer_rsrc_t k_rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(Kh), 0, reach, 0x00020000);
   const __amdgpu_buffer_rsrc_t v_rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(Vh), 0, reach, 0x00020000);
 
@@ -473,7 +464,7 @@ __global__ __launch_bounds__(64 * WAVES) void mha_decode_either_kernel(
 
   bf16x8 kf[2][2][KS];   // [register set][tile][k-step]
   auto issue_v = [&](int step, int set) {
-    const int at = (wlo + step * TK) * row_bytes;
+    const int at = (k_first + step * k_step) * row_bytes;
 #pragma unroll
     for (int i = 0; i < VINST; ++i)
       // (the cast keeps the offset's type from depending on the template: as a dependent expression
@@ -483,7 +474,7 @@ __global__ __launch_bounds__(64 * WAVES) void mha_decode_either_kernel(
   };
   auto issue = [&](int step, auto set_c) {
     constexpr int set = decltype(set_c)::value;
-    const int at = (wlo + step * TK) * row_bytes;
+    const int at = (k_first + step * k_step) * row_bytes;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -496,11 +487,11 @@ __global__ __launch_bounds__(64 * WAVES) void mha_decode_either_kernel(
   // in flight, so it needs no count of what the compiler may have moved.
   using set0 = std::integral_constant<int, 0>;
   using set1 = std::integral_constant<int, 1>;
-  if (steps > 0) {
+  if (has(0)) {
     issue_v(0, 0);
     issue(0, set0{});
   }
-  if (steps > 1) {
+  if (has(1)) {
     issue_v(1, 1);
     issue(1, set1{});
   }
@@ -542,10 +533,10 @@ __global__ __launch_bounds__(64 * WAVES) void mha_decode_either_kernel(
 #pragma unroll
       for (int s = 0; s < KS; ++s) sacc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[set][t][s], qf[s], sacc[t], 0, 0, 0);
     }
-    // Element i of tile t is key k0 + 16 t + 4 q + i; the wave's last step may reach past its run.
-    const int k0 = wlo + step * TK;
-    const int left = whi - k0 - 4 * q;   // keys of this lane's tile-0 quarter inside the run (may be <= 0)
-    const bool edge = k0 + TK > whi;
+    // Element i of tile t is key k0 + 16 t + 4 q + i; the last step of all may reach past the last key.
+    const int k0 = k_first + step * k_step;
+    const int left = kv_tokens - k0 - 4 * q;   // live keys of this lane's tile-0 quarter (may be <= 0)
+    const bool edge = k0 + TK > kv_tokens;
     if (edge) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
@@ -582,25 +573,37 @@ __global__ __launch_bounds__(64 * WAVES) void mha_decode_either_kernel(
         p[4 * t + i] = e;
         l_run += e;
       }
-    const bf16x8 pf = __builtin_bit_cast(bf16x8, pack8(p));
+    // The weights as two bf16 terms, together within 2^-17: the matrix cores idle.  The first is cut off and 2^-20 of the weight
+    // joins the second, so that both are positive and an infinite value stays what it is.
+    uint32_t high[4];
+    float rest[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) rest[i] = fmaf(p[i], 1.f + 0x1p-20f, -__uint_as_float(__float_as_uint(p[i]) & 0xffff0000u));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) high[i] = (__float_as_uint(p[2 * i]) >> 16) | (__float_as_uint(p[2 * i + 1]) & 0xffff0000u);
+    const bf16x8 pf = __builtin_bit_cast(bf16x8, make_uint4(high[0], high[1], high[2], high[3])), pr = __builtin_bit_cast(bf16x8, pack8(rest));
 #pragma unroll
     for (int dt = 0; dt < DT; dt += 2) {
       lds_tr_wait(vf[dt], vf[dt + 1]);
-      oacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tr_join(vf[dt]), pf, oacc[dt], 0, 0, 0);
-      oacc[dt + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tr_join(vf[dt + 1]), pf, oacc[dt + 1], 0, 0, 0);
+#pragma unroll
+      for (int e = dt; e < dt + 2; ++e) {
+        const bf16x8 v = tr_join(vf[e]);
+        oacc[e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pf, oacc[e], 0, 0, 0);
+        oacc[e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pr, oacc[e], 0, 0, 0);
+      }
     }
   };
 
-  for (int step = 0; step < steps; step += 2) {
+  for (int step = 0; has(step); step += 2) {
     wait_vmcnt<0>();
     compute(step, set0{});
-    if (step + 2 < steps) {
+    if (has(step + 2)) {
       issue_v(step + 2, 0);
       issue(step + 2, set0{});
     }
-    if (step + 1 < steps) {
+    if (has(step + 1)) {
       compute(step + 1, set1{});
-      if (step + 3 < steps) {
+      if (has(step + 3)) {
         issue_v(step + 3, 1);
         issue(step + 3, set1{});
       }
@@ -629,36 +632,31 @@ __global__ __launch_bounds__(64 * WAVES) void mha_decode_either_kernel(
     }
   }
   __syncthreads();
-  // Column hg = (head of the block's, query head of its group) lies in waves hw, hw + hpb, ...: entry
-  // hg + j hpb group of the hand-over for j < share.
-  const int share = 1 << share_log2;
-  const int wave_step = (group << hpb_log2) * (D + 2);
-  for (int idx = tid; idx < (group << hpb_log2) * (D / 2); idx += 64 * WAVES) {
+  // Column hg = (head of the block's, query head of its group) lies in waves hw, hw + HPB, ...: entry
+  // hg + j HPB group of the hand-over for j < SHARE.
+  const int wave_step = (group << HPB_LOG2) * (D + 2);
+  for (int idx = tid; idx < (group << HPB_LOG2) * (D / 2); idx += 64 * WAVES) {
     const int hg = idx / (D / 2), pair = idx % (D / 2);
     const float* col = hand + (size_t)hg * (D + 2);
-    float2 mlv[WAVES], av[WAVES];
+    float2 mlv[SHARE], av[SHARE];
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-      mlv[w] = make_float2(-INFINITY, 0.f);
-      av[w] = make_float2(0.f, 0.f);
-      if (w < share) {   // uniform over the block
-        mlv[w] = *reinterpret_cast<const float2*>(col + w * wave_step);
-        av[w] = *reinterpret_cast<const float2*>(col + w * wave_step + 2 + 2 * pair);
-      }
+    for (int w = 0; w < SHARE; ++w) {
+      mlv[w] = *reinterpret_cast<const float2*>(col + w * wave_step);
+      av[w] = *reinterpret_cast<const float2*>(col + w * wave_step + 2 + 2 * pair);
     }
     float mx = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) mx = fmaxf(mx, mlv[w].x);
+    for (int w = 0; w < SHARE; ++w) mx = fmaxf(mx, mlv[w].x);
     float lt = 0.f, at0 = 0.f, at1 = 0.f;
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
+    for (int w = 0; w < SHARE; ++w) {
       const float e = (mlv[w].x == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((mlv[w].x - mx) * scale_log2);
       lt = fmaf(mlv[w].y, e, lt);
       at0 = fmaf(av[w].x, e, at0);
       at1 = fmaf(av[w].y, e, at1);
     }
     // part layout: [head][split][D + 2] = {max in the exp2 domain, sum, O[D]}.
-    const int head = (blockIdx.x << hpb_log2) * group + hg;
+    const int head = (blockIdx.x << HPB_LOG2) * group + hg;
     float* out = part + ((size_t)head * nsplit + split) * (D + 2);
     *reinterpret_cast<float2*>(out + 2 + 2 * pair) = make_float2(at0, at1);
     if (pair == 0) *reinterpret_cast<float2*>(out) = make_float2((mx == -INFINITY) ? -INFINITY : mx * scale_log2, lt);
@@ -676,7 +674,7 @@ __global__ __launch_bounds__(64 * WAVES) void mha_decode_either_kernel(
 // themselves.
 template <int D, int PER>
 __global__ __launch_bounds__(4 * D) void mha_decode_either_merge_kernel(
-    const float* __restrict__ part, bf16_t* __restrict__ O, int nsplit, int share_log2, int kv_len, int window,
+    const float* __restrict__ part, bf16_t* __restrict__ O, int nsplit, int kv_len, int window,
     const int* __restrict__ kv_valid, int short_keys) {
   constexpr int PAIRS = D / 2;
   const int head = blockIdx.x, t = threadIdx.x % PAIRS, eighth = threadIdx.x / PAIRS;
@@ -692,14 +690,13 @@ __global__ __launch_bounds__(4 * D) void mha_decode_either_merge_kernel(
   const int first = (window >= 0) ? max(0, kv_tokens - 1 - window) : 0;
   const int live = kv_tokens - first;
   if (live <= short_keys) return;
-  const int chunk = decode_chunk(live, nsplit, share_log2);
-  const int used = (live + chunk - 1) / chunk;
+  auto used = [=](int split) { return split < nsplit && split * 32 < live; };
   float mx = -INFINITY, lt = 0.f, at0 = 0.f, at1 = 0.f;
-  for (int s0 = eighth; s0 < used; s0 += 8 * PER) {
+  for (int s0 = eighth; used(s0); s0 += 8 * PER) {
     if (s0 >= 8 * PER) {
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
-        const int s = min(s0 + 8 * i, used - 1);
+        const int s = min(s0 + 8 * i, nsplit - 1);
         ml[i] = *reinterpret_cast<const float2*>(p + s * (D + 2));
         a[i] = *reinterpret_cast<const float2*>(p + s * (D + 2) + 2 + 2 * t);
       }
@@ -707,14 +704,14 @@ __global__ __launch_bounds__(4 * D) void mha_decode_either_merge_kernel(
     float cm = mx;
 #pragma unroll
     for (int i = 0; i < PER; ++i)
-      if (s0 + 8 * i < used) cm = fmaxf(cm, ml[i].x);
+      if (used(s0 + 8 * i)) cm = fmaxf(cm, ml[i].x);
     const float keep = (mx == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mx - cm);
     lt *= keep;
     at0 *= keep;
     at1 *= keep;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const bool in = s0 + 8 * i < used && ml[i].x != -INFINITY;
+      const bool in = used(s0 + 8 * i) && ml[i].x != -INFINITY;
       const float e = in ? __builtin_amdgcn_exp2f(ml[i].x - cm) : 0.f;
       lt = fmaf(in ? ml[i].y : 0.f, e, lt);
       at0 = fmaf(in ? a[i].x : 0.f, e, at0);
@@ -764,35 +761,31 @@ static void launch_decode(const bf16_t* Q, const bf16_t* K, const bf16_t* V, bf1
 
 
 // The one-shape launch and, where the cache can hold more than `short_keys` rows, the merge behind it.
-template <int D, int WAVES>
+template <int D, int HPB_LOG2>
 static int launch_decode_either(const bf16_t* Q, const bf16_t* K, const bf16_t* V, bf16_t* O, float* part, int kv_heads,
                                 int group, int kv_len, float scale_log2, int window, long row_stride, long head_stride,
                                 const int* kv_valid, const int* kv_first, int kv_rows, int short_keys, hipStream_t s) {
-  constexpr size_t lds = (size_t)WAVES * 2 * 32 * D * 2;
+  constexpr size_t lds = (size_t)EITHER_WAVES * 2 * 32 * D * 2;
   static LdsOptIn opt_in;
-  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&mha_decode_either_kernel<D, WAVES>), lds); e != hipSuccess) {
+  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&mha_decode_either_kernel<D, HPB_LOG2>), lds); e != hipSuccess) {
     set_error("mha_decode: %s", hipGetErrorString(e));
     return (int)e;
   }
-  // A block of the split scan serves two KV heads where their number is even (with the heads
-  // interleaved in a cache row its loads then cover 256-byte pieces: measured a tenth faster than one
-  // head a block; four or eight heads a block stream faster still but leave more, smaller partial
-  // results), and there are as many blocks as the chip has CUs -- and no fewer than query heads,
-  // which the few-keys form needs -- whatever the cache's length.
-  const int hpb_log2 = kv_heads % 2 == 0 ? 1 : 0;
-  const int sets = kv_heads >> hpb_log2;
+  // As many blocks as the chip has CUs -- and no fewer than query heads, which the few-keys form
+  // needs -- whatever the cache's length.
+  const int sets = kv_heads >> HPB_LOG2;
   int nsplit = kComputeUnits / sets;
   while (sets * nsplit < kv_heads * group) ++nsplit;
   nsplit = nsplit < 1 ? 1 : (nsplit > kMaxSplits ? kMaxSplits : nsplit);
-  hipLaunchKernelGGL((mha_decode_either_kernel<D, WAVES>), dim3(sets, nsplit), dim3(64 * WAVES), lds, s, Q, K, V, O,
-                     part, kv_heads, group, hpb_log2, kv_len, scale_log2, window, row_stride, head_stride, kv_valid,
+  hipLaunchKernelGGL((mha_decode_either_kernel<D, HPB_LOG2>), dim3(sets, nsplit), dim3(64 * EITHER_WAVES), lds, s, Q, K, V, O,
+                     part, kv_heads, group, kv_len, scale_log2, window, row_stride, head_stride, kv_valid,
                      kv_first, kv_rows, short_keys);
   if (nsplit <= 64)
     hipLaunchKernelGGL((mha_decode_either_merge_kernel<D, 8>), dim3(kv_heads * group), dim3(4 * D), 0, s, part, O,
-                       nsplit, (WAVES == 16 ? 4 : 3) - hpb_log2, kv_len, window, kv_valid, short_keys);
+                       nsplit, kv_len, window, kv_valid, short_keys);
   else
     hipLaunchKernelGGL((mha_decode_either_merge_kernel<D, 16>), dim3(kv_heads * group), dim3(4 * D), 0, s, part, O,
-                       nsplit, (WAVES == 16 ? 4 : 3) - hpb_log2, kv_len, window, kv_valid, short_keys);
+                       nsplit, kv_len, window, kv_valid, short_keys);
   return 0;
 }
 
@@ -839,12 +832,15 @@ static int mha_decode(const uint16_t* Q, const uint16_t* K, const uint16_t* V, u
                            (long)kv_len * row_stride * 2 < (1L << 31) && heads <= kMaxSplits * kv_heads;
   IRON_REQUIRE(form != 2 || either_fits,
                "mha_decode: the one-shape launch takes d = 64 or 128, up to 16 query heads a KV head and keys within 2^31 bytes");
-  const int upto = short_keys > 0 ? short_keys : kShortKeys;
+  const int upto = short_keys > 0 ? short_keys : short_keys_of(d);
   if (form == 2 || (form == 0 && either_fits && kv_len > (short_keys > 0 ? short_keys : kSingleMaxKeys))) {
-    const int rc = d == 64 ? launch_decode_either<64, 16>(Q, K, V, O, part, kv_heads, G, kv_len, scale_log2, window, row_stride,
-                                                          head_stride, kv_valid, kv_first, kv_rows, upto, s)
-                           : launch_decode_either<128, 8>(Q, K, V, O, part, kv_heads, G, kv_len, scale_log2, window, row_stride,
-                                                          head_stride, kv_valid, kv_first, kv_rows, upto, s);
+    // A block of the split scan serves two KV heads where their number is even (with the heads
+    // interleaved in a cache row its loads then cover 256-byte pieces: measured a tenth faster than one
+    // head a block; four or eight heads a block stream faster still but leave more, smaller partial
+    // results).
+    const auto launch = d == 64 ? (kv_heads % 2 == 0 ? &launch_decode_either<64, 1> : &launch_decode_either<64, 0>)
+                                : (kv_heads % 2 == 0 ? &launch_decode_either<128, 1> : &launch_decode_either<128, 0>);
+    const int rc = launch(Q, K, V, O, part, kv_heads, G, kv_len, scale_log2, window, row_stride, head_stride, kv_valid, kv_first, kv_rows, upto, s);
     if (rc != 0) return rc;
     IRON_LAUNCH_CHECK();
   }

@@ -1963,3 +1963,34 @@ def test_eval_words_advances_a_decode_step(cuda):
                          dtype=torch.int32, device=cuda)
     K.eval_words(words, exprs)
     assert words.cpu().tolist() == [11, 41, 42, 5, 20, 6, 22, 0]
+
+
+# A wave's steps in turn: a step's edges, the splits' (64 or 32 times 32 keys a round) and the lines between the few keys' form and this; one KV head a block and two,
+# heads of one and of sixteen queries, a window that begins inside a step.
+@pytest.mark.parametrize("H,G,d,window", [(32, 8, 64, None), (32, 8, 128, None), (6, 3, 64, None), (16, 1, 128, None), (4, 4, 64, 1000)])
+def test_decode_attention_takes_keys_in_turn(cuda, H, G, d, window):
+    rng = np.random.default_rng(H + d)
+    L = 8200
+    g = torch.Generator(device="cuda")
+    g.manual_seed(d)
+    q, k, v = (torch.randn(n, w, d, generator=g, device="cuda").to(torch.bfloat16) for n, w in ((1, H), (L, G), (L, G)))
+    q *= 2
+    o, workspace = torch.empty(H, d, dtype=torch.bfloat16, device="cuda"), K.mha_decode_workspace(H, d)
+    for n in (384, 385, 512, 513, 544, 545, 1408, 2047, 2049, 2080, 4097, 8192, 8193, 8200, int(rng.integers(600, 8000))):
+        past = k[n:].clone()
+        k[n:] = float("nan")   # (what lies past the live keys is nobody's)
+        K.mha_decode(q, k, v, o, heads=H, kv_heads=G, d=d, kv_len=L, kv_interleaved=True, kv_valid=torch.tensor([n], dtype=torch.int32, device="cuda"),
+                     window=window, workspace=workspace)
+        k[n:] = past
+        lo = 0 if window is None else max(0, n - 1 - window)
+        kd, vd = k[lo:n].double(), v[lo:n].double()
+        p = torch.softmax(torch.einsum("ghd,kgd->ghk", q.double().reshape(G, H // G, d), kd) / d**0.5, -1)
+        want = torch.einsum("ghk,kgd->ghd", p, vd).reshape(H, d)
+        # the output's rounding; weights within 2^-17 of themselves, and scores' sums and exponentials in 32 bits
+        assert ((o.double() - want).abs() <= 2**-8 * want.abs() + 2**-12 * vd.abs().max()).all(), n
+        if n == 2049:   # an infinite value is the output where its key weighs anything
+            v[1500, 0, 3] = float("inf")
+            K.mha_decode(q, k, v, o, heads=H, kv_heads=G, d=d, kv_len=L, kv_interleaved=True, kv_valid=torch.tensor([n], dtype=torch.int32, device="cuda"),
+                         window=window, workspace=workspace)
+            assert torch.isinf(o[: H // G, 3]).all()
+            v[1500, 0, 3] = 0.0
