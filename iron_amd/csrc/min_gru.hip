@@ -8,15 +8,21 @@
 // The step from one state to the next is affine, S -> a S + b, and so is any run of steps.  Over a prompt's portion
 // a block takes GRU_CHUNK tokens of 64 or 128 channels, GRU_TOKENS a wave: the waves fold their tokens to an (a, b)
 // each, and those to one a chunk.  A first launch does this for every chunk; in a second a block starts from the
-// state the chunks before its own leave, a wave from the one the waves before it leave, and walks.  A portion's
-// first state is put ahead of its chunks, since the block of its last chunk may replace it: a slot has two states,
+// state the chunks before its own leave (its waves fold a run of those each), a wave from the one the waves before it leave, and walks.  A
+// portion's first state is put beside its chunks, since the block of its last chunk may replace it: a slot has two states,
 // position p's in row p % 2, so that a decode step's blocks leave the one they all read.
+//
+// Four quarter-rate instructions an element bound the first launch and six the second, so what counts is that they are spread: blocks of four
+// waves (of eight, 296 blocks of a ragged batch are two on some CUs and one on the rest), and a grid of the spans' chunks one after
+// the other, where that of every slot's every chunk dealt out eight times the blocks and looked through the spans for each.  2048 channels, us:
+// eight spans of 256 rows 25.6 -> 18.5, of 96 to 422 23.3 -> 19.4, of 90 to 140 18.9 -> 14.3, four of 90 to 500 19.2 -> 13.5, one of 2048 19.5 -> 18.6, of 300
+// 12.8 -> 10.9.  (Four channels a lane and eight tokens a wave: 18.6, 20.5, 14.0, 14.4, 21.2, 11.0.)
 #include "../../include/iron_hip.h"
 #include "rows.h"
 
 namespace iron {
 
-constexpr int GRU_WAVES = 8, GRU_TOKENS = 16, GRU_CHUNK = GRU_WAVES * GRU_TOKENS;
+constexpr int GRU_WAVES = 4, GRU_TOKENS = 16, GRU_CHUNK = GRU_WAVES * GRU_TOKENS;
 
 // Two neighbouring elements, or one.
 template <int VEC, typename T>
@@ -55,11 +61,41 @@ __device__ __forceinline__ void gru_step(float zx, float ux, float& a, float& b)
 
 struct GruShape {
   int slots, rows, stride, width;
+  int chunks;   // there can be
 };
 
-// Workspace: a (a, b) pair a chunk and channel, each span's chunks behind one more that holds its first state.
-__device__ __forceinline__ float2* gru_chunk(float2* work, const int* spans, const GruShape& g, int slot, int chunk) {
-  return work + (size_t)(first_chunk(spans, g.slots, slot, g.rows, GRU_CHUNK) * 2 + chunk) * g.width;
+// Chunk `index` of all the spans' one after the other, slot after slot: its slot (-1: there are not that many) and number in it.
+struct GruChunk {
+  int slot, chunk;
+  Span span;
+};
+__device__ __forceinline__ GruChunk gru_chunk(const int* __restrict__ spans, const GruShape& g, int index) {
+  const int lane = (int)threadIdx.x & 63;
+  for (int base = 0, before = 0; base < g.slots; base += 64) {
+    const Span mine = span_of(spans, min(base + lane, g.slots - 1), g.rows);
+    const int count = base + lane < g.slots ? (mine.rows + GRU_CHUNK - 1) / GRU_CHUNK : 0;
+    for (unsigned long long live = __builtin_amdgcn_ballot_w64(count > 0); live != 0; live &= live - 1) {
+      const int at = __builtin_ctzll(live), here = __builtin_amdgcn_readlane(count, at);
+      if (index < before + here) {
+        const Span s{__builtin_amdgcn_readlane(mine.row0, at), __builtin_amdgcn_readlane(mine.rows, at), __builtin_amdgcn_readlane(mine.start, at)};
+        return GruChunk{base + at, index - before, s};
+      }
+      before += here;
+    }
+  }
+  return GruChunk{-1, 0, Span{0, 0, 0}};
+}
+
+// Workspace: a (a, b) pair a chunk and channel, and behind all of them each chunk's first state, of which a span's first is used.
+template <int VEC>
+__device__ __forceinline__ void load_pairs(const float2* __restrict__ p, float2 (&f)[VEC]) {
+  if constexpr (VEC == 1) {
+    f[0] = p[0];
+  } else {
+    const float4 w = *reinterpret_cast<const float4*>(p);
+    f[0] = make_float2(w.x, w.y);
+    f[1] = make_float2(w.z, w.w);
+  }
 }
 
 // A wave's tokens of the columns `at ..` of the projection (its last again past the span's end).
@@ -75,18 +111,23 @@ __global__ __launch_bounds__(GRU_WAVES * 64) void min_gru_chunks_kernel(const T*
                                                                         const bf16_t* __restrict__ xb, float* __restrict__ state,
                                                                         const int* __restrict__ spans, float2* __restrict__ work,
                                                                         T* __restrict__ y, GruShape g) {
-  __shared__ float2 folded[GRU_WAVES][64 * VEC];
-  const int slot = blockIdx.z, chunk = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const Span s = span_of(spans, slot, g.rows);
+  __shared__ float2 folded[GRU_WAVES][64 * VEC], before[WALK ? GRU_WAVES : 1][WALK ? 64 * VEC : 1];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int index = (int)(blockIdx.z * gridDim.y + blockIdx.y);
+  if (index >= g.chunks) return;
+  const GruChunk mine = gru_chunk(spans, g, index);
+  if (mine.slot < 0) return;
+  const int slot = mine.slot, chunk = mine.chunk;
+  const Span s = mine.span;
   const int first = chunk * GRU_CHUNK, t0 = first + wave * GRU_TOKENS;
-  if (first >= s.rows) return;
   const bool last = first + GRU_CHUNK >= s.rows;
   const int c = (blockIdx.x * 64 + lane) * VEC, at = min(c, g.width - VEC);   // (a lane past the width: the last channels, not stored)
   const bool in = c < g.width;
-  float2* chunks = gru_chunk(work, spans, g, slot, 0) + at;
+  float2* chunks = work + (size_t)(index - chunk) * g.width + at;   // the span's
+  float* from = reinterpret_cast<float*>(work + (size_t)g.chunks * g.width) + (size_t)(index - chunk) * g.width + at;
   if (!WALK && chunk == 0 && wave == 0 && in)
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) chunks[j] = make_float2(0.f, s.start > 0 ? state[(size_t)(2 * slot + ((s.start - 1) & 1)) * g.width + at + j] : 0.f);
+    for (int j = 0; j < VEC; ++j) from[j] = s.start > 0 ? state[(size_t)(2 * slot + ((s.start - 1) & 1)) * g.width + at + j] : 0.f;
   if (!WALK && last) return;
   float z[GRU_TOKENS][VEC], u[GRU_TOKENS][VEC], o[GRU_TOKENS][VEC], zbias[VEC], xbias[VEC];
   gru_load<T, VEC>(x, g, s, t0, at, z);
@@ -109,17 +150,28 @@ __global__ __launch_bounds__(GRU_WAVES * 64) void min_gru_chunks_kernel(const T*
       b[j] = fmaf(p, b[j], q);
     }
 #pragma unroll
-  for (int j = 0; j < VEC; ++j) folded[wave][lane * VEC + j] = make_float2(a[j], b[j]);
-  if (WALK) {
+  for (int j = 0; j < VEC; ++j) folded[wave][j * 64 + lane] = make_float2(a[j], b[j]);
+  if (WALK && chunk > 0) {   // the chunks before this one, an equal run of them a wave
+    const int run = (chunk + GRU_WAVES - 1) / GRU_WAVES, k0 = wave * run;
+    float ca[VEC], cb[VEC];
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) S[j] = chunks[j].y;
-#pragma unroll 16
-    for (int k = 1; k <= chunk; ++k)
+    for (int j = 0; j < VEC; ++j) ca[j] = 1.f, cb[j] = 0.f;
+#pragma unroll 4
+    for (int k = k0; k < min(k0 + run, chunk); ++k) {
+      float2 ab[VEC];
+      load_pairs<VEC>(chunks + (size_t)k * g.width, ab);
 #pragma unroll
       for (int j = 0; j < VEC; ++j) {
-        const float2 ab = chunks[(size_t)k * g.width + j];
-        S[j] = fmaf(ab.x, S[j], ab.y);
+        ca[j] *= ab[j].x;
+        cb[j] = fmaf(ab[j].x, cb[j], ab[j].y);
       }
+    }
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) before[wave][j * 64 + lane] = make_float2(ca[j], cb[j]);
+  }
+  if (WALK) {
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) S[j] = from[j];
   }
   __syncthreads();
   if (!WALK) {
@@ -127,18 +179,27 @@ __global__ __launch_bounds__(GRU_WAVES * 64) void min_gru_chunks_kernel(const T*
     for (int w = 1; w < GRU_WAVES; ++w)
 #pragma unroll
       for (int j = 0; j < VEC; ++j) {
-        const float2 ab = folded[w][lane * VEC + j];
+        const float2 ab = folded[w][j * 64 + lane];
         a[j] *= ab.x;
         b[j] = fmaf(ab.x, b[j], ab.y);
       }
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) chunks[(size_t)(chunk + 1) * g.width + j] = make_float2(a[j], b[j]);
+    if constexpr (VEC == 1) chunks[(size_t)chunk * g.width] = make_float2(a[0], b[0]);
+    else *reinterpret_cast<float4*>(chunks + (size_t)chunk * g.width) = make_float4(a[0], b[0], a[1], b[1]);
     return;
+  }
+  if (chunk > 0) {
+#pragma unroll
+    for (int w = 0; w < GRU_WAVES; ++w)
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        const float2 ab = before[w][j * 64 + lane];
+        S[j] = fmaf(ab.x, S[j], ab.y);
+      }
   }
   for (int w = 0; w < wave; ++w)
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
-      const float2 ab = folded[w][lane * VEC + j];
+      const float2 ab = folded[w][j * 64 + lane];
       S[j] = fmaf(ab.x, S[j], ab.y);
     }
   T* out = y + (size_t)(s.row0 + t0) * g.width + c;
@@ -195,7 +256,7 @@ static int launch_min_gru(const T* x, const bf16_t* zb, const bf16_t* xb, float*
   const bool pairs = g.width % 2 == 0 && g.stride % 2 == 0 &&
                      ((((uintptr_t)x | (uintptr_t)y) & (2 * sizeof(T) - 1)) | (((uintptr_t)zb | (uintptr_t)xb) & 3)) == 0;
   const int vec = pairs ? 2 : 1;
-  const dim3 chunks((g.width + 64 * vec - 1) / (64 * vec), (g.rows + GRU_CHUNK - 1) / GRU_CHUNK, g.slots);
+  const dim3 chunks((g.width + 64 * vec - 1) / (64 * vec), g.chunks < 65535 ? g.chunks : 65535, (g.chunks + 65534) / 65535);
   const dim3 rows((g.width + 256 * vec - 1) / (256 * vec), g.slots);
 #define IRON_GRU(VEC)                                                                                                                \
   if (work != nullptr) {                                                                                                             \
@@ -222,10 +283,10 @@ extern "C" int iron_min_gru(const void* x, const uint16_t* z_bias, const uint16_
                             void* workspace, int slots, int rows, int stride, int width, int is_float, void* stream) {
   IRON_REQUIRE(x && z_bias && x_bias && state && spans && y, "min_gru: null operand");
   IRON_REQUIRE(((uintptr_t)spans & 15) == 0 && ((uintptr_t)workspace & 15) == 0, "min_gru: spans and workspace must be 16-byte aligned");
-  IRON_REQUIRE(slots > 0 && slots <= 65535 && rows > 0 && rows <= GRU_CHUNK * 65535L, "min_gru: slots (%d) and rows (%d) must be positive",
+  IRON_REQUIRE(slots > 0 && slots <= 65535 && rows > 0 && rows <= 128 * 65535L, "min_gru: slots (%d) and rows (%d) must be positive",
                slots, rows);
   IRON_REQUIRE(width > 0 && 3L * width <= stride, "min_gru: a row of %d holds no three projections of %d", stride, width);
-  const GruShape g{slots, rows, stride, width};
+  const GruShape g{slots, rows, stride, width, (int)chunks_of(rows, slots, GRU_CHUNK)};
   hipStream_t s = (hipStream_t)stream;
   if (is_float)
     return launch_min_gru<float>((const float*)x, z_bias, x_bias, state, spans, (float*)y, (float2*)workspace, g, s);

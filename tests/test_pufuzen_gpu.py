@@ -106,6 +106,20 @@ def test_a_gated_recurrence(cuda, dtype, chunked, width, stride):
     agrees(op, gru_inputs(rng, op, spans), 3e-6 if dtype is F32 else 5e-3, rows_of(spans), workspace=chunked)
 
 
+@BOTH
+@pytest.mark.parametrize("width,slots", [(258, 70), (33, 9)])
+def test_a_gated_recurrence_s_chunks(cuda, dtype, width, slots):
+    """Whole chunks, one token more, and more chunks than a block has waves; slots past a wave's lanes, most of them idle."""
+    rng = np.random.default_rng(slots)
+    lengths, at, spans = (64, 65, 128, 330, 1, 257), 3, []
+    for i, (slot, n) in enumerate(zip(rng.permutation(slots), lengths)):
+        spans.append((int(slot), at, n, (0, 7, 128)[i % 3]))
+        at += n + i % 2
+    spans = table(*spans, slots=slots)
+    op = MinGRU(slots=slots, rows=at + 2, stride=3 * width + 5, width=width, dtype=dtype)
+    agrees(op, gru_inputs(rng, op, spans), 3e-6 if dtype is F32 else 5e-3, rows_of(spans), workspace=True)
+
+
 @pytest.mark.parametrize("chunked", [False, True], ids=["tokens", "chunks"])
 def test_the_recurrence_goes_on_where_a_portion_ends(cuda, chunked):
     rng = np.random.default_rng(7)
