@@ -538,11 +538,11 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(const T* __restrict_
   if constexpr (AHEAD > 0) {
 #pragma unroll
     for (int i = 0; i < AHEAD; ++i) {
+      if (group + 16 * i >= a.dim) break;
       float f[8];
       unpack8(ahead[i], f);
-      const float q_at = group + 16 * i < a.dim ? x[i] : 0.f;   // (past the last: a finite weight of the last row)
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) acc[j] = fmaf(q_at, f[j], acc[j]);
+      for (int j = 0; j < VEC; ++j) acc[j] = fmaf(x[i], f[j], acc[j]);
     }
   }
 #pragma unroll 4
