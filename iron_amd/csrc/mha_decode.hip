@@ -41,6 +41,7 @@ __device__ __forceinline__ float across_rows(float x, F f) {
 }
 
 typedef __bf16 bf16x2_v __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 // The dot product of two 16-byte runs of bf16.
 __device__ __forceinline__ float dot8(const uint4& a, const uint4& b) {
   float d = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_v, a.x), __builtin_bit_cast(bf16x2_v, b.x), 0.f, false);
@@ -354,8 +355,8 @@ __global__ __launch_bounds__(1024) void mha_decode_single_kernel(
 // they go from global memory straight into registers.  A lane then owns one head column: the softmax
 // is in-lane but for the maximum over the four lanes of a column, which is only exchanged on the
 // (rare) steps where some lane's own maximum passes the column's reference.  The probabilities,
-// in two bf16 terms (their distance from 64 bits is then that of the form that keeps them in 32; rounded to one, 2000 to 16384 keys
-// were 1.06 to 1.09 times as far off), are already the B operand of O^T = V^T P^T; V^T comes from the transposing LDS read
+// in three bf16 terms (all 24 bits of them: 385 to 1408 keys are then 1.66593e-3 from 64 bits as the form that keeps them in 32 is, by two terms
+// 1.665933e-3 against 1.665929e-3; rounded to one, 1500 to 12000 keys were up to 1.22 times as far off), are already the B operand of O^T = V^T P^T; V^T comes from the transposing LDS read
 // of the wave's own 32-row V tile, which buffer loads put there as stored (16-byte chunks
 // XOR-swizzled by 2 (row & 3), as the prompt kernel's).  Rows past the last live key lie outside the
 // buffers and read as zeros.
@@ -363,7 +364,7 @@ __global__ __launch_bounds__(1024) void mha_decode_single_kernel(
 // At a few thousand keys the launch is as long as its instructions, which the waves of a SIMD take in turn, so there
 // are eight a block and not sixteen, and nothing of a block's shape is a variable.  32 / 8 heads of 64 with the merge, us: runs of whole steps of
 // sixteen waves a block, then of eight, then keys in turn: 1420 keys 8.65 / 6.55 / 6.4, 4000 8.75 / 7.4 / 7.3, 8000 9.65 / 8.8 / 8.55, 12003
-// 11.9 / 11.0 / 10.2, 16300 13.4 / 12.9 / 12.0 (the second term of the probabilities 0.05 to 0.1 more).
+// 11.9 / 11.0 / 10.2, 16300 13.4 / 12.9 / 12.0 (the second term of the probabilities 0.05 to 0.1 more, the third another 0.1).
 template <int D, int HPB_LOG2>
 __global__ __launch_bounds__(64 * EITHER_WAVES) void mha_decode_either_kernel(
     const bf16_t* __restrict__ Q, const bf16_t* __restrict__ K, const bf16_t* __restrict__ V,
@@ -573,23 +574,33 @@ __global__ __launch_bounds__(64 * EITHER_WAVES) void mha_decode_either_kernel(
         p[4 * t + i] = e;
         l_run += e;
       }
-    // The weights as two bf16 terms, together within 2^-17: the matrix cores idle.  The first is cut off and 2^-20 of the weight
-    // joins the second, so that both are positive and an infinite value stays what it is.
-    uint32_t high[4];
-    float rest[8];
+    // The weights as three bf16 terms of eight bits each, cut off one after the other: all 24 bits of them (the matrix cores idle).  No term is
+    // negative, and one that is zero is the smallest there is, so that an infinite value stays what it is.
+    uint32_t term[3][4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) rest[i] = fmaf(p[i], 1.f + 0x1p-20f, -__uint_as_float(__float_as_uint(p[i]) & 0xffff0000u));
+    for (int i = 0; i < 4; ++i) {
+      float a = p[2 * i], b = p[2 * i + 1];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) high[i] = (__float_as_uint(p[2 * i]) >> 16) | (__float_as_uint(p[2 * i + 1]) & 0xffff0000u);
-    const bf16x8 pf = __builtin_bit_cast(bf16x8, make_uint4(high[0], high[1], high[2], high[3])), pr = __builtin_bit_cast(bf16x8, pack8(rest));
+      for (int k = 0; k < 3; ++k) {
+        term[k][i] = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302);   // both high halves
+        a -= __uint_as_float(__float_as_uint(a) & 0xffff0000u);
+        b -= __uint_as_float(__float_as_uint(b) & 0xffff0000u);
+      }
+#pragma unroll
+      for (int k = 1; k < 3; ++k)
+        term[k][i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, term[k][i]), u16x2{0x0080, 0x0080}));
+    }
+    bf16x8 pf[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) pf[k] = __builtin_bit_cast(bf16x8, make_uint4(term[k][0], term[k][1], term[k][2], term[k][3]));
 #pragma unroll
     for (int dt = 0; dt < DT; dt += 2) {
       lds_tr_wait(vf[dt], vf[dt + 1]);
 #pragma unroll
       for (int e = dt; e < dt + 2; ++e) {
         const bf16x8 v = tr_join(vf[e]);
-        oacc[e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pf, oacc[e], 0, 0, 0);
-        oacc[e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pr, oacc[e], 0, 0, 0);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) oacc[e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pf[k], oacc[e], 0, 0, 0);
       }
     }
   };

@@ -1986,7 +1986,7 @@ def test_decode_attention_takes_keys_in_turn(cuda, H, G, d, window):
         kd, vd = k[lo:n].double(), v[lo:n].double()
         p = torch.softmax(torch.einsum("ghd,kgd->ghk", q.double().reshape(G, H // G, d), kd) / d**0.5, -1)
         want = torch.einsum("ghk,kgd->ghd", p, vd).reshape(H, d)
-        # the output's rounding; weights within 2^-17 of themselves, and scores' sums and exponentials in 32 bits
+        # the output's rounding; weights, scores' sums and exponentials in 32 bits
         assert ((o.double() - want).abs() <= 2**-8 * want.abs() + 2**-12 * vd.abs().max()).all(), n
         if n == 2049:   # an infinite value is the output where its key weighs anything
             v[1500, 0, 3] = float("inf")
@@ -1994,3 +1994,33 @@ def test_decode_attention_takes_keys_in_turn(cuda, H, G, d, window):
                          window=window, workspace=workspace)
             assert torch.isinf(o[: H // G, 3]).all()
             v[1500, 0, 3] = 0.0
+
+
+@pytest.mark.parametrize("d,n", [(64, 600), (64, 1400), (64, 5000), (128, 500), (128, 3000)])
+def test_decode_attention_s_weights_have_32_bits(cuda, d, n):
+    """Two values that cancel to their last bits, so that an output is what its weights were rounded by; and an infinite value behind a tiny weight."""
+    H, L, q0 = 8, 8200, np.float32(2 * d**0.5)
+    rng = np.random.default_rng(n)
+    score = -round_bf16(np.linspace(0.3, 4.7, H, dtype=np.float32))   # a head's every second key; the others have 0
+    weight = np.exp(score.astype(np.float64) * 2)
+    top = round_bf16(rng.uniform(1, 2, (H, d)).astype(np.float32))
+    q, k, v = np.zeros((1, H, d), np.float32), np.zeros((L, H, d), np.float32), np.zeros((L, H, d), np.float32)
+    q[..., 0] = q0 if d == 64 else round_bf16(q0)
+    k[1::2, :, 0], v[0::2], v[1::2] = score, top, -round_bf16((top / weight[:, None]).astype(np.float32))
+    scale = 2 / float(q[0, 0, 0])
+    n0, n1 = (n + 1) // 2, n // 2
+    sums = n0 + n1 * weight[:, None]
+    want = (n0 * top.astype(np.float64) + n1 * weight[:, None] * v[1]) / sums
+    size = (n0 * top + n1 * weight[:, None] * np.abs(v[1])) / sums
+    assert (np.abs(want) < 2**-13 * size).sum() > 2   # (elements that the output's own rounding hides nothing of)
+    o, workspace = torch.empty(H, d, dtype=torch.bfloat16, device="cuda"), K.mha_decode_workspace(H, d)
+    q, k, v = dev(q, cuda), dev(k, cuda), dev(v, cuda)
+
+    def run():
+        K.mha_decode(q, k, v, o, heads=H, kv_heads=H, d=d, kv_len=L, scale=scale, kv_interleaved=True, kv_valid=word(n, cuda), workspace=workspace)
+        return from_torch(o).astype(np.float64)
+
+    # the output's rounding; a weight's (its score's product with log2 e and its exponential, some 2^-22) and the sums'
+    assert (np.abs(run() - want) <= 2**-8 * np.abs(want) + 2**-20 * size).all()
+    k[33, :, 0], v[33, :, 1] = -43.25, float("inf")   # e^-86.5, which is still no denormal
+    assert np.isposinf(run()[:, 1]).all()
