@@ -25,6 +25,7 @@ constexpr int kSingleMaxKeys = 2048;  // lane-scan kernels: caches up to this ma
 constexpr int short_keys_of(int d) { return d == 64 ? 512 : 384; }
 constexpr int kComputeUnits = 256;    // MI355X: what the split count is sized for
 constexpr int EITHER_WAVES = 8;       // waves a block of the one-shape launch
+constexpr int EITHER_KEYS = 32;       // keys a wave of it takes at a time
 
 // 2^x for x <= 0 by the hardware's own instruction: a softmax weight small enough to be a denormal
 // counts as 0, which saves the library routine's rescaling around every call.
@@ -337,6 +338,9 @@ __global__ __launch_bounds__(1024) void mha_decode_single_kernel(
   }
 }
 
+// Whether a split of the one-shape launch holds any of the `live` keys: the scan's blocks that do not leave at once, and the merge reads none of theirs.
+__device__ __forceinline__ bool split_holds(int split, int live) { return split * EITHER_KEYS < live; }
+
 // ---- one query, one launch shape whatever the cache's length
 //
 // grid = (sets, nsplit) blocks of eight waves, as many as the chip has CUs; the blocks choose what to
@@ -375,7 +379,7 @@ __global__ __launch_bounds__(64 * EITHER_WAVES) void mha_decode_either_kernel(
   constexpr int KS = D / 32;             // 32-wide k-steps of S^T
   constexpr int DT = D / 16;             // 16-row tiles of O^T
   constexpr int CPR = D / 8;             // 16-byte chunks of a row
-  constexpr int TK = 32;                 // keys a step
+  constexpr int TK = EITHER_KEYS;        // keys a step
   constexpr int TILE = TK * ROWB;        // bytes of a V tile
   constexpr int VINST = TILE / 1024;     // 1 KB loads into LDS a tile
   constexpr int RPI = 1024 / ROWB;       // rows one of them covers
@@ -438,7 +442,7 @@ __global__ __launch_bounds__(64 * EITHER_WAVES) void mha_decode_either_kernel(
   const int split = blockIdx.y;
   const int kvh = (blockIdx.x << HPB_LOG2) + (wave & (HPB - 1));
   const int sub = wave >> HPB_LOG2;          // this wave's place among the SHARE on its head
-  if (split * TK >= live) return;   // the merge reads the splits that hold keys, no more
+  if (!split_holds(split, live)) return;
   // The wave's steps, SHARE * nsplit tiles of keys apart.
   const int k_first = first + (sub * nsplit + split) * TK, k_step = SHARE * nsplit * TK;
   auto has = [=](int step) { return k_first + step * k_step < kv_tokens; };
@@ -675,10 +679,10 @@ __global__ __launch_bounds__(64 * EITHER_WAVES) void mha_decode_either_kernel(
 }
 
 // The splits' merge, a block of 4 D threads a head: thread (part, pair) sums columns 2 pair and
-// 2 pair + 1 over the splits part, part + 8, ... that hold keys, PER of them at a time, and the eight
-// parts are folded through LDS.  A thread's first PER are requested together with the bound, before
+// 2 pair + 1 over the splits part, part + 8, ... that hold keys, at most PER of them, and the eight
+// parts are folded through LDS.  They are requested together with the bound, before
 // it is known how many of them hold anything (the workspace is the caller's own memory, whatever it
-// holds): one trip to memory, not two, for up to 8 PER splits (PER = 8 where the launch has at most
+// holds): one trip to memory, not two (PER = 8 where the launch has at most
 // 64 splits, so that no thread asks twice for a split).  Every load is 8 bytes -- a split's maximum
 // and sum, or two columns: the launch's time is its load instructions (one column and one word a
 // load took 1.3 us longer at 64 splits).  Leaves at once where the scan's blocks wrote the output
@@ -701,34 +705,18 @@ __global__ __launch_bounds__(4 * D) void mha_decode_either_merge_kernel(
   const int first = (window >= 0) ? max(0, kv_tokens - 1 - window) : 0;
   const int live = kv_tokens - first;
   if (live <= short_keys) return;
-  auto used = [=](int split) { return split < nsplit && split * 32 < live; };
+  auto used = [=](int i) { return eighth + 8 * i < nsplit && split_holds(eighth + 8 * i, live); };
   float mx = -INFINITY, lt = 0.f, at0 = 0.f, at1 = 0.f;
-  for (int s0 = eighth; used(s0); s0 += 8 * PER) {
-    if (s0 >= 8 * PER) {
 #pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int s = min(s0 + 8 * i, nsplit - 1);
-        ml[i] = *reinterpret_cast<const float2*>(p + s * (D + 2));
-        a[i] = *reinterpret_cast<const float2*>(p + s * (D + 2) + 2 + 2 * t);
-      }
-    }
-    float cm = mx;
+  for (int i = 0; i < PER; ++i)
+    if (used(i)) mx = fmaxf(mx, ml[i].x);
 #pragma unroll
-    for (int i = 0; i < PER; ++i)
-      if (used(s0 + 8 * i)) cm = fmaxf(cm, ml[i].x);
-    const float keep = (mx == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mx - cm);
-    lt *= keep;
-    at0 *= keep;
-    at1 *= keep;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const bool in = used(s0 + 8 * i) && ml[i].x != -INFINITY;
-      const float e = in ? __builtin_amdgcn_exp2f(ml[i].x - cm) : 0.f;
-      lt = fmaf(in ? ml[i].y : 0.f, e, lt);
-      at0 = fmaf(in ? a[i].x : 0.f, e, at0);
-      at1 = fmaf(in ? a[i].y : 0.f, e, at1);
-    }
-    mx = cm;
+  for (int i = 0; i < PER; ++i) {
+    const bool in = used(i) && ml[i].x != -INFINITY;
+    const float e = in ? __builtin_amdgcn_exp2f(ml[i].x - mx) : 0.f;
+    lt = fmaf(in ? ml[i].y : 0.f, e, lt);
+    at0 = fmaf(in ? a[i].x : 0.f, e, at0);
+    at1 = fmaf(in ? a[i].y : 0.f, e, at1);
   }
   __shared__ float fm[8][PAIRS], fl[8][PAIRS];
   __shared__ float2 fa[8][PAIRS];
@@ -791,6 +779,7 @@ static int launch_decode_either(const bf16_t* Q, const bf16_t* K, const bf16_t* 
   hipLaunchKernelGGL((mha_decode_either_kernel<D, HPB_LOG2>), dim3(sets, nsplit), dim3(64 * EITHER_WAVES), lds, s, Q, K, V, O,
                      part, kv_heads, group, kv_len, scale_log2, window, row_stride, head_stride, kv_valid,
                      kv_first, kv_rows, short_keys);
+  static_assert(kMaxSplits <= 8 * 16, "a thread of the merge has its splits at once");
   if (nsplit <= 64)
     hipLaunchKernelGGL((mha_decode_either_merge_kernel<D, 8>), dim3(kv_heads * group), dim3(4 * D), 0, s, part, O,
                        nsplit, kv_len, window, kv_valid, short_keys);
