@@ -338,8 +338,23 @@ __global__ __launch_bounds__(1024) void mha_decode_single_kernel(
   }
 }
 
-// Whether a split of the one-shape launch holds any of the `live` keys: the scan's blocks that do not leave at once, and the merge reads none of theirs.
-__device__ __forceinline__ bool split_holds(int split, int live) { return split * EITHER_KEYS < live; }
+// How the one-shape launch's split scan deals the live keys.  In turn, 32 at a time: the splits' first waves one after the other, then their second ones, and
+// round again.  Where a head's rows lie one behind the other (`run`: waves a head and split; else 0) and the live ones fill the same number of steps of every wave to five
+// sixths, heads of 128 have them in runs, of `steps` steps a wave, the splits' and their waves' side by side: in turn all waves read a power of two apart there.  32 / 8 heads,
+// 16384 rows a head, us in turn and in runs: 7200 keys 13.5 / 12.3, 8000 14.3 / 12.7, 16300 20.9 / 18.9; 16 / 16 heads, 12003 keys 26.1 / 23.1.  But less filled: 32 / 8
+// heads, 3000 keys 9.85 / 10.7, 6000 12.0 / 12.0, 16 / 16 heads, 5000 13.9 / 16.7; heads of 64: 16 / 16, 8000 12.1 / 14.0; rows of all heads together: 32 / 8 of 128, 8000
+// 12.5 / 13.5.  `inverse`: of a round's keys.
+struct Deal {
+  int per_split, steps;   // keys from a split's first to the next one's (a split whose first is not live holds none); steps a wave at most
+};
+template <int D>
+__device__ __forceinline__ Deal deal_keys(int nsplit, int live, int run, unsigned inverse) {
+  if (D == 128 && run > 0) {
+    const int steps = (int)__umulhi((unsigned)(live - 1), inverse) + 1, all = steps * nsplit * run * EITHER_KEYS;
+    if (live >= all - all / 6) return Deal{steps * run * EITHER_KEYS, steps};
+  }
+  return Deal{EITHER_KEYS, 0x7fffffff};
+}
 
 // ---- one query, one launch shape whatever the cache's length
 //
@@ -350,8 +365,8 @@ __device__ __forceinline__ bool split_holds(int split, int live) { return split 
 // n <= short_keys: the first `heads` blocks each scan all keys for one query head with the
 // lane-per-column scan above and write the output row; the others leave at once, and so does the merge launch behind.
 //
-// Otherwise the keys are dealt over the nsplit blocks of a set of KV heads, 32 at a time in turn -- all blocks
-// together read one run of them at a time, and no wave has two steps more than another --
+// Otherwise the keys are dealt over the nsplit blocks of a set of KV heads, 32 at a time (deal_keys) -- no wave has two
+// steps more than another --
 // and a block leaves (max, sum, O) per head for the merge.  Here the G query heads that share a KV
 // head are the columns of a 16-wide MFMA tile (G <= 16; the rest are zero columns), so a key row is
 // multiplied with all of them by one instruction stream whatever G is.  S^T = K Q^T (M = keys, N = heads): the K rows are the A operand exactly
@@ -374,7 +389,7 @@ __global__ __launch_bounds__(64 * EITHER_WAVES) void mha_decode_either_kernel(
     const bf16_t* __restrict__ Q, const bf16_t* __restrict__ K, const bf16_t* __restrict__ V,
     bf16_t* __restrict__ O, float* __restrict__ part, int kv_heads, int group, int kv_len,
     float scale_log2, int window, long row_stride, long head_stride, const int* __restrict__ kv_valid,
-    const int* __restrict__ kv_first, int kv_rows, int short_keys) {
+    const int* __restrict__ kv_first, int kv_rows, int short_keys, int run, unsigned run_inverse) {
   constexpr int ROWB = D * 2;            // bytes of a V row in LDS
   constexpr int KS = D / 32;             // 32-wide k-steps of S^T
   constexpr int DT = D / 16;             // 16-row tiles of O^T
@@ -442,10 +457,14 @@ __global__ __launch_bounds__(64 * EITHER_WAVES) void mha_decode_either_kernel(
   const int split = blockIdx.y;
   const int kvh = (blockIdx.x << HPB_LOG2) + (wave & (HPB - 1));
   const int sub = wave >> HPB_LOG2;          // this wave's place among the SHARE on its head
-  if (!split_holds(split, live)) return;
-  // The wave's steps, SHARE * nsplit tiles of keys apart.
-  const int k_first = first + (sub * nsplit + split) * TK, k_step = SHARE * nsplit * TK;
-  auto has = [=](int step) { return k_first + step * k_step < kv_tokens; };
+  const Deal deal = deal_keys<D>(nsplit, live, run, run_inverse);
+  if (split * deal.per_split >= live) return;
+  // (a block's own waves are kept from being a power of two apart, where there are splits enough: 32 / 8 heads of 64, 16384 rows a head, 8000 keys 9.95 -> 9.15 us)
+  const bool runs = deal.per_split > TK;
+  const int place = split + (run > 0 && nsplit >= 64 ? 5 * sub : 0);
+  const int k_first = first + (runs ? split * deal.per_split + sub * deal.steps * TK : (sub * nsplit + (place < nsplit ? place : place - nsplit)) * TK);
+  const int k_step = runs ? TK : SHARE * nsplit * TK;
+  auto has = [=](int step) { return step < deal.steps && k_first + step * k_step < kv_tokens; };
 
   const bf16_t* Kh = K + (size_t)kvh * head_stride + first_row * row_stride;
   const bf16_t* Vh = V + (size_t)kvh * head_stride + first_row * row_stride;
@@ -690,7 +709,7 @@ __global__ __launch_bounds__(64 * EITHER_WAVES) void mha_decode_either_kernel(
 template <int D, int PER>
 __global__ __launch_bounds__(4 * D) void mha_decode_either_merge_kernel(
     const float* __restrict__ part, bf16_t* __restrict__ O, int nsplit, int kv_len, int window,
-    const int* __restrict__ kv_valid, int short_keys) {
+    const int* __restrict__ kv_valid, int short_keys, int run, unsigned run_inverse) {
   constexpr int PAIRS = D / 2;
   const int head = blockIdx.x, t = threadIdx.x % PAIRS, eighth = threadIdx.x / PAIRS;
   const float* p = part + (size_t)head * nsplit * (D + 2);
@@ -705,7 +724,8 @@ __global__ __launch_bounds__(4 * D) void mha_decode_either_merge_kernel(
   const int first = (window >= 0) ? max(0, kv_tokens - 1 - window) : 0;
   const int live = kv_tokens - first;
   if (live <= short_keys) return;
-  auto used = [=](int i) { return eighth + 8 * i < nsplit && split_holds(eighth + 8 * i, live); };
+  const int per_split = deal_keys<D>(nsplit, live, run, run_inverse).per_split;
+  auto used = [=](int i) { return eighth + 8 * i < nsplit && (eighth + 8 * i) * per_split < live; };
   float mx = -INFINITY, lt = 0.f, at0 = 0.f, at1 = 0.f;
 #pragma unroll
   for (int i = 0; i < PER; ++i)
@@ -776,16 +796,19 @@ static int launch_decode_either(const bf16_t* Q, const bf16_t* K, const bf16_t* 
   int nsplit = kComputeUnits / sets;
   while (sets * nsplit < kv_heads * group) ++nsplit;
   nsplit = nsplit < 1 ? 1 : (nsplit > kMaxSplits ? kMaxSplits : nsplit);
+  const int run = row_stride == D ? EITHER_WAVES >> HPB_LOG2 : 0;
+  static_assert(5 * (EITHER_WAVES - 1) < 64, "a wave's place in turn wraps once");
+  const unsigned inverse = run > 0 ? (unsigned)((1ull << 32) / (unsigned)(nsplit * run * EITHER_KEYS) + 1) : 0;
   hipLaunchKernelGGL((mha_decode_either_kernel<D, HPB_LOG2>), dim3(sets, nsplit), dim3(64 * EITHER_WAVES), lds, s, Q, K, V, O,
                      part, kv_heads, group, kv_len, scale_log2, window, row_stride, head_stride, kv_valid,
-                     kv_first, kv_rows, short_keys);
+                     kv_first, kv_rows, short_keys, run, inverse);
   static_assert(kMaxSplits <= 8 * 16, "a thread of the merge has its splits at once");
   if (nsplit <= 64)
     hipLaunchKernelGGL((mha_decode_either_merge_kernel<D, 8>), dim3(kv_heads * group), dim3(4 * D), 0, s, part, O,
-                       nsplit, kv_len, window, kv_valid, short_keys);
+                       nsplit, kv_len, window, kv_valid, short_keys, run, inverse);
   else
     hipLaunchKernelGGL((mha_decode_either_merge_kernel<D, 16>), dim3(kv_heads * group), dim3(4 * D), 0, s, part, O,
-                       nsplit, kv_len, window, kv_valid, short_keys);
+                       nsplit, kv_len, window, kv_valid, short_keys, run, inverse);
   return 0;
 }
 

@@ -2024,3 +2024,27 @@ def test_decode_attention_s_weights_have_32_bits(cuda, d, n):
     assert (np.abs(run() - want) <= 2**-8 * np.abs(want) + 2**-20 * size).all()
     k[33, :, 0], v[33, :, 1] = -43.25, float("inf")   # e^-86.5, which is still no denormal
     assert np.isposinf(run()[:, 1]).all()
+
+
+# A head's rows one behind the other: a round of all waves filled to either side of five sixths, from where heads of 128 have their keys in runs; runs' and splits' edges, a round
+# and one key more, two rounds, and a window of them; heads two a block and one, splits of which a wave's place wraps.
+@pytest.mark.parametrize("H,G,d,window,round_", [(32, 8, 64, None, 8192), (8, 8, 128, None, 8192), (32, 16, 128, None, 4096), (6, 3, 128, None, 85 * 256),
+                                                 (4, 1, 128, None, 32768), (8, 8, 128, 6900, 8192)])
+def test_decode_attention_over_rows_of_a_head(cuda, H, G, d, window, round_):
+    line = round_ - round_ // 6
+    L = 2 * round_ + 700
+    g = torch.Generator(device="cuda")
+    g.manual_seed(d)
+    q, k, v = (torch.randn(*n, d, generator=g, device="cuda").to(torch.bfloat16) for n in ((H,), (G, L), (G, L)))
+    q *= 2
+    o, workspace = torch.empty(H, d, dtype=torch.bfloat16, device="cuda"), K.mha_decode_workspace(H, d)
+    for n in (2049, line - 1, line, line + 1, line + 33, line + 129, round_ - 31, round_, round_ + 1, 2 * line - 1, 2 * round_ - 33, 2 * round_ + 500):
+        past = k[:, n:].clone()
+        k[:, n:] = float("nan")   # (what lies past the live keys is nobody's)
+        workspace.fill_(float("nan"))
+        K.mha_decode(q, k, v, o, heads=H, kv_heads=G, d=d, kv_len=L, kv_valid=word(n, cuda), window=window, workspace=workspace)
+        k[:, n:] = past
+        lo = 0 if window is None else max(0, n - 1 - window)
+        p = torch.softmax((q.double().reshape(G, H // G, d) @ k[:, lo:n].double().transpose(1, 2).contiguous()) / d**0.5, -1)
+        want = (p @ v[:, lo:n].double()).reshape(H, d)
+        assert ((o.double() - want).abs() <= 2**-8 * want.abs() + 2**-12 * v.double().abs().max()).all(), n
