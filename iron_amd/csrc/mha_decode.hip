@@ -19,10 +19,15 @@ namespace iron {
 constexpr int kMaxSplits = 128;      // what the workspace holds per head
 constexpr int kScanMaxSplits = 128;  // the lane-scan kernels' own limit
 constexpr int kSingleMaxKeys = 2048;  // lane-scan kernels: caches up to this many rows take the one-launch kernel
-// One-shape launch: up to this many live keys one block a query head writes O itself.  Where the two
-// forms cost the same inside that launch shape (an 8192-row cache, us, one block a head / split + merge: 32 / 8 heads
-// of 64, 400 live keys 5.8 / 6.0, 500 5.9 / 6.1, 600 6.5 / 6.3, 1000 8.1 / 6.45; of 128, 300 6.4 / 7.2, 400 7.4 / 7.3, 600 8.1 / 7.4).
-constexpr int short_keys_of(int d) { return d == 64 ? 512 : 384; }
+// One-shape launch: up to this many live keys one block a query head writes O itself.  The line lies where the two
+// forms cost the same inside that launch shape, which is the later, the more columns the waves hand over and the more heads the merge has (an 8192-row cache, us, one block
+// a head / split + merge: 32 / 8 heads of 64, 512 live keys 6.3 / 6.7, 576 6.65 / 6.7, 640 6.95 / 6.75, 1000 8.2 / 6.9; 128 / 8 of 64, 640 7.0 / 7.3, 768 7.6 / 7.35;
+// 32 / 8 of 128, 384 7.2 / 7.85, 448 7.85 / 7.85, 640 8.75 / 8.0; 64 / 8 of 128, 512 8.05 / 8.35, 576 8.45 / 8.35; 128 / 8 of 128, 640 8.95 / 9.2, 768 9.8 / 9.35), and
+// with two heads a block and past sixteen of them a split has its second step (32 / 32 of 128, 512 8.35 / 8.2, 576 8.8 / 8.9, 640 9.2 / 9.0).
+constexpr int short_keys_of(int d, int group, int kv_heads) {
+  if (d == 64) return group > 8 ? 704 : 576;
+  return (group > 8 ? 736 : (group > 4 ? 544 : 448)) + (kv_heads > 16 ? 224 : 0);
+}
 constexpr int kComputeUnits = 256;    // MI355X: what the split count is sized for
 constexpr int EITHER_WAVES = 8;       // waves a block of the one-shape launch
 constexpr int EITHER_KEYS = 32;       // keys a wave of it takes at a time
@@ -855,7 +860,7 @@ static int mha_decode(const uint16_t* Q, const uint16_t* K, const uint16_t* V, u
                            (long)kv_len * row_stride * 2 < (1L << 31) && heads <= kMaxSplits * kv_heads;
   IRON_REQUIRE(form != 2 || either_fits,
                "mha_decode: the one-shape launch takes d = 64 or 128, up to 16 query heads a KV head and keys within 2^31 bytes");
-  const int upto = short_keys > 0 ? short_keys : short_keys_of(d);
+  const int upto = short_keys > 0 ? short_keys : short_keys_of(d, G, kv_heads);
   if (form == 2 || (form == 0 && either_fits && kv_len > (short_keys > 0 ? short_keys : kSingleMaxKeys))) {
     // A block of the split scan serves two KV heads where their number is even (with the heads
     // interleaved in a cache row its loads then cover 256-byte pieces: measured a tenth faster than one

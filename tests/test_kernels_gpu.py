@@ -1976,7 +1976,7 @@ def test_decode_attention_takes_keys_in_turn(cuda, H, G, d, window):
     q, k, v = (torch.randn(n, w, d, generator=g, device="cuda").to(torch.bfloat16) for n, w in ((1, H), (L, G), (L, G)))
     q *= 2
     o, workspace = torch.empty(H, d, dtype=torch.bfloat16, device="cuda"), K.mha_decode_workspace(H, d)
-    for n in (384, 385, 512, 513, 544, 545, 1408, 2047, 2049, 2080, 4097, 8192, 8193, 8200, int(rng.integers(600, 8000))):
+    for n in (384, 385, 448, 449, 512, 513, 544, 545, 576, 577, 704, 705, 736, 737, 1408, 2047, 2049, 2080, 4097, 8192, 8193, 8200, int(rng.integers(600, 8000))):
         past = k[n:].clone()
         k[n:] = float("nan")   # (what lies past the live keys is nobody's)
         K.mha_decode(q, k, v, o, heads=H, kv_heads=G, d=d, kv_len=L, kv_interleaved=True, kv_valid=torch.tensor([n], dtype=torch.int32, device="cuda"),
