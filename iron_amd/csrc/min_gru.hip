@@ -12,17 +12,18 @@
 // portion's first state is put beside its chunks, since the block of its last chunk may replace it: a slot has two states,
 // position p's in row p % 2, so that a decode step's blocks leave the one they all read.
 //
-// Four quarter-rate instructions an element bound the first launch and six the second, so what counts is that they are spread: blocks of four
-// waves (of eight, 296 blocks of a ragged batch are two on some CUs and one on the rest), and a grid of the spans' chunks one after
-// the other, where that of every slot's every chunk dealt out eight times the blocks and looked through the spans for each.  2048 channels, us:
-// eight spans of 256 rows 25.6 -> 18.5, of 96 to 422 23.3 -> 19.4, of 90 to 140 18.9 -> 14.3, four of 90 to 500 19.2 -> 13.5, one of 2048 19.5 -> 18.6, of 300
-// 12.8 -> 10.9.  (Four channels a lane and eight tokens a wave: 18.6, 20.5, 14.0, 14.4, 21.2, 11.0.)
+// Four quarter-rate instructions an element bound the first launch and six the second, a wave's one after the other where there are few rows, so what
+// counts is that they are spread: eight tokens a wave and eight waves a chunk, and a grid of the spans' chunks one after
+// the other (that of every slot's every chunk dealt out eight times the blocks), which a wave's lanes look up 64 slots at a time.  2048 channels, us, with chunks of 128
+// by eight waves in that wider grid, of 64 by four and so: one span of 64 8.5 / 7.9 / 7.1, of 65 8.45 / 9.85 / 8.55, of 100 8.8 / 10.1 / 8.55, of 300 12.2 / 10.4 / 9.0,
+// of 2048 19.5 / 18.2 / 16.1; four of 30 to 500 17.0 / 12.2 / 10.8, eight of 256 24.8 / 17.9 / 15.9, of 96 to 422 23.1 / 19.1 / 17.7, of 1000 50.5 / 46.0 / 43.7; forty of
+// 100 68.8 / 32.0 / 26.3 (37.6 where a wave looks from slot to slot).
 #include "../../include/iron_hip.h"
 #include "rows.h"
 
 namespace iron {
 
-constexpr int GRU_WAVES = 4, GRU_TOKENS = 16, GRU_CHUNK = GRU_WAVES * GRU_TOKENS;
+constexpr int GRU_WAVES = 8, GRU_TOKENS = 8, GRU_CHUNK = GRU_WAVES * GRU_TOKENS;
 
 // Two neighbouring elements, or one.
 template <int VEC, typename T>
@@ -74,14 +75,20 @@ __device__ __forceinline__ GruChunk gru_chunk(const int* __restrict__ spans, con
   for (int base = 0, before = 0; base < g.slots; base += 64) {
     const Span mine = span_of(spans, min(base + lane, g.slots - 1), g.rows);
     const int count = base + lane < g.slots ? (mine.rows + GRU_CHUNK - 1) / GRU_CHUNK : 0;
-    for (unsigned long long live = __builtin_amdgcn_ballot_w64(count > 0); live != 0; live &= live - 1) {
-      const int at = __builtin_ctzll(live), here = __builtin_amdgcn_readlane(count, at);
-      if (index < before + here) {
-        const Span s{__builtin_amdgcn_readlane(mine.row0, at), __builtin_amdgcn_readlane(mine.rows, at), __builtin_amdgcn_readlane(mine.start, at)};
-        return GruChunk{base + at, index - before, s};
-      }
-      before += here;
+    int upto = count;   // chunks of the lanes up to this one
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x111, 0xF, 0xF, false);   // row_shr:1, 2, 4, 8
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x112, 0xF, 0xF, false);
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x114, 0xF, 0xF, false);
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x118, 0xF, 0xF, false);
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x142, 0xA, 0xF, false);   // row_bcast15 into rows 1 and 3
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x143, 0xC, 0xF, false);   // row_bcast31 into rows 2 and 3
+    const unsigned long long past = __builtin_amdgcn_ballot_w64(before + upto > index);
+    if (past != 0) {
+      const int at = __builtin_ctzll(past);
+      const Span s{__builtin_amdgcn_readlane(mine.row0, at), __builtin_amdgcn_readlane(mine.rows, at), __builtin_amdgcn_readlane(mine.start, at)};
+      return GruChunk{base + at, index - before - __builtin_amdgcn_readlane(upto - count, at), s};
     }
+    before += __builtin_amdgcn_readlane(upto, 63);
   }
   return GruChunk{-1, 0, Span{0, 0, 0}};
 }

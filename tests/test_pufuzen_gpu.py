@@ -111,13 +111,26 @@ def test_a_gated_recurrence(cuda, dtype, chunked, width, stride):
 def test_a_gated_recurrence_s_chunks(cuda, dtype, width, slots):
     """Whole chunks, one token more, and more chunks than a block has waves; slots past a wave's lanes, most of them idle."""
     rng = np.random.default_rng(slots)
-    lengths, at, spans = (64, 65, 128, 330, 1, 257), 3, []
+    lengths, at, spans = (64, 65, 128, 330, 1, 257, 1100), 3, []
     for i, (slot, n) in enumerate(zip(rng.permutation(slots), lengths)):
         spans.append((int(slot), at, n, (0, 7, 128)[i % 3]))
         at += n + i % 2
     spans = table(*spans, slots=slots)
     op = MinGRU(slots=slots, rows=at + 2, stride=3 * width + 5, width=width, dtype=dtype)
     agrees(op, gru_inputs(rng, op, spans), 3e-6 if dtype is F32 else 5e-3, rows_of(spans), workspace=True)
+
+
+def test_a_gated_recurrence_over_many_spans(cuda):
+    """Chunks that are looked up past a wave's lanes, with idle slots among them: none, some and all of 64 slots' lanes, in another order than their rows'."""
+    rng = np.random.default_rng(5)
+    slots, at, spans = 200, 0, []
+    for slot in rng.permutation(np.r_[0:64, 70:128:3, 192:200]):
+        n = int(rng.choice([1, 2, 63, 64, 65, 130]))
+        spans.append((int(slot), at, n, int(rng.choice([0, 4]))))
+        at += n
+    spans = table(*spans, slots=slots)
+    op = MinGRU(slots=slots, rows=at, stride=3 * 40, width=40, dtype=F32)
+    agrees(op, gru_inputs(rng, op, spans), 3e-6, rows_of(spans), workspace=True)
 
 
 @pytest.mark.parametrize("chunked", [False, True], ids=["tokens", "chunks"])
