@@ -283,7 +283,7 @@ static int launch_min_gru(const T* x, const bf16_t* zb, const bf16_t* xb, float*
 using namespace iron;
 
 extern "C" int64_t iron_min_gru_workspace_bytes(int slots, int rows, int width) {
-  return slots > 0 && rows > 0 && width > 0 ? (int64_t)chunks_of(rows, slots, GRU_CHUNK) * 2 * width * (int64_t)sizeof(float2) : 0;
+  return slots > 0 && rows > 0 && width > 0 ? (int64_t)chunks_of(rows, slots, GRU_CHUNK) * width * (int64_t)(sizeof(float2) + sizeof(float)) : 0;
 }
 
 extern "C" int iron_min_gru(const void* x, const uint16_t* z_bias, const uint16_t* x_bias, float* state, const int* spans, void* y,

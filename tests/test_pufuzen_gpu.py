@@ -133,6 +133,19 @@ def test_a_gated_recurrence_over_many_spans(cuda):
     agrees(op, gru_inputs(rng, op, spans), 3e-6, rows_of(spans), workspace=True)
 
 
+def test_a_gated_recurrence_s_workspace(cuda):
+    """A pair and a state a chunk and channel, of as many chunks as there can be, and nothing behind them."""
+    slots, width, rows = 3, 48, 64 + 65 + 1
+    floats = K.lib().iron_min_gru_workspace_bytes(slots, rows, width) // 4
+    assert floats == ((rows + 63) // 64 + slots) * width * 3
+    rng = np.random.default_rng(3)
+    x, bias = device(bf(rng, rows, 3 * width), BF16), device(bf(rng, width), BF16)
+    work, state = torch.full((floats + 256,), 7.0, device="cuda"), torch.zeros(slots, 2, width, device="cuda")
+    spans, y = device(table((0, 0, 64, 0), (1, 64, 65, 0), (2, 129, 1, 0), slots=slots), np.int32), torch.empty(rows, width, dtype=torch.bfloat16, device="cuda")
+    K.min_gru(x, bias, bias, state, spans, y, slots=slots, rows=rows, stride=3 * width, width=width, workspace=work[:floats])
+    assert bool((work[floats:] == 7).all())
+
+
 @pytest.mark.parametrize("chunked", [False, True], ids=["tokens", "chunks"])
 def test_the_recurrence_goes_on_where_a_portion_ends(cuda, chunked):
     rng = np.random.default_rng(7)
