@@ -3140,19 +3140,19 @@ extern "C" int iron_gemm_gated_bf16(const uint16_t* A, const uint16_t* B, const 
 // G may be null: the gate's product is then stored nowhere.  It is as many bytes as the output, behind each tile's last product, where nothing is left to
 // hide them under (weights out of memory, us with and without: 2048 x 8192 x 2048 111 / 107, 857 rows 52 / 50, 4096 x 14336 x 4096 699 / 677, 1024 x 4096 x 1024
 // 23.4 / 21.5, 200 rows of 2048 x 512 8.0 / 7.65).
-static int gemm_gated_pair(const uint16_t* A, const uint16_t* Bg, const uint16_t* Bu, uint16_t* G, uint16_t* C, int M, int N, int K, int activation,
-                           const int* valid, void* stream) {
-  IRON_REQUIRE(A && Bg && Bu && C, "gemm_gated_pair: null operand");
-  IRON_REQUIRE(activation >= 1 && activation <= 3, "gemm_gated_pair: activation (%d) is 1 (SiLU), 2 (GELU, tanh form) or 3 (ReLU)",
+static int gemm_gated_pair(const char* what, const uint16_t* A, const uint16_t* Bg, const uint16_t* Bu, uint16_t* G, uint16_t* C, int M, int N, int K,
+                           int activation, const int* valid, void* stream) {
+  IRON_REQUIRE(A && Bg && Bu && C, "%s: null operand", what);
+  IRON_REQUIRE(activation >= 1 && activation <= 3, "%s: activation (%d) is 1 (SiLU), 2 (GELU, tanh form) or 3 (ReLU)", what,
                activation);
   if (M < 64 && valid == nullptr) return iron_gemm_few_bf16(A, Bg, Bu, C, M, N, K, activation, stream);
-  IRON_REQUIRE(G != C, "gemm_gated_pair: the gate's product and the output are different buffers");
+  IRON_REQUIRE(G != C, "%s: the gate's product and the output are different buffers", what);
   IRON_REQUIRE(K <= (1 << 22) && N <= (1 << 22),
-               "gemm_gated_pair: K (%d) and N (%d) may be at most 2^22 (a tile's rows are addressed with 32-bit offsets)", K, N);
+               "%s: K (%d) and N (%d) may be at most 2^22 (a tile's rows are addressed with 32-bit offsets)", what, K, N);
   IRON_REQUIRE(M >= 64 && N >= 64 && K > 0 && K % BK == 0,
-               "gemm_gated_pair: M (%d) and N (%d) at least 64, K (%d) a positive multiple of %d", M, N, K, BK);
+               "%s: M (%d) and N (%d) at least 64, K (%d) a positive multiple of %d", what, M, N, K, BK);
   IRON_REQUIRE((((uintptr_t)A | (uintptr_t)Bg | (uintptr_t)Bu | (uintptr_t)G | (uintptr_t)C) & 15) == 0,
-               "gemm_gated_pair: operands must be 16-byte aligned");
+               "%s: operands must be 16-byte aligned", what);
   return launch_gemm_gated_pair(A, Bg, Bu, G, C, M, N, K, valid, activation, (hipStream_t)stream);
 }
 
@@ -3160,12 +3160,12 @@ extern "C" int iron_gemm_gated_pair_bf16(const uint16_t* A, const uint16_t* Bg, 
                                          uint16_t* C, int M, int N, int K, int activation, const int* valid,
                                          void* stream) {
   IRON_REQUIRE(G || M < 64, "gemm_gated_pair: null operand");
-  return gemm_gated_pair(A, Bg, Bu, G, C, M, N, K, activation, valid, stream);
+  return gemm_gated_pair("gemm_gated_pair", A, Bg, Bu, G, C, M, N, K, activation, valid, stream);
 }
 
 extern "C" int iron_gemm_gated_product_bf16(const uint16_t* A, const uint16_t* Bg, const uint16_t* Bu, uint16_t* C, int M, int N, int K, int activation,
                                             const int* valid, void* stream) {
-  return gemm_gated_pair(A, Bg, Bu, nullptr, C, M, N, K, activation, valid, stream);
+  return gemm_gated_pair("gemm_gated_product", A, Bg, Bu, nullptr, C, M, N, K, activation, valid, stream);
 }
 
 static int prefill_qkv(const uint16_t* x, const uint16_t* Wq, const uint16_t* Wk, const uint16_t* Wv,

@@ -40,6 +40,11 @@ def test_argument_refusals_need_no_gpu():
     assert b"multiple of 8" in lib.iron_last_error()
     assert lib.iron_mha_prefill_bf16(one, one, one, one, 6, 4, 64, 8, 8, 8, 0.125, 1, -1, 0, 0, None, None, None) == 1
     assert b"multiple of kv_heads" in lib.iron_last_error()
+    for name, operands in (("gemm_gated_pair", 5), ("gemm_gated_product", 4)):   # (two entry points of one function)
+        call = getattr(lib, f"iron_{name}_bf16")
+        for sizes, why in (((64, 64, 64, 0), b"activation"), ((64, 64, 40, 1), b"multiple of 64"), ((64, 1 << 23, 64, 1), b"at most 2^22")):
+            assert call(*(ctypes.c_void_p(16 * i + 16) for i in range(operands)), *sizes, None, None) == 1
+            assert lib.iron_last_error().startswith(name.encode() + b":") and why in lib.iron_last_error()
 
 
 def test_every_entry_point_refuses_null_operands():
