@@ -630,19 +630,22 @@ __global__ __launch_bounds__(256) void latent_step_kernel(const float* __restric
 // columns of the scores' product, add their parts up in LDS, and deal the columns of the weighted sum.  Heads are
 // an MFMA's columns throughout.  NG: groups of 64 latent columns a wave sums.
 //
-// The grid is (head groups x STEP_RUN splits, slots, runs of splits): the slots' first splits, which are the ones with keys, are
-// dealt out ahead of all others, and STEP_RUN neighbours, one a chiplet, read one slot's keys (slots fastest, so that a
-// chiplet has one slot's, 4 slots of 4000 keys take 25.2 us instead of 23.9).
-constexpr int STEP_RUN = 8;
+// The grid is (head groups x a run of splits, slots, runs): the slots' first splits, which are the ones with keys, are
+// dealt out ahead of all others, and a run's eight neighbours, one a chiplet, read one slot's keys (slots fastest, so that a
+// chiplet has one slot's, 4 slots of 4000 keys take 25.2 us instead of 23.9).  Which split is a run's first turns with the slot: where few have keys, they are
+// on every chiplet and not all on one (16 heads over 512 + 64 columns, us with the launches around it: 64 slots of 20 keys 42.9 -> 34.2, 32 slots 25.2 -> 23.3).  A launch
+// of fewer splits has shorter runs (64 slots, a window of 43 keys, 3 heads over 1024 + 8: 46.6 -> 28.0).
+constexpr int STEP_RUN_LOG2 = 3;
 constexpr int TEAM_KEYS = 32, TEAM_PARTS = 4 * 2 * 64 * 16;   // keys, and bytes of scores in parts
 template <int NG>
 __global__ __launch_bounds__(512) void latent_step_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ latents,
                                                                const bf16_t* __restrict__ shared_keys, const int* __restrict__ spans,
-                                                               StepParts to, LatentShape a, int splits, unsigned lat_inverse, unsigned rot_inverse) {
+                                                               StepParts to, LatentShape a, int splits, int run_log2, unsigned lat_inverse, unsigned rot_inverse) {
   constexpr int LATENTS = 4 * NG, SHARED = NG;   // 16-byte pieces of a tile's latents and of its shared parts a thread stages
   constexpr int STEPS = (10 * NG + 3) / 4;       // 32-column steps of the scores' product a wave takes
   extern __shared__ __align__(16) unsigned char dyn[];
-  const int split = blockIdx.z * STEP_RUN + blockIdx.x % STEP_RUN, slot = blockIdx.y, head0 = blockIdx.x / STEP_RUN * 16;
+  const int slot = blockIdx.y, head0 = (blockIdx.x >> run_log2) * 16;
+  const int split = (blockIdx.z << run_log2) + ((blockIdx.x + (slot >> (STEP_RUN_LOG2 - run_log2))) & ((1 << run_log2) - 1));
   const int team = threadIdx.x >> 8, t = threadIdx.x & 255, lane = t & 63, wave = t >> 6, lo16 = lane & 15, quad = lane >> 4;
   const Span s = span_of(spans, slot, a.rows);
   const StepKeys k = step_keys(s, a, splits);
@@ -1045,7 +1048,9 @@ extern "C" int iron_mha_latent(const void* q, const void* latents, const void* s
     else IRON_ABSORB(bf16_t, float)
 #undef IRON_ABSORB
     if (mfma_lds) {
-      const dim3 grid((heads + 15) / 16 * STEP_RUN, slots, (splits + STEP_RUN - 1) / STEP_RUN);
+      int run_log2 = 0;
+      while (run_log2 < STEP_RUN_LOG2 && 1 << run_log2 < splits) ++run_log2;
+      const dim3 grid((heads + 15) / 16 << run_log2, slots, ((splits - 1) >> run_log2) + 1);
 #define IRON_STEP(NG)                                                                                                        \
   static LdsOptIn opted##NG;                                                                                                 \
   if (const hipError_t e = opted##NG.ensure((const void*)latent_step_mfma_kernel<NG>, 163840)) {                             \
@@ -1053,7 +1058,7 @@ extern "C" int iron_mha_latent(const void* q, const void* latents, const void* s
     return (int)e;                                                                                                           \
   }                                                                                                                          \
   hipLaunchKernelGGL((latent_step_mfma_kernel<NG>), grid, dim3(512), mfma_lds, s, (const bf16_t*)absorbed, (const bf16_t*)latents, \
-                     (const bf16_t*)shared_keys, spans, parts, a, splits, inverse_of(rank / 8), inverse_of(rot / 8))
+                     (const bf16_t*)shared_keys, spans, parts, a, splits, run_log2, inverse_of(rank / 8), inverse_of(rot / 8))
       if (rank <= 256) { IRON_STEP(1); }
       else if (rank <= 512) { IRON_STEP(2); }
       else { IRON_STEP(4); }
