@@ -951,10 +951,11 @@ static size_t step_mfma_lds(const LatentShape& a) {
 // Splits for a block a CU: each leaves a float32 sum of the rank a head, which is more than its keys' bytes under 64 keys a
 // split, and blocks whose runs hold no keys yet still have to be dealt out (16 heads over 512 + 64 columns, with the launches
 // around it, 512 blocks -> 256: 8 slots of 4000 keys 35.1 -> 29.8 us, 16 slots of 30 27.2 -> 20.2, of 4000 49.9 -> 44.4, 32 slots
-// of 30 33.0 -> 27.2).  No fewer than 8: 64 slots of 4000 keys take 135 us by 8 and 218 by 4.
-static int step_splits(const LatentShape& a) {
+// of 30 33.0 -> 27.2).  No fewer than 8: 64 slots of 4000 keys take 135 us by 8 and 218 by 4.  A block of the form for any sizes has one head, and its splits are
+// for twice as many (float32, 2 heads over 1024, 16 slots of 1294 keys 153 us by 32 splits a slot and 294 by 16; 4 heads over 512, 8 slots of 3660 keys 87 and 151).
+static int step_splits(const LatentShape& a, bool mfma) {
   const int most = a.window < a.ring ? a.window : a.ring, tiles = (most + STEP_KEYS - 1) / STEP_KEYS;
-  int splits = 256 / (a.slots * ((a.heads + 15) / 16));
+  int splits = (mfma ? 256 : 512) / (a.slots * ((a.heads + 15) / 16));
   splits = splits < 8 ? 8 : (splits > 64 ? 64 : splits);
   return tiles < splits ? tiles : splits;
 }
@@ -1013,8 +1014,9 @@ extern "C" int64_t iron_mha_latent_workspace_bytes(int slots, int rows, int head
     const size_t n = (size_t)expanded_rows(cap);
     return (int64_t)(16 + rounded16(n * rank * each) + rounded16(n * rot * each) + n * heads * (dim + vdim) * each);
   }
-  return (int64_t)(rounded16((size_t)slots * heads * (rank + rot) * 4) + rounded16((size_t)slots * step_splits(a) * heads * rank * 4) +
-                   (size_t)slots * step_splits(a) * heads * 8);
+  const int splits = step_splits(a, !is_float && step_mfma_lds(a) != 0);
+  return (int64_t)(rounded16((size_t)slots * heads * (rank + rot) * 4) + rounded16((size_t)slots * splits * heads * rank * 4) +
+                   (size_t)slots * splits * heads * 8);
 }
 
 extern "C" int iron_mha_latent(const void* q, const void* latents, const void* shared_keys, const uint16_t* up, const uint16_t* sink,
@@ -1030,8 +1032,8 @@ extern "C" int iron_mha_latent(const void* q, const void* latents, const void* s
   unsigned char* work = (unsigned char*)workspace;
   const int width = heads * (dim + vdim);
   if (single) {   // the caller's spans have one row at most
-    const int splits = step_splits(a);
     const size_t mfma_lds = is_float ? 0 : step_mfma_lds(a);
+    const int splits = step_splits(a, mfma_lds != 0);
     void* absorbed = work;
     StepParts parts;
     parts.sums = (float*)(work + rounded16((size_t)slots * heads * (rank + rot) * 4));

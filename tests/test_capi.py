@@ -59,6 +59,16 @@ def test_every_entry_point_refuses_null_operands():
         assert lib.iron_last_error(), name
 
 
+def test_a_latent_step_s_splits():
+    """As many as fill the chip: of blocks of sixteen heads in bf16, of twice as many of one head in float32 and in bf16 of sizes for any."""
+    room = _lib.lib().iron_mha_latent_workspace_bytes
+    for slots, heads, rank, rot, window, is_float, splits in ((16, 2, 1024, 0, 2048, 1, 32), (16, 2, 1024, 0, 2048, 0, 16), (16, 2, 1023, 0, 2048, 0, 32),
+                                                              (4, 16, 512, 64, 4096, 1, 64), (64, 33, 512, 64, 4096, 0, 8), (1, 4, 512, 64, 100, 1, 2)):
+        absorbed = -(-slots * heads * (rank + rot) * 4 // 16) * 16
+        sums = -(-slots * splits * heads * rank * 4 // 16) * 16
+        assert room(slots, slots, heads, 128, rot, 128, rank, window, window, 0, 1, is_float) == absorbed + sums + slots * splits * heads * 8
+
+
 def test_few_rows_over_a_long_k_share_no_tiles():
     """Up to sixteen rows against up to 2048 of a long K go by strips, whatever the product of rows and K; past that, and past
     K = 16384, their tiles' K is dealt over blocks where that takes less than the few rows would.  As (N,M) output the same with the operands' places changed."""
