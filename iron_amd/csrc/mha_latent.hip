@@ -515,13 +515,15 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(const T* __restrict_
   uint4 ahead[AHEAD > 0 ? AHEAD : 1];
 #pragma unroll
   for (int i = 0; i < AHEAD; ++i) ahead[i] = *reinterpret_cast<const uint4*>(w + (size_t)min(group + 16 * i, a.dim - 1) * a.rank);
-  // (an idle slot's loads are some row's, and nothing of it is stored: behind a branch the loads would wait for the span)
+  // (an idle slot's loads are some row's: behind a branch the loads would wait for the span)
   const T* qr = q + ((size_t)min(s.row0, a.rows - 1) * a.heads + head) * wide;
   float x[AHEAD > 0 ? AHEAD : 1];
 #pragma unroll
   for (int i = 0; i < AHEAD; ++i) x[i] = load_one(qr + min(group + 16 * i, a.dim - 1));
+  asm volatile("" ::: "memory");   // (or the loads would be moved behind the test)
+  if (s.rows == 0) return;
   OUT* to = out + ((size_t)slot * a.heads + head) * (a.rank + a.rot);
-  if (blockIdx.z == 0 && s.rows > 0) {
+  if (blockIdx.z == 0) {
     const float* turn = angles + (size_t)min(s.start, a.angle_rows - 1) * a.turned;
     for (int c = t; c < a.rot; c += 256) {
       float v = load_one(qr + a.dim + c);
@@ -556,7 +558,7 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(const T* __restrict_
 #pragma unroll
   for (int j = 0; j < VEC; ++j) red[group * COLUMNS + (t & 15) * VEC + j] = acc[j];
   __syncthreads();
-  if (s.rows > 0 && t < COLUMNS && blockIdx.z * COLUMNS + t < a.rank) {
+  if (t < COLUMNS && blockIdx.z * COLUMNS + t < a.rank) {
     float sum = 0.f;
 #pragma unroll
     for (int g = 0; g < 16; ++g) sum += red[g * COLUMNS + t];
