@@ -91,8 +91,8 @@ def test_a_product_over_few_rows(cuda, M, N, K_):
         assert np.abs(from_torch(C) - gated).max() <= 1.5e-2 * np.abs(gated).max(), act
 
 
-# Products that go by strips of K: a tile of B's rows and less, a block's first second tile, groups of eight tiles stored together and the
-# ninth, N no multiple of 8; K just over a strip, to eight strips and past them with waves that have none; the rows of A at every edge.
+# Products that go by strips of K: a tile of B's rows and less, a block's first second tile, past sixteen rows groups of eight tiles stored together and
+# the ninth, N no multiple of 8; K just over a strip, to eight strips and past them with waves that have none; the rows of A at every edge.
 @pytest.mark.parametrize("M,N,K_", [(1, 1024, 2048), (8, 2049, 1032), (9, 2056, 1960), (16, 16384 + 72, 320), (17, 30011, 1160), (32, 16392, 2048),
                                     (2, 1027, 2056), (8, 2048, 8192), (7, 4100, 2312), (8, 8200, 4104), (16, 520, 5000), (29, 2040, 2304),
                                     (33, 600, 4096), (47, 999, 2816)])
@@ -137,18 +137,31 @@ def test_a_product_over_few_rows_into_an_output_between_pieces(cuda, M, N, K_, a
     assert (C[:at] == 7).all() and (C[at + M * N :] == 7).all()
 
 
-def test_a_product_over_few_rows_of_more_columns_than_27_bits_count(cuda):
-    """One row against 2^27 + 1032 rows of 64: no column is left out, and those where a block's tiles begin and end are right."""
+# ... whose tiles' sums meet four or two at a time: several meetings, the last of them whole and not, where the second's overwrite A's strips, with
+# waves that have none; short of where a stage is filled again early, and past it.
+@pytest.mark.parametrize("M,N,K_", [(8, 10243, 2048), (5, 16383, 264), (3, 8192 + 2048, 1032), (13, 10243, 1032), (16, 8193, 2048), (8, 16384, 2048), (6, 26630, 520),
+                                    (11, 18437, 2040)])
+def test_a_product_over_few_rows_whose_tiles_meet(cuda, M, N, K_):
+    test_a_product_over_few_rows_by_strips(cuda, M, N, K_)
+
+
+@pytest.mark.parametrize("M", [1, 17])
+def test_a_product_over_few_rows_of_more_columns_than_27_bits_count(cuda, M):
+    """2^27 + 1032 rows of 64, against one row, whose blocks take rounds of tiles, and seventeen, whose blocks' tiles are neighbours: no column is left out, and those
+    where rounds, runs of blocks or a block's tiles begin and end are right."""
     N, K_ = 2**27 + 1032, 64
-    a, B = torch.randn((1, K_), device=cuda).bfloat16(), torch.empty((N, K_), dtype=torch.bfloat16, device=cuda).normal_()
-    C = torch.full((1, N), float("nan"), dtype=torch.bfloat16, device=cuda)
-    assert K.lib().iron_gemm_few_bf16(a.data_ptr(), B.data_ptr(), None, C.data_ptr(), 1, N, K_, 0, torch.cuda.current_stream().cuda_stream) == 0
-    assert not C.isnan().any()
-    edges = torch.arange(0, 257, device=cuda) * (N // 8) // 256 * 8
-    rows = (edges[:, None] + torch.arange(-40, 40, device=cuda)).flatten().clamp(0, N - 1)
-    want = (B[rows].double() * a.double()).sum(1)
-    bound = 2.0**-8 * want.abs() + K_ * 2.0**-24 * (B[rows].double() * a.double()).abs().sum(1)   # as above
-    assert ((C[0, rows].double() - want).abs() <= 1.01 * bound).all()
+    a, B = torch.randn((M, K_), device=cuda).bfloat16(), torch.empty((N, K_), dtype=torch.bfloat16, device=cuda).normal_()
+    C = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=cuda)
+    assert K.lib().iron_gemm_few_bf16(a.data_ptr(), B.data_ptr(), None, C.data_ptr(), M, N, K_, 0, torch.cuda.current_stream().cuda_stream) == 0
+    assert not any(row.isnan().any() for row in C)
+    rounds = (N + 2047) // 2048
+    whole = torch.tensor([0, 1, rounds // 2, rounds - 3, rounds - 2, rounds - 1], device=cuda)[:, None] * 2048 + torch.arange(2048, device=cuda)
+    edges = (torch.arange(0, 257, device=cuda) * (N // 8) // 256 * 8)[:, None] + torch.arange(-40, 40, device=cuda)
+    rows = torch.cat([whole.flatten(), edges.flatten()]).clamp(0, N - 1)
+    x, w = a.double(), B[rows].double().t().contiguous()
+    want, size = x @ w, x.abs() @ w.abs()
+    bound = 2.0**-8 * want.abs() + K_ * 2.0**-24 * size   # as above
+    assert ((C[:, rows].double() - want).abs() <= 1.01 * bound).all()
 
 
 # ---------------------------------------------------------------- recurrences

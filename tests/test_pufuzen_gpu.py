@@ -387,8 +387,8 @@ def test_a_row_s_product_joins_the_stream(cuda, M, K_):
                 assert np.array_equal(new[(start - 1) % 2], state[(start - 1) % 2]) and np.abs(new[start % 2] - S).max() <= 1e-5 * np.abs(S).max()
 
 
-# Few columns and many, more tiles than blocks, strips that end in a piece, waves without a strip, one row and all eight.
-@pytest.mark.parametrize("rows,N,K_", [(1, 64, 8), (3, 71, 264), (8, 2048, 2048), (5, 4103, 2040), (7, 20001, 1000)])
+# Few columns and many, more tiles than blocks, one to several meetings of four, strips that end in a piece, waves without a strip, one row and all eight.
+@pytest.mark.parametrize("rows,N,K_", [(1, 64, 8), (3, 71, 264), (8, 2048, 2048), (5, 4103, 2040), (7, 20001, 1000), (8, 10243, 2048), (5, 16383, 264)])
 def test_normed_rows_products(cuda, rows, N, K_):
     rng = np.random.default_rng(N)
     W, gain, x = bf(rng, N, K_, scale=1 / np.sqrt(K_)), bf(rng, K_), rng.standard_normal((rows, K_)).astype(F32) * 3
@@ -440,7 +440,8 @@ def test_a_recurrence_s_step_in_its_projection_s_launch(cuda, rows, width, K_):
 
 # One row and eight, fewer blocks than rows, latents of a piece and of as many as a wave holds, a waves' strip that ends in a piece, parts that turn whole, half and not.
 @pytest.mark.parametrize("rows,N,q_rank,rank,rot,turn", [(8, 3072, 1536, 512, 64, 64), (2, 2048, 1536, 512, 0, 0), (8, 24, 264, 8, 0, 0), (5, 8, 8, 40, 64, 32),
-                                                         (3, 4103, 2048, 4056, 40, 40), (1, 64, 2040, 520, 1528, 8)])
+                                                         (3, 4103, 2048, 4056, 40, 40), (1, 64, 2040, 520, 1528, 8),
+                                                         (7, 10241, 1536, 512, 64, 64), (8, 16390, 264, 40, 24, 16)])
 def test_rows_latents_in_their_queries_launch(cuda, rows, N, q_rank, rank, rot, turn):
     rng = np.random.default_rng(N)
     slots, ring, stride = rows + 2, 64, q_rank + rank + rot + 24
