@@ -21,8 +21,8 @@ namespace iron {
 // What bounds it is the way to the memory, so the shape follows that: eight rows a tile and not the MFMA's sixteen (half of each product is
 // dropped; the matrix cores idle anyway), because 2048 rows of B then occupy all 256 CUs; up to sixteen rows of A as contiguous runs, because
 // rows a power of two apart, read a fragment at a time by every block, meet on one L2 channel.  Eight rows of A over cold weights, us with
-// gemm_few_kernel and with this: 2048 x 2048 5.1 / 4.0, 2048 x 8192 14.1 / 9.2, 4160 x 2048 8.0 / 5.5, 8192 x 2048 10.2 / 7.7,
-// 10240 x 2048 15.0 / 9.1, 128256 x 2048 106 / 79 (6.6 TB/s); thirty-two rows: 4160 x 2048 14.3 / 9.5, 128256 x 2048 163 / 90.
+// gemm_few_kernel and with this: 2048 x 2048 5.2 / 3.9, 2048 x 8192 13.5 / 8.6, 4160 x 2048 7.9 / 5.4, 8192 x 2048 9.5 / 7.6,
+// 10240 x 2048 13.8 / 9.1, 128256 x 2048 95 / 77 (6.8 TB/s); thirty-two rows: 4160 x 2048 13.7 / 9.4, 128256 x 2048 148 / 87.
 constexpr int STRIP = 256, STRIP_BYTES = 512, STRIP_WAVES = 8, STRIP_ROWS = 8;
 constexpr unsigned STRIP_BLOCKS = 256;   // one a CU; fewer tiles: a block each
 // The blocks take rounds of 256 neighbouring tiles, so that all of them together read one run of B at a time; the blocks of a chiplet (every eighth) have
@@ -59,7 +59,7 @@ struct Strips {
 // A's rows are rows of the stream, RMS-normed (as in stream.hip), up to eight of them and K up to eight strips: every block makes all of A for
 // its own tiles, a wave its strip of K while the first of B is on its way.  The launch of a norm between two of 256 blocks takes 2.2 us, and making
 // the rows here 1.0: twice A's bytes out of L2, and a chain of sums, root and scale.  Eight rows over K = 2048, weights out of memory, a norm and a
-// product against both here: 2048 columns 6.1 / 5.1 us, 4160 8.2 / 6.7, 10240 11.6 / 10.3, 128256 86.2 / 85.4.  (A recurrence's step made the same
+// product against both here: 2048 columns 6.1 / 5.0 us, 4160 7.95 / 6.6, 10240 11.45 / 10.0, 128256 82.0 / 80.7.  (A recurrence's step made the same
 // way ahead of the product behind it was not the faster one, 8.9 / 9.3: three exponentials an element, 8 x 2048 of them a block.)
 struct StripsNorm {
   const bf16_t* gain;
@@ -687,21 +687,23 @@ static int launch_gemm_strips(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
 static bool strips_many(int N) { return N >= 8 * (int)STRIP_BLOCKS * STRIP_ROWS; }
 
 // Which products go by strips, by what both kernels took over three hundred shapes with weights out of memory (us, gemm_few_kernel against strips).
-// K up to eight strips: up to 16 rows of A (8 rows: 64 x 384 3.9 / 2.6, 1024 x 1024 4.4 / 2.9, 8192 x 2048 9.0 / 8.2, 16000 x 600 8.8 / 7.4, 128256 x 2048
-// 105 / 82; one row: 2048 x 2048 4.5 / 3.6, 7159 x 2048 8.1 / 7.7), but not many rows of B that are a cache line or less (6 rows: 3440 x 40 2.8 / 3.4)
-// nor rows that straddle lines where they make two tiles a block of gemm_few_kernel's one round (212 shapes of K 1280 to 2047: strips take 1.07 to 1.24 of
-// its time; 2656 x 136 3.1 / 3.5); up to 32 rows, whose sums take a second set of registers, over long rows
-// that keep to their lines (32 rows: 1024 x 2048 7.8 / 6.6, 4160 x 2048 13.8 / 9.5; but 2400 x 192 3.5 / 5.2) or a B of 64 MB (20 rows: 128256 x 2048 137 / 87).
-// A longer K: the strips of A that come with every tile cost as much as B's own.  Up to eight rows (2048 x 8192 13.9 / 8.9, 6000 x 6000 21.8 / 18.5,
-// 4096 x 14336 25.0 / 24.0, 4560 x 4416 19.5 / 12.6; two tiles a block of one round too: 3904 x 3072 10.7 / 7.2, 3656 x 4160 12.9 / 8.9, and the same weights
-// again, out of the last-level cache, 8.8 / 8.4 and 11.5 / 10.1; there rows that straddle lines from K = 8192 on: of 210 shapes short of it strips take 1.02 to 1.08 of the
-// other's time, one row of 2382 x 2488 5.4 / 6.0, past it 0.97, and go through the caches, which with the same weights again is 0.87 to 0.96 of going past them);
-// up to 16 where a block has one tile (2048 x 8192 16.7 / 10.2) or three and more (4788 x 6848 28.6 / 21.2, 9762 x 9056 60.9 / 46.7).  With
-// two tiles a block, or three and a half whose rows straddle lines, strips take the less of weights out of memory and gemm_few_kernel of the same weights again (3016 x
-// 4520 14.1 / 11.8 and 10.3 / 12.9, 2448 x 7456 17.8 / 16.3 and 12.5 / 17.4, 7562 x 2888 17.7 / 15.7 and 13.2 / 16.8): that kernel, which gains
-// more than it loses; more rows where that one's rows keep to their cache lines or are few (32 rows: 2048 x 4096
-// 13.2 / 12.2, 1024 x 8192 23.5 / 14.8; 20 rows of 1960 x 6512 13.8 / 15.1), and are not three or less (22 rows of 2 x 2688 6.2 / 6.9), past 32 rows from K = 2560 on,
-// or 3072 of rows that straddle lines (38 rows of 9 x 2200 7.1 / 8.9, 51 of 32 x 2080 8.3 / 9.5; of 110 drawn ones short of there strips take 1.05 to 1.29 of the other's time).  The loads go past the caches except where a block has
+// K up to eight strips: up to 16 rows of A (8 rows: 64 x 384 3.9 / 2.6, 1024 x 1024 4.7 / 2.9, 8192 x 2048 9.5 / 7.5, 16000 x 600 8.9 / 6.5, 128256 x 2048
+// 95 / 77; one row: 2048 x 2048 4.4 / 3.5, 7159 x 2048 7.4 / 6.8), but not many rows of B that are a cache line or less (6 rows: 3440 x 40 2.95 / 3.15)
+// nor, where they make two tiles a block of gemm_few_kernel's one round, rows of 1024 columns and more that straddle lines (of 120 shapes of K to 1280 strips take 0.86 of the other's
+// time, and the same weights again 0.99, of 120 to 2047 0.85 and 1.04; 480 shapes short of 1024 0.81 to 0.95 and 0.88 to 0.96, none of them slower); up to 32 rows, whose
+// sums take a second set of registers, over long rows
+// that keep to their lines (32 rows: 1024 x 2048 7.9 / 6.3, 4160 x 2048 13.7 / 9.4; but 2400 x 192 3.9 / 5.3) or a B of 64 MB (20 rows: 128256 x 2048 128 / 82).
+// A longer K: the strips of A that come with every tile cost as much as B's own.  Up to eight rows (2048 x 8192 13.5 / 8.6, 6000 x 6000 20.3 / 15.8,
+// 4096 x 14336 24.7 / 22.7, 4560 x 4416 18.2 / 10.9; two tiles a block of one round too: 3904 x 3072 7.9 / 6.5, 3656 x 4160 10.4 / 8.2, and the same weights
+// again, out of the last-level cache, 7.1 / 6.4 and 9.8 / 7.9; there rows that straddle lines from K = 8192 on: of 60 shapes of K to 4096 strips take 0.99 of the
+// other's time, a third of them more, of 60 to 8192 0.95, and through the caches, as past it, the same weights again no less);
+// up to 16 where a block has one tile (2048 x 8192 16.1 / 10.1) or three and more (4788 x 6848 28.9 / 20.1, 9762 x 9056 60.8 / 47.7).  With
+// two tiles a block, or three and a half whose rows straddle lines, strips take the less of weights out of memory, but of the same weights again that is the other for
+// a quarter of the sizes (on lines: K to 3072 0.82 and 0.95, to 4096 0.89 and 1.04, to 6144 0.87 and 0.97, past it 0.88 and 0.96; rows that straddle them 1.00 and 0.97, three and
+// a half tiles 1.03 and 1.04): that kernel; more rows where that one's rows keep to their cache lines or are few (32 rows: 2048 x 4096
+// 13.6 / 12.2, 1024 x 8192 24.7 / 19.2; 20 rows of 1960 x 6512 18.8 / 15.2, but the same weights again 12.1 / 13.7), and are not three or less (22 rows of 2 x 2688 5.9 / 6.6), past
+// 32 rows from K = 2560 on, or 3072 of rows that straddle lines (38 rows of 9 x 2200 6.7 / 8.6, 51 of 32 x 2080 7.6 / 9.3; of 110 drawn ones short of there strips take 1.05 to 1.29 of
+// the other's time).  The loads go past the caches except where a block has
 // one tile over a long K (2048 x 8192, 8 rows: 9.3, past them 10.5; 4096 x 4096 10.1 and 9.4), or two of rows that straddle lines, or of more
 // than eight rows any number of these (309 drawn ones: through them 0.93 of gemm_few_kernel's time and 0.91 with the same weights again, past them 0.92 and 1.15).
 // Returns -1 where it is not for them.
@@ -712,7 +714,7 @@ static int strips_for(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N,
     if (M > 32 || (M > 16 && !long_rows && !large)) return -1;
     if (M > 16) return launch_gemm_strips<2, 16, true, 2, true>(A, B, C, M, N, K, s);
     if (!one_tile && K < 64) return -1;
-    if (two_tiles && !on_lines) return -1;
+    if (two_tiles && !on_lines && K >= 1024) return -1;
     if (strips_many(N)) {
       if (M <= 8) return launch_gemm_strips<1, 8, true, 2, true, false, false, false, false, true>(A, B, C, M, N, K, s);
       return launch_gemm_strips<1, 16, true, 2, true, false, false, false, false, true>(A, B, C, M, N, K, s);

@@ -111,7 +111,8 @@ def test_a_product_over_few_rows_by_strips(cuda, M, N, K_):
 
 # ... the smallest sizes that go by strips, with waves that have none, and the others at the lines between the two kernels.
 @pytest.mark.parametrize("M,N,K_", [(1, 1, 8), (5, 40, 24), (16, 2047, 56), (3, 13, 264), (12, 3000, 1416), (6, 2048, 1400), (2, 3001, 2560), (9, 4104, 2056),
-                                    (16, 8200, 5640), (30, 1032, 1600), (20, 4200, 1664)])
+                                    (16, 8200, 5640), (30, 1032, 1600), (20, 4200, 1664),
+                                    (5, 2052, 72), (16, 4096, 1016), (2, 4089, 520), (7, 3000, 1032)])
 def test_a_product_over_few_rows_between_the_kernels(cuda, M, N, K_):
     test_a_product_over_few_rows_by_strips(cuda, M, N, K_)
 
