@@ -28,7 +28,9 @@ constexpr unsigned STRIP_BLOCKS = 256;   // one a CU; fewer tiles: a block each
 // The blocks take rounds of 256 neighbouring tiles, so that all of them together read one run of B at a time; the blocks of a chiplet (every eighth) have
 // eight neighbours, whose columns make a line of C in its L2.  Where a block's own tiles were neighbours the blocks read 256 places that are the same
 // power of two apart, and a stream alone took 6.6 us for 33 MB and 12.1 for 67 that takes 6.4 and 11.4 so (weights out of memory, us: 8 rows of 3072 x 1536 4.75 -> 4.1,
-// 4160 x 2048 5.95 -> 5.5, 8192 x 2048 8.0 -> 7.7, 50257 x 768 19.4 -> 15.9, 128256 x 2048 81.5 -> 79; 16 rows of 32000 x 1024 14.6 -> 12.5).  More than sixteen rows keep
+// 4160 x 2048 5.95 -> 5.5, 8192 x 2048 8.0 -> 7.7, 50257 x 768 19.4 -> 15.9, 128256 x 2048 81.5 -> 79; 16 rows of 32000 x 1024 14.6 -> 12.5).  But rows of B that
+// are 8192 columns or a multiple, give or take a line, put a round's tiles themselves a power of two apart: up to eight rows keep neighbours there (one row, 28672 x 8192 73.6, in
+// rounds 80.5; 28672 x 16384 143 and 148).  More than sixteen rows keep
 // neighbours, and STRIP_OUT columns of C leave as whole lines: a C that its chiplets do not hold until its lines are whole costs more than that (32 rows of
 // 128256 x 2048 90, in rounds 104).
 constexpr int STRIP_OUT = 64;
@@ -210,7 +212,7 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
   static_assert(!MANY || (SINGLE && STAGES == 2 && MT == 1 && !JOINS && !GRU && !LATENT), "a block's tiles follow each other strip by strip");
   static_assert(!LATENT || (NORMED && !JOINS && !GRU), "the query latents are normed rows");
   constexpr int W = STRIP_WAVES, R = STRIP_ROWS;
-  constexpr bool LINED = MT > 1 && !JOINS && !GRU;   // a block's tiles are neighbours, and the columns of GROUP of them are stored together
+  constexpr bool LINED = MT > 1 && !JOINS && !GRU;   // the columns of GROUP of a block's tiles are stored together
   constexpr int GROUP = STRIP_OUT / R;
   static_assert(STAGES <= 2, "the last item's wait is for all that is out");
   constexpr int NOWHERE = 0x7ffffff0;   // an offset past the end of every run of rows (64 rows of at most 2^22, the entry point's bound, are 2^29 bytes)
@@ -220,13 +222,14 @@ __global__ __launch_bounds__(STRIP_WAVES * 64) void gemm_strips_kernel(const bf1
   const unsigned tiles = ((unsigned)N + R - 1) / R;
   // (64 bits: 256 times the tiles of an N of 2^27 pass 32)
   auto neighbours = [&](unsigned block) { return (unsigned)((unsigned long long)block * tiles / STRIP_BLOCKS); };
-  const unsigned first = GRU || tiles <= STRIP_BLOCKS ? blockIdx.x : (LINED ? neighbours(blockIdx.x) : strip_place(blockIdx.x));
-  const unsigned end = LINED && tiles > STRIP_BLOCKS ? neighbours(blockIdx.x + 1) : tiles;
-  constexpr int STEP = LINED ? 1 : (int)STRIP_BLOCKS;
+  const bool next = LINED || (!SINGLE && MA == 8 && ((K + 64) & 8191) <= 128);   // a block's tiles are neighbours
+  const unsigned first = GRU || tiles <= STRIP_BLOCKS ? blockIdx.x : (next ? neighbours(blockIdx.x) : strip_place(blockIdx.x));
+  const unsigned end = next && tiles > STRIP_BLOCKS ? neighbours(blockIdx.x + 1) : tiles;
+  const int step = next ? 1 : (int)STRIP_BLOCKS;
   const bool idle = LATENT && blockIdx.x >= tiles;   // (a block for its row's latent alone; the tile that it fetches all the same is the first)
   const int tile0 = GRU || idle ? 0 : (int)first;
-  const int my_tiles = GRU ? 4 : (idle ? 0 : (tiles <= STRIP_BLOCKS ? 1 : (int)((end - first + STEP - 1) / STEP))), items = my_tiles * mine;
-  auto column_of = [&](int t) { return GRU ? t * (N >> 2) + (int)blockIdx.x * R : (tile0 + t * STEP) * R; };   // tile t's first
+  const int my_tiles = GRU ? 4 : (idle ? 0 : (tiles <= STRIP_BLOCKS ? 1 : (int)((end - first + step - 1) / step))), items = my_tiles * mine;
+  auto column_of = [&](int t) { return GRU ? t * (N >> 2) + (int)blockIdx.x * R : (tile0 + t * step) * R; };   // tile t's first
   char* const own = lds + wave * (S::OVER_A ? S::A_BYTES : S::WAVE);   // (with SINGLE A's strip)
   char* const held = S::OVER_A ? lds + W * S::A_BYTES + wave * (STAGES * S::ITEM) : own + (SINGLE ? S::A_BYTES : 0);
   const unsigned lds0 = (unsigned)(uintptr_t)IRON_LDS_PTR(lds), part0 = lds0 + S::SUMS;

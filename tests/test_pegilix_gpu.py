@@ -139,9 +139,9 @@ def test_a_product_over_few_rows_into_an_output_between_pieces(cuda, M, N, K_, a
 
 
 # ... whose tiles' sums meet four or two at a time: several meetings, the last of them whole and not, where the second's overwrite A's strips, with
-# waves that have none; short of where a stage is filled again early, and past it.
+# waves that have none; short of where a stage is filled again early, and past it; rows near a multiple of 8192, whose blocks keep to neighbouring tiles.
 @pytest.mark.parametrize("M,N,K_", [(8, 10243, 2048), (5, 16383, 264), (3, 8192 + 2048, 1032), (13, 10243, 1032), (16, 8193, 2048), (8, 16384, 2048), (6, 26630, 520),
-                                    (11, 18437, 2040)])
+                                    (11, 18437, 2040), (1, 4108, 8192), (8, 6150, 8128), (3, 2056, 16448)])
 def test_a_product_over_few_rows_whose_tiles_meet(cuda, M, N, K_):
     test_a_product_over_few_rows_by_strips(cuda, M, N, K_)
 
