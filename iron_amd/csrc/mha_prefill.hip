@@ -33,6 +33,12 @@ constexpr int BQ = 128;   // query rows per block (four waves of 32; 64 where a 
 constexpr int BKV = 64;   // key rows per tile
 constexpr float kLazyBits = 8.f;        // how far a maximum may run ahead of the reference the exponents are taken against
 constexpr float kSumLow = 0x1p-60f, kSumHigh = 0x1p24f;   // a tile's sum of exponentials outside this range: take its maximum and redo it
+// 128-wide heads of up to 1024 blocks by four waves: how many of a block's first tiles have their weights in two terms of bf16.  A weight rounds to bf16 against its
+// reference, and only the largest, exactly 1 against a reference that is its maximum, comes through whole; eight waves a block have a reference for each half
+// of the tiles and so two such weights.  Two terms in the first two tiles, all that the first 128 queries have, are nearer than that
+// (relative error against 64 bits, 32 heads, 3001 queries: eight waves 0.00209, four with one term 0.00212, so 0.00188, of which 0.00166 are the output's own rounding; window of
+// 1024 0.00211 / 0.00213 / 0.00192; 2500 queries, window of 129 0.00211 / 0.00222 / 0.00196) and cost 2 us (four tiles: 4).
+constexpr int kFineTiles = 2;
 constexpr int kCUs = 256;                // compute units the block orders below assume
 // Which 16-byte chunk of a key's (value's) row in LDS holds its first one: the others are XORed by it.  A row of 64 elements is half the banks, so sixteen
 // rows' fragments at one chunk, and four rows' at four, meet no bank twice by these; a row of 128 is all of them and takes the row itself
@@ -50,13 +56,10 @@ template <int D, int W>
 __host__ __device__ __forceinline__ bool few_rows_pay(int groups, int keys) { return groups <= (D == 64 && W == 4 ? 512 : 256) && keys >= 512; }
 constexpr int kFewBlocks = 512;          // launches of fewer blocks than this halve their blocks' queries (S = 1024 at 32 heads: 18.5 -> 13.9 us)
 constexpr int kWideBigBlocks = 512;     // wide heads: launches of at least this many 128-query blocks keep that size
-// Launches of up to this many blocks split each block's tiles over two halves of eight waves, which halves a block's chain of tiles; more fill the chip better
-// four waves each.  64-wide heads (two eight-wave blocks share a CU): S = 8192 at 32 heads 365 -> 353-360 us split, past S = 16384 not.  128-wide ones (two
-// four-wave blocks, which read a tile's keys ahead) would be the faster unsplit from 560 blocks on (32 heads, split against not, 2048 queries 45.4 / 52.4, 2305
-// 63.6 / 59.8, 3001 90.4 / 81.8, 4096 147 / 135; 16 heads, 6000 159 / 155), but split, a query has a reference for each half of its tiles, so that the
-// largest weight of either is 1, which bf16 holds exactly: 3001 queries are 0.00208 from 64 bits split and 0.00211 not (the output's own rounding
-// is 0.00166), and up to 1024 blocks the nearer one stays.
-constexpr int kSplitMaxBlocks64 = 4096, kSplitMaxBlocks128 = 1024;
+// Launches of few blocks split each block's tiles over two halves of eight waves, which halves a block's chain of tiles; more fill the chip better
+// four waves each.  64-wide heads (two eight-wave blocks share a CU): S = 8192 at 32 heads 365 -> 353-360 us split, past S = 16384 not.  128-wide ones: see
+// split_128.
+constexpr int kSplitMaxBlocks64 = 4096;
 
 // Few live queries over many keys (a turn late in a conversation: 40 rows of a 2048-row launch, 12 000 keys): by the
 // tiles below, a block a head and 128 queries, most of the chip would idle behind a block's chain
@@ -275,7 +278,7 @@ __device__ __forceinline__ void prefill_few_rows(
 //
 // W: the waves that share a tile's loads, each with 32 of the block's 32 W queries.  Four; two
 // where four would leave CUs without a block (a short prompt), so that twice as many blocks go out.
-template <int D, int SPLIT, int W, bool FEW>
+template <int D, int SPLIT, int W, bool FEW, bool FINE>
 __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(W == 4 ? (D == 64 && SPLIT == 2 ? 4 : 2) : 2))) void mha_prefill_kernel(
     const bf16_t* __restrict__ Q, const bf16_t* __restrict__ K, const bf16_t* __restrict__ V,
     bf16_t* __restrict__ O, int heads, int group, int seq, int seq_len, int kv_len, float scale_log2,
@@ -567,6 +570,21 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
           careful = true;
         }
         l_run = l_run * alpha + rsum;
+        // What rounding to bf16 leaves of the first tiles' weights (see kFineTiles).
+        const bool fine = FINE && tile < kFineTiles;
+        bf16x8 lo[2][2];
+        if (fine) {
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              float p[8], hi[8];
+              unpack8(__builtin_bit_cast(uint4, pf[t][h]), hi);
+#pragma unroll
+              for (int j = 0; j < 8; ++j) p[j] = __builtin_amdgcn_exp2f(fmaf(sacc[t][8 * h + j], scale_log2, -mc)) - hi[j];
+              lo[t][h] = __builtin_bit_cast(bf16x8, pack8(p));
+            }
+        }
         if (moves) {   // the output sums follow the reference (here, where the scores' registers are free again)
 #pragma unroll
           for (int t = 0; t < DT; ++t)
@@ -576,7 +594,7 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
 
         // O^T += V^T P^T, a 32-key half at a time so one wait covers a batch of reads; the key
         // offsets ride in the reads' offset fields.
-        auto pv_half = [&](auto half) {
+        auto pv_half = [&](auto half, const bf16x8 (&weights)[2][2]) {
           constexpr int t = decltype(half)::value;
           TrFrag vf[DT][2];
 #pragma unroll
@@ -592,11 +610,15 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
             lds_tr_wait(vf[dt][0], vf[dt][1]);
 #pragma unroll
             for (int h = 0; h < 2; ++h)
-              oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_join(vf[dt][h]), pf[t][h], oacc[dt], 0, 0, 0);
+              oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_join(vf[dt][h]), weights[t][h], oacc[dt], 0, 0, 0);
           }
         };
-        pv_half(std::integral_constant<int, 0>{});
-        pv_half(std::integral_constant<int, 1>{});
+        pv_half(std::integral_constant<int, 0>{}, pf);
+        pv_half(std::integral_constant<int, 1>{}, pf);
+        if (fine) {
+          pv_half(std::integral_constant<int, 0>{}, lo);
+          pv_half(std::integral_constant<int, 1>{}, lo);
+        }
       }
     };
     // A step of the loop on stage buffer `buf`.
@@ -1023,30 +1045,30 @@ struct PrefillArgs {
 };
 
 // The stage buffers are dynamic LDS (more than the 64 KB a kernel may declare statically).
-template <int D, int SPLIT, int W, bool FEW>
+template <int D, int SPLIT, int W, bool FEW, bool FINE>
 static int launch_prefill_as(const PrefillArgs& a, int blocks, void* stream) {
   constexpr int STAGES = D == 64 && SPLIT == 1 ? 3 : 2;
   constexpr size_t lds = (size_t)SPLIT * STAGES * 2 * BKV * D * 2;
   static LdsOptIn opt_in;
-  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&mha_prefill_kernel<D, SPLIT, W, FEW>), lds); e != hipSuccess) {
+  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&mha_prefill_kernel<D, SPLIT, W, FEW, FINE>), lds); e != hipSuccess) {
     set_error("mha_prefill: %s", hipGetErrorString(e));
     return (int)e;
   }
-  hipLaunchKernelGGL((mha_prefill_kernel<D, SPLIT, W, FEW>), dim3(blocks), dim3(64 * W * SPLIT), lds, (hipStream_t)stream, a.Q,
+  hipLaunchKernelGGL((mha_prefill_kernel<D, SPLIT, W, FEW, FINE>), dim3(blocks), dim3(64 * W * SPLIT), lds, (hipStream_t)stream, a.Q,
                      a.K, a.V, a.O, a.heads, a.group, a.seq, a.seq_len, a.kv_len, a.scale_log2, a.causal, a.window,
                      a.q_row, a.q_head, a.kv_row, a.kv_head, a.valid, a.kv_valid, a.kv_first, a.kv_rows);
   return 0;
 }
 
 // Bounds read on the device may leave few queries; else the sizes say whether there are.
-template <int D, int SPLIT, int W = 4>
+template <int D, int SPLIT, int W = 4, bool FINE = false>
 static int launch_prefill(const PrefillArgs& a, int blocks, void* stream) {
   const bool bounded = a.valid != nullptr || a.kv_valid != nullptr || a.seq_len != a.seq;
   // (a launch so short that all its queries may go 32 to a block has a block for each 32)
   const int groups = ((a.seq + 31) / 32) * a.heads;
   const bool few = few_rows_pay<D, W>(groups, a.kv_len);
-  if (a.kv_len < 512 || (!bounded && !few)) return launch_prefill_as<D, SPLIT, W, false>(a, blocks, stream);
-  return launch_prefill_as<D, SPLIT, W, true>(a, few && groups > blocks ? groups : blocks, stream);
+  if (a.kv_len < 512 || (!bounded && !few)) return launch_prefill_as<D, SPLIT, W, false, FINE>(a, blocks, stream);
+  return launch_prefill_as<D, SPLIT, W, true, FINE>(a, few && groups > blocks ? groups : blocks, stream);
 }
 
 // Whether a launch of 128-wide heads takes blocks of 64 queries (one a CU) and not of 128.  One round of them does: it is the shorter
@@ -1059,6 +1081,24 @@ static bool half_blocks_128(const PrefillArgs& a) {
   const long levels = (a.seq + 63) / 64;
   if (a.heads * levels <= kCUs) return true;
   return a.causal && (a.window < 0 || a.window >= a.kv_len) && a.heads * (levels + 5 + (a.kv_len - a.seq) / 64) <= 2 * kCUs;
+}
+
+// Whether a launch of 128-wide heads by blocks of 128 queries takes eight waves a block, one block a CU, or four, two blocks a CU, which read a tile's keys
+// ahead (kFineTiles).  Up to 512 blocks of four waves are one round, in which a block takes longer than of eight.  Past 832 blocks four are the faster (us, eight / four: 32
+// heads, 3400 queries behind 4000 keys 339 / 324, without a mask 217 / 203, 3780 behind 4000 366 / 361; 8 heads 13500 queries 372 / 359; but windows of 2048 keys 16 heads 6724 queries
+// 118 / 122, from 896 blocks on 127 / 125).  Between the two it is how the blocks' lengths differ.  As long as each other, they make a round more or less: eight waves stay (2500 queries
+// without a mask 123 / 132, behind 4000 keys 236 / 249).  Queries over their own keys: four where there are heads enough for the blocks that go out last to fill in behind the longest (32
+// heads 2500 queries 72.5 / 70.4, 3012 94.0 / 86.7, 24 heads 3780 106 / 103, 16 heads 6340 177 / 171, 64 heads 1092 41.5 / 35.2; short of the line 24 heads 3268 85.7 / 86.4,
+// 16 heads 5572 142 / 144, 8 heads 9200 185 / 211), and behind short windows (2116 queries, windows of 301 and 1024 34.7 / 30.2 and 47.4 / 42.7; 3012 queries 44.1 / 42.1 and
+// 70.9 / 68.9; window of 1401, 24 heads 3268 queries 65.0 / 62.6, 4164 86.8 / 89.7).  Bounds on the device may leave fewer: eight waves up to 1024 blocks.
+static bool split_128(const PrefillArgs& a, int blocks) {
+  if (a.valid != nullptr || a.kv_valid != nullptr || a.seq_len != a.seq) return blocks <= 4 * kCUs;
+  if (blocks <= 2 * kCUs) return true;
+  const bool windowed = a.window >= 0 && a.window < a.kv_len;
+  if (blocks > 832) return windowed && a.window >= 1536 && blocks < 896;
+  if (!a.causal || a.kv_len >= a.seq + BQ) return true;
+  if (windowed) return a.window >= (blocks <= 640 ? 1536 : 1024);
+  return 2 * blocks < 1000 + 13 * (blocks / a.heads);
 }
 
 template <int D, int QN, int W>
@@ -1109,9 +1149,6 @@ static int mha_prefill(const uint16_t* Q, const uint16_t* K, const uint16_t* V, 
                (long)kv_len * kv_row * 2);
   const float scale_log2 = scale * 1.4426950408889634f;
   const int blocks = ((seq + BQ - 1) / BQ) * heads;
-  // Few blocks (a short sequence): the longest block's chain of tiles bounds the launch, so its
-  // tiles are split over two halves of eight waves.  Many blocks fill the chip better four waves each.
-  const bool split = blocks <= (d == 64 ? kSplitMaxBlocks64 : kSplitMaxBlocks128);
   PrefillArgs a{Q, K, V, O, heads, heads / kv_heads, seq, seq_len, kv_len, scale_log2, causal, window,
                 q_row, q_head, kv_row, kv_head, valid, kv_valid, kv_first, kv_rows};
   int rc;
@@ -1126,12 +1163,13 @@ static int mha_prefill(const uint16_t* Q, const uint16_t* K, const uint16_t* V, 
                                       : launch_prefill_wide<256, 1, 4>(a, stream);
   // Fewer blocks of 128 queries than two a CU (a short prompt): blocks of 64, two waves a part.
   else if (d == 64 && blocks < kFewBlocks) rc = launch_prefill<64, 2, 2>(a, ((seq + 63) / 64) * heads, stream);
-  else if (d == 64) rc = split ? launch_prefill<64, 2>(a, blocks, stream) : launch_prefill<64, 1>(a, blocks, stream);
+  else if (d == 64) rc = blocks <= kSplitMaxBlocks64 ? launch_prefill<64, 2>(a, blocks, stream) : launch_prefill<64, 1>(a, blocks, stream);
   // (where the few-row form takes the whole launch, and the keys are many, its blocks have eight waves: 40 queries over 512 / 1024 / 2000 / 12043 keys
   // with four 9.5 / 12.8 / 19.0 / 87 us, with eight 10.9 / 13.3 / 18.0 / 69)
   else if (half_blocks_128(a) && !(kv_len >= 1536 && few_rows_pay<128, 4>(((seq + 31) / 32) * heads, kv_len)))
     rc = launch_prefill<128, 2, 2>(a, ((seq + 63) / 64) * heads, stream);
-  else if (split) rc = launch_prefill<128, 2>(a, blocks, stream);
+  else if (split_128(a, blocks)) rc = launch_prefill<128, 2>(a, blocks, stream);
+  else if (blocks <= 4 * kCUs) rc = launch_prefill<128, 1, 4, true>(a, blocks, stream);   // (those that eight waves would be as near for)
   else rc = launch_prefill<128, 1>(a, blocks, stream);
   if (rc != 0) return rc;
   IRON_LAUNCH_CHECK();

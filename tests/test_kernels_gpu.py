@@ -1230,6 +1230,30 @@ def test_mha_prefill_128_wide_heads_keep_a_reference_for_each_half_of_the_tiles(
     assert np.all(err <= (0.5 * step + 2.0**-18 * want)[..., None]), f"{(err > (0.5 * step + 2.0**-18 * want)[..., None]).mean():.3f} are off by more"
 
 
+# 600 and 832 blocks of 128 queries, four waves each (and one query past a block); windows of 1024 and 513 keys, 528 and 1020 blocks.
+@pytest.mark.parametrize("H,G,S,window", [(40, 8, 1900, None), (32, 8, 3201, None), (16, 4, 4170, 1023), (60, 4, 2100, 512)])
+def test_mha_prefill_128_wide_heads_first_tiles_weights_in_two_terms(cuda, H, G, S, window):
+    """As above by one reference a query: the two weights lie in the first two tiles, whose weights keep what bf16 leaves of them, so the answer is off by its own
+    rounding (half a step) and by the 2^-18 of a weight that two terms leave."""
+    rng = np.random.default_rng(S)
+    Q, Kc, Vc = np.zeros((S, H, 128), np.float32), np.zeros((S, G, 128), np.float32), np.zeros((S, G, 128), np.float32)
+    Q[..., 0] = round_bf16(rng.uniform(0.1, 3.0, (S, H)).astype(np.float32))
+    Q[..., 1] = 1.0
+    Kc[..., 1] = -300.0
+    Kc[5, :, 1] = 0.0
+    Kc[70, :, 0], Kc[70, :, 1] = -1.0, 0.0
+    Vc[70] = 1.0
+    O = out_like(Q.shape, cuda, fill=float("nan"))
+    K.mha_prefill(dev(Q, cuda), dev(Kc, cuda), dev(Vc, cuda), O, heads=H, kv_heads=G, d=128, seq=S, kv_len=S, scale=1.0, causal=True, window=window,
+                  q_interleaved=True, kv_interleaved=True)
+    got, last = from_torch(O).astype(np.float64), S if window is None else window + 6   # (past them the first key is out of sight)
+    w = np.exp(-Q[71:last, :, 0].astype(np.float64))
+    want = w / (1 + w)
+    step = 2.0 ** (np.floor(np.log2(want)) - 7)
+    assert np.all(np.abs(got[71:last] - want[..., None]) <= (0.5 * step + 2.0**-17 * want)[..., None])
+    assert not np.isnan(got).any() and np.all(got[:70] == 0) and (window is None or np.all(got[71 + window:] == 0))
+
+
 # Launches of more than 1024 blocks, four waves each, which read a tile's keys ahead and refill their place at the next step: one key, one tile and one
 # key more, two tiles, three and four (the first refill, the last step's reads past the end), a window, no mask, rows past the bounds.
 @pytest.mark.parametrize("H,G,S,rows,L,keys,window,causal", [
