@@ -273,6 +273,14 @@ int iron_mha_prefill_bf16(const uint16_t* Q, const uint16_t* K, const uint16_t* 
                           int heads, int kv_heads, int d, int seq, int seq_len, int kv_len,
                           float scale, int causal, int window, int q_interleaved,
                           int kv_interleaved, const int* valid, const int* kv_valid, void* stream);
+/* The same for few queries over many keys, d 64 or 128: the keys are dealt over blocks, each of which takes the queries of
+ * all of a KV head's query heads, and a second launch adds up what they leave in `workspace`
+ * (iron_mha_prefill_dealt_workspace_bytes of device memory, 16-byte aligned, any contents; 0: other widths, refused). */
+int iron_mha_prefill_dealt_bf16(const uint16_t* Q, const uint16_t* K, const uint16_t* V, uint16_t* O,
+                                int heads, int kv_heads, int d, int seq, int seq_len, int kv_len,
+                                float scale, int causal, int window, int q_interleaved,
+                                int kv_interleaved, const int* valid, const int* kv_valid, void* workspace, void* stream);
+int64_t iron_mha_prefill_dealt_workspace_bytes(int heads, int kv_heads, int d);
 /* The same over a window of a longer buffer of keys: K, V (kv_rows, kv_heads, d), of which the kv_len
  * rows from *kv_first on are the keys (the first row is held where they end inside the buffer).  What
  * a sliding-window layer's ring cache needs (iron/lm/blocks.py:504-529: the reference copies the

@@ -245,8 +245,9 @@ class Built:
     launch: Callable[[Mapping[str, Any], Mapping[str, Any]], None]
     # ``(per-call value, limit)``: while that value stays within the limit, ``launch`` has a cheaper
     # form, which it takes when ``words["__context__"]["bounded"]`` is true.  The caller vouches for
-    # the limit only as far as speed goes: the bounded form is correct for any value.
-    bounded: tuple[str, int] | None = None
+    # the limit only as far as speed goes: the bounded form is correct for any value.  Or ``(names of
+    # per-call values, within)``: while ``within(*values)`` holds (steps of equal ones are asked once).
+    bounded: tuple[str, int] | tuple[tuple[str, ...], Callable[..., bool]] | None = None
 
 
 class Operator:

@@ -1169,7 +1169,7 @@ class CompiledGraph:
         # What a step's launch may read of the call's context: ``bounded`` while every step that has a
         # cheaper form within a limit (``Built.bounded``) is being launched, or captured, in that form.
         self._context: dict[str, Any] = {"bounded": False}
-        self._bounds: list[tuple[Affine, int]] = []   # (per-call expression, limit) of those steps
+        self._bounds: list[tuple[tuple[Affine, ...], Any]] = []   # (per-call expressions, limit or what holds within it) of those steps
         self._launches: list = []
 
     def _slot(self, expr: Affine) -> int:
@@ -1283,9 +1283,14 @@ class CompiledGraph:
                 )
         if views:
             words = {**words, "__views__": views}
-        if built.bounded is not None and built.bounded[0] in step.values:
-            self._bounds.append((step.values[built.bounded[0]], int(built.bounded[1])))
-            words = {**words, "__context__": self._context}
+        if built.bounded is not None:
+            names, limit = built.bounded
+            names = (names,) if isinstance(names, str) else names
+            if all(n in step.values for n in names):
+                bound = (tuple(step.values[n] for n in names), limit)
+                if bound not in self._bounds:
+                    self._bounds.append(bound)
+                words = {**words, "__context__": self._context}
         slot = self._carry_by_draw.get(self.recording.steps.index(step)) if self._carry_by_draw else None
         if slot is not None:
             words = {**words, "__carry_token__": self.words[slot : slot + 1]}
@@ -1397,7 +1402,7 @@ class CompiledGraph:
     def _within_bounds(self, values: Mapping[str, int]) -> bool:
         """Whether every step with a bounded form stays within its limit at these per-call values."""
         at = {**values, "__const__": 0}
-        return all(expr.evaluate(at) <= limit for expr, limit in self._bounds)
+        return all(limit(*(e.evaluate(at) for e in exprs)) if callable(limit) else exprs[0].evaluate(at) <= limit for exprs, limit in self._bounds)
 
     def _replay_at(self, values: Mapping[str, int]) -> None:
         """One replay of the captured step from ``values`` (already on the device): the bounded
@@ -1501,7 +1506,9 @@ class CompiledGraph:
             if self.check:
                 self._run_checked(full)
             else:
+                self._context["bounded"] = bool(self._bounds) and self._within_bounds(full)
                 self._run_steps()
+                self._context["bounded"] = False
         outs = []
         for h, t in zip(rec.outputs, self.output_tensors):
             rows = h.valid[0].evaluate(full) if 0 in h.valid else None

@@ -258,6 +258,75 @@ __device__ __forceinline__ void prefill_few_rows(
                      pack_bf16(oacc[dt][4 * q + 2] * inv, oacc[dt][4 * q + 3] * inv));
 }
 
+// How a launch deals keys over blocks (DEALT below): a block has 128 queries of one KV head, those of all its query heads in turn, and one of `slices` slices of the
+// key tiles that they see.  `blocks`: a KV head's, by queries.  The launch is for few queries over many keys, whose blocks leave CUs without one: as many slices as
+// give each CU one block, or two where that is the less by what was measured, a step of a block's two tiles 1.2 us, of two on a CU 2.05, and a block's part out and
+// back 0.017; no slice of fewer tiles than kSliceTiles.  Us, 32 / 8 heads of 64, a block a CU and two (or as many of them as there are): 200 queries, 7000 keys 27.6 / 29.5,
+// 12043 42.9 / 38.4; 450, 4500 32.9 / 35.7, 12043 71.2 / 62; 600, 7000 64 / 51; 1000, 7000 69.5 / 71.5, 12043 127 / 114; 40 queries, slices of 6 tiles and of 12 at the least,
+// 3000 keys 15.4 / 18.1.
+struct PrefillDeal {
+  int blocks, slices;
+};
+constexpr int kSliceTiles = 6;
+constexpr int kDealtBlocks64 = 512, kDealtBlocks128 = 256;   // eight-wave blocks the chip holds at once
+template <int D>
+__device__ __forceinline__ PrefillDeal prefill_deal(int q_tokens, int kv_tokens, int heads, int group, int window) {
+  const int blocks = (q_tokens * group + BQ - 1) / BQ, all = max(1, blocks * (heads / group));
+  const int seen = window < 0 ? kv_tokens : min(kv_tokens, window + q_tokens), tiles = (seen + BKV - 1) / BKV, most = max(1, tiles / kSliceTiles);
+  const int one = max(1, min(kCUs / all, most)), two = D == 64 ? max(1, min(2 * kCUs / all, most)) : one;
+  const int some = min(tiles, 1 << 20);   // (in ns, whole numbers: both kernels have to come to the same)
+  const int ns1 = 600 * some / one + (one > 1 ? 17 * all * one : 0), ns2 = 1025 * some / two + (two > 1 ? 17 * all * two : 0);
+  return PrefillDeal{blocks, two > one && all * two > kCUs && ns2 < ns1 ? two : one};
+}
+
+// ... and the slices' parts of each query together.  Items: (KV head and query block, four columns, query).
+template <int D>
+__global__ __launch_bounds__(256) void mha_prefill_merge_kernel(const float* __restrict__ part, bf16_t* __restrict__ O, int heads, int group, int seq,
+                                                                int seq_len, int kv_len, float scale_log2, int masked, int window, long q_row_stride, long q_head_stride,
+                                                                const int* __restrict__ valid, const int* __restrict__ kv_valid) {
+  const int q_tokens = valid ? bound_or(valid, seq) : seq_len;
+  const int kv_tokens = kv_valid ? bound_or(kv_valid, kv_len) : (kv_len - seq + q_tokens);
+  const PrefillDeal deal = prefill_deal<D>(q_tokens, kv_tokens, heads, group, window);
+  if (deal.slices <= 1 || (masked && kv_tokens < q_tokens)) return;
+  constexpr int QUADS = D / 4, AHEAD = 4;
+  const int items = heads / group * deal.blocks * QUADS * BQ;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < items; i += gridDim.x * 256) {
+    const int in_block = i % BQ, quad = i / BQ % QUADS, unit = i / (BQ * QUADS), kvh = unit / deal.blocks;
+    const int nth = (unit - kvh * deal.blocks) * BQ + in_block, row = nth / group;
+    const float* from = part + (size_t)unit * deal.slices * (BQ * (D + 2)) + in_block;
+    float top = -INFINITY, sum = 0.f;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < deal.slices; s0 += AHEAD) {
+      float m[AHEAD], l[AHEAD];
+      f32x4 o[AHEAD];
+#pragma unroll
+      for (int s = 0; s < AHEAD; ++s) {   // (past the last: the last again, without weight)
+        const float* p = from + (size_t)min(s0 + s, deal.slices - 1) * (BQ * (D + 2));
+        m[s] = p[0];
+        l[s] = p[BQ];
+        o[s] = *reinterpret_cast<const f32x4*>(p - in_block + 2 * BQ + (quad * BQ + in_block) * 4);
+      }
+      float now = top;
+#pragma unroll
+      for (int s = 0; s < AHEAD; ++s) now = fmaxf(now, m[s]);
+      const float ref = now == -INFINITY ? 0.f : now * scale_log2, fade = top == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(fmaf(top, scale_log2, -ref));
+      sum *= fade;
+      acc *= fade;
+#pragma unroll
+      for (int s = 0; s < AHEAD; ++s) {
+        const float w = s0 + s < deal.slices && m[s] != -INFINITY ? __builtin_amdgcn_exp2f(fmaf(m[s], scale_log2, -ref)) : 0.f;
+        sum = fmaf(l[s], w, sum);
+        acc += o[s] * w;
+      }
+      top = now;
+    }
+    if (row >= q_tokens) continue;
+    const float inv = sum > 0.f ? 1.0f / sum : 0.f;
+    *reinterpret_cast<uint2*>(O + (size_t)(kvh * group + nth - row * group) * q_head_stride + (size_t)row * q_row_stride + quad * 4) =
+        make_uint2(pack_bf16(acc[0] * inv, acc[1] * inv), pack_bf16(acc[2] * inv, acc[3] * inv));
+  }
+}
+
 // K and V tiles go straight from global memory into LDS (buffer loads with the LDS bit, no register staging), as
 // stored: [64 keys][D], STAGES tiles deep.  16-byte chunks of a row are XOR-swizzled so unpadded
 // rows read without bank conflicts: K by k_swizzle for its 16-byte fragment reads, V by
@@ -278,13 +347,13 @@ __device__ __forceinline__ void prefill_few_rows(
 //
 // W: the waves that share a tile's loads, each with 32 of the block's 32 W queries.  Four; two
 // where four would leave CUs without a block (a short prompt), so that twice as many blocks go out.
-template <int D, int SPLIT, int W, bool FEW, bool FINE>
+template <int D, int SPLIT, int W, bool FEW, bool FINE, bool DEALT>
 __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(W == 4 ? (D == 64 && SPLIT == 2 ? 4 : 2) : 2))) void mha_prefill_kernel(
     const bf16_t* __restrict__ Q, const bf16_t* __restrict__ K, const bf16_t* __restrict__ V,
     bf16_t* __restrict__ O, int heads, int group, int seq, int seq_len, int kv_len, float scale_log2,
     int causal, int window, long q_row_stride, long q_head_stride, long kv_row_stride,
     long kv_head_stride, const int* __restrict__ valid, const int* __restrict__ kv_valid,
-    const int* __restrict__ kv_first, int kv_rows) {
+    const int* __restrict__ kv_first, int kv_rows, float* __restrict__ part) {
   constexpr int ROWB = D * 2;            // bytes of a tile row
   constexpr int KS = D / 16;             // k16 steps of S^T
   constexpr int DT = D / 32;             // 32-row tiles of O^T
@@ -314,21 +383,30 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
   // together: the long blocks start first and the short ones fill the tail.  Within a query block
   // the heads are dealt so that an XCD (block id mod 8) serves the heads of one KV group, whose
   // K and V it then reads from its own L2.
-  const int j = blockIdx.x % heads;
-  const int head = (heads % 8 == 0) ? (j % 8) * (heads / 8) + j / 8 : j;
-  const int kvh = head / group;
+  // (DEALT: a block's queries are those of all a KV head's heads, and its keys a slice of what they see, see prefill_deal.)
+  const int columns = DEALT ? __builtin_amdgcn_readfirstlane(heads / group) : heads, j = DEALT ? __builtin_amdgcn_readfirstlane(blockIdx.x % columns) : blockIdx.x % columns;
+  const int head_of_block = DEALT ? 0 : ((heads % 8 == 0) ? (j % 8) * (heads / 8) + j / 8 : j);
+  const int kvh = DEALT ? j : head_of_block / group;
   // A launch whose blocks are all resident two a CU (more blocks than CUs, no more than twice as
   // many): the second half of the ids runs from the lightest query block up, so the two blocks a CU
   // holds -- ids i and i + 256 -- are a heavy one and a light one, and every CU has the same work.
-  const int nqb = (int)(gridDim.x / heads), at = (int)(blockIdx.x / heads);
+  const int nqb = (int)(gridDim.x / columns), at = DEALT ? __builtin_amdgcn_readfirstlane(blockIdx.x / columns) : (int)(blockIdx.x / columns);
   const bool folded = causal && gridDim.x > kCUs && gridDim.x <= 2 * kCUs && SPLIT == 2 && W == 4 && D == 64;
-  const int qb = folded && at >= (nqb + 1) / 2 ? at - (nqb + 1) / 2 : nqb - 1 - at;
-  const int q0 = qb * BQW;
-
   const int q_tokens = valid ? bound_or(valid, seq) : seq_len;
   const int kv_tokens = kv_valid ? bound_or(kv_valid, kv_len) : (kv_len - seq + q_tokens);
   const bool masked_any = causal || window >= 0;
   const int offset = masked_any ? (kv_tokens - q_tokens) : 0;
+  // (what a division makes is made in vector registers: brought back, or each holds one through the whole loop)
+  auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+  PrefillDeal deal{nqb, 1};
+  int qb = folded && at >= (nqb + 1) / 2 ? at - (nqb + 1) / 2 : nqb - 1 - at, slice = 0;
+  if constexpr (DEALT) {
+    deal = prefill_deal<D>(q_tokens, kv_tokens, heads, group, window);
+    deal = PrefillDeal{uniform(deal.blocks), uniform(deal.slices)};
+    qb = uniform(at / deal.slices);
+    slice = at - qb * deal.slices;
+    qb = deal.blocks - 1 - qb;
+  }
 
   // Few live queries (FEW: the launch may have them; the code beside the tiles' costs those 1.5 to 2.5 % at d = 128): groups of 32 take the first blocks, all blocks the zeros of the rows past them.
   const int groups = FEW ? (q_tokens + 31) >> 5 : 0;
@@ -346,21 +424,34 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
     if (at >= groups) return;
     const long first_row = kv_first ? max(0, min(*kv_first, kv_rows - kv_len)) : 0;
     const size_t kv_at = (size_t)kvh * kv_head_stride + first_row * kv_row_stride;
-    prefill_few_rows<D, W * SPLIT>(smem_all, Q + (size_t)head * q_head_stride, K + kv_at, V + kv_at, O + (size_t)head * q_head_stride,
+    prefill_few_rows<D, W * SPLIT>(smem_all, Q + (size_t)head_of_block * q_head_stride, K + kv_at, V + kv_at, O + (size_t)head_of_block * q_head_stride,
                                    (groups - 1 - at) * 32, seq, q_tokens, kv_tokens, offset, scale_log2, causal, window,
                                    q_row_stride, kv_row_stride);
     return;
   }
 
-  const int my_q = q0 + wave * 32 + col;            // this lane's query row
+  // This lane's query row and head, and the first rows of the block and of the wave (DEALT: query `nth` of a KV head is head nth % group's of row nth / group).
+  const int nth = qb * BQW + wave * 32 + col;
+  const int my_q = DEALT ? nth / group : nth;
+  const int head = DEALT ? kvh * group + nth - my_q * group : head_of_block;
+  const int q0 = DEALT ? uniform(qb * BQW / group) : qb * BQW, wq0 = DEALT ? uniform((qb * BQW + wave * 32) / group) : q0 + wave * 32;
+  const int q_last = min(DEALT ? uniform((qb * BQW + BQW - 1) / group) : q0 + BQW - 1, q_tokens - 1);
+  const int wq_last = min(DEALT ? uniform((qb * BQW + wave * 32 + 31) / group) : wq0 + 31, q_tokens - 1);
   const bool q_live = my_q < q_tokens;
   const int qpos = offset + my_q;
-  const int wq_lo = offset + q0 + wave * 32;        // positions of the wave's first and last live query
-  const int wq_hi = offset + min(q0 + wave * 32 + 31, q_tokens - 1);
+  const int wq_lo = offset + wq0;        // positions of the wave's first and last live query
+  const int wq_hi = offset + wq_last;
 
   bf16_t* Oh = O + (size_t)head * q_head_stride;
-  // Rows of this block past the bound: zeros.  A block wholly past it does only that.
-  if (q0 >= q_tokens || offset < 0) {
+  // Rows past the bound: zeros.  A block wholly past it does only that.
+  if constexpr (DEALT) {
+    const int from = offset < 0 ? 0 : q_tokens, all = (seq - from) * heads * CPR;
+    for (int i = blockIdx.x * (64 * W * SPLIT) + tid; i < all; i += gridDim.x * (64 * W * SPLIT)) {
+      const int r = i / (heads * CPR), c = i - r * (heads * CPR), h = c / CPR;
+      *reinterpret_cast<uint4*>(O + (size_t)h * q_head_stride + (size_t)(from + r) * q_row_stride + (c - h * CPR) * 8) = make_uint4(0, 0, 0, 0);
+    }
+    if (offset < 0 || at >= deal.blocks * deal.slices) return;
+  } else if (q0 >= q_tokens || offset < 0) {
     for (int i = tid; i < BQW * CPR; i += 64 * W * SPLIT) {
       const int r = q0 + i / CPR, c = (i % CPR) * 8;
       if (r < seq) *reinterpret_cast<uint4*>(Oh + (size_t)r * q_row_stride + c) = make_uint4(0, 0, 0, 0);
@@ -389,13 +480,17 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
   float mc = 0.f;                         // the reference in the exp2 domain, 0 while it is -inf
 
   // Keys this block's live queries can see.
-  const int q_last = min(q0 + BQW, q_tokens) - 1;
   int kv_hi = kv_tokens;
   if (causal) kv_hi = min(kv_hi, offset + q_last + 1);
   else if (window >= 0) kv_hi = min(kv_hi, offset + q_last + window + 1);
   int kv_lo = 0;
   if (window >= 0) kv_lo = max(0, offset + q0 - window) / BKV * BKV;
-  const int ntiles = (kv_hi - kv_lo + BKV - 1) / BKV;
+  int ntiles = (kv_hi - kv_lo + BKV - 1) / BKV;
+  if constexpr (DEALT) {   // ... of which the block has a slice
+    const int from = uniform(slice * ntiles / deal.slices), to = uniform((slice + 1) * ntiles / deal.slices);
+    kv_lo += from * BKV;
+    ntiles = to - from;
+  }
   // This half's tiles are half, half + SPLIT, ...; both halves make the same number of steps (a
   // block's waves share its barriers), the last of which may be past this half's last tile: it
   // then loads the last tile again and computes nothing.
@@ -708,6 +803,7 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
     const float mc = (m_new == -INFINITY) ? 0.f : m_new * scale_log2;
     const float a_mine = __builtin_amdgcn_exp2f(fmaf(m_run, scale_log2, -mc));      // exp2(-inf) = 0: a half
     const float a_other = __builtin_amdgcn_exp2f(fmaf(m_other, scale_log2, -mc));   // that saw no key
+    if (DEALT) m_run = m_new;
     l_run = l_run * a_mine + l_other * a_other;
 #pragma unroll
     for (int t = 0; t < DT; ++t)
@@ -717,6 +813,37 @@ __global__ __launch_bounds__(64 * W * SPLIT) __attribute__((amdgpu_waves_per_eu(
 
   // Normalize and store: lane holds query `col`, columns 32 dt + 8 q + 4 g + 0..3.
   const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+  if constexpr (DEALT) {
+    // (What depends on the lane is made again: held through the loop, some of it spilled.)
+    int l = threadIdx.x;
+    asm volatile("" : "+v"(l));
+    const int gl = (l >> 5) & 1, in_block = wave * 32 + (l & 31);
+    if (deal.slices > 1) {   // the merge's part: the queries' references and sums, then four columns of each
+      float* to = part + ((size_t)(kvh * deal.blocks + qb) * deal.slices + slice) * (BQW * (D + 2));
+      if (gl == 0) {
+        to[in_block] = m_run;
+        to[BQW + in_block] = l_tot;
+      }
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<float4*>(to + 2 * BQW + ((8 * dt + 2 * q + gl) * BQW + in_block) * 4) =
+              make_float4(oacc[dt][4 * q], oacc[dt][4 * q + 1], oacc[dt][4 * q + 2], oacc[dt][4 * q + 3]);
+      return;
+    }
+    const int at_query = qb * BQW + in_block, row = at_query / group;
+    if (row >= q_tokens) return;   // (zeroed above)
+    const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+    bf16_t* op = O + (size_t)(kvh * group + at_query - row * group) * q_head_stride + (size_t)row * q_row_stride;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<uint2*>(op + 32 * dt + 8 * q + 4 * gl) =
+            make_uint2(pack_bf16(oacc[dt][4 * q] * inv, oacc[dt][4 * q + 1] * inv), pack_bf16(oacc[dt][4 * q + 2] * inv, oacc[dt][4 * q + 3] * inv));
+    return;
+  }
   const float inv = (q_live && l_tot > 0.f) ? 1.0f / l_tot : 0.f;
   if (my_q < seq) {
     // (The row's address is made here: computed where its inputs first are, it is 64 bits a lane held
@@ -1045,18 +1172,18 @@ struct PrefillArgs {
 };
 
 // The stage buffers are dynamic LDS (more than the 64 KB a kernel may declare statically).
-template <int D, int SPLIT, int W, bool FEW, bool FINE>
-static int launch_prefill_as(const PrefillArgs& a, int blocks, void* stream) {
+template <int D, int SPLIT, int W, bool FEW, bool FINE, bool DEALT = false>
+static int launch_prefill_as(const PrefillArgs& a, int blocks, void* stream, float* part = nullptr) {
   constexpr int STAGES = D == 64 && SPLIT == 1 ? 3 : 2;
   constexpr size_t lds = (size_t)SPLIT * STAGES * 2 * BKV * D * 2;
   static LdsOptIn opt_in;
-  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&mha_prefill_kernel<D, SPLIT, W, FEW, FINE>), lds); e != hipSuccess) {
+  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&mha_prefill_kernel<D, SPLIT, W, FEW, FINE, DEALT>), lds); e != hipSuccess) {
     set_error("mha_prefill: %s", hipGetErrorString(e));
     return (int)e;
   }
-  hipLaunchKernelGGL((mha_prefill_kernel<D, SPLIT, W, FEW, FINE>), dim3(blocks), dim3(64 * W * SPLIT), lds, (hipStream_t)stream, a.Q,
+  hipLaunchKernelGGL((mha_prefill_kernel<D, SPLIT, W, FEW, FINE, DEALT>), dim3(blocks), dim3(64 * W * SPLIT), lds, (hipStream_t)stream, a.Q,
                      a.K, a.V, a.O, a.heads, a.group, a.seq, a.seq_len, a.kv_len, a.scale_log2, a.causal, a.window,
-                     a.q_row, a.q_head, a.kv_row, a.kv_head, a.valid, a.kv_valid, a.kv_first, a.kv_rows);
+                     a.q_row, a.q_head, a.kv_row, a.kv_head, a.valid, a.kv_valid, a.kv_first, a.kv_rows, part);
   return 0;
 }
 
@@ -1101,6 +1228,16 @@ static bool split_128(const PrefillArgs& a, int blocks) {
   return 2 * blocks < 1000 + 13 * (blocks / a.heads);
 }
 
+template <int D>
+static int launch_prefill_dealt(const PrefillArgs& a, float* part, void* stream) {
+  const int columns = a.heads / a.group, blocks = ((int)(((long)a.seq * a.group + BQ - 1) / BQ)) * columns, room = (D == 64 ? kDealtBlocks64 : kDealtBlocks128) / columns * columns;   // (slices are dealt only where they fit)
+  const int rc = launch_prefill_as<D, 2, 4, false, false, true>(a, blocks > room ? blocks : room, stream, part);
+  if (rc != 0) return rc;
+  hipLaunchKernelGGL(mha_prefill_merge_kernel<D>, dim3(512), dim3(256), 0, (hipStream_t)stream, part, a.O, a.heads, a.group, a.seq, a.seq_len, a.kv_len, a.scale_log2,
+                     a.causal || a.window >= 0, a.window, a.q_row, a.q_head, a.valid, a.kv_valid);
+  return 0;
+}
+
 template <int D, int QN, int W>
 static int launch_prefill_wide(const PrefillArgs& a, void* stream) {
   constexpr size_t lds = (size_t)2 * 2 * 32 * D * 2;   // two stages of a 32-key K tile and V tile
@@ -1124,7 +1261,7 @@ using namespace iron;
 static int mha_prefill(const uint16_t* Q, const uint16_t* K, const uint16_t* V, uint16_t* O, int heads, int kv_heads,
                        int d, int seq, int seq_len, int kv_len, float scale, int causal, int window, int q_interleaved,
                        int kv_interleaved, const int* valid, const int* kv_valid, const int* kv_first, int kv_rows,
-                       void* stream) {
+                       void* stream, float* part = nullptr) {
   IRON_REQUIRE(Q && K && V && O, "mha_prefill: null operand");
   IRON_REQUIRE(kv_first == nullptr || (kv_interleaved && kv_rows >= kv_len),
                "mha_prefill: a window of the keys takes them row by row (kv_interleaved) out of kv_rows (%d) >= kv_len (%d)",
@@ -1152,6 +1289,11 @@ static int mha_prefill(const uint16_t* Q, const uint16_t* K, const uint16_t* V, 
   PrefillArgs a{Q, K, V, O, heads, heads / kv_heads, seq, seq_len, kv_len, scale_log2, causal, window,
                 q_row, q_head, kv_row, kv_head, valid, kv_valid, kv_first, kv_rows};
   int rc;
+  if (part != nullptr) {
+    rc = d == 64 ? launch_prefill_dealt<64>(a, part, stream) : launch_prefill_dealt<128>(a, part, stream);
+    if (rc != 0) return rc;
+    IRON_LAUNCH_CHECK();
+  }
   // Wide heads: 16-query groups on 16x16x32 tiles.  Blocks of 128 queries (eight waves) once those
   // fill the chip twice over, of 64 (four waves) below that; at 256, where two groups a wave fit the
   // registers, launches of a thousand blocks and more take two (half the LDS reads a flop: 32 heads at
@@ -1192,4 +1334,19 @@ extern "C" int iron_mha_prefill_at_bf16(const uint16_t* Q, const uint16_t* K, co
   IRON_REQUIRE(kv_first != nullptr, "mha_prefill_at: null kv_first");
   return mha_prefill(Q, K, V, O, heads, kv_heads, d, seq, seq_len, kv_len, scale, causal, window, q_interleaved, 1,
                      valid, kv_valid, kv_first, kv_rows, stream);
+}
+
+extern "C" int64_t iron_mha_prefill_dealt_workspace_bytes(int heads, int kv_heads, int d) {
+  if (heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0 || (d != 64 && d != 128)) return 0;
+  return (int64_t)(d == 64 ? kDealtBlocks64 : kDealtBlocks128) * BQ * (d + 2) * sizeof(float);
+}
+
+extern "C" int iron_mha_prefill_dealt_bf16(const uint16_t* Q, const uint16_t* K, const uint16_t* V, uint16_t* O, int heads, int kv_heads, int d, int seq, int seq_len,
+                                           int kv_len, float scale, int causal, int window, int q_interleaved, int kv_interleaved, const int* valid,
+                                           const int* kv_valid, void* workspace, void* stream) {
+  IRON_REQUIRE(workspace != nullptr && ((uintptr_t)workspace & 15) == 0, "mha_prefill_dealt: a workspace, 16-byte aligned");
+  IRON_REQUIRE(iron_mha_prefill_dealt_workspace_bytes(heads, kv_heads, d) > 0, "mha_prefill_dealt: d (%d) is 64 or 128, heads (%d) a multiple of kv_heads (%d)", d, heads, kv_heads);
+  IRON_REQUIRE(seq > 0 && (int64_t)seq * heads * (d / 8) < (1L << 31), "mha_prefill_dealt: %d rows of %d heads are more than its counters hold", seq, heads);
+  return mha_prefill(Q, K, V, O, heads, kv_heads, d, seq, seq_len, kv_len, scale, causal, window, q_interleaved, kv_interleaved, valid, kv_valid, nullptr, 0, stream,
+                     (float*)workspace);
 }

@@ -442,6 +442,31 @@ def mha_prefill(
     )
 
 
+def mha_prefill_dealt_workspace(heads, kv_heads, d, device="cuda"):
+    return torch.empty(lib().iron_mha_prefill_dealt_workspace_bytes(heads, kv_heads, d) // 4, dtype=torch.float32, device=device)
+
+
+def mha_prefill_dealt(Q, K, V, O, workspace, *, heads, kv_heads, d, seq, seq_len=None, kv_len, scale=None, causal=True, window=None,
+                      q_interleaved=False, kv_interleaved=False, valid=None, kv_valid=None):
+    """``mha_prefill`` for few queries over many keys (d 64 or 128): the keys dealt over blocks, whose parts meet by way of
+    ``workspace`` (any contents) in a second launch."""
+    _numel(_dev(Q, "Q"), seq * heads * d, "Q")
+    _numel(_dev(O, "O"), seq * heads * d, "O")
+    _numel(_dev(K, "K"), kv_len * kv_heads * d, "K")
+    _numel(_dev(V, "V"), kv_len * kv_heads * d, "V")
+    need = lib().iron_mha_prefill_dealt_workspace_bytes(heads, kv_heads, d)
+    if need and _dev(workspace, "workspace", None).numel() * workspace.element_size() < need:
+        raise ValueError(f"mha_prefill_dealt: workspace holds {workspace.numel() * workspace.element_size()} bytes, {need} needed")
+    check(
+        lib().iron_mha_prefill_dealt_bf16(
+            ptr(Q), ptr(K), ptr(V), ptr(O), heads, kv_heads, d, seq, seq if seq_len is None else seq_len, kv_len,
+            1.0 / math.sqrt(d) if scale is None else float(scale), int(causal), -1 if window is None else int(window), int(q_interleaved),
+            int(kv_interleaved), ptr(_word(valid, "valid")), ptr(_word(kv_valid, "kv_valid")), ptr(workspace), current_stream(),
+        ),
+        "iron_mha_prefill_dealt_bf16",
+    )
+
+
 def _window(K, V, kv_rows, kv_len, kv_heads, d, kv_interleaved):
     if not kv_interleaved or kv_rows is None or kv_rows < kv_len:
         raise ValueError(f"a window of the keys takes them row by row (kv_interleaved) out of kv_rows ({kv_rows}) "

@@ -9,6 +9,8 @@ not the cache.
 
 from __future__ import annotations
 
+import dataclasses
+
 import numpy as np
 
 from ..common.declare import Built, In, Operator, Out, Scratch, Select, ceildiv, param, per_call, tunable
@@ -18,6 +20,27 @@ from ..common.verify import Tolerance
 # One query: up to this many live keys one launch does it all (a block a query head); a cache that can
 # hold more takes the launch whose blocks choose by the live keys, and a merge launch behind it.
 SHORT_KEYS = 2048
+
+
+@dataclasses.dataclass(frozen=True)
+class WholeKeys:
+    """Whether a call of ``valid`` queries over ``kv_valid`` keys takes the launch whose blocks see all their keys,
+    rather than the one that deals them over blocks with a merge behind it.
+
+    Dealt, few queries over many keys give every CU work: 32 / 8 heads of 64, 40 queries over 12043 keys 64 -> 21 us, 600 over
+    7000 65 -> 51, 857 over 12043 131 -> 105, 1400 over 7000 100.6 -> 99.1 (past those blocks a launch fills the chip alone: 2048 over 6144 98 / 100).
+    By keys: from 6144 on with up to 352 blocks of 128 queries; from 4096 on with up to 40 (16 / 4 heads, 300 queries over 4200 26.7 ->
+    20.4; but 32 heads, 200 21.8 / 23.5); from 2560 on with up to 24 (40 queries, 32 heads over 2600 16.3 -> 15.3, 90 16.6 -> 16.4; 300 of 24 heads
+    19.9 / 21.1).  Heads of 128 gain more at each."""
+
+    heads: int
+
+    def __call__(self, valid: int, kv_valid: int) -> bool:
+        blocks = valid * self.heads / 128
+        return not (kv_valid >= 2560 and blocks <= (352 if kv_valid >= 6144 else 40 if kv_valid >= 4096 else 24))
+
+
+DEALT_KEYS = 2560   # the fewest keys that are dealt
 
 _CASES = [
     Case(dict(num_heads=1, seq_len=16384), bench=True),
@@ -61,23 +84,32 @@ class MHA(Operator):
     B_q: int = tunable()
     num_pipelines: int = tunable(default=1)
     pv_cores: int = tunable(repr=False)
+    # Many queries over a cache: keys may be dealt over blocks (``WholeKeys``).
+    deals: bool = param(derive=lambda op: op._deals(), repr=False, init=False)
+    scratched: bool = param(derive=lambda op: op.packed or op.deals, repr=False, init=False)
     workspace_words: int = param(derive=lambda op: op._workspace_words(), repr=False)
 
     Q = In(Select(heads_interleaved, (seq_pad, num_heads, d), (num_heads, seq_pad, d)))
     K = In(Select(kv_interleaved, (kv_len, num_KV_heads, d), (num_KV_heads, kv_len, d)))
     V = In(Select(kv_interleaved, (kv_len, num_KV_heads, d), (num_KV_heads, kv_len, d)))
     O = Out(Select(heads_interleaved, (seq_pad, num_heads, d), (num_heads, seq_pad, d)))  # noqa: E741
-    # Split-KV partial results of the one-query kernel.
-    workspace = Scratch(workspace_words, dtype=np.float32, when=packed)
+    # Partial results of the kernels that deal the keys over blocks.
+    workspace = Scratch(workspace_words, dtype=np.float32, when=scratched)
     # A bound on the queries limits the compute; a bound on the keys limits K's and V's rows.
     valid = per_call(bounds=seq_pad)
     kv_valid = per_call(bounds=kv_len)
 
+    def _deals(self) -> bool:
+        return (not self.packed and self.heads_interleaved and self.kv_interleaved and self.kv_len >= DEALT_KEYS and self.d in (64, 128)
+                and (self.window is None or self.window >= self.kv_len) and self.seq_pad * self.num_heads * (self.d // 8) < 2**31)
+
     def _workspace_words(self) -> int:
-        if self.seq_len != 1:
+        if not self.scratched:
             return 0
         from .._lib import lib
 
+        if self.deals:
+            return int(lib().iron_mha_prefill_dealt_workspace_bytes(self.num_heads, self.num_KV_heads, self.d)) // 4
         return int(lib().iron_mha_decode_workspace_bytes(self.num_heads, self.d)) // 4
 
     def seq_padding(self, seq_len: int) -> int:
@@ -203,14 +235,21 @@ class MHA(Operator):
             return Built("iron_mha_decode_bf16", launch, bounded)
         seq, seq_len, causal = self.seq_pad, self.seq_len, self.causal
         qi, kvi = self.heads_interleaved, self.kv_interleaved
+        bounded = (("valid", "kv_valid"), WholeKeys(H)) if self.deals else None
 
         def launch(t, words):
+            ring, context, ws = _key_window(words, G * d), words.get("__context__"), t.get("workspace")
+            if bounded and ws is not None and context is not None and not context.get("bounded") and not ring:
+                kernels.mha_prefill_dealt(t["Q"], t["K"], t["V"], t["O"], ws, heads=H, kv_heads=G, d=d, seq=seq, seq_len=seq_len, kv_len=L,
+                                          scale=scale, causal=causal, window=window, q_interleaved=qi, kv_interleaved=kvi,
+                                          valid=words.get("valid"), kv_valid=words.get("kv_valid"))
+                return
             kernels.mha_prefill(t["Q"], t["K"], t["V"], t["O"], heads=H, kv_heads=G, d=d, seq=seq,
                                 seq_len=seq_len, kv_len=L, scale=scale, causal=causal, window=window,
                                 q_interleaved=qi, kv_interleaved=kvi, valid=words.get("valid"),
-                                kv_valid=words.get("kv_valid"), **_key_window(words, G * d))
+                                kv_valid=words.get("kv_valid"), **ring)
 
-        return Built("iron_mha_prefill_bf16", launch)
+        return Built("iron_mha_prefill_bf16", launch, bounded)
 
 
 def _key_window(words, row: int) -> dict:

@@ -1192,6 +1192,50 @@ def test_mha_prefill_of_few_rows_over_many_keys(cuda, H, G, d, S, rows, L, keys,
         close(got[r : r + 1], want)
 
 
+# Queries of 4, 3, 1 and 8 heads a KV head: one, a block of 128 (row, head) pairs and one row more, one and one that a block's edge cuts; one slice, two, as many
+# as there are CUs, two blocks a CU (600 over 7000); slices that see no tile of the first queries'; windows, no mask; both layouts' strides in Q.
+@pytest.mark.parametrize("H,G,d,S,rows,L,keys,window,causal", [
+    (32, 8, 64, 256, 1, 4096, 3001, None, True), (32, 8, 64, 256, 32, 4096, 2560, None, True), (32, 8, 64, 256, 33, 4096, 4000, None, True),
+    (24, 8, 64, 200, 43, 3000, 2999, None, True), (12, 4, 128, 130, 129, 4000, 3900, None, True), (8, 8, 128, 64, 64, 2600, 2600, None, True),
+    (8, 1, 64, 64, 17, 2600, 2561, None, False), (32, 8, 64, 2048, 600, 7168, 7000, None, True), (4, 1, 64, 800, 800, 800, 800, None, True),
+    (16, 4, 64, 100, 40, 4096, 4096, 1500, True), (6, 2, 64, 300, 70, 3000, 2700, 700, False), (4, 4, 64, 33, 33, 65, 65, None, True),
+    (32, 8, 128, 256, 40, 9000, 8999, None, True)])
+@pytest.mark.parametrize("interleaved", [True, False])
+def test_mha_prefill_dealt_over_blocks(cuda, H, G, d, S, rows, L, keys, window, causal, interleaved):
+    """The keys dealt over blocks and the parts' sums by way of a workspace of NaNs: every head of a sample of rows against the oracle's attention
+    of that one query over the keys its mask leaves it; rows past the bound are zero, NaN past either bound reaches nothing, and the same bits again."""
+    rng = np.random.default_rng(rows + keys)
+    Q, Kc, Vc = bf(rng, S, H, d), bf(rng, L, G, d), bf(rng, L, G, d)
+    Q[rows:], Kc[keys:], Vc[keys:] = np.nan, np.nan, np.nan
+    own = (lambda x: x) if interleaved else (lambda x: np.ascontiguousarray(x.swapaxes(0, 1)))
+    ws = torch.full_like(K.mha_prefill_dealt_workspace(H, G, d, cuda), float("nan"))
+    outs = []
+    for _ in range(2):
+        O = out_like(own(Q).shape, cuda, fill=float("nan"))
+        K.mha_prefill_dealt(dev(own(Q), cuda), dev(own(Kc), cuda), dev(own(Vc), cuda), O, ws, heads=H, kv_heads=G, d=d, seq=S, kv_len=L, causal=causal, window=window,
+                            q_interleaved=interleaved, kv_interleaved=interleaved, valid=word(rows, cuda), kv_valid=word(keys, cuda))
+        outs.append(O)
+    assert torch.equal(*outs)
+    got = own(from_torch(outs[0]).reshape(own(Q).shape))
+    assert np.all(got[rows:] == 0)
+    for r in sorted({0, rows - 1, min(31, rows - 1), min(32, rows - 1), *rng.integers(0, rows, 5).tolist()}):
+        at = (keys - rows if causal or window is not None else 0) + r   # the query's position
+        last = at + 1 if causal else (min(keys, at + window + 1) if window is not None else keys)
+        first = max(0, at - window) if window is not None else 0
+        want = ops.mha(Q[r : r + 1], Kc[first:last], Vc[first:last], num_heads=H, num_KV_heads=G, seq_len=1, kv_len=last - first, d=d,
+                       causal=False, scale=d**-0.5, heads_interleaved=True, kv_interleaved=True)
+        close(got[r : r + 1], want)
+
+
+def test_mha_prefill_dealt_refuses_other_widths_and_small_workspaces(cuda):
+    t = out_like((64 * 256,), cuda, fill=0.0)
+    assert K.lib().iron_mha_prefill_dealt_workspace_bytes(4, 4, 256) == 0
+    with pytest.raises(ValueError, match="workspace holds"):
+        K.mha_prefill_dealt(t[: 64 * 64], t[: 64 * 64], t[: 64 * 64], t[: 64 * 64], torch.empty(16, device=cuda), heads=1, kv_heads=1, d=64, seq=64, kv_len=64)
+    with pytest.raises(Exception, match="iron_mha_prefill_dealt_bf16 refused"):
+        K.mha_prefill_dealt(t, t, t, t, torch.empty(16, device=cuda), heads=1, kv_heads=1, d=256, seq=64, kv_len=64)
+
+
 # 128-wide heads, more queries than a block of 64 has: all of a launch's in the few-row form, with four waves a block and with eight; one
 # more than that form takes; a second round of blocks that only a causal mask over the queries' own keys allows, and one it does not.
 @pytest.mark.parametrize("H,G,S,rows,L,keys,window,causal", [

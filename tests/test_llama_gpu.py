@@ -468,6 +468,29 @@ def test_prompt_deep_in_the_cache(deep):
     assert kl(want, got) <= 0.1
 
 
+@pytest.mark.parametrize("rows, behind", [(1, 2559), (40, 2520), (95, 2500), (160, 4000), (200, 7000)])
+def test_a_turn_deep_in_the_cache_by_dealt_keys_and_by_whole_ones(deep, rows, behind):
+    """The chunk's graph has both forms of attention, the one that a call's rows and keys choose: a turn behind filled caches by that choice and by
+    blocks that see all their keys, each against the host reference, replayed twice to the same bits."""
+    gpu, cpu, tokens, _ = deep
+    _fill_caches(gpu, cpu, len(tokens), behind)
+    chunk = np.resize(tokens, rows)
+    values = dict(token=int(chunk[-1]), position=behind + rows - 1, start=behind, rows=rows, rope_start=behind)
+    want, _ = cpu(cpu.session.prompt_ids(chunk), **values)
+    want = np.asarray(want.numpy()).ravel()[: gpu.config.vocab_size]
+    version = gpu.prompt_chunk
+    assert version._graph_bounded is not None and len(version._bounds) == 1
+    for within in (version._bounds, [(version._bounds[0][0], lambda *_: True)]):
+        held, version._bounds = version._bounds, within
+        try:
+            runs = [np.array(gpu(gpu.session.prompt_ids(chunk), **values)[0].numpy()).ravel()[: gpu.config.vocab_size] for _ in range(2)]
+        finally:
+            version._bounds = held
+        assert np.array_equal(*runs)
+        assert_close(runs[0], want, f"{rows} rows behind {behind}")
+        assert kl(want, runs[0]) <= 0.1
+
+
 def test_a_5000_token_prompt_in_three_chunks_then_replayed_steps(cuda):
     """Toy width, caches of 8192 rows: a prompt of three chunks (attention over a cache longer than
     the chunk), then eight device-carried decode steps past position 5000 (attention's keys dealt
