@@ -3,11 +3,19 @@
 // selects the k best of its 2048 logits into a list in the workspace; the block that finishes
 // last (a ticket) selects the k best of all lists, its first wave weighs them and one lane walks
 // the running sum.  A selection of k from entries dealt over 256 threads:
-//   1. each thread's best entry; the k-th best of those 256 is a floor no top-k entry is under;
-//   2. every entry at or over the floor goes to a list in LDS (about k of them), which is ranked.
+//   1. each thread's best entry; the k-th best of those 256, or one a few below it, is a floor no top-k entry is under;
+//   2. every entry at or over the floor goes to a list in LDS (about k of them), which the last block ranks.
 // Order everywhere: the larger logit first, of equals the lower index, NaN below every number.
+//
+// Greedy it is two trips to memory and a ticket (an empty launch takes 2 us); a selection on top is a chain of a wave's instructions, four waves
+// a CU, so what counts is how many of them follow each other: a greedy block's best in one word a lane, what the end needs requested at the start; a place in the
+// list asked for once a thread and not once an entry, no branch an entry, a search for the floor that stops when it is near enough, blocks' lists in any order, a
+// quarter of the ranking a wave, no division, the running sum from LDS.  us, before and now: greedy 128256 logits 5.05 / 4.05, 1024 (one block) 2.75 / 2.2; top-50
+// 128256 16.5 / 11.5, 32000 16.0 / 11.3, 1024 7.2 to 10.3 by how far the walk went / 6.3 to 7.1, 500000 35 / 23.8; top-8 at 128256 11.5 / 9.3.
 #include "../../include/iron_hip.h"
 #include "rows.h"
+
+#include <type_traits>
 
 namespace iron {
 
@@ -55,8 +63,9 @@ __device__ __forceinline__ uint64_t collect(const uint64_t* where) {
 
 struct SampleShared {
   __align__(16) uint64_t best[SAMPLE_THREADS];   // each thread's best entry
-  __align__(16) uint64_t list[SAMPLE_LIST];
+  __align__(16) uint64_t list[SAMPLE_LIST + 64];
   uint64_t cand[SAMPLE_K_MAX];
+  int rank[SAMPLE_K_MAX];
   uint64_t slots[SAMPLE_THREADS / 64];
   int listed;
   int last_block;
@@ -78,79 +87,115 @@ __device__ __forceinline__ uint64_t block_max(uint64_t mine, SampleShared& sh) {
   return best;
 }
 
+// The wave's largest, in every lane.
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+  auto with = [&](auto ctrl, auto rows) {   // (see wave_sum; a lane that gets none keeps its own)
+    const uint32_t other = (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+    v = other > v ? other : v;
+  };
+  using std::integral_constant;
+  with(integral_constant<int, 0xB1>(), integral_constant<int, 0xF>());
+  with(integral_constant<int, 0x4E>(), integral_constant<int, 0xF>());
+  with(integral_constant<int, 0x141>(), integral_constant<int, 0xF>());
+  with(integral_constant<int, 0x140>(), integral_constant<int, 0xF>());
+  with(integral_constant<int, 0x142>(), integral_constant<int, 0xA>());
+  with(integral_constant<int, 0x143>(), integral_constant<int, 0xC>());
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 __device__ __forceinline__ int wave_count(bool yes) {
   return __builtin_popcountll(__builtin_amdgcn_ballot_w64(yes));
 }
 
+constexpr int TIES = 6;            // bests past the k-th that a floor may leave: a few more to rank cost less than the search's last steps, up to 19 among equal keys
 constexpr int RANK_PADDED = 128;   // list entries zeroed ahead, so short lists are ranked in whole batches
 
-// The k best of the entries `each(f)` visits over the block's threads (each entry once, none 0,
-// all different), into sh.cand[0..k) from the best; slots past the number of entries are 0.
-template <typename Each>
-__device__ __forceinline__ void select_best(int k, SampleShared& sh, Each&& each) {
+// A floor that at least k and, but for equal keys by the hundred, at most k + TIES of the threads' bests `sh.best` reach (0 if fewer threads hold an entry), found
+// by every wave for itself, a bit at a time from the top: the largest v that k bests reach, or the first that hardly more do.
+__device__ __forceinline__ uint64_t floor_of(int k, const SampleShared& sh) {
+  const int lane = threadIdx.x & 63;
+  const uint64_t b0 = sh.best[lane], b1 = sh.best[lane + 64], b2 = sh.best[lane + 128], b3 = sh.best[lane + 192];
+  // The key's 16 bits on the high words alone; then, while many more than k bests still reach the
+  // floor (equal keys), the index's bits -- from bit 18: an index is under 2^19, so bits 19..31
+  // of its complement are set in every entry and are taken in one step.
+  const uint32_t h0 = (uint32_t)(b0 >> 32), h1 = (uint32_t)(b1 >> 32), h2 = (uint32_t)(b2 >> 32), h3 = (uint32_t)(b3 >> 32);
+  uint32_t high = 0;
+  int reach = SAMPLE_THREADS;
+  for (int bit = 15; bit >= 0 && reach > k + TIES; --bit) {
+    const uint32_t v = high | (1u << bit);
+    const int r = wave_count(h0 >= v) + wave_count(h1 >= v) + wave_count(h2 >= v) + wave_count(h3 >= v);
+    if (r >= k) {
+      high = v;
+      reach = r;
+    }
+  }
+  uint64_t floor = (uint64_t)high << 32;
+  if (high != 0 && reach > k + TIES) {
+    floor |= 0xfff80000u;
+    for (int bit = 18; bit >= 0 && reach > k + TIES; --bit) {
+      const uint64_t v = floor | (1ull << bit);
+      const int r = wave_count(b0 >= v) + wave_count(b1 >= v) + wave_count(b2 >= v) + wave_count(b3 >= v);
+      if (r >= k) {
+        floor = v;
+        reach = r;
+      }
+    }
+  }
+  return floor;
+}
+
+// The k best of the entries `each(f)` visits over the block's threads (each once, all different; 0 is none; `again`: the same, where it may take its time), into sh.cand[0..k) from the best; slots past the number of entries are 0.  Where no more than `any_order` are listed, all of these, in no
+// order and perhaps a few more than k.
+template <typename Each, typename Again>
+__device__ __forceinline__ void select_best(int k, int any_order, SampleShared& sh, Each&& each, Again&& again) {
   uint64_t mine = 0;
   each([&](uint64_t e) { mine = e > mine ? e : mine; });
   __syncthreads();   // whoever read best/list/cand before is done
   sh.best[threadIdx.x] = mine;
-  if (threadIdx.x < SAMPLE_K_MAX) sh.cand[threadIdx.x] = 0;
+  if (threadIdx.x < SAMPLE_K_MAX) {
+    sh.cand[threadIdx.x] = 0;
+    sh.rank[threadIdx.x] = 0;
+  }
   if (threadIdx.x < RANK_PADDED) sh.list[threadIdx.x] = 0;
   if (threadIdx.x == 0) sh.listed = 0;
   __syncthreads();
-  // 1. The floor: the k-th best of the threads' bests (0 if fewer threads hold an entry), found
-  // by every wave for itself, a bit at a time from the top: the largest v that k bests reach.
-  uint64_t floor = 0;
-  {
-    const int lane = threadIdx.x & 63;
-    const uint64_t b0 = sh.best[lane], b1 = sh.best[lane + 64], b2 = sh.best[lane + 128],
-                   b3 = sh.best[lane + 192];
-    // The key's 16 bits on the high words alone; then, while more than k bests still reach the
-    // floor (equal keys), the index's bits -- from bit 18: an index is under 2^19, so bits 19..31
-    // of its complement are set in every entry and are taken in one step.
-    const uint32_t h0 = (uint32_t)(b0 >> 32), h1 = (uint32_t)(b1 >> 32), h2 = (uint32_t)(b2 >> 32),
-                   h3 = (uint32_t)(b3 >> 32);
-    uint32_t high = 0;
-    int reach = SAMPLE_THREADS;
-    for (int bit = 15; bit >= 0 && reach != k; --bit) {
-      const uint32_t v = high | (1u << bit);
-      const int r = wave_count(h0 >= v) + wave_count(h1 >= v) + wave_count(h2 >= v) + wave_count(h3 >= v);
-      if (r >= k) {
-        high = v;
-        reach = r;
-      }
-    }
-    floor = (uint64_t)high << 32;
-    if (high != 0 && reach != k) {
-      floor |= 0xfff80000u;
-      for (int bit = 18; bit >= 0 && reach != k; --bit) {
-        const uint64_t v = floor | (1ull << bit);
-        const int r = wave_count(b0 >= v) + wave_count(b1 >= v) + wave_count(b2 >= v) + wave_count(b3 >= v);
-        if (r >= k) {
-          floor = v;
-          reach = r;
-        }
-      }
-    }
+  // 1. The floor.
+  const uint64_t found = floor_of(k, sh), floor = found != 0 ? found : 1;
+  // 2. The entries at or over it, listed in any order (a thread asks for the places of all of its own at once), then ranked by
+  // counting the better ones.
+  int over = 0;
+  each([&](uint64_t e) { over += e >= floor; });
+  int slot = over != 0 ? atomicAdd(&sh.listed, over) : 0;
+  if (over != 0) {   // (without a branch an entry: one that is not listed goes past the list)
+    const int past = SAMPLE_LIST + (threadIdx.x & 63);
+    each([&](uint64_t e) {
+      const bool in = e >= floor;
+      sh.list[in && slot < SAMPLE_LIST ? slot : past] = e;
+      slot += in;
+    });
   }
-  // 2. The entries at or over it, listed in any order, then ranked by counting the better ones.
-  each([&](uint64_t e) {
-    if (e >= floor) {
-      const int slot = atomicAdd(&sh.listed, 1);
-      if (slot < SAMPLE_LIST) sh.list[slot] = e;
-    }
-  });
   __syncthreads();
   const int m = sh.listed;
-  if (m <= SAMPLE_LIST) {
+  const ulonglong2* pairs = reinterpret_cast<const ulonglong2*>(sh.list);
+  auto better = [&](int j, uint64_t me) {   // of eight of them
+    const ulonglong2 v0 = pairs[j / 2], v1 = pairs[j / 2 + 1], v2 = pairs[j / 2 + 2], v3 = pairs[j / 2 + 3];
+    return (v0.x > me) + (v0.y > me) + (v1.x > me) + (v1.y > me) + (v2.x > me) + (v2.y > me) + (v3.x > me) + (v3.y > me);
+  };
+  if (m <= any_order) {
+    if (threadIdx.x < SAMPLE_K_MAX) sh.cand[threadIdx.x] = sh.list[threadIdx.x];
+  } else if (m <= SAMPLE_K_MAX) {   // a lane an entry, and a wave a quarter of the list
+    static_assert(SAMPLE_THREADS == 4 * 64 && SAMPLE_K_MAX == 64, "four waves' quarters of sixteen");
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint64_t me = sh.list[lane];
+    atomicAdd(&sh.rank[lane], better(16 * wave, me) + better(16 * wave + 8, me));
+    __syncthreads();
+    if ((int)threadIdx.x < m && sh.rank[lane] < k) sh.cand[sh.rank[lane]] = me;
+  } else if (m <= SAMPLE_LIST) {
     const int whole = (m <= RANK_PADDED - 8 ? m + 7 : m) & ~7;   // zeros past a short list rank nothing
-    const ulonglong2* pairs = reinterpret_cast<const ulonglong2*>(sh.list);
     for (int i = threadIdx.x; i < m; i += SAMPLE_THREADS) {
       const uint64_t me = sh.list[i];
       int rank = 0, j = 0;
-      for (; j < whole; j += 8) {
-        const ulonglong2 v0 = pairs[j / 2], v1 = pairs[j / 2 + 1], v2 = pairs[j / 2 + 2], v3 = pairs[j / 2 + 3];
-        rank += (v0.x > me) + (v0.y > me) + (v1.x > me) + (v1.y > me) + (v2.x > me) + (v2.y > me) +
-                (v3.x > me) + (v3.y > me);
-      }
+      for (; j < whole; j += 8) rank += better(j, me);
       for (; j < m; ++j) rank += sh.list[j] > me;
       if (rank < k) sh.cand[rank] = me;
     }
@@ -159,7 +204,7 @@ __device__ __forceinline__ void select_best(int k, SampleShared& sh, Each&& each
     uint64_t under = ~0ull;
     for (int r = 0; r < k; ++r) {
       uint64_t best = 0;
-      each([&](uint64_t e) { best = (e < under && e > best) ? e : best; });
+      again([&](uint64_t e) { best = (e < under && e > best) ? e : best; });
       under = block_max(best, sh);
       if (under == 0) break;
       if (threadIdx.x == 0) sh.cand[r] = under;
@@ -232,6 +277,25 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
   unsigned int* ticket = reinterpret_cast<unsigned int*>(workspace);
   uint64_t* lists = workspace + SAMPLE_TICKET_BYTES / 8;
 
+  // This thread's piece of the block's share: up to 8 logits from `first`, requested ahead of the draw row, which takes two trips.
+  const int first = blockIdx.x * SAMPLE_SHARE + threadIdx.x * 8;
+  const int count = n - first < 0 ? 0 : (n - first > 8 ? 8 : n - first);
+  uint4 raw = make_uint4(0, 0, 0, 0);
+  if (count == 8) raw = *reinterpret_cast<const uint4*>(logits + first);
+  // The step's own tail, where the caller asks for it (the word expressions of iron_eval_words: the
+  // carried position, then every word derived from it and from the token drawn here).  Its operands
+  // are requested now by the first wave, a word and an expression a lane, so that their trips to memory pass under the
+  // draw (nothing but the last block writes them): evaluated one after the other from memory they would cost a trip each.
+  const bool tail = n_exprs > 0, tail_in_lds = tail && n_words <= 64 && n_exprs <= 64;
+  int my_word = 0, rec[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  if (tail_in_lds && threadIdx.x < 64) {
+    if ((int)threadIdx.x < n_words) my_word = words[threadIdx.x];
+    if ((int)threadIdx.x < n_exprs) {
+#pragma unroll
+      for (int f = 0; f < 9; ++f) rec[f] = exprs[9 * threadIdx.x + f];
+    }
+  }
+  const int record_at = at ? *at : 0;
   // The draw row: {temperature (float32 bits), top-k, the 53-bit number's low and high word}.
   // A row outside the buffer, like a temperature that is not positive, is the greedy draw.
   const int at_word = slots.spans != nullptr ? 4 * place : (row ? *row : 0);
@@ -248,13 +312,9 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
   k = k > n ? n : k;
   if (!(temperature > 0.f)) k = 1;   // zero, negative or NaN
 
-  // This thread's piece of the block's share: up to 8 logits from `first`.
-  const int first = blockIdx.x * SAMPLE_SHARE + threadIdx.x * 8;
-  const int count = n - first < 0 ? 0 : (n - first > 8 ? 8 : n - first);
   uint32_t key[8];
   if (count == 8) {
-    const uint4 v = *reinterpret_cast<const uint4*>(logits + first);
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       key[2 * j] = order_key(w[j] & 0xffffu);
@@ -271,109 +331,134 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
   };
 
   const int blocks = gridDim.x;
+  const int room_log2 = min(6, 32 - __builtin_clz(k + k / 4 + TIES - 1));   // entries that a block's list has room for, of SAMPLE_K_MAX places (mostly all that its threads list)
+  // The lists are out: each thread's agent-scope stores have been acknowledged from past the
+  // XCD's L2 (the wait below counts them down) before the block's barrier, and the barrier comes
+  // before the ticket, so a block that sees the last ticket finds every list where its own
+  // agent-scope loads read: in device memory.  The ticket is relaxed on purpose: a release/acquire
+  // pair at agent scope would write back and invalidate the whole L2 on either side (the logits
+  // the head just wrote are dirty lines in it), which costs more than this kernel's other work.
+  auto take_ticket = [=] { return __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)blocks - 1; };
+  auto reset_ticket = [=] { __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  uint64_t top_entry = 0;
   if (k == 1) {
-    // Greedy, or a top-1 draw: the best entry of the block, then of the blocks.
-    uint64_t best = 0;
-    own([&](uint64_t e) { best = e > best ? e : best; });
-    best = block_max(best, sh);
-    if (threadIdx.x == 0) sh.cand[0] = best;
-    if (blocks > 1 && threadIdx.x == 0) publish(&lists[(size_t)blockIdx.x * SAMPLE_K_MAX], best);
-  } else {
-    select_best(k, sh, own);
-    if (blocks > 1 && threadIdx.x < SAMPLE_K_MAX)
-      publish(&lists[(size_t)blockIdx.x * SAMPLE_K_MAX + threadIdx.x], sh.cand[threadIdx.x]);
-  }
-  if (blocks > 1) {
-    // The lists are out: each thread's agent-scope stores have been acknowledged from past the
-    // XCD's L2 (the wait below counts them down) before the block's barrier, and the barrier comes
-    // before the ticket, so a block that sees the last ticket finds every list where its own
-    // agent-scope loads read: in device memory.  The ticket is relaxed on purpose: a release/acquire
-    // pair at agent scope would write back and invalidate the whole L2 on either side (the logits
-    // the head just wrote are dirty lines in it), which costs more than this kernel's other work.
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (threadIdx.x == 0)
-      sh.last_block = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                      (unsigned)blocks - 1;
-    __syncthreads();
-    if (!sh.last_block) return;
-    if (k == 1) {
-      uint64_t best = 0;
-      for (int b = threadIdx.x; b < blocks; b += SAMPLE_THREADS) {
-        const uint64_t e = collect(&lists[(size_t)b * SAMPLE_K_MAX]);
-        best = e > best ? e : best;
-      }
-      best = block_max(best, sh);
-      if (threadIdx.x == 0) sh.cand[0] = best;
-    } else {
-      // The lists' first k entries, a list every `stride` slots (odd, so the lists' heads fall to
-      // different threads); thread t owns slots t + 256 i.  The first HOLD of them are read once,
-      // all requested together, and kept in registers; the rest (longer rows) are read every pass.
-      constexpr int HOLD = 20;
-      const int stride = k | 1, slots = blocks * stride;
-      uint64_t held[HOLD];
+    // Greedy, or a top-1 draw: the best of the block, key and place in one word, then by the first wave alone the best of the blocks.
+    uint32_t mine = 0;
 #pragma unroll
-      for (int i = 0; i < HOLD; ++i) {
-        const int slot = threadIdx.x + SAMPLE_THREADS * i;
-        const int b = slot / stride, r = slot - b * stride;
-        held[i] = (slot < slots && r < k) ? collect(&lists[(size_t)b * SAMPLE_K_MAX + r]) : 0;
-      }
-      select_best(k, sh, [&](auto&& f) {
-#pragma unroll
-        for (int i = 0; i < HOLD; ++i)
-          if (held[i] != 0) f(held[i]);
-        for (int slot = threadIdx.x + SAMPLE_THREADS * HOLD; slot < slots; slot += SAMPLE_THREADS) {
-          const int b = slot / stride, r = slot - b * stride;
-          const uint64_t e = r < k ? collect(&lists[(size_t)b * SAMPLE_K_MAX + r]) : 0;
-          if (e != 0) f(e);
-        }
-      });
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t at = key[j] << 16 | (uint32_t)(SAMPLE_SHARE - 8 * (int)threadIdx.x - j);
+      mine = j < count && at > mine ? at : mine;
     }
-    if (threadIdx.x == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    mine = wave_max_u32(mine);
+    uint32_t* waves = reinterpret_cast<uint32_t*>(sh.slots);
+    if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = mine;
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+#pragma unroll
+    for (int w = 0; w < SAMPLE_THREADS / 64; ++w) mine = waves[w] > mine ? waves[w] : mine;
+    top_entry = entry(mine >> 16, (int)blockIdx.x * SAMPLE_SHARE + SAMPLE_SHARE - (int)(mine & 0xffffu));
+    if (blocks > 1) {
+      bool last = false;
+      if (threadIdx.x == 0) {
+        publish(&lists[(size_t)blockIdx.x * SAMPLE_K_MAX], top_entry);
+        __builtin_amdgcn_s_waitcnt(0);
+        last = take_ticket();
+      }
+      if (__builtin_amdgcn_ballot_w64(last) == 0) return;
+      uint64_t best[SAMPLE_BLOCKS_MAX / 64];
+#pragma unroll
+      for (int i = 0; i < SAMPLE_BLOCKS_MAX / 64; ++i) {
+        const int b = threadIdx.x + 64 * i;
+        best[i] = b < blocks ? collect(&lists[(size_t)b * SAMPLE_K_MAX]) : 0;
+      }
+#pragma unroll
+      for (int i = 1; i < SAMPLE_BLOCKS_MAX / 64; ++i) best[0] = best[i] > best[0] ? best[i] : best[0];
+      const uint32_t high = wave_max_u32((uint32_t)(best[0] >> 32)), low = wave_max_u32((uint32_t)(best[0] >> 32) == high ? (uint32_t)best[0] : 0u);
+      top_entry = (uint64_t)high << 32 | low;
+      if (threadIdx.x == 0) reset_ticket();
+    }
+  } else {
+    select_best(k, blocks > 1 ? 1 << room_log2 : 0, sh, own, own);   // (the last block's selection takes any order)
+    if (blocks > 1) {
+      if (threadIdx.x < SAMPLE_K_MAX) publish(&lists[(size_t)blockIdx.x * SAMPLE_K_MAX + threadIdx.x], sh.cand[threadIdx.x]);
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+      if (threadIdx.x == 0) sh.last_block = take_ticket();
+      __syncthreads();
+      if (!sh.last_block) return;
+      // A wave takes as many lists at a time as fill it, a lane an entry (another one each time, so that the best entries of lists in order fall to different
+      // threads); a thread keeps up to HOLD in registers, all requested together, and of the longest rows' lists four times as many: none is read twice.
+      constexpr int HOLD = 16, WAVES = SAMPLE_THREADS / 64, GROUPS = SAMPLE_BLOCKS_MAX / (HOLD * WAVES);
+      const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, at_once = 6 - room_log2;
+      auto far = [=](int i) { return (WAVES * i) << at_once < blocks; };
+      auto entry_of = [=](int i) {
+        const int b = ((wave + WAVES * i) << at_once) + (lane >> room_log2), r = (lane + 4 * i) & ((1 << room_log2) - 1);
+        return b < blocks ? collect(&lists[(size_t)b * SAMPLE_K_MAX + r]) : 0;
+      };
+      uint64_t held[GROUPS][HOLD];
+#pragma unroll
+      for (int g = 0; g < GROUPS; ++g)
+        if (far(g * HOLD))
+#pragma unroll
+          for (int i = 0; i < HOLD; ++i) held[g][i] = entry_of(g * HOLD + i);
+      select_best(k, 0, sh, [&](auto&& f) {
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g)
+          if (far(g * HOLD))
+#pragma unroll
+            for (int i = 0; i < HOLD; ++i)
+              f(held[g][i]);
+      }, [&](auto&& f) {
+#pragma unroll 1
+        for (int i = 0; far(i); ++i) f(entry_of(i));
+      });
+      if (threadIdx.x == 0) reset_ticket();
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    top_entry = sh.cand[0];
   }
-  __syncthreads();
 
   // The first wave: a candidate's weight a lane; every lane sums and walks them in order.
-  if (threadIdx.x >= 64) return;
-  // The step's own tail, where the caller asks for it (the word expressions of iron_eval_words: the
-  // carried position, then every word derived from it and from the token drawn here).  Its operands
-  // are requested now, a word and an expression a lane, so that their trips to memory pass under the
-  // draw: evaluated one after the other from memory they would cost a trip each.
-  const bool tail = n_exprs > 0, tail_in_lds = tail && n_words <= 64 && n_exprs <= 64;
-  int my_word = 0, rec[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  if (tail_in_lds) {
-    if ((int)threadIdx.x < n_words) my_word = words[threadIdx.x];
-    if ((int)threadIdx.x < n_exprs) {
-#pragma unroll
-      for (int f = 0; f < 9; ++f) rec[f] = exprs[9 * threadIdx.x + f];
-    }
-  }
-  int tok = entry_index(sh.cand[0]);
-  const float top = key_value((uint32_t)(sh.cand[0] >> 32));
+  int tok = entry_index(top_entry);
+  const float top = key_value((uint32_t)(top_entry >> 32));
   if (k > 1 && top - top == 0.f) {   // a finite best logit; else it draws itself
     double w = 0.0;
     const uint64_t mine = sh.cand[threadIdx.x];
     const uint32_t key_i = (uint32_t)(mine >> 32);
     if ((int)threadIdx.x < k && key_i != 0u)
       w = exp_det(((double)key_value(key_i) - (double)top) / (double)temperature);
-    const int w_lo = (int)(uint32_t)__double_as_longlong(w), w_hi = (int)(__double_as_longlong(w) >> 32);
-    auto weight = [&](int i) {
-      const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane(w_lo, i), hi = (uint32_t)__builtin_amdgcn_readlane(w_hi, i);
-      return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+    // The running sum, in order, by the first lane (past the last candidate the weights are zero, which change no sum); each lane then has what it is
+    // behind its own weight.
+    double *sums = reinterpret_cast<double*>(sh.best), *weights = sums + SAMPLE_K_MAX;
+    auto wave_sees = [] {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
-    double total = 0.0;
-    for (int i = 0; i < k; ++i) total += weight(i);
-    const double u = (double)(((uint64_t)(w3 & 0x1fffffu) << 32) | w2) * 0x1p-53;
-    const double threshold = u * total;
-    double running = 0.0;
-    int last = 0, drawn = -1;
-    for (int i = 0; i < k && drawn < 0; ++i) {
-      const double wi = weight(i);
-      running += wi;
-      if (running > threshold) drawn = i;
-      else if (wi > 0.0) last = i;
+    weights[threadIdx.x] = w;
+    wave_sees();
+    if (threadIdx.x == 0) {
+      double sum = 0.0;
+      for (int i0 = 0; i0 < k; i0 += 8) {
+        double some[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) some[i] = weights[i0 + i];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          sum += some[i];
+          some[i] = sum;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sums[i0 + i] = some[i];
+      }
     }
-    const int pick = drawn < 0 ? last : drawn;
+    wave_sees();
+    const double total = sums[k - 1], running = sums[threadIdx.x];   // (past the last eight: not read below)
+    const double u = (double)(((uint64_t)(w3 & 0x1fffffu) << 32) | w2) * 0x1p-53;
+    // The first candidate at which it passes the drawn part of the whole; none, by rounding: the last that has a weight.
+    const uint64_t passed = __builtin_amdgcn_ballot_w64((int)threadIdx.x < k && running > u * total), weighs = __builtin_amdgcn_ballot_w64(w > 0.0);
+    const int pick = passed != 0 ? __builtin_ctzll(passed) : (weighs != 0 ? 63 - __builtin_clzll(weighs) : 0);
     tok = entry_index(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(mine >> 32), pick) << 32) |
                       (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mine, pick));
   }
@@ -381,7 +466,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     *token = tok;
     if (token_copy != nullptr) *token_copy = tok;
     if (record != nullptr) {
-      const int where = slots.spans != nullptr ? place : (at ? *at : 0);
+      const int where = slots.spans != nullptr ? place : record_at;
       if (where >= 0 && where < record_len) record[where] = tok;
     }
     // (every other block of the slot has taken its ticket, so has read its span)

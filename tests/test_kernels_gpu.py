@@ -1976,6 +1976,21 @@ def test_sample_ties_at_the_cut_go_to_the_lower_index(cuda):
     assert _sample_rows(cuda, falling, rows) == [_host_draw(falling, r) for r in rows]
 
 
+# One block's logits and a block more, rows whose lists are one group of sixteen a thread and four; lists with room for 16, 32 and 64 entries (k = 8, 9, 20, 21),
+# blocks whose threads list more than 64 (k = 64); distinct values, few enough for equal ones at every cut, and whole blocks in falling order.
+@pytest.mark.parametrize("vocab", [2048, 2049, 131072, 131073, 500001])
+@pytest.mark.parametrize("values", ["spread", "close", "falling"])
+def test_sample_draws_the_host_token_for_every_room_of_its_lists(cuda, vocab, values):
+    from iron_amd.operators.sample import draw_row
+
+    rng = np.random.default_rng(vocab)
+    logits = {"spread": rng.normal(0, 3, vocab), "close": rng.normal(0, 0.3, vocab), "falling": -np.arange(vocab) % 2048 / 512.0}[values]
+    logits = round_bf16(logits.astype(np.float32))
+    rows = np.stack([draw_row(temperature, k, int(rng.integers(0, 1 << 53)))
+                     for k in (2, 7, 8, 9, 20, 21, 41, 50, 63, 64) for temperature in (0.7, 50.0)])
+    assert _sample_rows(cuda, logits, rows) == [_host_draw(logits, r) for r in rows]
+
+
 def test_sample_special_values_and_row_bounds(cuda):
     from iron_amd.operators.sample import draw_row
 
