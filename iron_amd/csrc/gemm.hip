@@ -465,8 +465,9 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
     const int r = (wave * INST + i) * 8 + lrow;
     const int lch = pch ^ ((r >> 1) & 7);
     a_head[i] = lch * 8;
-    // Rows past the end re-read the last row; what they produce is never stored.
-    a_voff[i] = (int)(((size_t)(min(m0 + r, M - 1) - m0) * K + lch * 8) * 2);
+    // Rows past the last live one bring zeros, without traffic (what they produce is never stored): a CU's few rows wait for what it draws, and a tile's dead rows
+    // were as much of that as live ones.  A 1B decoder's prompt, us, by dead rows read and not: 2 rows 1286 / 1208, 29 1306 / 1243, 513 2511 / 2281, 900 3034 / 2807.
+    a_voff[i] = m0 + r < Mv ? (r * K + lch * 8) * 2 : NOWHERE;
   }
 #pragma unroll
   for (int i = 0; i < B_INST; ++i) {
@@ -816,8 +817,7 @@ __device__ __forceinline__ void gemm_nt16_body(const bf16_t* __restrict__ A, con
   for (int i = 0; i < INST; ++i) {
     const int r = (wave * INST + i) * 8 + lrow;
     const int lch = pch ^ ((r >> 1) & 7);
-    // Rows past the end re-read the last row; what they produce is never stored.
-    a_voff[i] = (int)(((size_t)(min(m0 + r, M - 1) - m0) * K + lch * 8) * 2);
+    a_voff[i] = m0 + r < Mv ? (r * K + lch * 8) * 2 : NOWHERE;
     a_head[i] = b_head[i] = lch * 8;
     if constexpr (!B_KN) {
       b_voff[i] = (int)(((size_t)(min(n0 + r, N - 1) - n0) * K + lch * 8) * 2);
@@ -1265,7 +1265,7 @@ __device__ __forceinline__ void qkv_heads_body(const bf16_t* __restrict__ A, con
 #pragma unroll
   for (int i = 0; i < A_INST; ++i) {
     const int r = (wave * A_INST + i) * 8 + lrow;
-    a_voff[i] = (int)(((size_t)(min(m0 + r, M - 1) - m0) * K + (pch ^ ((r >> 1) & 7)) * 8) * 2);
+    a_voff[i] = m0 + r < Mv ? (r * K + (pch ^ ((r >> 1) & 7)) * 8) * 2 : NOWHERE;
   }
 #pragma unroll
   for (int i = 0; i < B_INST; ++i) {
@@ -1641,7 +1641,8 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
   static_assert(WAVES % 2 == 0, "a wave's instructions all begin on an even eight rows, or all on an odd");
   const int ld_off = (int)(((size_t)lrow * K + ld_head) * 2);
   const int pad = k_pad(K);
-  const __amdgpu_buffer_rsrc_t a_rows = stage_rows(A + (size_t)(m0 + wave * 8) * K - pad);
+  // (A ends at its last live row: a load past it brings zeros and costs no traffic.)
+  const __amdgpu_buffer_rsrc_t a_rows = bounded_bytes(A + (size_t)(m0 + wave * 8) * K - pad, (int)max(0L, min(0x7fffffffL, 2 * ((long)(Mv - m0 - wave * 8) * K + pad))));
   // B as (K,N) lands as stored: the stage's 64 k-rows of BN columns, a row's chunks XORed with kn_swizzle(row) so that the
   // transposing reads below find the four rows of a 16-lane group, and the groups of a pass, in different banks.
   constexpr int KN_CHUNKS = T::BN / 8, KN_ROWS = 64 / KN_CHUNKS;   // chunks of a k-row, k-rows of an instruction
@@ -2387,9 +2388,8 @@ __device__ __forceinline__ void gemm_nt16_pair_body(const bf16_t* __restrict__ A
   for (int i = 0; i < INST; ++i) {
     const int r = (wave * INST + i) * 8 + lrow;
     const int lch = pch ^ ((r >> 1) & 7);
-    // Rows past the end re-read the last row; what they produce is never stored.
     if constexpr (GROUPED) a_voff[i] = (int)(((size_t)a_rows[m0 + r] * K + lch * 8) * 2);
-    else a_voff[i] = (int)(((size_t)(min(m0 + r, M - 1) - m0) * K + lch * 8) * 2);
+    else a_voff[i] = m0 + r < Mv ? (r * K + lch * 8) * 2 : NOWHERE;
     b_voff[i] = (int)(((size_t)(min(n0 + r, N - 1) - n0) * K + lch * 8) * 2);
   }
   const bf16_t* a_tile = GROUPED ? A : A + (size_t)m0 * K;
