@@ -753,6 +753,137 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
   else pieces(std::false_type());
 }
 
+// Up to LONG_ROWS rows, one row of tiles, over a K of whole LONG_K, where the tiles are one round over the chip: few rows wait for what a CU draws, so as many CUs
+// as there are draw as little as there is to draw, and in long pieces: stages of LONG_K columns are runs of 512 bytes and eight k-steps between two barriers; B,
+// of which every block reads rows of its own once, goes past the caches.  A group is sixteen rows of B, an MFMA's: LONG_PAIR: eight of
+// the gate's and eight of the up projection's, four groups a block, a wave a group; LONG_QKV: eight of each half of a head, one group; LONG_PLAIN: eight rows, read
+// twice over.  Of the last two a block has one group, a wave sixteen rows of A each, and waves past those only fetch.  An element's sum is the chain of
+// 32-wide k-steps that it is in every other tile: the same bits.
+// us, 29 rows, weights out of memory, by the tiles of 32 and 64 rows below and by this: 2048 columns over 2048 with a residual 8.6 / 6.4, over 8192 20.9 / 13.4, over 14336
+// 37.3 / 22.0, 256 over 512 4.2 / 3.8; 48 heads of q, k and v over 2048 8.6 / 7.2 (64 rows 10.4 / 8.8); both of 8192 over 2048 18.9 / 15.8, of 1024 over 4096 17.9 / 16.1.  With
+// more than a round of them 1.01 to 1.08 of the others' time (2560 columns over 2048 8.95 / 9.4); 64 rows of a plain product 0.9 to 1.1, of a pair 18.5 / 19.5: those stay.
+constexpr int LONG_K = 256, LONG_ROW = LONG_K * 2;
+enum LongKind { LONG_PLAIN, LONG_PAIR, LONG_QKV };
+constexpr int long_b_rows(LongKind kind) { return kind == LONG_PAIR ? 64 : (kind == LONG_QKV ? 16 : 8); }
+constexpr int long_lds(LongKind kind, int rows, int stages) { return (rows + long_b_rows(kind)) * LONG_ROW * stages; }
+template <LongKind KIND, int LONG_ROWS, int STAGES>
+__device__ __forceinline__ void gemm_long_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, bf16_t* __restrict__ C, int N, int K, int Mv,
+                                               const QkvTail& qkv, const bf16_t* __restrict__ up = nullptr, bf16_t* __restrict__ gate_out = nullptr) {
+  constexpr int B_ROWS = long_b_rows(KIND), STAGE = long_lds(KIND, LONG_ROWS, 1);
+  constexpr int MI = KIND == LONG_PAIR ? LONG_ROWS / 16 : 1;                                  // tiles of A's rows a wave
+  constexpr int A_INST = LONG_ROWS / 8, B_INST = B_ROWS / 8, LOADS = A_INST + B_INST;   // loads of two rows each, a wave's share
+  static_assert(LONG_K == 256 && (LONG_ROWS == 32 || LONG_ROWS == 64), "two rows a load of 1 KB");
+  extern __shared__ __align__(16) char smem_nt[];
+  const int tile = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), fr = lane & 15, kq = lane >> 4;
+  const int group = KIND == LONG_PAIR ? wave : 0, wm = KIND == LONG_PAIR ? 0 : wave;
+  const bool computes = KIND == LONG_PAIR || wave < LONG_ROWS / 16;
+  // QKV: a tile is columns first .. + 7 and 32 + first .. of a 64-wide head of the list q | k | v.
+  const int q_heads = N >> 6, kv_heads = KIND == LONG_QKV ? qkv.kv_n >> 6 : 0, head = tile >> 2, first = (tile & 3) * 8;
+  const int which = KIND != LONG_QKV || head < q_heads ? 0 : (head < q_heads + kv_heads ? 1 : 2), own = head - (which == 0 ? 0 : q_heads + (which - 1) * kv_heads);
+  const int n0 = KIND == LONG_QKV ? first : tile * (KIND == LONG_PAIR ? B_ROWS / 2 : B_ROWS);
+  if (KIND == LONG_QKV ? head >= q_heads + 2 * kv_heads : n0 >= N) return;
+  if constexpr (KIND == LONG_QKV) B = (which == 0 ? B : (which == 1 ? qkv.Bk : qkv.Bv)) + (size_t)own * 64 * K;
+  else B += (size_t)n0 * K;
+  if (KIND == LONG_PAIR) up += (size_t)n0 * K;
+  int a_voff[A_INST], b_voff[B_INST];
+#pragma unroll
+  for (int i = 0; i < A_INST; ++i) {
+    const int r = (wave * A_INST + i) * 2 + (lane >> 5);
+    a_voff[i] = r < Mv ? (r * K + (((lane & 31) ^ (r & 15)) << 3)) * 2 : NOWHERE;
+  }
+#pragma unroll
+  for (int i = 0; i < B_INST; ++i) {
+    const int r = (wave * B_INST + i) * 2 + (lane >> 5), row = KIND == LONG_PAIR ? (r >> 4) * 8 + (r & 7) : (KIND == LONG_QKV ? first + (r >> 3) * 32 + (r & 7) : r);
+    b_voff[i] = (row * K + (((lane & 31) ^ (r & 15)) << 3)) * 2;
+  }
+  const int nk = K / LONG_K;
+  auto issue = [&](int buffer, int kt) {   // (a stage past the last: zeros out of empty buffers, so that the waits can count)
+    char* st = smem_nt + buffer * STAGE;
+    const int k0 = kt * LONG_K, room = kt < nk ? 0x7fffffff : 0;
+#pragma unroll
+    for (int i = 0; i < B_INST; ++i) {
+      const bool second = KIND == LONG_PAIR && ((wave * B_INST + i) * 2 & 15) >= 8;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(bounded_bytes((second ? up : B) + k0, room), IRON_LDS_PTR(st + LONG_ROWS * LONG_ROW + (wave * B_INST + i) * 1024), 16,
+                                               (int)b_voff[i], 0, 0, 2);   // non-temporal
+    }
+#pragma unroll
+    for (int i = 0; i < A_INST; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(bounded_bytes(A + k0, room), IRON_LDS_PTR(st + (wave * A_INST + i) * 1024), 16, (int)a_voff[i], 0, 0, 0);
+  };
+  f32x4 acc[MI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // acc[i][e]: row fr of the wave's i-th sixteen, row 4 kq + e of the group's of B.
+  const int m_own = wm * 16 + fr, n_own = n0 + group * 8 + 4 * (kq & 1);
+  uint2 res = make_uint2(0, 0);   // a residual's piece this lane will add
+  if (KIND == LONG_PLAIN && qkv.residual != nullptr && m_own < Mv) res = *reinterpret_cast<const uint2*>(qkv.residual + (size_t)m_own * N + n_own);
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s) issue(s, s);
+  const int a_off = (wm * 16 + fr) * LONG_ROW, b_row = KIND == LONG_PLAIN ? fr & 7 : group * 16 + fr, b_off = (LONG_ROWS + b_row) * LONG_ROW, b_swz = b_row & 15;
+  for (int kt = 0, buffer = 0; kt < nk; ++kt) {
+    wait_vmcnt<(STAGES - 2) * LOADS>();   // stage kt has landed once only the younger ones are out
+    block_barrier();                      // ... in every wave, and nobody reads stage kt - 1 any more
+    issue(buffer == 0 ? STAGES - 1 : buffer - 1, kt + STAGES - 1);
+    if (computes) {
+      const char* st = smem_nt + buffer * STAGE;
+      bf16x8 bf[LONG_K / 32], af[MI][LONG_K / 32];
+#pragma unroll
+      for (int ks = 0; ks < LONG_K / 32; ++ks) {
+        bf[ks] = *reinterpret_cast<const bf16x8*>(st + b_off + (((ks * 4 + kq) ^ b_swz) << 4));
+#pragma unroll
+        for (int i = 0; i < MI; ++i) af[i][ks] = *reinterpret_cast<const bf16x8*>(st + a_off + i * 16 * LONG_ROW + (((ks * 4 + kq) ^ fr) << 4));
+      }
+#pragma unroll
+      for (int ks = 0; ks < LONG_K / 32; ++ks)
+#pragma unroll
+        for (int i = 0; i < MI; ++i) mfma_16x16x32_in_place(acc[i], bf[ks], af[i][ks]);
+    }
+    buffer = buffer == STAGES - 1 ? 0 : buffer + 1;
+  }
+  wait_vmcnt<0>();   // the empty fetches land before the block's LDS is released
+  if (!computes) return;
+  asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");   // (the matrix cores' last results)
+#pragma unroll
+  for (int i = 0; i < MI; ++i) asm volatile("" : "+a"(acc[i]));
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int m = m_own + i * 16;
+    float x[4], other[4];   // rounded as the product would be stored; the group's other eight rows'
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      x[e] = acc[i][e];
+      if (KIND != LONG_PLAIN || qkv.residual != nullptr) x[e] = round_bf16(x[e]);
+      other[e] = KIND == LONG_PLAIN ? 0.f : __shfl_xor(x[e], 32, 64);
+    }
+    if (m >= Mv) continue;
+    bf16_t* to = C + (size_t)m * N + n_own;
+    if constexpr (KIND == LONG_PAIR) {
+      if (kq >= 2) tail_of(qkv, x, other);
+      else if (gate_out == nullptr) continue;
+      else to = gate_out + (size_t)m * N + n_own;
+    } else if constexpr (KIND == LONG_QKV) {
+      const int c = first + 4 * (kq & 1), row_len = which == 0 ? N : qkv.kv_n;   // ... of the head's half
+      to = (which == 0 ? C : (which == 1 ? qkv.Ck : qkv.Cv)) + (size_t)m * row_len + own * 64 + c + (kq >> 1) * 32;
+      if (which < 2) {
+        float cs[8];
+        unpack8(*reinterpret_cast<const uint4*>(qkv.angles + (size_t)m * 64 + 2 * c), cs);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float x1 = kq < 2 ? x[e] : other[e], x2 = kq < 2 ? other[e] : x[e];
+          x[e] = kq < 2 ? x1 * cs[2 * e] - x2 * cs[2 * e + 1] : x2 * cs[2 * e] + x1 * cs[2 * e + 1];
+        }
+      }
+    } else {
+      if (kq >= 2) continue;
+      if (qkv.residual != nullptr) {
+        const float rf[4] = {__uint_as_float(res.x << 16), __uint_as_float(res.x & 0xffff0000u), __uint_as_float(res.y << 16), __uint_as_float(res.y & 0xffff0000u)};
+        tail_of(qkv, x, rf);
+      }
+    }
+    store_loose(to, pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3]));
+  }
+}
+
 // 128 x 128 x 64 tiles, four stages of 32 KB fed straight from global memory into LDS (buffer loads:
 // the tile's rows from the stage's k on are the buffer, rebuilt per stage with scalar instructions,
 // a lane's place in it a constant 32-bit offset, so a load costs one scalar add for its LDS
@@ -1475,7 +1606,12 @@ __global__ __launch_bounds__(256) void qkv_either_kernel(const bf16_t* __restric
   const int Mv = bound_or(valid, M);
   const bool past = Mv > above;
   to_cache_rows(qkv, valid, M);
-  if (Mv <= half_upto) {   // ... or half-head ones of 64 rows
+  const bool longs = K % LONG_K == 0 && (heads + 2 * kv_heads) * 4 <= min(256, (int)gridDim.x);
+  if (longs && Mv <= 32) {
+    gemm_long_body<LONG_QKV, 32, 5>(A, Bq, Cq, heads * 64, K, Mv, qkv);
+  } else if (longs && Mv <= 64) {
+    gemm_long_body<LONG_QKV, 64, 3>(A, Bq, Cq, heads * 64, K, Mv, qkv);
+  } else if (Mv <= half_upto) {   // ... or half-head ones of 64 rows
     gemm_nt64_body<10, false, 1, 4, 2, true>(A, Bq, Cq, M, heads * 64, K, Mv, (M + 63) / 64, (heads + 2 * kv_heads) * 2, 0, qkv);
   } else if (Mv <= low_upto) {
     gemm_nt64_body<8, false, 2, 2, 2, true>(A, Bq, Cq, M, heads * 64, K, Mv, (M + 63) / 64, heads + 2 * kv_heads, 0, qkv);
@@ -1509,8 +1645,9 @@ static int launch_qkv_either(const bf16_t* A, const bf16_t* Bq, bf16_t* Cq, int 
   const Tiling wide{wide_ok ? tiles_m : 0, wide_ok ? total / 3 : 0, wide_ok ? patched_order(tiles_m, total / 3) : 0};
   const int thin_m = (thin_upto + 127) / 128;
   const Tiling thin{thin_m, total, patched_order(thin_m, total)};
-  const size_t lds_narrow = (size_t)NT_STAGES * 256 * BK * 2, lds_wide = (size_t)Q3_STAGES * Q3_STAGE_BYTES;
-  const size_t lds = lds_narrow > lds_wide ? lds_narrow : lds_wide;
+  constexpr size_t lds_narrow = (size_t)NT_STAGES * 256 * BK * 2, lds_wide = (size_t)Q3_STAGES * Q3_STAGE_BYTES;
+  constexpr size_t lds = lds_narrow > lds_wide ? lds_narrow : lds_wide;
+  static_assert(lds >= (size_t)long_lds(LONG_QKV, 32, 5) && lds >= (size_t)long_lds(LONG_QKV, 64, 3), "the few rows' stages fit too");
   static LdsOptIn opt_in;
   if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&qkv_either_kernel), lds); e != hipSuccess) {
     set_error("prefill_qkv: %s", hipGetErrorString(e));
@@ -2105,8 +2242,10 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const bf16_t* __restrict
     case ROWS_64X32:
       gemm_nt64_body<13, false, 1, 4>(A, B, C, M, N, K, Mv, (M + 63) / 64, (N + 31) / 32, patched, tail);
       break;
-    default:
-      gemm_nt64_body<20, false, 1, 2, 1>(A, B, C, M, N, K, Mv, (M + 31) / 32, (N + 31) / 32, patched, tail);
+    default: {
+      if (Mv <= 32 && K % LONG_K == 0 && N % 8 == 0 && N / 8 <= min(256, (int)gridDim.x)) gemm_long_body<LONG_PLAIN, 32, 7>(A, B, C, N, K, Mv, tail);
+      else gemm_nt64_body<20, false, 1, 2, 1>(A, B, C, M, N, K, Mv, (M + 31) / 32, (N + 31) / 32, patched, tail);
+    }
   }
 #undef IRON_ROWS
 }
@@ -2169,7 +2308,7 @@ static int launch_gemm_rows(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, 
   if (two_a_cu(M, N, K, valid != nullptr)) return launch_gemm_nt<false, false, 1>(A, B, C, M, N, K, valid, s, tail);
   const FormPlan plan = rows_plan(M, N, K, valid != nullptr, tail.residual != nullptr);
   constexpr size_t lds = Tile256Four::LDS_BYTES;
-  static_assert(lds >= (size_t)NT_STAGES * 256 * BK * 2, "the other bodies' stages fit too");
+  static_assert(lds >= (size_t)NT_STAGES * 256 * BK * 2 && lds >= (size_t)long_lds(LONG_PLAIN, 32, 7), "the other bodies' stages fit too");
   static LdsOptIn opt_in[2];
   const auto kernel = tail.residual != nullptr ? &gemm_rows_kernel<true> : &gemm_rows_kernel<false>;
   if (hipError_t e = opt_in[tail.residual != nullptr].ensure(reinterpret_cast<const void*>(kernel), lds); e != hipSuccess) {
@@ -2604,7 +2743,8 @@ __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __re
     default: {
       QkvTail gate{};
       gate.gated = activation;
-      gemm_nt64_body<8, true>(A, Bg, C, M, N, K, Mv, (M + 63) / 64, (N + 31) / 32, patched, gate, Bu, G);
+      if (Mv <= 32 && K % LONG_K == 0 && N % 32 == 0) gemm_long_body<LONG_PAIR, 32, 3>(A, Bg, C, N, K, Mv, gate, Bu, G);
+      else gemm_nt64_body<8, true>(A, Bg, C, M, N, K, Mv, (M + 63) / 64, (N + 31) / 32, patched, gate, Bu, G);
     }
   }
 #undef IRON_PAIR
@@ -2619,7 +2759,8 @@ static int launch_gemm_gated_pair(const bf16_t* A, const bf16_t* Bg, const bf16_
                                   int N, int K, const int* valid, int activation, hipStream_t s) {
   const FormPlan plan = pair_plan(M, N, K, valid != nullptr);
   constexpr size_t lds = Tile256Four::LDS_BYTES;   // the largest tile's, more than the others'
-  static_assert(lds >= (size_t)PAIR_STAGES * 3 * 128 * BK * 2 && lds >= (size_t)NT_STAGES * 256 * BK * 2, "the other bodies' stages fit too");
+  static_assert(lds >= (size_t)PAIR_STAGES * 3 * 128 * BK * 2 && lds >= (size_t)NT_STAGES * 256 * BK * 2 && lds >= (size_t)long_lds(LONG_PAIR, 32, 3),
+                "the other bodies' stages fit too");
   static LdsOptIn opt_in;
   if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_gated_pair_kernel), lds); e != hipSuccess) {
     set_error("gemm_gated_pair: %s", hipGetErrorString(e));

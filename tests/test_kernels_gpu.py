@@ -601,6 +601,64 @@ def test_a_row_s_products_are_the_same_bits_under_every_bound(cuda, M, Kdim, N, 
             assert (got[rows:] == 7).all(), rows
 
 
+# One row of tiles, whose stages are 256 columns of K: one stage, fewer than the ring holds, more; one tile of eight columns, some, one a CU (and a tile more, which
+# the others take); rows on either side of sixteen and of the tile's.
+@pytest.mark.parametrize("Kdim", [256, 768, 2304])
+@pytest.mark.parametrize("N", [8, 200, 2048, 2056])
+@pytest.mark.parametrize("form", ["plain", "residual", "gated", "pair"])
+def test_few_rows_over_long_stages_are_the_same_bits_as_among_many(cuda, Kdim, N, form):
+    rng = np.random.default_rng(Kdim + N)
+    M = 600
+    N = N if form == "plain" else max(64, 32 * -(-N // 32) if form == "pair" else N)   # (the fewest columns that a second operand is taken with)
+    A, B, B2, R = (bf(rng, *s, scale=x) for s, x in (((M, Kdim), 1.0), ((N, Kdim), 0.05), ((N, Kdim), 0.05), ((M, N), 1.0)))
+    dB, dB2, dR, kw = dev(B, cuda), dev(B2, cuda), dev(R, cuda), dict(M=M, N=N, K=Kdim)
+
+    def run(rows):
+        C, G = out_like((M, N), cuda, fill=7.0), out_like((M, N), cuda, fill=7.0)
+        held = A.copy()
+        held[rows:] = np.nan
+        dA, bound = dev(held, cuda), word(rows, cuda)
+        if form == "plain":
+            K.gemm(dA, dB, C, b_col_maj=True, valid=bound, **kw)
+        elif form == "residual":
+            K.gemm_residual(dA, dB, dR, C, residual_scale=0.5, valid=bound, **kw)
+        elif form == "gated":
+            K.gemm_gated(dA, dB, dR, C, activation="silu", valid=bound, **kw)
+        else:
+            K.gemm_gated_pair(dA, dB, dB2, G, C, activation="silu", valid=bound, **kw)
+        return C, G
+
+    whole = run(M)
+    if form in ("plain", "pair"):
+        close(whole[form == "pair"][:33], ops.gemm(A[:33], B, b_col_maj=True), rtol=1e-2, atol=1e-2)
+    for rows in (1, 8, 16, 17, 31, 32):
+        for got, want in zip(run(rows), whole):
+            assert torch.equal(got[:rows], want[:rows]), rows
+            assert (got[rows:] == 7).all(), rows
+
+
+@pytest.mark.parametrize("E", [256, 1280])
+@pytest.mark.parametrize("H,G", [(32, 8), (48, 8), (56, 8), (4, 2)])   # the most heads whose tiles are one round, and more
+def test_few_rows_projections_are_the_same_bits_as_among_many(cuda, E, H, G):
+    rng = np.random.default_rng(E + H)
+    rows, D = 1024, 64
+    x, Wq, Wk, Wv = bf(rng, rows, E), bf(rng, H * D, E, scale=0.05), bf(rng, G * D, E, scale=0.05), bf(rng, G * D, E, scale=0.05)
+    fixed = [dev(a, cuda) for a in (Wq, Wk, Wv, round_bf16(ops.rope_angles(D, rows, 500000.0)))]
+
+    def run(bound):
+        held = x.copy()
+        held[bound:] = np.nan
+        outs = [out_like((rows, n), cuda, fill=7.0) for n in (H * D, G * D, G * D)]
+        K.prefill_qkv(dev(held, cuda), *fixed, *outs, rows=rows, hidden=E, heads=H, kv_heads=G, d=D, valid=word(bound, cuda))
+        return outs
+
+    many = run(100)   # tiles of 64 columns of K
+    for bound in (1, 16, 17, 32, 33, 63, 64):
+        for got, want in zip(run(bound), many):
+            assert torch.equal(got[:bound], want[:bound]), bound
+            assert (got[bound:] == 7).all(), bound
+
+
 @pytest.mark.parametrize("rows,bound,H,G", [(2048, None, 32, 8), (256, 150, 16, 4), (128, None, 2, 2),
                                             # bounds on either side of where the 192-wide tiles take over
                                             (2048, 1280, 32, 8), (2048, 1281, 32, 8), (2048, 1999, 32, 8),
