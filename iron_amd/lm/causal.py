@@ -272,6 +272,13 @@ class CausalLM(iron.Graph):
             raise RuntimeError(f"{type(self).__name__}: load_versions() first")
         return self.decode_step(**values) if ids is None else self.prompt_chunk(ids, **values)
 
+    def run(self, ids=None, **values):
+        """A loaded version's logits without what it carries, which a call would wait for."""
+        if self.decode_step is None:
+            raise RuntimeError(f"{type(self).__name__}: load_versions() first")
+        (row,) = self.decode_step.run(**values) if ids is None else self.prompt_chunk.run(ids, **values)
+        return row
+
     # ------------------------------------------------------------------ use
     def logits(self, tokens) -> np.ndarray:
         """Logits after the last of ``tokens`` (see ``Session.logits``)."""
@@ -337,6 +344,9 @@ class _HostVersion:
     def __call__(self, *tensors, **values):
         outs, carried = iron.Graph.reference(self.graph, *tensors, **values)
         return (*(_HostOutput(o) for o in outs), iron.Carry(carried))
+
+    def run(self, *tensors, **values):
+        return self(*tensors, **values)[:-1]
 
     def write(self, resident, array) -> None:
         resident.host = np.array(array).reshape(-1)

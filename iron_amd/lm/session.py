@@ -119,13 +119,13 @@ class Session:
         model = self.lm
         shared = self._reusable(ids)
         if shared == self.cached.size == ids.size - 1:
-            row, _ = model(token=int(ids[-1]), position=ids.size - 1)
+            row = model.run(token=int(ids[-1]), position=ids.size - 1)
         else:
             begin = self.resume(shared)
             self.cached = ids[:begin]
             row = None
             for inputs, words in self.chunk_calls(ids, begin):
-                row, _ = model(*inputs, **words)
+                row = model.run(*inputs, **words)
         self.cached = ids
         # The output buffer is the arena's and the next launch reuses it: hand out a copy, without
         # the columns that only pad an odd vocabulary.
@@ -157,14 +157,21 @@ class Session:
         begin = self.resume(self._reusable(ids))
         # Until the run is over nobody knows how far it got (the caller may stop iterating).
         self.cached = self.cached[:0]
-        carried = None
-        for inputs, words in self.chunk_calls(ids, begin):
+        remaining, step = max_tokens - 1, model.decode_step
+        *chunks, (inputs, words) = self.chunk_calls(ids, begin)
+        for others, at in chunks:
+            model.run(*others, **at)
+        replayed = bool(remaining) and step.captured and not each
+        started = replayed and model.prompt_chunk.hands_over(step)   # (the first step behind the prompt, while its token is on its way here)
+        if started:
+            carried = model.prompt_chunk.run_and_start(step, *inputs, **words)
+        else:
             _, carried = model(*inputs, **words)
         out = [int(carried["token"])]
         yield out[0]
-        remaining, step = max_tokens - 1, model.decode_step
-        if remaining and step.captured and not each:
-            step.start(**carried)
+        if replayed:
+            if not started:
+                step.start(**carried)
             step.replay(remaining - 1)
             record = step.read(model.drawn)       # position p holds the token drawn at p
             for token in record[prompt_len : prompt_len + remaining]:

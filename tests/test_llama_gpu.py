@@ -394,6 +394,22 @@ def _fill_caches(gpu, cpu, n: int, upto: int) -> None:
         cpu.decode_step.write(on_host, rows)
 
 
+def test_a_draw_starts_its_second_step_behind_the_prompt_on_the_device(toy, monkeypatch):
+    """The first step behind a prompt is launched before the prompt's token is read: the tokens are those of steps started
+    from the host, one after the other, also behind a draw that was given up after its first token; versions that cannot hand over are not asked to."""
+    prompt = np.random.default_rng(31).integers(0, SCALED.vocab_size, 60).tolist()
+    assert toy.prompt_chunk.hands_over(toy.decode_step)
+    stepwise = list(toy.session.draw(prompt, 12, each=True))
+    for count in (12, 2, 1):
+        given_up = toy.session.draw(prompt[:5], 9)
+        next(given_up)
+        given_up.close()
+        assert list(toy.session.draw(prompt, count)) == stepwise[:count]
+        assert toy.logits(prompt + stepwise[:count]).argmax() == (stepwise + list(toy.session.draw(prompt + stepwise, 1)))[count]
+    monkeypatch.setattr(type(toy.prompt_chunk), "hands_over", lambda *_: False)
+    assert list(toy.session.draw(prompt, 12)) == stepwise
+
+
 @pytest.fixture(scope="module")
 def deep(cuda):
     """Two layers at Llama-3.2-1B's width over caches of 16384 rows in 2048-row chunks, on the GPU and
