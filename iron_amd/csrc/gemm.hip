@@ -2176,7 +2176,8 @@ static FormTable form_table(int M, bool bounded, Best best, int* upto) {
 // launches of every form up to 1024, of which the cheapest by them takes 1.0002 of the best on average and 1.03 at the most (by the long K's prices 1.08 below
 // K = 512, 1.02 from there on, and up to 2.1: 2048 x 2560 x 64 by 64 x 64 tiles 15.5, by 192 x 128 7.2; 2048 x 6144 x 512 27.3 / 20.0; from 1088 to 1536
 // 87 launches of few rows by many columns 1.002 and 1.11: 3 rows of 64 x 26574 x 1152 with a second operand by two rounds of 64 x 64 tiles 21.2, by one of 128 x 128 15.9).
-enum RowsForm { ROWS_32X32, ROWS_64X32, ROWS_64X64, ROWS_128X64, ROWS_128X128, ROWS_160X128, ROWS_192X128, ROWS_256X128, ROWS_160X256, ROWS_192X256, ROWS_256X256, ROWS_FORMS };
+enum RowsForm { ROWS_32X32, ROWS_64X32, ROWS_64X64, ROWS_128X64, ROWS_128X128, ROWS_96X128, ROWS_160X128, ROWS_192X128, ROWS_224X128, ROWS_256X128, ROWS_160X256, ROWS_192X256, ROWS_224X256,
+                ROWS_256X256, ROWS_FORMS };
 constexpr int SHORT_STAGES = 24;
 struct RoundPrice {
   float start, stage;
@@ -2188,11 +2189,18 @@ struct RowsPrice {
 constexpr RowsPrice ROWS_PRICES[ROWS_FORMS] = {
     {32, 32, {0.8f, 0.15f}, {{2.f, 0.142f}, {2.2f, 0.146f}}},     {64, 32, {0.8f, 0.2f}, {{2.45f, 0.171f}, {2.85f, 0.17f}}},
     {64, 64, {0.8f, 0.28f}, {{2.5f, 0.235f}, {3.3f, 0.235f}}},    {128, 64, {2.f, 0.34f}, {{3.05f, 0.357f}, {4.55f, 0.362f}}},
-    {128, 128, {4.f, 0.45f}, {{3.4f, 0.515f}, {5.1f, 0.53f}}},    {160, 128, {3.4f, 0.52f}, {{3.4f, 0.583f}, {5.4f, 0.6f}}},
-    {192, 128, {5.f, 0.57f}, {{3.9f, 0.645f}, {6.f, 0.665f}}},    {256, 128, {6.5f, 0.69f}, {{4.3f, 0.743f}, {9.f, 0.76f}}},
+    {128, 128, {4.f, 0.45f}, {{3.4f, 0.515f}, {5.1f, 0.53f}}},    {96, 128, {3.4f, 0.39f}, {{3.3f, 0.46f}, {4.8f, 0.47f}}},
+    {160, 128, {3.4f, 0.52f}, {{3.4f, 0.583f}, {5.4f, 0.6f}}},
+    {192, 128, {5.f, 0.57f}, {{3.9f, 0.645f}, {6.f, 0.665f}}},    {224, 128, {5.7f, 0.63f}, {{4.1f, 0.69f}, {7.5f, 0.71f}}},
+    {256, 128, {6.5f, 0.69f}, {{4.3f, 0.743f}, {9.f, 0.76f}}},
     {160, 256, {8.f, 0.8f}, {{4.85f, 0.872f}, {10.5f, 0.93f}}},   {192, 256, {9.f, 0.85f}, {{5.5f, 0.9f}, {13.f, 0.96f}}},
+    {224, 256, {12.f, 0.93f}, {{6.1f, 1.f}, {16.5f, 1.07f}}},
     {256, 256, {15.f, 1.f}, {{6.7f, 1.1f}, {20.f, 1.19f}}},
 };
+// Tiles of 96 and 224 rows are for the runs of rows that leave the last round of the others' a quarter empty; up to K = 512, where a round is its start and its end, a
+// twentieth at the most (256 blocks, 4096 columns, us by 96 x 128 / 128 x 128 tiles: K = 256 8.5 / 8.8, 512 9.9 / 10.2, 1024 12.6 / 13.4, 2048 21.5 / 23.9, 8192 63.3 / 72.9; by 192, 224
+// and 256 x 256: K = 2048 46.6, 50.6, 55.1), so they begin past that.  2048 columns over 2048, 1102 rows 17.3 / 15.1, over 8192, 1379 rows 62.9 / 54.3; 10240 over 2048, 213 rows
+// 21.8 / 18.8; 4544 over 5184, 615 rows 51.0 / 41.3; of 280 drawn ones 58 take them, at 0.90 of the time.
 struct RowsChoice {
   RowsForm form;
   float us;
@@ -2205,6 +2213,7 @@ static RowsChoice rows_form(int rows, int M, int N, int K, bool second) {
   for (int form = first; form < ROWS_FORMS; ++form) {
     const RowsPrice& p = ROWS_PRICES[form];
     if (form > ROWS_128X128 && (M < p.bm || N < p.bn || (second && N % 8 != 0))) continue;
+    if (stages <= 8 && (form == ROWS_96X128 || form == ROWS_224X128 || form == ROWS_224X256)) continue;
     const RoundPrice& of = stages > SHORT_STAGES ? p.long_k : p.short_k[second];
     const long tiles = (long)((rows + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
     const float us = (float)((tiles + 255) / 256) * (of.start + of.stage * stages);
@@ -2224,11 +2233,14 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const bf16_t* __restrict
                                                                     patched, GatedPair{}, tail); \
     break
   switch (chosen.form) {
+    IRON_ROWS(ROWS_96X128, 3, 4);
     IRON_ROWS(ROWS_160X128, 5, 4);
     IRON_ROWS(ROWS_192X128, 6, 4);
+    IRON_ROWS(ROWS_224X128, 7, 4);
     IRON_ROWS(ROWS_256X128, 8, 4);
     IRON_ROWS(ROWS_160X256, 5, 8);
     IRON_ROWS(ROWS_192X256, 6, 8);
+    IRON_ROWS(ROWS_224X256, 7, 8);
     IRON_ROWS(ROWS_256X256, 8, 8);
     case ROWS_128X128:
       gemm_nt16_body<false>(A, B, C, M, N, K, Mv, (M + 127) / 128, (N + 127) / 128, patched, tail);
@@ -2355,8 +2367,11 @@ __global__ __launch_bounds__(256) void gemm_splitk_kernel(const bf16_t* __restri
   const int Mv = bound_or(valid, M);
   const int tiles_n = whole.tiles_n, tile_rows = (Mv + 127) / 128, live_tiles = tile_rows * tiles_n;
   const int splits = splitk_for(tile_rows, tiles_n, K), id = blockIdx.x;
-  if (splits == 1) {   // whole K a block, the residual in its epilogue: iron_gemm_residual_bf16's 128 x 128 launch
-    if (id < whole.tiles_m * whole.tiles_n)
+  if (splits == 1) {   // whole K a block, the residual in its epilogue: iron_gemm_residual_bf16's 128 x 128 launch, or tiles of 96 rows where they are one round
+    const int tiles96 = (Mv + 95) / 96 * tiles_n;
+    if (tiles96 <= min(256, (int)gridDim.x) && M >= 96 && N % 128 == 0)
+      gemm_big_body<BigTile<2, 2, 3, 4>, false, false, false, true>(A, B, C, M, N, K, Mv, (M + 95) / 96, tiles_n, 0, GatedPair{}, tail);
+    else if (id < whole.tiles_m * whole.tiles_n)
       gemm_nt16_body<false>(A, B, C, M, N, K, Mv, whole.tiles_m, whole.tiles_n, whole.patched, tail);
     return;
   }
@@ -2689,14 +2704,15 @@ __device__ __forceinline__ void gemm_nt16_pair_body(const bf16_t* __restrict__ A
 // Which tile: by rounds of blocks over the CUs, as big_form, at what a round was measured to take with weights out of memory.  8192 columns over
 // K = 2048, us, by 64 x (32 + 32), 128 x (128 + 128) and 256 x (128 + 128) tiles alone and by these: 128 rows 27.9 / 25.9, 256 38.5 / 27.4, 384 39.6 /
 // 33.2, 500 41.3 / 38.6, 640 58.5 / 45.7, 768 59.1 / 48.8, 1280 111 / 87, 1536 113 / 93, 1792 114 / 105.
-enum PairForm { PAIR_64X32, PAIR_EDGED, PAIR_128X64, PAIR_160X64, PAIR_192X64, PAIR_128X128, PAIR_160X128, PAIR_192X128, PAIR_224X128, PAIR_256X128, PAIR_FORMS };
+// (96 and 224 rows as in RowsForm: 8192 columns over 2048, 119 rows 25.8 / 21.1, 394 34.7 / 31.8, 411 36.6 / 32.9, 133 to 187 23.2 / 22.3 to 23.6 / 23.9; 240 drawn ones, 69 of them, at 0.93.)
+enum PairForm { PAIR_64X32, PAIR_EDGED, PAIR_96X64, PAIR_128X64, PAIR_160X64, PAIR_192X64, PAIR_224X64, PAIR_128X128, PAIR_160X128, PAIR_192X128, PAIR_224X128, PAIR_256X128, PAIR_FORMS };
 struct PairPrice {
   int bm, bn;   // rows and columns of each product
   float start, stage;
 };
 constexpr PairPrice PAIR_PRICES[PAIR_FORMS] = {
     {64, 32, 3.f, 0.28f},    {128, 128, 7.f, 0.95f},    // (a product whose columns are no whole tiles: 128 rows at the edges' cost)
-    {128, 64, 4.f, 0.58f},   {160, 64, 4.5f, 0.64f},  {192, 64, 5.f, 0.73f},   {128, 128, 6.f, 0.90f},
+    {96, 64, 3.9f, 0.505f},  {128, 64, 4.f, 0.58f},   {160, 64, 4.5f, 0.64f},  {192, 64, 5.f, 0.73f},   {224, 64, 5.5f, 0.815f}, {128, 128, 6.f, 0.90f},
     {160, 128, 6.5f, 1.12f}, {192, 128, 7.5f, 1.2f},  {224, 128, 8.5f, 1.36f}, {256, 128, 9.5f, 1.5f},
 };
 // Whole tiles of 128 x (128 + 128) are made by the body that takes edges up to K = 2048 (us, by gemm_big_body and by that: 2048 x 2048 x 1920 33.5 / 29.6, x 960 20.9 / 19.3,
@@ -2709,6 +2725,7 @@ static PairForm pair_form(int rows, int M, int N, int K) {
     if (edged && form == PAIR_128X128) continue;
     const PairPrice& p = PAIR_PRICES[edged && form == PAIR_EDGED ? PAIR_128X128 : form];
     if (form > PAIR_EDGED && (M < p.bm || N % p.bn != 0)) continue;
+    if (K <= 8 * BK && (form == PAIR_96X64 || form == PAIR_224X64)) continue;   // (as in rows_form)
     const long tiles = (long)((rows + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
     const float us = (float)((tiles + 255) / 256) * (p.start + p.stage * (K / BK));
     if (form == PAIR_64X32 || us < price) best = (PairForm)form, price = us;
@@ -2729,9 +2746,11 @@ __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __re
     gemm_big_body<BigTile<2, 2, MI, NT>, false, false, true>(A, Bg, C, M, N, K, Mv, (M + 32 * MI - 1) / (32 * MI), N / (16 * NT), patched, pair); \
     break
   switch (chosen.form) {
+    IRON_PAIR(PAIR_96X64, 3, 4);
     IRON_PAIR(PAIR_128X64, 4, 4);
     IRON_PAIR(PAIR_160X64, 5, 4);
     IRON_PAIR(PAIR_192X64, 6, 4);
+    IRON_PAIR(PAIR_224X64, 7, 4);
     IRON_PAIR(PAIR_128X128, 4, 8);
     IRON_PAIR(PAIR_160X128, 5, 8);
     IRON_PAIR(PAIR_192X128, 6, 8);
@@ -3249,6 +3268,7 @@ extern "C" int iron_gemm_residual_norm_bf16(const uint16_t* A, const uint16_t* B
   tail.residual = R;
   tail.residual_scale = residual_scale;
   constexpr size_t lds = (size_t)NT_STAGES * 256 * BK * 2;
+  static_assert(lds >= BigTile<2, 2, 3, 4>::LDS_BYTES, "the tiles of 96 rows fit too");
   static LdsOptIn opt_in;
   if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_splitk_kernel), lds); e != hipSuccess) {
     set_error("gemm_residual_norm: %s", hipGetErrorString(e));

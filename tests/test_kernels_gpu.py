@@ -572,6 +572,14 @@ def test_every_form_of_a_launch_under_a_bound(cuda, kind, tile, size):
             assert torch.equal(run(held, held)[:rows], C[:rows]) and torch.equal(held[rows:], dR[rows:])
 
 
+# ... and tiles of 96 and 224 rows, which begin past K = 512; the last ones moved back.
+@pytest.mark.parametrize("kind,tile,size", [*((k, *f) for k in ("plain", "residual", "gated") for f in (((96, 128), (131, 576, 8208)), ((224, 128), (579, 576, 9224)),
+                                                                                                      ((224, 256), (1155, 576, 9224) if k == "plain" else (579, 1088, 16392)))),
+                                            ("pair", (96, 64), (131, 576, 2752)), ("pair", (224, 64), (387, 576, 5504))])
+def test_tiles_of_96_and_224_rows_under_a_bound(cuda, kind, tile, size):
+    test_every_form_of_a_launch_under_a_bound(cuda, kind, tile, size)
+
+
 @pytest.mark.parametrize("M,Kdim,N,form", [(*s, f) for s in ((2048, 2048, 2048), (2048, 1024, 8192), (1500, 320, 4160))
                                            for f in ("plain", "residual", "gated", "pair")] +
                          [(2048, 200, 8192, "plain"), (2048, 128, 5632, "pair"), (2000, 192, 888, "pair")])
@@ -840,6 +848,12 @@ def test_gemm_residual_then_rmsnorm_with_k_dealt_over_many_blocks(cuda, M, Kdim,
                          valid=None if rows is None else word(rows, cuda))
     sums = ws[~ws.isnan()]
     assert (sums == Kdim // slices).all() and sums.numel() == slices * (rows or M) * N
+
+
+# Whole K by tiles of 96 rows while they are one round: the last one moved back, the most rows there are, and one more.
+@pytest.mark.parametrize("M,rows", [(1500, 1473), (2048, 1536), (2048, 1537)])
+def test_gemm_residual_then_rmsnorm_by_tiles_of_96_rows(cuda, M, rows):
+    test_gemm_residual_then_rmsnorm_with_k_dealt_over_blocks(cuda, M, 4096, 2048, rows, 1.0)
 
 
 def test_gemm_residual_then_rmsnorm_refuses_other_shapes(cuda):
