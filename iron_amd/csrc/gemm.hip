@@ -2112,10 +2112,12 @@ __device__ __forceinline__ void gemm_big_body(const bf16_t* __restrict__ A, cons
 }
 
 typedef BigTile<2, 4, 8, 4> Tile256;       // 256 x 256, eight waves
+typedef BigTile<2, 4, 7, 4> Tile224x256;
 typedef BigTile<2, 4, 6, 4> Tile192x256;
 typedef BigTile<2, 4, 5, 4> Tile160x256;
 typedef BigTile<2, 4, 4, 4> Tile128x256;
-typedef BigTile<2, 4, 4, 3> Tile128x192;   // B (N,K) only
+typedef BigTile<2, 4, 4, 3> Tile128x192;   // B (N,K) only, and the following
+typedef BigTile<2, 2, 3, 4> Tile96x128;    // four waves
 typedef BigTile<2, 2, 8, 8> Tile256Four;   // 256 x 256 by four waves, for launches whose other tilings are four waves
 
 template <class T, bool B_KN = false, bool STREAM_OUT = false>
@@ -2933,7 +2935,10 @@ static int launch_gemm_big_as(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
 // The stage grows with the tile's area, so what a product gains is the part of its rounds that is not filled (us, by 128 x 128 or 256 x 256 tiles
 // alone and by the tile chosen here): 777 x 10240 x 2560 53 -> 37 (weights out of memory 63 -> 50), 2012 x 3008 x 1608 34.4 -> 24.4, 2856 x 2325 x 3176 77 -> 51, 1636 x 5256 x 6200 with
 // B (K,N) 153 -> 119, 908 x 5328 x 344 with B (K,N) 14.8 -> 9.9, 3000 x 3000 x 3000 74 -> 54.
-enum BigForm { BIG_NONE, BIG_256, BIG_192X256, BIG_160X256, BIG_128X256, BIG_128X192, BIG_FORMS };
+// Tiles of 96 x 128 by four waves and of 224 x 256 past K = 512 (up to there a round is its start and its end): 1903 x 1298 x 4440 44.3 -> 38.5, 137 x 8852 x 6136 58.4 ->
+// 49.4, 1958 x 12862 x 1248 65.7 -> 60.8, 2592 x 10736 x 1848 with B (K,N) 96.6 -> 90.9; fifty drawn products that take them 0.927 of the time, the worst 1.06 (8100 x 296 x
+// 3696).  160 x 128 and 224 x 128 by four waves take what 128 x 192 and 128 x 256 by eight do.
+enum BigForm { BIG_NONE, BIG_256, BIG_192X256, BIG_160X256, BIG_128X256, BIG_128X192, BIG_224X256, BIG_96X128, BIG_FORMS };
 struct BigPrice {
   int bm, bn;
   float start, stage[2], loose[2];
@@ -2943,6 +2948,7 @@ constexpr BigPrice BIG_PRICES[BIG_FORMS] = {
     {256, 256, 7.5f, {1.36f, 1.42f}, {1.63f, 1.48f}},  {192, 256, 5.9f, {1.10f, 1.16f}, {1.38f, 1.22f}},
     {160, 256, 4.9f, {0.92f, 0.955f}, {1.08f, 1.00f}}, {128, 256, 4.4f, {0.76f, 0.80f}, {0.95f, 0.835f}},
     {128, 192, 3.2f, {0.595f, 0.f}, {0.76f, 0.f}},     // (a stage of (K,N) rows of 192 columns is no whole number of loads)
+    {224, 256, 6.8f, {1.243f, 1.283f}, {1.505f, 1.35f}}, {96, 128, 2.f, {0.366f, 0.f}, {0.54f, 0.f}},
 };
 static float big_price(BigForm form, int M, int N, int K, bool b_nk) {
   const BigPrice& p = BIG_PRICES[form];
@@ -2956,7 +2962,7 @@ static BigForm big_form(int M, int N, int K, bool b_nk, float& price, float& pri
   price = price128 = big_price(BIG_NONE, M, N, K, b_nk);
   if (!b_nk && (long)(K + BK) * N * 2 >= (1L << 31)) return best;   // (a (K,N) matrix is addressed with 32-bit byte offsets)
   for (int form = BIG_256; form < BIG_FORMS; ++form) {
-    if (M < BIG_PRICES[form].bm || N < BIG_PRICES[form].bn || (form == BIG_128X192 && !b_nk)) continue;
+    if (M < BIG_PRICES[form].bm || N < BIG_PRICES[form].bn || (!b_nk && BIG_PRICES[form].bn != 256) || (form > BIG_128X192 && K <= 8 * BK)) continue;
     const float p = big_price((BigForm)form, M, N, K, b_nk);
     // (past four rounds of 256 x 256 tiles the smaller ones' traffic tells: 5540 x 12392 x 7728 1011 us by those, 1024 by 160 x 256, 881 by its price; with B (K,N) 128 x 128
     // tiles take more than theirs, a larger one's first rounds less: by them and by the larger 8192 x 1400 x 1608 53 / 42, 32000 x 1040 x 3904 359 / 275, 749 x 26520 x 4912
@@ -2971,10 +2977,12 @@ static int launch_gemm_big(BigForm form, const bf16_t* A, const bf16_t* B, bf16_
   // Over a long K the tiles leave by non-temporal stores (see the body's epilogue).
   if (form == BIG_256 && K >= 4096) return launch_gemm_big_as<Tile256, B_KN, true>(A, B, C, M, N, K, valid, s);
   if (form == BIG_256) return launch_gemm_big_as<Tile256, B_KN, false>(A, B, C, M, N, K, valid, s);
+  if (form == BIG_224X256) return launch_gemm_big_as<Tile224x256, B_KN, false>(A, B, C, M, N, K, valid, s);
   if (form == BIG_192X256) return launch_gemm_big_as<Tile192x256, B_KN, false>(A, B, C, M, N, K, valid, s);
   if (form == BIG_160X256) return launch_gemm_big_as<Tile160x256, B_KN, false>(A, B, C, M, N, K, valid, s);
   if constexpr (!B_KN)
-    if (form == BIG_128X192) return launch_gemm_big_as<Tile128x192, false, false>(A, B, C, M, N, K, valid, s);
+    if (form == BIG_128X192 || form == BIG_96X128)
+      return form == BIG_96X128 ? launch_gemm_big_as<Tile96x128, false, false>(A, B, C, M, N, K, valid, s) : launch_gemm_big_as<Tile128x192, false, false>(A, B, C, M, N, K, valid, s);
   return launch_gemm_big_as<Tile128x256, B_KN, false>(A, B, C, M, N, K, valid, s);
 }
 

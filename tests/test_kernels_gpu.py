@@ -572,6 +572,22 @@ def test_every_form_of_a_launch_under_a_bound(cuda, kind, tile, size):
             assert torch.equal(run(held, held)[:rows], C[:rows]) and torch.equal(held[rows:], dR[rows:])
 
 
+# Tiles of 96 x 128 and 224 x 256 without a bound, which begin past K = 512: the last ones moved back, a K that is no whole number of stages, rows that straddle lines.
+@pytest.mark.parametrize("tile,M,Kdim,N,col", [((96, 128), 902, 520, 2059, True), ((96, 128), 1798, 520, 1032, True), ((224, 256), 1413, 520, 8200, True), ((224, 256), 1350, 520, 8200, False)])
+def test_tiles_of_96_and_224_rows_without_a_bound(cuda, tile, M, Kdim, N, col):
+    code = K.lib().iron_gemm_tile(0, M, N, Kdim, col, 0, 0)
+    assert (code >> 16, code & 65535) == tile
+    rng = np.random.default_rng(M + N)
+    A, B = bf(rng, M, Kdim), bf(rng, *((N, Kdim) if col else (Kdim, N)), scale=0.05)
+    C, bounded = out_like((M, N), cuda, fill=7.0), out_like((M, N), cuda, fill=7.0)
+    kw = dict(M=M, N=N, K=Kdim, b_col_maj=col)
+    K.gemm(dev(A, cuda), dev(B, cuda), C, **kw)
+    K.gemm(dev(A, cuda), dev(B, cuda), bounded, valid=word(M, cuda), **kw)
+    assert torch.equal(C, bounded)   # the same chain of products whatever the tile
+    sample = np.unique(np.concatenate([[0, 95, 96, 223, 224, M - 97, M - 1], rng.integers(0, M, 40)]))
+    close(from_torch(C)[sample], ops.gemm(A[sample], B, b_col_maj=col), rtol=1e-2, atol=1e-2)
+
+
 # ... and tiles of 96 and 224 rows, which begin past K = 512; the last ones moved back.
 @pytest.mark.parametrize("kind,tile,size", [*((k, *f) for k in ("plain", "residual", "gated") for f in (((96, 128), (131, 576, 8208)), ((224, 128), (579, 576, 9224)),
                                                                                                       ((224, 256), (1155, 576, 9224) if k == "plain" else (579, 1088, 16392)))),
