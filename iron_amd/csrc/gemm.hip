@@ -765,18 +765,18 @@ __device__ __forceinline__ void gemm_nt64_body(const bf16_t* __restrict__ A, con
 constexpr int LONG_K = 256, LONG_ROW = LONG_K * 2;
 enum LongKind { LONG_PLAIN, LONG_PAIR, LONG_QKV };
 constexpr int long_b_rows(LongKind kind) { return kind == LONG_PAIR ? 64 : (kind == LONG_QKV ? 16 : 8); }
-constexpr int long_lds(LongKind kind, int rows, int stages) { return (rows + long_b_rows(kind)) * LONG_ROW * stages; }
-template <LongKind KIND, int LONG_ROWS, int STAGES>
+constexpr int long_lds(int rows, int b_rows, int stages) { return (rows + b_rows) * LONG_ROW * stages; }
+template <LongKind KIND, int LONG_ROWS, int STAGES, int B_ROWS = long_b_rows(KIND), bool RAGGED = false>
 __device__ __forceinline__ void gemm_long_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, bf16_t* __restrict__ C, int N, int K, int Mv,
                                                const QkvTail& qkv, const bf16_t* __restrict__ up = nullptr, bf16_t* __restrict__ gate_out = nullptr) {
-  constexpr int B_ROWS = long_b_rows(KIND), STAGE = long_lds(KIND, LONG_ROWS, 1);
-  constexpr int MI = KIND == LONG_PAIR ? LONG_ROWS / 16 : 1;                                  // tiles of A's rows a wave
+  constexpr int STAGE = long_lds(LONG_ROWS, B_ROWS, 1), GROUPS = B_ROWS < 16 ? 1 : B_ROWS / 16, WM = 4 / GROUPS;   // WM: waves a group
+  constexpr int MI = LONG_ROWS / 16 > WM ? LONG_ROWS / 16 / WM : 1;                                // tiles of A's rows a wave
   constexpr int A_INST = LONG_ROWS / 8, B_INST = B_ROWS / 8, LOADS = A_INST + B_INST;   // loads of two rows each, a wave's share
   static_assert(LONG_K == 256 && (LONG_ROWS == 32 || LONG_ROWS == 64), "two rows a load of 1 KB");
   extern __shared__ __align__(16) char smem_nt[];
   const int tile = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), fr = lane & 15, kq = lane >> 4;
-  const int group = KIND == LONG_PAIR ? wave : 0, wm = KIND == LONG_PAIR ? 0 : wave;
-  const bool computes = KIND == LONG_PAIR || wave < LONG_ROWS / 16;
+  const int group = wave / WM, wm = wave % WM;
+  const bool computes = wm * MI < LONG_ROWS / 16;
   // QKV: a tile is columns first .. + 7 and 32 + first .. of a 64-wide head of the list q | k | v.
   const int q_heads = N >> 6, kv_heads = KIND == LONG_QKV ? qkv.kv_n >> 6 : 0, head = tile >> 2, first = (tile & 3) * 8;
   const int which = KIND != LONG_QKV || head < q_heads ? 0 : (head < q_heads + kv_heads ? 1 : 2), own = head - (which == 0 ? 0 : q_heads + (which - 1) * kv_heads);
@@ -793,10 +793,17 @@ __device__ __forceinline__ void gemm_long_body(const bf16_t* __restrict__ A, con
   }
 #pragma unroll
   for (int i = 0; i < B_INST; ++i) {
-    const int r = (wave * B_INST + i) * 2 + (lane >> 5), row = KIND == LONG_PAIR ? (r >> 4) * 8 + (r & 7) : (KIND == LONG_QKV ? first + (r >> 3) * 32 + (r & 7) : r);
+    const int r = (wave * B_INST + i) * 2 + (lane >> 5);
+    if (RAGGED && n0 + r >= N) {
+      b_voff[i] = NOWHERE;
+      continue;
+    }
+    const int row = KIND == LONG_PAIR ? (r >> 4) * 8 + (r & 7) : (KIND == LONG_QKV ? first + (r >> 3) * 32 + (r & 7) : r);
     b_voff[i] = (row * K + (((lane & 31) ^ (r & 15)) << 3)) * 2;
   }
-  const int nk = K / LONG_K;
+  const int nk = RAGGED ? (K + LONG_K - 1) / LONG_K : K / LONG_K;
+  // (RAGGED: of the last stage what lies past K comes from nowhere, for A and B alike)
+  auto at = [&](int voff, int r, int kt) { return RAGGED && kt == nk - 1 && (((lane & 31) ^ (r & 15)) << 3) >= K - kt * LONG_K ? NOWHERE : voff; };
   auto issue = [&](int buffer, int kt) {   // (a stage past the last: zeros out of empty buffers, so that the waits can count)
     char* st = smem_nt + buffer * STAGE;
     const int k0 = kt * LONG_K, room = kt < nk ? 0x7fffffff : 0;
@@ -804,22 +811,22 @@ __device__ __forceinline__ void gemm_long_body(const bf16_t* __restrict__ A, con
     for (int i = 0; i < B_INST; ++i) {
       const bool second = KIND == LONG_PAIR && ((wave * B_INST + i) * 2 & 15) >= 8;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(bounded_bytes((second ? up : B) + k0, room), IRON_LDS_PTR(st + LONG_ROWS * LONG_ROW + (wave * B_INST + i) * 1024), 16,
-                                               (int)b_voff[i], 0, 0, 2);   // non-temporal
+                                               (int)at(b_voff[i], (wave * B_INST + i) * 2 + (lane >> 5), kt), 0, 0, 2);   // non-temporal
     }
 #pragma unroll
     for (int i = 0; i < A_INST; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(bounded_bytes(A + k0, room), IRON_LDS_PTR(st + (wave * A_INST + i) * 1024), 16, (int)a_voff[i], 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(bounded_bytes(A + k0, room), IRON_LDS_PTR(st + (wave * A_INST + i) * 1024), 16, (int)at(a_voff[i], (wave * A_INST + i) * 2 + (lane >> 5), kt), 0, 0, 0);
   };
   f32x4 acc[MI];
 #pragma unroll
   for (int i = 0; i < MI; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   // acc[i][e]: row fr of the wave's i-th sixteen, row 4 kq + e of the group's of B.
-  const int m_own = wm * 16 + fr, n_own = n0 + group * 8 + 4 * (kq & 1);
+  const int m_own = wm * MI * 16 + fr, n_own = KIND == LONG_PLAIN && B_ROWS > 8 ? n0 + group * 16 + 4 * kq : n0 + group * 8 + 4 * (kq & 1);
   uint2 res = make_uint2(0, 0);   // a residual's piece this lane will add
   if (KIND == LONG_PLAIN && qkv.residual != nullptr && m_own < Mv) res = *reinterpret_cast<const uint2*>(qkv.residual + (size_t)m_own * N + n_own);
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s) issue(s, s);
-  const int a_off = (wm * 16 + fr) * LONG_ROW, b_row = KIND == LONG_PLAIN ? fr & 7 : group * 16 + fr, b_off = (LONG_ROWS + b_row) * LONG_ROW, b_swz = b_row & 15;
+  const int a_off = (wm * MI * 16 + fr) * LONG_ROW, b_row = B_ROWS == 8 ? fr & 7 : group * 16 + fr, b_off = (LONG_ROWS + b_row) * LONG_ROW, b_swz = b_row & 15;
   for (int kt = 0, buffer = 0; kt < nk; ++kt) {
     wait_vmcnt<(STAGES - 2) * LOADS>();   // stage kt has landed once only the younger ones are out
     block_barrier();                      // ... in every wave, and nobody reads stage kt - 1 any more
@@ -874,7 +881,13 @@ __device__ __forceinline__ void gemm_long_body(const bf16_t* __restrict__ A, con
         }
       }
     } else {
-      if (kq >= 2) continue;
+      if (B_ROWS == 8 && kq >= 2) continue;
+      if (RAGGED && n_own + 4 > N) {
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+          if (n_own + e < N) to[e] = f32_to_bf16(x[e]);
+        continue;
+      }
       if (qkv.residual != nullptr) {
         const float rf[4] = {__uint_as_float(res.x << 16), __uint_as_float(res.x & 0xffff0000u), __uint_as_float(res.y << 16), __uint_as_float(res.y & 0xffff0000u)};
         tail_of(qkv, x, rf);
@@ -1647,7 +1660,7 @@ static int launch_qkv_either(const bf16_t* A, const bf16_t* Bq, bf16_t* Cq, int 
   const Tiling thin{thin_m, total, patched_order(thin_m, total)};
   constexpr size_t lds_narrow = (size_t)NT_STAGES * 256 * BK * 2, lds_wide = (size_t)Q3_STAGES * Q3_STAGE_BYTES;
   constexpr size_t lds = lds_narrow > lds_wide ? lds_narrow : lds_wide;
-  static_assert(lds >= (size_t)long_lds(LONG_QKV, 32, 5) && lds >= (size_t)long_lds(LONG_QKV, 64, 3), "the few rows' stages fit too");
+  static_assert(lds >= (size_t)long_lds(32, 16, 5) && lds >= (size_t)long_lds(64, 16, 3), "the few rows' stages fit too");
   static LdsOptIn opt_in;
   if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&qkv_either_kernel), lds); e != hipSuccess) {
     set_error("prefill_qkv: %s", hipGetErrorString(e));
@@ -2322,7 +2335,7 @@ static int launch_gemm_rows(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, 
   if (two_a_cu(M, N, K, valid != nullptr)) return launch_gemm_nt<false, false, 1>(A, B, C, M, N, K, valid, s, tail);
   const FormPlan plan = rows_plan(M, N, K, valid != nullptr, tail.residual != nullptr);
   constexpr size_t lds = Tile256Four::LDS_BYTES;
-  static_assert(lds >= (size_t)NT_STAGES * 256 * BK * 2 && lds >= (size_t)long_lds(LONG_PLAIN, 32, 7), "the other bodies' stages fit too");
+  static_assert(lds >= (size_t)NT_STAGES * 256 * BK * 2 && lds >= (size_t)long_lds(32, 8, 7), "the other bodies' stages fit too");
   static LdsOptIn opt_in[2];
   const auto kernel = tail.residual != nullptr ? &gemm_rows_kernel<true> : &gemm_rows_kernel<false>;
   if (hipError_t e = opt_in[tail.residual != nullptr].ensure(reinterpret_cast<const void*>(kernel), lds); e != hipSuccess) {
@@ -2780,7 +2793,7 @@ static int launch_gemm_gated_pair(const bf16_t* A, const bf16_t* Bg, const bf16_
                                   int N, int K, const int* valid, int activation, hipStream_t s) {
   const FormPlan plan = pair_plan(M, N, K, valid != nullptr);
   constexpr size_t lds = Tile256Four::LDS_BYTES;   // the largest tile's, more than the others'
-  static_assert(lds >= (size_t)PAIR_STAGES * 3 * 128 * BK * 2 && lds >= (size_t)NT_STAGES * 256 * BK * 2 && lds >= (size_t)long_lds(LONG_PAIR, 32, 3),
+  static_assert(lds >= (size_t)PAIR_STAGES * 3 * 128 * BK * 2 && lds >= (size_t)NT_STAGES * 256 * BK * 2 && lds >= (size_t)long_lds(32, 64, 3),
                 "the other bodies' stages fit too");
   static LdsOptIn opt_in;
   if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_gated_pair_kernel), lds); e != hipSuccess) {
@@ -2928,6 +2941,29 @@ static int launch_gemm_big_as(const bf16_t* A, const bf16_t* B, bf16_t* C, int M
   hipLaunchKernelGGL((gemm_big_kernel<T, B_KN, STREAM_OUT>), dim3(tiles_m * tiles_n), dim3(T::WAVES * 64), T::LDS_BYTES, s,
                      A, B, C, M, N, K, valid, tiles_m, tiles_n, patched_order(tiles_m, tiles_n));
   IRON_LAUNCH_CHECK();
+}
+
+// The same without a bound: a product of up to 32 rows, B_ROWS rows of B a block.
+template <int B_ROWS, int STAGES>
+__global__ __launch_bounds__(256) void gemm_long_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, bf16_t* __restrict__ C, int M, int N, int K) {
+  gemm_long_body<LONG_PLAIN, 32, STAGES, B_ROWS, true>(A, B, C, N, K, M, QkvTail{});
+}
+template <int B_ROWS, int STAGES>
+static int launch_gemm_long(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s) {
+  constexpr size_t lds = long_lds(32, B_ROWS, STAGES);
+  static LdsOptIn opt_in;
+  if (hipError_t e = opt_in.ensure(reinterpret_cast<const void*>(&gemm_long_kernel<B_ROWS, STAGES>), lds); e != hipSuccess) {
+    set_error("gemm: %s", hipGetErrorString(e));
+    return (int)e;
+  }
+  hipLaunchKernelGGL((gemm_long_kernel<B_ROWS, STAGES>), dim3((N + B_ROWS - 1) / B_ROWS), dim3(256), lds, s, A, B, C, M, N, K);
+  IRON_LAUNCH_CHECK();
+}
+static int launch_gemm_long(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s) {
+  if (N <= 8 * 256) return launch_gemm_long<8, 8>(A, B, C, M, N, K, s);
+  if (N <= 16 * 256) return launch_gemm_long<16, 6>(A, B, C, M, N, K, s);
+  if (N <= 32 * 256) return launch_gemm_long<32, 5>(A, B, C, M, N, K, s);
+  return launch_gemm_long<64, 3>(A, B, C, M, N, K, s);
 }
 
 // Whole tiles larger than 128 x 128, by how the rounds they make over the chip's 256 CUs come out: a round of a tile was measured
@@ -3079,6 +3115,15 @@ static bool gemm_of_few_rows(int M, int N, int K) {
   return 1.05f * few < tiles;
 }
 
+// Seventeen to thirty-two rows against B (N,K) while a round of blocks takes all of it: long stages (gemm_long_body) instead of strips, whose two tiles of rows come straight from memory
+// a fragment at a time, of 64 x 32 tiles or of shared ones.  us with the same weights again and out of memory, those / this: 31 x 2048 x 4096 11.0 / 8.9 and 12.2 / 8.9, 21 x 4096 x
+// 8192 20.6 / 16.2, 21.8 / 18.2, 26 x 16384 x 4096 40.4 / 25.2, 42.5 / 25.9, 27 x 10240 x 1024 8.8 / 6.7, 10.5 / 6.8, 22 x 1024 x 8192 14.3 / 13.3, 15.4 / 12.8; but where the
+// last-level cache holds more weights than that, or rows straddle lines, 29 x 4857 x 5648 13.4 / 18.2, 28 x 10240 x 8192 26.3 / 33.6, 22 x 5808 x 1848 7.7 / 8.2 (11.6 / 8.4 out of memory), 19 x 1925 x 3552 7.5 / 8.1,
+// over few columns 18 x 140 x 5920 9.0 / 10.0, over a short K 28 x 2048 x 512 5.6 / 6.0, and up to sixteen rows strips stay: 10 x 8192 x 4096 16.0 / 18.1, 13 x 422 x 5976 8.0 / 10.4.
+static bool gemm_of_long_stages(int M, int N, int K) {
+  return M > 16 && M <= 32 && (K > 1024 || (N > 32 * 256 && K >= LONG_K)) && N >= 256 && N <= 64 * 256 && (K % BK == 0 ? K <= (N <= 16 * 256 ? 8192 : 4096) : N <= 16 * 256 && K <= 2048);
+}
+
 // Whether the direct-to-LDS kernels take a product, B (N,K) with C (N,M) turned round before.  They take any K from one stage on (k_pad),
 // any M, and any N of B (N,K); against the general kernel, which loads through registers: 2048 x 2048 x 2056 42.5 -> 26.0 us, 86 x 1728 x
 // 5560 59 -> 26.5, (K,N) 2048 x 2048 x 2040 65 -> 22.0, 300 x 1000 x 1000 33.6 -> 9.8, 2048 x 2616 x 72 9.8 -> 6.9, 7137 x 6620 x 80 49.0 -> 30.8.
@@ -3096,7 +3141,7 @@ static bool gemm_direct_to_lds(int M, int N, int K, int b_col_maj, int c_col_maj
 // `deal`: how its tiles' K is shared where the caller brings a workspace.  Small tiles are the cheaper wherever they are one round, 128 tiles of 128 x 128
 // with a dimension of at most 64 among them (us, weights out of memory, half-empty 128 x 128 tiles / shared / small: 64 x 16384 x 8192 with B (K,N) 70 / 58 / 54,
 // 16384 x 64 71 / 87 / 59; 64 x 16320 x 200 6.0 unshared, 5.0 small).
-enum class GemmForm { FEW_ROWS, SMALL, BIG, TILES_64, TILES_128, GENERAL };
+enum class GemmForm { FEW_ROWS, LONG_STAGES, SMALL, BIG, TILES_64, TILES_128, GENERAL };
 struct GemmPlan {
   GemmForm form;
   SmallTiles small;
@@ -3105,6 +3150,10 @@ struct GemmPlan {
 };
 static GemmPlan gemm_plan(int M, int N, int K, bool b_nk, bool c_nm) {
   GemmPlan plan{GemmForm::GENERAL, {0, 0.f}, BIG_NONE, {0, 0, 0}};
+  if (b_nk && !c_nm && gemm_of_long_stages(M, N, K)) {
+    plan.form = GemmForm::LONG_STAGES;
+    return plan;
+  }
   if (b_nk && !c_nm && gemm_of_few_rows(M, N, K)) {   // fewer rows than the smallest tile: bound by streaming B
     plan.form = GemmForm::FEW_ROWS;
     return plan;
@@ -3147,6 +3196,8 @@ extern "C" int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C,
     switch (plan.form) {
       case GemmForm::FEW_ROWS:
         return iron_gemm_few_bf16(A, B, nullptr, C, M, N, K, 0, stream);
+      case GemmForm::LONG_STAGES:
+        return launch_gemm_long(A, B, C, M, N, K, s);
       case GemmForm::SMALL:
         if (b_col_maj) return high ? launch_gemm_small<13, 1, 4, 2>(A, B, C, M, N, K, s) : launch_gemm_small<20, 1, 2, 1>(A, B, C, M, N, K, s);
         if (c_col_maj) return high ? launch_gemm_small<10, 2, 2, 2, true, true>(A, B, C, M, N, K, s) : launch_gemm_small<13, 1, 2, 2, true, true>(A, B, C, M, N, K, s);

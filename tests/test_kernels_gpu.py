@@ -661,6 +661,23 @@ def test_few_rows_over_long_stages_are_the_same_bits_as_among_many(cuda, Kdim, N
             assert (got[rows:] == 7).all(), rows
 
 
+# Without a bound: eight, sixteen, thirty-two and sixty-four rows of B a block, the last block's cut; one stage, a last one of eight columns and of all but eight, more than the ring holds.
+@pytest.mark.parametrize("M", [17, 31, 32])
+@pytest.mark.parametrize("Kdim,N", [(1088, 256), (1032, 2047), (1272, 2049), (2304, 300), (2040, 1001), (1032, 4095), (1088, 4097), (1344, 8189), (320, 8200), (256, 16383)])
+@pytest.mark.parametrize("turned", [False, True])
+def test_few_rows_over_long_stages_without_a_bound(cuda, M, Kdim, N, turned):
+    """Against the oracle; turned: the (N,M) output of B and A, the same product."""
+    rng = np.random.default_rng(M + N)
+    A, B = bf(rng, M, Kdim), bf(rng, N, Kdim, scale=0.05)
+    C = out_like((M + 1, N), cuda, fill=7.0)
+    if turned:
+        K.gemm(dev(B, cuda), dev(A, cuda), C[:M], M=N, N=M, K=Kdim, b_col_maj=True, c_col_maj=True)
+    else:
+        K.gemm(dev(A, cuda), dev(B, cuda), C[:M], M=M, N=N, K=Kdim, b_col_maj=True)
+    close(from_torch(C)[:M], ops.gemm(A, B, b_col_maj=True), rtol=1e-2, atol=1e-2)
+    assert (C[M] == 7).all()
+
+
 @pytest.mark.parametrize("E", [256, 1280])
 @pytest.mark.parametrize("H,G", [(32, 8), (48, 8), (56, 8), (4, 2)])   # the most heads whose tiles are one round, and more
 def test_few_rows_projections_are_the_same_bits_as_among_many(cuda, E, H, G):
