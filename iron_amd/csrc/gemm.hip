@@ -1646,7 +1646,7 @@ static int patched_order(int tiles_m, int tiles_n) {
 
 // The rows up to which 64-row tiles of `columns` (a whole head's 64 or 32, q | k | v of `total` heads) are one round over the chip: few rows wait
 // for what a CU draws, so a tile of fewer operand rows is the faster one as long as each has a CU of its own.  Hidden 2048, 32 + 8 + 8 heads,
-// weights out of memory, us by 128 x 64 tiles and by these: 8 rows 15.8 / 10.0, 45 15.9 / 10.1, 128 16.5 / 10.2, 200 16.2 / 12.4, 320 16.4 / 13.0.
+// weights out of memory, us by 128 x 64 tiles and by these (up to 64 rows gemm_long_body's are the faster): 8 rows 15.8 / 10.0, 45 15.9 / 10.1, 128 16.5 / 10.2, 200 16.2 / 12.4, 320 16.4 / 13.0.
 static int few_qkv_rows(int total, int K, int columns) { return K < 8 * BK ? 0 : 256 / (total * 64 / columns) * 64; }
 // wide_ok: the head count comes in threes (else the 192-wide tiling is never chosen).  thin_upto: the
 // row bound up to which the one-head tiles run (0: never).
@@ -2715,7 +2715,7 @@ __device__ __forceinline__ void gemm_nt16_pair_body(const bf16_t* __restrict__ A
 
 // A gated feed-forward's two first projections over many rows as ONE launch, the tile chosen on the
 // device by the row bound as in gemm_rows_kernel.  Tiles of BN / 2 columns of both weights: a wave's columns are half gate and half up projection, so
-// the gated product is made in its registers (64 rows: on the 64 x 64 tile's loop, two waves a product; 29 x 8192 x 2048 29.7 -> 20.5 us).
+// the gated product is made in its registers (64 rows: on the 64 x 64 tile's loop, two waves a product; 29 x 8192 x 2048 29.7 -> 20.5 us; up to 32 rows by gemm_long_body, 15.8).
 // Which tile: by rounds of blocks over the CUs, as big_form, at what a round was measured to take with weights out of memory.  8192 columns over
 // K = 2048, us, by 64 x (32 + 32), 128 x (128 + 128) and 256 x (128 + 128) tiles alone and by these: 128 rows 27.9 / 25.9, 256 38.5 / 27.4, 384 39.6 /
 // 33.2, 500 41.3 / 38.6, 640 58.5 / 45.7, 768 59.1 / 48.8, 1280 111 / 87, 1536 113 / 93, 1792 114 / 105.
