@@ -2368,6 +2368,9 @@ __device__ __host__ inline int splitk_for(int tile_rows, int tiles_n, int K) {
   };
   if (keeps(16)) return 16;
   if (keeps(8)) return 8;
+  // Between eight and two, as many as the chip has CUs for, though their stages do not come out even (us with the norm, weights out of memory, four slices and five: 2048 columns
+  // over 8192, 300 rows 26.5 / 25.2, 384 30.9 / 28.2; two and three: 600 rows 44.0 / 35.0, 3072 over 8192, 384 48.1 / 38.2, 2560 over 9728, 512 55.9 / 44.3; four and six, 130 28.3 / 25.7).
+  if (live_tiles * 8 > 256 && live_tiles * 2 <= 256) return 256 / live_tiles;
   return live_tiles * 4 <= 256 ? 4 : (live_tiles * 2 <= 256 ? 2 : 1);
 }
 // Rows a slice of the workspace holds when K is dealt `splits` ways: the most that split count runs for.
@@ -2396,7 +2399,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_kernel(const bf16_t* __restri
   const int live = live_tiles * splits;
   if (id >= live) return;
   int tile, split;
-  if (live % 8 == 0 && splits <= 8) {
+  if (live % 8 == 0 && 8 % splits == 0) {
     const int xcd = id & 7, per = 8 / splits;
     split = xcd % splits;
     tile = (id >> 3) * per + xcd / splits;
@@ -2405,8 +2408,9 @@ __global__ __launch_bounds__(256) void gemm_splitk_kernel(const bf16_t* __restri
     tile = id / splits;
   }
   tail.residual = nullptr;   // the second launch adds it
-  tail.k_len = K / splits;
-  tail.k_begin = split * tail.k_len;
+  const int stages = K / BK, first = split * stages / splits;
+  tail.k_begin = first * BK;
+  tail.k_len = ((split + 1) * stages / splits - first) * BK;
   tail.partial = partial + (size_t)split * splitk_slice_rows(splits, tiles_n) * N;
   tail.tile_plus1 = tile + 1;
   gemm_nt16_body<false>(A, B, C, M, N, K, Mv, (Mv + 127) / 128, tiles_n, 0, tail);
@@ -2468,7 +2472,7 @@ __global__ __launch_bounds__(256) void gemm_finish_rows_kernel(const float* __re
         for (int sl = 1; sl < kSplitKMax; ++sl)
           if (sl < splits) sum[i][h] += __builtin_bit_cast(f32x4, part[i][sl][h]);
       }
-    for (int first = kSplitKMax; first < splits; first += kSplitKMax) {   // (past four, the split count is a multiple of it)
+    for (int first = kSplitKMax; first < splits; first += kSplitKMax) {   // (slices past the last: zeros)
       request(first);
 #pragma unroll
       for (int i = 0; i < CHUNKS; ++i)

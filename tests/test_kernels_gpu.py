@@ -883,6 +883,19 @@ def test_gemm_residual_then_rmsnorm_with_k_dealt_over_many_blocks(cuda, M, Kdim,
     assert (sums == Kdim // slices).all() and sums.numel() == slices * (rows or M) * N
 
 
+# Three, five, six and seven slices, whose stages do not come out even: rows on either side of a count, a K of 64 and of 72 stages, a bound inside a tile.
+@pytest.mark.parametrize("M,Kdim,N,rows,slices", [(1024, 4096, 2048, 640, 3), (1024, 4096, 2048, 641, 2), (384, 4608, 2048, 300, 5), (128, 4096, 5120, 77, 6), (512, 4096, 1152, 500, 7),
+                                                  (512, 4608, 1024, 512, 4)])
+def test_gemm_residual_then_rmsnorm_with_k_dealt_unevenly(cuda, M, Kdim, N, rows, slices):
+    test_gemm_residual_then_rmsnorm_with_k_dealt_over_blocks(cuda, M, Kdim, N, rows, 1.0)
+    A, B, R = (torch.ones(s, dtype=torch.bfloat16, device=cuda) for s in ((M, Kdim), (N, Kdim), (M, N)))
+    ws = torch.full((K.gemm_residual_norm_workspace_bytes(M, N, Kdim) // 4,), float("nan"), dtype=torch.float32, device=cuda)
+    K.gemm_residual_norm(A, B, R, R[0], torch.empty_like(R), torch.empty_like(R), ws, M=M, N=N, K=Kdim, eps=1e-6, valid=word(rows, cuda))
+    sums, stages = ws[~ws.isnan()], Kdim // 64
+    assert sums.numel() == slices * rows * N and int(sums.double().sum()) == Kdim * rows * N
+    assert set(sums.unique().tolist()) <= {64.0 * (stages // slices), 64.0 * -(-stages // slices)}
+
+
 # Whole K by tiles of 96 rows while they are one round: the last one moved back, the most rows there are, and one more.
 @pytest.mark.parametrize("M,rows", [(1500, 1473), (2048, 1536), (2048, 1537)])
 def test_gemm_residual_then_rmsnorm_by_tiles_of_96_rows(cuda, M, rows):
