@@ -1033,6 +1033,7 @@ class ScratchArena:
         self.buffer = None  # torch.uint8 on the GPU
         self.uploaded: set[int] = set()
         self.generation = 0
+        self.launched = 0   # calls, starts and runs of replays of any version so far
 
     def place_resident(self, r: Resident) -> int:
         if id(r) not in self.resident_offsets:
@@ -1522,6 +1523,11 @@ class CompiledGraph:
                 carried[k] = int(v)
         return carried
 
+    @property
+    def launched(self) -> int:
+        """How often a version of the arena was launched so far: who finds another count than it left has been interrupted."""
+        return self.arena.launched
+
     def _launch_once(self, tensors, values):
         """One launch of everything; the outputs and the call's values."""
         import torch
@@ -1548,6 +1554,7 @@ class CompiledGraph:
         defaults = {v.name: v.default for v in rec.values if v.default is not None}
         full = rec.check_values({**defaults, **values})  # refused before any dispatch
         self.load()
+        self.arena.launched += 1
         for i, (dst, src) in enumerate(zip(self.input_tensors, staged)):
             if src.device.type == "cpu" and not src.is_pinned():
                 # A host array goes through a pinned buffer of this input's own (pageable memory would
@@ -1594,6 +1601,7 @@ class CompiledGraph:
         defaults = {v.name: v.default for v in rec.values if v.default is not None}
         full = rec.check_values({**defaults, **values})
         self.load()
+        self.arena.launched += 1
         self._write_words(full)
         if self._graph is None:
             raise RuntimeError(f"{rec.name}: this version is not captured in a HIP graph")
@@ -1618,6 +1626,7 @@ class CompiledGraph:
             self.recording.check_values(last)
         except IndexError as e:
             raise IndexError(f"{e}; {n} replay(s) from {known} leave the limits") from None
+        self.arena.launched += 1
         if self._graph_bounded is None:
             for _ in range(n):
                 self._graph.replay()

@@ -279,6 +279,11 @@ class CausalLM(iron.Graph):
         (row,) = self.decode_step.run(**values) if ids is None else self.prompt_chunk.run(ids, **values)
         return row
 
+    @property
+    def launched(self):
+        """What the versions say has been launched so far (see ``CompiledGraph.launched``)."""
+        return tuple(getattr(v, "launched", None) for v in (self.decode_step, self.prompt_chunk))
+
     # ------------------------------------------------------------------ use
     def logits(self, tokens) -> np.ndarray:
         """Logits after the last of ``tokens`` (see ``Session.logits``)."""
@@ -337,11 +342,13 @@ class _HostVersion:
     """A version stood in by the graph's host reference: same call, numpy underneath."""
 
     captured = False
+    launched = 0
 
     def __init__(self, graph, takes_ids: bool):
         self.graph, self.takes_ids = graph, takes_ids
 
     def __call__(self, *tensors, **values):
+        self.launched += 1
         outs, carried = iron.Graph.reference(self.graph, *tensors, **values)
         return (*(_HostOutput(o) for o in outs), iron.Carry(carried))
 

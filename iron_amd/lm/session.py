@@ -141,6 +141,9 @@ class Session:
         token as soon as its step has run, or the step is not captured: then the host starts each
         step from the last one's carried values.
 
+        Between two tokens the model may be called, also by other draws: what that replaced in the
+        caches and the draw rows is put back before the next token, and the tokens are the same.
+
         Raises:
             ValueError: the history and the draws do not fit the caches.
             RuntimeError: the model's versions are not loaded.
@@ -153,7 +156,8 @@ class Session:
             raise RuntimeError(f"{type(model).__name__}: load_versions() first")
         self._claim()
         prompt_len = ids.size
-        self._stage_draw_rows(sampler, prompt_len, max_tokens)
+        table = self._draw_rows(sampler, prompt_len, max_tokens)
+        self._stage_draw_rows(table)
         begin = self.resume(self._reusable(ids))
         # Until the run is over nobody knows how far it got (the caller may stop iterating).
         self.cached = self.cached[:0]
@@ -168,31 +172,65 @@ class Session:
         else:
             _, carried = model(*inputs, **words)
         out = [int(carried["token"])]
+        ran = model.launched
         yield out[0]
         if replayed:
+            if self._interrupted(ran):
+                self._regain(ids, [], table)
+                step, started = model.decode_step, False
             if not started:
                 step.start(**carried)
             step.replay(remaining - 1)
             record = step.read(model.drawn)       # position p holds the token drawn at p
-            for token in record[prompt_len : prompt_len + remaining]:
-                out.append(int(token))
-                yield out[-1]
+            ran = model.launched
+            for token in record[prompt_len : prompt_len + remaining].tolist():
+                out.append(token)
+                yield token
         else:
             for _ in range(remaining):
+                if self._interrupted(ran):
+                    self._regain(ids, out[:-1], table)
                 _, carried = model(**carried)
                 out.append(int(carried["token"]))
+                ran = model.launched
                 yield out[-1]
-        # Every drawn token but the last has been through a step and has its cache rows.
-        self.cached = np.concatenate([ids, np.asarray(out[:-1], dtype=np.int64)])
+        if not self._interrupted(ran):
+            # Every drawn token but the last has been through a step and has its cache rows.
+            self.cached = np.concatenate([ids, np.asarray(out[:-1], dtype=np.int64)])
 
-    def _stage_draw_rows(self, sampler, prompt_len: int, count: int) -> None:
-        """Write the draw rows for positions ``prompt_len - 1`` onwards; all-zero rows draw greedily.
-        A greedy run after a greedy run finds the table already zero and writes nothing."""
+    def _interrupted(self, ran) -> bool:
+        """Whether anything of the model ran since ``ran`` was its count of launches."""
+        return self.lm.holder is not self or self.lm.launched != ran
+
+    def _regain(self, prompt: np.ndarray, drawn, table) -> None:
+        """Draw rows and caches as a draw had them behind ``prompt`` and the ``drawn`` tokens: what another run left of them
+        stays, the rest is run again, a prompt's rows by chunks and a drawn token's by its step."""
         model = self.lm
-        if sampler is None and not model.sampled:
+        if model.prompt_chunk is None or model.decode_step is None:
+            raise RuntimeError(f"{type(model).__name__}: load_versions() first")
+        self._claim()
+        self._stage_draw_rows(table)
+        ids = np.concatenate([prompt, np.asarray(drawn, dtype=np.int64)])
+        begin = self.resume(_common_prefix(ids, self.cached))
+        self.cached = self.cached[:0]
+        for inputs, words in self.chunk_calls(prompt, begin):
+            model.run(*inputs, **words)
+        for position in range(max(begin, prompt.size), ids.size):
+            model.run(token=int(ids[position]), position=position)
+
+    def _draw_rows(self, sampler, prompt_len: int, count: int) -> np.ndarray | None:
+        """The draw rows of ``count`` tokens from position ``prompt_len - 1`` on; none for a greedy run."""
+        if sampler is None:
+            return None
+        table = np.zeros((self.lm.config.max_seq_len, ROW_WORDS), dtype=np.int32)
+        table[prompt_len - 1 : prompt_len - 1 + count] = sampler.rows(count, self.lm.k_max)
+        return table
+
+    def _stage_draw_rows(self, table: np.ndarray | None) -> None:
+        """Write the draw rows; all-zero rows draw greedily.  A greedy run after a greedy run finds
+        the table already zero and writes nothing."""
+        model = self.lm
+        if table is None and not model.sampled:
             return
-        table = np.zeros((model.config.max_seq_len, ROW_WORDS), dtype=np.int32)
-        if sampler is not None:
-            table[prompt_len - 1 : prompt_len - 1 + count] = sampler.rows(count, model.k_max)
-        model.decode_step.write(model.draws, table)
-        model.sampled = sampler is not None
+        model.decode_step.write(model.draws, np.zeros((model.config.max_seq_len, ROW_WORDS), np.int32) if table is None else table)
+        model.sampled = table is not None

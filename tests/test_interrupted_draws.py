@@ -1,0 +1,161 @@
+"""A draw whose consumer uses the model between two of its tokens: its tokens, and what the session then says the caches hold,
+are those of a draw that nothing came between.  Device-free: the versions are the graph's host reference, also stood in as
+captured ones (the first step launched behind the prompt, the rest replayed)."""
+
+import dataclasses
+import functools
+
+import numpy as np
+import pytest
+
+import oracle
+from iron_amd.applications.llama import Llama
+from iron_amd.lm import Sampler
+from iron_amd.lm.causal import OnHost, _HostVersion
+from iron_amd.lm.session import Session
+from tests.llama_support import SCALED, weights
+
+oracle.install()
+
+CONFIG = dataclasses.replace(SCALED, prefill_chunk=16, max_seq_len=48, num_hidden_layers=1)
+RING = dataclasses.replace(CONFIG, max_seq_len=192, sliding_window=5)
+
+
+class Captured(_HostVersion):
+    """A captured version's contract: ``start`` sets the words, ``replay`` goes on from what the last run carried."""
+
+    captured = True
+    hands = True
+
+    def start(self, **values):
+        *_, self.words = self(**values)
+
+    def replay(self, n=1):
+        for _ in range(n):
+            self.start(**self.words)
+
+    def hands_over(self, to):
+        return self.hands
+
+    def run_and_start(self, to, *tensors, **values):
+        *_, carried = self(*tensors, **values)
+        to.start(**carried)
+        return carried
+
+
+class Eager(OnHost, Llama):
+    pass
+
+
+class Replayed(OnHost, Llama):
+    def load_versions(self, **_):
+        self.use(Captured(self, False), Captured(self, True))
+
+
+class Started(Replayed):
+    """As captured versions that cannot hand over."""
+
+    def load_versions(self, **_):
+        super().load_versions()
+        self.prompt_chunk.hands = False
+
+
+def loaded(cls, config):
+    model = cls(config, weights(config))
+    model.load_versions()
+    return model
+
+
+def other(token):
+    return (int(token) + 1) % CONFIG.vocab_size
+
+
+def another_token(model, prompt, drawn):
+    model.logits([*prompt, *drawn[:-1], other(drawn[-1])])
+
+
+def another_token_and_a_step(model, prompt, drawn):
+    foreign = [*prompt, *drawn[:-1], other(drawn[-1])]
+    model.logits(foreign)
+    model.logits([*foreign, 3])
+
+
+def another_history(model, prompt, drawn):
+    model.logits(prompt[::-1])
+
+
+def another_draw(model, prompt, drawn):
+    given_up = model.session.draw(prompt[:5], 6, Sampler(1.5, 50, seed=9))
+    next(given_up), next(given_up)
+    given_up.close()
+
+
+def another_greedy_draw(model, prompt, drawn):
+    assert len(list(model.session.draw(prompt[:5], 6))) == 6
+
+
+def another_session(model, prompt, drawn):
+    Session(model).logits(prompt[3:])
+
+
+def a_call_of_its_own(model, prompt, drawn):
+    model(token=7, position=2)
+
+
+BETWEEN = [another_token, another_token_and_a_step, another_history, another_draw, another_greedy_draw, another_session, a_call_of_its_own]
+
+
+@functools.cache
+def alone(config, sampler, cls, each):
+    """A prompt, what is drawn behind it, and the logits behind that."""
+    prompt = np.random.default_rng(4).integers(0, config.vocab_size, 21).tolist()
+    model = loaded(cls, config)
+    tokens = list(model.session.draw(prompt, 4, sampler(), each=each))
+    return prompt, tokens, model.logits([*prompt, *tokens])
+
+
+def sampled():
+    return Sampler(1.5, 50, seed=2)
+
+
+def greedy():
+    return None
+
+
+@pytest.mark.parametrize("between", BETWEEN, ids=lambda f: f.__name__)
+@pytest.mark.parametrize("config, sampler, cls, each", [(CONFIG, sampled, Eager, False), (CONFIG, sampled, Replayed, False), (CONFIG, greedy, Replayed, False),
+                                                        (CONFIG, sampled, Replayed, True), (CONFIG, sampled, Started, False), (RING, greedy, Replayed, False),
+                                                        (RING, greedy, Eager, False)])
+def test_what_a_consumer_does_between_two_tokens_changes_nothing(config, sampler, cls, each, between):
+    prompt, tokens, behind = alone(config, sampler, cls, each)
+    model = loaded(cls, config)
+    for places in ((1,), (1, 3), (4,)):
+        model.session.forget(0)
+        drawn = []
+        for token in model.session.draw(prompt, 4, sampler(), each=each):
+            drawn.append(token)
+            if len(drawn) in places:
+                between(model, prompt, drawn)
+        assert drawn == tokens, places
+        # Whatever the session now takes the caches to hold is there (rows made by a chunk and by steps differ by roundings).
+        got = model.logits([*prompt, *tokens])
+        assert np.abs(got - behind).max() <= 0.02 * np.abs(behind).max(), places
+
+
+@pytest.mark.parametrize("cls", [Eager, Replayed, Started])
+def test_two_draws_of_one_session_taken_in_turn(cls):
+    prompts = [np.random.default_rng(s).integers(0, CONFIG.vocab_size, n).tolist() for s, n in ((4, 21), (5, 9))]
+    want = [list(loaded(cls, CONFIG).session.draw(p, 5)) for p in prompts]
+    model = loaded(cls, CONFIG)
+    assert list(zip(*(model.session.draw(p, 5) for p in prompts))) == list(zip(*want))
+
+
+def test_a_draw_that_nothing_came_between_runs_nothing_twice():
+    model, runs = loaded(Replayed, CONFIG), []
+    prompt = np.random.default_rng(4).integers(0, CONFIG.vocab_size, 21).tolist()
+    call = Captured.__call__
+    for version in (model.decode_step, model.prompt_chunk):
+        version.__class__ = type("Counted", (Captured,), {"__call__": lambda self, *t, **v: (runs.append(v["position"]), call(self, *t, **v))[1]})
+    assert len(list(model.session.draw(prompt, 5))) == 5
+    assert runs == [15, 20, 21, 22, 23, 24]
+    assert model.session.cached.size == 25

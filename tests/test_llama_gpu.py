@@ -410,6 +410,38 @@ def test_a_draw_starts_its_second_step_behind_the_prompt_on_the_device(toy, monk
     assert list(toy.session.draw(prompt, 12)) == stepwise
 
 
+@pytest.mark.parametrize("hands_over", [True, False])
+def test_a_draw_goes_on_as_if_its_consumer_had_not_used_the_model(toy, monkeypatch, hands_over):
+    """Behind the first token, whose step is already on the device, and behind later ones: another token in the row that this step fills, a step of its
+    own behind that, another sampled draw, another history; then the tokens and what the caches hold are those of an undisturbed draw."""
+    from iron_amd.lm.generation import Sampler
+
+    prompt = np.random.default_rng(33).integers(0, SCALED.vocab_size, 60).tolist()
+    if not hands_over:
+        monkeypatch.setattr(type(toy.prompt_chunk), "hands_over", lambda *_: False)
+    for sampler in (lambda: None, lambda: Sampler(1.5, 50, seed=6)):
+        toy.session.forget(0)
+        stepwise = list(toy.session.draw(prompt, 12, sampler(), each=True))
+        behind = toy.logits(prompt + stepwise)
+        foreign = prompt + [(stepwise[0] + 1) % SCALED.vocab_size]
+        between = [lambda: toy.logits(foreign), lambda: (toy.logits(foreign), toy.logits([*foreign, 3])), lambda: next(toy.session.draw(prompt[:9], 4, Sampler(1.5, 50, seed=7))),
+                   lambda: toy.logits(prompt[::-1])]
+        for disturb in between:
+            for places in ((1,), (1, 2, 12)):
+                toy.session.forget(0)
+                drawn = []
+                for token in toy.session.draw(prompt, 12, sampler()):
+                    drawn.append(token)
+                    if len(drawn) in places:
+                        disturb()
+                assert drawn == stepwise
+                got = toy.logits(prompt + stepwise)
+                assert np.abs(got - behind).max() <= 0.02 * np.abs(behind).max()
+    toy.session.forget(0)
+    pair = [list(toy.session.draw(p, 12)) for p in (prompt, prompt[7:30])]
+    assert list(zip(*(toy.session.draw(p, 12) for p in (prompt, prompt[7:30])))) == list(zip(*pair))
+
+
 @pytest.fixture(scope="module")
 def deep(cuda):
     """Two layers at Llama-3.2-1B's width over caches of 16384 rows in 2048-row chunks, on the GPU and
