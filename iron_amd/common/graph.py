@@ -1034,6 +1034,7 @@ class ScratchArena:
         self.uploaded: set[int] = set()
         self.generation = 0
         self.launched = 0   # calls, starts and runs of replays of any version so far
+        self.running = None   # the end of what a call left running behind its return
 
     def place_resident(self, r: Resident) -> int:
         if id(r) not in self.resident_offsets:
@@ -1077,7 +1078,33 @@ class ScratchArena:
         n = math.prod(shape) * itemsize(dtype)
         return self.buffer[offset : offset + n].view(tdtype).view(tuple(shape) or (1,))
 
+    def leave_running(self) -> None:
+        """A call returns with work on the arena still queued on this stream: whoever touches the arena next, on whatever stream, is behind it
+        (``enter``), and so is whoever is given the memory next."""
+        import torch
+
+        self.running = torch.cuda.Event()
+        self.running.record()
+        self.buffer.record_stream(torch.cuda.current_stream())
+
+    def enter(self) -> None:
+        if self.running is None:
+            return
+        import torch
+
+        if self.running.query():
+            self.running = None
+        else:
+            torch.cuda.current_stream().wait_event(self.running)
+
+    def settle(self) -> None:
+        """Wait on the host for what was left running."""
+        if self.running is not None:
+            self.running.synchronize()
+            self.running = None
+
     def release(self) -> None:
+        self.settle()
         self.buffer = None
         self.uploaded.clear()
 
@@ -1432,12 +1459,14 @@ class CompiledGraph:
     def write(self, resident: Resident, array) -> None:
         """Write a state or weight of the graph from a host array."""
         self.load()
+        self.arena.enter()
         off = self.arena.resident_offsets[id(resident)]
         self.arena.view(off, resident.shape, resident.dtype).copy_(_host_tensor(np.asarray(array), resident.dtype))
 
     def read(self, resident: Resident) -> np.ndarray:
         """A state or weight as the device left it: a host copy, which ``push`` sends back."""
         self.load()
+        self.arena.enter()
         off = self.arena.resident_offsets[id(resident)]
         array = from_torch(self.arena.view(off, resident.shape, resident.dtype))
         vars(self).setdefault("_read", {})[id(resident)] = array
@@ -1479,7 +1508,8 @@ class CompiledGraph:
 
     def run_and_start(self, to: CompiledGraph, *tensors, **values) -> Carry:
         """Run the version, and ``to`` once (``start``) from the values it carries, those that the device makes handed over there; returns them.  The host waits
-        for them behind both launches: the device goes from one to the other at once (10 of the 40 to 50 us that it stood still remain)."""
+        for them behind both launches: the device goes from one to the other at once (10 of the 40 to 50 us that it stood still remain), and still runs
+        ``to`` when this returns."""
         import torch
 
         from .. import kernels
@@ -1507,6 +1537,7 @@ class CompiledGraph:
         for k, (tensor, _) in made.items():
             kernels.copy_rows(tensor.view(1), to.words[to.slots[k] : to.slots[k] + 1], rows=1, row_elems=1, src_rows=1, dst_rows=1)
         to._replay_at(start)
+        self.arena.leave_running()
         arrived.synchronize()
         for k, (_, host) in made.items():
             known[k] = to._host_values[k] = int(host[0])
@@ -1555,6 +1586,7 @@ class CompiledGraph:
         full = rec.check_values({**defaults, **values})  # refused before any dispatch
         self.load()
         self.arena.launched += 1
+        self.arena.enter()
         for i, (dst, src) in enumerate(zip(self.input_tensors, staged)):
             if src.device.type == "cpu" and not src.is_pinned():
                 # A host array goes through a pinned buffer of this input's own (pageable memory would
@@ -1602,6 +1634,7 @@ class CompiledGraph:
         full = rec.check_values({**defaults, **values})
         self.load()
         self.arena.launched += 1
+        self.arena.enter()
         self._write_words(full)
         if self._graph is None:
             raise RuntimeError(f"{rec.name}: this version is not captured in a HIP graph")
@@ -1627,6 +1660,7 @@ class CompiledGraph:
         except IndexError as e:
             raise IndexError(f"{e}; {n} replay(s) from {known} leave the limits") from None
         self.arena.launched += 1
+        self.arena.enter()
         if self._graph_bounded is None:
             for _ in range(n):
                 self._graph.replay()
@@ -1664,6 +1698,7 @@ class CompiledGraph:
                 raise AssertionError(f"{self.recording.name}: step {op.name}: {bad}")
 
     def release(self) -> None:
+        self.arena.settle()
         self._graph = self._graph_bounded = None
         self._launches = []
         self._loaded_generation = None

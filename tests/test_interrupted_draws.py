@@ -1,6 +1,7 @@
 """A draw whose consumer uses the model between two of its tokens: its tokens, and what the session then says the caches hold,
-are those of a draw that nothing came between.  Device-free: the versions are the graph's host reference, also stood in as
-captured ones (the first step launched behind the prompt, the rest replayed)."""
+are those of a draw that nothing came between; and whatever it uses it on, a stream of its own too, is behind the step that a draw
+leaves running.  Device-free: the versions are the graph's host reference, also stood in as captured ones (the first step
+launched behind the prompt, the rest replayed), or compiled ones whose streams and graphs only take notes."""
 
 import dataclasses
 import functools
@@ -159,3 +160,86 @@ def test_a_draw_that_nothing_came_between_runs_nothing_twice():
     assert len(list(model.session.draw(prompt, 5))) == 5
     assert runs == [15, 20, 21, 22, 23, 24]
     assert model.session.cached.size == 25
+
+
+class Notes:
+    """Streams, events and graphs that note, a stream each, what would be put on it."""
+
+    def __init__(self, monkeypatch):
+        import torch
+
+        self.on = {"own": [], "other": []}
+        self.stream = "own"
+        notes = self
+
+        class Event:
+            def record(self):
+                self.at = (notes.stream, len(notes.on[notes.stream]))
+
+            def query(self):
+                return False
+
+            def synchronize(self):
+                notes.on["host"] = notes.on.get("host", []) + [self.at]
+
+        class Stream:
+            def wait_event(self, event):
+                notes.on[notes.stream].append(("behind", event.at))
+
+        monkeypatch.setattr(torch.cuda, "Event", Event)
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda: Stream())
+        monkeypatch.setattr(torch.Tensor, "record_stream", lambda tensor, stream: notes.put("held"))
+
+    def put(self, what):
+        self.on[self.stream].append(what)
+
+    def replay(self):   # a captured graph's
+        self.put("graph")
+
+
+USES = {
+    "a call": lambda model, prompt: prompt.run(np.zeros(CONFIG.prefill_chunk, np.int32), token=1, position=0, start=0, rows=1, rope_start=0),
+    "a start": lambda model, prompt: model.decode_step.start(token=1, position=3),
+    "a replay": lambda model, prompt: model.decode_step.replay(2),
+    "a write": lambda model, prompt: model.decode_step.write(model.draws, np.zeros((CONFIG.max_seq_len, 4), np.int32)),
+    "a read": lambda model, prompt: model.decode_step.read(model.drawn),
+}
+
+
+@pytest.mark.parametrize("use", [*USES, "a release"])
+def test_the_step_that_a_draw_leaves_running_is_ahead_of_whatever_comes_next(monkeypatch, use):
+    import torch
+
+    from iron_amd import kernels
+    from iron_amd.common.graph import WORD_SLOTS, CompiledGraph
+
+    model = Llama(CONFIG, weights(CONFIG))
+    decode, prompt = (model.compile(capture=True, **shapes) for shapes in model.shapes())
+    model.use(decode, prompt)
+    notes = Notes(monkeypatch)
+    arena = model.arena
+    arena.buffer = torch.zeros(arena.nbytes, dtype=torch.uint8)
+    monkeypatch.setattr(CompiledGraph, "load", lambda self: self)
+    monkeypatch.setattr(kernels, "copy_rows", lambda *a, **k: notes.put("token"))
+    pinned_empty = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *shape, pin_memory=False, **kw: pinned_empty(*shape, **kw))
+    monkeypatch.setattr(torch.Tensor, "pin_memory", lambda tensor: tensor)
+    for version in (decode, prompt):
+        version.words = arena.view(arena.resident_offsets[id(version._words_resident)], (WORD_SLOTS,), np.int32)
+        version.host_words = torch.zeros(WORD_SLOTS, dtype=torch.int32)
+        version._host_words_np, version._staging, version._graph = version.host_words.numpy(), {}, notes
+        version.input_tensors = [version._tensor(h) for h in version.recording.inputs]
+        version.output_tensors = [version._tensor(h) for h in version.recording.outputs]
+    assert prompt.hands_over(decode)
+    *_, (inputs, words) = model.session.chunk_calls([1, 2, 3])
+    prompt.run_and_start(decode, *inputs, **words)
+    own = notes.on["own"]
+    assert own[:3] == ["graph", "token", "graph"] and "held" in own   # the portion, its token's way into the words, the step; the memory is this stream's too
+    end = ("own", 3)
+    notes.stream = "other"
+    if use == "a release":
+        model.release()
+        assert notes.on["host"][-1] == end and decode._graph is None
+        return
+    USES[use](model, prompt)
+    assert notes.on["other"][0] == ("behind", end)

@@ -442,6 +442,24 @@ def test_a_draw_goes_on_as_if_its_consumer_had_not_used_the_model(toy, monkeypat
     assert list(zip(*(toy.session.draw(p, 12) for p in (prompt, prompt[7:30])))) == list(zip(*pair))
 
 
+def test_a_draw_s_consumer_may_use_the_model_on_another_stream(toy):
+    """The step that is still running at the first token is ahead of another stream's call, and of the draw where it goes on there."""
+    import torch
+
+    prompt, aside = np.random.default_rng(35).integers(0, SCALED.vocab_size, 60).tolist(), torch.cuda.Stream()
+    stepwise = list(toy.session.draw(prompt, 12, each=True))
+    want = toy.logits(foreign := prompt + [(stepwise[0] + 1) % SCALED.vocab_size])
+    for uses in (True, False):
+        draw = toy.session.draw(prompt, 12)
+        drawn = [next(draw)]
+        with torch.cuda.stream(aside):
+            if uses:
+                assert np.array_equal(toy.logits(foreign), want)
+            drawn += draw
+        assert drawn == stepwise
+    toy.session.forget(0)
+
+
 @pytest.fixture(scope="module")
 def deep(cuda):
     """Two layers at Llama-3.2-1B's width over caches of 16384 rows in 2048-row chunks, on the GPU and
