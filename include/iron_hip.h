@@ -39,7 +39,8 @@ int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int
 /* The same product where its tiles come out badly as rounds over the chip (a few tiles over a long K, or
  * a last round nearly empty): some tiles' K is dealt over several blocks whose float32 sums meet in
  * `workspace` (16-byte aligned, iron_gemm_workspace_bytes of it; what it holds does not matter).  0 bytes: the product
- * shares no tiles, and iron_gemm_shared_bf16 refuses it. */
+ * shares no tiles, and iron_gemm_shared_bf16 refuses it, or, where tiles of another size or long stages have become
+ * cheaper than shared ones, makes it by those and leaves the workspace alone. */
 int64_t iron_gemm_workspace_bytes(int M, int N, int K, int b_col_maj, int c_col_maj);
 int iron_gemm_shared_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K, int b_col_maj,
                           int c_col_maj, void* workspace, void* stream);

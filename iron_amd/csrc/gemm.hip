@@ -2995,13 +2995,13 @@ static float big_price(BigForm form, int M, int N, int K, bool b_nk) {
   const long tiles = (long)((M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
   return (float)((tiles + 255) / 256) * (p.start + (K % BK == 0 ? p.stage : p.loose)[!b_nk] * ((K + BK - 1) / BK));
 }
-// The form for a product without a row bound, and what it and the 128 x 128 tiles are expected to take.
-static BigForm big_form(int M, int N, int K, bool b_nk, float& price, float& price128) {
+// The form before `end` for a product without a row bound, and what it and the 128 x 128 tiles are expected to take.
+static BigForm big_form(int M, int N, int K, bool b_nk, float& price, float& price128, int end = BIG_FORMS) {
   const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
   BigForm best = BIG_NONE;
   price = price128 = big_price(BIG_NONE, M, N, K, b_nk);
   if (!b_nk && (long)(K + BK) * N * 2 >= (1L << 31)) return best;   // (a (K,N) matrix is addressed with 32-bit byte offsets)
-  for (int form = BIG_256; form < BIG_FORMS; ++form) {
+  for (int form = BIG_256; form < end; ++form) {
     if (M < BIG_PRICES[form].bm || N < BIG_PRICES[form].bn || (!b_nk && BIG_PRICES[form].bn != 256) || (form > BIG_128X192 && K <= 8 * BK)) continue;
     const float p = big_price((BigForm)form, M, N, K, b_nk);
     // (past four rounds of 256 x 256 tiles the smaller ones' traffic tells: 5540 x 12392 x 7728 1011 us by those, 1024 by 160 x 256, 881 by its price; with B (K,N) 128 x 128
@@ -3152,9 +3152,10 @@ struct GemmPlan {
   BigForm big;
   TileShares deal;
 };
-static GemmPlan gemm_plan(int M, int N, int K, bool b_nk, bool c_nm) {
+// `all`: false leaves out long stages and the tiles of 96 and 224 rows, for iron_gemm_shared_bf16.
+static GemmPlan gemm_plan(int M, int N, int K, bool b_nk, bool c_nm, bool all = true) {
   GemmPlan plan{GemmForm::GENERAL, {0, 0.f}, BIG_NONE, {0, 0, 0}};
-  if (b_nk && !c_nm && gemm_of_long_stages(M, N, K)) {
+  if (all && b_nk && !c_nm && gemm_of_long_stages(M, N, K)) {
     plan.form = GemmForm::LONG_STAGES;
     return plan;
   }
@@ -3166,7 +3167,7 @@ static GemmPlan gemm_plan(int M, int N, int K, bool b_nk, bool c_nm) {
   const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
   float big = 0.f, price128 = 0.f, shared = 0.f;
   plan.small = small_tiles(M, N, K, b_nk);
-  if (!c_nm && tiles128 >= 128) plan.big = big_form(M, N, K, b_nk, big, price128);
+  if (!c_nm && tiles128 >= 128) plan.big = big_form(M, N, K, b_nk, big, price128, all ? BIG_FORMS : BIG_224X256);
   // 128 x 128 tiles that would occupy under half the CUs give way to 64 x 64 ones, and so do tiles that up to 64 rows would half fill at
   // most (64 x 16384 x 8184: 93 -> 68 us).
   plan.form = plan.small.rows > 0 ? GemmForm::SMALL : (plan.big != BIG_NONE ? GemmForm::BIG : (b_nk && (tiles128 < 128 || M <= 64) ? GemmForm::TILES_64 : GemmForm::TILES_128));
@@ -3246,6 +3247,9 @@ extern "C" int iron_gemm_shared_bf16(const uint16_t* A, const uint16_t* B, uint1
     c_col_maj = 0;
   }
   const TileShares deal = gemm_plan(M, N, K, b_col_maj, c_col_maj).deal;
+  // (Products that tiles of 96 and 224 rows or long stages made cheaper than shared ones are taken all the same, by those: whoever brings a workspace of their own
+  // size for them need not ask first.)
+  if (deal.slices == 0 && gemm_plan(M, N, K, b_col_maj, c_col_maj, false).deal.slices > 0) return iron_gemm_bf16(A, B, C, M, N, K, b_col_maj, c_col_maj, nullptr, nullptr, stream);
   IRON_REQUIRE(deal.slices > 0, "gemm_shared: a product of %d x %d over %d shares no tiles (iron_gemm_workspace_bytes is 0)", M, N, K);
   hipStream_t s = (hipStream_t)stream;
   float* sums = (float*)workspace;

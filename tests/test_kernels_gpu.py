@@ -275,6 +275,20 @@ def test_gemm_that_shares_no_tiles_is_refused_a_workspace(cuda):
     assert K.lib().iron_gemm_shared_bf16(t.data_ptr(), t.data_ptr(), t.data_ptr(), 1024, 1024, 1024, 1, 0, t.data_ptr(), 0) == 1
 
 
+# Few rows by long stages, as (N,M) output too; 600 and more by tiles of 96.
+@pytest.mark.parametrize("M,N,Kdim,b_col_maj,c_col_maj", [(25, 364, 5632, 1, 0), (2199, 31, 8000, 1, 1), (8603, 615, 6464, 1, 0), (617, 8242, 4480, 1, 1)])
+def test_gemm_that_another_form_made_cheaper_than_shared_tiles_takes_a_workspace_all_the_same(cuda, M, N, Kdim, b_col_maj, c_col_maj):
+    """A caller with a workspace of its own size is not refused what shared its tiles before those forms came: it is made by them, and the workspace left alone."""
+    assert K.lib().iron_gemm_workspace_bytes(M, N, Kdim, b_col_maj, c_col_maj) == 0
+    rng = np.random.default_rng(M)
+    A, B, ws = dev(bf(rng, M, Kdim), cuda), dev(bf(rng, N, Kdim, scale=0.05), cuda), out_like((8,), cuda, fill=5.0)
+    C = out_like((N, M) if c_col_maj else (M, N), cuda, fill=float("nan"))
+    assert K.lib().iron_gemm_shared_bf16(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, Kdim, b_col_maj, c_col_maj, ws.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
+    want = torch.empty_like(C)
+    K.gemm(A, B, want, M=M, N=N, K=Kdim, b_col_maj=b_col_maj, c_col_maj=c_col_maj)
+    assert torch.equal(C, want) and bool((ws == 5).all())
+
+
 @pytest.mark.parametrize("b_col_maj", [True, False])
 @pytest.mark.parametrize("n", [4096, 8192])
 def test_gemm_large_squares_on_sampled_rows(cuda, n, b_col_maj):
