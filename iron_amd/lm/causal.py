@@ -276,7 +276,10 @@ class CausalLM(iron.Graph):
         """A loaded version's logits without what it carries, which a call would wait for."""
         if self.decode_step is None:
             raise RuntimeError(f"{type(self).__name__}: load_versions() first")
-        (row,) = self.decode_step.run(**values) if ids is None else self.prompt_chunk.run(ids, **values)
+        version, inputs = (self.decode_step, ()) if ids is None else (self.prompt_chunk, (ids,))
+        if not hasattr(version, "run"):   # (one stood in by what can be called)
+            return version(*inputs, **values)[0]
+        (row,) = version.run(*inputs, **values)
         return row
 
     @property

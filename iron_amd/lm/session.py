@@ -166,7 +166,8 @@ class Session:
         for others, at in chunks:
             model.run(*others, **at)
         replayed = bool(remaining) and step.captured and not each
-        started = replayed and model.prompt_chunk.hands_over(step)   # (the first step behind the prompt, while its token is on its way here)
+        hands_over = getattr(model.prompt_chunk, "hands_over", None)
+        started = replayed and hands_over is not None and hands_over(step)   # (the first step behind the prompt, while its token is on its way here)
         if started:
             carried = model.prompt_chunk.run_and_start(step, *inputs, **words)
         else:

@@ -162,6 +162,26 @@ def test_a_draw_that_nothing_came_between_runs_nothing_twice():
     assert model.session.cached.size == 25
 
 
+def test_versions_stood_in_by_what_is_called_started_and_replayed_alone():
+    """``use`` takes versions that hold no more than a session needs of them: they run, and none is asked to hand over."""
+    whole = loaded(Replayed, CONFIG)
+
+    class Called:
+        def __init__(self, version, **more):
+            self.version = version
+            vars(self).update(more)
+
+        def __call__(self, *tensors, **values):
+            return self.version(*tensors, **values)
+
+    model = Llama(CONFIG, weights(CONFIG))
+    step = whole.decode_step
+    model.use(Called(step, captured=True, start=step.start, replay=step.replay, write=step.write, read=lambda resident: step.read(whole.drawn)), Called(whole.prompt_chunk))
+    prompt, tokens, behind = alone(CONFIG, greedy, Replayed, False)
+    assert list(model.session.draw(prompt, 4)) == tokens
+    assert np.array_equal(model.logits([*prompt, *tokens]), behind)
+
+
 class Notes:
     """Streams, events and graphs that note, a stream each, what would be put on it."""
 
