@@ -21,6 +21,7 @@ The subset of the reference's graph layer the Llama decoder records
 
 from __future__ import annotations
 
+import contextlib
 import dataclasses
 import inspect
 import logging
@@ -1388,19 +1389,18 @@ class CompiledGraph:
             # Steps with a cheaper form within a limit are captured both ways; a call or a replay
             # takes the bounded graph while the values the host follows stay within every limit.
             for bounded in ((False, True) if self._bounds else (False,)):
-                self._context["bounded"] = bounded
-                self._derive()
-                self._run_steps()
-                stream.synchronize()
-                graph = torch.cuda.CUDAGraph()
-                with torch.cuda.graph(graph, stream=stream):
-                    # The host wrote every word, derived ones included, before the first replay; each
-                    # replay re-derives them for the next as it carries.
+                with self._in_form(bounded):
+                    self._derive()
                     self._run_steps()
-                    self._carry_on_device()
+                    stream.synchronize()
+                    graph = torch.cuda.CUDAGraph()
+                    with torch.cuda.graph(graph, stream=stream):
+                        # The host wrote every word, derived ones included, before the first replay; each
+                        # replay re-derives them for the next as it carries.
+                        self._run_steps()
+                        self._carry_on_device()
                 stream.synchronize()
                 graphs[bounded] = graph
-            self._context["bounded"] = False
         torch.cuda.current_stream().wait_stream(stream)
         self._graph, self._graph_bounded = graphs[False], graphs.get(True)
         self._host_values = None   # the warm-up's values start no run of replays
@@ -1427,6 +1427,15 @@ class CompiledGraph:
         if copied is None:
             copied = self._words_copied = torch.cuda.Event()
         copied.record()
+
+    @contextlib.contextmanager
+    def _in_form(self, bounded: bool):
+        """Launch steps that have a cheaper form within a limit in that form (``bounded``), and from then on in the other again, whatever is raised."""
+        self._context["bounded"] = bounded
+        try:
+            yield
+        finally:
+            self._context["bounded"] = False
 
     def _within_bounds(self, values: Mapping[str, int]) -> bool:
         """Whether every step with a bounded form stays within its limit at these per-call values."""
@@ -1608,12 +1617,12 @@ class CompiledGraph:
         if self._graph is not None:
             self._replay_at(full)
         else:
-            if self.check:
-                self._run_checked(full)
-            else:
-                self._context["bounded"] = bool(self._bounds) and self._within_bounds(full)
-                self._run_steps()
-                self._context["bounded"] = False
+            # (the form by the call's values, as for a captured version's replays: attention's bits do not depend on the capture)
+            with self._in_form(bool(self._bounds) and self._within_bounds(full)):
+                if self.check:
+                    self._run_checked(full)
+                else:
+                    self._run_steps()
         outs = []
         for h, t in zip(rec.outputs, self.output_tensors):
             rows = h.valid[0].evaluate(full) if 0 in h.valid else None

@@ -557,6 +557,21 @@ def test_a_turn_deep_in_the_cache_by_dealt_keys_and_by_whole_ones(deep, rows, be
         assert kl(want, runs[0]) <= 0.1
 
 
+def test_an_eager_version_takes_the_forms_that_a_captured_one_does(cuda):
+    """Short and long histories by chunks and by decode steps, with few keys and with many behind them: the same bits eager and captured."""
+    config = dataclasses.replace(SCALED, num_hidden_layers=1, max_seq_len=8192, prefill_chunk=1024)
+    w = weights(config)
+    tokens = np.random.default_rng(36).integers(0, config.vocab_size, 4300)
+    rows = []
+    for capture in (True, False):
+        model = Llama(config, w)
+        model.load_versions(capture=capture)
+        rows.append([model.logits(tokens[:n]) for n in (700, 701, 1500, 2040, 2041, 2700, 2701, 4296, 4297)])
+        model.release()
+    for captured, eager in zip(*rows):
+        assert np.array_equal(captured, eager)
+
+
 def test_a_5000_token_prompt_in_three_chunks_then_replayed_steps(cuda):
     """Toy width, caches of 8192 rows: a prompt of three chunks (attention over a cache longer than
     the chunk), then eight device-carried decode steps past position 5000 (attention's keys dealt

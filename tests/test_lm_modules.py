@@ -8,6 +8,7 @@ import pytest
 
 import oracle
 from iron_amd.applications.llama import Llama
+from iron_amd.common import graph
 from iron_amd.lm.blocks import Attention, KVCache, Rope
 from iron_amd.lm.causal import OnHost
 from tests.llama_support import SCALED, weights
@@ -249,3 +250,27 @@ def test_partial_rotary_narrows_the_table_and_turns_the_leading_columns_in_one_s
     assert np.array_equal(got[:, :32], ops.rope(x[:, :32], table)) and np.array_equal(got[:, 32:], x[:, 32:])
     with pytest.raises(ValueError, match="rotary_dim"):
         dataclasses.replace(cfg, rotary_dim=40)
+
+
+@pytest.mark.parametrize("check", [False, True])
+def test_a_launch_that_raises_leaves_the_next_one_its_own_form(monkeypatch, check):
+    """An eager version whose steps have a form within a limit launches them in the one that a call's values choose, checked or not, and
+    is in the general one behind a call whatever that raised."""
+    model = small(num_hidden_layers=1, prefill_chunk=16, max_seq_len=48)
+    version = model.compile(capture=False, check=check)
+    monkeypatch.setattr(type(version), "load", lambda self: self)
+    monkeypatch.setattr(type(version), "_write_words", lambda self, full: None)
+    version._bounds, version._fused, version.input_tensors, version.output_tensors, version._staging = [((graph.Affine("position"),), 7)], {}, [], [], {}
+    asked = []
+
+    def launch(tensors, words):
+        asked.append(version._context["bounded"])
+        raise RuntimeError("refused")
+
+    version._launches = [(launch, {n: None for n in (*s.inputs, *s.outputs)}, {}) for s in version.recording.steps]
+    monkeypatch.setattr(graph, "from_torch", lambda tensor: np.zeros(1))
+    for position in (7, 8):
+        with pytest.raises(RuntimeError, match="refused"):
+            version.run(token=1, position=position)
+        assert version._context["bounded"] is False
+    assert asked == [True, False]
