@@ -33,7 +33,7 @@ constexpr int BQ = 128;   // query rows per block (four waves of 32; 64 where a 
 constexpr int BKV = 64;   // key rows per tile
 constexpr float kLazyBits = 8.f;        // how far a maximum may run ahead of the reference the exponents are taken against
 constexpr float kSumLow = 0x1p-60f, kSumHigh = 0x1p24f;   // a tile's sum of exponentials outside this range: take its maximum and redo it
-// 128-wide heads of up to 1024 blocks by four waves: how many of a block's first tiles have their weights in two terms of bf16.  A weight rounds to bf16 against its
+// 128-wide heads of up to 1024 blocks by four waves (calls without bounds): how many of a block's first tiles have their weights in two terms of bf16.  A weight rounds to bf16 against its
 // reference, and only the largest, exactly 1 against a reference that is its maximum, comes through whole; eight waves a block have a reference for each half
 // of the tiles and so two such weights.  Two terms in the first two tiles, all that the first 128 queries have, are nearer than that
 // (relative error against 64 bits, 32 heads, 3001 queries: eight waves 0.00209, four with one term 0.00212, so 0.00188, of which 0.00166 are the output's own rounding; window of
@@ -1188,14 +1188,14 @@ static int launch_prefill_as(const PrefillArgs& a, int blocks, void* stream, flo
 }
 
 // Bounds read on the device may leave few queries; else the sizes say whether there are.
-template <int D, int SPLIT, int W = 4, bool FINE = false>
+template <int D, int SPLIT, int W = 4>
 static int launch_prefill(const PrefillArgs& a, int blocks, void* stream) {
   const bool bounded = a.valid != nullptr || a.kv_valid != nullptr || a.seq_len != a.seq;
   // (a launch so short that all its queries may go 32 to a block has a block for each 32)
   const int groups = ((a.seq + 31) / 32) * a.heads;
   const bool few = few_rows_pay<D, W>(groups, a.kv_len);
-  if (a.kv_len < 512 || (!bounded && !few)) return launch_prefill_as<D, SPLIT, W, false, FINE>(a, blocks, stream);
-  return launch_prefill_as<D, SPLIT, W, true, FINE>(a, few && groups > blocks ? groups : blocks, stream);
+  if (a.kv_len < 512 || (!bounded && !few)) return launch_prefill_as<D, SPLIT, W, false, false>(a, blocks, stream);
+  return launch_prefill_as<D, SPLIT, W, true, false>(a, few && groups > blocks ? groups : blocks, stream);
 }
 
 // Whether a launch of 128-wide heads takes blocks of 64 queries (one a CU) and not of 128.  One round of them does: it is the shorter
@@ -1217,7 +1217,8 @@ static bool half_blocks_128(const PrefillArgs& a) {
 // without a mask 123 / 132, behind 4000 keys 236 / 249).  Queries over their own keys: four where there are heads enough for the blocks that go out last to fill in behind the longest (32
 // heads 2500 queries 72.5 / 70.4, 3012 94.0 / 86.7, 24 heads 3780 106 / 103, 16 heads 6340 177 / 171, 64 heads 1092 41.5 / 35.2; short of the line 24 heads 3268 85.7 / 86.4,
 // 16 heads 5572 142 / 144, 8 heads 9200 185 / 211), and behind short windows (2116 queries, windows of 301 and 1024 34.7 / 30.2 and 47.4 / 42.7; 3012 queries 44.1 / 42.1 and
-// 70.9 / 68.9; window of 1401, 24 heads 3268 queries 65.0 / 62.6, 4164 86.8 / 89.7).  Bounds on the device may leave fewer: eight waves up to 1024 blocks.
+// 70.9 / 68.9; window of 1401, 24 heads 3268 queries 65.0 / 62.6, 4164 86.8 / 89.7).  Bounds on the device may leave fewer: eight waves up to 1024
+// blocks, so a decoder's prompt, whose launches all have bounds, takes none of this.
 static bool split_128(const PrefillArgs& a, int blocks) {
   if (a.valid != nullptr || a.kv_valid != nullptr || a.seq_len != a.seq) return blocks <= 4 * kCUs;
   if (blocks <= 2 * kCUs) return true;
@@ -1311,7 +1312,8 @@ static int mha_prefill(const uint16_t* Q, const uint16_t* K, const uint16_t* V, 
   else if (half_blocks_128(a) && !(kv_len >= 1536 && few_rows_pay<128, 4>(((seq + 31) / 32) * heads, kv_len)))
     rc = launch_prefill<128, 2, 2>(a, ((seq + 63) / 64) * heads, stream);
   else if (split_128(a, blocks)) rc = launch_prefill<128, 2>(a, blocks, stream);
-  else if (blocks <= 4 * kCUs) rc = launch_prefill<128, 1, 4, true>(a, blocks, stream);   // (those that eight waves would be as near for)
+  // (those that eight waves would be as near for; without bounds, so no queries are few, see split_128)
+  else if (blocks <= 4 * kCUs) rc = launch_prefill_as<128, 1, 4, false, true>(a, blocks, stream);
   else rc = launch_prefill<128, 1>(a, blocks, stream);
   if (rc != 0) return rc;
   IRON_LAUNCH_CHECK();
