@@ -44,8 +44,8 @@ int iron_gemm_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int
 int64_t iron_gemm_workspace_bytes(int M, int N, int K, int b_col_maj, int c_col_maj);
 int iron_gemm_shared_bf16(const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K, int b_col_maj,
                           int c_col_maj, void* workspace, void* stream);
-/* The tile a product is made of, rows << 16 | columns of what a block computes (0: the few-row and the general kernels), as the launches decide
- * it on the host; for tests.  kind 0: M rows, no bound, no workspace; 1: under a bound of `rows` (B (N,K)); 2: iron_gemm_residual_bf16 and
+/* The tile a product is made of, rows << 16 | columns of what a block computes (0: the few-row and the general kernels; 1 << 15 more: up to 32
+ * rows by long stages of K), as the launches decide it, for tests.  kind 0: M rows, no bound, no workspace; 1: under a bound of `rows` (B (N,K)); 2: iron_gemm_residual_bf16 and
  * iron_gemm_gated_bf16 under it (0: without one); 3: iron_gemm_gated_pair_bf16 under it, columns of each product. */
 int iron_gemm_tile(int kind, int M, int N, int K, int b_col_maj, int c_col_maj, int rows);
 

@@ -2180,6 +2180,14 @@ static FormTable form_table(int M, bool bounded, Best best, int* upto) {
   return t;
 }
 
+// Whether a launch of `blocks` blocks that has chosen its tiles of 32 x 32 (64 x (32 + 32) of a gated pair) makes up to 32 rows by long stages instead.  The blocks
+// are as many as the chosen tiles need, at most for all rows of the bound's buffer, so a buffer of few rows may have too few for a tile of eight columns a block
+// (64 rows of 2048 columns over 2048 are 128 tiles of 32 x 32): those keep the tiles.
+__device__ __host__ inline bool rows_by_long_stages(int rows, int N, int K, int blocks) {
+  return rows <= 32 && K % LONG_K == 0 && N % 8 == 0 && N / 8 <= (blocks < 256 ? blocks : 256);
+}
+__device__ __host__ inline bool pair_by_long_stages(int rows, int N, int K) { return rows <= 32 && K % LONG_K == 0 && N % 32 == 0; }
+
 // A product under a row bound that is read on the device: the blocks of ONE launch take the form that is the cheapest at the bound (512 valid rows of
 // 2048 leave 64 of 256 large tiles).  Each form's grid covers only the rows it can be chosen for; the launch's grid is the largest of
 // them and a block past its tiling's tiles leaves at once.  LDS is the largest tiling's, so a CU
@@ -2270,7 +2278,7 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const bf16_t* __restrict
       gemm_nt64_body<13, false, 1, 4>(A, B, C, M, N, K, Mv, (M + 63) / 64, (N + 31) / 32, patched, tail);
       break;
     default: {
-      if (Mv <= 32 && K % LONG_K == 0 && N % 8 == 0 && N / 8 <= min(256, (int)gridDim.x)) gemm_long_body<LONG_PLAIN, 32, 7>(A, B, C, N, K, Mv, tail);
+      if (rows_by_long_stages(Mv, N, K, (int)gridDim.x)) gemm_long_body<LONG_PLAIN, 32, 7>(A, B, C, N, K, Mv, tail);
       else gemm_nt64_body<20, false, 1, 2, 1>(A, B, C, M, N, K, Mv, (M + 31) / 32, (N + 31) / 32, patched, tail);
     }
   }
@@ -2781,7 +2789,7 @@ __global__ __launch_bounds__(256) void gemm_gated_pair_kernel(const bf16_t* __re
     default: {
       QkvTail gate{};
       gate.gated = activation;
-      if (Mv <= 32 && K % LONG_K == 0 && N % 32 == 0) gemm_long_body<LONG_PAIR, 32, 3>(A, Bg, C, N, K, Mv, gate, Bu, G);
+      if (pair_by_long_stages(Mv, N, K)) gemm_long_body<LONG_PAIR, 32, 3>(A, Bg, C, N, K, Mv, gate, Bu, G);
       else gemm_nt64_body<8, true>(A, Bg, C, M, N, K, Mv, (M + 63) / 64, (N + 31) / 32, patched, gate, Bu, G);
     }
   }
@@ -2963,11 +2971,14 @@ static int launch_gemm_long(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, 
   hipLaunchKernelGGL((gemm_long_kernel<B_ROWS, STAGES>), dim3((N + B_ROWS - 1) / B_ROWS), dim3(256), lds, s, A, B, C, M, N, K);
   IRON_LAUNCH_CHECK();
 }
+static int long_columns(int N) { return N <= 8 * 256 ? 8 : (N <= 16 * 256 ? 16 : (N <= 32 * 256 ? 32 : 64)); }
 static int launch_gemm_long(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, int K, hipStream_t s) {
-  if (N <= 8 * 256) return launch_gemm_long<8, 8>(A, B, C, M, N, K, s);
-  if (N <= 16 * 256) return launch_gemm_long<16, 6>(A, B, C, M, N, K, s);
-  if (N <= 32 * 256) return launch_gemm_long<32, 5>(A, B, C, M, N, K, s);
-  return launch_gemm_long<64, 3>(A, B, C, M, N, K, s);
+  switch (long_columns(N)) {
+    case 8: return launch_gemm_long<8, 8>(A, B, C, M, N, K, s);
+    case 16: return launch_gemm_long<16, 6>(A, B, C, M, N, K, s);
+    case 32: return launch_gemm_long<32, 5>(A, B, C, M, N, K, s);
+    default: return launch_gemm_long<64, 3>(A, B, C, M, N, K, s);
+  }
 }
 
 // Whole tiles larger than 128 x 128, by how the rounds they make over the chip's 256 CUs come out: a round of a tile was measured
@@ -3262,15 +3273,19 @@ extern "C" int iron_gemm_shared_bf16(const uint16_t* A, const uint16_t* B, uint1
 extern "C" int iron_gemm_tile(int kind, int M, int N, int K, int b_col_maj, int c_col_maj, int rows) {
   if (kind < 0 || kind > 3 || M <= 0 || N <= 0 || K <= 0 || K % 8 != 0 || K > (1 << 22) || N > (1 << 22)) return 0;
   auto tile = [](int bm, int bn) { return bm << 16 | bn; };
+  auto by_long_stages = [=](int columns) { return tile(32, 1 << 15 | columns); };
   if (kind > 0) {
     if (kind < 3 && two_a_cu(M, N, K, rows > 0)) return tile(64, 64);
     const FormPlan plan = kind == 3 ? pair_plan(M, N, K, true) : rows_plan(M, N, K, true, kind == 2);
-    const int form = form_of_rows(plan.table, rows > 0 && rows < M ? rows : M);
+    const int live = rows > 0 && rows < M ? rows : M, form = form_of_rows(plan.table, live);
+    if (kind == 3 && form == PAIR_64X32 && pair_by_long_stages(live, N, K)) return by_long_stages(long_b_rows(LONG_PAIR) / 2);
+    if (kind < 3 && form == ROWS_32X32 && rows_by_long_stages(live, N, K, plan.blocks)) return by_long_stages(long_b_rows(LONG_PLAIN));
     return kind == 3 ? tile(PAIR_PRICES[form].bm, PAIR_PRICES[form].bn) : tile(ROWS_PRICES[form].bm, ROWS_PRICES[form].bn);
   }
   const bool turned = b_col_maj && c_col_maj;
   const GemmPlan plan = gemm_plan(turned ? N : M, turned ? M : N, K, b_col_maj, c_col_maj && !turned);
   switch (plan.form) {
+    case GemmForm::LONG_STAGES: return by_long_stages(long_columns(turned ? M : N));
     case GemmForm::SMALL: return tile(plan.small.rows, b_col_maj ? 32 : 64);
     case GemmForm::BIG: return tile(BIG_PRICES[plan.big].bm, BIG_PRICES[plan.big].bn);
     case GemmForm::TILES_64: return tile(64, 64);

@@ -136,6 +136,18 @@ def test_large_products_without_a_bound_reach_every_size_of_tile():
         assert tile(0, M, N, K, 0, 0, 0) != 128 << 16 | 128, (M, N, K)
 
 
+def test_few_rows_go_by_long_stages_where_a_launch_has_the_blocks():
+    """Up to 32 rows over whole 256 of K, eight columns a block (32 of each of a pair): as many blocks as the buffer's most rows have tiles, so a buffer of few rows
+    has too few for many columns; not a K of other lengths, nor more rows, nor more columns than CUs have room for."""
+    tile = _lib.lib().iron_gemm_tile
+    for kind, M, N, K, rows, long in ((1, 600, 2048, 2048, 32, 8), (1, 600, 2048, 2048, 33, 0), (1, 64, 2048, 2048, 32, 0), (1, 64, 1024, 2048, 32, 0), (1, 128, 2048, 2048, 32, 8),
+                                      (2, 600, 2048, 8192, 1, 8), (2, 600, 2056, 8192, 1, 0), (1, 600, 2048, 2112, 32, 0), (1, 600, 2044, 2048, 32, 0),
+                                      (3, 64, 8192, 2048, 32, 32), (3, 600, 8192, 2048, 32, 32), (3, 600, 8192, 2048, 33, 0), (3, 600, 8200, 2048, 32, 0), (3, 600, 8192, 2112, 9, 0),
+                                      (0, 17, 4096, 2048, 0, 16), (0, 16, 4096, 2048, 0, 0), (0, 33, 4096, 2048, 0, 0)):
+        got = tile(kind, M, N, K, 1, 0, rows)
+        assert (got & 32767 if got >> 15 & 1 else 0) == long, (kind, M, N, K, rows, hex(got))
+
+
 def test_what_a_bound_chooses_is_decided_once_for_the_same_sizes():
     """A launch under a row bound prices every form for every run of rows: the same sizes again cost no more than a launch without a bound,
     and more sizes than are held, or another thread, change no answer."""

@@ -639,9 +639,9 @@ def test_a_row_s_products_are_the_same_bits_under_every_bound(cuda, M, Kdim, N, 
             assert (got[rows:] == 7).all(), rows
 
 
-# One row of tiles, whose stages are 256 columns of K: one stage, fewer than the ring holds, more; one tile of eight columns, some, one a CU (and a tile more, which
-# the others take); rows on either side of sixteen and of the tile's.
-@pytest.mark.parametrize("Kdim", [256, 768, 2304])
+# One row of tiles, whose stages are 256 columns of K: one stage (a pair's; of the others two, shorter ones go by tiles of 64 x 64), fewer than the ring holds, more; one
+# tile of eight columns, some, one a CU (and a tile more, which the others take); rows on either side of sixteen and of the tile's.
+@pytest.mark.parametrize("Kdim", [256, 512, 768, 2304])
 @pytest.mark.parametrize("N", [8, 200, 2048, 2056])
 @pytest.mark.parametrize("form", ["plain", "residual", "gated", "pair"])
 def test_few_rows_over_long_stages_are_the_same_bits_as_among_many(cuda, Kdim, N, form):
@@ -650,6 +650,10 @@ def test_few_rows_over_long_stages_are_the_same_bits_as_among_many(cuda, Kdim, N
     N = N if form == "plain" else max(64, 32 * -(-N // 32) if form == "pair" else N)   # (the fewest columns that a second operand is taken with)
     A, B, B2, R = (bf(rng, *s, scale=x) for s, x in (((M, Kdim), 1.0), ((N, Kdim), 0.05), ((N, Kdim), 0.05), ((M, N), 1.0)))
     dB, dB2, dR, kw = dev(B, cuda), dev(B2, cuda), dev(R, cuda), dict(M=M, N=N, K=Kdim)
+    by_long_stages = form == "pair" or (Kdim >= 512 and N <= 2048)
+    for rows in (1, 32, 33, M):   # (1 << 15: by long stages)
+        code = K.lib().iron_gemm_tile({"plain": 1, "residual": 2, "gated": 2, "pair": 3}[form], M, N, Kdim, 1, 0, rows)
+        assert code >> 15 & 1 == (by_long_stages and rows <= 32) and (rows > 32 or not by_long_stages or code & 32767 == (32 if form == "pair" else 8))
 
     def run(rows):
         C, G = out_like((M, N), cuda, fill=7.0), out_like((M, N), cuda, fill=7.0)
@@ -681,6 +685,8 @@ def test_few_rows_over_long_stages_are_the_same_bits_as_among_many(cuda, Kdim, N
 @pytest.mark.parametrize("turned", [False, True])
 def test_few_rows_over_long_stages_without_a_bound(cuda, M, Kdim, N, turned):
     """Against the oracle; turned: the (N,M) output of B and A, the same product."""
+    code = K.lib().iron_gemm_tile(0, *((N, M) if turned else (M, N)), Kdim, 1, turned, 0)
+    assert code == 32 << 16 | 1 << 15 | (8 if N <= 2048 else 16 if N <= 4096 else 32 if N <= 8192 else 64)
     rng = np.random.default_rng(M + N)
     A, B = bf(rng, M, Kdim), bf(rng, N, Kdim, scale=0.05)
     C = out_like((M + 1, N), cuda, fill=7.0)
