@@ -2358,12 +2358,13 @@ static int launch_gemm_rows(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, 
 // down projection: 512 live rows x 2048 columns over K = 8192, then the next layer's input norm).
 // 128 x 128 tiles would occupy a quarter of the CUs and the 64 x 64 ones that fill the chip fetch
 // every operand row twice as often, so a tile's K is dealt over `splits` blocks -- chosen on the
-// device by the row bound and K: 16, 8 and 4 while the live tiles fill that part of the chip, 2 up to half, else
-// whole K -- each leaving its float32 sums in a workspace slice.  A second launch, a block a row,
+// device by the row bound and K: 16 or 8 where that many a tile fit the chip in slices of eight stages or more, 4 where those would be too
+// short, else as many as the chip has CUs for, 7 to 2, in slices that differ by a stage; past half the chip whole K, by tiles of 96 rows while
+// those are one round -- each leaving its float32 sums in a workspace slice.  A second launch, a block a row,
 // adds a row's slices in slice order (the same sums whatever ran first), rounds once, adds the
 // residual, stores the row and norms it as rmsnorm_kernel does: that launch stands where the
 // norm's own stood, so the slices' sum costs no launch of its own.
-constexpr int kSplitKMax = 4;    // slices the second launch asks for at a time, and every K can be cut into
+constexpr int kSplitKMax = 4;    // slices the second launch asks for at a time; K is whole stages of as many
 __device__ __host__ inline int splitk_for(int tile_rows, int tiles_n, int K) {
   const int live_tiles = tile_rows * tiles_n;
   // Past four slices while the chip would idle and a slice keeps eight stages; ten where the slices of several tile rows pass half
@@ -3322,7 +3323,7 @@ extern "C" int iron_gemm_residual_bf16(const uint16_t* A, const uint16_t* B, con
 extern "C" int64_t iron_gemm_residual_norm_workspace_bytes(int M, int N, int K) {
   if (M < 128 || N < 128 || N % 128 != 0 || N > 8192 || K < 4096 || K % (BK * kSplitKMax) != 0) return 0;
   const int tiles_n = N / 128;
-  // splits x the rows a split count runs for is the same for every split count: 256 tiles' worth of rows.
+  // 256 tiles' worth of rows are room for every split count: splits * ((256 / splits) / tiles_n) <= 256 / tiles_n.
   return (int64_t)(256 / tiles_n) * 128 * N * (int64_t)sizeof(float);
 }
 
