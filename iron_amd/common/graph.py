@@ -1035,7 +1035,7 @@ class ScratchArena:
         self.uploaded: set[int] = set()
         self.generation = 0
         self.launched = 0   # calls, starts and runs of replays of any version so far
-        self.running = None   # the end of what a call left running behind its return
+        self.stream = None   # the last one that the arena was used on
 
     def place_resident(self, r: Resident) -> int:
         if id(r) not in self.resident_offsets:
@@ -1079,34 +1079,26 @@ class ScratchArena:
         n = math.prod(shape) * itemsize(dtype)
         return self.buffer[offset : offset + n].view(tdtype).view(tuple(shape) or (1,))
 
-    def leave_running(self) -> None:
-        """A call returns with work on the arena still queued on this stream: whoever touches the arena next, on whatever stream, is behind it
-        (``enter``), and so is whoever is given the memory next."""
-        import torch
-
-        self.running = torch.cuda.Event()
-        self.running.record()
-        self.buffer.record_stream(torch.cuda.current_stream())
-
     def enter(self) -> None:
-        if self.running is None:
-            return
+        """The arena's next use is on the current stream: behind the last one on whatever stream that was, which may still run (a draw hands out a token with the
+        next step under way), and the memory is not given to others before it is over.  On the stream of the last one that costs nothing but the question."""
         import torch
 
-        if self.running.query():
-            self.running = None
-        else:
-            torch.cuda.current_stream().wait_event(self.running)
+        stream = torch.cuda.current_stream()
+        if stream != self.stream and not torch.cuda.is_current_stream_capturing():   # (a caller's own capture begins on an idle device)
+            if self.stream is not None:
+                stream.wait_stream(self.stream)
+            self.buffer.record_stream(stream)
+            self.stream = stream
 
     def settle(self) -> None:
-        """Wait on the host for what was left running."""
-        if self.running is not None:
-            self.running.synchronize()
-            self.running = None
+        """Wait on the host for the last use."""
+        if self.stream is not None:
+            self.stream.synchronize()
 
     def release(self) -> None:
         self.settle()
-        self.buffer = None
+        self.buffer = self.stream = None
         self.uploaded.clear()
 
 
@@ -1546,7 +1538,6 @@ class CompiledGraph:
         for k, (tensor, _) in made.items():
             kernels.copy_rows(tensor.view(1), to.words[to.slots[k] : to.slots[k] + 1], rows=1, row_elems=1, src_rows=1, dst_rows=1)
         to._replay_at(start)
-        self.arena.leave_running()
         arrived.synchronize()
         for k, (_, host) in made.items():
             known[k] = to._host_values[k] = int(host[0])

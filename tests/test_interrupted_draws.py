@@ -188,26 +188,33 @@ class Notes:
     def __init__(self, monkeypatch):
         import torch
 
-        self.on = {"own": [], "other": []}
+        self.on = {"own": [], "other": [], "host": []}
         self.stream = "own"
         notes = self
 
         class Event:
             def record(self):
-                self.at = (notes.stream, len(notes.on[notes.stream]))
-
-            def query(self):
-                return False
+                pass
 
             def synchronize(self):
-                notes.on["host"] = notes.on.get("host", []) + [self.at]
+                pass
 
         class Stream:
-            def wait_event(self, event):
-                notes.on[notes.stream].append(("behind", event.at))
+            def __init__(self):
+                self.name = notes.stream
+
+            def __eq__(self, other):
+                return other is not None and self.name == other.name
+
+            def wait_stream(self, other):
+                notes.on[self.name].append(("behind", other.name))
+
+            def synchronize(self):
+                notes.on["host"].append(("behind", self.name))
 
         monkeypatch.setattr(torch.cuda, "Event", Event)
-        monkeypatch.setattr(torch.cuda, "current_stream", lambda: Stream())
+        monkeypatch.setattr(torch.cuda, "current_stream", Stream)
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
         monkeypatch.setattr(torch.Tensor, "record_stream", lambda tensor, stream: notes.put("held"))
 
     def put(self, what):
@@ -238,7 +245,7 @@ def test_the_step_that_a_draw_leaves_running_is_ahead_of_whatever_comes_next(mon
     model.use(decode, prompt)
     notes = Notes(monkeypatch)
     arena = model.arena
-    arena.buffer = torch.zeros(arena.nbytes, dtype=torch.uint8)
+    arena.load("cpu")
     monkeypatch.setattr(CompiledGraph, "load", lambda self: self)
     monkeypatch.setattr(kernels, "copy_rows", lambda *a, **k: notes.put("token"))
     pinned_empty = torch.empty
@@ -253,13 +260,14 @@ def test_the_step_that_a_draw_leaves_running_is_ahead_of_whatever_comes_next(mon
     assert prompt.hands_over(decode)
     *_, (inputs, words) = model.session.chunk_calls([1, 2, 3])
     prompt.run_and_start(decode, *inputs, **words)
-    own = notes.on["own"]
-    assert own[:3] == ["graph", "token", "graph"] and "held" in own   # the portion, its token's way into the words, the step; the memory is this stream's too
-    end = ("own", 3)
+    assert notes.on["own"] == ["held", "graph", "token", "graph"]   # the memory is this stream's too; the portion, its token's way into the words, the step
     notes.stream = "other"
     if use == "a release":
         model.release()
-        assert notes.on["host"][-1] == end and decode._graph is None
+        assert notes.on["host"][-1] == ("behind", "own") and decode._graph is None
         return
     USES[use](model, prompt)
-    assert notes.on["other"][0] == ("behind", end)
+    assert notes.on["other"][:2] == [("behind", "own"), "held"] and notes.on["other"].count(("behind", "own")) == 1
+    notes.stream = "own"
+    USES[use](model, prompt)
+    assert ("behind", "other") in notes.on["own"]
