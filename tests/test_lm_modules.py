@@ -260,6 +260,7 @@ def test_a_launch_that_raises_leaves_the_next_one_its_own_form(monkeypatch, chec
     version = model.compile(capture=False, check=check)
     monkeypatch.setattr(type(version), "load", lambda self: self)
     monkeypatch.setattr(type(version), "_write_words", lambda self, full: None)
+    monkeypatch.setattr(type(version.arena), "enter", lambda self: None)
     version._bounds, version._fused, version.input_tensors, version.output_tensors, version._staging = [((graph.Affine("position"),), 7)], {}, [], [], {}
     asked = []
 
