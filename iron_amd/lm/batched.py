@@ -69,6 +69,8 @@ class Batch:
         self.held: dict[Hashable, int] = {}     # tokens of each request that have been run
         self._free = list(range(lm.config.slots))
         self._rows: np.ndarray | None = None    # the draw rows as the device has them
+        self._runs = 0                          # launches that ran some request's tokens so far
+        self._ran: dict[Hashable, int] = {}     # the last of them for each request
 
     # ------------------------------------------------------------------ slots
     def _claim(self) -> None:
@@ -76,6 +78,7 @@ class Batch:
             self.lm.holder = self
             self.slots.clear()
             self.held.clear()
+            self._ran.clear()
             self._free = list(range(self.lm.config.slots))
             self._rows = None
 
@@ -90,7 +93,20 @@ class Batch:
         slot = self.slots.pop(key, None)
         if slot is not None:
             self.held.pop(key)
+            self._ran.pop(key, None)
             self._free.append(slot)
+
+    def _count(self, keys, tokens) -> None:
+        """A launch has run ``tokens`` of each of the requests."""
+        self._runs += 1
+        for key, n in zip(keys, tokens):
+            self.held[key] += n
+            self._ran[key] = self._runs
+
+    def last_run(self, key: Hashable) -> int | None:
+        """The last launch that ran tokens of the request: who finds another than it left, or none, has been interrupted."""
+        self._claim()
+        return self._ran.get(key)
 
     def _admit(self, entries: Sequence[Entry], more: int = 0) -> list[np.ndarray]:
         model = self.lm
@@ -145,8 +161,7 @@ class Batch:
         self._spans(spans)
         model.decode_step.write(model.token, tokens)
         logits = model()
-        for e in entries:
-            self.held[e.key] += 1
+        self._count([e.key for e in entries], [1] * len(entries))
         if not any(len(e.want) for e in entries):
             return [np.empty((0, c.vocab_size), np.float32) for _ in entries]
         rows = logits.numpy()
@@ -160,7 +175,7 @@ class Batch:
         room = c.key_room
         out = [np.empty((len(e.want), c.vocab_size), np.float32) for e in entries]
         while True:
-            row, keys, spans, portion, asked = 0, 0, np.zeros((c.slots, 4), np.int32), np.zeros(c.prefill_chunk, np.int32), []
+            row, keys, spans, portion, asked, run = 0, 0, np.zeros((c.slots, 4), np.int32), np.zeros(c.prefill_chunk, np.int32), [], {}
             for i, (e, t) in enumerate(zip(entries, ids)):
                 n = min(t.size - done[i], c.prefill_chunk - row)
                 if n > 0 and room is not None:   # (a request alone always fits: it has no more keys than positions)
@@ -172,12 +187,13 @@ class Batch:
                 portion[row : row + n] = t[done[i] : done[i] + n]
                 asked += [(i, k, row + w - done[i]) for k, w in enumerate(e.want) if done[i] <= w < done[i] + n]
                 done[i] += n
-                self.held[e.key] += n
+                run[e.key] = n
                 row += n
             if row == 0:
                 return out
             self._spans(spans)
             tails = model(portion, rows=row)
+            self._count(run, run.values())
             at_tail = {int(s[0] + s[1] - 1): slot for slot, s in enumerate(spans) if s[1]}
             if all(r in at_tail for _, _, r in asked):
                 got = tails.numpy() if asked else None
@@ -204,6 +220,19 @@ class Batch:
         if sampler is not None:
             self._rows[slot, start : start + count] = sampler.rows(count, model.k_max)
         model.decode_step.write(model.draws, self._rows)
+
+    def _draw_rows(self, key: Hashable) -> np.ndarray | None:
+        """A copy of the request's draw rows; none where no sampler has been here."""
+        return None if self._rows is None else self._rows[self.slots[key]].copy()
+
+    def _put_draw_rows(self, key: Hashable, rows: np.ndarray | None) -> None:
+        c, slot = self.lm.config, self.slots[key]
+        if rows is None and self._rows is None:
+            return
+        if self._rows is None:
+            self._rows = np.zeros((c.slots, c.max_seq_len, ROW_WORDS), np.int32)
+        self._rows[slot] = 0 if rows is None else rows
+        self.lm.decode_step.write(self.lm.draws, self._rows)
 
     def _prefill(self, entries: Sequence[Entry], count: int, samplers) -> None:
         """Run the requests' prompts, packed into as few portions as they fill."""
@@ -232,24 +261,28 @@ class Batch:
         else:
             for _ in range(steps):
                 model()
-        for key in last:
-            self.held[key] += steps
+        self._count(last, [steps] * len(last))
+
+    def _go_on(self, key: Hashable, token: int, steps: int) -> list[int]:
+        """What ``steps`` decode steps of the request draw, from its last drawn token."""
+        at = self.held[key]
+        self._run({key: token}, steps)
+        return self._drawn()[self.slots[key], at : at + steps].tolist()
 
     def draw(self, key: Hashable, tokens, max_tokens: int, sampler=None, each: bool = False) -> Iterator[int]:
         """Yield ``max_tokens`` tokens drawn on the device after ``tokens`` of one request."""
         self._prefill([Entry(key, tokens)], max_tokens, [sampler])
-        slot = self.slots[key]
-        token = int(self._drawn()[slot, self.held[key] - 1])
+        token = self._first_drawn(key)
         yield token
         left = max_tokens - 1
         while left:
             n = 1 if each else left
-            at = self.held[key]
-            self._run({key: token}, n)
-            for token in self._drawn()[slot, at : at + n]:
-                token = int(token)
+            for token in self._go_on(key, token, n):
                 yield token
             left -= n
+
+    def _first_drawn(self, key: Hashable) -> int:
+        return int(self._drawn()[self.slots[key], self.held[key] - 1])
 
     def generate(self, prompts: Sequence[Sequence[int]], max_tokens: int, samplers=None, round_steps: int = 32) -> list[list[int]]:
         """Up to ``max_tokens`` tokens after each of the prompts, as many of them in flight as there are
@@ -340,13 +373,33 @@ class SlotSession(Session):
         self._fits(ids.size, max_tokens - 1)
         if model.decode_step is None:
             raise RuntimeError(f"{type(model).__name__}: load_versions() first")
-        rest = self._start(ids)
+        batch, rest = model.batch, self._start(ids)
         self.cached = self.cached[:0]
-        out: list[int] = []
-        for token in model.batch.draw(self, rest, max_tokens, sampler, each):
-            out.append(token)
-            yield token
-        self.cached = np.concatenate([ids, np.asarray(out[:-1], dtype=np.int64)])
+        batch._prefill([Entry(self, rest)], max_tokens, [sampler])
+        rows, out = batch._draw_rows(self), [batch._first_drawn(self)]
+        ran = batch.last_run(self)
+        yield out[0]
+        while len(out) < max_tokens:
+            if batch.last_run(self) != ran:   # (this conversation itself, between two tokens, or the model loaded anew)
+                self._run_again(ids, out[:-1], rows)
+            drawn = batch._go_on(self, out[-1], 1 if each else max_tokens - len(out))
+            ran = batch.last_run(self)
+            for token in drawn:
+                out.append(token)
+                yield token
+        if batch.last_run(self) == ran:
+            self.cached = np.concatenate([ids, np.asarray(out[:-1], dtype=np.int64)])
+
+    def _run_again(self, prompt: np.ndarray, drawn: Sequence[int], rows: np.ndarray | None) -> None:
+        """The request as a draw had it behind ``prompt`` and the ``drawn`` tokens, from its start."""
+        batch = self.lm.batch
+        batch.end(self)
+        self.cached = self.cached[:0]
+        entries = [Entry(self, prompt)]
+        batch._portions(entries, batch._admit(entries, more=len(drawn)), whole=True)
+        for token in drawn:
+            batch.step([Entry(self, [token])])
+        batch._put_draw_rows(self, rows)
 
 
 class StreamDecoder(Decoder):

@@ -11,10 +11,13 @@ import pytest
 
 import oracle
 from iron_amd.applications.llama import Llama
+from iron_amd.applications.tilarax import Tilarax
 from iron_amd.lm import Sampler
+from iron_amd.lm.batched import BatchedOnHost, _HostBatchVersion
 from iron_amd.lm.causal import OnHost, _HostVersion
 from iron_amd.lm.session import Session
 from tests.llama_support import SCALED, weights
+from tests.tilarax_support import built as tilarax
 
 oracle.install()
 
@@ -67,16 +70,16 @@ def loaded(cls, config):
     return model
 
 
-def other(token):
-    return (int(token) + 1) % CONFIG.vocab_size
+def other(model, token):
+    return (int(token) + 1) % model.config.vocab_size
 
 
 def another_token(model, prompt, drawn):
-    model.logits([*prompt, *drawn[:-1], other(drawn[-1])])
+    model.logits([*prompt, *drawn[:-1], other(model, drawn[-1])])
 
 
 def another_token_and_a_step(model, prompt, drawn):
-    foreign = [*prompt, *drawn[:-1], other(drawn[-1])]
+    foreign = [*prompt, *drawn[:-1], other(model, drawn[-1])]
     model.logits(foreign)
     model.logits([*foreign, 3])
 
@@ -86,7 +89,7 @@ def another_history(model, prompt, drawn):
 
 
 def another_draw(model, prompt, drawn):
-    given_up = model.session.draw(prompt[:5], 6, Sampler(1.5, 50, seed=9))
+    given_up = model.session.draw(prompt[:5], 6, Sampler(1.5, 20, seed=9))
     next(given_up), next(given_up)
     given_up.close()
 
@@ -180,6 +183,70 @@ def test_versions_stood_in_by_what_is_called_started_and_replayed_alone():
     prompt, tokens, behind = alone(CONFIG, greedy, Replayed, False)
     assert list(model.session.draw(prompt, 4)) == tokens
     assert np.array_equal(model.logits([*prompt, *tokens]), behind)
+
+
+# ---------------------------------------------------------------- a conversation as one request of a batched model
+class ReplayedBatch(_HostBatchVersion):
+    captured = True
+
+    def start(self):
+        self()
+
+    def replay(self, n=1):
+        for _ in range(n):
+            self()
+
+
+class EagerTilarax(BatchedOnHost, Tilarax):
+    pass
+
+
+class ReplayedTilarax(BatchedOnHost, Tilarax):
+    def load_versions(self, **_):
+        self.use(ReplayedBatch(self), ReplayedBatch(self, "ids"), ReplayedBatch(self, "picks"))
+
+
+def batched(cls):
+    model, _ = tilarax("mixed", cls, activations=np.float32, max_seq_len=64, prefill_chunk=16, slots=2)
+    model.load_versions()
+    return model
+
+
+def a_batch_of_others(model, prompt, drawn):
+    model.generate_batch([prompt[:3]], 3, [Sampler(1.5, 20, seed=9)])
+
+
+def everything_forgotten(model, prompt, drawn):
+    model.session.forget(0)
+    assert len(model.generate_batch([prompt[:3], prompt[:4]], 2)) == 2
+
+
+@functools.cache
+def alone_in_a_batch(cls, each):
+    model = batched(cls)
+    prompt = np.random.default_rng(4).integers(0, model.config.vocab_size, 21).tolist()
+    tokens = list(model.session.draw(prompt, 4, Sampler(1.5, 20, seed=2), each=each))
+    return prompt, tokens, model.logits([*prompt, *tokens])
+
+
+@pytest.mark.parametrize("between", [another_token, another_token_and_a_step, another_history, another_draw, another_greedy_draw, a_batch_of_others, everything_forgotten],
+                         ids=lambda f: f.__name__)
+@pytest.mark.parametrize("cls, each", [(EagerTilarax, False), (ReplayedTilarax, False), (ReplayedTilarax, True)])
+def test_what_a_consumer_does_between_two_tokens_of_a_request_changes_nothing(cls, each, between):
+    prompt, tokens, behind = alone_in_a_batch(cls, each)
+    model = batched(cls)
+    for places in ((1,), (1, 3), (4,)):
+        model.session.forget(0)
+        drawn = []
+        for token in model.session.draw(prompt, 4, Sampler(1.5, 20, seed=2), each=each):
+            drawn.append(token)
+            if len(drawn) in places:
+                between(model, prompt, drawn)
+        assert drawn == tokens, places
+        got = model.logits([*prompt, *tokens])
+        assert np.abs(got - behind).max() <= 1e-4 * np.abs(behind).max(), places   # (float32 states, in whatever portions)
+    pair = [list(batched(cls).session.draw(p, 4)) for p in (prompt, prompt[7:15])]
+    assert list(zip(*(model.session.draw(p, 4) for p in (prompt, prompt[7:15])))) == list(zip(*pair))
 
 
 class Notes:
