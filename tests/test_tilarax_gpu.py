@@ -405,6 +405,13 @@ def test_generation_replays_what_stepwise_decoding_draws(cuda):
         samplers = [[Sampler(0.9, 30, seed=s) for s in range(5)] for _ in range(2)]
         assert model.generate_batch(prompts, 25, samplers[0]) == model.generate_batch(prompts, 25, samplers[1])
         assert model.generate_batch(prompts, 40) == together   # greedy again
+        # A draw goes on as it was whatever its consumer has the conversation do in between.
+        drawn = []
+        for token in model.session.draw(prompts[0], 30, Sampler(0.9, 30, seed=1)):
+            drawn.append(token)
+            if len(drawn) in (1, 4):
+                model.logits(prompts[2]), next(model.session.draw(prompts[1], 3))
+        assert drawn == list(model.session.draw(prompts[0], 30, Sampler(0.9, 30, seed=1)))
     finally:
         model.release()
 
