@@ -31,6 +31,7 @@ from typing import Any, Generic, TypeVar
 
 import numpy as np
 
+from .._lib import current_stream
 from ..bf16 import bfloat16, from_torch, itemsize, round_bf16, to_bits
 from .declare import Operator, Precision, graph_recorder  # noqa: F401
 
@@ -1035,7 +1036,7 @@ class ScratchArena:
         self.uploaded: set[int] = set()
         self.generation = 0
         self.launched = 0   # calls, starts and runs of replays of any version so far
-        self.stream = None   # the last one that the arena was used on
+        self.stream, self.address = None, None   # the last one that the arena was used on
 
     def place_resident(self, r: Resident) -> int:
         if id(r) not in self.resident_offsets:
@@ -1082,14 +1083,18 @@ class ScratchArena:
     def enter(self) -> None:
         """The arena's next use is on the current stream: behind the last one on whatever stream that was, which may still run (a draw hands out a token with the
         next step under way), and the memory is not given to others before it is over.  On the stream of the last one that costs nothing but the question."""
+        address = current_stream()
+        if address == self.address:
+            return
         import torch
 
+        if torch.cuda.is_current_stream_capturing():   # (a caller's own capture begins on an idle device)
+            return
         stream = torch.cuda.current_stream()
-        if stream != self.stream and not torch.cuda.is_current_stream_capturing():   # (a caller's own capture begins on an idle device)
-            if self.stream is not None:
-                stream.wait_stream(self.stream)
-            self.buffer.record_stream(stream)
-            self.stream = stream
+        if self.stream is not None:
+            stream.wait_stream(self.stream)
+        self.buffer.record_stream(stream)
+        self.stream, self.address = stream, address
 
     def settle(self) -> None:
         """Wait on the host for the last use."""
@@ -1098,7 +1103,7 @@ class ScratchArena:
 
     def release(self) -> None:
         self.settle()
-        self.buffer = self.stream = None
+        self.buffer = self.stream = self.address = None
         self.uploaded.clear()
 
 
@@ -1230,6 +1235,7 @@ class CompiledGraph:
         self.arena.load()
         if self._loaded_generation == self.arena.generation:
             return self
+        self.arena.enter()
         base = self.arena.resident_offsets[id(self._words_resident)]
         self.words = self.arena.view(base, (WORD_SLOTS,), np.int32)
         self.expr_table = self.arena.view(base + WORD_SLOTS * 4, (WORD_SLOTS * EXPR_WORDS,), np.int32)

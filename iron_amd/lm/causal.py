@@ -284,8 +284,8 @@ class CausalLM(iron.Graph):
 
     @property
     def launched(self):
-        """What the versions say has been launched so far (see ``CompiledGraph.launched``)."""
-        return tuple(getattr(v, "launched", None) for v in (self.decode_step, self.prompt_chunk))
+        """How much has been launched so far, as the versions count it (see ``CompiledGraph.launched``; one that does not count: none)."""
+        return getattr(self.decode_step, "launched", None)
 
     # ------------------------------------------------------------------ use
     def logits(self, tokens) -> np.ndarray:
@@ -345,13 +345,16 @@ class _HostVersion:
     """A version stood in by the graph's host reference: same call, numpy underneath."""
 
     captured = False
-    launched = 0
 
     def __init__(self, graph, takes_ids: bool):
         self.graph, self.takes_ids = graph, takes_ids
 
+    @property
+    def launched(self) -> int:
+        return vars(self.graph).get("_launched_on_host", 0)
+
     def __call__(self, *tensors, **values):
-        self.launched += 1
+        vars(self.graph)["_launched_on_host"] = self.launched + 1
         outs, carried = iron.Graph.reference(self.graph, *tensors, **values)
         return (*(_HostOutput(o) for o in outs), iron.Carry(carried))
 

@@ -175,10 +175,11 @@ class Session:
         out = [int(carried["token"])]
         ran = model.launched
         yield out[0]
+        if replayed and self._interrupted(ran):
+            self._regain(ids, [], table)
+            step, started, ran = model.decode_step, False, model.launched
+            replayed = step.captured
         if replayed:
-            if self._interrupted(ran):
-                self._regain(ids, [], table)
-                step, started = model.decode_step, False
             if not started:
                 step.start(**carried)
             step.replay(remaining - 1)

@@ -12,6 +12,7 @@ import pytest
 import oracle
 from iron_amd.applications.llama import Llama
 from iron_amd.applications.tilarax import Tilarax
+from iron_amd.common import graph
 from iron_amd.lm import Sampler
 from iron_amd.lm.batched import BatchedOnHost, _HostBatchVersion
 from iron_amd.lm.causal import OnHost, _HostVersion
@@ -106,7 +107,15 @@ def a_call_of_its_own(model, prompt, drawn):
     model(token=7, position=2)
 
 
-BETWEEN = [another_token, another_token_and_a_step, another_history, another_draw, another_greedy_draw, another_session, a_call_of_its_own]
+def versions_loaded_anew(model, prompt, drawn):
+    model.load_versions()
+
+
+def versions_loaded_anew_and_not_captured(model, prompt, drawn):
+    OnHost.load_versions(model)
+
+
+BETWEEN = [versions_loaded_anew, versions_loaded_anew_and_not_captured, another_token, another_token_and_a_step, another_history, another_draw, another_greedy_draw, another_session, a_call_of_its_own]
 
 
 @functools.cache
@@ -270,9 +279,6 @@ class Notes:
             def __init__(self):
                 self.name = notes.stream
 
-            def __eq__(self, other):
-                return other is not None and self.name == other.name
-
             def wait_stream(self, other):
                 notes.on[self.name].append(("behind", other.name))
 
@@ -281,6 +287,7 @@ class Notes:
 
         monkeypatch.setattr(torch.cuda, "Event", Event)
         monkeypatch.setattr(torch.cuda, "current_stream", Stream)
+        monkeypatch.setattr(graph, "current_stream", lambda: notes.stream)
         monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
         monkeypatch.setattr(torch.Tensor, "record_stream", lambda tensor, stream: notes.put("held"))
 
